@@ -1,80 +1,174 @@
-// C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) with float accumulation in a fixed order.
+// C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) with float operands and float accumulation in a fixed order.
 //
-// This is the exact matrix product of the engine: every output element is the fused
-// multiply-add chain over k = 0 .. K-1, whatever M is and wherever the row lies in the
-// batch, so a row's result never depends on what else is in the step. It serves the
-// float32 path entirely, and the bfloat16 path wherever a weight is stored in float or
-// no faster kernel takes the shape. Inputs are converted to float on load (exact for
-// bf16); there is no reduced-precision mode.
+// This is the exact matrix product of the engine: every output element is the sum of GF_WAVES partial sums, partial w over
+// the blocks of 16 values of k whose number is w modulo GF_WAVES, in the order of k, added pairwise at the end; whatever M
+// is and wherever the row lies in the batch, so a row's result never depends on what else is in the step. It serves the
+// float32 path entirely, and the bfloat16 path wherever a weight is stored in float or no faster kernel takes the shape.
+// Inputs are converted to float on load (exact for bf16) and multiplied as floats (v_mfma_f32_16x16x4_f32); there is no
+// reduced-precision mode.
+//
+// What bounds it: the float matrix unit (256 flops a cycle and compute unit) where M is large, the bytes of W where it is
+// small. A wave of 16x16x4 products needs an operand value only once in 8 cycles, so the operands come straight from the
+// caches into registers, a block ahead of the products, without LDS; the waves of a workgroup split K instead of the tile,
+// so that a few hundred rows against a narrow weight still give every compute unit a tile with eight waves on it.
+// Measured (float, us in a model step of 221 tokens; before: a 64x64 tile of scalar multiply-adds a workgroup): N x K of
+// 1024 x 2048 and 1024 x 3072 405 -> 26, 4096 x 1024 164 -> 35, 6144 x 1024 168 -> 51; alone at 1,024 rows 24576 x 4096 runs at
+// 98 TFLOP/s, where a large library product reaches 135.
 #include "dispatch.h"
 
-#define RB_M 64
-#define RB_N 64
-#define RB_K 16
+typedef float gf_acc_t __attribute__((ext_vector_type(4)));
 
-template <typename TA, typename TW, typename TC>
-__global__ void __launch_bounds__(256)
-gemm_nt_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw, const TW* __restrict__ bias,
-               TC* __restrict__ C, long ldc, int M, int N, int K) {
-    __shared__ float As[RB_K][RB_M + 1];
-    __shared__ float Ws[RB_K][RB_N + 1];
-    const int tid = threadIdx.x;
-    const int tx = tid % 16;  // column direction
-    const int ty = tid / 16;  // row direction
-    const int m0 = blockIdx.y * RB_M;
-    const int n0 = blockIdx.x * RB_N;
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+#define GF_WAVES 8                  // of a workgroup; they split K
 
-    for (int k0 = 0; k0 < K; k0 += RB_K) {
-#pragma unroll
-        for (int l = 0; l < 4; ++l) {
-            const int idx = tid + 256 * l;
-            const int r = idx / RB_K;
-            const int k = idx % RB_K;
-            const int gm = m0 + r, gn = n0 + r, gk = k0 + k;
-            As[k][r] = (gm < M && gk < K) ? to_f(A[(size_t)gm * lda + gk]) : 0.f;
-            Ws[k][r] = (gn < N && gk < K) ? to_f(W[(size_t)gn * ldw + gk]) : 0.f;
+// four neighbours of a row from k on; beyond K (TAIL) zeros
+template <typename T, bool VEC, bool TAIL>
+__device__ __forceinline__ float4 gf_load(const T* __restrict__ row, int k, int K) {
+    if constexpr (VEC && !TAIL) {
+        if constexpr (sizeof(T) == 4) {
+            return *reinterpret_cast<const float4*>(row + k);
+        } else {
+            const uint2 u = *reinterpret_cast<const uint2*>(row + k);
+            return float4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                          __uint_as_float(u.y & 0xffff0000u)};
         }
-        __syncthreads();
+    } else {
+        float v[4];
 #pragma unroll
-        for (int kk = 0; kk < RB_K; ++kk) {
-            float a[4], w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) w[j] = Ws[kk][tx + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
+        for (int e = 0; e < 4; ++e) {
+            const float x = to_f(row[k + e < K ? k + e : 0]);
+            v[e] = k + e < K ? x : 0.f;
         }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int gm = m0 + ty + 16 * i;
-        if (gm >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int gn = n0 + tx + 16 * j;
-            if (gn >= N) continue;
-            float v = acc[i][j];
-            if (bias) v += to_f(bias[gn]);
-            C[(size_t)gm * ldc + gn] = from_f<TC>(v);
-        }
+        return float4{v[0], v[1], v[2], v[3]};
     }
 }
 
+// RM x RN: tiles of 16 rows and 16 columns a workgroup. VEC: rows of both operands start at addresses that four elements
+// can be loaded from at once.
+template <typename TA, typename TW, typename TC, int RM, int RN, int AHEAD, bool VEC>
+__global__ void __launch_bounds__(64 * GF_WAVES)
+gemm_nt_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw, const TW* __restrict__ bias,
+               TC* __restrict__ C, long ldc, int M, int N, int K) {
+    __shared__ gf_acc_t part[GF_WAVES / 2][RM * RN][64];
+    const int lane = threadIdx.x % MV_WAVE, wave = threadIdx.x / MV_WAVE, i = lane % 16, g = lane / 16;
+    const int m0 = blockIdx.y * (16 * RM), n0 = blockIdx.x * (16 * RN);
+    const TA* a_row[RM];
+    const TW* w_row[RN];
+#pragma unroll
+    for (int r = 0; r < RM; ++r) a_row[r] = A + (size_t)min(m0 + 16 * r + i, M - 1) * lda;      // (rows beyond the last are not stored)
+#pragma unroll
+    for (int c = 0; c < RN; ++c) w_row[c] = W + (size_t)min(n0 + 16 * c + i, N - 1) * ldw;
+    gf_acc_t acc[RM][RN];
+#pragma unroll
+    for (int r = 0; r < RM; ++r)
+#pragma unroll
+        for (int c = 0; c < RN; ++c) acc[r][c] = gf_acc_t{0.f, 0.f, 0.f, 0.f};
+    float4 a[RM], w[RN];
+    // a lane takes four neighbours in k for four products; they then sum over k in another order, the same for both operands
+    auto products = [&]() {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int r = 0; r < RM; ++r)
+#pragma unroll
+                for (int c = 0; c < RN; ++c)
+                    acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float*>(&a[r])[e],
+                                                                     reinterpret_cast<const float*>(&w[c])[e], acc[r][c], 0, 0, 0);
+    };
+    const int whole = K / 16;                        // blocks of 16; the wave's own: wave, wave + GF_WAVES, ...
+    float4 an[AHEAD][RM], wn[AHEAD][RN];
+    auto fetch = [&](int d, int b) {                 // (always issued, from a block that exists)
+        const int k = 16 * (b < whole ? b : 0) + 4 * g;
+#pragma unroll
+        for (int r = 0; r < RM; ++r) an[d][r] = gf_load<TA, VEC, false>(a_row[r], k, K);
+#pragma unroll
+        for (int c = 0; c < RN; ++c) wn[d][c] = gf_load<TW, VEC, false>(w_row[c], k, K);
+    };
+    if (whole > 0) {
+#pragma unroll
+        for (int d = 0; d < AHEAD; ++d) fetch(d, wave + d * GF_WAVES);
+    }
+    for (int b0 = wave; b0 < whole; b0 += AHEAD * GF_WAVES) {
+#pragma unroll
+        for (int d = 0; d < AHEAD; ++d) {
+            const int b = b0 + d * GF_WAVES;
+            if (b < whole) {
+#pragma unroll
+                for (int r = 0; r < RM; ++r) a[r] = an[d][r];
+#pragma unroll
+                for (int c = 0; c < RN; ++c) w[c] = wn[d][c];
+                fetch(d, b + AHEAD * GF_WAVES);      // flies under the products of the blocks between
+                products();
+            }
+        }
+    }
+    if (K % 16 != 0 && whole % GF_WAVES == wave) {
+#pragma unroll
+        for (int r = 0; r < RM; ++r) a[r] = gf_load<TA, VEC, true>(a_row[r], 16 * whole + 4 * g, K);
+#pragma unroll
+        for (int c = 0; c < RN; ++c) w[c] = gf_load<TW, VEC, true>(w_row[c], 16 * whole + 4 * g, K);
+        products();
+    }
+    // the waves' sums, pairwise: 4..7 into 0..3, 2..3 into 0..1, 1 into 0
+#pragma unroll
+    for (int half = GF_WAVES / 2; half >= 1; half /= 2) {
+        if (wave >= half && wave < 2 * half)
+#pragma unroll
+            for (int t = 0; t < RM * RN; ++t) part[wave - half][t][lane] = acc[t / RN][t % RN];
+        __syncthreads();
+        if (wave < half)
+#pragma unroll
+            for (int t = 0; t < RM * RN; ++t) acc[t / RN][t % RN] += part[wave][t][lane];
+        __syncthreads();
+    }
+    if (wave != 0) return;
+#pragma unroll
+    for (int c = 0; c < RN; ++c) {
+        const int n = n0 + 16 * c + i;
+        if (n >= N) continue;
+        const float add = bias ? to_f(bias[n]) : 0.f;
+#pragma unroll
+        for (int r = 0; r < RM; ++r)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int m = m0 + 16 * r + 4 * g + e;
+                if (m < M) C[(size_t)m * ldc + n] = from_f<TC>(bias ? acc[r][c][e] + add : acc[r][c][e]);
+            }
+    }
+}
+
+template <typename TA, typename TW, typename TC, int RM, int RN, int AHEAD>
+static void launch_tiles(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, long ldc, int M, int N, int K,
+                         hipStream_t stream) {
+    const bool vec = lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % (4 * sizeof(TA)) == 0 && (uintptr_t)W % (4 * sizeof(TW)) == 0;
+    dim3 grid((N + 16 * RN - 1) / (16 * RN), (M + 16 * RM - 1) / (16 * RM));
+    if (vec)
+        hipLaunchKernelGGL((gemm_nt_kernel<TA, TW, TC, RM, RN, AHEAD, true>), grid, dim3(64 * GF_WAVES), 0, stream, (const TA*)A, lda,
+                           (const TW*)W, ldw, (const TW*)bias, (TC*)C, ldc, M, N, K);
+    else
+        hipLaunchKernelGGL((gemm_nt_kernel<TA, TW, TC, RM, RN, AHEAD, false>), grid, dim3(64 * GF_WAVES), 0, stream, (const TA*)A, lda,
+                           (const TW*)W, ldw, (const TW*)bias, (TC*)C, ldc, M, N, K);
+}
+
+// The largest tile that still gives every compute unit one, since a larger one reads less a product; the bits do not depend
+// on it. Tiles of 32 x 64 where whole rounds of the chip by 64 x 64 leave it a quarter idle or more (221 x 6144 x 1024: 1.5
+// rounds, 57 us against 50), but not below 64 rows, where they are all of it (40 x 24576 x 4096: 235 us against 177).
 template <typename TA, typename TW, typename TC>
 static void launch_gemm(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, long ldc,
                         int M, int N, int K, hipStream_t stream) {
-    dim3 grid((N + RB_N - 1) / RB_N, (M + RB_M - 1) / RB_M);
-    hipLaunchKernelGGL((gemm_nt_kernel<TA, TW, TC>), grid, dim3(256), 0, stream, (const TA*)A, lda, (const TW*)W,
-                       ldw, (const TW*)bias, (TC*)C, ldc, M, N, K);
+    const long units = mv_compute_units();
+    auto tiles = [&](int rm, int rn) { return ((M + 16L * rm - 1) / (16 * rm)) * ((N + 16L * rn - 1) / (16 * rn)); };
+    // work of the unit that gets the most tiles, in tiles of 16 x 16
+    auto rounds = [&](int rm, int rn) { return (tiles(rm, rn) + units - 1) / units * rm * rn; };
+    if (M > 65535 * 32 || (M > 32 && tiles(4, 4) >= units && (M <= 64 || 4 * rounds(4, 4) <= 5 * rounds(2, 4))))
+        launch_tiles<TA, TW, TC, 4, 4, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+    else if (M > 64 && tiles(2, 4) >= units)
+        launch_tiles<TA, TW, TC, 2, 4, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+    else if (M > 16)
+        launch_tiles<TA, TW, TC, 2, 2, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+    else if (tiles(1, 4) >= units)
+        launch_tiles<TA, TW, TC, 1, 4, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+    else
+        launch_tiles<TA, TW, TC, 1, 1, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
 }
 
 // a_dtype: activations; w_dtype: weight and bias as stored; c_dtype: a_dtype or float.
@@ -88,7 +182,7 @@ extern "C" int mv_gemm_ref(const void* A, long lda, int a_dtype, const void* W, 
     MV_REQUIRE(c_dtype == a_dtype || c_dtype == MV_F32, "gemm: output dtype %d must be the activation dtype %d "
                "or float", c_dtype, a_dtype);
     if (M == 0) return 0;
-    MV_REQUIRE((M + RB_M - 1) / RB_M <= 65535, "gemm: M=%d too large for one launch", M);
+    MV_REQUIRE((M + 63) / 64 <= 65535, "gemm: M=%d too large for one launch", M);
     MV_DISPATCH_T(a_dtype, "gemm", {
         if (w_dtype == MV_F32) {
             if (c_dtype == MV_F32) launch_gemm<T, float, float>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
