@@ -224,7 +224,7 @@ template <typename T, int R, int L, bool V4>
 __global__ void __launch_bounds__(256)
 delta_scan_kernel(const T* __restrict__ packed, long ld, const float* __restrict__ coef, float* __restrict__ state,
                   const int* __restrict__ cu_seqlens, const int* __restrict__ state_slots, int H, int D,
-                  float* __restrict__ out, int n) {
+                  float* __restrict__ out, int n, int below) {
     constexpr int DPAD = L * R;                     // padded key size
     constexpr int COLS = 256 / L;                   // value columns of a workgroup
     constexpr int TT = DPAD > 128 ? 4 : (DPAD > 64 ? 8 : 16);          // tokens staged at a time
@@ -234,7 +234,7 @@ delta_scan_kernel(const T* __restrict__ packed, long ld, const float* __restrict
     __shared__ float svv[2][TT][COLS];
     const int seq = blockIdx.x, head = blockIdx.y, j0 = blockIdx.z * COLS;
     const int begin = cu_seqlens[seq], end = cu_seqlens[seq + 1];
-    if (end <= begin) return;
+    if (end <= begin || (below > 0 && end - begin >= below)) return;
     const int tid = threadIdx.x;
     const int sub = tid % L;
     const int col = tid / L;
@@ -332,8 +332,9 @@ delta_scan_kernel(const T* __restrict__ packed, long ld, const float* __restrict
     delta_state_io<R, true>(s, S, sub, D, live);
 }
 
+// below > 0: requests of at least so many tokens are left alone (mv_delta_chunks takes them)
 extern "C" int mv_delta_scan(const void* packed, long ld, const float* coef, float* state, const int* cu_seqlens,
-                             const int* state_slots, int n_seqs, int n, int H, int D, float* out, int dtype,
+                             const int* state_slots, int n_seqs, int n, int H, int D, int below, float* out, int dtype,
                              hipStream_t stream) {
     MV_REQUIRE(n >= 0 && n_seqs >= 0 && H > 0 && D > 0, "delta_scan: bad sizes n=%d seqs=%d H=%d D=%d", n, n_seqs, H, D);
     MV_REQUIRE(D <= 256, "delta_scan: head size %d exceeds the supported maximum 256", D);
@@ -350,11 +351,11 @@ extern "C" int mv_delta_scan(const void* packed, long ld, const float* coef, flo
     if (v4) {                                                                                                            \
         MV_DISPATCH_T(dtype, "delta_scan",                                                                               \
                       hipLaunchKernelGGL((delta_scan_kernel<T, RR, LL, true>), grid, dim3(256), 0, stream, (const T*)packed, \
-                                         ld, coef, state, cu_seqlens, state_slots, H, D, out, n))                        \
+                                         ld, coef, state, cu_seqlens, state_slots, H, D, out, n, below))                        \
     } else {                                                                                                             \
         MV_DISPATCH_T(dtype, "delta_scan",                                                                               \
                       hipLaunchKernelGGL((delta_scan_kernel<T, RR, LL, false>), grid, dim3(256), 0, stream, (const T*)packed, \
-                                         ld, coef, state, cu_seqlens, state_slots, H, D, out, n))                        \
+                                         ld, coef, state, cu_seqlens, state_slots, H, D, out, n, below))                        \
     }
     if (R == 4 && L == 4) {
         DS_LAUNCH(4, 4);
@@ -880,7 +881,7 @@ template <int R, int L, bool READ>
 __global__ void __launch_bounds__(256)
 state_scan_kernel(const float* __restrict__ qk, const float* __restrict__ vals, const float* __restrict__ gates,
                   float* __restrict__ state, const int* __restrict__ cu_seqlens, const int* __restrict__ state_slots, int H,
-                  int G, int DK, int DV, float* __restrict__ out) {
+                  int G, int DK, int DV, int below, float* __restrict__ out) {
     constexpr int DPAD = L * R;
     constexpr int COLS = 256 / L;
     constexpr int TT = DPAD > 128 ? 4 : (DPAD > 64 ? 8 : 16);
@@ -889,7 +890,7 @@ state_scan_kernel(const float* __restrict__ qk, const float* __restrict__ vals, 
     __shared__ float sg[TT][2];
     const int seq = blockIdx.x, head = blockIdx.y, j0 = blockIdx.z * COLS;
     const int begin = cu_seqlens[seq], end = cu_seqlens[seq + 1];
-    if (end <= begin) return;
+    if (end <= begin || (below > 0 && end - begin >= below)) return;
     const int tid = threadIdx.x, sub = tid % L, col = tid / L;
     const int j = j0 + col;
     const bool live = j < DV;
@@ -957,8 +958,9 @@ state_scan_kernel(const float* __restrict__ qk, const float* __restrict__ vals, 
     delta_state_io<R, true>(s, S, sub, DK, live);
 }
 
+// below > 0: requests of at least so many tokens are left alone (mv_delta_chunks takes them)
 extern "C" int mv_state_scan(const float* qk, const float* vals, const float* gates, float* state, const int* cu_seqlens,
-                             const int* state_slots, int n_seqs, int n, int H, int G, int DK, int DV, int read,
+                             const int* state_slots, int n_seqs, int n, int H, int G, int DK, int DV, int read, int below,
                              float* out, hipStream_t stream) {
     MV_REQUIRE(n >= 0 && n_seqs >= 0 && H > 0 && G > 0 && H % G == 0 && DK > 0 && DV > 0,
                "state_scan: bad sizes n=%d seqs=%d H=%d G=%d DK=%d DV=%d", n, n_seqs, H, G, DK, DV);
@@ -973,10 +975,10 @@ extern "C" int mv_state_scan(const float* qk, const float* vals, const float* ga
 #define MS_LAUNCH(RR, LL)                                                                                                  \
     if (read)                                                                                                              \
         hipLaunchKernelGGL((state_scan_kernel<RR, LL, true>), grid, dim3(256), 0, stream, qk, vals, gates, state, cu_seqlens, \
-                           state_slots, H, G, DK, DV, out);                                                                \
+                           state_slots, H, G, DK, DV, below, out);                                                         \
     else                                                                                                                   \
         hipLaunchKernelGGL((state_scan_kernel<RR, LL, false>), grid, dim3(256), 0, stream, qk, vals, gates, state,         \
-                           cu_seqlens, state_slots, H, G, DK, DV, out);
+                           cu_seqlens, state_slots, H, G, DK, DV, below, out);
     if (R == 4 && L == 4) {
         MS_LAUNCH(4, 4)
     } else if (R == 4 && L == 8) {

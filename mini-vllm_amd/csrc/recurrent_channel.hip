@@ -283,7 +283,7 @@ template <int R, int L, bool V4>
 __global__ void __launch_bounds__(256)
 channel_scan_kernel(const float* __restrict__ qk, const float* __restrict__ vals, const float* __restrict__ beta,
                     const float* __restrict__ decay, long ldz, float* __restrict__ state, const int* __restrict__ cu_seqlens,
-                    const int* __restrict__ state_slots, int H, int G, int DK, int DV, float* __restrict__ out) {
+                    const int* __restrict__ state_slots, int H, int G, int DK, int DV, int below, float* __restrict__ out) {
     constexpr int DPAD = L * R;
     constexpr int COLS = 256 / L;
     constexpr int TT = DPAD > 128 ? 4 : (DPAD > 64 ? 8 : 16);          // tokens staged at a time
@@ -295,7 +295,7 @@ channel_scan_kernel(const float* __restrict__ qk, const float* __restrict__ vals
     __shared__ float sb[2][TT];
     const int seq = blockIdx.x, head = blockIdx.y, j0 = blockIdx.z * COLS;
     const int begin = cu_seqlens[seq], end = cu_seqlens[seq + 1];
-    if (end <= begin) return;
+    if (end <= begin || (below > 0 && end - begin >= below)) return;
     const int tid = threadIdx.x, sub = tid % L, col = tid / L;
     const int j = j0 + col;
     const bool live = j < DV;
@@ -385,9 +385,10 @@ channel_scan_kernel(const float* __restrict__ qk, const float* __restrict__ vals
     delta_state_io<R, true>(s, S, sub, DK, live);
 }
 
+// below > 0: requests of at least so many tokens are left alone (mv_delta_chunks takes them)
 extern "C" int mv_channel_scan(const float* qk, const float* vals, const float* beta, const float* decay, long ldz, float* state,
                                const int* cu_seqlens, const int* state_slots, int n_seqs, int n, int H, int G, int DK, int DV,
-                               float* out, hipStream_t stream) {
+                               int below, float* out, hipStream_t stream) {
     MV_REQUIRE(n >= 0 && n_seqs >= 0 && H > 0 && G > 0 && H % G == 0 && DK > 0 && DV > 0,
                "channel_scan: bad sizes n=%d seqs=%d H=%d G=%d DK=%d DV=%d", n, n_seqs, H, G, DK, DV);
     MV_REQUIRE(DK <= 256, "channel_scan: key size %d exceeds the supported maximum 256", DK);
@@ -402,10 +403,10 @@ extern "C" int mv_channel_scan(const float* qk, const float* vals, const float* 
 #define CS_LAUNCH(RR, LL)                                                                                                     \
     if (v4)                                                                                                                   \
         hipLaunchKernelGGL((channel_scan_kernel<RR, LL, true>), grid, dim3(256), 0, stream, qk, vals, beta, decay, ldz, state, \
-                           cu_seqlens, state_slots, H, G, DK, DV, out);                                                       \
+                           cu_seqlens, state_slots, H, G, DK, DV, below, out);                                                       \
     else                                                                                                                      \
         hipLaunchKernelGGL((channel_scan_kernel<RR, LL, false>), grid, dim3(256), 0, stream, qk, vals, beta, decay, ldz, state, \
-                           cu_seqlens, state_slots, H, G, DK, DV, out);
+                           cu_seqlens, state_slots, H, G, DK, DV, below, out);
     if (R == 4 && L == 4) {
         CS_LAUNCH(4, 4)
     } else if (R == 4 && L == 8) {

@@ -1,0 +1,583 @@
+// The recurrences of recurrent.hip and recurrent_channel.hip for requests that bring many tokens in a step: a request's
+// tokens are cut into chunks of DC_TOKENS, everything that concerns one chunk alone is a product of small matrices on the
+// MFMA units (float operands, v_mfma_f32_16x16x4_f32), chunks and heads side by side, and only a walk along the chunks
+// with one product each is left in a row. All four rules are, per head with S [key size DK][columns DV],
+//     p = a^T S;   S <- diag(w) S + b p^T + x v^T;   o = S^T r
+//   RULE_GENERAL  Bolapel's delta rule: w the decay, a = u, b = -(rate u), x = k
+//   RULE_CHANNEL  the gated delta rule with a decay g per key channel: w = g, a = g k, x = beta k, b = -x
+//   RULE_GATED    the same with one decay per head
+//   RULE_SUM      the mLSTM's matrix memory: w the forget gate, no p, x = k, v times the input gate
+// With tokens s, t counted inside a chunk, P_t = w_0 .. w_t per channel, P_{-1} = 1 and S_0 the state in front of the chunk,
+//     A[t][s] = sum_i a_t (P_{t-1} / P_s) x_s (s < t),  B[t][s] = sum_i r_t (P_t / P_s) x_s (s <= t),  A', B' with b for x,
+//     T = (I - A')^-1,  W = T (a_t P_{t-1})_t,  U = T A V        (then p = W S_0 + U)
+//     S_1 = M S_0 + N,  M = diag(P_last) + B_e W,  N = X_e V + B_e U,  X_e = (x_s P_last / P_s)^T, B_e with b
+//     o   = Q S_0 + O,  Q = (r_t P_t)_t + B' W,     O = B V + B' U
+// The first kernel leaves M, N, Q and (in the output's rows) O; the second walks S <- M S + N and adds Q S to the output.
+// Only quotients P_t / P_s with s <= t occur, as products of decays (never a division, so decays down to zero and chunks
+// that forget everything are exact): inside a run of DC_RUN tokens term by term, between the two runs of a chunk as (what
+// is left of s at its run's end) times (what is left of that at t), which is a product on the MFMA units again.
+//
+// What bounded these before was one chain of about 0.2 us a token for every (request, head, 16 columns), 64 workgroups
+// for a head count of 16; the chunks' work is spread over every compute unit and the chain is one product of DK x DK with
+// DK x 16 a chunk. Measured on one prompt of
+// 2,048 tokens, 16 heads of 64 x 64 (us, scan against the two kernels here): GENERAL 438 -> 68 + 57, GATED 477 -> 41 + 58,
+// SUM with 65 columns 411 -> 30 + 36; CHANNEL on prompts of 1,137 and 463 tokens 216 -> 36 + 31. The chunk kernel waits for
+// its own phases (eight waves a workgroup hide that best: four took 90, 49, 36 and 45), the walk for a round of matrix unit,
+// LDS and barrier a chunk, 0.9 us.
+//
+// Layouts are those of the scans: states and N [..][H][DV][DK] (a head's matrix column by column), M [chunks][H][DK][DK],
+// Q [n][H][DK], out [n][H][DV].
+#include "recurrent_chunk.h"
+
+#define DC_TOKENS 32
+#define DC_RUN 16                  // half a chunk: two runs
+// Requests with fewer tokens of a step are left to the scans. There a token's bits do not depend on how the request was cut;
+// here they depend on where the chunks lie. A
+// scan of 128 tokens takes 28 us, the two kernels for one such request about 15: the line lies where there is something to
+// gain, and above the portions that are worth having bit for bit.
+#define DC_LINE 128
+
+enum DeltaRule { RULE_GENERAL = 0, RULE_CHANNEL = 1, RULE_GATED = 2, RULE_SUM = 3 };
+
+struct DeltaChunkArgs {
+    const float* vec;              // GENERAL: coef [n][H][5][DK] (w, rate u, u, k, r); else qk [n][G][2][DK]
+    const float* gates;            // CHANNEL: beta [n][H]; GATED, SUM: [n][H][4] (decay, strength, ..)
+    const float* decay; long ldz;  // CHANNEL: rows whose first H*DK columns are the decays
+    const void* vals; long ldv;    // GENERAL: packed rows, the values in columns 2*H*DK ..; else [n][H][DV] floats
+    int H, G, DV;
+    const int* cu_seqlens; int n_seqs;
+    float* M; float* N; float* Q; float* out;
+};
+
+#define DC_THREADS 512
+
+// find_chunk, for requests of at least DC_LINE tokens and DC_THREADS threads (the first 256 search)
+__device__ __forceinline__ void find_long_chunk(const int* __restrict__ cu, int n_seqs, int unit, int* sh, int& seq, int& row0, int& count) {
+    const int tid = threadIdx.x, lane = tid % MV_WAVE, wave = tid / MV_WAVE;
+    if (tid == 0) sh[4] = -1;
+    int base = 0;
+    for (int s0 = 0; s0 < n_seqs; s0 += 256) {
+        const int s = s0 + tid;
+        const int first = s < n_seqs ? cu[s] : 0, len = s < n_seqs ? cu[s + 1] - first : 0;
+        const int mine = tid < 256 && len >= DC_LINE ? (len + DC_TOKENS - 1) / DC_TOKENS : 0;
+        int incl = mine;
+#pragma unroll
+        for (int o = 1; o < MV_WAVE; o <<= 1) {
+            const int t = __shfl_up(incl, o, MV_WAVE);
+            if (lane >= o) incl += t;
+        }
+        __syncthreads();
+        if (lane == MV_WAVE - 1 && wave < 4) sh[wave] = incl;
+        __syncthreads();
+        int before = base;
+        for (int w = 0; w < wave && w < 4; ++w) before += sh[w];
+        incl += before;
+        if (unit < incl && unit >= incl - mine) {
+            const int c = unit - (incl - mine);
+            sh[4] = s;
+            sh[5] = first + c * DC_TOKENS;
+            sh[6] = min(len - c * DC_TOKENS, DC_TOKENS);
+        }
+        base += sh[0] + sh[1] + sh[2] + sh[3];
+        if (base > unit) break;                        // (the same for every thread)
+    }
+    __syncthreads();
+    seq = sh[4];
+    row0 = sh[5];
+    count = seq >= 0 ? sh[6] : 0;
+}
+
+// acc += A B over 16 values of k: A's rows hold neighbouring k side by side, B's rows are k
+__device__ __forceinline__ void mfma_row_col(floatx4_t& acc, const float* a_row, const float* b_k0, int pitch, int g) {
+    const float4 a = *reinterpret_cast<const float4*>(a_row + 4 * g);
+    const float* b = b_k0 + (size_t)(4 * g) * pitch;
+    mfma4(acc, a, float4{b[0], b[pitch], b[2 * pitch], b[3 * pitch]});
+}
+// acc += A^T B over 16 values of k: the rows of both are k
+__device__ __forceinline__ void mfma_col_col(floatx4_t& acc, const float* a_k0, int pa, const float* b_k0, int pb, int g) {
+    const float* a = a_k0 + (size_t)(4 * g) * pa;
+    const float* b = b_k0 + (size_t)(4 * g) * pb;
+    mfma4(acc, float4{a[0], a[pa], a[2 * pa], a[3 * pa]}, float4{b[0], b[pb], b[2 * pb], b[3 * pb]});
+}
+
+// ---- what concerns one chunk alone: workgroup (chunk, head)
+template <typename T, int DK, int RULE>
+__global__ void __launch_bounds__(DC_THREADS)
+delta_chunk_kernel(DeltaChunkArgs A) {
+    constexpr int C = DC_TOKENS, R16 = DC_RUN;
+    constexpr bool PAIR = RULE == RULE_GENERAL;                // b is not -x: sources of two kinds
+    constexpr bool READ = RULE != RULE_SUM;
+    constexpr int P = DK + 4;                                  // pitch of rows of key channels
+    constexpr int DVMAX = DK + 16, PV = DVMAX + 4;             // of value columns
+    constexpr int PC = C + 4;                                  // of tokens
+    __shared__ __attribute__((aligned(16))) float sA[READ ? C : 1][P], sX[C][P], sR[C][P], sW[C][P], sB[PAIR ? C : 1][P];
+    __shared__ __attribute__((aligned(16))) float sV[C][PV], sU[READ ? C : 1][PV];
+    __shared__ __attribute__((aligned(16))) float mA[READ ? C : 1][PC], mB[C][PC], mA2[PAIR ? C : 1][PC], mB2[PAIR ? C : 1][PC], mT[READ ? C : 1][PC],
+        mG[READ ? C : 1][PC];
+    __shared__ float full[2][DK];                              // a run's decays multiplied
+    __shared__ int sh[8];
+    int seq, row0, count;
+    find_long_chunk(A.cu_seqlens, A.n_seqs, blockIdx.x, sh, seq, row0, count);
+    if (count <= 0) return;
+    const int head = blockIdx.y, H = A.H, DV = A.DV;
+    const int tid = threadIdx.x, lane = tid % MV_WAVE, wave = tid / MV_WAVE, i = lane % 16, g = lane / 16;
+    const int NT = (DV + 15) / 16;                             // tiles of value columns
+
+    // the chunk's vectors; rows beyond its tokens change nothing (decay one, everything else zero)
+    const int group = RULE == RULE_GENERAL ? head : head / (H / A.G);
+    for (int x = tid; x < C * (DK / 4); x += DC_THREADS) {
+        const int t = x / (DK / 4), c = (x % (DK / 4)) * 4;
+        const bool ok = t < count;
+        const size_t row = row0 + (ok ? t : 0);
+        const float4 zero{0.f, 0.f, 0.f, 0.f};
+        auto at = [&](const float* p) __attribute__((always_inline)) { return *reinterpret_cast<const float4*>(p + c); };
+        float4 w, a = zero, xx, r, b = zero;
+        if constexpr (RULE == RULE_GENERAL) {
+            const float* v = A.vec + (row * H + head) * 5 * DK;
+            w = at(v); b = at(v + DK); a = at(v + 2 * DK); xx = at(v + 3 * DK); r = at(v + 4 * DK);
+            b = float4{-b.x, -b.y, -b.z, -b.w};
+        } else {
+            const float* v = A.vec + (row * A.G + group) * 2 * DK;
+            r = at(v);
+            xx = at(v + DK);
+            if constexpr (RULE == RULE_CHANNEL) {
+                w = at(A.decay + row * A.ldz + (size_t)head * DK);
+            } else {
+                const float d = A.gates[(row * H + head) * 4];
+                w = float4{d, d, d, d};
+            }
+            if constexpr (READ) {
+                const float beta = RULE == RULE_CHANNEL ? A.gates[row * H + head] : A.gates[(row * H + head) * 4 + 1];
+                a = float4{w.x * xx.x, w.y * xx.y, w.z * xx.z, w.w * xx.w};
+                xx = float4{beta * xx.x, beta * xx.y, beta * xx.z, beta * xx.w};
+            }
+        }
+        *reinterpret_cast<float4*>(&sW[t][c]) = ok ? w : float4{1.f, 1.f, 1.f, 1.f};
+        *reinterpret_cast<float4*>(&sX[t][c]) = ok ? xx : float4{0.f, 0.f, 0.f, 0.f};
+        *reinterpret_cast<float4*>(&sR[t][c]) = ok ? r : float4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (READ) *reinterpret_cast<float4*>(&sA[t][c]) = ok ? a : float4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (PAIR) *reinterpret_cast<float4*>(&sB[t][c]) = ok ? b : float4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int x = tid; x < C * DVMAX; x += DC_THREADS) {
+        const int t = x / DVMAX, j = x % DVMAX;
+        const bool ok = t < count && j < DV;
+        const size_t row = row0 + (ok ? t : 0);
+        const int jj = ok ? j : 0;
+        float v;
+        if constexpr (RULE == RULE_GENERAL) v = to_f(((const T*)A.vals)[row * A.ldv + 2 * (size_t)H * DK + (size_t)head * DK + jj]);
+        else v = ((const float*)A.vals)[(row * H + head) * DV + jj];
+        if constexpr (RULE == RULE_SUM) v *= A.gates[(row * H + head) * 4 + 1];
+        sV[t][j] = ok ? v : 0.f;
+    }
+    __syncthreads();
+
+    // A and B inside a run: LP lanes share a source token s and walk t along its run with what is left of x_s
+    constexpr int LP = 16, CH = DK / LP;                       // channels of a lane
+    static_assert(C * LP == DC_THREADS, "a source token for every sixteen lanes");
+    {
+        const int src = tid / LP, first = src / R16 * R16, s = src % R16, c = (tid % LP) * CH;
+        float d[CH], e[CH];
+        auto take = [&](float (&v)[CH], const float* p) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < CH; q += 4) {
+                const float4 x = *reinterpret_cast<const float4*>(p + q);
+                v[q] = x.x; v[q + 1] = x.y; v[q + 2] = x.z; v[q + 3] = x.w;
+            }
+        };
+        take(d, &sX[src][c]);
+        if constexpr (PAIR) take(e, &sB[src][c]);
+#pragma unroll 4
+        for (int t = 0; t < R16; ++t) {
+            const int row = first + t;
+            float w[CH], r[CH], da = 0.f, db = 0.f, ea = 0.f, eb = 0.f;
+            take(w, &sW[row][c]);
+            take(r, &sR[row][c]);
+            const bool behind = t > s;
+            if constexpr (READ) {
+                float a[CH];
+                take(a, &sA[row][c]);
+#pragma unroll
+                for (int q = 0; q < CH; ++q) {
+                    da = fmaf(a[q], d[q], da);
+                    if constexpr (PAIR) ea = fmaf(a[q], e[q], ea);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < CH; ++q) {
+                d[q] = behind ? d[q] * w[q] : d[q];
+                db = fmaf(r[q], d[q], db);
+                if constexpr (PAIR) {
+                    e[q] = behind ? e[q] * w[q] : e[q];
+                    eb = fmaf(r[q], e[q], eb);
+                }
+            }
+            if constexpr (READ) da = lanes_sum<LP>(da);
+            db = lanes_sum<LP>(db);
+            if constexpr (PAIR) { ea = lanes_sum<LP>(ea); eb = lanes_sum<LP>(eb); }
+            if (tid % LP == 0) {
+                if constexpr (READ) mA[row][src] = behind ? da : 0.f;
+                mB[row][src] = t >= s ? db : 0.f;
+                if constexpr (PAIR) {
+                    mA2[row][src] = behind ? ea : 0.f;
+                    mB2[row][src] = t >= s ? eb : 0.f;
+                }
+            }
+        }
+    }
+    __syncthreads();
+
+    // what is left of a token's sources at its run's end, and of a run's start at a token
+    for (int x = tid; x < 4 * DK; x += DC_THREADS) {
+        const int c = x % DK, run = (x / DK) % 2, first = run * R16;
+        float f = 1.f;
+        if (x < 2 * DK) {
+            for (int t = 0; t < R16; ++t) {
+                if constexpr (READ) sA[first + t][c] *= f;
+                f *= sW[first + t][c];
+                sR[first + t][c] *= f;
+            }
+            full[run][c] = f;
+        } else {
+            for (int t = R16 - 1; t >= 0; --t) {
+                sX[first + t][c] *= f;
+                if constexpr (PAIR) sB[first + t][c] *= f;
+                f *= sW[first + t][c];
+            }
+        }
+    }
+    // (no token of the first run sees the second)
+    if (tid < R16 * R16) {
+        const int t = tid / R16, s = R16 + tid % R16;
+        mB[t][s] = 0.f;
+        if constexpr (READ) mA[t][s] = 0.f;
+        if constexpr (PAIR) mA2[t][s] = mB2[t][s] = 0.f;
+        if constexpr (READ) mT[t][s] = 0.f;
+    }
+    __syncthreads();
+
+    // between the runs, and (first wave) the inverses of the two runs' own blocks, a column a lane
+    auto between = [&](float (&dst)[C][PC], const float (&rows)[C][P], const float (&cols)[C][P]) __attribute__((always_inline)) {
+        floatx4_t acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < DK; k += 16)
+            mfma4(acc, *reinterpret_cast<const float4*>(&rows[R16 + i][k + 4 * g]), *reinterpret_cast<const float4*>(&cols[i][k + 4 * g]));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) dst[R16 + 4 * g + q][i] = acc[q];
+    };
+    if (wave == 1) between(mB, sR, sX);
+    if constexpr (READ) {
+        if (wave == 2) between(mA, sA, sX);
+        if constexpr (PAIR) {
+            if (wave == 3) between(mA2, sA, sB);
+            if (wave == 5) between(mB2, sR, sB);
+        }
+        if (wave == 0 && lane < C) {
+            const int first = lane / R16 * R16, c = lane % R16;
+            float col[R16];
+#pragma unroll
+            for (int t = 0; t < R16; ++t) {
+                float acc = t == c ? 1.f : 0.f;
+#pragma unroll
+                for (int s = 0; s < t; ++s) {
+                    if constexpr (PAIR) acc = fmaf(mA2[first + t][first + s], col[s], acc);
+                    else acc = fmaf(-mA[first + t][first + s], col[s], acc);
+                }
+                col[t] = acc;
+                mT[first + t][first + c] = acc;
+            }
+        }
+    }
+    __syncthreads();
+    // the inverse's block between the runs: T22 (A'21 T11); the sources of the first run reach the chunk's end, the
+    // second run's tokens the chunk's start
+    if constexpr (READ) {
+        if (wave == 0) {
+            floatx4_t acc{0.f, 0.f, 0.f, 0.f};
+            mfma_row_col(acc, PAIR ? &mA2[R16 + i][0] : &mA[R16 + i][0], &mT[0][i], PC, g);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) mG[4 * g + q][i] = PAIR ? acc[q] : -acc[q];
+        }
+    }
+    for (int x = tid; x < R16 * DK; x += DC_THREADS) {
+        const int t = x / DK, c = x % DK;
+        sR[R16 + t][c] *= full[0][c];
+        if constexpr (READ) sA[R16 + t][c] *= full[0][c];
+        sX[t][c] *= full[1][c];
+        if constexpr (PAIR) sB[t][c] *= full[1][c];
+    }
+    __syncthreads();
+    if constexpr (READ) {
+        if (wave == 0) {
+            floatx4_t acc{0.f, 0.f, 0.f, 0.f};
+            mfma_row_col(acc, &mT[R16 + i][R16], &mG[0][i], PC, g);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) mT[R16 + 4 * g + q][i] = acc[q];
+        }
+        __syncthreads();
+        // W = T (a P) over the decays' rows, which are used up; G = T A
+        for (int job = wave; job < 2 * (DK / 16) + 4; job += DC_THREADS / 64) {
+            const bool is_w = job < 2 * (DK / 16);
+            const int rt = is_w ? job % 2 : (job - 2 * (DK / 16)) % 2, ct = is_w ? job / 2 : (job - 2 * (DK / 16)) / 2;
+            floatx4_t acc{0.f, 0.f, 0.f, 0.f};
+            for (int k = 0; k <= 16 * rt; k += 16)
+                mfma_row_col(acc, &mT[16 * rt + i][k], is_w ? &sA[k][16 * ct + i] : &mA[k][16 * ct + i], is_w ? P : PC, g);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (is_w) sW[16 * rt + 4 * g + q][16 * ct + i] = acc[q];
+                else mG[16 * rt + 4 * g + q][16 * ct + i] = acc[q];
+            }
+        }
+        __syncthreads();
+        // U = G V, or what replaces V where b = -x: V - U
+        for (int job = wave; job < 2 * NT; job += DC_THREADS / 64) {
+            const int rt = job % 2, ct = job / 2;
+            floatx4_t acc{0.f, 0.f, 0.f, 0.f};
+            for (int k = 0; k <= 16 * rt; k += 16) mfma_row_col(acc, &mG[16 * rt + i][k], &sV[k][16 * ct + i], PV, g);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int t = 16 * rt + 4 * g + q;
+                sU[t][16 * ct + i] = PAIR ? acc[q] : sV[t][16 * ct + i] - acc[q];
+            }
+        }
+        __syncthreads();
+    }
+    // what the walk needs
+    const size_t unit = (size_t)blockIdx.x * H + head;
+    const float (*E)[PV] = (READ && !PAIR) ? sU : sV;          // the values the sources x carry
+    constexpr int KT = DK / 16;
+    const int jobs_n = NT * KT, jobs_m = READ ? KT * KT : 0, jobs_q = READ ? 2 * KT : 0, jobs_o = 2 * NT;
+    for (int job = wave; job < jobs_n + jobs_m + jobs_q + jobs_o; job += DC_THREADS / 64) {
+        floatx4_t acc{0.f, 0.f, 0.f, 0.f};
+        int j = job;
+        if (j < jobs_n) {                                      // N, column by column: rows of the product are value columns
+            const int vt = j / KT, kt = j % KT;
+#pragma unroll
+            for (int k = 0; k < C; k += 16) {
+                mfma_col_col(acc, &E[k][16 * vt + i], PV, &sX[k][16 * kt + i], P, g);
+                if constexpr (PAIR) mfma_col_col(acc, &sU[k][16 * vt + i], PV, &sB[k][16 * kt + i], P, g);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int v = 16 * vt + 4 * g + q;
+                if (v < DV) A.N[(unit * DV + v) * DK + 16 * kt + i] = acc[q];
+            }
+            continue;
+        }
+        j -= jobs_n;
+        if (j < jobs_m) {
+            const int rt = j / KT, ct = j % KT;
+#pragma unroll
+            for (int k = 0; k < C; k += 16)
+                mfma_col_col(acc, PAIR ? &sB[k][16 * rt + i] : &sX[k][16 * rt + i], P, &sW[k][16 * ct + i], P, g);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = 16 * rt + 4 * g + q, c = 16 * ct + i;
+                const float m = PAIR ? acc[q] : -acc[q];
+                A.M[(unit * DK + r) * DK + c] = r == c ? full[0][c] * full[1][c] + m : m;
+            }
+            continue;
+        }
+        j -= jobs_m;
+        if (j < jobs_q) {
+            const int rt = j % 2, ct = j / 2;
+            for (int k = 0; k <= 16 * rt; k += 16)
+                mfma_row_col(acc, PAIR ? &mB2[16 * rt + i][k] : &mB[16 * rt + i][k], &sW[k][16 * ct + i], P, g);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int t = 16 * rt + 4 * g + q, c = 16 * ct + i;
+                if (t < count) A.Q[((size_t)(row0 + t) * H + head) * DK + c] = PAIR ? sR[t][c] + acc[q] : sR[t][c] - acc[q];
+            }
+            continue;
+        }
+        j -= jobs_q;
+        const int rt = j % 2, ct = j / 2;
+        for (int k = 0; k <= 16 * rt; k += 16) {
+            mfma_row_col(acc, &mB[16 * rt + i][k], &E[k][16 * ct + i], PV, g);
+            if constexpr (PAIR) mfma_row_col(acc, &mB2[16 * rt + i][k], &sU[k][16 * ct + i], PV, g);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int t = 16 * rt + 4 * g + q, v = 16 * ct + i;
+            if (t < count && v < DV) A.out[((size_t)(row0 + t) * H + head) * DV + v] = acc[q];
+        }
+    }
+    if constexpr (!READ) {                                     // M is the one decay of the chunk, Q the queries as they are left
+        if (tid == 0) A.M[unit] = full[0][0] * full[1][0];
+        for (int x = tid; x < C * DK; x += DC_THREADS) {
+            const int t = x / DK, c = x % DK;
+            if (t < count) A.Q[((size_t)(row0 + t) * H + head) * DK + c] = sR[t][c];
+        }
+    }
+}
+
+// ---- the walk: workgroup (request, head, 16 value columns). The first KT waves own 16 rows of the state each, the last
+// four the output: waves of one SIMD unit then share its matrix unit evenly. An output wave owns 16 tokens and half of
+// the key channels; the two halves of a tile meet in LDS a step later. What a step reads of memory is asked for DEPTH
+// steps ahead, and always asked for, also by steps beyond the last chunk (DEPTH divides the number of steps) and by
+// lanes that have no use for it: a load that some path leaves out makes the wait for an older one a wait for all
+// (1.4 us a step; 64 steps of 16 heads took 92 us, 57 without).
+template <int DK, bool READ>
+__global__ void __launch_bounds__((DK / 16 + 4) * 64)
+delta_chunk_walk_kernel(DeltaChunkArgs A, float* __restrict__ state, const int* __restrict__ state_slots) {
+    constexpr int KT = DK / 16, DEPTH = DK <= 64 ? 4 : 2, P = DK + 4;
+    __shared__ __attribute__((aligned(16))) float sS[2][16][P];            // the state in front of the chunk, column by column
+    __shared__ floatx4_t sO[2][2][MV_WAVE];                                // half of an output tile
+    __shared__ int part[8];
+    const int seq = blockIdx.x, head = blockIdx.y, v0 = blockIdx.z * 16, H = A.H, DV = A.DV;
+    const int begin = A.cu_seqlens[seq], len = A.cu_seqlens[seq + 1] - begin;
+    if (len < DC_LINE) return;
+    const int tid = threadIdx.x, lane = tid % MV_WAVE, wave = tid / MV_WAVE, i = lane % 16, g = lane / 16;
+    int before = 0;                                                        // chunks in front of the request's
+    for (int s = tid; s < seq; s += 256) {
+        const int l = A.cu_seqlens[s + 1] - A.cu_seqlens[s];
+        if (tid < 256 && l >= DC_LINE) before += (l + DC_TOKENS - 1) / DC_TOKENS;
+    }
+#pragma unroll
+    for (int o = MV_WAVE / 2; o > 0; o >>= 1) before += __shfl_xor(before, o, MV_WAVE);
+    if (lane == 0 && wave < 4) part[wave] = before;
+    __syncthreads();
+    const size_t c0 = part[0] + part[1] + part[2] + part[3];
+    const int chunks = (len + DC_TOKENS - 1) / DC_TOKENS;
+    const int v = v0 + i;
+    const bool live = v < DV;
+    const int vc = live ? v : 0;
+    const size_t step = (size_t)H;                                          // (chunk, head) units from chunk to chunk
+    const size_t unit0 = c0 * H + head;
+
+    if (wave < KT) {
+        float* st = state + (((size_t)state_slots[seq] * H + head) * DV + vc) * DK + 16 * wave + 4 * g;
+        float4 s = *reinterpret_cast<const float4*>(st);
+        if (!live) s = float4{0.f, 0.f, 0.f, 0.f};
+        *reinterpret_cast<float4*>(&sS[0][i][16 * wave + 4 * g]) = s;
+        float4 m[DEPTH][READ ? KT : 1], nn[DEPTH];
+        float decay[DEPTH];
+        auto fetch = [&](int d, int c) {
+            const size_t unit = unit0 + (size_t)(c < chunks ? c : chunks - 1) * step;
+            if constexpr (READ) {
+                const float* p = A.M + (unit * DK + 16 * wave + i) * DK + 4 * g;
+#pragma unroll
+                for (int k = 0; k < KT; ++k) m[d][k] = *reinterpret_cast<const float4*>(p + 16 * k);
+            } else {
+                decay[d] = A.M[unit];
+            }
+            nn[d] = *reinterpret_cast<const float4*>(A.N + (unit * DV + vc) * DK + 16 * wave + 4 * g);
+        };
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) fetch(d, d);
+        __syncthreads();
+        for (int b = 0; b < chunks; b += DEPTH) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) {
+                const int c = b + d;
+                floatx4_t acc{nn[d].x, nn[d].y, nn[d].z, nn[d].w}, acc2{0.f, 0.f, 0.f, 0.f};
+                if constexpr (READ) {
+#pragma unroll
+                    for (int k = 0; k < KT; k += 2) {
+                        mfma4(acc, m[d][k], *reinterpret_cast<const float4*>(&sS[d % 2][i][16 * k + 4 * g]));
+                        mfma4(acc2, m[d][k + 1], *reinterpret_cast<const float4*>(&sS[d % 2][i][16 * (k + 1) + 4 * g]));
+                    }
+                    acc += acc2;
+                } else {
+                    acc[0] = fmaf(decay[d], s.x, acc[0]);
+                    acc[1] = fmaf(decay[d], s.y, acc[1]);
+                    acc[2] = fmaf(decay[d], s.z, acc[2]);
+                    acc[3] = fmaf(decay[d], s.w, acc[3]);
+                }
+                const bool moves = live && c < chunks;
+                s = float4{moves ? acc[0] : s.x, moves ? acc[1] : s.y, moves ? acc[2] : s.z, moves ? acc[3] : s.w};
+                *reinterpret_cast<float4*>(&sS[(d + 1) % 2][i][16 * wave + 4 * g]) = s;
+                fetch(d, c + DEPTH);
+                __syncthreads();
+            }
+        }
+        if (live) *reinterpret_cast<float4*>(st) = s;
+        __syncthreads();
+    } else {
+        const int tile = (wave - KT) % 2, half = (wave - KT) / 2;           // 16 tokens, half of the key channels
+        float4 qv[DEPTH][KT / 2];
+        float ov[DEPTH][4];
+        auto fetch = [&](int d, int c) {
+            const int first = begin + (c < chunks ? c : chunks - 1) * DC_TOKENS + 16 * tile, last = begin + len - 1;
+            const float* p = A.Q + ((size_t)min(first + i, last) * H + head) * DK + half * (DK / 2) + 4 * g;
+#pragma unroll
+            for (int k = 0; k < KT / 2; ++k) qv[d][k] = *reinterpret_cast<const float4*>(p + 16 * k);
+            // (both halves ask for the rows: a load that some path leaves out makes every wait behind it one for all loads)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) ov[d][q] = A.out[((size_t)min(first + 4 * g + q, last) * H + head) * DV + vc];
+        };
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) fetch(d, d);
+        floatx4_t held{0.f, 0.f, 0.f, 0.f};                                 // half 0: the tile of the step before
+        auto store = [&](int c) {                                           // the tile of chunk c, its other half from LDS
+            const floatx4_t o = held + sO[c % 2][tile][lane];
+            const int first = begin + c * DC_TOKENS + 16 * tile;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (live && first + 4 * g + q < begin + len) A.out[((size_t)(first + 4 * g + q) * H + head) * DV + v] = o[q];
+        };
+        __syncthreads();
+        for (int b = 0; b < chunks; b += DEPTH) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) {
+                const int c = b + d;
+                if (half == 0 && c > 0) store(c - 1);
+                floatx4_t acc{ov[d][0], ov[d][1], ov[d][2], ov[d][3]};
+                if (half != 0) acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int k = 0; k < KT / 2; ++k)
+                    mfma4(acc, qv[d][k], *reinterpret_cast<const float4*>(&sS[d % 2][i][half * (DK / 2) + 16 * k + 4 * g]));
+                if (half == 0) held = acc;
+                else sO[d % 2][tile][lane] = acc;
+                fetch(d, c + DEPTH);
+                __syncthreads();
+            }
+        }
+        __syncthreads();
+        if (half == 0) store((chunks + DEPTH - 1) / DEPTH * DEPTH - 1);
+    }
+}
+
+extern "C" int mv_delta_chunk_tokens() { return DC_TOKENS; }
+extern "C" int mv_delta_chunk_line() { return DC_LINE; }
+// 1: heads of these sizes are served
+extern "C" int mv_delta_chunks_serve(int rule, int DK, int DV) {
+    return rule >= RULE_GENERAL && rule <= RULE_SUM && (DK == 64 || DK == 128) && DV >= 1 && DV <= DK + 16;
+}
+
+template <typename T, int DK, int RULE>
+static int launch_delta_chunks(const DeltaChunkArgs& A, float* state, const int* state_slots, int chunks, hipStream_t stream) {
+    hipLaunchKernelGGL((delta_chunk_kernel<T, DK, RULE>), dim3(chunks, A.H), dim3(DC_THREADS), 0, stream, A);
+    if (mv_check_launch("delta_chunk")) return 1;
+    hipLaunchKernelGGL((delta_chunk_walk_kernel<DK, RULE != RULE_SUM>), dim3(A.n_seqs, A.H, (A.DV + 15) / 16), dim3((DK / 16 + 4) * 64), 0,
+                       stream, A, state, state_slots);
+    return mv_check_launch("delta_chunk_walk");
+}
+
+// The requests of at least mv_delta_chunk_line() tokens; `chunks`: an upper bound of their chunks (the rest of the grid
+// ends at once). M [chunks][H][DK][DK] (RULE_SUM: [chunks][H]), N [chunks][H][DV][DK] and Q [n][H][DK] are scratch.
+extern "C" int mv_delta_chunks(int rule, const float* vec, const float* gates, const float* decay, long ldz, const void* vals, long ldv,
+                               float* state, const int* cu_seqlens, const int* state_slots, int n_seqs, int n, int H, int G, int DK, int DV,
+                               int chunks, float* M, float* N, float* Q, float* out, int dtype, hipStream_t stream) {
+    MV_REQUIRE(n >= 0 && n_seqs >= 0 && H > 0 && G > 0 && H % G == 0 && chunks >= 0, "delta_chunks: bad sizes n=%d seqs=%d H=%d G=%d", n, n_seqs, H, G);
+    MV_REQUIRE(mv_delta_chunks_serve(rule, DK, DV), "delta_chunks: rule %d with heads of %d x %d is not served", rule, DK, DV);
+    MV_REQUIRE(vec && vals && state && cu_seqlens && state_slots && M && N && Q && out, "delta_chunks: missing operand");
+    MV_REQUIRE(rule != RULE_GENERAL || (G == H && DV == DK && ldv >= 3L * H * DK && mv_valid_dtype(dtype)), "delta_chunks: rows do not hold r, k and v");
+    MV_REQUIRE(rule == RULE_GENERAL || gates, "delta_chunks: missing gates");
+    MV_REQUIRE(rule != RULE_CHANNEL || (decay && ldz >= (long)H * DK && ldz % 4 == 0 && (uintptr_t)decay % 16 == 0), "delta_chunks: decays do not fit");
+    MV_REQUIRE((uintptr_t)vec % 16 == 0 && (uintptr_t)state % 16 == 0 && (uintptr_t)M % 16 == 0 && (uintptr_t)N % 16 == 0 && (uintptr_t)Q % 16 == 0,
+               "delta_chunks: operands must be 16-byte aligned");
+    MV_REQUIRE(H <= 65535, "delta_chunks: too many heads");
+    if (n == 0 || n_seqs == 0 || chunks == 0) return 0;
+    const DeltaChunkArgs A{vec, gates, decay, ldz, vals, ldv, H, G, DV, cu_seqlens, n_seqs, M, N, Q, out};
+#define DC_LAUNCH(T, RULE)                                                                                   \
+    return DK == 64 ? launch_delta_chunks<T, 64, RULE>(A, state, state_slots, chunks, stream)               \
+                    : launch_delta_chunks<T, 128, RULE>(A, state, state_slots, chunks, stream)
+    switch (rule) {
+        case RULE_GENERAL: MV_DISPATCH_T(dtype, "delta_chunks", { DC_LAUNCH(T, RULE_GENERAL); }); break;
+        case RULE_CHANNEL: DC_LAUNCH(float, RULE_CHANNEL);
+        case RULE_GATED: DC_LAUNCH(float, RULE_GATED);
+        default: DC_LAUNCH(float, RULE_SUM);
+    }
+#undef DC_LAUNCH
+    return 0;
+}

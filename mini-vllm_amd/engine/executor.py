@@ -869,6 +869,7 @@ class Executor:
                 # ... and every cut of its size class: nothing recorded may follow this step's own lengths
                 plan.decode_only, plan.max_q_len, plan.q_lens = False, mixed_key[0], ()
                 plan.bound = (mixed_key[0], mixed_key[1])
+                plan.bound_least = max((b for b in TOKEN_BUCKETS if b < mixed_key[0]), default=0) + 1
                 ctx.q_lens = ctx.starts = ctx.host_state_slots = None
             else:
                 # ... and any number of sequences up to the bucket, of which this step may fill only some

@@ -70,6 +70,8 @@ class AttentionPlan:
     # steps recorded into a graph that serves any cut of up to (tokens, sequences): the kernels' grids
     # are then sized for the worst cut, not for ``q_lens`` (workgroups without work end at once)
     bound: Optional[tuple] = None
+    # ... whose steps hold at least this many tokens
+    bound_least: int = 1
     # for measurement: keys in the cache of the step's sequences after the step (summed), and the
     # number of (query, visible key) pairs without windows
     kv_tokens: int = 0
@@ -86,6 +88,16 @@ class AttentionPlan:
             tokens, seqs = self.bound
             return tokens // unit_tokens + seqs
         return sum(-(-ql // unit_tokens) for ql in self.q_lens)
+
+    def has_long(self, tokens: int) -> bool:
+        """Whether a sequence may bring at least so many tokens to the step."""
+        return self.bound[0] >= tokens if self.bound is not None else any(q >= tokens for q in self.q_lens)
+
+    def has_short(self, tokens: int) -> bool:
+        """Whether a sequence may bring fewer."""
+        if self.bound is not None:
+            return self.bound[1] > 1 or self.bound_least < tokens
+        return any(0 < q < tokens for q in self.q_lens)
 
     def busy_units(self, unit_tokens: int) -> int:
         """The units that hold tokens, for rules that weigh the work against the device: the count

@@ -89,9 +89,9 @@ _SIGNATURES = {
     "mv_channel_prepare": (c_int, [c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
                                    c_void_p, c_int, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                    c_void_p, c_long, c_int, c_void_p]),
-    # qk, vals, beta, decay, ldz, state, cu_seqlens, state_slots, n_seqs, n, H, G, DK, DV, out, stream
+    # qk, vals, beta, decay, ldz, state, cu_seqlens, state_slots, n_seqs, n, H, G, DK, DV, below, out, stream
     "mv_channel_scan": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
-                                c_int, c_int, c_int, c_void_p, c_void_p]),
+                                c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     # packed, ld, n, n_seqs, H, G, DK, DV, taps, b_off, low_off, ra, rg, conv_w, a_log, dt_bias, a2t, g2t, norm_w, weight_dtype,
     # conv_state, state, unit_eps, eps, token_seq, cu_seqlens, state_slots, out, ldo, dtype, stream
     "mv_channel_step": (c_int, [c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -126,8 +126,8 @@ _SIGNATURES = {
     # state_slots, out, ldo, dtype, stream
     "mv_delta_step": (c_int, [c_void_p, c_long, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                               c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_int, c_void_p]),
-    # packed, ld, coef, state, cu_seqlens, state_slots, n_seqs, n, H, D, out, dtype, stream
-    "mv_delta_scan": (c_int, [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+    # packed, ld, coef, state, cu_seqlens, state_slots, n_seqs, n, H, D, below, out, dtype, stream
+    "mv_delta_scan": (c_int, [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                               c_void_p, c_int, c_void_p]),
     # raw, packed, ld, weight, weight_dtype, n, H, D, eps, out, ldo, dtype, stream
     "mv_delta_finish": (c_int, [c_void_p, c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_int, c_float, c_void_p,
@@ -283,9 +283,16 @@ _OPTIONAL_SIGNATURES = {
     # qk, vals, gates, dtype, stream
     "mv_mlstm_prepare": (c_int, [c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_float,
                                  c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
-    # qk, vals, gates, state, cu_seqlens, state_slots, n_seqs, n, H, G, DK, DV, read, out, stream
+    # qk, vals, gates, state, cu_seqlens, state_slots, n_seqs, n, H, G, DK, DV, read, below, out, stream
     "mv_state_scan": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
-                              c_int, c_int, c_void_p, c_void_p]),
+                              c_int, c_int, c_int, c_void_p, c_void_p]),
+    "mv_delta_chunk_tokens": (c_int, []),
+    "mv_delta_chunk_line": (c_int, []),
+    "mv_delta_chunks_serve": (c_int, [c_int, c_int, c_int]),
+    # rule, vec, gates, decay, ldz, vals, ldv, state, cu_seqlens, state_slots, n_seqs, n, H, G, DK, DV, chunks, M, N, Q, out, dtype,
+    # stream
+    "mv_delta_chunks": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int,
+                                c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
     # mode, packed, ld, n, n_seqs, H, G, DK, DV, taps, conv_w, a_log, dt_bias, i_bias, f_bias, norm_w, weight_dtype, conv_state,
     # max_state, state, unit_eps, cap, denom_eps, eps, token_seq, cu_seqlens, state_slots, out, ldo, dtype, stream
     "mv_state_step": (c_int, [c_int, c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,

@@ -687,27 +687,75 @@ class Ops:
             raise KernelLibraryError(f"{what}: the state must be float32 [slots, {heads}, {dim}, {dim}]")
 
     def delta_scan(self, packed: torch.Tensor, coef: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor,
-                   state_slots: torch.Tensor, n_seqs: int, heads: int, dim: int, out: torch.Tensor) -> None:
+                   state_slots: torch.Tensor, n_seqs: int, heads: int, dim: int, out: torch.Tensor, below: int = 0) -> None:
         """The delta rule over the step's rows, request by request (rows cu_seqlens[s] .. cu_seqlens[s+1]
         of request s, state row state_slots[s]): S <- diag(w) S - (a*u)(u^T S) + k v^T, out = S^T r, with
         v from the packed rows and w, a*u, u, k, r from ``coef``. state float32 [slots, heads, dim, dim]
         holds each head's matrix column by column (state[.., j, i] = S[i][j], i the key channel); it is
-        read and left advanced. out float32 [n, heads*dim]."""
-        self._act(packed, "delta rows")
+        read and left advanced. out float32 [n, heads*dim]. ``below`` > 0: requests of at least so many tokens
+        are left alone (``delta_chunks`` takes them)."""
         n, inner = packed.shape[0], heads * dim
-        if coef.dtype != torch.float32 or tuple(coef.shape) != (n, heads, 5, dim) or not coef.is_contiguous():
-            raise KernelLibraryError(f"delta_scan: coefficients must be float32 [{n}, {heads}, 5, {dim}]")
-        if out.dtype != torch.float32 or tuple(out.shape) != (n, inner) or not out.is_contiguous():
-            raise KernelLibraryError(f"delta_scan: the output must be float32 [{n}, {inner}]")
-        self._delta_state(state, heads, dim, "delta_scan")
-        if packed.dim() != 2 or packed.stride(1) != 1 or packed.shape[1] < 3 * inner:
-            raise KernelLibraryError(f"delta_scan: rows {tuple(packed.shape)} do not hold r, k and v")
-        self._ints(n, cu_seqlens=(cu_seqlens, n_seqs + 1), state_slots=(state_slots, n_seqs))
+        self._delta_scan_operands("delta_scan", packed, coef, state, cu_seqlens, state_slots, n_seqs, heads, dim, out)
         self._note("mv_delta_scan", n * inner * packed.element_size() + self._size(coef, out)
                    + 2 * min(n_seqs, max(n, 1)) * inner * dim * 4, 8 * n * inner * dim)
         self.lib.call("mv_delta_scan", packed.data_ptr(), packed.stride(0) if n > 1 else packed.shape[1], coef.data_ptr(),
-                      state.data_ptr(), cu_seqlens.data_ptr(), state_slots.data_ptr(), n_seqs, n, heads, dim,
+                      state.data_ptr(), cu_seqlens.data_ptr(), state_slots.data_ptr(), n_seqs, n, heads, dim, int(below),
                       out.data_ptr(), self.code, self._stream())
+
+    def _delta_scan_operands(self, what: str, packed: torch.Tensor, coef: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor,
+                             state_slots: torch.Tensor, n_seqs: int, heads: int, dim: int, out: torch.Tensor) -> None:
+        self._act(packed, "delta rows")
+        n, inner = packed.shape[0], heads * dim
+        if coef.dtype != torch.float32 or tuple(coef.shape) != (n, heads, 5, dim) or not coef.is_contiguous():
+            raise KernelLibraryError(f"{what}: coefficients must be float32 [{n}, {heads}, 5, {dim}]")
+        if out.dtype != torch.float32 or tuple(out.shape) != (n, inner) or not out.is_contiguous():
+            raise KernelLibraryError(f"{what}: the output must be float32 [{n}, {inner}]")
+        self._delta_state(state, heads, dim, what)
+        if packed.dim() != 2 or packed.stride(1) != 1 or packed.shape[1] < 3 * inner:
+            raise KernelLibraryError(f"{what}: rows {tuple(packed.shape)} do not hold r, k and v")
+        self._ints(n, cu_seqlens=(cu_seqlens, n_seqs + 1), state_slots=(state_slots, n_seqs))
+
+    # ---- the recurrences with a matrix state, for requests that bring many tokens ----------------------------------
+    CHUNK_RULES = {"delta": 0, "channel": 1, "gated": 2, "sum": 3}
+
+    def delta_chunk_tokens(self) -> int:
+        """Tokens in a chunk of ``delta_chunks`` and its siblings."""
+        return int(self.lib.dll.mv_delta_chunk_tokens())
+
+    def delta_chunk_line(self) -> int:
+        """They take the requests that bring at least this many tokens."""
+        return int(self.lib.dll.mv_delta_chunk_line())
+
+    def delta_chunks_serve(self, rule: str, dk: int, dv: int) -> bool:
+        """Whether heads of these sizes are served, ``rule`` one of CHUNK_RULES (``dv`` columns, an mLSTM's normaliser among them)."""
+        return bool(self.lib.dll.mv_delta_chunks_serve(self.CHUNK_RULES[rule], dk, dv))
+
+    def _matrix_chunks(self, what: str, rule: str, vec, gates, decay, vals, ldv: int, state, cu_seqlens, state_slots, n_seqs: int, n: int,
+                       heads: int, groups: int, dk: int, dv: int, maps, sums, queries, out) -> None:
+        chunks = sums.shape[0]
+        for t, shape, name in ((maps, (chunks, heads, dk, dk) if rule != "sum" else (chunks, heads), "chunk maps"),
+                               (sums, (chunks, heads, dv, dk), "chunk sums"), (queries, (n, heads, dk), "chunk queries")):
+            _dev(t, name)
+            if t.dtype != torch.float32 or tuple(t.shape) != tuple(shape) or not t.is_contiguous():
+                raise KernelLibraryError(f"{what}: the {name} must be contiguous float32 {shape}")
+        C = self.delta_chunk_tokens()
+        size = self._size(vec, out) + 2 * self._size(maps, sums, queries) + n * heads * dv * 4 + 2 * min(n_seqs, max(n, 1)) * heads * dv * dk * 4
+        self._note("mv_delta_chunks", size, n * heads * (2 * C * (2 * dk + dv) + 2 * dk * (dk + dv) * (2 if rule != "sum" else 1)))
+        self.lib.call("mv_delta_chunks", self.CHUNK_RULES[rule], vec.data_ptr(), _ptr(gates), _ptr(decay),
+                      0 if decay is None else (decay.stride(0) if n > 1 else decay.shape[1]), vals.data_ptr(), int(ldv), state.data_ptr(),
+                      cu_seqlens.data_ptr(), state_slots.data_ptr(), n_seqs, n, heads, groups, dk, dv, chunks, maps.data_ptr(),
+                      sums.data_ptr(), queries.data_ptr(), out.data_ptr(), self.code, self._stream())
+
+    def delta_chunks(self, packed: torch.Tensor, coef: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor,
+                     state_slots: torch.Tensor, n_seqs: int, heads: int, dim: int, maps: torch.Tensor, sums: torch.Tensor,
+                     queries: torch.Tensor, out: torch.Tensor) -> None:
+        """``delta_scan`` for the requests of at least ``delta_chunk_line`` tokens, as products over chunks of
+        ``delta_chunk_tokens``. Scratch, float32: maps [chunks, heads, dim, dim], sums the same, queries [n, heads, dim],
+        ``chunks`` at least the requests' chunks."""
+        self._delta_scan_operands("delta_chunks", packed, coef, state, cu_seqlens, state_slots, n_seqs, heads, dim, out)
+        n = packed.shape[0]
+        self._matrix_chunks("delta_chunks", "delta", coef, None, None, packed, packed.stride(0) if n > 1 else packed.shape[1], state,
+                            cu_seqlens, state_slots, n_seqs, n, heads, heads, dim, dim, maps, sums, queries, out)
 
     def delta_step(self, packed: torch.Tensor, heads: int, dim: int, rank: int, w2t: torch.Tensor, w0: torch.Tensor,
                    a_bias: torch.Tensor, norm_weight: torch.Tensor, decay_rate: float, key_eps: float, eps: float,
@@ -816,22 +864,39 @@ class Ops:
 
     def state_scan(self, qk: torch.Tensor, vals: torch.Tensor, gates: torch.Tensor, state: torch.Tensor,
                    cu_seqlens: torch.Tensor, state_slots: torch.Tensor, n_seqs: int, heads: int, groups: int, dk: int,
-                   dvs: int, read: bool, out: torch.Tensor) -> None:
+                   dvs: int, read: bool, out: torch.Tensor, below: int = 0) -> None:
         """Per request and head, token by token: S <- a S; u = b (v - [read] S^T k); S <- S + k u^T; out = S^T q, with
         (a, b) = gates[..., :2]. state float32 [slots, heads, dvs, dk] (a head's matrix column by column) is read and
-        left advanced; out float32 [n, heads, dvs]."""
+        left advanced; out float32 [n, heads, dvs]. ``below`` > 0: requests of at least so many tokens are left alone
+        (``state_chunks`` takes them)."""
         n = vals.shape[0]
-        self._state_vectors(n, heads, groups, dk, dvs, qk, vals, gates, "state_scan")
-        _dev(state, "matrix state"); _dev(out, "scan output")
-        if state.dtype != torch.float32 or state.dim() != 4 or tuple(state.shape[1:]) != (heads, dvs, dk) or not state.is_contiguous():
-            raise KernelLibraryError(f"state_scan: the state must be float32 [slots, {heads}, {dvs}, {dk}]")
-        if out.dtype != torch.float32 or tuple(out.shape) != (n, heads, dvs) or not out.is_contiguous():
-            raise KernelLibraryError(f"state_scan: the output must be float32 [{n}, {heads}, {dvs}]")
-        self._ints(n, cu_seqlens=(cu_seqlens, n_seqs + 1), state_slots=(state_slots, n_seqs))
+        self._state_scan_operands("state_scan", qk, vals, gates, state, cu_seqlens, state_slots, n_seqs, heads, groups, dk, dvs, out)
         self._note("mv_state_scan", self._size(qk, vals, gates, out) + 2 * min(n_seqs, max(n, 1)) * heads * dvs * dk * 4,
                    (6 if read else 4) * n * heads * dvs * dk)
         self.lib.call("mv_state_scan", qk.data_ptr(), vals.data_ptr(), gates.data_ptr(), state.data_ptr(), cu_seqlens.data_ptr(),
-                      state_slots.data_ptr(), n_seqs, n, heads, groups, dk, dvs, int(bool(read)), out.data_ptr(), self._stream())
+                      state_slots.data_ptr(), n_seqs, n, heads, groups, dk, dvs, int(bool(read)), int(below), out.data_ptr(),
+                      self._stream())
+
+    def _state_scan_operands(self, what: str, qk, vals, gates, state, cu_seqlens, state_slots, n_seqs: int, heads: int, groups: int, dk: int,
+                             dvs: int, out) -> None:
+        n = vals.shape[0]
+        self._state_vectors(n, heads, groups, dk, dvs, qk, vals, gates, what)
+        _dev(state, "matrix state"); _dev(out, "scan output")
+        if state.dtype != torch.float32 or state.dim() != 4 or tuple(state.shape[1:]) != (heads, dvs, dk) or not state.is_contiguous():
+            raise KernelLibraryError(f"{what}: the state must be float32 [slots, {heads}, {dvs}, {dk}]")
+        if out.dtype != torch.float32 or tuple(out.shape) != (n, heads, dvs) or not out.is_contiguous():
+            raise KernelLibraryError(f"{what}: the output must be float32 [{n}, {heads}, {dvs}]")
+        self._ints(n, cu_seqlens=(cu_seqlens, n_seqs + 1), state_slots=(state_slots, n_seqs))
+
+    def state_chunks(self, qk: torch.Tensor, vals: torch.Tensor, gates: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor,
+                     state_slots: torch.Tensor, n_seqs: int, heads: int, groups: int, dk: int, dvs: int, read: bool, maps: torch.Tensor,
+                     sums: torch.Tensor, queries: torch.Tensor, out: torch.Tensor) -> None:
+        """``state_scan`` for the requests of at least ``delta_chunk_line`` tokens, as products over chunks of
+        ``delta_chunk_tokens``; scratch as for ``delta_chunks`` (sums [chunks, heads, dvs, dk]; maps [chunks, heads] when not
+        ``read``)."""
+        self._state_scan_operands("state_chunks", qk, vals, gates, state, cu_seqlens, state_slots, n_seqs, heads, groups, dk, dvs, out)
+        self._matrix_chunks("state_chunks", "gated" if read else "sum", qk, gates, None, vals, 0, state, cu_seqlens, state_slots, n_seqs,
+                            vals.shape[0], heads, groups, dk, dvs, maps, sums, queries, out)
 
     def state_finish(self, raw: torch.Tensor, gates: Optional[torch.Tensor], packed: torch.Tensor, gate_offset: int, weight: torch.Tensor,
                      heads: int, dv: int, eps: float, token_seq: torch.Tensor, out: torch.Tensor, shared_weight: bool,
@@ -968,25 +1033,40 @@ class Ops:
 
     def channel_scan(self, qk: torch.Tensor, vals: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor, state: torch.Tensor,
                      cu_seqlens: torch.Tensor, state_slots: torch.Tensor, n_seqs: int, heads: int, groups: int, dk: int, dv: int,
-                     out: torch.Tensor) -> None:
+                     out: torch.Tensor, below: int = 0) -> None:
         """Per request and head, token by token: S <- diag(g) S; u = beta (v - S^T k); S <- S + k u^T; out = S^T q, g the
-        head's dk columns of ``decay`` (float32 rows). state float32 [slots, heads, dv, dk] is read and left advanced."""
+        head's dk columns of ``decay`` (float32 rows). state float32 [slots, heads, dv, dk] is read and left advanced.
+        ``below`` > 0: requests of at least so many tokens are left alone (``channel_chunks`` takes them)."""
+        n = vals.shape[0]
+        self._channel_scan_operands("channel_scan", qk, vals, beta, decay, state, cu_seqlens, state_slots, n_seqs, heads, groups, dk, dv, out)
+        self._note("mv_channel_scan", self._size(qk, vals, beta, out) + 4 * n * heads * dk
+                   + 2 * min(n_seqs, max(n, 1)) * heads * dv * dk * 4, 7 * n * heads * dv * dk)
+        self.lib.call("mv_channel_scan", qk.data_ptr(), vals.data_ptr(), beta.data_ptr(), decay.data_ptr(),
+                      decay.stride(0) if n > 1 else decay.shape[1], state.data_ptr(), cu_seqlens.data_ptr(), state_slots.data_ptr(),
+                      n_seqs, n, heads, groups, dk, dv, int(below), out.data_ptr(), self._stream())
+
+    def channel_chunks(self, qk: torch.Tensor, vals: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor, state: torch.Tensor,
+                       cu_seqlens: torch.Tensor, state_slots: torch.Tensor, n_seqs: int, heads: int, groups: int, dk: int, dv: int,
+                       maps: torch.Tensor, sums: torch.Tensor, queries: torch.Tensor, out: torch.Tensor) -> None:
+        """``channel_scan`` for the requests of at least ``delta_chunk_line`` tokens, as products over chunks of
+        ``delta_chunk_tokens``; scratch as for ``delta_chunks`` (sums [chunks, heads, dv, dk])."""
+        self._channel_scan_operands("channel_chunks", qk, vals, beta, decay, state, cu_seqlens, state_slots, n_seqs, heads, groups, dk, dv, out)
+        self._matrix_chunks("channel_chunks", "channel", qk, beta, decay, vals, 0, state, cu_seqlens, state_slots, n_seqs, vals.shape[0],
+                            heads, groups, dk, dv, maps, sums, queries, out)
+
+    def _channel_scan_operands(self, what: str, qk, vals, beta, decay, state, cu_seqlens, state_slots, n_seqs: int, heads: int, groups: int,
+                               dk: int, dv: int, out) -> None:
         n = vals.shape[0]
         for t, shape, name in ((qk, (n, groups, 2, dk), "queries and keys"), (vals, (n, heads, dv), "values"), (beta, (n, heads), "beta"),
                                (out, (n, heads, dv), "scan output")):
             _dev(t, name)
             if t.dtype != torch.float32 or tuple(t.shape) != shape or not t.is_contiguous():
-                raise KernelLibraryError(f"channel_scan: {name} must be contiguous float32 {shape}")
+                raise KernelLibraryError(f"{what}: {name} must be contiguous float32 {shape}")
         _dev(decay, "decays")
         if decay.dtype != torch.float32 or decay.dim() != 2 or decay.shape[0] != n or decay.shape[1] < heads * dk or decay.stride(1) != 1:
-            raise KernelLibraryError(f"channel_scan: decays must be float32 [{n}, >= {heads * dk}]")
-        self._matrix_state("channel_scan", state, heads, dv, dk)
+            raise KernelLibraryError(f"{what}: decays must be float32 [{n}, >= {heads * dk}]")
+        self._matrix_state(what, state, heads, dv, dk)
         self._ints(n, cu_seqlens=(cu_seqlens, n_seqs + 1), state_slots=(state_slots, n_seqs))
-        self._note("mv_channel_scan", self._size(qk, vals, beta, out) + 4 * n * heads * dk
-                   + 2 * min(n_seqs, max(n, 1)) * heads * dv * dk * 4, 7 * n * heads * dv * dk)
-        self.lib.call("mv_channel_scan", qk.data_ptr(), vals.data_ptr(), beta.data_ptr(), decay.data_ptr(),
-                      decay.stride(0) if n > 1 else decay.shape[1], state.data_ptr(), cu_seqlens.data_ptr(), state_slots.data_ptr(),
-                      n_seqs, n, heads, groups, dk, dv, out.data_ptr(), self._stream())
 
     def channel_step(self, packed: torch.Tensor, heads: int, groups: int, dk: int, dv: int, taps: int, b_off: int, low_off: int,
                      conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor, a2t: torch.Tensor, g2t: torch.Tensor,

@@ -50,6 +50,22 @@ from ..kernels.ops import RowSums
 from .base import Mixer, PartSpec, Runtime, TensorDecl, register_mixer
 
 
+def recurrence(rt: Runtime, ctx, rule: str, n: int, heads: int, dk: int, dv: int, raw: torch.Tensor, scan, chunks, *operands) -> None:
+    """A mixer's recurrence over the step's rows into ``raw``: requests of many tokens as products over chunks of tokens
+    (``chunks``), the others, and heads of sizes these do not take, token by token (``scan``)."""
+    ops, ws, plan = rt.ops, rt.workspace, ctx.attention_plan
+    line = ops.delta_chunk_line()
+    if plan is None or not plan.has_long(line) or not ops.delta_chunks_serve(rule, dk, dv):
+        scan(*operands, raw)
+        return
+    units = plan.units(ops.delta_chunk_tokens())
+    chunks(*operands, ws.get("mstate.chunk_maps", (units, heads) + ((dk, dk) if rule != "sum" else ()), torch.float32),
+           ws.get("mstate.chunks", (units, heads, dv, dk), torch.float32),
+           ws.get("mstate.chunk_queries", (n, heads, dk), torch.float32), raw)
+    if plan.has_short(line):
+        scan(*operands, raw, below=line)
+
+
 def _pack(tensors: Dict[str, torch.Tensor], names, hidden: int, what: str):
     dtypes = {tensors[p].dtype for p in names}
     if len(dtypes) != 1:
@@ -139,7 +155,8 @@ class GatedDelta(Mixer):
                                 ctx.state(call, "conv") if spec.conv_taps > 1 else None, spec.unit_eps, ctx.token_seq,
                                 ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, gates)
         raw = ws.get("mstate.raw", (n, H, dv), torch.float32)
-        ops.state_scan(qk, vals, gates, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv, True, raw)
+        recurrence(rt, ctx, "gated", n, H, dk, dv, raw, ops.state_scan, ops.state_chunks, qk, vals, gates, ctx.state(call), ctx.cu_seqlens,
+                   ctx.state_slots, ctx.n_seqs, H, G, dk, dv, True)
         ops.state_finish(raw, gates, packed, self.gate_offset, self.norm, H, dv, spec.out_norm_eps, ctx.token_seq, gated,
                          shared_weight=True, silu_gate=True)
         return ops.gemm(gated, self.w_o, y, defer_sum=True) or y
@@ -207,7 +224,8 @@ class MLSTM(Mixer):
         ops.mlstm_prepare(packed, H, dk, dv, self.i_bias, self.f_bias, spec.gate_cap, ctx.state(call, "max"), ctx.token_seq,
                           ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, gates)
         raw = ws.get("mstate.raw", (n, H, dv + 1), torch.float32)
-        ops.state_scan(qk, vals, gates, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, H, dk, dv + 1, False, raw)
+        recurrence(rt, ctx, "sum", n, H, dk, dv + 1, raw, ops.state_scan, ops.state_chunks, qk, vals, gates, ctx.state(call),
+                   ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, H, dk, dv + 1, False)
         ops.state_finish(raw, gates, packed, self.gate_offset, self.norm, H, dv, spec.out_norm_eps, ctx.token_seq, gated,
                          shared_weight=False, silu_gate=False, normaliser=True, denom_eps=spec.denom_eps)
         return ops.gemm(gated, self.w_o, y, defer_sum=True) or y
@@ -310,7 +328,8 @@ class ChannelDelta(Mixer):
         ops.channel_prepare(packed, H, G, dk, dv, spec.conv_taps, self.b_offset, self.conv_w, self.a_log, self.dt_bias, conv_state,
                             spec.unit_eps, ctx.token_seq, ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, beta, z)
         raw = ws.get("mstate.raw", (n, H, dv), torch.float32)
-        ops.channel_scan(qk, vals, beta, z, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv, raw)
+        recurrence(rt, ctx, "channel", n, H, dk, dv, raw, ops.channel_scan, ops.channel_chunks, qk, vals, beta, z, ctx.state(call),
+                   ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv)
         ops.state_finish(raw, None, z, H * dk, self.norm, H, dv, spec.out_norm_eps, ctx.token_seq, gated, shared_weight=True,
                          silu_gate=False)
         return ops.gemm(gated, self.w_o, y, defer_sum=True, fold=fold) or y
