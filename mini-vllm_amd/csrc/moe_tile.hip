@@ -1,0 +1,319 @@
+// A mixture's products over the chosen (token, expert) pairs only (bfloat16, MFMA; see moe.hip for what the mixture is),
+// through the LDS ring of gemm_tile.hip: the rows of a tile are pairs of one expert, gathered by the addresses their loads
+// take, so that a weight is read once for up to 128 pairs.
+//
+//   moe_pairs     lays the pairs out expert by expert (`sorted`: pair numbers, a pair is token * top + place; a shared expert
+//                 that every token uses is one more expert, its pairs n * top + token) and cuts every expert's run into tiles
+//                 of `rows` (`tile_expert`, `tile_row0`, `tile_rows`; entries behind the last hold expert -1). Identity experts
+//                 and pairs without an expert are left out. Within an expert the order of the pairs is whatever the counters
+//                 gave; no result depends on it (a row's products read only its own row).
+//   moe_tile<GATED>  act[pair] = weight[pair] * pair(x W_gate^T, x W_up^T), rounded once
+//   moe_tile      out[pair] = act[pair] W_down^T as floats
+//   moe_combine   y[token] = its places' out rows in order, the shared expert's, (identity weights) * x[token], added in float
+//
+// What bounds it: at 2,048 tokens, 32 experts of 768 x 1024 and 4 a token, the bytes (151 MB of weights) are worth 30 us, the
+// products 57; measured 70 (gate and up) + 42 (down) + 9 (moe_pairs) + 7 (combine) us a layer, where every expert for every
+// token took 167 + 175 through the library and 38 for the activation between; 1,000 tokens beside a shared expert 54 + 38 + 6 + 5
+// against 110 + 154 + 26. Eight rows: 19 + 13 + 5 + 5 against 22 + 12 + 7 + 5 (the unchosen experts' weights are not read).
+#include "gemm_ring.h"
+
+#define MT_MAX_E 1024
+
+struct PairTables {
+    int* sorted;
+    int* tile_expert;
+    int* tile_row0;
+    int* tile_rows;
+    int max_tiles;
+};
+
+// exclusive prefix sums over the workgroup's 1024 threads; scratch holds 16 ints
+__device__ __forceinline__ int mt_prefix(int v, int* scratch) {
+    const int lane = threadIdx.x % MV_WAVE, wave = threadIdx.x / MV_WAVE;
+    int incl = v;
+#pragma unroll
+    for (int o = 1; o < MV_WAVE; o <<= 1) {
+        const int t = __shfl_up(incl, o, MV_WAVE);
+        if (lane >= o) incl += t;
+    }
+    __syncthreads();
+    if (lane == MV_WAVE - 1) scratch[wave] = incl;
+    __syncthreads();
+    int before = 0;
+    for (int w = 0; w < wave; ++w) before += scratch[w];
+    return before + incl - v;
+}
+
+__global__ void __launch_bounds__(1024)
+moe_pairs_kernel(const int* __restrict__ ids, int n_pairs, int n_real, int shared_pairs, int rows, PairTables t) {
+    __shared__ int count[MT_MAX_E], cursor[MT_MAX_E], scratch[16];
+    const int tid = threadIdx.x;
+    count[tid] = tid == n_real ? shared_pairs : 0;             // (n_real < MT_MAX_E)
+    __syncthreads();
+    for (int p = tid; p < n_pairs; p += 1024) {
+        const int e = ids[p];
+        if (e >= 0 && e < n_real) atomicAdd(&count[e], 1);
+    }
+    __syncthreads();
+    const int c = count[tid], tiles = (c + rows - 1) / rows;
+    const int first = mt_prefix(c, scratch);
+    int tile = mt_prefix(tiles, scratch);
+    cursor[tid] = first;
+    for (int r = 0; r < c && tile < t.max_tiles; r += rows, ++tile) {
+        t.tile_expert[tile] = tid;
+        t.tile_row0[tile] = first + r;
+        t.tile_rows[tile] = min(rows, c - r);
+    }
+    if (tid == 1023)
+        for (; tile < t.max_tiles; ++tile) t.tile_expert[tile] = -1;
+    __syncthreads();
+    for (int p = tid; p < n_pairs; p += 1024) {
+        const int e = ids[p];
+        if (e >= 0 && e < n_real) t.sorted[atomicAdd(&cursor[e], 1)] = p;
+    }
+    for (int s = tid; s < shared_pairs; s += 1024) t.sorted[cursor[n_real] + s] = n_pairs + s;
+}
+
+struct MoeTileArgs {
+    const bf16* A;                 // GATED: the tokens' rows; else the pairs' activations
+    long lda;
+    const bf16* W;                 // GATED: [E gate blocks of F rows | E up blocks | gate of the shared expert (FS rows) | its up]
+    long ldw;                      // else: [N rows], the experts' F columns side by side, the shared expert's FS behind them
+    PairTables t;
+    const float* weights;          // GATED: of the pairs; a shared expert's weigh one
+    int top, n_pairs, n_real, F, FS, N;
+    bf16* act;                     // GATED: [pairs][ld_act]
+    float* out;                    // else: [pairs][N]
+    long ld_act;
+    int K;                         // GATED: columns of W
+    int tiles_n;
+    GatedPair pair;
+};
+
+template <int WM, int WN, bool GATED, int STAGES, int OCC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
+moe_tile_kernel(MoeTileArgs a) {
+    constexpr int BM = 32 * WM, BN = 32 * WN;
+    constexpr int ROWS = BM + BN, INSTR = ROWS / 8, REPS = INSTR / 4;
+    static_assert(INSTR % 4 == 0 && (!GATED || WN % 2 == 0) && STAGES >= 2 && STAGES <= 4 && (STAGES - 2) * REPS <= 63, "");
+    constexpr int STAGE = ROWS * 8;
+    __shared__ uint4 ring[STAGES * STAGE];
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / MV_WAVE);
+    const int lane = tid % MV_WAVE, i = lane % 16, g = lane / 16;
+    const int wm = wave / 2, wn = wave % 2;
+    // an XCD walks a run of tiles with all their columns: an expert's tiles stand side by side, so its weights go into one L2
+    const int total = gridDim.x, id = (blockIdx.x % GT_XCDS) * (total / GT_XCDS) + blockIdx.x / GT_XCDS;
+    const int tile = id / a.tiles_n, tn = id % a.tiles_n;
+    if (tile >= a.t.max_tiles) return;
+    const int expert = a.t.tile_expert[tile];
+    if (expert < 0) return;
+    const bool is_shared = expert == a.n_real;
+    const int width = is_shared ? a.FS : a.F;                  // of the expert
+    const int n_out = GATED ? width : a.N;
+    const int n0 = tn * (GATED ? BN / 2 : BN);
+    if (n0 >= n_out) return;
+    const int row0 = a.t.tile_row0[tile], count = a.t.tile_rows[tile];
+    const int n = (GATED ? a.K : width) / GT_KC;               // chunks
+
+    const int lrow = lane / 8, piece = (lane % 8) ^ lrow;
+    const char* src[REPS];
+    int slot[REPS];
+#pragma unroll
+    for (int rep = 0; rep < REPS; ++rep) {
+        const int j = wave + 4 * rep, row = 8 * j + lrow;
+        slot[rep] = j * 64;
+        if (row < BM) {
+            const int p = a.t.sorted[row0 + (row < count ? row : 0)];          // rows past the end: some pair; never stored
+            const long at = GATED ? (p < a.n_pairs ? p / a.top : p - a.n_pairs) : p;
+            src[rep] = reinterpret_cast<const char*>(a.A + at * a.lda + 8 * piece);
+        } else {
+            const int r = row - BM;
+            long w;
+            if (GATED) {
+                const int c = r < BN / 2 ? n0 + r : n0 + (r - BN / 2);
+                const long gate0 = is_shared ? 2L * a.n_real * a.F : (long)expert * a.F;
+                const long up0 = is_shared ? gate0 + a.FS : (long)(a.n_real + expert) * a.F;
+                w = ((r < BN / 2 ? gate0 : up0) + (c < width ? c : width - 1)) * a.ldw;
+            } else {
+                const int c = n0 + r;
+                w = (long)(c < a.N ? c : a.N - 1) * a.ldw + (is_shared ? (long)a.n_real * a.F : (long)expert * a.F);
+            }
+            src[rep] = reinterpret_cast<const char*>(a.W + w + 8 * piece);
+        }
+    }
+    auto fetch = [&](int c, uint4* stage) {
+#pragma unroll
+        for (int rep = 0; rep < REPS; ++rep)
+            gt_load_to_lds(src[rep] + (size_t)c * (GT_KC * sizeof(bf16)), (__attribute__((address_space(3))) void*)(stage + slot[rep]));
+    };
+    int a_off[WM], w_off[WN];
+#pragma unroll
+    for (int t = 0; t < WM; ++t) a_off[t] = (16 * (WM * wm + t) + i) * 8;
+#pragma unroll
+    for (int t = 0; t < WN; ++t) {
+        int group;
+        if (GATED) group = t < WN / 2 ? (WN / 2) * wn + t : WN + (WN / 2) * wn + (t - WN / 2);
+        else group = WN * wn + t;
+        w_off[t] = (BM + 16 * group + i) * 8;
+    }
+    const int sw0 = g ^ (i & 7), sw1 = (4 + g) ^ (i & 7);
+    floatx4_t acc[WN][WM];
+#pragma unroll
+    for (int t = 0; t < WN; ++t)
+#pragma unroll
+        for (int u = 0; u < WM; ++u) acc[t][u] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const uint4* stage) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int sw = ks ? sw1 : sw0;
+            TFrag af[WM], wf[WN];
+#pragma unroll
+            for (int u = 0; u < WM; ++u) af[u].u = stage[a_off[u] + sw];
+#pragma unroll
+            for (int t = 0; t < WN; ++t) wf[t].u = stage[w_off[t] + sw];
+#pragma unroll
+            for (int t = 0; t < WN; ++t)
+#pragma unroll
+                for (int u = 0; u < WM; ++u)
+                    acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t].v, af[u].v, acc[t][u], 0, 0, 0);
+        }
+    };
+    // the ring: see gemm_tile.hip. (The loads of `sorted` above have been waited for: addresses depend on them.)
+#pragma unroll
+    for (int k = 0; k < STAGES - 1; ++k)
+        if (k < n) fetch(k, ring + k * STAGE);
+    int st = 0, st_fetch = STAGES - 1;
+    for (int k = 0; k < n; ++k) {
+        const int later = n - k - 1 < STAGES - 2 ? n - k - 1 : STAGES - 2;
+        switch (later) {
+            case 0: GT_WAIT_VMCNT(0); break;
+            case 1: GT_WAIT_VMCNT(REPS); break;
+            default: GT_WAIT_VMCNT(2 * REPS); break;
+        }
+        __builtin_amdgcn_s_barrier();
+        if (k + STAGES - 1 < n) fetch(k + STAGES - 1, ring + st_fetch * STAGE);
+        multiply(ring + st * STAGE);
+        st = st + 1 == STAGES ? 0 : st + 1;
+        st_fetch = st_fetch + 1 == STAGES ? 0 : st_fetch + 1;
+    }
+    // lane l holds C[pair row 16 u + l%16][weight row of tile t + 4 (l/16) + 0..3]
+    constexpr int TOUT = GATED ? WN / 2 : WN;
+#pragma unroll
+    for (int u = 0; u < WM; ++u) {
+        const int row = 16 * (WM * wm + u) + i;
+        if (row >= count) continue;
+        const int p = a.t.sorted[row0 + row];
+        const float weight = !GATED || p >= a.n_pairs ? 1.f : a.weights[p];
+#pragma unroll
+        for (int t = 0; t < TOUT; ++t) {
+            const int col = n0 + 16 * ((GATED ? WN / 2 : WN) * wn + t) + 4 * g;
+            if (col >= n_out) continue;                        // (n_out is a multiple of four)
+            if constexpr (GATED) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = weight * a.pair.of(acc[t][u][e], acc[t + WN / 2][u][e]);
+                *reinterpret_cast<uint2*>(a.act + (size_t)p * a.ld_act + col) =
+                    uint2{f32x2_to_bf16x2_bits(v[0], v[1]), f32x2_to_bf16x2_bits(v[2], v[3])};
+            } else {
+                *reinterpret_cast<float4*>(a.out + (size_t)p * a.N + col) = float4{acc[t][u][0], acc[t][u][1], acc[t][u][2], acc[t][u][3]};
+            }
+        }
+    }
+}
+
+// four columns a thread (width a multiple of four, rows of x and y at addresses that four elements can be moved at)
+__global__ void __launch_bounds__(256)
+moe_pairs_combine_kernel(const float* __restrict__ out, const int* __restrict__ ids, int top, int n_pairs, int n_real, int shared,
+                         const bf16* __restrict__ x, long ldx, const float* __restrict__ dense, int ld_dense, int identity,
+                         bf16* __restrict__ y, long ldy, int width) {
+    const int t = blockIdx.x;
+    float idw = 0.f;
+    for (int e = 0; e < identity; ++e) idw += dense[(size_t)t * ld_dense + n_real + e];
+    for (int c = threadIdx.x * 4; c < width; c += 1024) {
+        float4 v{0.f, 0.f, 0.f, 0.f};
+        auto add = [&](size_t pair) {
+            const float4 o = *reinterpret_cast<const float4*>(out + pair * width + c);
+            v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w;
+        };
+        for (int k = 0; k < top; ++k) {
+            const int e = ids[(size_t)t * top + k];
+            if (e >= 0 && e < n_real) add((size_t)t * top + k);
+        }
+        if (shared) add((size_t)n_pairs + t);
+        if (idw != 0.f) {
+            const uint2 u = *reinterpret_cast<const uint2*>(x + (size_t)t * ldx + c);
+            v.x = fmaf(idw, __uint_as_float(u.x << 16), v.x);
+            v.y = fmaf(idw, __uint_as_float(u.x & 0xffff0000u), v.y);
+            v.z = fmaf(idw, __uint_as_float(u.y << 16), v.z);
+            v.w = fmaf(idw, __uint_as_float(u.y & 0xffff0000u), v.w);
+        }
+        *reinterpret_cast<uint2*>(y + (size_t)t * ldy + c) = uint2{f32x2_to_bf16x2_bits(v.x, v.y), f32x2_to_bf16x2_bits(v.z, v.w)};
+    }
+}
+
+template <bool GATED>
+static int launch_moe_tiles(MoeTileArgs& a, int wm, int wn, hipStream_t stream) {
+    const int n_out = GATED ? (a.F > a.FS ? a.F : a.FS) : a.N, bn = (GATED ? 16 : 32) * wn;
+    a.tiles_n = (n_out + bn - 1) / bn;
+    const long blocks = ((long)a.t.max_tiles * a.tiles_n + GT_XCDS - 1) / GT_XCDS * GT_XCDS;
+    MV_REQUIRE(blocks < (1L << 31), "moe_tile: too many tiles");
+#define MT_LAUNCH(WM, WN, STAGES, OCC) \
+    hipLaunchKernelGGL((moe_tile_kernel<WM, WN, GATED, STAGES, OCC>), dim3((unsigned)blocks), dim3(256), 0, stream, a)
+    if (wm == 1 && wn == 2) MT_LAUNCH(1, 2, 4, 2);
+    else if (wm == 1) MT_LAUNCH(1, 4, 4, 2);
+    else if (wm == 2) MT_LAUNCH(2, 4, 3, 2);
+    else MT_LAUNCH(4, 4, 2, 2);
+#undef MT_LAUNCH
+    return mv_check_launch("moe_tile");
+}
+
+// ints of scratch: sorted pairs and the three tile tables, for tiles of 32 rows
+extern "C" long mv_moe_pairs_ints(int n, int top, int n_real, int shared) {
+    const long pairs = (long)n * (top + (shared ? 1 : 0));
+    return pairs + 3L * (pairs / 32 + n_real + 2);
+}
+
+// y[t] = sum over t's chosen experts of weight * down_e(pair(gate_e x, up_e x)) + the shared expert's (FS > 0) + (identity weights) * x[t].
+// act: bf16 [pairs][max(F, FS)], out: float [pairs][hidden] with pairs = n * top, and n more with a shared expert.
+// Returns 2 (nothing done) for sizes it does not serve.
+extern "C" int mv_moe_pairs(const void* x, long ldx, int n, int hidden, const void* w_gate_up, const void* w_down, int n_real,
+                            int identity, int F, int FS, const int* ids, const float* weights, int top, const float* dense, int ld_dense,
+                            int* ints, void* act, float* out, void* y, long ldy, float limit, float slope, hipStream_t stream) {
+    MV_REQUIRE(n >= 0 && hidden > 0 && n_real > 0 && F > 0 && FS >= 0 && top > 0 && identity >= 0 && limit >= 0.f, "moe_pairs: bad sizes");
+    if (hidden % GT_KC || F % GT_KC || FS % GT_KC || ldx % 8 || ldy % 4 || (uintptr_t)x % 16 || (uintptr_t)y % 8 || (uintptr_t)w_gate_up % 16
+        || (uintptr_t)w_down % 16 || (uintptr_t)act % 16 || (uintptr_t)out % 16 || n_real >= MT_MAX_E)
+        return 2;
+    MV_REQUIRE(x && w_gate_up && w_down && ids && weights && ints && act && out && y && ldx >= hidden && ldy >= hidden
+               && (identity == 0 || (dense && ld_dense >= n_real + identity)), "moe_pairs: missing operand");
+    if (n == 0) return 0;
+    const long n_pairs = (long)n * top, pairs = n_pairs + (FS ? n : 0);
+    MV_REQUIRE(pairs < (1L << 30), "moe_pairs: too many pairs");
+    // rows of a tile: about what an expert has on average, since a tile that is mostly empty costs its products all the same
+    // and one that is too low reads its weights twice
+    const long mean = n_pairs / n_real;
+    const int wm = mean > 48 ? 4 : mean > 24 ? 2 : 1, rows = 32 * wm;
+    PairTables t;
+    t.max_tiles = (int)(pairs / rows + (n_real < n_pairs ? n_real : n_pairs) + 1);
+    t.sorted = ints;
+    t.tile_expert = ints + pairs;
+    t.tile_row0 = t.tile_expert + t.max_tiles;
+    t.tile_rows = t.tile_row0 + t.max_tiles;
+    hipLaunchKernelGGL(moe_pairs_kernel, dim3(1), dim3(1024), 0, stream, ids, (int)n_pairs, n_real, FS ? n : 0, rows, t);
+    if (mv_check_launch("moe_pairs")) return 1;
+    // columns of a tile: half as many where a step's few tiles leave compute units idle
+    const int units = mv_compute_units();
+    MoeTileArgs a{(const bf16*)x, ldx, (const bf16*)w_gate_up, (long)hidden, t, weights, top, (int)n_pairs, n_real, F, FS, hidden,
+                  (bf16*)act, out, (long)(F > FS ? F : FS), hidden, 0, GatedPair{limit, slope}};
+    const long busy = n_pairs < n_real ? n_pairs : n_real;                     // tiles, at most, of a step of few rows
+    if (launch_moe_tiles<true>(a, wm, wm == 1 && busy * ((F + 63) / 64) < units ? 2 : 4, stream)) return 1;
+    a.A = (const bf16*)act;
+    a.lda = a.ld_act;
+    a.W = (const bf16*)w_down;
+    a.ldw = (long)n_real * F + FS;
+    if (launch_moe_tiles<false>(a, wm, wm == 1 && busy * ((hidden + 127) / 128) < units ? 2 : 4, stream)) return 1;
+    hipLaunchKernelGGL(moe_pairs_combine_kernel, dim3(n), dim3(256), 0, stream, out, ids, top, (int)n_pairs, n_real, FS ? 1 : 0, (const bf16*)x,
+                       ldx, dense, ld_dense, identity, (bf16*)y, ldy, hidden);
+    return mv_check_launch("moe_pairs_combine");
+}

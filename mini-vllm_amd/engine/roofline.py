@@ -77,6 +77,7 @@ KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_group_norm_rows": (r"\bgroup_norm_rows_kernel", None, 1),
     "mv_group_norm_add_norm": (r"\bgroup_norm_add_norm(_vec)?_kernel", None, 1),
     "mv_xielu": (r"\bxielu(_vec)?_kernel", None, 1),
+    "mv_moe_pairs": (r"\bmoe_pairs_kernel", r"\bmoe_(tile|pairs_combine)_kernel", 4),
     "mv_moe_grouped": (r"\bmoe_sort_kernel", r"\bmoe_(expert_product|combine)_kernel", 4),
     "mv_hyper_step": (r"\bhyper_step(_vec)?_kernel", None, 1),
     "mv_qkv_rotate_norm_store": (r"\bqkv_rotate_norm_store(_vec)?_kernel", r"\bstore_v_pages_kernel", 2),

@@ -203,6 +203,11 @@ _OPTIONAL_SIGNATURES = {
     # limit, slope, stream
     "mv_moe_grouped": (c_int, [c_void_p, c_long, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int,
                                c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_float, c_float, c_void_p]),
+    "mv_moe_pairs_ints": (c_long, [c_int, c_int, c_int, c_int]),
+    # x, ldx, n, hidden, w_gate_up, w_down, n_real, identity, F, FS, ids, weights, top, dense, ld_dense, ints, act, out, y, ldy,
+    # limit, slope, stream
+    "mv_moe_pairs": (c_int, [c_void_p, c_long, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int,
+                             c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_float, c_float, c_void_p]),
     "mv_gemm_skinny": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_long, c_int,
                                c_int, c_int, c_int, c_int, c_void_p]),
     # A, lda, W, bias, out, ldo, M, I, K, limit, slope, stream

@@ -1643,6 +1643,48 @@ class Ops:
                    2 * n * top * 3 * ff * hidden)
         return True
 
+    def moe_pairs(self, x: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, experts: int, identity: int, ff: int, shared: int,
+                  ids: torch.Tensor, weights: torch.Tensor, dense: Optional[torch.Tensor], ints: torch.Tensor, act: torch.Tensor,
+                  out: torch.Tensor, y: torch.Tensor, limit: float = 0.0, slope: float = 1.0) -> bool:
+        """What ``moe_grouped`` computes, for widths that are multiples of 64, every expert's pairs in tiles of up to 128 rows;
+        ``shared`` > 0: a shared expert of that width is added, its gate and up rows behind the others' in ``w_gate_up``
+        [2 * experts * ff + 2 * shared, hidden], its columns behind the others' in ``w_down`` [hidden, experts * ff + shared]. With
+        pairs = n * top (n more with a shared expert), ``act`` [pairs, max(ff, shared)] and ``out`` float32 [pairs, hidden] are scratch,
+        ``ints`` int32 of at least ``moe_pairs_ints``. ``dense`` may be None without identity experts. False when the sizes are
+        not served (nothing was done)."""
+        if self.dtype != torch.bfloat16 or not self.lib.has("mv_moe_pairs") or w_gate_up.dtype != torch.bfloat16 \
+                or w_down.dtype != torch.bfloat16:
+            return False
+        self._act(x, "feed-forward input"); self._act(y, "feed-forward output"); self._act(act, "expert activations")
+        n, hidden = x.shape
+        top = ids.shape[1]
+        pairs = n * (top + (1 if shared else 0))
+        if tuple(w_gate_up.shape) != (2 * experts * ff + 2 * shared, hidden) or tuple(w_down.shape) != (hidden, experts * ff + shared) \
+                or not w_gate_up.is_contiguous() or not w_down.is_contiguous() or x.stride(1) != 1 or y.stride(1) != 1 \
+                or tuple(y.shape) != (n, hidden) or tuple(act.shape) != (pairs, max(ff, shared)) or not act.is_contiguous() \
+                or out.dtype != torch.float32 or tuple(out.shape) != (pairs, hidden) or not out.is_contiguous() \
+                or ids.dtype != torch.int32 or tuple(ids.shape) != (n, top) or tuple(weights.shape) != (n, top) \
+                or weights.dtype != torch.float32 or not ids.is_contiguous() or not weights.is_contiguous() \
+                or (identity and (dense is None or dense.dtype != torch.float32 or dense.shape[0] != n
+                                  or dense.shape[1] < experts + identity or dense.stride(1) != 1)) \
+                or ints.dtype != torch.int32 or ints.numel() < self.moe_pairs_ints(n, top, experts, shared):
+            raise KernelLibraryError("moe_pairs: operands do not fit")
+        for t in (w_gate_up, w_down, ids, weights, ints, out) + (() if dense is None else (dense,)):
+            _dev(t, "moe_pairs operand")
+        if not self.lib.offer("mv_moe_pairs", x.data_ptr(), x.stride(0) if n > 1 else hidden, n, hidden, w_gate_up.data_ptr(),
+                              w_down.data_ptr(), experts, identity, ff, shared, ids.data_ptr(), weights.data_ptr(), top, _ptr(dense),
+                              0 if dense is None else (dense.stride(0) if n > 1 else dense.shape[1]), ints.data_ptr(), act.data_ptr(),
+                              out.data_ptr(), y.data_ptr(), y.stride(0) if n > 1 else hidden, float(limit), float(slope), self._stream()):
+            return False
+        used = min(experts, n * top)
+        self._note("mv_moe_pairs", self._size(x, y) + (used * ff + shared) * 3 * hidden * 2 + self._size(act, out) * 2,
+                   2 * n * (top * ff + shared) * 3 * hidden)
+        return True
+
+    def moe_pairs_ints(self, n: int, top: int, experts: int, shared: int) -> int:
+        """Integers of scratch that ``moe_pairs`` takes."""
+        return int(self.lib.dll.mv_moe_pairs_ints(n, top, experts, int(bool(shared))))
+
     def hyper_step(self, lanes: torch.Tensor, out: Optional[torch.Tensor] = None, first: Optional[torch.Tensor] = None,
                    write=None, read=None, total: Optional[torch.Tensor] = None) -> None:
         """Several residual streams, float32 ``lanes`` [S, n, W]. ``write`` = (y [n, W] of the activation type, mix float32

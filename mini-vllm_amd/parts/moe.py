@@ -9,21 +9,17 @@ largest (outputs of other groups cannot be chosen whatever their number). The we
 experts' scores divided by their sum (+ weight_sum_eps); the result is the weighted sum of the
 chosen experts' outputs.
 
-How it runs: gate and up matrices of all experts form one packed product and all down matrices one
-second product; between them one kernel applies SiLU, the up factor and the router's weight (zero
-for experts that were not chosen) before the single rounding, so the second product sums exactly the
-chosen experts. That is exact, replays from graphs and runs at the library product's rate, but computes
-every expert: eight times the useful multiply-adds when a token uses an eighth of the experts, and every
-expert's bytes in a decode step. With ``grouped`` (bfloat16, widths that are multiples of 32) the chosen
-(token, expert) pairs are instead sorted by expert on the device, every expert's pairs are cut into tiles
-of 64 rows, and two MFMA kernels compute gate/up with the weighted activation and the down product for
-those tiles only; a last kernel sums a token's pairs in the order of choice and adds the identity experts'
-share. Its plain MFMA kernels (operands straight from memory) win where bytes decide, steps of few rows
-against large experts (8B-sized layers, 32 experts, 4 a token: a step of one request 8.8 against 13.1 ms,
-of eight 12.2 against 13.4), and lose or draw elsewhere (0.6B-sized layers at eight requests 3.0 against
-2.4 ms; a prompt of 2,048 tokens 440 against 465 us a layer at 0.6B sizes, but 186 against 151 ms for the
-whole prompt at 8B sizes), so the spec's thresholds send only the former there. Either way everything is decided on the device;
-nothing about a step's routing reaches the host, so steps replay from graphs.
+How it runs: in bfloat16, with widths that are multiples of 64, the chosen (token, expert) pairs are sorted by expert on the
+device, every expert's pairs are cut into tiles of up to 128 rows, and two MFMA kernels compute gate/up with the weighted
+activation and the down product for those tiles only; a last kernel sums a token's pairs in the order of choice and adds
+the identity experts' share (csrc/moe_tile.hip). Otherwise gate and up matrices of all experts form one packed product and
+all down matrices one second product; between them one kernel applies SiLU, the up factor and the router's weight (zero
+for experts that were not chosen) before the single rounding, so the second product sums exactly the chosen experts.
+That is exact and replays from graphs, but computes every expert: eight times the useful multiply-adds when a token uses an
+eighth of the experts, and every expert's bytes in a decode step. Widths that are odd multiples of 32 may take the pairs
+through plain MFMA kernels instead (``grouped``; operands straight from memory): only in steps of few rows against large
+experts, as the spec's thresholds say, where bytes decide. Either way everything is decided on the device; nothing about
+a step's routing reaches the host, so steps replay from graphs.
 
 Options of the spec, each with the default that gives the above: ``scoring`` "sigmoid" scores every router
 output by sigmoid(z) on its own; ``group_worth`` "top2" ranks a group by the sum of its two largest choices
@@ -33,9 +29,10 @@ g * sigmoid(gate_slope * g) * (u + 1).
 
 ``router`` "table": there is no router. A stored integer table [``table_rows``, ``top``] names the experts of every
 token id (the step's ``ctx.token_ids``), each with the weight 1 / top; with all experts at once the activation kernel
-looks the weights up itself, the chosen-pairs path gets the usual lists from ``moe_table_route``. ``shared_size`` > 0:
+looks the weights up itself, the chosen-pairs paths get the usual lists from ``moe_table_route``. ``shared_size`` > 0:
 a shared expert (a gated pair like the others) runs for every token and is added: its rows ride in the two packed
-products, or, where steps may take the chosen pairs only, it keeps two products of its own.
+products (and are one more expert of the tiled pairs), or, where steps may take the plain chosen-pairs kernels, it keeps two
+products of its own.
 """
 from __future__ import annotations
 
@@ -156,6 +153,23 @@ class RoutedExperts(FeedForward):
         return (spec.grouped and n * spec.top < spec.grouped_max_rows * spec.num_experts
                 and spec.expert_size * spec.hidden_size >= spec.grouped_min_weight)
 
+    def wants_pairs(self) -> bool:
+        """Whether the tiled products over the chosen pairs take these experts."""
+        spec, FS = self.spec, self.spec.shared_size if self.shared_packed else 0
+        return (spec.grouped and self.rt.ops.use_fast_kernels and self.rt.dtype == torch.bfloat16
+                and not (spec.hidden_size % 64 or spec.expert_size % 64 or FS % 64) and self.w_gate_up.dtype == torch.bfloat16)
+
+    def _pairs(self, x: torch.Tensor, dense, ids, weights, y) -> bool:
+        """The chosen (token, expert) pairs only, a packed shared expert among them. False: the sizes are not served."""
+        spec, rt, ops, ws = self.spec, self.rt, self.rt.ops, self.rt.workspace
+        n, n_e, F, FS = x.shape[0], spec.num_experts, spec.expert_size, spec.shared_size if self.shared_packed else 0
+        pairs = n * (spec.top + (1 if FS else 0))
+        return ops.lib.has("mv_moe_pairs") and ops.moe_pairs(
+            x, self.w_gate_up, self.w_down, n_e, spec.identity_experts, F, FS, ids, weights, dense,
+            ws.get("moe.ints", (ops.moe_pairs_ints(n, spec.top, n_e, FS),), torch.int32),
+            ws.get("moe.pair_act", (pairs, max(F, FS)), rt.dtype), ws.get("moe.pair_out", (pairs, spec.hidden_size), torch.float32), y,
+            limit=spec.limit if spec.activation == "clamped" else 0.0, slope=spec.gate_slope)
+
     def _grouped(self, x: torch.Tensor, ctx, dense, ids, weights, y) -> bool:
         """The chosen (token, expert) pairs only: sorted by expert on the device, tiles of 64 rows through MFMA.
         False: the sizes are not served."""
@@ -194,8 +208,9 @@ class RoutedExperts(FeedForward):
         ids = ws.get("moe.ids", (n, spec.top), torch.int32)
         weights = ws.get("moe.weights", (n, spec.top), torch.float32)
         by_table = spec.router == "table"
+        pairs = bool(n_e) and self.wants_pairs()
         grouped = bool(n_e) and ops.use_fast_kernels and self.wants_grouped(n)
-        if by_table and grouped:
+        if by_table and (pairs or grouped):
             ops.moe_table_route(ctx.token_ids, self.table, n_e, dense, ids, weights)
         elif by_table:
             pass                  # all experts at once: the activation kernel looks the weights up itself
@@ -205,12 +220,11 @@ class RoutedExperts(FeedForward):
             ops.moe_route(logits, self.correction, spec.groups, spec.keep_groups, spec.top, spec.weight_sum_eps, dense, ids, weights,
                           scoring=spec.scoring, group_worth=spec.group_worth, normalize=spec.normalize)
         y = ws.get("ffn.out", (n, spec.hidden_size), rt.dtype)
-        if grouped and self._grouped(x, ctx, dense, ids, weights, y):
+        # (sizes that are not served after all: the kernel below takes the dense weights or the table)
+        if (pairs and self._pairs(x, dense, ids, weights, y)) or (grouped and self._grouped(x, ctx, dense, ids, weights, y)):
             if apart:
                 self._add_shared(x, y)
             return y
-        if grouped and by_table:
-            grouped = False       # the sizes were not served after all: the lists are there, the kernel below takes the table
         if n_e:
             gu = ws.get("moe.gate_up", (n, 2 * n_e * F + 2 * FS), rt.dtype)
             ops.gemm(x, self.w_gate_up, gu)
