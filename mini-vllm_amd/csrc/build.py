@@ -33,7 +33,7 @@ COMMON_SOURCES = ["runtime.hip", "elementwise.hip", "gemm_ref.hip", "attention_r
 VARIANT_SOURCES: Dict[str, List[str]] = {
     "f32": COMMON_SOURCES,
     "bf16": COMMON_SOURCES + ["gemm_skinny.hip", "gemm_mid.hip", "gemm_tile.hip", "moe_tile.hip", "gemm_lt.hip", "attention_fast.hip",
-                              "attention_prefill.hip"],
+                              "attention_prefill.hip", "attention_latent_prompt.hip"],
 }
 # libraries a variant links against
 VARIANT_LIBS: Dict[str, List[str]] = {

@@ -194,6 +194,12 @@ _OPTIONAL_SIGNATURES = {
     # stream
     "mv_attention_latent_mfma": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
                                          c_void_p, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p]),
+    "mv_attention_latent_prompt_tokens": (c_int, []),
+    # q, ldq, out, ldo, pages, pages_t, block_table, bt_width, page_size, positions, token_seq, cu_seqlens, n_seqs, units, n, padding,
+    # H, R, DR, scale, window, sink, stream
+    "mv_attention_latent_prompt": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
+                                           c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p,
+                                           c_void_p]),
     # the same up to sink, then max_context, work, work_floats, stream
     "mv_attention_latent_split_mfma": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
                                                c_void_p, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p, c_int, c_void_p, c_long,

@@ -1438,8 +1438,9 @@ class Ops:
         key part] of each row's request (pages [pages, page_size, kv_rank + rot_dim]); out float32 [n, heads, kv_rank] is
         the weighted sum of the latents. With ``window`` the query at position p sees the keys from p - window on; ``sink`` float32
         [heads]: the softmax's denominator has one more term exp(sink[h]). Steps of single tokens take the kernel that deals a row's keys out over workgroups;
-        in bfloat16 other steps take the MFMA kernel where it serves the sizes (it reads the values from ``pages_t``
-        [pages, kv_rank, page_size], the latents with a page's slots side by side); everything else the general kernel."""
+        in bfloat16 other steps take an MFMA kernel where one serves the sizes (they read the values from ``pages_t``
+        [pages, kv_rank, page_size], the latents with a page's slots side by side), the one that shares key rows among neighbouring
+        tokens where a request brings several (its rows then stand at neighbouring positions); everything else the general kernel."""
         _dev(q, "latent queries"); _dev(out, "latent attention output"); self._act(pages, "latent pages")
         n, dk = q.shape[0], kv_rank + rot_dim
         if q.dtype != torch.float32 or tuple(q.shape) != (n, heads, dk) or not q.is_contiguous():
@@ -1468,8 +1469,21 @@ class Ops:
                 q, out, pages, pages_t, block_table, page_size, positions, token_seq, n, heads, kv_rank, rot_dim, scale, w, sink,
                 plan.max_context_len, kv_tokens):
             return
-        if pages_t is not None and self.use_fast_kernels and self.lib.has("mv_attention_latent_mfma") \
-                and not (plan is not None and plan.decode_only):
+        fast = pages_t is not None and self.use_fast_kernels and not (plan is not None and plan.decode_only)
+        # (a request that fills a workgroup's tokens; with less, a wave for every row is all the sharing there is)
+        unit = int(self.lib.dll.mv_attention_latent_prompt_tokens()) if self.lib.has("mv_attention_latent_prompt") else 0
+        if fast and unit and plan is not None and plan.cu_seqlens is not None and plan.has_long(unit):
+            units = plan.units(unit)
+            self._ints(n, cu_seqlens=(plan.cu_seqlens, plan.n_seqs + 1))
+            if self.lib.offer("mv_attention_latent_prompt", q.data_ptr(), heads * dk, out.data_ptr(), heads * kv_rank, pages.data_ptr(),
+                              pages_t.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size, positions.data_ptr(),
+                              token_seq.data_ptr(), plan.cu_seqlens.data_ptr(), plan.n_seqs, units, n,
+                              int(plan.bound is not None or sum(plan.q_lens) != n), heads, kv_rank, rot_dim, float(scale), w, _ptr(sink),
+                              self._stream()):
+                self._note("mv_attention_latent_prompt", self._size(q, out) + kv_tokens * (dk + kv_rank) * pages.element_size(),
+                           2 * pairs * heads * (dk + kv_rank))
+                return
+        if fast and self.lib.has("mv_attention_latent_mfma"):
             if self.lib.offer("mv_attention_latent_mfma", q.data_ptr(), heads * dk, out.data_ptr(), heads * kv_rank, pages.data_ptr(),
                               pages_t.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size, positions.data_ptr(),
                               token_seq.data_ptr(), n, heads, kv_rank, rot_dim, float(scale), w, _ptr(sink), self._stream()):
