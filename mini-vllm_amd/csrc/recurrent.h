@@ -118,3 +118,126 @@ conv_state_kernel(const T* __restrict__ packed, long ld, int C, int taps, T* __r
     }
     for (int i = 0; i < taps - 1; ++i) hist[(size_t)i * C + c] = keep[i];
 }
+
+// ---------------------------------------------------------------------------------------
+// The causal convolution and SiLU of CP_ROWS neighbouring rows by one wave, a channel a lane: a lane's filter stays in
+// registers and a row's input is read once for all the taps it falls under. The sums are those of one row alone, term by term.
+// A prompt's rows are bound by how many loads are on their way, not by their bytes: a workgroup a (row, head) took 63 us for
+// 2,048 rows of 24 heads (gated delta rule) and 8 rows by a workgroup of 128, half of them idle at 64 channels, 38 us for
+// 1,600 rows of 32 heads (channel decays); a wave for 8 rows of a head takes 18.7
+// and 23.9 us.
+// ---------------------------------------------------------------------------------------
+#define CP_ROWS 8
+
+// taps and head sizes these serve, where they give every compute unit eight waves. Fewer rows fill the chip only one a
+// workgroup; both forms, 16 heads in 16 groups, channel decays: 15.9 us one a workgroup against 16.6 at 256 rows of 64
+// channels (12,288 rows x jobs), 19.1 against 17.1 at 384, 88.2 against 38.7 at 2,048; 128 channels 25.7 against 26.3 at 384,
+// 99.3 against 55.8 at 2,048; 8 heads of 128: 17.6 against 22.8 at 512, 31.9 against 25.8 at 1,024; 4 of 256: 31.2 against
+// 37.3 at 1,024, 51.3 against 43.3 at 2,048 (with the kept inputs' kernel behind, about 5 us).
+static inline bool conv_rows_serve(int taps, int DK, int n, int jobs) {
+    return taps >= 2 && taps <= 4 && DK <= 256 && (long)n * jobs >= 8L * CP_ROWS * mv_compute_units();
+}
+
+template <int TAPS>
+struct ConvRows {
+    int first[CP_ROWS], slot[CP_ROWS];       // of a row's request: its first row of the step, its row of the kept inputs
+    bool live[CP_ROWS];
+    __device__ __forceinline__ ConvRows(const int* __restrict__ token_seq, const int* __restrict__ cu_seqlens,
+                                        const int* __restrict__ state_slots, int t0, int n) {
+#pragma unroll
+        for (int r = 0; r < CP_ROWS; ++r) {
+            // (a row that does not count is computed as if its request began far in front of it, and not stored)
+            const int seq = t0 + r < n ? token_seq[t0 + r] : -1;
+            live[r] = seq >= 0;
+            first[r] = live[r] ? cu_seqlens[seq] : -TAPS;
+            slot[r] = live[r] ? state_slots[seq] : 0;
+        }
+    }
+};
+
+// x[r] = silu(convolution) of channel c (of C) in row t0 + r
+template <typename T, int TAPS>
+__device__ __forceinline__ void conv_rows(float (&x)[CP_ROWS], const ConvRows<TAPS>& rows, const T* __restrict__ packed, long ld,
+                                          const WeightPtr& conv_w, const T* __restrict__ conv_state, int t0, int n, int C, int c) {
+    float w[TAPS], in[CP_ROWS + TAPS - 1];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) w[j] = conv_w.at((size_t)c * TAPS + j);
+#pragma unroll
+    for (int i = 0; i < CP_ROWS + TAPS - 1; ++i) in[i] = to_f(packed[(size_t)min(max(t0 - (TAPS - 1) + i, 0), n - 1) * ld + c]);
+#pragma unroll
+    for (int r = 0; r < CP_ROWS; ++r) {
+        float acc = 0.f;
+        if (t0 + r - (TAPS - 1) >= rows.first[r]) {
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) acc = fmaf(w[j], in[r + j], acc);
+        } else {
+            const T* hist = conv_state + (size_t)rows.slot[r] * (TAPS - 1) * C;
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j)
+                acc = fmaf(w[j], conv_input(packed, ld, hist, C, TAPS, rows.first[r], t0 + r - (TAPS - 1) + j, c), acc);
+        }
+        x[r] = silu_f(acc);
+    }
+}
+
+// job 2 * group: unit queries (times DK^-1/2), 2 * group + 1: unit keys, into qk [n][G][2][DK]; lane d keeps channels d, d + 64 ..
+// (UNITS of them). The squares are added up as the kernels of one row do with their 128 threads.
+template <typename T, int TAPS, int UNITS>
+__device__ __forceinline__ void conv_unit_rows(const ConvRows<TAPS>& rows, const T* __restrict__ packed, long ld, const WeightPtr& conv_w,
+                                               const T* __restrict__ conv_state, int t0, int n, int C, int G, int DK, int job, int d,
+                                               float unit_eps, float* __restrict__ qk) {
+    const int group = job / 2, which = job % 2;
+    float x[UNITS][CP_ROWS];
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+        const int c = u * MV_WAVE + d;
+        conv_rows<T, TAPS>(x[u], rows, packed, ld, conv_w, conv_state, t0, n, C, which * G * DK + group * DK + (c < DK ? c : 0));
+#pragma unroll
+        for (int r = 0; r < CP_ROWS; ++r) x[u][r] = c < DK ? x[u][r] : 0.f;
+    }
+    const float scale = which == 0 ? 1.f / sqrtf((float)DK) : 1.f;
+#pragma unroll
+    for (int r = 0; r < CP_ROWS; ++r) {
+        float even = fmaf(x[0][r], x[0][r], 0.f), odd = 0.f;         // (as there: a bare product could be fused into the sum)
+        if constexpr (UNITS >= 2) odd = fmaf(x[1][r], x[1][r], 0.f);
+        if constexpr (UNITS == 4) {
+            even = fmaf(x[2][r], x[2][r], even);
+            odd = fmaf(x[3][r], x[3][r], odd);
+        }
+        float ss = wave_sum(even);
+        if constexpr (UNITS >= 2) ss += wave_sum(odd);
+        const float inv = scale / sqrtf(ss + unit_eps);
+        float* o = qk + (((size_t)(t0 + r) * G + group) * 2 + which) * DK;
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u)
+            if (rows.live[r] && u * MV_WAVE + d < DK) o[u * MV_WAVE + d] = x[u][r] * inv;
+    }
+}
+
+// a head's values, vals [n][H][DV], from column c0 on
+template <typename T, int TAPS>
+__device__ __forceinline__ void conv_value_rows(const ConvRows<TAPS>& rows, const T* __restrict__ packed, long ld, const WeightPtr& conv_w,
+                                                const T* __restrict__ conv_state, int t0, int n, int C, int c0, int H, int DV, int head, int lane,
+                                                float* __restrict__ vals) {
+    for (int d = lane; d < DV; d += MV_WAVE) {
+        float x[CP_ROWS];
+        conv_rows<T, TAPS>(x, rows, packed, ld, conv_w, conv_state, t0, n, C, c0 + head * DV + d);
+#pragma unroll
+        for (int r = 0; r < CP_ROWS; ++r)
+            if (rows.live[r]) vals[((size_t)(t0 + r) * H + head) * DV + d] = x[r];
+    }
+}
+
+// LAUNCH(taps, units) for what conv_rows_serve accepts
+#define CONV_ROWS_DISPATCH(taps, DK, LAUNCH)                        \
+    switch ((taps) * 8 + ((DK) <= 64 ? 1 : (DK) <= 128 ? 2 : 4)) {  \
+        case 2 * 8 + 1: LAUNCH(2, 1); break;                        \
+        case 2 * 8 + 2: LAUNCH(2, 2); break;                        \
+        case 2 * 8 + 4: LAUNCH(2, 4); break;                        \
+        case 3 * 8 + 1: LAUNCH(3, 1); break;                        \
+        case 3 * 8 + 2: LAUNCH(3, 2); break;                        \
+        case 3 * 8 + 4: LAUNCH(3, 4); break;                        \
+        case 4 * 8 + 1: LAUNCH(4, 1); break;                        \
+        case 4 * 8 + 2: LAUNCH(4, 2); break;                        \
+        default: LAUNCH(4, 4);                                      \
+    }

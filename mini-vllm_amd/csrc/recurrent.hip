@@ -630,6 +630,34 @@ gdelta_prepare_kernel(const T* __restrict__ packed, long ld, int H, int G, int D
     }
 }
 
+// The same with CP_ROWS neighbouring rows a wave (2 to 4 taps): waves 0 .. 2 G - 1 of a run of
+// rows make the groups' queries and keys, the H behind them a head's values and gates.
+template <typename T, int TAPS, int UNITS>
+__global__ void __launch_bounds__(256)
+gdelta_prepare_rows_kernel(const T* __restrict__ packed, long ld, int n, int H, int G, int DK, int DV, WeightPtr conv_w,
+                           const T* __restrict__ conv_state, WeightPtr a_log, WeightPtr dt_bias, float unit_eps,
+                           const int* __restrict__ token_seq, const int* __restrict__ cu_seqlens, const int* __restrict__ state_slots,
+                           float* __restrict__ qk, float* __restrict__ vals, float* __restrict__ gates) {
+    const int t0 = blockIdx.x * CP_ROWS, job = blockIdx.y * 4 + threadIdx.x / MV_WAVE, d = threadIdx.x % MV_WAVE;
+    if (job >= 2 * G + H) return;
+    const int C = 2 * G * DK + H * DV;
+    ConvRows<TAPS> rows(token_seq, cu_seqlens, state_slots, t0, n);
+    if (job < 2 * G) {
+        conv_unit_rows<T, TAPS, UNITS>(rows, packed, ld, conv_w, conv_state, t0, n, C, G, DK, job, d, unit_eps, qk);
+        return;
+    }
+    const int head = job - 2 * G, row = t0 + d;
+    conv_value_rows<T, TAPS>(rows, packed, ld, conv_w, conv_state, t0, n, C, 2 * G * DK, H, DV, head, d, vals);
+    if (d < CP_ROWS && row < n && token_seq[row] >= 0) {
+        const T* p = packed + (size_t)row * ld + 2 * (size_t)G * DK + 2 * (size_t)H * DV;
+        float* g = gates + ((size_t)row * H + head) * 4;
+        g[0] = expf(-expf(a_log.at(head)) * softplus_f(to_f(p[H + head]) + dt_bias.at(head)));
+        g[1] = sigmoid_f(to_f(p[head]));
+        g[2] = 0.f;
+        g[3] = 0.f;
+    }
+}
+
 // A causal convolution over time added to its own input, channel by channel:
 //   out[t][c] = h[t][c] + sum_j w[c][j] * h[t - taps + 1 + j][c]      (the last tap multiplies h[t] itself)
 // Rows in front of a request's first row of the step come from its kept inputs conv_state[slot][taps-1][C]
@@ -747,10 +775,20 @@ extern "C" int mv_gdelta_prepare(const void* packed, long ld, int n, int n_seqs,
     MV_REQUIRE(unit_eps > 0.f && G + H <= 65535 && (C + 255) / 256 <= 65535, "gdelta_prepare: bad constants");
     if (n == 0) return 0;
     WeightPtr cw{conv_w, weight_dtype}, al{a_log, weight_dtype}, db{dt_bias, weight_dtype};
-    MV_DISPATCH_T(dtype, "gdelta_prepare",
-                  hipLaunchKernelGGL(gdelta_prepare_kernel<T>, dim3(n, G + H), dim3(128), 0, stream, (const T*)packed, ld, H,
-                                     G, DK, DV, taps, cw, (const T*)conv_state, al, db, unit_eps, token_seq, cu_seqlens,
-                                     state_slots, qk, vals, gates));
+    if (!conv_rows_serve(taps, DK, n, 2 * G + H)) {
+        MV_DISPATCH_T(dtype, "gdelta_prepare",
+                      hipLaunchKernelGGL(gdelta_prepare_kernel<T>, dim3(n, G + H), dim3(128), 0, stream, (const T*)packed, ld, H,
+                                         G, DK, DV, taps, cw, (const T*)conv_state, al, db, unit_eps, token_seq, cu_seqlens,
+                                         state_slots, qk, vals, gates));
+    } else {
+#define GDELTA_ROWS(TAPS, UNITS)                                                                                                      \
+    MV_DISPATCH_T(dtype, "gdelta_prepare",                                                                                           \
+                  hipLaunchKernelGGL((gdelta_prepare_rows_kernel<T, TAPS, UNITS>), dim3((n + CP_ROWS - 1) / CP_ROWS, (2 * G + H + 3) / 4), \
+                                     dim3(256), 0, stream, (const T*)packed, ld, n, H, G, DK, DV, cw, (const T*)conv_state, al, db,  \
+                                     unit_eps, token_seq, cu_seqlens, state_slots, qk, vals, gates))
+        CONV_ROWS_DISPATCH(taps, DK, GDELTA_ROWS);
+#undef GDELTA_ROWS
+    }
     if (mv_check_launch("gdelta_prepare")) return 1;
     if (taps > 1 && n_seqs > 0) {
         MV_DISPATCH_T(dtype, "conv_state",
@@ -766,38 +804,70 @@ extern "C" int mv_gdelta_prepare(const void* packed, long ld, int n, int n_seqs,
 // input gate i = cap tanh((i + i_bias) / cap), the log forget gate f = logsigmoid(cap tanh((f + f_bias) / cap))
 // and the running maximum m (kept per request and head, 0 at the start):
 //     m' = max(f + m, i);   a = exp(f + m - m');   b = exp(i - m');   gates = (a, b, exp(-m'), 0)
-// One wave per (request, head) walks the request's rows 64 at a time: the gates' functions are computed
-// a row a lane, the maximum itself in the order of the rows.
+// Workgroup (request, head). Requests of fewer than MG_LINE tokens: its first wave walks the rows 64 at a time, the gates'
+// functions a row a lane, the maximum itself in the order of the rows, so that its bits do not depend on how a request was
+// cut. Longer ones (whose recurrence is cut into chunks anyway, from the same length on): all waves take the maxima of a run
+// of rows as a prefix over the pairs (sum of f, max of i behind later f), (F, M)(F', M') = (F + F', max(M + F', M')); the
+// result holds for any maxima, a and b are made from the ones that are stored, so these may round differently. One wave took
+// 134 us for 2,048 rows of 16 heads (a chain of lane exchanges), the prefix 12.6 us.
 // ---------------------------------------------------------------------------------------
+#define MG_THREADS 1024
+#define MG_LINE 128
 template <typename T>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(MG_THREADS)
 mlstm_gates_kernel(const T* __restrict__ packed, long ld, int H, long gate_off, WeightPtr i_bias, WeightPtr f_bias, float cap,
                    float* __restrict__ max_state, const int* __restrict__ cu_seqlens, const int* __restrict__ state_slots,
                    float* __restrict__ gates) {
-    const int seq = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
+    __shared__ float sF[MG_THREADS / MV_WAVE], sM[MG_THREADS / MV_WAVE];
+    const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x, lane = tid % MV_WAVE, wave = tid / MV_WAVE;
     const int first = cu_seqlens[seq], end = cu_seqlens[seq + 1];
-    if (end <= first) return;
+    const bool wide = end - first >= MG_LINE;
+    if (end <= first || (!wide && wave > 0)) return;
     float* ms = max_state + (size_t)state_slots[seq] * H + head;
     float m = *ms;
     const float bi = i_bias.at(head), bf = f_bias.at(head);
-    for (int base = first; base < end; base += 64) {
-        const int t = base + lane;
+    for (int base = first; base < end; base += wide ? MG_THREADS : MV_WAVE) {
+        const int t = base + tid;
         const bool live = t < end;
         const T* p = packed + (size_t)(live ? t : first) * ld + gate_off;
         const float gi = __fmul_rn(cap, tanhf((to_f(p[head]) + bi) / cap));      // (rounded here: never fused into a later sum)
         const float gf = logsigmoid_f(cap * tanhf((to_f(p[H + head]) + bf) / cap));
-        // the maximum runs token by token, in the same order however the request was cut into steps: every lane
-        // walks the 64 rows (their gates come by lane broadcasts), lane j keeps the values of row j
         float m_prev = m, m_new = m;
-        const int nt = min(64, end - base);
-        for (int j = 0; j < nt; ++j) {
-            const float fj = __shfl(gf, j, 64), ij = __shfl(gi, j, 64);
-            const float next = fmaxf(fj + m, ij);
-            if (lane == j) {
-                m_prev = m;
-                m_new = next;
+        if (wide) {
+            float F = live ? gf : 0.f, M = live ? gi : -INFINITY;
+#pragma unroll
+            for (int o = 1; o < MV_WAVE; o <<= 1) {
+                const float F0 = __shfl_up(F, o, MV_WAVE), M0 = __shfl_up(M, o, MV_WAVE);
+                if (lane >= o) {
+                    M = fmaxf(M0 + F, M);
+                    F += F0;
+                }
             }
-            m = next;
+            if (lane == MV_WAVE - 1) {
+                sF[wave] = F;
+                sM[wave] = M;
+            }
+            __syncthreads();
+            float in = m;                                        // the maximum in front of the wave's rows, and behind the run
+            for (int w = 0; w < MG_THREADS / MV_WAVE; ++w) {
+                m = fmaxf(m + sF[w], sM[w]);
+                if (w < wave) in = m;
+            }
+            m_new = fmaxf(in + F, M);
+            m_prev = __shfl_up(m_new, 1, MV_WAVE);
+            if (lane == 0) m_prev = in;
+            __syncthreads();
+        } else {
+            const int nt = min(MV_WAVE, end - base);
+            for (int j = 0; j < nt; ++j) {
+                const float fj = __shfl(gf, j, 64), ij = __shfl(gi, j, 64);
+                const float next = fmaxf(fj + m, ij);
+                if (lane == j) {
+                    m_prev = m;
+                    m_new = next;
+                }
+                m = next;
+            }
         }
         if (live) {
             float* g = gates + ((size_t)t * H + head) * 4;
@@ -807,7 +877,7 @@ mlstm_gates_kernel(const T* __restrict__ packed, long ld, int H, long gate_off, 
             g[3] = 0.f;
         }
     }
-    if (lane == 0) *ms = m;
+    if (tid == 0) *ms = m;
 }
 
 // mLSTM, the vectors of the scan: q * DK^-1/2 and k as floats, the values with a one behind them.
@@ -842,7 +912,7 @@ extern "C" int mv_mlstm_prepare(const void* packed, long ld, int n, int n_seqs, 
     if (n == 0 || n_seqs == 0) return 0;
     WeightPtr ib{i_bias, weight_dtype}, fb{f_bias, weight_dtype};
     MV_DISPATCH_T(dtype, "mlstm_gates",
-                  hipLaunchKernelGGL(mlstm_gates_kernel<T>, dim3(n_seqs, H), dim3(64), 0, stream, (const T*)packed, ld, H,
+                  hipLaunchKernelGGL(mlstm_gates_kernel<T>, dim3(n_seqs, H), dim3(MG_THREADS), 0, stream, (const T*)packed, ld, H,
                                      gate_off, ib, fb, cap, max_state, cu_seqlens, state_slots, gates));
     if (mv_check_launch("mlstm_gates")) return 1;
     MV_DISPATCH_T(dtype, "mlstm_prepare",
