@@ -34,6 +34,8 @@
 // Layouts: K[page][kv_head][slot][d], V[page][kv_head][d][slot]; page size a multiple of 16.
 #include "attention_score.h"
 
+#include <type_traits>
+
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
@@ -79,7 +81,9 @@ struct SigmoidArgs {
 };
 
 // SCORED (softmax weights): capped scores, a distance bias, a sink in the denominator (see attention_score.h).
-template <int D, int NT, int KW, bool SIG = false, bool SCORED = false>
+// NARROW: units whose columns fit one tile take a walk of their own (below). Only for steps that may have such units: the
+// code beside it costs the others' walk 3 us of 43 at 2,048 tokens, though not one of its instructions is executed there.
+template <int D, int NT, int KW, bool SIG, bool SCORED, bool NARROW>
 __global__ void __launch_bounds__(AP_THREADS * KW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __restrict__ out, long out_stride,
                          const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
@@ -104,7 +108,6 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
     __shared__ uint4 stage1[KW * TILE];
     __shared__ uint4 stage2[KW * TILE];
     __shared__ uint4 stage3[KW * TILE];
-    __shared__ int sh_unit[3];
     __shared__ int sh_range[2][AP_WAVES * KW];
 
     const int G = H / Hkv;
@@ -123,36 +126,56 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
     const int g = lane / 16;
     const int tpu = COLS / G;  // tokens of a unit (the host made sure it is >= 1)
 
-    if (tid == 0) {
-        int seq = -1, t0 = 0, nt = 0;
-        // Units with the most keys start first. When the whole grid is resident at once (two
-        // workgroups a compute unit, dealt out in order), the second half of the grid runs from
-        // the lightest unit upwards instead, so that the two workgroups that share a compute unit
-        // bring about the same number of key blocks together.
+    // Units with the most keys start first. When the whole grid is resident at once (two
+    // workgroups a compute unit, dealt out in order), the second half of the grid runs from
+    // the lightest unit upwards instead, so that the two workgroups that share a compute unit
+    // bring about the same number of key blocks together.
+    // Every wave finds the unit by itself, 64 requests at a time: a walk over the requests by one thread waits for
+    // memory at each of them (2 us of a step of 20 requests).
+    int seq = -1, t0 = 0, nt = 0;
+    {
         const int n_all = gridDim.y, half = (n_all + 1) / 2;
         int u = (!fold || (int)blockIdx.y < half) ? n_all - 1 - (int)blockIdx.y : (int)blockIdx.y - half;
-        for (int s = 0; s < n_seqs; ++s) {
-            const int ql = cu_seqlens[s + 1] - cu_seqlens[s];
-            const int nu = (ql + tpu - 1) / tpu;
-            if (u < nu) {
-                seq = s;
-                t0 = cu_seqlens[s] + u * tpu;
-                nt = ql - u * tpu;
-                if (nt > tpu) nt = tpu;
+        // (a step of one prompt needs no more than its first request's two numbers)
+        const int first0 = cu_seqlens[0], len0 = cu_seqlens[1] - first0;
+        const bool in_first = u < (len0 + tpu - 1) / tpu;
+        if (in_first) {
+            seq = 0;
+            t0 = first0 + u * tpu;
+            nt = len0 - u * tpu;
+            nt = nt < tpu ? nt : tpu;
+        }
+        for (int s0 = 0; !in_first && s0 < n_seqs; s0 += MV_WAVE) {
+            const int s = s0 + lane;
+            const int first = s < n_seqs ? cu_seqlens[s] : 0, len = s < n_seqs ? cu_seqlens[s + 1] - first : 0;
+            const int mine = (len + tpu - 1) / tpu;
+            int incl = mine;
+#pragma unroll
+            for (int o = 1; o < MV_WAVE; o <<= 1) {
+                const int t = __shfl_up(incl, o, MV_WAVE);
+                if (lane >= o) incl += t;
+            }
+            const unsigned long long hit = __ballot(u < incl && u >= incl - mine);
+            if (hit != 0) {
+                const int at = __ffsll(hit) - 1;
+                const int in = u - __shfl(incl - mine, at, MV_WAVE);          // which of the request's units
+                seq = s0 + at;
+                t0 = __shfl(first, at, MV_WAVE) + in * tpu;
+                nt = __shfl(len, at, MV_WAVE) - in * tpu;
+                nt = nt < tpu ? nt : tpu;
                 break;
             }
-            u -= nu;
+            u -= __shfl(incl, MV_WAVE - 1, MV_WAVE);
         }
-        sh_unit[0] = seq;
-        sh_unit[1] = t0;
-        sh_unit[2] = nt;
     }
-    __syncthreads();
-    const int seq = __builtin_amdgcn_readfirstlane(sh_unit[0]);
-    const int t0 = __builtin_amdgcn_readfirstlane(sh_unit[1]);
-    const int nt = __builtin_amdgcn_readfirstlane(sh_unit[2]);
+    seq = __builtin_amdgcn_readfirstlane(seq);
+    t0 = __builtin_amdgcn_readfirstlane(t0);
+    nt = __builtin_amdgcn_readfirstlane(nt);
     if (seq < 0 || nt <= 0) return;
     const int ncols = nt * G;
+    // a unit whose columns fit one tile (a decoding request in a step with prompts, a prompt's last tokens)
+    static_assert(!NARROW || KW > 1 || NT == 1, "this form has no registers to spare");
+    const bool narrow = NARROW && ncols <= 16;
     const int* bt = block_table + (size_t)seq * bt_width;
 
     // ---- this lane's columns
@@ -163,7 +186,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
     int hi_w = -1, lo_w = 0x7fffffff;
 #pragma unroll
     for (int ct = 0; ct < NT; ++ct) {
-        const int col = (cw * NT + ct) * 16 + i;
+        const int col = ((narrow ? 0 : cw) * NT + ct) * 16 + i;
         col_ok[ct] = col < ncols;
         col_tok[ct] = t0 + (col_ok[ct] ? col / G : 0);
         col_head[ct] = kvh * G + (col_ok[ct] ? col % G : 0);
@@ -264,7 +287,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
         unsigned k_off[KREP], v_off[VREP];
 #pragma unroll
         for (int rep = 0; rep < KREP; ++rep) {
-            const int pair = cw + AP_WAVES * rep;   // (score tile, k-step): LDS chunks pair * 64 ...
+            const int pair = (narrow ? 0 : cw) + AP_WAVES * rep;   // (score tile, k-step): LDS chunks pair * 64 ...
             const int t = pair / DS, ks = pair % DS;
             const int slot = 8 * ((rho / 4) % 2) + 4 * t + rho % 4;    // within its half
             k_off[rep] = (unsigned)((slot * D + 32 * ks + 8 * g) * sizeof(bf16));
@@ -273,7 +296,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
         // V: lane group g holds keys 8g .. 8g+7 of d row 16*dt + rho
 #pragma unroll
         for (int rep = 0; rep < VREP; ++rep) {
-            const int dt = cw + AP_WAVES * rep;
+            const int dt = (narrow ? 0 : cw) + AP_WAVES * rep;
             v_off[rep] = (unsigned)(((16 * dt + rho) * page_size + 8 * (g % 2)) * sizeof(bf16));
             v_step[rep] = v_off[rep] - v_off[0];
         }
@@ -400,15 +423,15 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
     // The two products with the softmax between them. ask_k / ask_v: behind the score product, ask
     // for the keys of the next block (from k_next into op_next) and for this block's values (from
     // v_now into vo_w, which is `vo`). Inlined always: as a call it would keep the accumulators in memory.
-    auto compute = [&](int j, const KOps& op, const VOps& vo, const uint4* k_next, KOps& op_next, const uint4* v_now, VOps& vo_w, const bool ask_k, const bool ask_v) __attribute__((always_inline)) {
-        const int base = 32 * block_of(j);
-        const bool masked = block_of(j) > bm_hi || block_of(j) < bm_lo;
+    auto compute = [&](auto tiles, int j, const KOps& op, const VOps& vo, const uint4* k_next, KOps& op_next, const uint4* v_now, VOps& vo_w, const bool ask_k, const bool ask_v) __attribute__((always_inline)) {
+        constexpr int NC = decltype(tiles)::value;      // column tiles the wave holds
+        const int block = block_of(j), base = 32 * block;
         // scores^T for the two 16-key tiles
-        float p[NT][2][4];
+        float p[NC][2][4];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
 #pragma unroll
-            for (int ct = 0; ct < NT; ++ct) {
+            for (int ct = 0; ct < NC; ++ct) {
                 floatx4_t sacc = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int s = 0; s < DS; ++s)
@@ -425,7 +448,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (SCORED) {
 #pragma unroll
-            for (int ct = 0; ct < NT; ++ct) {
+            for (int ct = 0; ct < NC; ++ct) {
                 const float ahead = (float)(col_pos[ct] - base - 8 * g);      // how far the lane's first key lies behind
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
@@ -433,23 +456,36 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
                     for (int r = 0; r < 4; ++r) p[ct][t][r] = fmaf(-col_bias[ct], ahead - (float)(4 * t + r), scored.of(p[ct][t][r]));
             }
         }
-        if (masked) {
+        // Masks, behind branches that are the same for a wave and that the empty statements keep: as selects (what the compiler
+        // makes of a plain condition) they took 60 of a block's 250 instructions. 32 heads on 8, 32 columns a wave:
+        // 171.7 -> 147.8 us for 4,096 tokens, 109.3 -> 98.4 for 3,000; 16 heads, 8,000 tokens 332.8 -> 290.8.
+        if (block > bm_hi) {
+            asm volatile("");
 #pragma unroll
-            for (int ct = 0; ct < NT; ++ct)
+            for (int ct = 0; ct < NC; ++ct) {
+                const int hi = col_pos[ct] - base - 8 * g;       // (a column that is none: -1 and below)
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int key = base + 8 * g + 4 * t + r;
-                        const bool ok = col_ok[ct] && key <= col_pos[ct] && (key >= col_lo[ct] || key < kept_first);
-                        p[ct][t][r] = ok ? p[ct][t][r] : -INFINITY;
-                    }
+                    for (int r = 0; r < 4; ++r) p[ct][t][r] = 4 * t + r <= hi ? p[ct][t][r] : -INFINITY;
+            }
+        }
+        if (block < bm_lo) {
+            asm volatile("");
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct) {
+                const int lo = col_lo[ct] - base - 8 * g, kept = kept_first - base - 8 * g;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) p[ct][t][r] = 4 * t + r >= lo || 4 * t + r < kept ? p[ct][t][r] : -INFINITY;
+            }
         }
         // online softmax per column
-        Frag pop[NT];
+        Frag pop[NC];
         if constexpr (SIG) {
 #pragma unroll
-            for (int ct = 0; ct < NT; ++ct)
+            for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -460,7 +496,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
                     }
         } else
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
+        for (int ct = 0; ct < NC; ++ct) {
             float mx = -INFINITY;
 #pragma unroll
             for (int t = 0; t < 2; ++t)
@@ -500,9 +536,133 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int ct = 0; ct < NT; ++ct)
+            for (int ct = 0; ct < NC; ++ct)
                 acc_o[ct][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vo.vop[dt].v, pop[ct].v, acc_o[ct][dt], 0, 0, 0);
     };
+
+    const std::integral_constant<int, NT> all{};
+    // what a column's sums are multiplied by in the end
+    auto finish = [&](int ct, float m, float l) {
+        float inv = 1.f;
+        if constexpr (!SIG) {
+            if (SCORED && form.sink) {          // one more score, 0, without a value
+                const float m_fin = fmaxf(m, 0.f);
+                const float f = exp2f(m - m_fin);
+                inv = f / fmaf(f, l, exp2f(-m_fin));
+            } else {
+                inv = 1.f / l;
+            }
+        }
+        if (sig.gate != nullptr) {
+            const float z = to_f(sig.gate[(size_t)col_tok[ct] * sig.gate_stride + col_head[ct]]);
+            inv *= 1.f / (1.f + __expf(-z));
+        }
+        return inv;
+    };
+
+    // ---- a narrow unit: every wave walks blocks of its own, operands from the pages straight into registers a block ahead
+    // (each is used by this wave alone: LDS would only add a barrier to every two blocks), and the waves' sums are joined at the
+    // end. In the wide form one wave of four has columns, and a walk takes four times the rounds: 17 decoding requests of
+    // 700 keys beside three prompts, 8 kv heads, took 34.0 us a launch, 27.9 so (25.9 with the search above). What is left is
+    // the latency of five dependent loads and of the longest walk, 5 rounds a wave.
+    if constexpr (NARROW) if (narrow) {
+        constexpr int NW = AP_WAVES * KW;
+        const std::integral_constant<int, 1> one{};
+        auto load = [&](int j, const PageIds& ids, KOps& ko, VOps& vo) {
+            int b = block_of(j);
+            b = b < b1 ? b : b1;
+            const unsigned sb = (unsigned)((32 * b) & page_mask);
+            const unsigned pgk = ids.k < 0 ? 0u : (unsigned)ids.k, pgv = ids.v < 0 ? 0u : (unsigned)ids.v;
+            const char* kb = k_lane + (size_t)pgk * page_bytes + sb * (unsigned)(D * sizeof(bf16));
+            const char* vb = v_lane + (size_t)pgv * page_bytes + sb * (unsigned)sizeof(bf16);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int s = 0; s < DS; ++s) ko.kop[t][s].u = *reinterpret_cast<const uint4*>(kb + (4 * t * D + 32 * s) * sizeof(bf16));
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) vo.vop[dt].u = *reinterpret_cast<const uint4*>(vb + (size_t)(16 * dt) * page_size * sizeof(bf16));
+            return ids.v < 0;
+        };
+        // as mend(): values that were never written, or whose page was given back
+        auto clear = [&](int j, bool gone, VOps& vo) {
+            const int b = block_of(j);
+            if (32 * b + 31 <= hi_g && !__any(gone)) return;
+            const int n_ok = gone ? 0 : hi_g + 1 - (32 * b + 8 * g);      // of the lane's eight keys
+            uint32_t keep[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) keep[e] = n_ok >= 2 * e + 2 ? 0xffffffffu : n_ok == 2 * e + 1 ? 0xffffu : 0u;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                vo.vop[dt].u.x &= keep[0];
+                vo.vop[dt].u.y &= keep[1];
+                vo.vop[dt].u.z &= keep[2];
+                vo.vop[dt].u.w &= keep[3];
+            }
+        };
+        // round r of a wave is walk step AP_WAVES * r + cw of its key group: between them the waves take every block once
+        const int last = nf + b1 - b0;                   // the walk's last block
+        auto in_walk = [&](int j) { return j * KW + kg <= last; };
+        VOps vals_odd;
+        KOps k_even, k_odd;
+        VOps vals;
+        bool gone_a = load(cw, page_ids(cw), k_even, vals), gone_b;
+        PageIds ids = page_ids(cw + AP_WAVES);
+        for (int j = cw; in_walk(j); j += 2 * AP_WAVES) {
+            gone_b = load(j + AP_WAVES, ids, k_odd, vals_odd);       // (past the end: the last block again)
+            ids = page_ids(j + 2 * AP_WAVES);
+            clear(j, gone_a, vals);
+            compute(one, j, k_even, vals, stage0, k_even, stage0, vals, false, false);
+            if (!in_walk(j + AP_WAVES)) break;
+            gone_a = load(j + 2 * AP_WAVES, ids, k_even, vals);
+            ids = page_ids(j + 3 * AP_WAVES);
+            clear(j + AP_WAVES, gone_b, vals_odd);
+            compute(one, j + AP_WAVES, k_odd, vals_odd, stage0, k_odd, stage0, vals_odd, false, false);
+        }
+        l_run[0] += __shfl_xor(l_run[0], 16, MV_WAVE);
+        l_run[0] += __shfl_xor(l_run[0], 32, MV_WAVE);
+        // sums of 2 * KW waves to a stage, [DT][4][64] each
+        static_assert(sizeof(stage0) >= 2 * KW * DT * 4 * MV_WAVE * sizeof(float) && sizeof(stage2) >= 2 * NW * 16 * sizeof(float),
+                      "the stages are too small for the exchange");
+        constexpr int SUMS = DT * 4 * MV_WAVE;
+        float* mine = reinterpret_cast<float*>(wave < 2 * KW ? stage0 : stage1) + (wave % (2 * KW)) * SUMS;
+        float* xm = reinterpret_cast<float*>(stage2);    // [NW][16] maxima, then sums
+        float* xl = xm + NW * 16;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mine[(dt * 4 + r) * MV_WAVE + lane] = acc_o[0][dt][r];
+        if (g == 0) {
+            xm[wave * 16 + i] = m_run[0];
+            xl[wave * 16 + i] = l_run[0];
+        }
+        __syncthreads();
+        float m_fin = -INFINITY, l_fin = 0.f, f[NW];
+#pragma unroll
+        for (int w = 0; w < NW; ++w) m_fin = fmaxf(m_fin, xm[w * 16 + i]);
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float m = xm[w * 16 + i];
+            f[w] = SIG ? 1.f : (m == -INFINITY ? 0.f : exp2f(m - m_fin));
+            l_fin = fmaf(f[w], xl[w * 16 + i], l_fin);
+        }
+        if (!col_ok[0]) return;
+        const float inv = finish(0, m_fin, l_fin);
+        bf16* orow = out + (size_t)col_tok[0] * out_stride + (size_t)col_head[0] * D;
+        for (int dt = wave; dt < DT; dt += NW) {
+            float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const float* from = reinterpret_cast<const float*>(w < 2 * KW ? stage0 : stage1) + (w % (2 * KW)) * SUMS;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[r] = fmaf(f[w], from[(dt * 4 + r) * MV_WAVE + lane], o[r]);
+            }
+            uint2 packed;
+            packed.x = f32x2_to_bf16x2_bits(o[0] * inv, o[1] * inv);
+            packed.y = f32x2_to_bf16x2_bits(o[2] * inv, o[3] * inv);
+            *reinterpret_cast<uint2*>(orow + 16 * dt + 4 * g) = packed;
+        }
+        return;
+    }
 
     const int rounds = (nf + b1 - b0 + KW) / KW;    // the same for every wave: they meet at the barriers
     PageIds ids_a, ids_b;
@@ -521,7 +681,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
         // same: every key of it is masked; the walk has no branches around the reads and the products.)
         bool gone_a = false, gone_b = false;
         auto two_rounds = [&](int j, uint4* cur0, uint4* cur1, uint4* nxt0, uint4* nxt1) {
-            compute(j, k_even, vals, cur1, k_odd, cur0, vals, true, true);
+            compute(all, j, k_even, vals, cur1, k_odd, cur0, vals, true, true);
             read_v(cur1, vals);
             // (asked for here and not a block earlier: 32 columns a wave have no registers to spare
             // for them during the block, and the wait that follows is for the loads of two blocks)
@@ -539,7 +699,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
             }
             ids_a = nid_a;
             ids_b = nid_b;
-            compute(j + 1, k_odd, vals, nxt0, k_even, nxt0, vals, true, false);
+            compute(all, j + 1, k_odd, vals, nxt0, k_even, nxt0, vals, true, false);
         };
         {
             const PageIds i0 = page_ids(0), i1 = page_ids(1);
@@ -590,11 +750,11 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
                 ids_a = page_ids(j + 4);
                 ids_b = page_ids(j + 5);
             }
-            if (busy0) compute(j, k_even, vals, cur0, k_even, cur0, vals, false, false);
+            if (busy0) compute(all, j, k_even, vals, cur0, k_even, cur0, vals, false, false);
             if (busy1) {
                 read_k(cur1, k_even);
                 read_v(cur1, vals);
-                compute(j + 1, k_even, vals, cur1, k_even, cur1, vals, false, false);
+                compute(all, j + 1, k_even, vals, cur1, k_even, cur1, vals, false, false);
             }
             AP_WAIT_VMCNT(0);
             if (more) {
@@ -676,26 +836,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
 #pragma unroll
     for (int ct = 0; ct < NT; ++ct) {
         if (!col_ok[ct]) continue;
-        float inv;
-        if constexpr (SIG) {
-            inv = 1.f;
-            if (sig.gate != nullptr) {
-                const float z = to_f(sig.gate[(size_t)col_tok[ct] * sig.gate_stride + col_head[ct]]);
-                inv = 1.f / (1.f + __expf(-z));
-            }
-        } else {
-            if (SCORED && form.sink) {          // one more score, 0, without a value
-                const float m_fin = fmaxf(m_run[ct], 0.f);
-                const float f = exp2f(m_run[ct] - m_fin);
-                inv = f / fmaf(f, l_run[ct], exp2f(-m_fin));
-            } else {
-                inv = 1.f / l_run[ct];
-            }
-            if (sig.gate != nullptr) {
-                const float z = to_f(sig.gate[(size_t)col_tok[ct] * sig.gate_stride + col_head[ct]]);
-                inv *= 1.f / (1.f + __expf(-z));
-            }
-        }
+        const float inv = finish(ct, m_run[ct], l_run[ct]);
         bf16* orow = out + (size_t)col_tok[ct] * out_stride + (size_t)col_head[ct] * D;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
@@ -714,28 +855,39 @@ extern "C" int mv_attention_prefill_unit_tokens(int group, int nt) {
 }
 
 template <int D, int NT, int KW, bool SIG = false, bool SCORED = false>
-static int launch_prefill(dim3 grid, hipStream_t stream, const void* q, long q_stride, void* out, long out_stride,
+static int launch_prefill(int narrow, dim3 grid, hipStream_t stream, const void* q, long q_stride, void* out, long out_stride,
                           const void* k_pages, const void* v_pages, const int* block_table, int bt_width,
                           int page_size, int page_shift, const int* positions, const int* cu_seqlens, int n_seqs,
                           int H, int Hkv, float scale, int window, int fold, SigmoidArgs sig = SigmoidArgs{0, nullptr, nullptr, 0, 0},
                           ScoreForm form = ScoreForm{0.f, nullptr, 0}) {
     // the stages of K and V tiles are static LDS (four of 16 KiB per key group with D = 128)
-    hipLaunchKernelGGL((attention_prefill_kernel<D, NT, KW, SIG, SCORED>), grid, dim3(AP_THREADS * KW), 0, stream, (const bf16*)q,
-                       q_stride, (bf16*)out, out_stride, (const bf16*)k_pages, (const bf16*)v_pages, block_table,
-                       bt_width, page_size, page_shift, positions, cu_seqlens, n_seqs, H, Hkv, scale, window, fold, sig, form);
+    const dim3 threads(AP_THREADS * KW);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, threads, 0, stream, (const bf16*)q, q_stride, (bf16*)out, out_stride, (const bf16*)k_pages,
+                           (const bf16*)v_pages, block_table, bt_width, page_size, page_shift, positions, cu_seqlens, n_seqs, H, Hkv, scale,
+                           window, fold, sig, form);
+    };
+    if constexpr (KW > 1 || NT == 1) {
+        if (narrow) {
+            launch(attention_prefill_kernel<D, NT, KW, SIG, SCORED, true>);
+            return 0;
+        }
+    }
+    launch(attention_prefill_kernel<D, NT, KW, SIG, SCORED, false>);
     return 0;
 }
 
 // nt: column tiles per wave (2 = 128 columns per workgroup, for long prompts; 1 = 64 columns, twice
 // the workgroups, for steps too small to fill the chip otherwise).
 // kw: key groups per workgroup (2: eight waves, the walk over a unit's keys takes half as many rounds).
+// narrow: some request may bring so few tokens that its columns fit one tile of 16 (the kernel that serves these apart).
 // n_units = sum over sequences of ceil(q_len / unit tokens(group, nt)), or an upper bound of it (units
 // beyond the step's own end at once); n_busy = the units that hold tokens, as far as the caller knows
 // (n_units if it knows no better): it decides how the units are dealt out. grid = (kv heads, units).
 extern "C" int mv_attention_prefill(const void* q, long q_stride, void* out, long out_stride, const void* k_pages,
                                     const void* v_pages, const int* block_table, int bt_width, int page_size,
                                     const int* positions, const int* cu_seqlens, int n_seqs, int n_units, int n_busy,
-                                    int nt, int kw, int H, int Hkv, int D, float scale, int window, int first,
+                                    int nt, int kw, int narrow, int H, int Hkv, int D, float scale, int window, int first,
                                     const void* gate, long gate_stride, float cap, const float* slopes, int sink,
                                     hipStream_t stream) {
     MV_REQUIRE(kw == 1 || kw == 2, "attention_prefill: %d key groups per workgroup (1 or 2)", kw);
@@ -768,10 +920,10 @@ extern "C" int mv_attention_prefill(const void* q, long q_stride, void* out, lon
     const ScoreForm form{cap, slopes, sink};
     const bool scored = cap > 0.f || slopes != nullptr || sink;
 #define AP_LAUNCH(DD, NN, KK)                                                                                      \
-    rc = scored ? launch_prefill<DD, NN, KK, false, true>(grid, stream, q, q_stride, out, out_stride, k_pages, v_pages,   \
+    rc = scored ? launch_prefill<DD, NN, KK, false, true>(narrow, grid, stream, q, q_stride, out, out_stride, k_pages, v_pages,   \
                                                           block_table, bt_width, page_size, page_shift, positions,      \
                                                           cu_seqlens, n_seqs, H, Hkv, scale, window, fold, extra, form) \
-                : launch_prefill<DD, NN, KK>(grid, stream, q, q_stride, out, out_stride, k_pages, v_pages, block_table, \
+                : launch_prefill<DD, NN, KK>(narrow, grid, stream, q, q_stride, out, out_stride, k_pages, v_pages, block_table, \
                                              bt_width, page_size, page_shift, positions, cu_seqlens, n_seqs, H, Hkv,    \
                                              scale, window, fold, extra)
     if (kw == 2) {
@@ -796,7 +948,7 @@ extern "C" int mv_attention_prefill(const void* q, long q_stride, void* out, lon
 extern "C" int mv_attention_prefill_sigmoid(const void* q, long q_stride, void* out, long out_stride, const void* k_pages,
                                             const void* v_pages, const int* block_table, int bt_width, int page_size,
                                             const int* positions, const int* cu_seqlens, int n_seqs, int n_units,
-                                            int n_busy, int nt, int kw, int H, int Hkv, int D, float scale, int window,
+                                            int n_busy, int nt, int kw, int narrow, int H, int Hkv, int D, float scale, int window,
                                             int chunk, const float* bias, const void* gate, long gate_stride,
                                             hipStream_t stream) {
     MV_REQUIRE(kw == 1 || kw == 2, "attention_prefill_sigmoid: %d key groups per workgroup (1 or 2)", kw);
@@ -824,7 +976,7 @@ extern "C" int mv_attention_prefill_sigmoid(const void* q, long q_stride, void* 
     const SigmoidArgs sig{chunk, bias, (const bf16*)gate, gate_stride, 0};
     int rc = 0;
 #define AP_LAUNCH(DD, NN, KK)                                                                                          \
-    rc = launch_prefill<DD, NN, KK, true>(grid, stream, q, q_stride, out, out_stride, k_pages, v_pages, block_table,     \
+    rc = launch_prefill<DD, NN, KK, true>(narrow, grid, stream, q, q_stride, out, out_stride, k_pages, v_pages, block_table,     \
                                           bt_width, page_size, page_shift, positions, cu_seqlens, n_seqs, H, Hkv, scale, \
                                           window, fold, sig)
     if (kw == 2) {

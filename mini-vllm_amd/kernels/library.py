@@ -278,12 +278,12 @@ _OPTIONAL_SIGNATURES = {
     # ..., positions, cu_seqlens, n_seqs, n_units, n_busy, nt, kw, H, Hkv, D, scale, window, first, gate, gate_stride, cap, slopes,
     # sink, stream
     "mv_attention_prefill": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int,
-                                     c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+                                     c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                      c_float, c_int, c_int, c_void_p, c_long, c_float, c_void_p, c_int, c_void_p]),
     "mv_attention_prefill_unit_tokens": (c_int, [c_int, c_int]),
     # as mv_attention_prefill up to window, then chunk, bias, gate, gate_stride, stream
     "mv_attention_prefill_sigmoid": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int,
-                                             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+                                             c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                              c_float, c_int, c_int, c_void_p, c_void_p, c_long, c_void_p]),
     # packed, ld, n, n_seqs, H, G, DK, DV, taps, conv_w, a_log, dt_bias, weight_dtype, conv_state, unit_eps, token_seq,
     # cu_seqlens, state_slots, qk, vals, gates, dtype, stream

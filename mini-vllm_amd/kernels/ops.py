@@ -2224,7 +2224,7 @@ class Ops:
                                      head_dim, 2)
                 self.lib.call("mv_attention_prefill_sigmoid", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
                               v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size,
-                              positions.data_ptr(), plan.cu_seqlens.data_ptr(), plan.n_seqs, n_units, n_busy, nt, kw,
+                              positions.data_ptr(), plan.cu_seqlens.data_ptr(), plan.n_seqs, n_units, n_busy, nt, kw, int(plan.has_short(16 // group + 1)),
                               num_heads, num_kv_heads, head_dim, float(scale), w, c, _ptr(bias), _ptr(gate), gate_stride,
                               self._stream())
                 return
@@ -2963,7 +2963,8 @@ class Ops:
         self._note_attention("mv_attention_prefill", priced, q.shape[0], H, Hkv, D, 2)
         self.lib.call("mv_attention_prefill", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
                       v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size,
-                      positions.data_ptr(), plan.cu_seqlens.data_ptr(), n_seqs, n_units, n_busy, nt, kw, H, Hkv, D,
+                      positions.data_ptr(), plan.cu_seqlens.data_ptr(), n_seqs, n_units, n_busy, nt, kw,
+                      int(plan.has_short(16 // group + 1)), H, Hkv, D,
                       float(scale), window, first, _ptr(gate), gs, *form, self._stream())
         return True
 
