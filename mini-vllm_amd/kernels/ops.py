@@ -7,6 +7,7 @@ from __future__ import annotations
 
 from typing import Optional
 
+import math
 import os
 
 import torch
@@ -2370,6 +2371,20 @@ class Ops:
         return out.dtype == self.dtype or (out.dtype == torch.float32 and self.lib.has("mv_gemm_lt")
                                            and out.data_ptr() % 16 == 0)
 
+    def _rows_behind_whole_rounds(self, M: int, N: int) -> int:
+        """How many of M rows the library is given in a call of their own: those behind the rows whose tiles of 256 x 256 fill
+        the compute units a whole number of times. Just above such a size its choice of a kernel goes wrong. On MI355X, whole
+        against in two calls (us; N x K, rows in front + behind): 4096 x 12288, 4096 + 200: 632 / 301, + 640: 378 / 348, 8192 +
+        384: 961 / 603; 24576 x 4096, 2048 + 640: 475 / 395, 4096 + 384: 761 / 623, + 1024: 700 / 708; 4096 x 4096, 4096 + 200:
+        137 / 110; 4096 x 1024, 4096 + 200: 45 / 41; over eleven shapes at up to 13,312 rows the two calls took 0.46 to 1.04 of
+        the one's time, on average 0.86. With more rows behind, or where the rounds end at other numbers of rows (6144 x 4096:
+        155 / 172), the two are alike or one call is faster."""
+        if N % 256 or M <= 2048:
+            return 0
+        step = 256 * (self.compute_units // math.gcd(self.compute_units, N // 256))
+        rest = M % step
+        return rest if step in (2048, 4096) and M > step and rest <= 1024 else 0
+
     def _library_product(self, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor) -> bool:
         """out = a @ w^T (+ bias) by the library (hipBLASLt), bf16 in, bf16 or float32 out. It is
         called directly where the kernel library was built with it (a call costs a third of the host
@@ -2378,6 +2393,10 @@ class Ops:
         no algorithm for the shape."""
         M, K = a.shape
         N = w.shape[0]
+        rest = self._rows_behind_whole_rounds(M, N)
+        if rest:
+            return self._library_product(a[:M - rest], w, bias, out[:M - rest]) and \
+                self._library_product(a[M - rest:], w, bias, out[M - rest:])
         if self.lib.has("mv_gemm_lt") and a.stride(1) == 1 and out.stride(1) == 1 and a.data_ptr() % 16 == 0 \
                 and out.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
             if self._lt_work is None:
