@@ -4,7 +4,7 @@
 //
 //   moe_pairs     lays the pairs out expert by expert (`sorted`: pair numbers, a pair is token * top + place; a shared expert
 //                 that every token uses is one more expert, its pairs n * top + token) and cuts every expert's run into tiles
-//                 of `rows` (`tile_expert`, `tile_row0`, `tile_rows`; entries behind the last hold expert -1). Identity experts
+//                 of `rows` (`tile_expert`, `tile_row0`, `tile_rows`, `n_tiles` of them). Identity experts
 //                 and pairs without an expert are left out. Within an expert the order of the pairs is whatever the counters
 //                 gave; no result depends on it (a row's products read only its own row).
 //   moe_tile<GATED>  act[pair] = weight[pair] * pair(x W_gate^T, x W_up^T), rounded once
@@ -12,9 +12,9 @@
 //   moe_combine   y[token] = its places' out rows in order, the shared expert's, (identity weights) * x[token], added in float
 //
 // What bounds it: at 2,048 tokens, 32 experts of 768 x 1024 and 4 a token, the bytes (151 MB of weights) are worth 30 us, the
-// products 57; measured 70 (gate and up) + 42 (down) + 9 (moe_pairs) + 7 (combine) us a layer, where every expert for every
-// token took 167 + 175 through the library and 38 for the activation between; 1,000 tokens beside a shared expert 54 + 38 + 6 + 5
-// against 110 + 154 + 26. Eight rows: 19 + 13 + 5 + 5 against 22 + 12 + 7 + 5 (the unchosen experts' weights are not read).
+// products 57; measured 54 (gate and up) + 41 (down) + 9 (moe_pairs) + 8 (combine) us a layer, where every expert for every
+// token took 167 + 175 through the library and 38 for the activation between; 1,000 tokens beside a shared expert 54 + 28 + 6 + 5
+// against 110 + 154 + 26. Eight rows: 47 us a layer with the routing against 55 (the unchosen experts' weights are not read).
 #include "gemm_ring.h"
 
 #define MT_MAX_E 1024
@@ -24,6 +24,7 @@ struct PairTables {
     int* tile_expert;
     int* tile_row0;
     int* tile_rows;
+    int* n_tiles;
     int max_tiles;
 };
 
@@ -64,8 +65,7 @@ moe_pairs_kernel(const int* __restrict__ ids, int n_pairs, int n_real, int share
         t.tile_row0[tile] = first + r;
         t.tile_rows[tile] = min(rows, c - r);
     }
-    if (tid == 1023)
-        for (; tile < t.max_tiles; ++tile) t.tile_expert[tile] = -1;
+    if (tid == 1023) *t.n_tiles = tile;
     __syncthreads();
     for (int p = tid; p < n_pairs; p += 1024) {
         const int e = ids[p];
@@ -103,12 +103,15 @@ moe_tile_kernel(MoeTileArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid / MV_WAVE);
     const int lane = tid % MV_WAVE, i = lane % 16, g = lane / 16;
     const int wm = wave / 2, wn = wave % 2;
-    // an XCD walks a run of tiles with all their columns: an expert's tiles stand side by side, so its weights go into one L2
-    const int total = gridDim.x, id = (blockIdx.x % GT_XCDS) * (total / GT_XCDS) + blockIdx.x / GT_XCDS;
+    // An XCD walks a run of tiles with all their columns: an expert's tiles stand side by side, so its weights go into one L2.
+    // The runs are cut from the tiles that there are, not from the most there could be (what the grid is sized for): so cut, the
+    // last XCDs had none: 2,048 tokens, 32 experts, 4 a token 70.2 -> 53.6 us (gate and up), 42.2 -> 40.9 (down); 1,000 tokens
+    // beside a shared expert 54 -> 53.5 and 38 -> 28; 64 rows beside one 66 -> 59 us a layer.
+    const int total = *a.t.n_tiles * a.tiles_n, run = (total + GT_XCDS - 1) / GT_XCDS, at = blockIdx.x / GT_XCDS;
+    const int id = blockIdx.x % GT_XCDS * run + at;
+    if (at >= run || id >= total) return;
     const int tile = id / a.tiles_n, tn = id % a.tiles_n;
-    if (tile >= a.t.max_tiles) return;
     const int expert = a.t.tile_expert[tile];
-    if (expert < 0) return;
     const bool is_shared = expert == a.n_real;
     const int width = is_shared ? a.FS : a.F;                  // of the expert
     const int n_out = GATED ? width : a.N;
@@ -126,8 +129,8 @@ moe_tile_kernel(MoeTileArgs a) {
         slot[rep] = j * 64;
         if (row < BM) {
             const int p = a.t.sorted[row0 + (row < count ? row : 0)];          // rows past the end: some pair; never stored
-            const long at = GATED ? (p < a.n_pairs ? p / a.top : p - a.n_pairs) : p;
-            src[rep] = reinterpret_cast<const char*>(a.A + at * a.lda + 8 * piece);
+            const long row_of = GATED ? (p < a.n_pairs ? p / a.top : p - a.n_pairs) : p;
+            src[rep] = reinterpret_cast<const char*>(a.A + row_of * a.lda + 8 * piece);
         } else {
             const int r = row - BM;
             long w;
@@ -269,7 +272,7 @@ static int launch_moe_tiles(MoeTileArgs& a, int wm, int wn, hipStream_t stream) 
     return mv_check_launch("moe_tile");
 }
 
-// ints of scratch: sorted pairs and the three tile tables, for tiles of 32 rows
+// ints of scratch: sorted pairs, the three tile tables, for tiles of 32 rows, and the number of tiles
 extern "C" long mv_moe_pairs_ints(int n, int top, int n_real, int shared) {
     const long pairs = (long)n * (top + (shared ? 1 : 0));
     return pairs + 3L * (pairs / 32 + n_real + 2);
@@ -300,6 +303,7 @@ extern "C" int mv_moe_pairs(const void* x, long ldx, int n, int hidden, const vo
     t.tile_expert = ints + pairs;
     t.tile_row0 = t.tile_expert + t.max_tiles;
     t.tile_rows = t.tile_row0 + t.max_tiles;
+    t.n_tiles = t.tile_rows + t.max_tiles;
     hipLaunchKernelGGL(moe_pairs_kernel, dim3(1), dim3(1024), 0, stream, ids, (int)n_pairs, n_real, FS ? n : 0, rows, t);
     if (mv_check_launch("moe_pairs")) return 1;
     // columns of a tile: half as many where a step's few tiles leave compute units idle
