@@ -50,12 +50,22 @@ from ..kernels.ops import RowSums
 from .base import Mixer, PartSpec, Runtime, TensorDecl, register_mixer
 
 
+# In a step that brings short requests too both paths run, one behind the other (a scan of up to 127 tokens, 28 us, and the
+# chunks' two kernels, 20 us and more), where the scan alone takes 0.22 us a token of the longest. So such a step takes the
+# chunks only for longer requests, or, recorded for a class of steps, in classes large enough to hold them (us a step, Bolapel
+# 0.6B, both paths against the scan alone: prompts of 40 to 227 tokens 4,829 / 4,323, two of 120 beside eight decoding
+# 4,628 / 4,072; five of 400 on average 7,364 / 7,939).
+CHUNKS_BESIDE_SHORT = 384
+CHUNKS_BESIDE_SHORT_CLASS = 1024
+
+
 def recurrence(rt: Runtime, ctx, rule: str, n: int, heads: int, dk: int, dv: int, raw: torch.Tensor, scan, chunks, *operands) -> None:
     """A mixer's recurrence over the step's rows into ``raw``: requests of many tokens as products over chunks of tokens
     (``chunks``), the others, and heads of sizes these do not take, token by token (``scan``)."""
     ops, ws, plan = rt.ops, rt.workspace, ctx.attention_plan
     line = ops.delta_chunk_line()
-    if plan is None or not plan.has_long(line) or not ops.delta_chunks_serve(rule, dk, dv):
+    least = line if plan is None or not plan.has_short(line) else CHUNKS_BESIDE_SHORT_CLASS if plan.bound is not None else CHUNKS_BESIDE_SHORT
+    if plan is None or not plan.has_long(least) or not ops.delta_chunks_serve(rule, dk, dv):
         scan(*operands, raw)
         return
     units = plan.units(ops.delta_chunk_tokens())
