@@ -43,6 +43,7 @@ struct DeltaChunkArgs {
     const float* vec;              // GENERAL: coef [n][H][5][DK] (w, rate u, u, k, r); else qk [n][G][2][DK]
     const float* gates;            // CHANNEL: beta [n][H]; GATED, SUM: [n][H][4] (decay, strength, ..)
     const float* decay; long ldz;  // CHANNEL: rows whose first H*DK columns are the decays
+    int decay4;                    // ... whose rows start at addresses that four floats can be loaded from at once
     const void* vals; long ldv;    // GENERAL: packed rows, the values in columns 2*H*DK ..; else [n][H][DV] floats
     int H, G, DV;
     const int* cu_seqlens; int n_seqs;
@@ -141,7 +142,8 @@ delta_chunk_kernel(DeltaChunkArgs A) {
             r = at(v);
             xx = at(v + DK);
             if constexpr (RULE == RULE_CHANNEL) {
-                w = at(A.decay + row * A.ldz + (size_t)head * DK);
+                const float* d = A.decay + row * A.ldz + (size_t)head * DK;
+                w = A.decay4 ? at(d) : float4{d[c], d[c + 1], d[c + 2], d[c + 3]};
             } else {
                 const float d = A.gates[(row * H + head) * 4];
                 w = float4{d, d, d, d};
@@ -563,12 +565,13 @@ extern "C" int mv_delta_chunks(int rule, const float* vec, const float* gates, c
     MV_REQUIRE(vec && vals && state && cu_seqlens && state_slots && M && N && Q && out, "delta_chunks: missing operand");
     MV_REQUIRE(rule != RULE_GENERAL || (G == H && DV == DK && ldv >= 3L * H * DK && mv_valid_dtype(dtype)), "delta_chunks: rows do not hold r, k and v");
     MV_REQUIRE(rule == RULE_GENERAL || gates, "delta_chunks: missing gates");
-    MV_REQUIRE(rule != RULE_CHANNEL || (decay && ldz >= (long)H * DK && ldz % 4 == 0 && (uintptr_t)decay % 16 == 0), "delta_chunks: decays do not fit");
+    MV_REQUIRE(rule != RULE_CHANNEL || (decay && ldz >= (long)H * DK), "delta_chunks: decays do not fit");
     MV_REQUIRE((uintptr_t)vec % 16 == 0 && (uintptr_t)state % 16 == 0 && (uintptr_t)M % 16 == 0 && (uintptr_t)N % 16 == 0 && (uintptr_t)Q % 16 == 0,
                "delta_chunks: operands must be 16-byte aligned");
     MV_REQUIRE(H <= 65535, "delta_chunks: too many heads");
     if (n == 0 || n_seqs == 0 || chunks == 0) return 0;
-    const DeltaChunkArgs A{vec, gates, decay, ldz, vals, ldv, H, G, DV, cu_seqlens, n_seqs, M, N, Q, out};
+    const int decay4 = ldz % 4 == 0 && (uintptr_t)decay % 16 == 0;
+    const DeltaChunkArgs A{vec, gates, decay, ldz, decay4, vals, ldv, H, G, DV, cu_seqlens, n_seqs, M, N, Q, out};
 #define DC_LAUNCH(T, RULE)                                                                                   \
     return DK == 64 ? launch_delta_chunks<T, 64, RULE>(A, state, state_slots, chunks, stream)               \
                     : launch_delta_chunks<T, 128, RULE>(A, state, state_slots, chunks, stream)

@@ -488,6 +488,33 @@ def test_channel_delta_steps_of_many_rows(dtype, H, G, dk, dv, taps, q_lens):
     test_channel_delta_step(dtype, H, G, dk, dv, taps, 7, 9, q_lens)
 
 
+@pytest.mark.parametrize("H, G, dk, dv", [(3, 3, 64, 66), (1, 1, 64, 65), (2, 1, 128, 33)])
+def test_channel_delta_long_requests_of_odd_widths(H, G, dk, dv):
+    """Requests long enough for the products over chunks, with rows of decays and gates that are no whole number of four floats:
+    the decays of every second or fourth row cannot be loaded four at once."""
+    rt = runtime(torch.bfloat16)
+    hid, eps = 96, 1e-5
+    w = channel_case(H, G, dk, dv, 4, 16, 16, hid, seed=H * 100 + dk)
+    part = build_channel(rt, w, H, G, dk, dv, 4, 16, 16, hid, eps)
+    lens, slots = [rt.ops.delta_chunk_line() + 25, 2 * rt.ops.delta_chunk_line() + 3], [1, 0]
+    g = torch.Generator().manual_seed(6)
+    x = torch.randn(sum(lens), hid, generator=g).bfloat16()
+    state = torch.zeros(2, H, dv, dk, device=DEV)
+    conv = torch.zeros(2, 3, 2 * G * dk + H * dv, dtype=torch.bfloat16, device=DEV)
+    rt.ops.ledger = []
+    y = part.forward(x.to(DEV), state_ctx(lens, slots, state, conv=conv), 0)
+    y = y if isinstance(y, torch.Tensor) else y.materialize()
+    torch.cuda.synchronize()
+    ran, rt.ops.ledger = [e[0] for e in rt.ops.ledger], None
+    assert "mv_delta_chunks" in ran
+    base = 0
+    for q, slot in zip(lens, slots):
+        want, after = plain_channel(x[base:base + q], w, {"heads": H, "kv_heads": G, "dim": dk, "vdim": dv}, eps, None, torch.bfloat16)
+        close(y[base:base + q], want, 2e-2, f"request of {q}")
+        close(state[slot].transpose(1, 2), after["S"], 5e-3, "state")
+        base += q
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("G", [4, 2])
 def test_channel_delta_portions(dtype, G):
