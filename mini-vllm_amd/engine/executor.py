@@ -262,7 +262,8 @@ class Executor:
 
     def _warmup(self, num_tokens: int) -> None:
         """One dry step of ``num_tokens`` tokens against a throw-away cache, so that every scratch
-        buffer reaches its final size before the cache is sized from what is left."""
+        buffer reaches its final size before the cache is sized from what is left. It cuts the tokens into many
+        sequences; what other cuts need is reserved."""
         ps = self.page_size
         n_seqs = max(1, min(self.config.max_num_batched_seqs, _cdiv(num_tokens, ps)))
         # (no step holds more tokens of a request than max_model_len)
@@ -274,6 +275,7 @@ class Executor:
             table = list(range(s * pages_per_seq, (s + 1) * pages_per_seq))
             seqs.append(SeqStep(tokens=[0] * per_seq, start=0, block_tables=[table] * len(self.groups),
                                 state_slot=s % self.num_state_slots, want=[per_seq - 1]))
+        self.model.reserve(num_tokens, self.config.max_num_batched_seqs)
         self.step(seqs)
         if self.config.use_cuda_graph and self.model.graph_safe:
             # the scratch area that all decode graphs share, at the size of the largest batch they serve
@@ -740,6 +742,7 @@ class Executor:
                 plan = pad_ctx.attention_plan
                 plan.decode_only, plan.max_q_len, plan.q_lens, plan.bound = False, tokens, (), (tokens, largest)
                 plan.max_context_len = self.config.max_model_len
+                self.model.reserve(tokens, largest)
                 self.model.forward(pad_ctx)
             torch.cuda.synchronize()
         finally:

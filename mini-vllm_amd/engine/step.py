@@ -51,6 +51,12 @@ class KVView:
         return self.pages["v"]
 
 
+def most_units(tokens: int, seqs: int, unit_tokens: int, least: int = 1) -> int:
+    """The most runs of up to ``unit_tokens`` tokens that up to ``seqs`` sequences of at least ``least`` tokens each, ``tokens``
+    in all, can have: each adds less than one to what its tokens fill."""
+    return tokens // unit_tokens + min(seqs, tokens // least)
+
+
 @dataclass
 class AttentionPlan:
     """Host-side facts about the step that let the attention pick a kernel."""
@@ -81,13 +87,12 @@ class AttentionPlan:
     starts: Sequence[int] = ()
     step_q_lens: Sequence[int] = ()
 
-    def units(self, unit_tokens: int) -> int:
-        """Runs of up to ``unit_tokens`` consecutive tokens of one sequence in the step: counted from
-        the host's lengths, or the most that any cut within ``bound`` can have."""
+    def units(self, unit_tokens: int, least: int = 1) -> int:
+        """Runs of up to ``unit_tokens`` consecutive tokens of one sequence in the step, of the sequences that
+        bring at least ``least``: counted from the host's lengths, or the most that any cut within ``bound`` can have."""
         if self.bound is not None:
-            tokens, seqs = self.bound
-            return tokens // unit_tokens + seqs
-        return sum(-(-ql // unit_tokens) for ql in self.q_lens)
+            return most_units(*self.bound, unit_tokens, least)
+        return sum(-(-ql // unit_tokens) for ql in self.q_lens if ql >= least)
 
     def has_long(self, tokens: int) -> bool:
         """Whether a sequence may bring at least so many tokens to the step."""

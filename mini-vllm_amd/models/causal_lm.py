@@ -173,6 +173,12 @@ class CausalLM:
                         for name, (dims, dt) in shapes.items()} or None)
         return out
 
+    def reserve(self, tokens: int, seqs: int) -> None:
+        """Sizes the mixers' scratch for any cut of up to ``tokens`` tokens into up to ``seqs`` sequences."""
+        for mixer in self.mixers:
+            if mixer is not None:
+                mixer.reserve(tokens, seqs)
+
     # ------------------------------------------------------------------------------------
     def forward(self, ctx) -> torch.Tensor:
         """Runs the step described by ``ctx`` and returns float32 logits [len(logit_rows), vocab]."""

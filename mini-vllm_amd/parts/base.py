@@ -517,6 +517,10 @@ class Mixer(Part):
         one = cls.state_shape(spec)
         return {} if one is None else {"state": one}
 
+    def reserve(self, tokens: int, seqs: int) -> None:
+        """Sizes the scratch (``rt.workspace``) whose need depends on how a step is cut, for any cut of up to ``tokens``
+        tokens into up to ``seqs`` sequences. (What depends on the number of tokens alone, a run of that many sizes.)"""
+
     def forward(self, x: torch.Tensor, ctx, call: int) -> torch.Tensor:
         raise NotImplementedError
 

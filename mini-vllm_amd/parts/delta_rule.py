@@ -26,8 +26,8 @@ from typing import Dict, Optional
 
 import torch
 
-from .base import Mixer, PartSpec, Runtime, TensorDecl, register_mixer
-from .matrix_state import recurrence
+from .base import PartSpec, Runtime, TensorDecl, register_mixer
+from .matrix_state import ChunkedRecurrence, recurrence
 
 
 @dataclass(frozen=True)
@@ -47,7 +47,7 @@ class DeltaRuleSpec(PartSpec):
 
 
 @register_mixer(DeltaRuleSpec.kind)
-class DeltaRule(Mixer):
+class DeltaRule(ChunkedRecurrence):
     spec_class = DeltaRuleSpec
     PACKED = ("r", "k", "v", "g", "a", "w1")
 
@@ -72,6 +72,7 @@ class DeltaRule(Mixer):
         if spec.num_heads < 1 or spec.head_dim < 1 or spec.decay_rank < 1:
             raise ValueError(f"delta rule: bad sizes {spec}")
         self.spec, self.rt = spec, rt
+        self.recurrence_sizes = ("delta", spec.num_heads, spec.head_dim, spec.head_dim)
         dtypes = {tensors[p].dtype for p in self.PACKED}
         if len(dtypes) != 1:
             raise ValueError(f"delta rule: the projections are stored in different dtypes {dtypes}; cannot pack them")

@@ -46,6 +46,7 @@ from typing import Dict, Optional, Tuple
 
 import torch
 
+from ..engine.step import most_units
 from ..kernels.ops import RowSums
 from .base import Mixer, PartSpec, Runtime, TensorDecl, register_mixer
 
@@ -68,12 +69,26 @@ def recurrence(rt: Runtime, ctx, rule: str, n: int, heads: int, dk: int, dv: int
     if plan is None or not plan.has_long(least) or not ops.delta_chunks_serve(rule, dk, dv):
         scan(*operands, raw)
         return
-    units = plan.units(ops.delta_chunk_tokens())
-    chunks(*operands, ws.get("mstate.chunk_maps", (units, heads) + ((dk, dk) if rule != "sum" else ()), torch.float32),
-           ws.get("mstate.chunks", (units, heads, dv, dk), torch.float32),
-           ws.get("mstate.chunk_queries", (n, heads, dk), torch.float32), raw)
+    chunks(*operands, *_chunk_scratch(ws, rule, n, heads, dk, dv, plan.units(ops.delta_chunk_tokens(), line)), raw)
     if plan.has_short(line):
         scan(*operands, raw, below=line)
+
+
+def _chunk_scratch(ws, rule: str, n: int, heads: int, dk: int, dv: int, units: int):
+    return (ws.get("mstate.chunk_maps", (units, heads) + ((dk, dk) if rule != "sum" else ()), torch.float32),
+            ws.get("mstate.chunks", (units, heads, dv, dk), torch.float32),
+            ws.get("mstate.chunk_queries", (n, heads, dk), torch.float32))
+
+
+class ChunkedRecurrence(Mixer):
+    """A mixer that calls ``recurrence``."""
+    recurrence_sizes: Tuple[str, int, int, int]          # the rule, heads, key channels, columns
+
+    def reserve(self, tokens: int, seqs: int) -> None:
+        (rule, heads, dk, dv), ops = self.recurrence_sizes, self.rt.ops
+        line = ops.delta_chunk_line()
+        if tokens >= line and ops.delta_chunks_serve(rule, dk, dv):
+            _chunk_scratch(self.rt.workspace, rule, tokens, heads, dk, dv, most_units(tokens, seqs, ops.delta_chunk_tokens(), line))
 
 
 def _pack(tensors: Dict[str, torch.Tensor], names, hidden: int, what: str):
@@ -106,7 +121,7 @@ class GatedDeltaSpec(PartSpec):
 
 
 @register_mixer(GatedDeltaSpec.kind)
-class GatedDelta(Mixer):
+class GatedDelta(ChunkedRecurrence):
     spec_class = GatedDeltaSpec
     PACKED = ("q", "k", "v", "g", "b", "a")
 
@@ -135,6 +150,7 @@ class GatedDelta(Mixer):
                 or spec.num_heads % spec.num_kv_heads:
             raise ValueError(f"gated delta rule: bad sizes {spec}")
         self.spec, self.rt = spec, rt
+        self.recurrence_sizes = ("gated", spec.num_heads, spec.key_dim, spec.value_dim)
         self.w_packed = _pack(tensors, self.PACKED, spec.hidden_size, "gated delta rule")
         self.width = self.w_packed.shape[0]
         self.gate_offset = spec.conv_channels
@@ -185,7 +201,7 @@ class MLSTMSpec(PartSpec):
 
 
 @register_mixer(MLSTMSpec.kind)
-class MLSTM(Mixer):
+class MLSTM(ChunkedRecurrence):
     spec_class = MLSTMSpec
     PACKED = ("q", "k", "v", "g", "i", "f")
 
@@ -208,6 +224,7 @@ class MLSTM(Mixer):
         if min(spec.num_heads, spec.key_dim, spec.value_dim) < 1 or not spec.gate_cap > 0:
             raise ValueError(f"mlstm: bad sizes {spec}")
         self.spec, self.rt = spec, rt
+        self.recurrence_sizes = ("sum", spec.num_heads, spec.key_dim, spec.value_dim + 1)
         self.w_packed = _pack(tensors, self.PACKED, spec.hidden_size, "mlstm")
         self.width = self.w_packed.shape[0]
         self.gate_offset = spec.num_heads * (2 * spec.key_dim + spec.value_dim)
@@ -261,7 +278,7 @@ class ChannelDeltaSpec(PartSpec):
 
 
 @register_mixer(ChannelDeltaSpec.kind)
-class ChannelDelta(Mixer):
+class ChannelDelta(ChunkedRecurrence):
     """Packed rows: [q | k | v | b, padded to a multiple of 8 | W_a1 h | W_g1 h, padded to a multiple of 32]. In steps with
     prompt portions the two second matrices are one product against the low-rank columns (block-diagonal, in float32
     rows [decays | gates]); in steps of single tokens the step's kernel makes them itself."""
@@ -293,6 +310,7 @@ class ChannelDelta(Mixer):
                 or spec.num_heads % spec.num_kv_heads:
             raise ValueError(f"channel-wise delta rule: bad sizes {spec}")
         self.spec, self.rt = spec, rt
+        self.recurrence_sizes = ("channel", spec.num_heads, spec.key_dim, spec.value_dim)
         hid, H, dk, dv = spec.hidden_size, spec.num_heads, spec.key_dim, spec.value_dim
         ra, rg = spec.decay_rank, spec.gate_rank
         front = _pack(tensors, ("q", "k", "v", "b"), hid, "channel-wise delta rule")

@@ -1,0 +1,48 @@
+"""What the recurrences over chunks take as scratch is there before the cache is sized, however later steps are cut."""
+import random
+
+import pytest
+import torch
+
+from minivllm_amd.engine.step import AttentionPlan
+
+
+def test_no_cut_has_more_units():
+    from minivllm_amd.engine.step import most_units
+    rng = random.Random(1)
+    for _ in range(300):
+        least, seqs = rng.choice([1, 128]), rng.randint(1, 40)
+        lens = [rng.randint(1, rng.choice([3, 150, 1000])) for _ in range(seqs)]
+        plan = AttentionPlan(decode_only=False, max_q_len=max(lens), max_context_len=4096, n_seqs=seqs, q_lens=lens)
+        assert plan.units(32, least) <= most_units(sum(lens), seqs, 32, least)
+    lens = [129] * 7
+    plan = AttentionPlan(decode_only=False, max_q_len=129, max_context_len=4096, n_seqs=7, q_lens=lens)
+    assert plan.units(32, 128) == 35 == most_units(7 * 129, 40, 32, 128)
+    plan.q_lens = [1] * 500 + [160]
+    assert plan.units(32, 128) == 5, "requests that do not go in chunks count"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("graphs", [True, False])
+def test_scratch_stands_at_the_start(graphs):
+    """An engine that sizes its cache from the memory that is left: first long prompts of every kind of cut allocate no scratch."""
+    from minivllm_amd.config import EngineConfig
+    from minivllm_amd.engine.executor import Executor
+    from minivllm_amd.engine.step import SeqStep
+    from minivllm_amd.models import config_from_dict, expected_tensors
+    from minivllm_amd.weights.device_random import DeviceRandomSource
+    mlp = {"kind": "dense", "ff": 128}
+    arch, cfg = config_from_dict({"architecture": "Bolapel", "vocab": 256, "width": 128, "norm": {"eps": 1e-5}, "torch_dtype": "bfloat16",
+                                  "logit_softcap": 20.0,
+                                  "layers": [{"type": "general_delta", "mixer": {"heads": 2, "dim": 64, "rank": 8}, "mlp": mlp}]})
+    source = DeviceRandomSource(expected_tensors(arch, cfg), 1, torch.bfloat16, torch.device("cuda:0"), std=0.05)
+    ex = Executor(EngineConfig(model="", dtype="bfloat16", max_model_len=1024, max_num_batched_tokens=1024, max_num_batched_seqs=64,
+                               kv_cache_block_size=16, gpu_memory_utilization=0.05, use_cuda_graph=graphs), model=(arch, cfg, source))
+    areas = lambda: [ws.bytes() for ws in (ex.rt.workspace, ex._graph_workspace) if ws is not None]
+    at_start = areas()
+    assert len(at_start) == 1 + graphs
+    for lens in ([1024], [129] * 7, [700] + [1] * 60, [128], [383, 385, 200, 50]):
+        ex.step([SeqStep(tokens=[i % 256 for i in range(q)], start=0, block_tables=[[]] * len(ex.groups), state_slot=s, want=[q - 1])
+                 for s, q in enumerate(lens)])
+        torch.cuda.synchronize()
+        assert areas() == at_start, lens
