@@ -806,7 +806,7 @@ extern "C" int mv_gdelta_prepare(const void* packed, long ld, int n, int n_seqs,
 //     m' = max(f + m, i);   a = exp(f + m - m');   b = exp(i - m');   gates = (a, b, exp(-m'), 0)
 // Workgroup (request, head). Requests of fewer than MG_LINE tokens: its first wave walks the rows 64 at a time, the gates'
 // functions a row a lane, the maximum itself in the order of the rows, so that its bits do not depend on how a request was
-// cut. Longer ones (whose recurrence is cut into chunks anyway, from the same length on): all waves take the maxima of a run
+// cut; so all requests of the float engine. Longer ones otherwise (as their recurrences may): all waves take the maxima of a run
 // of rows as a prefix over the pairs (sum of f, max of i behind later f), (F, M)(F', M') = (F + F', max(M + F', M')); the
 // result holds for any maxima, a and b are made from the ones that are stored, so these may round differently. One wave took
 // 134 us for 2,048 rows of 16 heads (a chain of lane exchanges), the prefix 12.6 us.
@@ -821,7 +821,7 @@ mlstm_gates_kernel(const T* __restrict__ packed, long ld, int H, long gate_off, 
     __shared__ float sF[MG_THREADS / MV_WAVE], sM[MG_THREADS / MV_WAVE];
     const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x, lane = tid % MV_WAVE, wave = tid / MV_WAVE;
     const int first = cu_seqlens[seq], end = cu_seqlens[seq + 1];
-    const bool wide = end - first >= MG_LINE;
+    const bool wide = sizeof(T) < sizeof(float) && end - first >= MG_LINE;
     if (end <= first || (!wide && wave > 0)) return;
     float* ms = max_state + (size_t)state_slots[seq] * H + head;
     float m = *ms;

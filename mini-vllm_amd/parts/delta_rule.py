@@ -106,8 +106,9 @@ class DeltaRule(ChunkedRecurrence):
             ops.delta_prepare(packed, spec.num_heads, spec.head_dim, spec.decay_rank, self.w2_t, self.w0, self.a_bias,
                               spec.decay_rate, spec.key_eps, coef)
             raw = ws.get("delta.raw", (n, inner), torch.float32)
-            recurrence(rt, ctx, "delta", n, spec.num_heads, spec.head_dim, spec.head_dim, raw, ops.delta_scan, ops.delta_chunks,
-                       packed, coef, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, spec.num_heads, spec.head_dim)
+            recurrence(rt, ctx, "delta", n, spec.num_heads, spec.head_dim, spec.head_dim, raw, ops.delta_scan,
+                       self.chunks(ops.delta_chunks), packed, coef, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs,
+                       spec.num_heads, spec.head_dim)
             ops.delta_finish(raw, packed, self.norm, spec.num_heads, spec.head_dim, spec.out_norm_eps, gated)
         y = ws.get("mixer.out", (n, spec.hidden_size), rt.dtype)
         return ops.gemm(gated, self.w_o, y, defer_sum=True) or y

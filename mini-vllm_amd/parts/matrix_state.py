@@ -62,11 +62,11 @@ CHUNKS_BESIDE_SHORT_CLASS = 1024
 
 def recurrence(rt: Runtime, ctx, rule: str, n: int, heads: int, dk: int, dv: int, raw: torch.Tensor, scan, chunks, *operands) -> None:
     """A mixer's recurrence over the step's rows into ``raw``: requests of many tokens as products over chunks of tokens
-    (``chunks``), the others, and heads of sizes these do not take, token by token (``scan``)."""
+    (``chunks``, None: not in this engine), the others, and heads of sizes these do not take, token by token (``scan``)."""
     ops, ws, plan = rt.ops, rt.workspace, ctx.attention_plan
     line = ops.delta_chunk_line()
     least = line if plan is None or not plan.has_short(line) else CHUNKS_BESIDE_SHORT_CLASS if plan.bound is not None else CHUNKS_BESIDE_SHORT
-    if plan is None or not plan.has_long(least) or not ops.delta_chunks_serve(rule, dk, dv):
+    if plan is None or chunks is None or not plan.has_long(least) or not ops.delta_chunks_serve(rule, dk, dv):
         scan(*operands, raw)
         return
     chunks(*operands, *_chunk_scratch(ws, rule, n, heads, dk, dv, plan.units(ops.delta_chunk_tokens(), line)), raw)
@@ -84,10 +84,15 @@ class ChunkedRecurrence(Mixer):
     """A mixer that calls ``recurrence``."""
     recurrence_sizes: Tuple[str, int, int, int]          # the rule, heads, key channels, columns
 
+    def chunks(self, entry):
+        """``entry`` (the products over chunks), or None in float32: there every sum's order depends on the request alone,
+        not on how it is cut or what else is in the step, and which requests go in chunks depends on both."""
+        return None if self.rt.dtype == torch.float32 else entry
+
     def reserve(self, tokens: int, seqs: int) -> None:
         (rule, heads, dk, dv), ops = self.recurrence_sizes, self.rt.ops
         line = ops.delta_chunk_line()
-        if tokens >= line and ops.delta_chunks_serve(rule, dk, dv):
+        if self.rt.dtype != torch.float32 and tokens >= line and ops.delta_chunks_serve(rule, dk, dv):
             _chunk_scratch(self.rt.workspace, rule, tokens, heads, dk, dv, most_units(tokens, seqs, ops.delta_chunk_tokens(), line))
 
 
@@ -181,8 +186,8 @@ class GatedDelta(ChunkedRecurrence):
                                 ctx.state(call, "conv") if spec.conv_taps > 1 else None, spec.unit_eps, ctx.token_seq,
                                 ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, gates)
         raw = ws.get("mstate.raw", (n, H, dv), torch.float32)
-        recurrence(rt, ctx, "gated", n, H, dk, dv, raw, ops.state_scan, ops.state_chunks, qk, vals, gates, ctx.state(call), ctx.cu_seqlens,
-                   ctx.state_slots, ctx.n_seqs, H, G, dk, dv, True)
+        recurrence(rt, ctx, "gated", n, H, dk, dv, raw, ops.state_scan, self.chunks(ops.state_chunks), qk, vals, gates,
+                   ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv, True)
         ops.state_finish(raw, gates, packed, self.gate_offset, self.norm, H, dv, spec.out_norm_eps, ctx.token_seq, gated,
                          shared_weight=True, silu_gate=True)
         return ops.gemm(gated, self.w_o, y, defer_sum=True) or y
@@ -251,7 +256,7 @@ class MLSTM(ChunkedRecurrence):
         ops.mlstm_prepare(packed, H, dk, dv, self.i_bias, self.f_bias, spec.gate_cap, ctx.state(call, "max"), ctx.token_seq,
                           ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, gates)
         raw = ws.get("mstate.raw", (n, H, dv + 1), torch.float32)
-        recurrence(rt, ctx, "sum", n, H, dk, dv + 1, raw, ops.state_scan, ops.state_chunks, qk, vals, gates, ctx.state(call),
+        recurrence(rt, ctx, "sum", n, H, dk, dv + 1, raw, ops.state_scan, self.chunks(ops.state_chunks), qk, vals, gates, ctx.state(call),
                    ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, H, dk, dv + 1, False)
         ops.state_finish(raw, gates, packed, self.gate_offset, self.norm, H, dv, spec.out_norm_eps, ctx.token_seq, gated,
                          shared_weight=False, silu_gate=False, normaliser=True, denom_eps=spec.denom_eps)
@@ -356,8 +361,8 @@ class ChannelDelta(ChunkedRecurrence):
         ops.channel_prepare(packed, H, G, dk, dv, spec.conv_taps, self.b_offset, self.conv_w, self.a_log, self.dt_bias, conv_state,
                             spec.unit_eps, ctx.token_seq, ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, beta, z)
         raw = ws.get("mstate.raw", (n, H, dv), torch.float32)
-        recurrence(rt, ctx, "channel", n, H, dk, dv, raw, ops.channel_scan, ops.channel_chunks, qk, vals, beta, z, ctx.state(call),
-                   ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv)
+        recurrence(rt, ctx, "channel", n, H, dk, dv, raw, ops.channel_scan, self.chunks(ops.channel_chunks), qk, vals, beta, z,
+                   ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv)
         ops.state_finish(raw, None, z, H * dk, self.norm, H, dv, spec.out_norm_eps, ctx.token_seq, gated, shared_weight=True,
                          silu_gate=False)
         return ops.gemm(gated, self.w_o, y, defer_sum=True, fold=fold) or y
