@@ -157,8 +157,8 @@ class Executor:
         self._graphs: Dict[Tuple[int, int], Tuple[torch.cuda.CUDAGraph, StepContext, torch.Tensor, torch.Tensor]] = {}
         self._graph_pool = None
         self._repeat_graphs: Dict[Tuple[int, int, int], Tuple[torch.cuda.CUDAGraph, torch.Tensor, torch.Tensor]] = {}
-        # steps with prompt portions: (token bucket, sequence bucket, logit rows, context cap) -> graph
-        self._mixed_graphs: Dict[Tuple[int, int, int, int], Tuple] = {}
+        # steps with prompt portions: (token bucket, sequence bucket, logit rows, context cap, the mixers' choices) -> graph
+        self._mixed_graphs: Dict[tuple, Tuple] = {}
         self._graph_workspace: Optional[Workspace] = None
         # what each recorded graph holds, by kind of node (see _record)
         self.graph_census: Dict[Tuple, Dict[str, int]] = {}
@@ -547,7 +547,7 @@ class Executor:
     def _step_mixed_graph(self, seqs: Sequence[SeqStep], n_tokens: int) -> torch.Tensor:
         """A step with prompt portions from the graph of its size class: tokens and sequences are
         padded with inert rows up to the class's sizes, the kernels' grids are those of the worst
-        cut the class holds. A class is recorded at its first use."""
+        cut the class holds. A class is recorded at its first use, once for every choice of the mixers."""
         S = len(seqs)
         Sp = next(b for b in GRAPH_BUCKETS if b >= S)
         Np = next(b for b in TOKEN_BUCKETS if b >= n_tokens)
@@ -560,7 +560,7 @@ class Executor:
         cap = min(cap, max(self.config.max_model_len, 1))
         widths = [self.max_pages_per_seq] * len(self.groups)
         arr, off, facts = self._fill(seqs, pad_to=Sp, pad_tokens=Np, pad_rows=Mp, bt_widths=widths)
-        key = (Np, Sp, Mp, cap)
+        key = (Np, Sp, Mp, cap) + self.model.step_paths(facts["q_lens"])
         entry = self._mixed_graphs.pop(key, None)
         if entry is None:
             entry = self._capture(Sp, cap, arr, off, facts, seqs, mixed_key=key)
@@ -849,9 +849,9 @@ class Executor:
         arr[o:o + size] = 0
 
     def _capture(self, bucket: int, cap: int, arr: np.ndarray, off, facts, seqs: Sequence[SeqStep],
-                 mixed_key: Optional[Tuple[int, int, int, int]] = None):
+                 mixed_key: Optional[tuple] = None):
         """Records the graph of a decode step of ``bucket`` sequences, or (``mixed_key`` = (tokens,
-        sequences, logit rows, cap)) of a step with prompt portions of that size class."""
+        sequences, logit rows, cap, the mixers' choices)) of a step with prompt portions of that size class."""
         if mixed_key is None:
             logger.info("capturing the decode graph for %d sequences, contexts up to %d", bucket, cap)
         else:
@@ -873,6 +873,7 @@ class Executor:
                 plan.decode_only, plan.max_q_len, plan.q_lens = False, mixed_key[0], ()
                 plan.bound = (mixed_key[0], mixed_key[1])
                 plan.bound_least = max((b for b in TOKEN_BUCKETS if b < mixed_key[0]), default=0) + 1
+                plan.path_lens = tuple(facts["q_lens"])
                 ctx.q_lens = ctx.starts = ctx.host_state_slots = None
             else:
                 # ... and any number of sequences up to the bucket, of which this step may fill only some

@@ -78,6 +78,8 @@ class AttentionPlan:
     bound: Optional[tuple] = None
     # ... whose steps hold at least this many tokens
     bound_least: int = 1
+    # ... and for which every part that chooses by the sequences' lengths (``Mixer.step_path``) chooses as for these
+    path_lens: Sequence[int] = ()
     # for measurement: keys in the cache of the step's sequences after the step (summed), and the
     # number of (query, visible key) pairs without windows
     kv_tokens: int = 0

@@ -10,7 +10,7 @@ has, in which order layers run and whose cache a call reads are all read from th
 """
 from __future__ import annotations
 
-from typing import Dict, List, Optional, Tuple
+from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
@@ -108,6 +108,7 @@ class CausalLM:
         self.graph_safe = True          # every part allows its forward to be captured in a graph
         self.blocks = []
         self.mixers = []
+        self._choosers: Optional[List] = None      # one mixer of each kind and size that chooses by a step's lengths
         for i, layer in enumerate(plan.layers):
             norms = {}
             for slot, nspec in layer.norms:
@@ -172,6 +173,13 @@ class CausalLM:
             out.append({name: (tuple(dims), self.rt.dtype if dt is None else dt)
                         for name, (dims, dt) in shapes.items()} or None)
         return out
+
+    def step_paths(self, lens: Sequence[int]) -> tuple:
+        """What the mixers choose for a step whose sequences bring ``lens`` tokens (``Mixer.step_path``)."""
+        if self._choosers is None:
+            alike = {(type(m), getattr(m, "spec", m)): m for m in self.mixers if m is not None and m.step_path([1]) is not None}
+            self._choosers = list(alike.values())
+        return tuple(m.step_path(lens) for m in self._choosers)
 
     def reserve(self, tokens: int, seqs: int) -> None:
         """Sizes the mixers' scratch for any cut of up to ``tokens`` tokens into up to ``seqs`` sequences."""

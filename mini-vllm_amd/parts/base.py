@@ -517,6 +517,11 @@ class Mixer(Part):
         one = cls.state_shape(spec)
         return {} if one is None else {"state": one}
 
+    def step_path(self, lens: Sequence[int]):
+        """What this mixer chooses by how many tokens each sequence brings to a step (``lens``), or None. Steps with another
+        choice get recordings of their own."""
+        return None
+
     def reserve(self, tokens: int, seqs: int) -> None:
         """Sizes the scratch (``rt.workspace``) whose need depends on how a step is cut, for any cut of up to ``tokens``
         tokens into up to ``seqs`` sequences. (What depends on the number of tokens alone, a run of that many sizes.)"""

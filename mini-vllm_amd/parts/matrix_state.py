@@ -42,7 +42,7 @@ whatever the activation type. All projections of the mixer's input are one packe
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import Dict, Optional, Tuple
+from typing import Dict, Optional, Sequence, Tuple
 
 import torch
 
@@ -53,25 +53,42 @@ from .base import Mixer, PartSpec, Runtime, TensorDecl, register_mixer
 
 # In a step that brings short requests too both paths run, one behind the other (a scan of up to 127 tokens, 28 us, and the
 # chunks' two kernels, 20 us and more), where the scan alone takes 0.22 us a token of the longest. So such a step takes the
-# chunks only for longer requests, or, recorded for a class of steps, in classes large enough to hold them (us a step, Bolapel
-# 0.6B, both paths against the scan alone: prompts of 40 to 227 tokens 4,829 / 4,323, two of 120 beside eight decoding
-# 4,628 / 4,072; five of 400 on average 7,364 / 7,939).
+# chunks only for longer requests (us a step, Bolapel 0.6B, both paths against the scan alone: prompts of 40 to 227 tokens
+# 4,829 / 4,323, two of 120 beside eight decoding 4,628 / 4,072; five of 400 on average 7,364 / 7,939).
 CHUNKS_BESIDE_SHORT = 384
+# ... and a recording that has to serve any cut, in classes large enough to hold them.
 CHUNKS_BESIDE_SHORT_CLASS = 1024
+
+
+def _paths(ops, rule: str, dk: int, dv: int, lens: Sequence[int]) -> Tuple[bool, bool]:
+    """Whether the requests of many tokens go in chunks, and whether any requests are scanned."""
+    line = ops.delta_chunk_line()
+    short = any(0 < q < line for q in lens)
+    if max(lens, default=0) < (CHUNKS_BESIDE_SHORT if short else line) or not ops.delta_chunks_serve(rule, dk, dv):
+        return False, True
+    return True, short
 
 
 def recurrence(rt: Runtime, ctx, rule: str, n: int, heads: int, dk: int, dv: int, raw: torch.Tensor, scan, chunks, *operands) -> None:
     """A mixer's recurrence over the step's rows into ``raw``: requests of many tokens as products over chunks of tokens
     (``chunks``, None: not in this engine), the others, and heads of sizes these do not take, token by token (``scan``)."""
     ops, ws, plan = rt.ops, rt.workspace, ctx.attention_plan
-    line = ops.delta_chunk_line()
-    least = line if plan is None or not plan.has_short(line) else CHUNKS_BESIDE_SHORT_CLASS if plan.bound is not None else CHUNKS_BESIDE_SHORT
-    if plan is None or chunks is None or not plan.has_long(least) or not ops.delta_chunks_serve(rule, dk, dv):
+    if plan is None or chunks is None:
         scan(*operands, raw)
         return
-    chunks(*operands, *_chunk_scratch(ws, rule, n, heads, dk, dv, plan.units(ops.delta_chunk_tokens(), line)), raw)
-    if plan.has_short(line):
-        scan(*operands, raw, below=line)
+    line = ops.delta_chunk_line()
+    if plan.bound is None or plan.path_lens:
+        in_chunks, scanned = _paths(ops, rule, dk, dv, plan.q_lens if plan.bound is None else plan.path_lens)
+    else:
+        short = plan.has_short(line)
+        in_chunks = plan.has_long(CHUNKS_BESIDE_SHORT_CLASS if short else line) and ops.delta_chunks_serve(rule, dk, dv)
+        scanned = short or not in_chunks
+    if in_chunks:
+        chunks(*operands, *_chunk_scratch(ws, rule, n, heads, dk, dv, plan.units(ops.delta_chunk_tokens(), line)), raw)
+        if scanned:
+            scan(*operands, raw, below=line)
+    else:
+        scan(*operands, raw)
 
 
 def _chunk_scratch(ws, rule: str, n: int, heads: int, dk: int, dv: int, units: int):
@@ -89,10 +106,14 @@ class ChunkedRecurrence(Mixer):
         not on how it is cut or what else is in the step, and which requests go in chunks depends on both."""
         return None if self.rt.dtype == torch.float32 else entry
 
+    def step_path(self, lens: Sequence[int]):
+        rule, _, dk, dv = self.recurrence_sizes
+        return None if self.chunks(rule) is None else _paths(self.rt.ops, rule, dk, dv, lens)
+
     def reserve(self, tokens: int, seqs: int) -> None:
         (rule, heads, dk, dv), ops = self.recurrence_sizes, self.rt.ops
         line = ops.delta_chunk_line()
-        if self.rt.dtype != torch.float32 and tokens >= line and ops.delta_chunks_serve(rule, dk, dv):
+        if self.chunks(rule) is not None and tokens >= line and ops.delta_chunks_serve(rule, dk, dv):
             _chunk_scratch(self.rt.workspace, rule, tokens, heads, dk, dv, most_units(tokens, seqs, ops.delta_chunk_tokens(), line))
 
 
