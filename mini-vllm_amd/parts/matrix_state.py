@@ -60,13 +60,37 @@ CHUNKS_BESIDE_SHORT = 384
 CHUNKS_BESIDE_SHORT_CLASS = 1024
 
 
-def _paths(ops, rule: str, dk: int, dv: int, lens: Sequence[int]) -> Tuple[bool, bool]:
+# A scan takes the time of its longest request, however many requests and heads walk beside it, until they fill the chip; the
+# chunks' kernels write, read and multiply matrices for every chunk and head, so their time grows with both. What the two
+# take (us, by key channels): a token of the longest request scanned; the chunks' two kernels, and a token of the longest
+# there; nanoseconds a token and head there. Fitted to 18 cuts of 128 to 8,192 tokens, for 16 and 64 heads: the smaller of
+# the two was chosen to within 3 % of the scan everywhere and missed up to 18 % of the chunks' gain where the two are close.
+# Measured, scan / chunks: 64 requests of 128 tokens, 16 heads of 64, general rule 198 / 405, per-head decay 141 / 278, sum
+# 140 / 168, channel decays 151 / 285; four of 512, 64 heads 235 / 361, 171 / 236, 167 / 151, 167 / 247; one of 2,048,
+# 64 heads 450 / 342, 476 / 216, 411 / 155, 474 / 230; 16 of 256, 16 heads of 128 442 / 548, 237 / 512, 227 / 225, 274 / 525.
+_SCAN_TOKEN = {64: 0.22, 128: 0.32}
+_CHUNKS_ONCE = {64: (18.0, 0.013), 128: (29.0, 0.018)}
+_CHUNKS_TOKEN_HEAD = {"delta": {64: 2.4, 128: 7.6}, "gated": {64: 1.55, 128: 7.0}, "channel": {64: 1.6, 128: 7.1},
+                      "sum": {64: 1.0, 128: 3.1}}
+
+
+def _chunk_tokens_worth(rule: str, heads: int, dk: int, dv: int, longest: int, longest_scanned: int = 0) -> float:
+    """Up to how many tokens, in all the requests that go in chunks, the chunks (and a scan of the others beside them) take
+    less time than a scan of all."""
+    once, token = _CHUNKS_ONCE[dk]
+    if longest_scanned:
+        once += 3.0 + _SCAN_TOKEN[dk] * longest_scanned
+    return ((_SCAN_TOKEN[dk] - token) * longest - once) * 1e3 / (_CHUNKS_TOKEN_HEAD[rule][dk] * heads * (dk + dv) / (2 * dk))
+
+
+def _paths(ops, rule: str, heads: int, dk: int, dv: int, lens: Sequence[int]) -> Tuple[bool, bool]:
     """Whether the requests of many tokens go in chunks, and whether any requests are scanned."""
     line = ops.delta_chunk_line()
-    short = any(0 < q < line for q in lens)
-    if max(lens, default=0) < (CHUNKS_BESIDE_SHORT if short else line) or not ops.delta_chunks_serve(rule, dk, dv):
+    longest, scanned = max(lens, default=0), max((q for q in lens if q < line), default=0)
+    if longest < (CHUNKS_BESIDE_SHORT if scanned else line) or not ops.delta_chunks_serve(rule, dk, dv) \
+            or sum(q for q in lens if q >= line) > _chunk_tokens_worth(rule, heads, dk, dv, longest, scanned):
         return False, True
-    return True, short
+    return True, scanned > 0
 
 
 def recurrence(rt: Runtime, ctx, rule: str, n: int, heads: int, dk: int, dv: int, raw: torch.Tensor, scan, chunks, *operands) -> None:
@@ -78,7 +102,7 @@ def recurrence(rt: Runtime, ctx, rule: str, n: int, heads: int, dk: int, dv: int
         return
     line = ops.delta_chunk_line()
     if plan.bound is None or plan.path_lens:
-        in_chunks, scanned = _paths(ops, rule, dk, dv, plan.q_lens if plan.bound is None else plan.path_lens)
+        in_chunks, scanned = _paths(ops, rule, heads, dk, dv, plan.q_lens if plan.bound is None else plan.path_lens)
     else:
         short = plan.has_short(line)
         in_chunks = plan.has_long(CHUNKS_BESIDE_SHORT_CLASS if short else line) and ops.delta_chunks_serve(rule, dk, dv)
@@ -107,14 +131,15 @@ class ChunkedRecurrence(Mixer):
         return None if self.rt.dtype == torch.float32 else entry
 
     def step_path(self, lens: Sequence[int]):
-        rule, _, dk, dv = self.recurrence_sizes
-        return None if self.chunks(rule) is None else _paths(self.rt.ops, rule, dk, dv, lens)
+        return None if self.chunks(self) is None else _paths(self.rt.ops, *self.recurrence_sizes, lens)
 
     def reserve(self, tokens: int, seqs: int) -> None:
         (rule, heads, dk, dv), ops = self.recurrence_sizes, self.rt.ops
         line = ops.delta_chunk_line()
         if self.chunks(rule) is not None and tokens >= line and ops.delta_chunks_serve(rule, dk, dv):
-            _chunk_scratch(self.rt.workspace, rule, tokens, heads, dk, dv, most_units(tokens, seqs, ops.delta_chunk_tokens(), line))
+            most = min(tokens, int(_chunk_tokens_worth(rule, heads, dk, dv, min(tokens, self.rt.max_positions))))
+            if most >= line:
+                _chunk_scratch(self.rt.workspace, rule, tokens, heads, dk, dv, most_units(most, seqs, ops.delta_chunk_tokens(), line))
 
 
 def _pack(tensors: Dict[str, torch.Tensor], names, hidden: int, what: str):
