@@ -869,6 +869,7 @@ mlstm_gates_kernel(const T* __restrict__ packed, long ld, int H, long gate_off, 
                 m = next;
             }
         }
+        if (wide && t == end - 1) *ms = m_new;                   // (exactly what the row's factors were made from)
         if (live) {
             float* g = gates + ((size_t)t * H + head) * 4;
             g[0] = expf(gf + m_prev - m_new);
@@ -877,7 +878,7 @@ mlstm_gates_kernel(const T* __restrict__ packed, long ld, int H, long gate_off, 
             g[3] = 0.f;
         }
     }
-    if (tid == 0) *ms = m;
+    if (!wide && lane == 0) *ms = m;
 }
 
 // mLSTM, the vectors of the scan: q * DK^-1/2 and k as floats, the values with a one behind them.
