@@ -912,8 +912,10 @@ extern "C" int mv_mlstm_prepare(const void* packed, long ld, int n, int n_seqs, 
     MV_REQUIRE(cap > 0.f && H <= 65535, "mlstm_prepare: bad constants");
     if (n == 0 || n_seqs == 0) return 0;
     WeightPtr ib{i_bias, weight_dtype}, fb{f_bias, weight_dtype};
+    // (a workgroup of one wave where no request can be wide: 64 single tokens of 64 heads 11.1 -> 8.7 us)
+    const int threads = dtype == MV_F32 || n < MG_LINE ? MV_WAVE : MG_THREADS;
     MV_DISPATCH_T(dtype, "mlstm_gates",
-                  hipLaunchKernelGGL(mlstm_gates_kernel<T>, dim3(n_seqs, H), dim3(MG_THREADS), 0, stream, (const T*)packed, ld, H,
+                  hipLaunchKernelGGL(mlstm_gates_kernel<T>, dim3(n_seqs, H), dim3(threads), 0, stream, (const T*)packed, ld, H,
                                      gate_off, ib, fb, cap, max_state, cu_seqlens, state_slots, gates));
     if (mv_check_launch("mlstm_gates")) return 1;
     MV_DISPATCH_T(dtype, "mlstm_prepare",
