@@ -9,12 +9,13 @@ largest (outputs of other groups cannot be chosen whatever their number). The we
 experts' scores divided by their sum (+ weight_sum_eps); the result is the weighted sum of the
 chosen experts' outputs.
 
-How it runs: in bfloat16, with widths that are multiples of 64, the chosen (token, expert) pairs are sorted by expert on the
-device, every expert's pairs are cut into tiles of up to 128 rows, and two MFMA kernels compute gate/up with the weighted
-activation and the down product for those tiles only; a last kernel sums a token's pairs in the order of choice and adds
-the identity experts' share (csrc/moe_tile.hip). Otherwise gate and up matrices of all experts form one packed product and
-all down matrices one second product; between them one kernel applies SiLU, the up factor and the router's weight (zero
-for experts that were not chosen) before the single rounding, so the second product sums exactly the chosen experts.
+How it runs: in bfloat16, with widths that are multiples of 64 and where it takes less time (``wants_pairs``: many experts of
+which few are chosen, or large steps), the chosen (token, expert) pairs are sorted by expert on the device, every expert's
+pairs are cut into tiles of up to 128 rows, and two MFMA kernels compute gate/up with the weighted activation and the down
+product for those tiles only; a last kernel sums a token's pairs in the order of choice and adds the identity experts'
+share (csrc/moe_tile.hip). Otherwise gate and up matrices of all experts form one packed product and all down matrices one
+second product; between them one kernel applies SiLU, the up factor and the router's weight (zero for experts that were not
+chosen) before the single rounding, so the second product sums exactly the chosen experts.
 That is exact and replays from graphs, but computes every expert: eight times the useful multiply-adds when a token uses an
 eighth of the experts, and every expert's bytes in a decode step. Widths that are odd multiples of 32 may take the pairs
 through plain MFMA kernels instead (``grouped``; operands straight from memory): only in steps of few rows against large
@@ -153,11 +154,26 @@ class RoutedExperts(FeedForward):
         return (spec.grouped and n * spec.top < spec.grouped_max_rows * spec.num_experts
                 and spec.expert_size * spec.hidden_size >= spec.grouped_min_weight)
 
-    def wants_pairs(self) -> bool:
-        """Whether the tiled products over the chosen pairs take these experts."""
+    def wants_pairs(self, n: int) -> bool:
+        """Whether a step of n rows goes through the tiled products over the chosen pairs (where the kernels take the sizes).
+        They save the products and weights of the experts that are not chosen, and cost one launch more and rows of tiles that
+        few pairs fill. Both sides on an MI355X (us a layer, pairs / all experts), width x expert, experts and choices:
+        always, 1024 x 768, 32 of 4: 34 / 62 at one row, 66 / 80 at 128, 131 / 406 at 2,048; 16 of 4 33 / 40, 51 / 56, 115 / 210;
+        12 of 4 32 / 37, 47 / 50, 109 / 176; 4096 x 3072, 8 of 2 66 / 233, 162 / 186, 593 / 1,108. In large steps only: 1024 x 768,
+        8 of 4 53 / 48 at 128, 69 / 78 at 1,024; 4 of 2 49 / 32 and 55 / 51, 67 / 69 at 2,048; 16 of 8 67 / 56, 116 / 142. Large experts
+        in steps that leave experts unchosen: 4096 x 3072, 8 of 4 95 / 252 at one row, 275 / 235 at 256; 4 of 2 68 / 229, 162 / 136.
+        Small mixtures, bound by launches, never: 64 x 64, 8 of 2 19 / 16 and 35 / 27; 128 x 128, 16 of 4 22 / 18, 45 / 42."""
         spec, FS = self.spec, self.spec.shared_size if self.shared_packed else 0
-        return (spec.grouped and self.rt.ops.use_fast_kernels and self.rt.dtype == torch.bfloat16
-                and not (spec.hidden_size % 64 or spec.expert_size % 64 or FS % 64) and self.w_gate_up.dtype == torch.bfloat16)
+        if not spec.grouped or not self.rt.ops.use_fast_kernels or self.rt.dtype != torch.bfloat16 \
+                or spec.hidden_size % 64 or spec.expert_size % 64 or FS % 64 or self.w_gate_up.dtype != torch.bfloat16:
+            return False
+        E, top, expert = spec.num_experts, spec.top, spec.expert_size * spec.hidden_size
+        large, shared = expert >= 4 * 1024 * 1024, 1 if FS else 0
+        if large and n * top < E:
+            return True
+        if E * expert < 1024 * 1024:
+            return False
+        return (E >= 3 * top and (E >= 12 or large)) or (E + shared >= 2 * (top + shared) and n * E >= 8192)
 
     def _pairs(self, x: torch.Tensor, dense, ids, weights, y) -> bool:
         """The chosen (token, expert) pairs only, a packed shared expert among them. False: the sizes are not served."""
@@ -208,7 +224,7 @@ class RoutedExperts(FeedForward):
         ids = ws.get("moe.ids", (n, spec.top), torch.int32)
         weights = ws.get("moe.weights", (n, spec.top), torch.float32)
         by_table = spec.router == "table"
-        pairs = bool(n_e) and self.wants_pairs()
+        pairs = bool(n_e) and self.wants_pairs(n)
         grouped = bool(n_e) and ops.use_fast_kernels and self.wants_grouped(n)
         if by_table and (pairs or grouped):
             ops.moe_table_route(ctx.token_ids, self.table, n_e, dense, ids, weights)
