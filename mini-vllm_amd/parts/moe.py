@@ -57,9 +57,11 @@ class RoutedExpertsSpec(PartSpec):
     keep_groups: int = 1
     correction: bool = False             # a stored number per router output added to the scores for the choice
     weight_sum_eps: float = 1e-20
-    # bfloat16, widths that are multiples of 32: the experts' products over the chosen (token, expert) pairs only, in steps
-    # with fewer than ``grouped_max_rows`` chosen rows an expert on average and experts of at least ``grouped_min_weight``
-    # elements a matrix (there a step is bound by the bytes of the experts it reads, and most experts are not chosen)
+    # bfloat16: the experts' products over the chosen (token, expert) pairs only. Widths that are multiples of 64 go in tiles
+    # where that takes less time (``RoutedExperts.wants_pairs``); other multiples of 32, and steps that the tiles leave,
+    # through plain kernels, with fewer than ``grouped_max_rows`` chosen rows an expert on average and experts of at
+    # least ``grouped_min_weight`` elements a matrix (there a step is bound by the bytes of the experts it reads, and most
+    # experts are not chosen)
     grouped: bool = True
     grouped_max_rows: float = 2.0
     grouped_min_weight: int = 4 * 1024 * 1024
@@ -132,8 +134,10 @@ class RoutedExperts(FeedForward):
                 raise ValueError(f"routed experts: the experts are stored in different dtypes {dtypes}; cannot pack them")
             # rows: every expert's gate block, then every expert's up block; the down matrices side by side. A shared
             # expert's gate and up rows come behind those and its down matrix behind the others' (one pair of products
-            # serves all), unless steps may take the chosen pairs only: then it keeps matrices and products of its own
-            self.shared_packed = bool(spec.shared_size) and not self._grouped_possible()
+            # serves all), unless steps may take the plain chosen-pairs kernels, which know no shared expert: then it keeps
+            # matrices and products of its own
+            always_tiled = self._tiled(dtypes.pop(), spec.shared_size) and self._always_pairs()
+            self.shared_packed = bool(spec.shared_size) and (always_tiled or not self._grouped_possible())
             shared_rows = [tensors["shared.gate"], tensors["shared.up"]] if spec.shared_size else []
             self.w_gate_up = torch.cat([tensors[f"gate.{e}"] for e in range(n_e)] + [tensors[f"up.{e}"] for e in range(n_e)]
                                        + (shared_rows if self.shared_packed else []), dim=0).contiguous()
@@ -154,6 +158,17 @@ class RoutedExperts(FeedForward):
         return (spec.grouped and n * spec.top < spec.grouped_max_rows * spec.num_experts
                 and spec.expert_size * spec.hidden_size >= spec.grouped_min_weight)
 
+    def _tiled(self, stored: torch.dtype, shared_size: int) -> bool:
+        """Whether the tiled products over the chosen pairs take these widths."""
+        spec = self.spec
+        return (spec.grouped and self.rt.ops.use_fast_kernels and self.rt.dtype == torch.bfloat16 and stored == torch.bfloat16
+                and not (spec.hidden_size % 64 or spec.expert_size % 64 or shared_size % 64))
+
+    def _always_pairs(self) -> bool:
+        """Experts of which the chosen ones alone take less time whatever the number of rows (see ``wants_pairs``)."""
+        E, expert = self.spec.num_experts, self.spec.expert_size * self.spec.hidden_size
+        return E * expert >= 1024 * 1024 and E >= 3 * self.spec.top and (E >= 12 or expert >= 4 * 1024 * 1024)
+
     def wants_pairs(self, n: int) -> bool:
         """Whether a step of n rows goes through the tiled products over the chosen pairs (where the kernels take the sizes).
         They save the products and weights of the experts that are not chosen, and cost one launch more and rows of tiles that
@@ -164,16 +179,11 @@ class RoutedExperts(FeedForward):
         in steps that leave experts unchosen: 4096 x 3072, 8 of 4 95 / 252 at one row, 275 / 235 at 256; 4 of 2 68 / 229, 162 / 136.
         Small mixtures, bound by launches, never: 64 x 64, 8 of 2 19 / 16 and 35 / 27; 128 x 128, 16 of 4 22 / 18, 45 / 42."""
         spec, FS = self.spec, self.spec.shared_size if self.shared_packed else 0
-        if not spec.grouped or not self.rt.ops.use_fast_kernels or self.rt.dtype != torch.bfloat16 \
-                or spec.hidden_size % 64 or spec.expert_size % 64 or FS % 64 or self.w_gate_up.dtype != torch.bfloat16:
+        if not self._tiled(self.w_gate_up.dtype, FS):
             return False
-        E, top, expert = spec.num_experts, spec.top, spec.expert_size * spec.hidden_size
-        large, shared = expert >= 4 * 1024 * 1024, 1 if FS else 0
-        if large and n * top < E:
-            return True
-        if E * expert < 1024 * 1024:
-            return False
-        return (E >= 3 * top and (E >= 12 or large)) or (E + shared >= 2 * (top + shared) and n * E >= 8192)
+        E, top, expert, shared = spec.num_experts, spec.top, spec.expert_size * spec.hidden_size, 1 if FS else 0
+        return self._always_pairs() or (expert >= 4 * 1024 * 1024 and n * top < E) \
+            or (E * expert >= 1024 * 1024 and E + shared >= 2 * (top + shared) and n * E >= 8192)
 
     def _pairs(self, x: torch.Tensor, dense, ids, weights, y) -> bool:
         """The chosen (token, expert) pairs only, a packed shared expert among them. False: the sizes are not served."""
@@ -225,7 +235,7 @@ class RoutedExperts(FeedForward):
         weights = ws.get("moe.weights", (n, spec.top), torch.float32)
         by_table = spec.router == "table"
         pairs = bool(n_e) and self.wants_pairs(n)
-        grouped = bool(n_e) and ops.use_fast_kernels and self.wants_grouped(n)
+        grouped = bool(n_e) and not FS and ops.use_fast_kernels and self.wants_grouped(n)
         if by_table and (pairs or grouped):
             ops.moe_table_route(ctx.token_ids, self.table, n_e, dense, ids, weights)
         elif by_table:

@@ -75,3 +75,52 @@ def test_widths_that_are_not_served_are_left_alone():
     for hid, F in ((96, 64), (64, 32)):
         assert not ops.moe_pairs(z(2, hid), z(2 * F, hid), z(hid, F), 1, 0, F, 0, z(2, 1, dt=torch.int32), z(2, 1, dt=torch.float32), None,
                                  z(ops.moe_pairs_ints(2, 1, 1, 0), dt=torch.int32), z(2, F), z(2, hid, dt=torch.float32), z(2, hid))
+
+
+@pytest.mark.parametrize("n", [3, 200])
+@pytest.mark.parametrize("hid, F, FS, E, identity, top, router, activation", [
+    (256, 256, 0, 16, 2, 4, "learned", "swiglu"), (256, 256, 192, 20, 0, 3, "table", "swiglu"), (256, 320, 64, 16, 0, 2, "learned", "clamped"),
+    (2048, 2048, 1024, 12, 0, 2, "table", "swiglu"), (2048, 2048, 1024, 12, 0, 2, "learned", "clamped")])
+def test_the_part_takes_its_shared_expert_along(n, hid, F, FS, E, identity, top, router, activation):
+    """The feed-forward part at widths the tiles take: the routing and one call for the pairs, a shared expert among them also
+    where the experts are large enough for the plain pairs' kernels. Against float64, choices from the part's own logits."""
+    from types import SimpleNamespace
+    from minivllm_amd.kernels.ops import get_ops
+    from minivllm_amd.parts.base import Runtime, Workspace
+    from minivllm_amd.parts.moe import RoutedExperts, RoutedExpertsSpec
+    ops = get_ops(torch.bfloat16)
+    spec = RoutedExpertsSpec(hidden_size=hid, expert_size=F, num_experts=E, identity_experts=identity, top=top, router=router, table_rows=50,
+                             shared_size=FS, activation=activation, limit=1.5 if activation == "clamped" else 0.0)
+    g = torch.Generator(device=DEV).manual_seed(n + hid)
+    w = {}
+    for name, decl in RoutedExperts.tensors(spec).items():
+        if decl.integer:
+            w[name] = torch.rand(decl.shape[0], E, generator=g, device=DEV).argsort(1)[:, :top].to(torch.int32).contiguous()
+        else:
+            w[name] = (torch.randn(decl.shape, generator=g, device=DEV) / decl.shape[1] ** 0.5).bfloat16()
+    rt = Runtime(device=torch.device(DEV), dtype=torch.bfloat16, ops=ops, workspace=Workspace(torch.device(DEV)), max_positions=64)
+    part = RoutedExperts(spec, w, rt)
+    assert part.shared_packed == bool(FS)
+    x = torch.randn(n, hid, generator=g, device=DEV).bfloat16()
+    ctx = SimpleNamespace(token_ids=torch.randint(0, 50, (n,), generator=g, device=DEV, dtype=torch.int32))
+    ops.ledger = []
+    y = part.forward(x, ctx)
+    torch.cuda.synchronize()
+    ran, ops.ledger = [e[0] for e in ops.ledger], None
+    assert ran[-1] == "mv_moe_pairs" and len(ran) == (3 if router == "learned" else 2), ran
+    ids, weights = (rt.workspace.get(name, (n, top), dt) for name, dt in (("moe.ids", torch.int32), ("moe.weights", torch.float32)))
+
+    def pair(rows, gate, up, down):
+        p, u = rows @ gate.double().T, rows @ up.double().T
+        if activation == "clamped":
+            p, u = p.clamp(max=1.5), u.clamp(-1.5, 1.5)
+            return (p * torch.sigmoid(1.702 * p) * (u + 1)) @ down.double().T
+        return (p * torch.sigmoid(p) * u) @ down.double().T
+    xd = x.double()
+    want = pair(xd, w["shared.gate"], w["shared.up"], w["shared.down"]) if FS else torch.zeros_like(xd)
+    for e in range(E + identity):
+        t, k = (ids == e).nonzero(as_tuple=True)
+        if t.numel():
+            rows = pair(xd[t], w[f"gate.{e}"], w[f"up.{e}"], w[f"down.{e}"]) if e < E else xd[t]
+            want.index_add_(0, t, weights[t, k].double()[:, None] * rows)
+    assert float((y.double() - want).abs().max() / want.abs().max()) <= 1e-2
