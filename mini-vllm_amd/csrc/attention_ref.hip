@@ -37,7 +37,7 @@ attention_ref_kernel(const T* __restrict__ q, long q_stride, T* __restrict__ out
                      const int* __restrict__ positions, const int* __restrict__ token_seq, int H, int Hkv, int D, int Dv,
                      float scale, int window, int first, const T* __restrict__ gate, long gate_stride, ScoreForm form, int vec) {
     __shared__ __attribute__((aligned(16))) float qs[AR_MAX_D];
-    __shared__ __attribute__((aligned(16))) float ps[AR_THREADS];
+    __shared__ __attribute__((aligned(16))) float ps[AR_THREADS + 4];
     __shared__ long voff[AR_THREADS];
     __shared__ float scratch[17];
 
@@ -71,6 +71,7 @@ attention_ref_kernel(const T* __restrict__ q, long q_stride, T* __restrict__ out
 #pragma unroll
     for (int i = 0; i < AR_MAX_D / AR_THREADS; ++i) acc[i] = 0.f;
 
+    const int lean = (lo - nfirst) & 3;      // a tile's keys stand as far behind a multiple of four in ps as in their pages
     for (int base = lo - nfirst; base <= hi; base += AR_THREADS) {
         const int jj0 = base + tid;
         const int j = jj0 < lo ? jj0 - (lo - nfirst) : jj0;
@@ -99,7 +100,7 @@ attention_ref_kernel(const T* __restrict__ q, long q_stride, T* __restrict__ out
         const float tmax = block_max(s, scratch);
         const float m_new = fmaxf(m, tmax);
         const float p = valid ? expf(s - m_new) : 0.f;
-        ps[tid] = p;
+        ps[lean + tid] = p;
         voff[tid] = vo;
         const float tsum = block_sum(p, scratch);  // its barriers also publish ps and voff
         const float corr = expf(m - m_new);        // first tile: exp(-inf) = 0
@@ -113,13 +114,15 @@ attention_ref_kernel(const T* __restrict__ q, long q_stride, T* __restrict__ out
                 float a = acc[i] * corr;
                 const T* vcol = v_pages + (long)d * page_size;
                 int jj = 0;
-                if (vec && base % 4 == 0 && base >= lo)      // four slots of a page a load
+                if (vec && base >= lo) {                     // four slots of a page a load, from the first multiple of four on
+                    for (; jj < ((4 - lean) & 3) && jj < cnt; ++jj) a = fmaf(ps[lean + jj], to_f(vcol[voff[jj]]), a);
 #pragma unroll 4
                     for (; jj + 4 <= cnt; jj += 4) {
-                        const float4 v4 = load4(vcol + voff[jj]), p4 = *reinterpret_cast<const float4*>(&ps[jj]);
+                        const float4 v4 = load4(vcol + voff[jj]), p4 = *reinterpret_cast<const float4*>(&ps[lean + jj]);
                         a = fmaf(p4.w, v4.w, fmaf(p4.z, v4.z, fmaf(p4.y, v4.y, fmaf(p4.x, v4.x, a))));
                     }
-                for (; jj < cnt; ++jj) a = fmaf(ps[jj], to_f(vcol[voff[jj]]), a);
+                }
+                for (; jj < cnt; ++jj) a = fmaf(ps[lean + jj], to_f(vcol[voff[jj]]), a);
                 acc[i] = a;
             }
         }
