@@ -11,9 +11,9 @@
 // small. A wave of 16x16x4 products needs an operand value only once in 8 cycles, so the operands come straight from the
 // caches into registers, a block ahead of the products, without LDS; the waves of a workgroup split K instead of the tile,
 // so that a few hundred rows against a narrow weight still give every compute unit a tile with eight waves on it.
-// Measured (float, us in a model step of 221 tokens; before: a 64x64 tile of scalar multiply-adds a workgroup): N x K of
-// 1024 x 2048 and 1024 x 3072 405 -> 26, 4096 x 1024 164 -> 35, 6144 x 1024 168 -> 51; alone at 1,024 rows 24576 x 4096 runs at
-// 98 TFLOP/s, where a large library product reaches 135.
+// Measured (float, us in a model's step of 200 tokens, recorded with 224 rows; before: a 64x64 tile of scalar multiply-adds a
+// workgroup): N x K of 1024 x 2048 and 1024 x 3072 405 -> 27, 4096 x 1024 164 -> 35, 6144 x 1024 169 -> 52; alone at 1,024
+// rows 24576 x 4096 runs at 98 TFLOP/s, where a large library product reaches 135.
 #include "dispatch.h"
 
 typedef float gf_acc_t __attribute__((ext_vector_type(4)));
@@ -150,8 +150,8 @@ static void launch_tiles(const void* A, long lda, const void* W, long ldw, const
 }
 
 // The largest tile that still gives every compute unit one, since a larger one reads less a product; the bits do not depend
-// on it. Tiles of 32 x 64 where whole rounds of the chip by 64 x 64 leave it a quarter idle or more (221 x 6144 x 1024: 1.5
-// rounds, 57 us against 50), but not below 64 rows, where they are all of it (40 x 24576 x 4096: 235 us against 177).
+// on it. Tiles of 32 x 64 where whole rounds of the chip by 64 x 64 leave it a quarter idle or more (224 x 6144 x 1024: 1.5
+// rounds, 61 us against 55), but not below 64 rows, where they are all of it (40 x 24576 x 4096: 235 us against 177).
 template <typename TA, typename TW, typename TC>
 static void launch_gemm(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, long ldc,
                         int M, int N, int K, hipStream_t stream) {

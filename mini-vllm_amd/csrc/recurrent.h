@@ -124,8 +124,7 @@ conv_state_kernel(const T* __restrict__ packed, long ld, int C, int taps, T* __r
 // registers and a row's input is read once for all the taps it falls under. The sums are those of one row alone, term by term.
 // A prompt's rows are bound by how many loads are on their way, not by their bytes: a workgroup a (row, head) took 63 us for
 // 2,048 rows of 24 heads (gated delta rule) and 8 rows by a workgroup of 128, half of them idle at 64 channels, 38 us for
-// 1,600 rows of 32 heads (channel decays); a wave for 8 rows of a head takes 18.7
-// and 23.9 us.
+// 1,536 rows of 16 heads in 16 groups (channel decays); a wave for 8 rows of a head takes 18.7 and 28.4 us.
 // ---------------------------------------------------------------------------------------
 #define CP_ROWS 8
 

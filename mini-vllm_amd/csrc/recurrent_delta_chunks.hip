@@ -21,7 +21,7 @@
 // for a head count of 16; the chunks' work is spread over every compute unit and the chain is one product of DK x DK with
 // DK x 16 a chunk. Measured on one prompt of
 // 2,048 tokens, 16 heads of 64 x 64 (us, scan against the two kernels here): GENERAL 438 -> 68 + 57, GATED 477 -> 41 + 58,
-// SUM with 65 columns 411 -> 30 + 36; CHANNEL on prompts of 1,137 and 463 tokens 216 -> 36 + 31. The chunk kernel waits for
+// SUM with 65 columns 411 -> 30 + 36; CHANNEL on prompts of 941 and 483 tokens 215 -> 36 + 31. The chunk kernel waits for
 // its own phases (eight waves a workgroup hide that best: four took 90, 49, 36 and 45), the walk for a round of matrix unit,
 // LDS and barrier a chunk, 0.9 us.
 //
@@ -32,9 +32,10 @@
 #define DC_TOKENS 32
 #define DC_RUN 16                  // half a chunk: two runs
 // Requests with fewer tokens of a step are left to the scans. There a token's bits do not depend on how the request was cut;
-// here they depend on where the chunks lie. A
-// scan of 128 tokens takes 28 us, the two kernels for one such request about 15: the line lies where there is something to
-// gain, and above the portions that are worth having bit for bit.
+// here they depend on where the chunks lie, and which steps come here depends on all of a step's requests and heads
+// (parts/matrix_state.py weighs both paths), so a bfloat16 request's sums may be added in another order in other company.
+// The float32 engine scans. One request of 128 tokens, 16 heads of 64, takes the scan 33 us (28 to 34 by rule) and the two
+// kernels 28 (19 to 28): the line lies where there is something to gain.
 #define DC_LINE 128
 
 enum DeltaRule { RULE_GENERAL = 0, RULE_CHANNEL = 1, RULE_GATED = 2, RULE_SUM = 3 };

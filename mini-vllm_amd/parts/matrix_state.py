@@ -53,8 +53,9 @@ from .base import Mixer, PartSpec, Runtime, TensorDecl, register_mixer
 
 # In a step that brings short requests too both paths run, one behind the other (a scan of up to 127 tokens, 28 us, and the
 # chunks' two kernels, 20 us and more), where the scan alone takes 0.22 us a token of the longest. So such a step takes the
-# chunks only for longer requests (us a step, Bolapel 0.6B, both paths against the scan alone: prompts of 40 to 227 tokens
-# 4,829 / 4,323, two of 120 beside eight decoding 4,628 / 4,072; five of 400 on average 7,364 / 7,939).
+# chunks only for longer requests (us, 16 heads of 64, the scan alone / both paths: requests of 400, 300 and 150 tokens
+# beside 17 single ones, general rule 100 / 77, per-head decay 94 / 64, sum 86 / 51, channel decays 97 / 65; of 230, 176 and
+# 90 tokens 63 / 69, 58 / 66, 54 / 53, 59 / 67).
 CHUNKS_BESIDE_SHORT = 384
 # ... and a recording that has to serve any cut, in classes large enough to hold them.
 CHUNKS_BESIDE_SHORT_CLASS = 1024
