@@ -8,7 +8,8 @@
 // them, and what is left is LDS, 288 KB of operands a block. (Two tokens a wave share the operands too, but their 128
 // accumulators and 80 registers of queries do not fit beside anything else: the moves between the register files took
 // 4.7 us a block, 305 us for 2,048 tokens.) One request of 2,048 tokens, 16 heads, a latent of 256 and 64 rotary channels:
-// 290 us a launch with a wave a (row, 16 heads), 143 us here, 270 TFLOP/s of what causality leaves.
+// 290 us a launch with a wave a (row, 16 heads), 143 us here, 270 TFLOP/s of what causality leaves. Short contexts, and steps
+// whose many decoding requests would need rounds of workgroups with one busy wave each, stay there (Ops.latent_shares).
 //
 // Blocks lie at multiples of 32 positions, so the order of additions depends on a query's position (and window) alone. Keys are
 // masked in S; a block's slots outside the keys that the workgroup's tokens see (they may hold anything) are zeroed in LDS.

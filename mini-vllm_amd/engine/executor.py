@@ -560,7 +560,7 @@ class Executor:
         cap = min(cap, max(self.config.max_model_len, 1))
         widths = [self.max_pages_per_seq] * len(self.groups)
         arr, off, facts = self._fill(seqs, pad_to=Sp, pad_tokens=Np, pad_rows=Mp, bt_widths=widths)
-        key = (Np, Sp, Mp, cap) + self.model.step_paths(facts["q_lens"])
+        key = (Np, Sp, Mp, cap) + self.model.step_paths(facts["q_lens"], [s.start for s in seqs])
         entry = self._mixed_graphs.pop(key, None)
         if entry is None:
             entry = self._capture(Sp, cap, arr, off, facts, seqs, mixed_key=key)
@@ -873,7 +873,7 @@ class Executor:
                 plan.decode_only, plan.max_q_len, plan.q_lens = False, mixed_key[0], ()
                 plan.bound = (mixed_key[0], mixed_key[1])
                 plan.bound_least = max((b for b in TOKEN_BUCKETS if b < mixed_key[0]), default=0) + 1
-                plan.path_lens = tuple(facts["q_lens"])
+                plan.path_lens, plan.path_starts = tuple(facts["q_lens"]), tuple(s.start for s in seqs)
                 ctx.q_lens = ctx.starts = ctx.host_state_slots = None
             else:
                 # ... and any number of sequences up to the bucket, of which this step may fill only some

@@ -78,16 +78,23 @@ class AttentionPlan:
     bound: Optional[tuple] = None
     # ... whose steps hold at least this many tokens
     bound_least: int = 1
-    # ... and for which every part that chooses by the sequences' lengths (``Mixer.step_path``) chooses as for these
+    # ... and for which every part that chooses by the sequences' lengths and places (``Mixer.step_path``) chooses as for these
     path_lens: Sequence[int] = ()
+    path_starts: Sequence[int] = ()
     # for measurement: keys in the cache of the step's sequences after the step (summed), and the
     # number of (query, visible key) pairs without windows
     kv_tokens: int = 0
     attention_pairs: int = 0
-    # for measurement: the position of each sequence's first token of the step and its number of tokens, on the
+    # the position of each sequence's first token of the step and, for measurement, its number of tokens, on the
     # host (a recording for a size class clears ``q_lens``; these stay those of the step that was recorded)
     starts: Sequence[int] = ()
     step_q_lens: Sequence[int] = ()
+
+    def cut(self) -> tuple:
+        """Tokens and first positions of the sequences by which parts may choose: the step's own, or those that stand for a
+        recording's; both empty where neither is known."""
+        lens, starts = (self.q_lens, self.starts) if self.bound is None else (self.path_lens, self.path_starts)
+        return (lens[:len(starts)], starts) if starts else ((), ())
 
     def units(self, unit_tokens: int, least: int = 1) -> int:
         """Runs of up to ``unit_tokens`` consecutive tokens of one sequence in the step, of the sequences that

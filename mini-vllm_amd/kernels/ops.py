@@ -5,11 +5,13 @@ the HIP library on the current stream. Tensors must live on the GPU: there is no
 """
 from __future__ import annotations
 
-from typing import Optional
+from typing import Optional, Sequence
 
 import math
+import operator
 import os
 
+import numpy as np
 import torch
 
 from . import library
@@ -1441,7 +1443,8 @@ class Ops:
         [heads]: the softmax's denominator has one more term exp(sink[h]). Steps of single tokens take the kernel that deals a row's keys out over workgroups;
         in bfloat16 other steps take an MFMA kernel where one serves the sizes (they read the values from ``pages_t``
         [pages, kv_rank, page_size], the latents with a page's slots side by side), the one that shares key rows among neighbouring
-        tokens where a request brings several (its rows then stand at neighbouring positions); everything else the general kernel."""
+        tokens where a request brings several (its rows then stand at neighbouring positions) and ``latent_shares`` says so;
+        everything else the general kernel."""
         _dev(q, "latent queries"); _dev(out, "latent attention output"); self._act(pages, "latent pages")
         n, dk = q.shape[0], kv_rank + rot_dim
         if q.dtype != torch.float32 or tuple(q.shape) != (n, heads, dk) or not q.is_contiguous():
@@ -1473,7 +1476,8 @@ class Ops:
         fast = pages_t is not None and self.use_fast_kernels and not (plan is not None and plan.decode_only)
         # (a request that fills a workgroup's tokens; with less, a wave for every row is all the sharing there is)
         unit = int(self.lib.dll.mv_attention_latent_prompt_tokens()) if self.lib.has("mv_attention_latent_prompt") else 0
-        if fast and unit and plan is not None and plan.cu_seqlens is not None and plan.has_long(unit):
+        if fast and unit and plan is not None and plan.cu_seqlens is not None and plan.has_long(unit) \
+                and self.latent_shares(heads, w, *plan.cut()):
             units = plan.units(unit)
             self._ints(n, cu_seqlens=(plan.cu_seqlens, plan.n_seqs + 1))
             if self.lib.offer("mv_attention_latent_prompt", q.data_ptr(), heads * dk, out.data_ptr(), heads * kv_rank, pages.data_ptr(),
@@ -1496,6 +1500,35 @@ class Ops:
         self.lib.call("mv_attention_latent", q.data_ptr(), heads * dk, out.data_ptr(), heads * kv_rank, pages.data_ptr(),
                       block_table.data_ptr(), block_table.shape[1], page_size, positions.data_ptr(), token_seq.data_ptr(),
                       n, heads, kv_rank, rot_dim, float(scale), w, _ptr(sink), self.code, self._stream())
+
+    def latent_shares(self, heads: int, window: int, lens: Sequence[int], starts: Sequence[int]) -> bool:
+        """Whether the workgroups of a step with prompt portions share key rows among eight tokens of a request (requests of
+        ``lens`` tokens from positions ``starts`` on; nothing known of them: yes), or every (row, 16 heads) is a wave of its own.
+        A workgroup holds a compute unit, and a request's one decoded token holds it as long as eight, so many such requests and
+        heads come in rounds, where waves of their own stand beside each other. It also takes 4 us longer to its first key.
+        Both times as fitted to 78 cuts each of 16 and 64 heads, latents of 256 + 64 and of 128; chosen so they are on average 0.6 %
+        above the better one of both. Measured on an MI355X (us, 256 + 64, shared / apart): one prompt of 20 tokens 12.3 / 8.6, 64
+        14.5 / 12.6, 128 19.0 / 20.2, 800 63 / 100; 16 heads, 8 requests decoding at 1,900 beside 16 tokens 98 / 284, 300 at 40 25.7 /
+        14.1, 300 at 1,900 204 / 423; 64 heads, 100 decoding at 1,000 117 / 160, 200 at 300 99 / 61, 300 at 1,000 301 / 233."""
+        if not lens:
+            return True
+        units, blocks, tokens = self.compute_units, -(-heads // 16), sum(lens)
+        far = 1 << 30 if window < 0 else window + 8
+        longest = min(max(map(operator.add, starts, lens)), far)
+        if max(lens) < 8 or (longest <= 64 and blocks * tokens < 4 * units):
+            return False
+        if blocks * (tokens // 8 + len(lens)) <= units:             # (at most: one round)
+            return True
+        q, s = np.asarray(lens), np.asarray(starts)
+        of_request = (q + 7) // 8
+        groups = blocks * int(of_request.sum())
+        if groups <= units:
+            return True
+        # blocks of 32 keys that workgroups and that rows walk, by the middle of a request's tokens
+        keys = 1 + np.minimum(s + q // 2, far) // 32
+        of_units, of_rows = blocks * int(of_request @ keys), blocks * int(q @ keys)
+        rounds = (groups / units + -(-groups // units)) / 2         # (the last one is rarely full, and rarely the longest)
+        return rounds * (9.0 + 1.6 * of_units / groups) <= max(8.0 + 4.6 * (1 + longest // 32), 0.005 * of_rows * 256 / units)
 
     def _attention_latent_split(self, q, out, pages, pages_t, block_table, page_size, positions, token_seq, n, heads, kv_rank, rot_dim,
                                 scale, window, sink, max_context, kv_tokens) -> bool:

@@ -174,12 +174,13 @@ class CausalLM:
                         for name, (dims, dt) in shapes.items()} or None)
         return out
 
-    def step_paths(self, lens: Sequence[int]) -> tuple:
-        """What the mixers choose for a step whose sequences bring ``lens`` tokens (``Mixer.step_path``)."""
+    def step_paths(self, lens: Sequence[int], starts: Sequence[int]) -> tuple:
+        """What the mixers choose for a step whose sequences bring ``lens`` tokens from positions ``starts`` on
+        (``Mixer.step_path``)."""
         if self._choosers is None:
-            alike = {(type(m), getattr(m, "spec", m)): m for m in self.mixers if m is not None and m.step_path([1]) is not None}
+            alike = {(type(m), getattr(m, "spec", m)): m for m in self.mixers if m is not None and m.step_path([1], [0]) is not None}
             self._choosers = list(alike.values())
-        return tuple(m.step_path(lens) for m in self._choosers)
+        return tuple(m.step_path(lens, starts) for m in self._choosers)
 
     def reserve(self, tokens: int, seqs: int) -> None:
         """Sizes the mixers' scratch for any cut of up to ``tokens`` tokens into up to ``seqs`` sequences."""

@@ -517,9 +517,9 @@ class Mixer(Part):
         one = cls.state_shape(spec)
         return {} if one is None else {"state": one}
 
-    def step_path(self, lens: Sequence[int]):
-        """What this mixer chooses by how many tokens each sequence brings to a step (``lens``), or None. Steps with another
-        choice get recordings of their own."""
+    def step_path(self, lens: Sequence[int], starts: Sequence[int]):
+        """What this mixer chooses by how many tokens each sequence brings to a step (``lens``) and at which position they begin
+        (``starts``), or None. Steps with another choice get recordings of their own."""
         return None
 
     def reserve(self, tokens: int, seqs: int) -> None:

@@ -29,7 +29,7 @@ applied to the weighted sum of latents. Norms, rotation, scores, weights and sum
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import Dict, Optional, Tuple
+from typing import Dict, Optional, Sequence, Tuple
 
 import torch
 
@@ -152,6 +152,11 @@ class LatentAttention(Mixer):
         self.w_uk_rows = self.w_uk.transpose(1, 2).contiguous()
         self.w_uv_rows = tensors["uv"].view(spec.num_heads, spec.value_dim, spec.kv_rank).contiguous()
         self.w_o = tensors["o"]
+
+    def step_path(self, lens: Sequence[int], starts: Sequence[int]):
+        if self.rt.dtype == torch.float32:
+            return None
+        return self.rt.ops.latent_shares(self.spec.num_heads, -1 if self.spec.window is None else self.spec.window, lens, starts)
 
     def forward(self, x: torch.Tensor, ctx, call: int) -> torch.Tensor:
         spec, rt, ops, ws = self.spec, self.rt, self.rt.ops, self.rt.workspace

@@ -131,7 +131,7 @@ class ChunkedRecurrence(Mixer):
         not on how it is cut or what else is in the step, and which requests go in chunks depends on both."""
         return None if self.rt.dtype == torch.float32 else entry
 
-    def step_path(self, lens: Sequence[int]):
+    def step_path(self, lens: Sequence[int], starts: Sequence[int]):
         return None if self.chunks(self) is None else _paths(self.rt.ops, *self.recurrence_sizes, lens)
 
     def reserve(self, tokens: int, seqs: int) -> None:

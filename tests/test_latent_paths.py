@@ -1,0 +1,35 @@
+"""Steps with prompt portions: when the latent attention's workgroups share key rows among a request's tokens."""
+from types import SimpleNamespace
+
+import pytest
+
+from minivllm_amd.engine.step import AttentionPlan
+from minivllm_amd.kernels.ops import Ops
+
+
+@pytest.mark.parametrize("heads, prompts, decoding, want", [
+    # (tokens, first position) of prompts, (requests, position) of decoded tokens: both sides measured, at least 8 % apart
+    (16, [(20, 0)], (0, 0), False), (16, [(48, 0)], (0, 0), False), (16, [(160, 0)], (0, 0), True), (16, [(8, 200)], (0, 0), True),
+    (16, [(9, 0)] * 100, (0, 0), False), (64, [(60, 0)] * 5, (0, 0), True), (64, [(9, 0)] * 100, (0, 0), False), (64, [(128, 0)] * 16, (0, 0), True),
+    (16, [(16, 0)], (8, 1900), True), (16, [(16, 0)], (300, 40), False), (16, [(16, 0)], (300, 1000), True), (64, [(16, 0)], (100, 1000), True),
+    (64, [(16, 0)], (200, 300), False), (64, [(16, 0)], (300, 1000), False), (64, [(9, 500)] * 100, (0, 0), True),
+    (16, [(7, 500)], (8, 1900), False)])
+@pytest.mark.parametrize("window", [-1, 1 << 20])
+def test_the_kernel_that_is_faster(heads, prompts, decoding, want, window):
+    lens, starts = [1] * decoding[0] + [q for q, _ in prompts], [decoding[1] - 1] * decoding[0] + [s for _, s in prompts]
+    assert Ops.latent_shares(SimpleNamespace(compute_units=256), heads, window, lens, starts) is want
+
+
+def test_keys_in_front_of_a_window_do_not_count():
+    shares = lambda window: Ops.latent_shares(SimpleNamespace(compute_units=256), 16, window, [20], [2000])
+    assert shares(-1) and shares(500) and not shares(30)
+
+
+def test_the_cut_that_choices_follow():
+    plan = AttentionPlan(decode_only=False, max_q_len=9, max_context_len=30, n_seqs=3, q_lens=[9, 1, 0], starts=[0, 29])
+    assert plan.cut() == ([9, 1], [0, 29])
+    plan.bound, plan.q_lens = (16, 4), ()
+    assert plan.cut() == ((), ())                       # a recording that has to serve any cut
+    plan.path_lens, plan.path_starts = (9, 1), (0, 29)
+    assert plan.cut() == ((9, 1), (0, 29))
+    assert Ops.latent_shares(SimpleNamespace(compute_units=256), 16, -1, *AttentionPlan(False, 9, 30, 1, q_lens=[9]).cut())
