@@ -136,8 +136,9 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
     {
         const int n_all = gridDim.y, half = (n_all + 1) / 2;
         int u = (!fold || (int)blockIdx.y < half) ? n_all - 1 - (int)blockIdx.y : (int)blockIdx.y - half;
-        // (a step of one prompt needs no more than its first request's two numbers)
-        const int first0 = cu_seqlens[0], len0 = cu_seqlens[1] - first0;
+        // (a step of one prompt needs no more than its first request's two numbers, which come with the other lanes' own)
+        int s = lane, first = s < n_seqs ? cu_seqlens[s] : 0, len = s < n_seqs ? cu_seqlens[s + 1] - first : 0;
+        const int first0 = __builtin_amdgcn_readfirstlane(first), len0 = __builtin_amdgcn_readfirstlane(len);
         const bool in_first = u < (len0 + tpu - 1) / tpu;
         if (in_first) {
             seq = 0;
@@ -146,8 +147,11 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
             nt = nt < tpu ? nt : tpu;
         }
         for (int s0 = 0; !in_first && s0 < n_seqs; s0 += MV_WAVE) {
-            const int s = s0 + lane;
-            const int first = s < n_seqs ? cu_seqlens[s] : 0, len = s < n_seqs ? cu_seqlens[s + 1] - first : 0;
+            if (s0 > 0) {
+                s = s0 + lane;
+                first = s < n_seqs ? cu_seqlens[s] : 0;
+                len = s < n_seqs ? cu_seqlens[s + 1] - first : 0;
+            }
             const int mine = (len + tpu - 1) / tpu;
             int incl = mine;
 #pragma unroll
