@@ -31,7 +31,15 @@ __device__ __forceinline__ float4 gf_load(const T* __restrict__ row, int k, int 
             return float4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
                           __uint_as_float(u.y & 0xffff0000u)};
         }
+    } else if constexpr (!TAIL) {
+        return float4{to_f(row[k]), to_f(row[k + 1]), to_f(row[k + 2]), to_f(row[k + 3])};
     } else {
+        if constexpr (VEC) {
+            if (K % 4 == 0) {                        // all four or none
+                const float4 v = gf_load<T, true, false>(row, k < K ? k : 0, K);
+                return k < K ? v : float4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -39,6 +47,24 @@ __device__ __forceinline__ float4 gf_load(const T* __restrict__ row, int k, int 
             v[e] = k + e < K ? x : 0.f;
         }
         return float4{v[0], v[1], v[2], v[3]};
+    }
+}
+
+template <typename TW, typename TC, int RM, int RN>
+__device__ __forceinline__ void gf_store(const gf_acc_t (&acc)[RM][RN], const TW* __restrict__ bias, TC* __restrict__ C, long ldc, int m0,
+                                         int n0, int i, int g, int M, int N) {
+#pragma unroll
+    for (int c = 0; c < RN; ++c) {
+        const int n = n0 + 16 * c + i;
+        if (n >= N) continue;
+        const float add = bias ? to_f(bias[n]) : 0.f;
+#pragma unroll
+        for (int r = 0; r < RM; ++r)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int m = m0 + 16 * r + 4 * g + e;
+                if (m < M) C[(size_t)m * ldc + n] = from_f<TC>(bias ? acc[r][c][e] + add : acc[r][c][e]);
+            }
     }
 }
 
@@ -85,7 +111,8 @@ gemm_nt_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lon
     };
     if (whole > 0) {
 #pragma unroll
-        for (int d = 0; d < AHEAD; ++d) fetch(d, wave + d * GF_WAVES);
+        for (int d = 0; d < AHEAD; ++d)
+            if (VEC || wave + d * GF_WAVES < whole) fetch(d, wave + d * GF_WAVES);       // (a scalar form has loads to spare)
     }
     for (int b0 = wave; b0 < whole; b0 += AHEAD * GF_WAVES) {
 #pragma unroll
@@ -96,7 +123,7 @@ gemm_nt_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lon
                 for (int r = 0; r < RM; ++r) a[r] = an[d][r];
 #pragma unroll
                 for (int c = 0; c < RN; ++c) w[c] = wn[d][c];
-                fetch(d, b + AHEAD * GF_WAVES);      // flies under the products of the blocks between
+                if (VEC || b + AHEAD * GF_WAVES < whole) fetch(d, b + AHEAD * GF_WAVES);      // flies under the products of the blocks between
                 products();
             }
         }
@@ -111,6 +138,7 @@ gemm_nt_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lon
     // the waves' sums, pairwise: 4..7 into 0..3, 2..3 into 0..1, 1 into 0
 #pragma unroll
     for (int half = GF_WAVES / 2; half >= 1; half /= 2) {
+        if (K <= 16 * half) continue;                // (they hold zeros, which change no sum)
         if (wave >= half && wave < 2 * half)
 #pragma unroll
             for (int t = 0; t < RM * RN; ++t) part[wave - half][t][lane] = acc[t / RN][t % RN];
@@ -120,20 +148,77 @@ gemm_nt_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, lon
             for (int t = 0; t < RM * RN; ++t) acc[t / RN][t % RN] += part[wave][t][lane];
         __syncthreads();
     }
-    if (wave != 0) return;
+    if (wave == 0) gf_store<TW, TC, RM, RN>(acc, bias, C, ldc, m0, n0, i, g, M, N);
+}
+
+// The same sums, all GF_WAVES of a tile by one wave one after the other: for products of many rows and a short K, where a
+// split leaves every wave a block or two and one of eight the tile's output (4096 x 1024 x 16: 28 us -> 10).
+template <typename TA, typename TW, typename TC, int RM, int RN, bool VEC>
+struct WaveTile {
+    const TA* a_row[RM];
+    const TW* w_row[RN];
+    int K, g;
+    struct Sums { gf_acc_t t[RM][RN]; };
+
+    template <bool TAIL>
+    __device__ __forceinline__ void add(Sums& s, int b) const {
+        float4 a[RM], w[RN];
 #pragma unroll
-    for (int c = 0; c < RN; ++c) {
-        const int n = n0 + 16 * c + i;
-        if (n >= N) continue;
-        const float add = bias ? to_f(bias[n]) : 0.f;
+        for (int r = 0; r < RM; ++r) a[r] = gf_load<TA, VEC, TAIL>(a_row[r], 16 * b + 4 * g, K);
 #pragma unroll
-        for (int r = 0; r < RM; ++r)
+        for (int c = 0; c < RN; ++c) w[c] = gf_load<TW, VEC, TAIL>(w_row[c], 16 * b + 4 * g, K);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int m = m0 + 16 * r + 4 * g + e;
-                if (m < M) C[(size_t)m * ldc + n] = from_f<TC>(bias ? acc[r][c][e] + add : acc[r][c][e]);
-            }
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int r = 0; r < RM; ++r)
+#pragma unroll
+                for (int c = 0; c < RN; ++c)
+                    s.t[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float*>(&a[r])[e],
+                                                                     reinterpret_cast<const float*>(&w[c])[e], s.t[r][c], 0, 0, 0);
     }
+    // partial sums FIRST, FIRST + STEP, ..., added up as the waves' are
+    template <int FIRST, int STEP>
+    __device__ __forceinline__ void sum(Sums& s) const {
+        if constexpr (STEP == GF_WAVES) {
+#pragma unroll
+            for (int r = 0; r < RM; ++r)
+#pragma unroll
+                for (int c = 0; c < RN; ++c) s.t[r][c] = gf_acc_t{0.f, 0.f, 0.f, 0.f};
+            const int whole = K / 16;
+            int b = FIRST;
+            for (; b < whole; b += GF_WAVES) add<false>(s, b);
+            if (b == whole && K % 16 != 0) add<true>(s, b);
+        } else {
+            sum<FIRST, 2 * STEP>(s);
+            if (16 * (FIRST + STEP) < K) {           // (the others are zero)
+                Sums o;
+                sum<FIRST + STEP, 2 * STEP>(o);
+#pragma unroll
+                for (int r = 0; r < RM; ++r)
+#pragma unroll
+                    for (int c = 0; c < RN; ++c) s.t[r][c] += o.t[r][c];
+            }
+        }
+    }
+};
+
+template <typename TA, typename TW, typename TC, int RM, int RN, bool VEC>
+__global__ void __launch_bounds__(256)
+gemm_nt_wave_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw, const TW* __restrict__ bias,
+                    TC* __restrict__ C, long ldc, int M, int N, int K) {
+    const int lane = threadIdx.x % MV_WAVE, i = lane % 16, g = lane / 16;
+    const int m0 = (blockIdx.y * 4 + threadIdx.x / MV_WAVE) * (16 * RM), n0 = blockIdx.x * (16 * RN);
+    if (m0 >= M) return;
+    WaveTile<TA, TW, TC, RM, RN, VEC> tile;
+    tile.K = K;
+    tile.g = g;
+#pragma unroll
+    for (int r = 0; r < RM; ++r) tile.a_row[r] = A + (size_t)min(m0 + 16 * r + i, M - 1) * lda;
+#pragma unroll
+    for (int c = 0; c < RN; ++c) tile.w_row[c] = W + (size_t)min(n0 + 16 * c + i, N - 1) * ldw;
+    typename WaveTile<TA, TW, TC, RM, RN, VEC>::Sums s;
+    tile.template sum<0, 1>(s);
+    gf_store<TW, TC, RM, RN>(s.t, bias, C, ldc, m0, n0, i, g, M, N);
 }
 
 template <typename TA, typename TW, typename TC, int RM, int RN, int AHEAD>
@@ -149,9 +234,26 @@ static void launch_tiles(const void* A, long lda, const void* W, long ldw, const
                            (const TW*)W, ldw, (const TW*)bias, (TC*)C, ldc, M, N, K);
 }
 
+template <typename TA, typename TW, typename TC, int RM, int RN>
+static void launch_waves(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, long ldc, int M, int N, int K,
+                         hipStream_t stream) {
+    const bool vec = lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % (4 * sizeof(TA)) == 0 && (uintptr_t)W % (4 * sizeof(TW)) == 0;
+    dim3 grid((N + 16 * RN - 1) / (16 * RN), (M + 64 * RM - 1) / (64 * RM));
+    if (vec)
+        hipLaunchKernelGGL((gemm_nt_wave_kernel<TA, TW, TC, RM, RN, true>), grid, dim3(256), 0, stream, (const TA*)A, lda, (const TW*)W, ldw,
+                           (const TW*)bias, (TC*)C, ldc, M, N, K);
+    else
+        hipLaunchKernelGGL((gemm_nt_wave_kernel<TA, TW, TC, RM, RN, false>), grid, dim3(256), 0, stream, (const TA*)A, lda, (const TW*)W, ldw,
+                           (const TW*)bias, (TC*)C, ldc, M, N, K);
+}
+
 // The largest tile that still gives every compute unit one, since a larger one reads less a product; the bits do not depend
 // on it. Tiles of 32 x 64 where whole rounds of the chip by 64 x 64 leave it a quarter idle or more (224 x 6144 x 1024: 1.5
 // rounds, 61 us against 55), but not below 64 rows, where they are all of it (40 x 24576 x 4096: 235 us against 177).
+// Up to 512 values of k one wave makes a tile alone where that gives the chip two waves a compute unit, or fewer where K has
+// few blocks (us, eight waves / one: 64 x 256 x 32 8.5 / 7.9, 500 x 1024 x 128 13.4 / 11.5, 4096 x 1024 x 128 46 / 26, x 256 56 / 39,
+// 16384 x 4096 x 48 392 / 125; but 200 x 1024 x 128 10.2 / 11.2, 2000 x 1024 x 1024 64 / 70), in tiles of 32 x 64 from 128 values
+// on where these are enough (4096 x 1024 x 512 63 against 74).
 template <typename TA, typename TW, typename TC>
 static void launch_gemm(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, long ldc,
                         int M, int N, int K, hipStream_t stream) {
@@ -159,7 +261,10 @@ static void launch_gemm(const void* A, long lda, const void* W, long ldw, const 
     auto tiles = [&](int rm, int rn) { return ((M + 16L * rm - 1) / (16 * rm)) * ((N + 16L * rn - 1) / (16 * rn)); };
     // work of the unit that gets the most tiles, in tiles of 16 x 16
     auto rounds = [&](int rm, int rn) { return (tiles(rm, rn) + units - 1) / units * rm * rn; };
-    if (M > 65535 * 32 || (M > 32 && tiles(4, 4) >= units && (M <= 64 || 4 * rounds(4, 4) <= 5 * rounds(2, 4))))
+    if (M > 16 && M <= 65535 * 32 && K <= 512 && (K <= 32 || tiles(2, 2) >= (K <= 64 ? units / 2 : 2 * units))) {
+        if (K > 128 && tiles(2, 4) > 4 * units) launch_waves<TA, TW, TC, 2, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+        else launch_waves<TA, TW, TC, 2, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+    } else if (M > 65535 * 32 || (M > 32 && tiles(4, 4) >= units && (M <= 64 || 4 * rounds(4, 4) <= 5 * rounds(2, 4))))
         launch_tiles<TA, TW, TC, 4, 4, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
     else if (M > 64 && tiles(2, 4) >= units)
         launch_tiles<TA, TW, TC, 2, 4, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
