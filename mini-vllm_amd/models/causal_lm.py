@@ -108,6 +108,7 @@ class CausalLM:
         self.graph_safe = True          # every part allows its forward to be captured in a graph
         self.blocks = []
         self.mixers = []
+        self.ffns = []
         self._choosers: Optional[List] = None      # one mixer of each kind and size that chooses by a step's lengths
         for i, layer in enumerate(plan.layers):
             norms = {}
@@ -129,6 +130,7 @@ class CausalLM:
                 ffn_cls = FEED_FORWARDS.get(layer.ffn.kind)
                 ffn = ffn_cls(layer.ffn, fetch(i, "ffn", ffn_cls.tensors(layer.ffn)), rt)
             self.mixers.append(mixer)
+            self.ffns.append(ffn)
             block_cls = BLOCKS.get(layer.block.kind)
             if getattr(block_cls, "wants_runtime", False):
                 block = block_cls(layer.block, norms, mixer, ffn,
@@ -183,10 +185,13 @@ class CausalLM:
         return tuple(m.step_path(lens, starts) for m in self._choosers)
 
     def reserve(self, tokens: int, seqs: int) -> None:
-        """Sizes the mixers' scratch for any cut of up to ``tokens`` tokens into up to ``seqs`` sequences."""
+        """Sizes the scratch of mixers and feed-forwards for any cut of up to ``tokens`` tokens into up to ``seqs`` sequences."""
         for mixer in self.mixers:
             if mixer is not None:
                 mixer.reserve(tokens, seqs)
+        for ffn in self.ffns:
+            if ffn is not None:
+                ffn.reserve(tokens)
 
     # ------------------------------------------------------------------------------------
     def forward(self, ctx) -> torch.Tensor:

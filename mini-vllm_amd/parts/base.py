@@ -533,6 +533,9 @@ class Mixer(Part):
 class FeedForward(Part):
     """forward(x, ctx) -> y, token by token."""
 
+    def reserve(self, tokens: int) -> None:
+        """Sizes the scratch (``rt.workspace``) that a step of fewer than ``tokens`` tokens needs and one of so many does not."""
+
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         raise NotImplementedError
 

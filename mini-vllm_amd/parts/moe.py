@@ -183,7 +183,21 @@ class RoutedExperts(FeedForward):
             return False
         E, top, expert, shared = spec.num_experts, spec.top, spec.expert_size * spec.hidden_size, 1 if FS else 0
         return self._always_pairs() or (expert >= 4 * 1024 * 1024 and n * top < E) \
-            or (E * expert >= 1024 * 1024 and E + shared >= 2 * (top + shared) and n * E >= 8192)
+            or (E * expert >= 1024 * 1024 and E + shared >= 2 * (top + shared) and n * E >= self.LARGE_STEP)
+
+    LARGE_STEP = 8192                    # (token, expert) pairs, chosen or not, from which a step is a large one
+
+    def reserve(self, tokens: int) -> None:
+        # a step of ``tokens`` may take the chosen pairs where a smaller one takes all experts
+        for n in (tokens, min(tokens, (self.LARGE_STEP - 1) // max(1, self.spec.num_experts))):
+            if n > 0 and self.spec.num_experts and not self.wants_pairs(n):
+                self._all_experts_scratch(n)
+                return
+
+    def _all_experts_scratch(self, n: int):
+        spec, rt = self.spec, self.rt
+        F, FS = spec.num_experts * spec.expert_size, spec.shared_size if self.shared_packed else 0
+        return rt.workspace.get("moe.gate_up", (n, 2 * F + 2 * FS), rt.dtype), rt.workspace.get("moe.act", (n, F + FS), rt.dtype)
 
     def _pairs(self, x: torch.Tensor, dense, ids, weights, y) -> bool:
         """The chosen (token, expert) pairs only, a packed shared expert among them. False: the sizes are not served."""
@@ -252,9 +266,8 @@ class RoutedExperts(FeedForward):
                 self._add_shared(x, y)
             return y
         if n_e:
-            gu = ws.get("moe.gate_up", (n, 2 * n_e * F + 2 * FS), rt.dtype)
+            gu, act = self._all_experts_scratch(n)
             ops.gemm(x, self.w_gate_up, gu)
-            act = ws.get("moe.act", (n, n_e * F + FS), rt.dtype)
             table = (ctx.token_ids, self.table) if by_table else None
             if spec.activation == "clamped":
                 ops.moe_swiglu_scale(gu, None if by_table else dense, n_e, F, act, limit=spec.limit, slope=spec.gate_slope,
