@@ -38,7 +38,7 @@ KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_gemm_skinny_fold": (r"\bgemm_skinny_kernel", None, 1),
     "mv_gemm_skinny_scaled": (r"\bgemm_skinny_kernel", None, 1),
     "mv_scale_rows": (r"\bscale_rows_kernel", None, 1),
-    "mv_gemm_ref": (r"\bgemm_nt_kernel", None, 1),
+    "mv_gemm_ref": (r"\bgemm_nt(_wave)?_kernel", None, 1),
     "mv_gemm_mid": (r"\bgemm_mid_kernel", r"\bgemm_mid_reduce_kernel", 2),
     "mv_gemm_tile": (r"\bgemm_tile_kernel", r"\bgemm_mid_reduce_kernel", 2),
     "mv_gemm_lt": (_LIBRARY, _LIBRARY, 3),
