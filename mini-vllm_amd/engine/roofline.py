@@ -56,7 +56,7 @@ KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_soft_cap": (r"\bsoft_cap_kernel", None, 1),
     "mv_attention_sigmoid_ref": (r"\battention_sigmoid_kernel", None, 1),
     "mv_attention_prefill_sigmoid": (r"\battention_prefill_kernel", None, 1),
-    "mv_gdelta_prepare": (r"\bgdelta_prepare_kernel", r"\bconv_state_kernel", 2),
+    "mv_gdelta_prepare": (r"\bgdelta_prepare(_rows)?_kernel", r"\bconv_state_kernel", 2),
     "mv_mlstm_prepare": (r"\bmlstm_gates_kernel", r"\bmlstm_prepare_kernel", 2),
     "mv_state_scan": (r"\bstate_scan_kernel", None, 1),
     "mv_delta_chunks": (r"\bdelta_chunk_kernel", r"\bdelta_chunk_walk_kernel", 2),
