@@ -273,6 +273,10 @@ attention_latent_prompt_kernel(AlpArgs a) {
 }
 
 extern "C" int mv_attention_latent_prompt_tokens() { return ALP_TOKENS; }
+// 1: a latent of R numbers and DR rotary channels is served
+extern "C" int mv_attention_latent_prompt_serves(int R, int DR) {
+    return (DR == 0 && (R == 64 || R == 128 || R == 192 || R == 256)) || (DR == 64 && (R == 128 || R == 256));
+}
 
 // `units`: the runs of ALP_TOKENS tokens of the step's requests, or an upper bound (the rest of the grid ends at once). A
 // request's rows stand at neighbouring positions. `padding`: there may be rows of no request; they become zeros. Returns 2 (nothing done) for sizes it does not serve.
@@ -281,8 +285,7 @@ extern "C" int mv_attention_latent_prompt(const float* q, long ldq, float* out, 
                                           const int* cu_seqlens, int n_seqs, int units, int n, int padding, int H, int R, int DR, float scale,
                                           int window, const float* sink, hipStream_t stream) {
     MV_REQUIRE(n >= 0 && n_seqs >= 0 && units >= 0 && H > 0 && R > 0 && DR >= 0, "attention_latent_prompt: bad sizes n=%d H=%d R=%d DR=%d", n, H, R, DR);
-    const bool plain = DR == 0 && (R == 64 || R == 128 || R == 192 || R == 256);
-    if (!(plain || (R == 128 && DR == 64) || (R == 256 && DR == 64)) || page_size % 8 || !pages_t || (uintptr_t)pages % 16
+    if (!mv_attention_latent_prompt_serves(R, DR) || page_size % 8 || !pages_t || (uintptr_t)pages % 16
         || (uintptr_t)pages_t % 16)
         return 2;
     MV_REQUIRE(bt_width > 0 && ldq >= (long)H * (R + DR) && ldo >= (long)H * R && H <= 65535 * 16, "attention_latent_prompt: pitches too small");

@@ -195,6 +195,7 @@ _OPTIONAL_SIGNATURES = {
     "mv_attention_latent_mfma": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
                                          c_void_p, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p]),
     "mv_attention_latent_prompt_tokens": (c_int, []),
+    "mv_attention_latent_prompt_serves": (c_int, [c_int, c_int]),
     # q, ldq, out, ldo, pages, pages_t, block_table, bt_width, page_size, positions, token_seq, cu_seqlens, n_seqs, units, n, padding,
     # H, R, DR, scale, window, sink, stream
     "mv_attention_latent_prompt": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,

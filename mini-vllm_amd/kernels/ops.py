@@ -1501,6 +1501,11 @@ class Ops:
                       block_table.data_ptr(), block_table.shape[1], page_size, positions.data_ptr(), token_seq.data_ptr(),
                       n, heads, kv_rank, rot_dim, float(scale), w, _ptr(sink), self.code, self._stream())
 
+    def latent_shares_serve(self, kv_rank: int, rot_dim: int) -> bool:
+        """Whether ``attention_latent`` has a kernel for latents of these sizes whose workgroups share key rows."""
+        return self.use_fast_kernels and self.lib.has("mv_attention_latent_prompt") \
+            and bool(self.lib.dll.mv_attention_latent_prompt_serves(kv_rank, rot_dim))
+
     def latent_shares(self, heads: int, window: int, lens: Sequence[int], starts: Sequence[int]) -> bool:
         """Whether the workgroups of a step with prompt portions share key rows among eight tokens of a request (requests of
         ``lens`` tokens from positions ``starts`` on; nothing known of them: yes), or every (row, 16 heads) is a wave of its own.

@@ -154,7 +154,7 @@ class LatentAttention(Mixer):
         self.w_o = tensors["o"]
 
     def step_path(self, lens: Sequence[int], starts: Sequence[int]):
-        if self.rt.dtype == torch.float32:
+        if not self.rt.ops.latent_shares_serve(self.spec.kv_rank, self.spec.rot_dim):
             return None
         return self.rt.ops.latent_shares(self.spec.num_heads, -1 if self.spec.window is None else self.spec.window, lens, starts)
 

@@ -51,3 +51,12 @@ def test_kernels_of_recorded_steps():
             assert float((got - plain).abs().max() / plain.abs().max()) <= 2e-2, cut
     # (the third step has the choice of the first, and its recording)
     assert len(recorded.graph_ledger) == 5
+
+
+def test_sizes_without_a_choice_are_recorded_once():
+    """Latents that the sharing kernel does not take, and the float32 engine, have no choice to make."""
+    from minivllm_amd.kernels.ops import get_ops
+    ops = get_ops(torch.bfloat16)
+    assert all(ops.latent_shares_serve(*sizes) for sizes in ((64, 0), (128, 0), (192, 0), (256, 0), (128, 64), (256, 64)))
+    assert not any(ops.latent_shares_serve(*sizes) for sizes in ((64, 32), (128, 32), (192, 64), (16, 4), (512, 64)))
+    assert not get_ops(torch.float32).latent_shares_serve(256, 64)
