@@ -8,7 +8,8 @@
 //   out^T    = V^T P^T   which is what the second product takes: nothing is exchanged between the two.
 // Maximum, sum and accumulator are float, and nothing is rounded between. Blocks lie at multiples of 16 positions and a wave's
 // blocks do not depend on the request, so a row's bits depend on its position alone: what a unit's later tokens see beyond
-// it adds zeros.
+// it adds zeros. (Where a later value of the block is no number, the products of the block are added up one by one instead: the
+// row keeps its value to rounding.)
 //
 // What bounds it: the round trips of a workgroup's start (the request's place, page ids, keys), then the lines of keys that a
 // compute unit asks for; the kernel of a workgroup a (token, head) reads every key row once for every query row. A prompt of
@@ -210,9 +211,10 @@ attention_exact_kernel(const float* __restrict__ q, long q_stride, float* __rest
     ax_acc_t o{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < AX_WAVES; ++w) {
-        const float mw = sm_m[w][i];
-        if (mw == -INFINITY) continue;                // no key of this wave's is seen
-        const float f = expf(mw - top);
+        // No key of this wave's is seen. (Its maximum does not say so: fmaxf passes over scores that are no numbers, and a wave that
+        // sees nothing else keeps minus infinity, with the sum that has to come through.)
+        if (AX_KEYS * w > pos) continue;
+        const float f = expf(sm_m[w][i] - top);
         total += f * sm_l[w][i];
         o += f * sm_o[w][wave][lane];
     }
