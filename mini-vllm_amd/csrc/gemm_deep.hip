@@ -297,7 +297,7 @@ static int deep_launch(const char* what, DeepArgs p, int shape, hipStream_t stre
 }
 
 // C[M, N] = A W^T (+ bias), or with `gated` C[M, N / 2] = pair(A Wg^T (+ bias), A Wu^T (+ bias)) for the packed weight [N, K]; bf16 A
-// (row stride lda) and W (contiguous rows of K), C bf16 or float. With `partial` [M, P] output row m is first divided by
+// (row stride lda) and W (contiguous rows of K), C bf16 or float (the entry points in front of this one keep float outputs). With `partial` [M, P] output row m is first divided by
 // sqrt(sum_p partial[m][p] / K + eps). square_relu: C = max(., 0)^2. shape: see deep_tiles; 0 lets the rule choose.
 extern "C" int mv_gemm_deep(const void* A, long lda, const void* W, const void* bias, void* C, long ldc, int c_dtype, int M, int N, int K,
                             int gated, const float* partial, int P, float eps, float limit, float slope, int square_relu, int shape,

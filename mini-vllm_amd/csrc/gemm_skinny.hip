@@ -675,9 +675,9 @@ extern "C" int mv_gemm_skinny(const void* A, long lda, const void* W, long ldw, 
     MV_REQUIRE(ldw == K, "gemm_skinny: the weight must be contiguous (ldw=%ld, K=%d)", ldw, K);
     MV_REQUIRE(c_dtype == MV_F32 || c_dtype == MV_BF16, "gemm_skinny: bad output dtype %d", c_dtype);
     if (M == 0) return 0;
-    // (float outputs, scores that choices are made by, keep one order of additions for every number of rows: that product takes
-    // small weights from some number of rows on)
-    if (mv_gemm_deep_shape(M, N, K, 0) && (c_dtype == MV_BF16 || mv_gemm_deep_shape(1, N, K, 0)))
+    // (float outputs, scores that choices are made by, stay here: that product takes small weights from some number of rows on, and
+    // adds in another order)
+    if (c_dtype == MV_BF16 && mv_gemm_deep_shape(M, N, K, 0))
         return mv_gemm_deep(A, lda, W, bias, C, ldc, c_dtype, M, N, K, 0, nullptr, 0, 0.f, 0.f, 1.f, square_relu, 0, stream);
     int S, R, rows;
     skinny_shape(M, N, K, S, R, rows);

@@ -406,8 +406,9 @@ static int tile_launch(const void* A, long lda, const void* W, const void* bias,
     MV_REQUIRE(ldc >= (gated ? N / 2 : N), "gemm_tile: ldc=%ld too small for N=%d", ldc, N);
     MV_REQUIRE((long)M * N < (1L << 31), "gemm_tile: %d x %d outputs exceed the index range", M, N);
     const TilePlan p = tile_plan(M, gated ? N / 2 : N, K, gated != 0, force);
-    // (a split K stays here: its sums may go straight into the norm behind the product, and have the same bits either way)
-    if (force == 0 && p.F == 1 && mv_gemm_deep_shape(M, N, K, gated))
+    // (a split K stays here: its sums may go straight into the norm behind the product, and have the same bits either way; so do
+    // float outputs, scores that choices are made by: one order of additions for every number of rows)
+    if (force == 0 && p.F == 1 && c_dtype == MV_BF16 && mv_gemm_deep_shape(M, N, K, gated))
         return mv_gemm_deep(A, lda, W, bias, C, ldc, c_dtype, M, N, K, gated, partial, P, eps, pair.limit, pair.slope, square_relu, 0, stream);
     MV_REQUIRE(tile_shape_served(p, gated != 0), "gemm_tile: no kernel for wave tiles %d x %d%s", p.wm, p.wn,
                p.deep ? " with the deep ring" : "");
