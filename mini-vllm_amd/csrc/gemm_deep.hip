@@ -248,14 +248,23 @@ static long deep_tiles(int shape, int M, int columns, bool gated) {
 // Which products come here, and with which tile: the smallest of which every compute unit gets at most one. (The more units pull at a
 // weight that comes from memory, the faster it is there: 64 rows against 1024 columns in front of a norm, 0.6B-sized steps, 8.8 us
 // with 64 tiles and 6.9 with 256; a second round costs more than it saves: 192 x 4096 x 1024 9.6 us in two, the library 7.2.)
-// Weights of 1 to 8 Mi elements from 9 rows on (below 1 Mi everything takes the fixed cost, 4 to 5 us, and the order of additions is
-// left as it is): for fewer rows the weight-streaming product, whose workgroups take four
+// Weights of 1 to 8 Mi elements from 9 rows on (below 1 Mi everything takes the fixed cost, 4 to 5 us): for fewer rows the
+// weight-streaming product, whose workgroups take four
 // columns, reads them as fast or faster (a step of one request 1,000 us with it, 1,043 here; of eight 1,130 and 1,135), at 16, 24,
 // 40 and 64 requests steps take 1,355 / 1,214, 1,515 / 1,314, 1,812 / 1,552 and 3,117 / 2,819. Larger weights up to 16 rows, where
 // 16 columns a unit cover them, or 32 up to 32 Mi elements (8 requests of the 8B sizes 3,997 / 3,856), whatever the number of rows:
 // a row's bits do not depend on it there; from 17 rows on the tiled product with its split of K is ahead (32 x 4096 x 12288
 // 23.0 us against 33.1). A K of one chunk stays where it was: there is nothing to walk, and the others are as fast to 1 us.
-static int deep_shape(int M, int N, int K, bool gated) {
+// The other kernels add in other orders, so which one serves is decided by the rows that a recorded step is padded to (all shapes
+// here add in one order): a step gives the same bits recorded and not.
+static int class_rows(int M) {
+    if (M <= 8) return M;
+    int step = 16;                                   // at most an eighth more
+    while (M > 8 * step) step *= 2;
+    return (M + step - 1) / step * step;
+}
+
+static int served_shape(int M, int N, int K, bool gated) {
     if (M <= 0 || N <= 0 || K < 2 * GD_KC || K % GD_KC || (gated && N % 2)) return 0;
     const int columns = gated ? N / 2 : N;
     const long units = mv_compute_units(), weight = (long)N * K;
@@ -268,6 +277,10 @@ static int deep_shape(int M, int N, int K, bool gated) {
     for (const int shape : {11, 12, 22, 24})
         if (!(gated && shape == 11) && deep_tiles(shape, M, columns, gated) <= units) return shape;
     return 0;
+}
+
+static int deep_shape(int M, int N, int K, bool gated) {
+    return M < (1 << 24) && served_shape(class_rows(M), N, K, gated) ? served_shape(M, N, K, gated) : 0;
 }
 
 extern "C" int mv_gemm_deep_shape(int M, int N, int K, int gated) { return deep_shape(M, N, K, gated != 0); }
