@@ -399,13 +399,32 @@ static void launch_waves(const void* A, long lda, const void* W, long ldw, const
                            (const TW*)bias, (TC*)C, ldc, M, N, K);
 }
 
-// Float operands whose K is whole chunks of 128 and whose rows start at 16-byte addresses go through the ring, from 17 rows on, and
+// The tile of float operands that go through the ring, in sixteens (rows x columns: 22, 24 or 44), 0: they don't. Rows that start at
+// 16-byte addresses and a K of whole chunks of 128 do, from 17 rows on, and
 // below that where the columns give half of the compute units a tile (us, registers / ring: 16 x 4096 x 1024 10.4 / 8.2,
 // 16 x 151936 x 1024 195 / 123; but 1 x 1024 x 3072 13.1 / 16.5, 16 x 1024 x 3072 16.8 / 16.7). Its tile is the one whose rounds
 // of the chip take the least time. Measured (us, registers / 32 x 32 / 32 x 64 / 64 x 64): 224 x 4096 x 1024 35 / 25.8 / 25.4 / 23.8,
 // 224 x 6144 x 1024 54 / 36.9 / 36.2 / 42.7, 224 x 1024 x 3072 30 / 18.7 / 31 / 54, 64 x 6144 x 1024 25 / 14.7 / 14.4 / 22,
-// 1024 x 24576 x 4096 2073 / 1898 / 1742 / 1627 (127 TFLOP/s), 4096 x 1024 x 128 24.2 / 25.1 / 25.9 / 22.8.
-// The others:
+// 1024 x 24576 x 4096 2073 / 1898 / 1742 / 1627 (127 TFLOP/s).
+// Where one wave would make a tile alone (below) the ring is ahead too (one wave / ring: 500 x 1024 x 128 10.4 / 6.4, 200 x 4096 x 128
+// 10.6 / 8.6, 1000 x 1024 x 256 15.3 / 11.4, 4096 x 1024 x 256 36.0 / 33.2, x 512 57.9 / 48.8, 8192 x 4096 x 512 420 / 350), but for a
+// single chunk and eight tiles a compute unit or more: then there is nothing to walk (2048 x 1024 x 128 13.9 / 14.1, 4096 x 1024 x 128
+// 25.0 / 25.2, 200 x 151936 x 128 166 / 170).
+static int ring_shape(int M, int N, int K) {
+    const long units = mv_compute_units();
+    auto tiles = [&](int rm, int rn) { return ((M + 16L * rm - 1) / (16 * rm)) * ((N + 16L * rn - 1) / (16 * rn)); };
+    if (M <= 0 || N <= 0 || K <= 0 || K % 128 || (M <= 16 && 2 * tiles(2, 2) < units) || (K == 128 && tiles(2, 2) >= 8 * units)) return 0;
+    // us of a chunk and of a tile's end, per shape, fitted to what they take alone and in rounds
+    auto cost = [&](int rm, int rn, double chunk, double last) {
+        return (double)((tiles(rm, rn) + units - 1) / units) * (K / 128 * chunk + last);
+    };
+    const double c22 = cost(2, 2, 0.57, 1.2), c24 = cost(2, 4, 1.07, 2.0), c44 = cost(4, 4, 2.0, 3.0);
+    return c44 <= c24 && c44 <= c22 ? 44 : c24 <= c22 ? 24 : 22;
+}
+
+extern "C" int mv_gemm_ref_ring_shape(int M, int N, int K) { return ring_shape(M, N, K); }
+
+// The others (rows at any address, another K, types of 16 bits):
 // The largest tile that still gives every compute unit one, since a larger one reads less a product; the bits do not depend
 // on it. Tiles of 32 x 64 where whole rounds of the chip by 64 x 64 leave it a quarter idle or more (224 x 6144 x 1024: 1.5
 // rounds, 61 us against 55), but not below 64 rows, where they are all of it (40 x 24576 x 4096: 235 us against 177).
@@ -422,14 +441,10 @@ static void launch_gemm(const void* A, long lda, const void* W, long ldw, const 
     auto rounds = [&](int rm, int rn) { return (tiles(rm, rn) + units - 1) / units * rm * rn; };
     if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4) {
         const bool vec = lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
-        if (vec && K % 128 == 0 && (M > 16 || 2 * tiles(2, 2) >= units)) {
-            // us of a chunk and of a tile's end, per shape, fitted to what they take alone and in rounds
-            auto cost = [&](int rm, int rn, double chunk, double last) {
-                return (double)((tiles(rm, rn) + units - 1) / units) * (K / 128 * chunk + last);
-            };
-            const double c22 = cost(2, 2, 0.57, 1.2), c24 = cost(2, 4, 1.07, 2.0), c44 = cost(4, 4, 2.0, 3.0);
-            if (c44 <= c24 && c44 <= c22) launch_ring<4, 4, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
-            else if (c24 <= c22) launch_ring<2, 4, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+        const int shape = vec ? ring_shape(M, N, K) : 0;
+        if (shape) {
+            if (shape == 44) launch_ring<4, 4, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+            else if (shape == 24) launch_ring<2, 4, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
             else launch_ring<2, 2, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
             return;
         }

@@ -43,6 +43,8 @@ _SIGNATURES = {
     "mv_swiglu": (c_int, [c_void_p, c_void_p, c_int, c_int, c_float, c_float, c_int, c_void_p]),
     "mv_gemm_ref": (c_int, [c_void_p, c_long, c_int, c_void_p, c_long, c_int, c_void_p, c_void_p, c_long, c_int,
                             c_int, c_int, c_int, c_void_p]),
+    # M, N, K
+    "mv_gemm_ref_ring_shape": (c_int, [c_int, c_int, c_int]),
     # q, q_stride, out, out_stride, k_pages, v_pages, block_table, bt_width, page_size, positions, token_seq, n, H, Hkv, D,
     # Dv, scale, window, first, gate, gate_stride, cap, slopes, sink, dtype, stream
     "mv_attention_ref": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int,
