@@ -1,5 +1,5 @@
 // C[M, N] = A[M, K] * W[N, K]^T (+ bias) or its gated pair in bf16 for products whose tiles hardly fill the chip once (up to a few hundred
-// rows against the weights of a small model, up to 64 against larger ones), so that their time is that of one tile: how often a
+// rows against the weights of a small model, up to 16 against larger ones), so that their time is that of one tile: how often a
 // workgroup goes to memory and back, and how many lines it asks for.
 //
 // A chunk is 256 values of k, 32 for each of the eight waves: the waves split K, not the tile, and K = 2048 is eight steps of a
@@ -17,7 +17,8 @@
 // these read besides (sums, residual, weights) is asked for before the first chunk and used behind the last.
 //
 // What bounds it: the operands of a tile, (rows + columns) x K, that a compute unit can pull from the caches, and a fixed 3 to
-// 4 us. Measured alone (us; weight-streaming, tiled or the library's, whichever served / here): 8 x 4096 x 1024 behind a norm 5.6 / 4.8,
+// 4 us. Measured alone (us; weight-streaming, tiled or the library's, whichever served / here; what is faster alone is not always so in
+// a model, see the rule): 8 x 4096 x 1024 behind a norm 5.6 / 4.8,
 // 8 x 6144 x 1024 gated behind a norm 7.5 / 6.2, 8 x 1024 x 3072 in front of one 6.2 / 5.6, 8 x 6144 x 4096 14.1 / 11.8; 64 x 4096 x 1024
 // 7.4 / 4.9, 64 x 1024 x 3072 in front of a norm 8.7 / 7.2; 512 x 1024 x 2048 9.8 / 7.7, 512 x 1024 x 3072 12.5 / 9.6.
 #include "gemm_ring.h"
@@ -252,9 +253,11 @@ static long deep_tiles(int shape, int M, int columns, bool gated) {
 // weight-streaming product, whose workgroups take four
 // columns, reads them as fast or faster (a step of one request 1,000 us with it, 1,043 here; of eight 1,130 and 1,135), at 16, 24,
 // 40 and 64 requests steps take 1,355 / 1,214, 1,515 / 1,314, 1,812 / 1,552 and 3,117 / 2,819. Larger weights up to 16 rows, where
-// 16 columns a unit cover them, or 32 up to 32 Mi elements (8 requests of the 8B sizes 3,997 / 3,856), whatever the number of rows:
-// a row's bits do not depend on it there; from 17 rows on the tiled product with its split of K is ahead (32 x 4096 x 12288
-// 23.0 us against 33.1). A K of one chunk stays where it was: there is nothing to walk, and the others are as fast to 1 us.
+// 16 columns a unit cover them, or 32 up to 32 Mi elements, from the first row on
+// (steps of the 8B sizes at 1,024 tokens, before / with it: 1 request 3,545 / 3,515, 2 3,579 / 3,543, 4 3,710 / 3,656, 8 4,005 / 3,860;
+// one request of Dutilix 5,271 / 5,183, Bolapel 4,558 / 4,532, Sorulix 4,883 / 4,844, Zedudra 4,587 / 4,531, Furanex 5,795 / 5,774,
+// Setirax 4,775 / 4,801), so a row's bits are the same for 1 to 16 rows; from 17 rows on the tiled product with its split of K is
+// ahead (32 x 4096 x 12288 23.0 us against 33.1). A K of one chunk stays where it was: there is nothing to walk, and the others are as fast to 1 us.
 // The other kernels add in other orders, so which one serves is decided by the rows that a recorded step is padded to (all shapes
 // here add in one order): a step gives the same bits recorded and not.
 static int class_rows(int M) {

@@ -1,5 +1,5 @@
 // The library's matrix product for many rows (prompt portions, decode steps of more than 64
-// sequences), called directly:
+// sequences), called directly, but for the shapes that gemm_deep.hip takes:
 //     C[M, N] = A[M, K] * W[N, K]^T (+ bias),   bf16 in, bf16 or float out, float accumulation
 //     (hipBLASLt).
 // Going through a tensor library's dispatcher costs about 18 us of host time per product on this

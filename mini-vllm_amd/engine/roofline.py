@@ -35,7 +35,7 @@ KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_qk_norm_rope_store": (r"\b(qk_norm_rope_store(_vec)?_kernel|qkv_prompt_vec_kernel)", r"\bstore_v_pages_kernel", 2),
     "mv_swiglu": (r"\bswiglu(_vec)?_kernel", None, 1),
     "mv_gemm_skinny": (r"\bgemm_(skinny|deep)_kernel", None, 1),
-    "mv_gemm_skinny_norm": (r"\bgemm_(skinny|deep)_kernel", None, 1),
+    "mv_gemm_skinny_norm": (r"\bgemm_skinny_kernel", None, 1),
     "mv_gemm_skinny_swiglu": (r"\bgemm_(skinny|deep)_kernel", None, 1),
     "mv_gemm_skinny_fold": (r"\bgemm_(skinny|deep)_kernel", None, 1),
     "mv_gemm_skinny_scaled": (r"\bgemm_(skinny|deep)_kernel", None, 1),

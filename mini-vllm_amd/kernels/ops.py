@@ -2424,7 +2424,8 @@ class Ops:
         return rest if step in (2048, 4096) and M > step and rest <= 1024 else 0
 
     def _library_product(self, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor) -> bool:
-        """out = a @ w^T (+ bias) by the library (hipBLASLt), bf16 in, bf16 or float32 out. It is
+        """out = a @ w^T (+ bias) by the library (hipBLASLt), bf16 in, bf16 or float32 out; bf16 outputs of shapes that
+        ``gemm_deep.hip`` is faster at are made there, inside the same entry point. The library is
         called directly where the kernel library was built with it (a call costs a third of the host
         time of the tensor library's dispatcher, which matters for prompt steps of small models);
         else, for bf16 output, through ``torch.mm``. False, with nothing done, when the library has

@@ -248,8 +248,8 @@ def test_gemm_exact(dtype, wdtype, M, N, K):
                                    (300, 6100, 128), (16, 8190, 128)])
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_exact_product_through_the_ring(M, N, K, with_bias):
-    """Every tile shape, one chunk and several, one tile a workgroup and several, ragged edges, rows with a stride of their
-    own. The bits are those of the product that takes rows at any address: the same rows shifted by one element. Against
+    """Every tile shape, one chunk and several, one tile a workgroup (at most two of one chunk; more in test_gpu_float_ring.py),
+    ragged edges, rows with a stride of their own. The bits are those of the product that takes rows at any address: the same rows shifted by one element. Against
     64 bits: K products of numbers of size 1 and 1/sqrt(K), summed in floats, 3e-6 of the largest as above."""
     ops = ops_for(torch.float32)
     g = torch.Generator().manual_seed(M + N + K)
