@@ -258,6 +258,11 @@ static long deep_tiles(int shape, int M, int columns, bool gated) {
 // one request of Dutilix 5,271 / 5,183, Bolapel 4,558 / 4,532, Sorulix 4,883 / 4,844, Zedudra 4,587 / 4,531, Furanex 5,795 / 5,774,
 // Setirax 4,775 / 4,801), so a row's bits are the same for 1 to 16 rows; from 17 rows on the tiled product with its split of K is
 // ahead (32 x 4096 x 12288 23.0 us against 33.1). A K of one chunk stays where it was: there is nothing to walk, and the others are as fast to 1 us.
+// What stays with the library's split of K and the tiled product (us, these / here): above 96 rows a K of more than 4096 (500 x 128 x
+// 8192 11.0 / 14.8, 800 x 512 x 16384 44.0 / 51.5; 200 x 768 x 8192 would be 19.9 / 15.4), and one of 4096 in tiles of 32 x 64 or above 512
+// rows (800 x 576 x 4096 15.2 / 16.5, 800 x 256 x 4096 11.8 / 12.6; but 100 x 1024 x 4096 11.9 / 9.0, 300 x 576 x 4096 11.8 / 9.7); and
+// two chunks in tiles of 32 x 64 above 32 rows (128 x 4096 x 512 5.8 / 5.9, gated 64 x 8192 x 512 6.4 / 6.6; 32 x 16384 x 512 8.6 / 7.4). Gated
+// pairs of a longer K have no such end: 500 x 1024 x 8192 56.7 / 27.1.
 // The other kernels add in other orders, so which one serves is decided by the rows that a recorded step is padded to (all shapes
 // here add in one order): a step gives the same bits recorded and not.
 static int class_rows(int M) {
@@ -277,8 +282,12 @@ static int served_shape(int M, int N, int K, bool gated) {
         return deep_tiles(12, M, columns, gated) <= units && weight <= 32L << 20 ? 12 : 0;
     }
     if (M <= 8 || weight < 1L << 20) return 0;
-    for (const int shape : {11, 12, 22, 24})
-        if (!(gated && shape == 11) && deep_tiles(shape, M, columns, gated) <= units) return shape;
+    if (!gated && M > 96 && (K > 4096 || (K == 4096 && M > 512))) return 0;
+    for (const int shape : {11, 12, 22, 24}) {
+        if ((gated && shape == 11) || deep_tiles(shape, M, columns, gated) > units) continue;
+        const bool slow = shape == 24 && (K <= 2 * GD_KC ? M > 32 : !gated && K == 4096 && M > 96);
+        return slow ? 0 : shape;
+    }
     return 0;
 }
 
