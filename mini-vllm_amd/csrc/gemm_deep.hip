@@ -7,7 +7,11 @@
 // of 64 takes 32 steps, each with a barrier and a wait; the weight-streaming one loads sixteen rows an instruction, half lines
 // or single ones, and every workgroup all activation rows). A row's 512 bytes of a chunk are loaded as whole lines straight
 // into LDS; a wave has the operands of its next block in registers before the products of the current one. At the end the
-// waves' sums are added in the order ((0+4)+(2+6))+((1+5)+(3+7)) through LDS, in float, and rounded once.
+// waves' sums are added in the order ((0+4)+(2+6))+((1+5)+(3+7)) through LDS, in float, and rounded once. Against weights of 8 Mi
+// elements and more a wave adds up even and odd chunks apart (CHAINS), so that a sum has sixteen chains, as it has in the weight-streaming
+// product there, and no larger an error (16 rows of N(0, 1) operands, weight-streaming / eight chains / sixteen: K = 4096 1.06e-7 / 1.34e-7 /
+// 1.02e-7, 12288 1.68e-7 / 2.34e-7 / 1.65e-7). Below that its sums have eight, and so has this one (K = 1024 8.2e-8 / 7.6e-8, 3072 1.21e-7 /
+// 1.18e-7): two accumulators a tile cost 2 % where tiles are many.
 // LDS: rows of 512 bytes, 16-byte piece p of row r in place p ^ (r & 15): sixteen lanes that read one piece of sixteen rows
 // meet in no bank.
 //
@@ -53,7 +57,7 @@ enum DeepForm { DEEP_PLAIN = 0, DEEP_GATED = 1, DEEP_FOLD = 2 };
 
 // RM x RN tiles of 16 tokens x 16 weight rows a workgroup; gated: the second half of the weight rows are the up rows of the
 // first half's columns
-template <int RM, int RN, int STAGES, int FORM>
+template <int RM, int RN, int STAGES, int FORM, int CHAINS>
 __global__ void __launch_bounds__(64 * GD_WAVES)
 gemm_deep_kernel(DeepArgs p) {
     constexpr bool GATED = FORM == DEEP_GATED, FOLD = FORM == DEEP_FOLD;
@@ -123,11 +127,11 @@ gemm_deep_kernel(DeepArgs p) {
 #pragma unroll
         for (int c = 0; c < RN; ++c) w[to][c].u = ring[stage][16 * (RM + c) + i][slot];
     };
-    floatx4_t acc[RM][RN];
+    floatx4_t acc[CHAINS][RM][RN];                   // two: of the even chunks, of the odd ones
 #pragma unroll
     for (int r = 0; r < RM; ++r)
 #pragma unroll
-        for (int c = 0; c < RN; ++c) acc[r][c] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+        for (int c = 0; c < RN; ++c) acc[0][r][c] = acc[CHAINS - 1][r][c] = floatx4_t{0.f, 0.f, 0.f, 0.f};
     // this wave's loads have landed but for those of the newest `left` chunks, and what it read of LDS has arrived; then all waves'
     auto meet = [&](int left) __attribute__((always_inline)) {
 #define GD_WAIT(N) __builtin_amdgcn_s_waitcnt(0x0070 | (((N) * LOADS) & 15) | ((((N) * LOADS) >> 4) << 14))
@@ -159,7 +163,7 @@ gemm_deep_kernel(DeepArgs p) {
 #pragma unroll
         for (int r = 0; r < RM; ++r)
 #pragma unroll
-            for (int k = 0; k < RN; ++k) acc[r][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[cur][k].v, a[cur][r].v, acc[r][k], 0, 0, 0);
+            for (int k = 0; k < RN; ++k) acc[cur % CHAINS][r][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[cur][k].v, a[cur][r].v, acc[cur % CHAINS][r][k], 0, 0, 0);
     };
     for (int c = 0; c < chunks; c += 2) {
         turn(c, 0);
@@ -172,7 +176,7 @@ gemm_deep_kernel(DeepArgs p) {
 #pragma unroll
     for (int r = 0; r < RM; ++r)
 #pragma unroll
-        for (int c = 0; c < RN; ++c) part[((r * RN + c) * GD_WAVES + wave) * MV_WAVE + lane] = acc[r][c];
+        for (int c = 0; c < RN; ++c) part[((r * RN + c) * GD_WAVES + wave) * MV_WAVE + lane] = CHAINS == 1 ? acc[0][r][c] : acc[0][r][c] + acc[CHAINS - 1][r][c];
     if (scaled) {
         float t = 0.f;
 #pragma unroll
@@ -264,7 +268,7 @@ static long deep_tiles(int shape, int M, int columns, bool gated) {
 // two chunks in tiles of 32 x 64 above 32 rows (128 x 4096 x 512 5.8 / 5.9, gated 64 x 8192 x 512 6.4 / 6.6; 32 x 16384 x 512 8.6 / 7.4). Gated
 // pairs of a longer K have no such end: 500 x 1024 x 8192 56.7 / 27.1.
 // The other kernels add in other orders, so which one serves is decided by the rows that a recorded step is padded to (all shapes
-// here add in one order): a step gives the same bits recorded and not.
+// here add a weight up in one order): a step gives the same bits recorded and not.
 static int class_rows(int M) {
     if (M <= 8) return M;
     int step = 16;                                   // at most an eighth more
@@ -313,11 +317,18 @@ static int deep_launch(const char* what, DeepArgs p, int shape, hipStream_t stre
     MV_REQUIRE(tiles < (1L << 24), "%s: too many tiles", what);
     p.tiles = (int)tiles;
     const dim3 grid((p.tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS), block(64 * GD_WAVES);
+    const bool chains = (long)p.N * p.K >= 8L << 20;
+#define GD_LAUNCH(RM, RN, STAGES)                                                                                                   \
+    do {                                                                                                                            \
+        if (chains) hipLaunchKernelGGL((gemm_deep_kernel<RM, RN, STAGES, FORM, 2>), grid, block, 0, stream, p);                     \
+        else hipLaunchKernelGGL((gemm_deep_kernel<RM, RN, STAGES, FORM, 1>), grid, block, 0, stream, p);                            \
+    } while (0)
     if constexpr (!(FORM == DEEP_GATED))
-        if (shape == 11) hipLaunchKernelGGL((gemm_deep_kernel<1, 1, 6, FORM>), grid, block, 0, stream, p);
-    if (shape == 12) hipLaunchKernelGGL((gemm_deep_kernel<1, 2, 6, FORM>), grid, block, 0, stream, p);
-    else if (shape == 22) hipLaunchKernelGGL((gemm_deep_kernel<2, 2, 4, FORM>), grid, block, 0, stream, p);
-    else if (shape == 24) hipLaunchKernelGGL((gemm_deep_kernel<2, 4, 3, FORM>), grid, block, 0, stream, p);
+        if (shape == 11) GD_LAUNCH(1, 1, 6);
+    if (shape == 12) GD_LAUNCH(1, 2, 6);
+    else if (shape == 22) GD_LAUNCH(2, 2, 4);
+    else if (shape == 24) GD_LAUNCH(2, 4, 3);
+#undef GD_LAUNCH
     return mv_check_launch(what);
 }
 

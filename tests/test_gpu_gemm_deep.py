@@ -107,3 +107,25 @@ def test_which_sizes_come_here():
         [11, 12, 11, 12, 22, 24, 24, 11, 22, 24]
     assert [shape(*s) for s in [(8, 4096, 1024, 0), (16, 4096, 256, 0), (16, 4096, 1000, 0), (17, 4096, 4096, 0), (8, 24576, 4096, 1),
                                 (129, 4096, 1024, 0), (513, 1024, 1024, 0), (0, 1024, 1024, 0), (16, 1023, 1024, 0)]] == [0] * 9
+
+
+# (weights of 8 Mi elements, where the kernel in front changes its form, and on both sides of it)
+@pytest.mark.parametrize("N,K", [(4096, 1024), (1024, 2048), (1024, 3072), (2048, 4096), (2032, 4096), (8192, 1024), (4096, 4096), (4096, 12288)])
+def test_sums_are_as_exact_as_those_of_the_kernel_in_front(N, K):
+    """Float sums of N(0, 1) operands against 64 bits, 2-norms over 16 rows of four draws, which are good to a percent."""
+    ops = ops_for(BF)
+    errors = {"mv_gemm_skinny": 0.0, "mv_gemm_deep": 0.0}
+    for seed in range(4):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        a = torch.randn(16, K, generator=g, device="cuda").to(BF)
+        w = (torch.randn(N, K, generator=g, device="cuda") / math.sqrt(K)).to(BF)
+        want = a.double() @ w.double().T
+        for entry in errors:
+            out = torch.empty(16, N, device="cuda")
+            if entry == "mv_gemm_skinny":
+                ops.lib.call(entry, a.data_ptr(), K, w.data_ptr(), K, 0, out.data_ptr(), N, 0, 16, N, K, 0, ops._stream())
+            else:
+                ops.lib.call(entry, a.data_ptr(), K, w.data_ptr(), 0, out.data_ptr(), N, 0, 16, N, K, 0, 0, 0, 0.0, 0.0, 1.0, 0, 0, ops._stream())
+            errors[entry] += float(((out.double() - want).norm() / want.norm()) ** 2)
+    print(K, {entry: math.sqrt(e / 4) for entry, e in errors.items()})
+    assert math.sqrt(errors["mv_gemm_deep"]) <= 1.02 * math.sqrt(errors["mv_gemm_skinny"])
