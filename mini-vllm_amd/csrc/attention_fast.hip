@@ -720,7 +720,7 @@ static int decode_common(bool fused, const FusedInput& fz, const void* q, long q
     dim3 grid((unsigned)n_seqs * Hkv, nsplit);
     float* part = nsplit > 1 ? partials : nullptr;
     // With more workgroups than compute units, two of them share a unit (the kernel is then held to
-    // 256 registers a lane, which costs it three spilled ones at head size 128): one's set-up and
+    // 256 registers a lane, which costs it eleven spilled ones at head size 128): one's set-up and
     // tail overlap the other's stream of keys, 4-6 % on a step of 64 to 256 sequences. A grid that
     // fits the chip at once keeps all registers.
     const int occ = ((long)n_seqs * Hkv > mv_compute_units() && nsplit == 1) ? 2 : 1;
