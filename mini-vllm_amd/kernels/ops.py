@@ -106,6 +106,8 @@ DECODE_ATTENTION_WAVES = 4
 # the workgroup kernel splits a sequence's keys until about one workgroup for every compute unit is
 # in flight (``Ops.compute_units``)
 # (sequence, kv head) pairs of one decode step whose keys may be split over workgroups
+# (block of 32 keys, head) pairs whose keys and values a latent attention may make at a time: 16 KiB each, 512 MiB of scratch
+LATENT_HEADS_MOST = 1 << 15
 SPLIT_COUNTERS = 1 << 16
 # from this many tokens on, value rows are written to their pages 16 tokens of a kv head at a time
 STORE_V_SPLIT_TOKENS = 64
@@ -126,6 +128,12 @@ def _ptr(t: Optional[torch.Tensor]) -> int:
 def _dev(t: torch.Tensor, what: str) -> None:
     if not t.is_cuda:
         raise KernelLibraryError(f"{what} is on {t.device}; the engine's kernels run on the GPU only")
+
+
+def latent_operands(w: torch.Tensor) -> torch.Tensor:
+    """A map [heads, 128, kv_rank] of a latent in the order of the matrix unit's operands (see ``Ops.latent_expand``)."""
+    h, rows, rank = w.shape
+    return w.reshape(h, rows // 16, 16, rank // 32, 4, 8).permute(0, 1, 3, 4, 2, 5).contiguous()
 
 
 def _weight_code(w: torch.Tensor, what: str) -> int:
@@ -1505,6 +1513,98 @@ class Ops:
         """Whether ``attention_latent`` has a kernel for latents of these sizes whose workgroups share key rows."""
         return self.use_fast_kernels and self.lib.has("mv_attention_latent_prompt") \
             and bool(self.lib.dll.mv_attention_latent_prompt_serves(kv_rank, rot_dim))
+
+    def latent_heads_serve(self, plain_dim: int, value_dim: int, kv_rank: int, rot_dim: int) -> bool:
+        """Whether ``latent_expand`` and ``attention_latent_heads`` have kernels for heads and latents of these sizes."""
+        return self.use_fast_kernels and self.lib.has("mv_attention_latent_heads") \
+            and bool(self.lib.dll.mv_attention_latent_heads_serves(plain_dim, value_dim, kv_rank, rot_dim))
+
+    def latent_heads(self, heads: int, lens: Sequence[int], starts: Sequence[int]) -> int:
+        """For requests of ``lens`` tokens from positions ``starts`` on: the blocks of 32 keys that scratch and grid are made for where
+        the heads' own keys and values are made from the latents (``latent_expand``), or 0: attention stays in the latent's space.
+        Making them costs every key of a request's context once, however few its tokens, so a step of decoding requests beside a
+        prompt stays where it is unless the contexts are short. Both times in us as measured on an MI355X (256 + 64, 16 and 64 heads): the
+        maps 0.26 a thousand (key, head) pairs; a walk 0.8 a block of 32 keys, 512 workgroups of 64 tokens at a time; against
+        1.6 a thousand (token, head) pairs for carrying queries in and sums out, and ``latent_shares``' 1.6 a block, 256 workgroups at a
+        time. Own keys / latents: one prompt of 20 tokens 11 / 20, 200 16 / 50, 2,048 55 / 193, 16 tokens behind 2,000 50 / 147; beside 16
+        tokens 8 requests decoding at 1,000 62 / 69, at 300 27 / 36, 64 at 1,000 420 / 85; beside 300 tokens 16 at 1,900 192 / 128.
+        The count is a multiple of 4, of an eighth of it or more, so that steps of similar sizes share a recording."""
+        if not lens or max(lens) < 2:
+            return 0
+        q, s = np.asarray(lens), np.asarray(starts)
+        of_request = (q + s + 31) // 32
+        blocks, longest = int(of_request.sum()), int(of_request.max())
+        step = max(4, 1 << max(0, blocks.bit_length() - 3))
+        room = -(-blocks // step) * step
+        if room * heads > LATENT_HEADS_MOST:
+            return 0
+        keys = 1 + (s + q // 2) // 32                              # a walk, by the middle of a request's tokens
+        own = 9.0 + 0.26e-3 * heads * 32 * blocks + 0.8 * max(longest, heads * int(((q + 63) // 64) @ keys) / (2 * self.compute_units))
+        groups = -(-heads // 16) * ((q + 7) // 8)
+        latent = 12.0 + 1.6e-3 * heads * int(q.sum()) + max(9.0 + 1.6 * longest, float(groups @ (9.0 + 1.6 * keys)) / self.compute_units)
+        return room if own < latent else 0
+
+    def latent_heads_most(self, heads: int, tokens: int, seqs: int, positions: int) -> int:
+        """The most that ``latent_heads`` says for any step of up to ``tokens`` tokens of ``seqs`` requests of up to ``positions`` positions."""
+        blocks = seqs * -(-positions // 32)
+        return min(LATENT_HEADS_MOST // heads, blocks + max(4, blocks // 4)) if tokens > 1 else 0
+
+    def latent_expand(self, pages: torch.Tensor, block_table: torch.Tensor, page_size: int, plan, context_lens: torch.Tensor, w_k: torch.Tensor,
+                      w_v: torch.Tensor, heads: int, kv_rank: int, rot_dim: int, blocks: int, k: torch.Tensor, kr: torch.Tensor,
+                      v: torch.Tensor) -> None:
+        """The heads' own keys and values of every key of the step's requests, from the cached latents (``pages`` as for
+        ``attention_latent``, the keys of this step already in them): into k and v [blocks, heads, 4096], kr [blocks, 32 rot_dim], in the
+        order that ``attention_latent_heads`` reads. w_k, w_v as ``latent_operands`` orders the stored matrices; ``blocks``: as
+        ``latent_heads`` says for the step, or more."""
+        self._act(pages, "latent pages"); self._act(w_k, "key maps"); self._act(w_v, "value maps"); self._act(k, "keys"); self._act(v, "values")
+        dk = kv_rank + rot_dim
+        if pages.dim() != 3 or tuple(pages.shape[1:]) != (page_size, dk) or not pages.is_contiguous():
+            raise KernelLibraryError(f"latent_expand: pages must be [pages, {page_size}, {dk}]")
+        if block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.shape[0] < plan.n_seqs or not block_table.is_contiguous():
+            raise KernelLibraryError("latent_expand: the block table must be contiguous int32 [sequences, width]")
+        if w_k.numel() != heads * 128 * kv_rank or w_v.numel() != w_k.numel() or not w_k.is_contiguous() or not w_v.is_contiguous():
+            raise KernelLibraryError(f"latent_expand: the maps must hold {heads} x 128 x {kv_rank} numbers each")
+        if k.numel() < blocks * heads * 4096 or v.numel() < blocks * heads * 4096 or kr.numel() < blocks * 32 * rot_dim:
+            raise KernelLibraryError("latent_expand: the scratch is too small")
+        self._ints(plan.n_seqs, context_lens=(context_lens, plan.n_seqs), cu_seqlens=(plan.cu_seqlens, plan.n_seqs + 1))
+        self._note("mv_latent_expand", self._size(w_k, w_v) + 2 * blocks * heads * 4096 * 2 + plan.kv_tokens * dk * 2, 4 * plan.kv_tokens * heads * 128 * kv_rank)
+        self.lib.call("mv_latent_expand", pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size, plan.cu_seqlens.data_ptr(),
+                      context_lens.data_ptr(), plan.n_seqs, w_k.data_ptr(), w_v.data_ptr(), heads, kv_rank, rot_dim, k.data_ptr(), kr.data_ptr(),
+                      v.data_ptr(), blocks, self._stream())
+
+    def attention_latent_heads(self, q: torch.Tensor, out: torch.Tensor, k: torch.Tensor, kr: torch.Tensor, v: torch.Tensor, plan,
+                               positions: torch.Tensor, token_seq: torch.Tensor, context_lens: torch.Tensor, heads: int, rot_dim: int,
+                               scale: float, table: Optional[torch.Tensor] = None, sink: Optional[torch.Tensor] = None,
+                               gate: Optional[torch.Tensor] = None, gate_per_head: bool = False) -> None:
+        """Causal softmax attention of q [n, heads * (128 + rot_dim)] (the rotary channels rotated here, by ``table``) over the keys and
+        values that ``latent_expand`` left, into out [n, heads * 128], times sigmoid(gate) where gates are given ([n, heads * 128], or
+        [n, >= heads] with ``gate_per_head``); rows of no request become zeros. ``sink`` as for ``attention_latent``."""
+        self._act(q, "latent queries"); self._act(out, "latent attention output")
+        n, dq = q.shape[0], heads * (128 + rot_dim)
+        if q.dim() != 2 or q.shape[1] != dq or q.stride(1) != 1 or out.dim() != 2 or tuple(out.shape) != (n, heads * 128) or out.stride(1) != 1:
+            raise KernelLibraryError(f"attention_latent_heads: queries [{n}, {dq}] and an output [{n}, {heads * 128}] are needed")
+        self._ints(n, positions=(positions, n), token_seq=(token_seq, n), context_lens=(context_lens, plan.n_seqs),
+                   cu_seqlens=(plan.cu_seqlens, plan.n_seqs + 1))
+        if rot_dim:
+            _dev(table, "rotary table")
+            if table.dtype != torch.float32 or table.dim() != 2 or table.shape[1] != rot_dim or not table.is_contiguous():
+                raise KernelLibraryError(f"attention_latent_heads: the rotary table must be float32 [positions, {rot_dim}]")
+        if sink is not None and (sink.dtype != torch.float32 or sink.numel() != heads or not sink.is_contiguous()):
+            raise KernelLibraryError(f"attention_latent_heads: the sinks must be float32 [{heads}]")
+        if gate is not None:
+            self._act(gate, "output gate")
+            if gate.dim() != 2 or gate.shape[0] != n or gate.stride(1) != 1 or (gate.shape[1] < heads if gate_per_head else gate.shape[1] != heads * 128):
+                raise KernelLibraryError("attention_latent_heads: the gate must be [n, heads * 128], or [n, >= heads] with one number a head")
+        tokens = self.lib.dll.mv_attention_latent_heads_tokens
+        wide = plan.busy_units(tokens(1)) * heads >= 2 * self.compute_units
+        units, busy = plan.units(tokens(int(wide))), plan.busy_units(tokens(int(wide)))
+        pitch = lambda t: t.stride(0) if n > 1 else t.shape[1]
+        self._note("mv_attention_latent_heads", self._size(q, out) + plan.kv_tokens * heads * (256 + rot_dim) * 2,
+                   2 * plan.attention_pairs * heads * (256 + rot_dim))
+        self.lib.call("mv_attention_latent_heads", q.data_ptr(), pitch(q), out.data_ptr(), pitch(out), k.data_ptr(), kr.data_ptr(), v.data_ptr(),
+                      positions.data_ptr(), token_seq.data_ptr(), plan.cu_seqlens.data_ptr(), context_lens.data_ptr(), plan.n_seqs, units, busy,
+                      int(wide), n, int(plan.bound is not None or sum(plan.q_lens) != n), heads, rot_dim, float(scale), _ptr(table), _ptr(sink),
+                      _ptr(gate), pitch(gate) if gate is not None else 0, int(gate_per_head), self._stream())
 
     def latent_shares(self, heads: int, window: int, lens: Sequence[int], starts: Sequence[int]) -> bool:
         """Whether the workgroups of a step with prompt portions share key rows among eight tokens of a request (requests of

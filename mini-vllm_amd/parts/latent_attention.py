@@ -22,9 +22,11 @@ on (None: all). ``sink``: the softmax's denominator has one more term e^sink_h, 
 and that no key or value belongs to.
 
 Only [c | k_rot] is cached, one row of ``kv_rank + rot_dim`` numbers per token, and c once more in
-the slot-contiguous layout that the MFMA kernel's second product reads (``LatentNeed``). Keys and values are never expanded: the query is carried into the latent's space
-(W_uk,h^T q_plain), attention runs on the cached rows with the latent as the value, and W_uv,h is
-applied to the weighted sum of latents. Norms, rotation, scores, weights and sums are float32.
+the slot-contiguous layout that the MFMA kernel's second product reads (``LatentNeed``). Steps of single tokens never expand keys and
+values: the query is carried into the latent's space (W_uk,h^T q_plain), attention runs on the cached rows with the latent as the value,
+and W_uv,h is applied to the weighted sum of latents. Steps whose requests bring many tokens make the heads' own keys and values of
+the step's contexts once and attend to those, where that takes less time (``Ops.latent_heads``; bfloat16, heads of 128). Norms,
+rotation, scores, weights and sums are float32.
 """
 from __future__ import annotations
 
@@ -33,6 +35,7 @@ from typing import Dict, Optional, Sequence, Tuple
 
 import torch
 
+from ..kernels.ops import latent_operands
 from .base import CacheNeed, KeepAll, KeepWindow, Mixer, PartSpec, Retention, Runtime, TensorDecl, register_mixer
 
 
@@ -152,11 +155,29 @@ class LatentAttention(Mixer):
         self.w_uk_rows = self.w_uk.transpose(1, 2).contiguous()
         self.w_uv_rows = tensors["uv"].view(spec.num_heads, spec.value_dim, spec.kv_rank).contiguous()
         self.w_o = tensors["o"]
+        # ... and in the order in which the heads' own keys and values are made from the latents
+        self.heads_operands = None
+        if spec.window is None and rt.dtype == torch.bfloat16 == self.w_uk.dtype == self.w_uv.dtype \
+                and rt.ops.latent_heads_serve(spec.plain_dim, spec.value_dim, spec.kv_rank, spec.rot_dim):
+            self.heads_operands = latent_operands(self.w_uk), latent_operands(self.w_uv_rows)
 
     def step_path(self, lens: Sequence[int], starts: Sequence[int]):
+        blocks = self.rt.ops.latent_heads(self.spec.num_heads, lens, starts) if self.heads_operands is not None else 0
+        if blocks:
+            return "heads", blocks
         if not self.rt.ops.latent_shares_serve(self.spec.kv_rank, self.spec.rot_dim):
             return None
         return self.rt.ops.latent_shares(self.spec.num_heads, -1 if self.spec.window is None else self.spec.window, lens, starts)
+
+    def reserve(self, tokens: int, seqs: int) -> None:
+        most = self.rt.ops.latent_heads_most(self.spec.num_heads, tokens, seqs, self.rt.max_positions) if self.heads_operands is not None else 0
+        if most:
+            self._heads_scratch(most)
+
+    def _heads_scratch(self, blocks: int):
+        ws, H = self.rt.workspace, self.spec.num_heads
+        return (ws.get("latent.k", (blocks, H, 4096), self.rt.dtype), ws.get("latent.kr", (blocks, 32 * max(1, self.spec.rot_dim)), self.rt.dtype),
+                ws.get("latent.v", (blocks, H, 4096), self.rt.dtype))
 
     def forward(self, x: torch.Tensor, ctx, call: int) -> torch.Tensor:
         spec, rt, ops, ws = self.spec, self.rt, self.rt.ops, self.rt.workspace
@@ -173,16 +194,25 @@ class LatentAttention(Mixer):
             ops.gemm(cq, self.w_uq, q)
         else:
             q = packed[:, self.q_offset:self.q_offset + H * (spec.plain_dim + dr)]
+        heads = ws.get("latent.heads", (n, H * spec.value_dim), rt.dtype)
+        gate = None
+        if spec.output_gate:
+            gate = packed[:, self.gate_offset:self.gate_offset + (H if spec.head_gate else H * spec.value_dim)]
+        plan = ctx.attention_plan
+        blocks = ops.latent_heads(H, *plan.cut()) if self.heads_operands is not None and not plan.decode_only else 0
+        if blocks and q.data_ptr() % 16 == 0 and q.stride(0) % 8 == 0:
+            k, kr, v = self._heads_scratch(blocks)
+            ops.latent_expand(pages, kv.block_table, kv.page_size, plan, ctx.context_lens, *self.heads_operands, H, R, dr, blocks, k, kr, v)
+            ops.attention_latent_heads(q, heads, k, kr, v, plan, ctx.positions, ctx.token_seq, ctx.context_lens, H, dr, spec.scale, self.table,
+                                       self.sink, gate, spec.head_gate)
+            y = ws.get("mixer.out", (n, spec.hidden_size), rt.dtype)
+            return ops.gemm(heads, self.w_o, y, defer_sum=True) or y
         qa = ws.get("latent.qa", (n, H, R + dr), torch.float32)
         ops.head_linear(q.unflatten(1, (H, spec.plain_dim + dr)), self.w_uk, qa, ctx.token_seq, tail=dr, table=self.table,
                         positions=ctx.positions, w_rows=self.w_uk_rows)
         mixed = ws.get("latent.mixed", (n, H, R), torch.float32)
         ops.attention_latent(qa, mixed, pages, kv.block_table, kv.page_size, ctx.positions, ctx.token_seq, H, R, dr,
                              spec.scale, plan=ctx.attention_plan, pages_t=pages_t, window=spec.window, sink=self.sink)
-        heads = ws.get("latent.heads", (n, H * spec.value_dim), rt.dtype)
-        gate = None
-        if spec.output_gate:
-            gate = packed[:, self.gate_offset:self.gate_offset + (H if spec.head_gate else H * spec.value_dim)]
         ops.head_linear(mixed, self.w_uv, heads, ctx.token_seq, gate=gate, w_rows=self.w_uv_rows, gate_per_head=spec.head_gate)
         y = ws.get("mixer.out", (n, spec.hidden_size), rt.dtype)
         return ops.gemm(heads, self.w_o, y, defer_sum=True) or y

@@ -1,0 +1,127 @@
+"""The heads' own keys and values from a cached latent, and attention on them, against the same computation in float64."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def reference(q, latents, cut, w_k, w_v, table, scale, sink, gate, per_head, R, dr):
+    """Keys, values and turned queries rounded to bfloat16 where the kernels round them; everything else float64."""
+    H = w_k.shape[0]
+    rounded = lambda t: t.float().bfloat16().double()
+    q = q.double().view(q.shape[0], H, 128 + dr)
+    outs, row = [], 0
+    for (count, start), lat in zip(cut, latents):
+        c, kr = lat[:, :R].double(), lat[:, R:].double()
+        k, v = rounded(torch.einsum("hdr,nr->hnd", w_k.double(), c)), rounded(torch.einsum("hdr,nr->hnd", w_v.double(), c))
+        for i in range(count):
+            pos, x = start + i, q[row]
+            s = torch.einsum("hd,hnd->hn", x[:, :128], k[:, :pos + 1])
+            if dr:
+                cos, sin = table[pos, :32].double(), table[pos, 32:].double()
+                a, b = x[:, 128:160], x[:, 160:]
+                s = s + rounded(torch.cat([a * cos - b * sin, b * cos + a * sin], -1)) @ kr[:pos + 1].T
+            s = s * scale
+            if sink is not None:
+                s = torch.cat([s, sink.double()[:, None]], 1)
+            w = torch.softmax(s, -1)[:, :pos + 1]
+            o = torch.einsum("hn,hnd->hd", w, v[:, :pos + 1])
+            if gate is not None:
+                g = torch.sigmoid(gate[row].double())
+                o = o * (g[:H, None] if per_head else g.view(H, 128))
+            outs.append(o.flatten())
+            row += 1
+    return torch.stack(outs)
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("R, dr, H, ps, cut, gate, sinks", [
+    # one to three blocks, ends inside blocks and units; a request behind a context beside whole prompts; walks of several turns
+    (256, 64, 2, 16, [(1, 0), (31, 0), (32, 0), (33, 0), (64, 0), (65, 0)], "channel", False),
+    (256, 64, 3, 8, [(200, 0), (5, 130), (129, 31)], "head", False),
+    (256, 0, 1, 16, [(1, 95), (2, 300), (128, 1)], None, True),
+    (128, 64, 2, 32, [(70, 0), (1, 0), (161, 64)], None, False),
+    (128, 0, 5, 16, [(97, 0)] + [(2, 3)] * 70, "head", True),
+])
+def test_against_float64(R, dr, H, ps, cut, gate, sinks, wide, monkeypatch):
+    from minivllm_amd.engine.step import AttentionPlan
+    from minivllm_amd.kernels.ops import Ops, latent_operands
+    from minivllm_amd.parts import Workspace
+    ops = Ops(torch.bfloat16)
+    monkeypatch.setattr(ops, "compute_units", 0 if wide else 1 << 20)
+    gen = torch.Generator().manual_seed(5)
+    rand = lambda *shape: torch.randn(*shape, generator=gen)
+    lens, starts = [c for c, _ in cut], [s for _, s in cut]
+    context = [c + s for c, s in cut]
+    n, pad = sum(lens), 3                                  # three rows of no request at the end
+    latents = [rand(c, R + dr).bfloat16() for c in context]
+    per = [-(-c // ps) for c in context]
+    order, at = torch.randperm(sum(per) + 2, generator=gen).tolist(), 0
+    pages = torch.full((sum(per) + 2, ps, R + dr), float("nan"))       # slots that were never written
+    table_of = torch.full((len(cut) + 1, max(per) + 1), -1, dtype=torch.int32)
+    for i, (lat, p) in enumerate(zip(latents, per)):
+        table_of[i, :p] = torch.tensor(order[at:at + p], dtype=torch.int32)
+        for j in range(p):
+            rows = lat[j * ps:(j + 1) * ps]
+            pages[order[at + j], :rows.shape[0]] = rows.float()
+        at += p
+    i32 = lambda x: torch.tensor(list(x), dtype=torch.int32, device=DEV)
+    cu = i32([0] + torch.tensor(lens).cumsum(0).tolist() + [n])        # (one request without a token)
+    positions = i32([p for c, s in cut for p in range(s, s + c)] + [0] * pad)
+    token_seq = i32([i for i, c in enumerate(lens) for _ in range(c)] + [-1] * pad)
+    q = (rand(n + pad, H * (128 + dr)) / math.sqrt(128 + dr) * 4).bfloat16()
+    w_k, w_v = (rand(H, 128, R) / math.sqrt(R)).bfloat16(), (rand(H, 128, R) / math.sqrt(R)).bfloat16()
+    angle = rand(max(context), 32)
+    table = torch.cat([angle.cos(), angle.sin()], 1) if dr else None
+    sink = rand(H) if sinks else None
+    g = rand(n + pad, H if gate == "head" else H * 128).bfloat16() if gate else None
+    dev = lambda t: None if t is None else t.to(DEV)
+    plan = AttentionPlan(decode_only=False, max_q_len=max(lens), max_context_len=max(context), n_seqs=len(cut) + 1, q_lens=lens + [0],
+                         cu_seqlens=cu, workspace=Workspace(torch.device(DEV)), starts=starts)
+    blocks = sum(-(-c // 32) for c in context) + 3         # (more than there are)
+    k = torch.full((blocks, H, 4096), float("nan"), dtype=torch.bfloat16, device=DEV)
+    v, kr = torch.full_like(k, float("nan")), torch.full((blocks, 32 * max(dr, 1)), float("nan"), dtype=torch.bfloat16, device=DEV)
+    out = torch.full((n + pad, H * 128), float("nan"), dtype=torch.bfloat16, device=DEV)
+    lens_d = i32(context + [0])
+    ops.latent_expand(dev(pages).bfloat16(), dev(table_of), ps, plan, lens_d, dev(latent_operands(w_k)), dev(latent_operands(w_v)), H, R, dr, blocks, k, kr, v)
+    ops.attention_latent_heads(dev(q), out, k, kr, v, plan, positions, token_seq, lens_d, H, dr, 0.3, dev(table), dev(sink), dev(g), gate == "head")
+    want = reference(q[:n], latents, cut, w_k, w_v, table, 0.3, sink, None if g is None else g[:n], gate == "head", R, dr)
+    got = out.double().cpu()
+    assert not got[n:].abs().max()
+    # a weight and the result are rounded to eight bits each, 2^-9 of either at most (float32 sums of keys may round the other way, rarely)
+    assert (got[:n] - want).norm() / want.norm() <= 2 * 2.0 ** -9
+    worst = (got[:n] - want).abs().amax(1) / want.pow(2).mean(1).sqrt()
+    assert worst.max() <= 16 * 2.0 ** -9                   # every row, its largest channel four times its mean
+
+
+def test_a_recorded_model_follows_the_eager_one():
+    """Prompts of one size class whose attention makes the heads' keys, beside a context and without, recorded and eagerly."""
+    from minivllm_amd.config import EngineConfig
+    from minivllm_amd.engine.executor import Executor
+    from minivllm_amd.engine.step import SeqStep
+    from minivllm_amd.models import config_from_dict, expected_tensors
+    from minivllm_amd.weights.device_random import DeviceRandomSource
+    latent = {"heads": 2, "dim": 128, "rot_dim": 64, "vdim": 128, "q_rank": 64, "kv_rank": 128, "scale": 0.07, "rot": {"dims": 64, "base": 1e4}}
+
+    def executor(graphs):
+        arch, cfg = config_from_dict({"architecture": "Dutilix", "vocab": 256, "width": 128, "norm": {"eps": 1e-5}, "torch_dtype": "bfloat16",
+                                      "logit_scale": 1.0, "layers": [{"type": "latent_attention", "mixer": latent,
+                                                                      "mlp": {"kind": "dense", "ff": 128}}] * 2})
+        source = DeviceRandomSource(expected_tensors(arch, cfg), 1, torch.bfloat16, torch.device(DEV), std=0.08)
+        return Executor(EngineConfig(model="", dtype="bfloat16", max_model_len=1024, max_num_batched_tokens=1024, max_num_batched_seqs=16,
+                                     kv_cache_block_size=16, kv_cache_num_blocks=256, use_cuda_graph=graphs), model=(arch, cfg, source))
+    recorded, eager = executor(True), executor(False)
+    gen = torch.Generator().manual_seed(3)
+    text = [torch.randint(0, 256, (700,), generator=gen).tolist() for _ in range(3)]
+    tables = [list(range(44 * s, 44 * s + 44)) for s in range(3)]
+    for turn in range(3):
+        for cut in ([(100, 0)], [(97, 0)], [(60, 0), (45, 0)], [(90, 0), (1, 0), (14, 0)], [(100, 97)], [(99, 90)]):
+            made = [SeqStep(tokens=text[s][start:start + q], start=start, block_tables=[tables[s]], state_slot=s, want=[q - 1])
+                    for s, (q, start) in enumerate(cut)]
+            got, plain = recorded.step(made).clone(), eager.step(made).clone()
+            assert float((got - plain).abs().max() / plain.abs().max()) <= 2e-2, cut
+    entries = [{e[0] for e in ledger} for ledger in recorded.graph_ledger.values()]
+    assert entries and all("mv_attention_latent_heads" in e and "mv_attention_latent_prompt" not in e for e in entries)

@@ -33,3 +33,27 @@ def test_the_cut_that_choices_follow():
     plan.path_lens, plan.path_starts = (9, 1), (0, 29)
     assert plan.cut() == ((9, 1), (0, 29))
     assert Ops.latent_shares(SimpleNamespace(compute_units=256), 16, -1, *AttentionPlan(False, 9, 30, 1, q_lens=[9]).cut())
+
+
+@pytest.mark.parametrize("heads, prompts, decoding, own", [
+    # both sides measured, at least 8 % apart: (tokens, first position) of prompts, (requests, position) of decoded tokens
+    (16, [(20, 0)], (0, 0), True), (16, [(2048, 0)], (0, 0), True), (16, [(16, 2000)], (0, 0), True), (16, [(16, 0)], (8, 1000), True),
+    (16, [(64, 0)], (17, 700), False), (16, [(300, 0)], (16, 1900), False), (16, [(16, 0)], (64, 1000), False), (16, [(9, 500)] * 40, (0, 0), False),
+    (64, [(100, 0)], (0, 0), True), (64, [(64, 1000)], (0, 0), True), (64, [(16, 0)], (16, 1000), False), (64, [(300, 0)], (16, 1000), False)])
+def test_when_the_heads_have_keys_of_their_own(heads, prompts, decoding, own):
+    lens, starts = [1] * decoding[0] + [q for q, _ in prompts], [decoding[1] - 1] * decoding[0] + [s for _, s in prompts]
+    room = Ops.latent_heads(SimpleNamespace(compute_units=256), heads, lens, starts)
+    assert (room > 0) is own
+    assert room == 0 or room * 32 >= sum(lens) + sum(starts)
+
+
+def test_room_for_own_keys_is_bounded():
+    """Steps of similar sizes have one room; no step has more than what is reserved for the engine's sizes."""
+    ops = SimpleNamespace(compute_units=256)
+    rooms = {Ops.latent_heads(ops, 16, [n], [0]) for n in range(1800, 2049)}
+    assert rooms == {64}
+    assert Ops.latent_heads(ops, 16, [], []) == 0 and Ops.latent_heads(ops, 16, [1, 1], [900, 20]) == 0
+    most = Ops.latent_heads_most(ops, 16, 512, 4, 1024)
+    for lens, starts in (([512], [0]), ([128] * 4, [896] * 4), ([2] * 4, [1022] * 4), ([2], [0]), ([100, 100, 100], [924, 100, 0])):
+        assert Ops.latent_heads(ops, 16, lens, starts) <= most
+    assert Ops.latent_heads(ops, 64, [64], [40000]) == 0 and Ops.latent_heads_most(ops, 64, 8192, 256, 40960) == 512
