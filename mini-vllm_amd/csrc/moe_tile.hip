@@ -11,11 +11,16 @@
 //   moe_tile      out[pair] = act[pair] W_down^T as floats
 //   moe_combine   y[token] = its places' out rows in order, the shared expert's, (identity weights) * x[token], added in float
 //
-// What bounds it: at 2,048 tokens, 32 experts of 768 x 1024 and 4 a token, the bytes (151 MB of weights) are worth 30 us, the
-// products 57; measured 54 (gate and up) + 41 (down) + 9 (moe_pairs) + 8 (combine) us a layer, where every expert for every
-// token took 167 + 175 through the library and 38 for the activation between; 1,000 tokens beside a shared expert 54 + 28 + 6 + 5
-// against 110 + 154 + 26. Eight rows: 47 us a layer with the routing against 55 (the unchosen experts' weights are not read).
+// What bounds it: the bytes of the weights that were chosen, and how evenly tiles fill the compute units: 32 experts of 768 x 1024, 4 a
+// token, are 151 MB, worth 30 us. With tiles of 128 x 128 and two workgroups a compute unit 1,000 tokens (125 pairs an expert, so every third
+// expert had a second tile, nearly empty) beside a shared expert took 89 us a layer, 2,048 tokens 109, 500 62; with tiles of up to 160
+// rows and 256 columns, one workgroup of eight waves a unit, chosen so that no round is nearly empty (mt_rows), and an activation of few
+// instructions (GatedPair::of_short; alone 4 us of 89) 67.5, 97 and 56, of which 6 to 9 are moe_pairs and 5 to 8 the combination. Every
+// expert for every token took 110 + 154 + 26 at 1,000. Eight rows: 47 us a layer with the routing against 55 (the unchosen experts' weights
+// are not read).
 #include "gemm_ring.h"
+
+#include <cmath>
 
 #define MT_MAX_E 1024
 
@@ -90,19 +95,20 @@ struct MoeTileArgs {
     GatedPair pair;
 };
 
-template <int WM, int WN, bool GATED, int STAGES, int OCC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
+// Waves stand GM down the rows and GN along the columns, each with WM x WN products of 16 x 16.
+template <int WM, int WN, int GM, int GN, bool GATED, int STAGES>
+__global__ void __launch_bounds__(64 * GM * GN) __attribute__((amdgpu_waves_per_eu(2, 2)))
 moe_tile_kernel(MoeTileArgs a) {
-    constexpr int BM = 32 * WM, BN = 32 * WN;
-    constexpr int ROWS = BM + BN, INSTR = ROWS / 8, REPS = INSTR / 4;
-    static_assert(INSTR % 4 == 0 && (!GATED || WN % 2 == 0) && STAGES >= 2 && STAGES <= 4 && (STAGES - 2) * REPS <= 63, "");
+    constexpr int BM = 16 * WM * GM, BN = 16 * WN * GN, WAVES = GM * GN;
+    constexpr int ROWS = BM + BN, INSTR = ROWS / 8, REPS = (INSTR + WAVES - 1) / WAVES, LEAST = INSTR / WAVES;
+    static_assert((!GATED || WN % 2 == 0) && STAGES >= 2 && STAGES <= 4 && (STAGES - 2) * REPS <= 63, "");
     constexpr int STAGE = ROWS * 8;
     __shared__ uint4 ring[STAGES * STAGE];
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / MV_WAVE);
     const int lane = tid % MV_WAVE, i = lane % 16, g = lane / 16;
-    const int wm = wave / 2, wn = wave % 2;
+    const int wm = wave / GN, wn = wave % GN;
     // An XCD walks a run of tiles with all their columns: an expert's tiles stand side by side, so its weights go into one L2.
     // The runs are cut from the tiles that there are, not from the most there could be (what the grid is sized for): so cut, the
     // last XCDs had none: 2,048 tokens, 32 experts, 4 a token 70.2 -> 53.6 us (gate and up), 42.2 -> 40.9 (down); 1,000 tokens
@@ -125,7 +131,7 @@ moe_tile_kernel(MoeTileArgs a) {
     int slot[REPS];
 #pragma unroll
     for (int rep = 0; rep < REPS; ++rep) {
-        const int j = wave + 4 * rep, row = 8 * j + lrow;
+        const int j = wave + WAVES * rep, row = 8 * j + lrow;
         slot[rep] = j * 64;
         if (row < BM) {
             const int p = a.t.sorted[row0 + (row < count ? row : 0)];          // rows past the end: some pair; never stored
@@ -149,7 +155,8 @@ moe_tile_kernel(MoeTileArgs a) {
     auto fetch = [&](int c, uint4* stage) {
 #pragma unroll
         for (int rep = 0; rep < REPS; ++rep)
-            gt_load_to_lds(src[rep] + (size_t)c * (GT_KC * sizeof(bf16)), (__attribute__((address_space(3))) void*)(stage + slot[rep]));
+            if (INSTR % WAVES == 0 || rep < LEAST || wave < INSTR % WAVES)
+                gt_load_to_lds(src[rep] + (size_t)c * (GT_KC * sizeof(bf16)), (__attribute__((address_space(3))) void*)(stage + slot[rep]));
     };
     int a_off[WM], w_off[WN];
 #pragma unroll
@@ -157,7 +164,7 @@ moe_tile_kernel(MoeTileArgs a) {
 #pragma unroll
     for (int t = 0; t < WN; ++t) {
         int group;
-        if (GATED) group = t < WN / 2 ? (WN / 2) * wn + t : WN + (WN / 2) * wn + (t - WN / 2);
+        if (GATED) group = t < WN / 2 ? (WN / 2) * wn + t : (WN / 2) * (GN + wn) + (t - WN / 2);
         else group = WN * wn + t;
         w_off[t] = (BM + 16 * group + i) * 8;
     }
@@ -190,10 +197,11 @@ moe_tile_kernel(MoeTileArgs a) {
     int st = 0, st_fetch = STAGES - 1;
     for (int k = 0; k < n; ++k) {
         const int later = n - k - 1 < STAGES - 2 ? n - k - 1 : STAGES - 2;
+        // (a wave has LEAST or one more loads a chunk on their way; a wait for the fewer covers both)
         switch (later) {
             case 0: GT_WAIT_VMCNT(0); break;
-            case 1: GT_WAIT_VMCNT(REPS); break;
-            default: GT_WAIT_VMCNT(2 * REPS); break;
+            case 1: GT_WAIT_VMCNT(LEAST); break;
+            default: GT_WAIT_VMCNT(2 * LEAST); break;
         }
         __builtin_amdgcn_s_barrier();
         if (k + STAGES - 1 < n) fetch(k + STAGES - 1, ring + st_fetch * STAGE);
@@ -216,7 +224,7 @@ moe_tile_kernel(MoeTileArgs a) {
             if constexpr (GATED) {
                 float v[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = weight * a.pair.of(acc[t][u][e], acc[t + WN / 2][u][e]);
+                for (int e = 0; e < 4; ++e) v[e] = weight * a.pair.of_short(acc[t][u][e], acc[t + WN / 2][u][e]);
                 *reinterpret_cast<uint2*>(a.act + (size_t)p * a.ld_act + col) =
                     uint2{f32x2_to_bf16x2_bits(v[0], v[1]), f32x2_to_bf16x2_bits(v[2], v[3])};
             } else {
@@ -257,19 +265,90 @@ moe_pairs_combine_kernel(const float* __restrict__ out, const int* __restrict__ 
 }
 
 template <bool GATED>
-static int launch_moe_tiles(MoeTileArgs& a, int wm, int wn, hipStream_t stream) {
-    const int n_out = GATED ? (a.F > a.FS ? a.F : a.FS) : a.N, bn = (GATED ? 16 : 32) * wn;
+static int launch_moe_tiles(MoeTileArgs& a, int wm, int columns, hipStream_t stream) {
+    const int n_out = GATED ? (a.F > a.FS ? a.F : a.FS) : a.N, bn = columns / (GATED ? 2 : 1);
     a.tiles_n = (n_out + bn - 1) / bn;
     const long blocks = ((long)a.t.max_tiles * a.tiles_n + GT_XCDS - 1) / GT_XCDS * GT_XCDS;
     MV_REQUIRE(blocks < (1L << 31), "moe_tile: too many tiles");
-#define MT_LAUNCH(WM, WN, STAGES, OCC) \
-    hipLaunchKernelGGL((moe_tile_kernel<WM, WN, GATED, STAGES, OCC>), dim3((unsigned)blocks), dim3(256), 0, stream, a)
-    if (wm == 1 && wn == 2) MT_LAUNCH(1, 2, 4, 2);
-    else if (wm == 1) MT_LAUNCH(1, 4, 4, 2);
-    else if (wm == 2) MT_LAUNCH(2, 4, 3, 2);
-    else MT_LAUNCH(4, 4, 2, 2);
+#define MT_LAUNCH(WM, WN, GN, STAGES) \
+    hipLaunchKernelGGL((moe_tile_kernel<WM, WN, 2, GN, GATED, STAGES>), dim3((unsigned)blocks), dim3(128 * GN), 0, stream, a)
+    if (columns == 256) {
+        if (wm == 1) MT_LAUNCH(1, 4, 4, 4);
+        else if (wm == 2) MT_LAUNCH(2, 4, 4, 4);
+        else if (wm == 3) MT_LAUNCH(3, 4, 4, 3);
+        else if (wm == 4) MT_LAUNCH(4, 4, 4, 3);
+        else MT_LAUNCH(5, 4, 4, 3);
+    } else if (columns == 64) MT_LAUNCH(1, 2, 2, 4);
+    else if (wm == 1) MT_LAUNCH(1, 4, 2, 4);
+    else if (wm == 2) MT_LAUNCH(2, 4, 2, 3);
+    else if (wm == 3) MT_LAUNCH(3, 4, 2, 2);
+    else if (wm == 4) MT_LAUNCH(4, 4, 2, 2);
+    else MT_LAUNCH(5, 4, 2, 2);
 #undef MT_LAUNCH
     return mv_check_launch("moe_tile");
+}
+
+// Tiles of `rows` pairs that `experts` runs of `mean` pairs on average have in all: a run's length taken as normal around its mean, a
+// third wider than dice would make it.
+static double mt_tiles(int experts, double mean, int rows) {
+    const double width = 1.3 * sqrt(mean) * 1.41421356;
+    double tiles = 0;
+    for (int k = 0; k * (double)rows < mean + 5 * width; ++k) tiles += 0.5 * erfc((k * (double)rows + 0.5 - mean) / width);
+    return experts * (tiles < mean ? tiles : mean);
+}
+
+// Columns of a tile (W's rows) where a product has so many tiles of rows and columns: 256, one workgroup of eight waves a compute unit,
+// where those find work for more than half of the units; else 128, two workgroups of four waves each.
+static int mt_columns(double row_tiles, int n_out, int halves, int units) {
+    return row_tiles * ((n_out * halves + 255) / 256) >= 0.55 * units ? 256 : 128;
+}
+
+// Rows of a tile, in 32s. A tile takes as long as its operands take through its compute unit, 77 KB a us: (rows + columns) * 128 bytes a
+// chunk of 64 columns of K; tiles come in rounds; and the weights come from memory whatever the tiles. Of 1 to 5 the one with the least
+// sum over both products: within 2 % of the best of all ten shapes over 22 mixtures (mean pairs an expert 5 to 750, 8 to 64 experts,
+// 768 x 1024, 768 x 2048 and 3072 x 4096), the worst one 12 %. 32 experts of 768 x 1024, 4 a token, and a shared one: 256 tokens tiles of 64
+// rows 50 us, of 128 55; 1,000 tokens (125 pairs an expert) 160 rows 66.5, 128 rows 78, the last tiles of the experts with more than 128
+// being a round of their own; 1,500 tokens 128 rows 96, 160 rows 103; 2,048 tokens 160 rows 112, 128 rows 118.
+static int mt_rows(int n, long n_pairs, int n_real, int hidden, int F, int FS, int units) {
+    const double mean = (double)n_pairs / n_real, used = n_pairs < n_real ? n_pairs : n_real;
+    int best = 1;
+    double least = 0;
+    for (int wm = 1; wm <= 5; ++wm) {
+        const int rows = 32 * wm;
+        const double tiles = mt_tiles(n_real, mean, rows) + (FS ? (n + rows - 1) / rows : 0);
+        double cost = 0;
+        for (int gated = 0; gated < 2; ++gated) {
+            const int K = gated ? hidden : F, n_out = gated ? (F > FS ? F : FS) : hidden;
+            const int columns = mt_columns(tiles, n_out, gated ? 2 : 1, units);
+            const double rounds = tiles * ((n_out * (gated ? 2 : 1) + columns - 1) / columns) / units;
+            const double whole = fmax(1.0, 0.5 * (rounds + ceil(rounds)));
+            const double port = whole * (rows + columns + (columns == 256 ? 100 : 150)) * (K / 64.0) * 128 / 77e3;
+            const double memory = (used * F + FS) * hidden * (gated ? 4.0 : 2.0) / 6.2e6;
+            cost += fmax(port, memory) + 0.3 * fmin(port, memory);
+        }
+        if (wm == 1 || cost < least) {
+            best = wm;
+            least = cost;
+        }
+    }
+    return best;
+}
+
+struct MtShape {
+    int wm, in, down;          // rows of a tile in 32s, columns of a tile of the first product and of the second
+};
+static MtShape mt_shape(int n, int top, int n_real, int hidden, int F, int FS, int units) {
+    const long n_pairs = (long)n * top, busy = n_pairs < n_real ? n_pairs : n_real;      // tiles, at most, of a step of few rows
+    const int wm = mt_rows(n, n_pairs, n_real, hidden, F, FS, units), rows = 32 * wm;
+    const double tiles = mt_tiles(n_real, (double)n_pairs / n_real, rows) + (FS ? (n + rows - 1) / rows : 0);
+    // (a step of few rows whose tiles leave compute units idle has narrow ones)
+    return MtShape{wm, wm == 1 && busy * ((F + 63) / 64) < units ? 64 : mt_columns(tiles, F > FS ? F : FS, 2, units),
+                   wm == 1 && busy * ((hidden + 127) / 128) < units ? 64 : mt_columns(tiles, hidden, 1, units)};
+}
+// rows | columns << 10 | columns of the second product << 20 of the tiles that mv_moe_pairs has on a device of so many compute units
+extern "C" int mv_moe_pairs_shape(int n, int top, int n_real, int hidden, int F, int FS, int units) {
+    const MtShape s = mt_shape(n, top, n_real, hidden, F, FS, units);
+    return 32 * s.wm | s.in << 10 | s.down << 20;
 }
 
 // ints of scratch: sorted pairs, the three tile tables, for tiles of 32 rows, and the number of tiles
@@ -293,10 +372,8 @@ extern "C" int mv_moe_pairs(const void* x, long ldx, int n, int hidden, const vo
     if (n == 0) return 0;
     const long n_pairs = (long)n * top, pairs = n_pairs + (FS ? n : 0);
     MV_REQUIRE(pairs < (1L << 30), "moe_pairs: too many pairs");
-    // rows of a tile: about what an expert has on average, since a tile that is mostly empty costs its products all the same
-    // and one that is too low reads its weights twice
-    const long mean = n_pairs / n_real;
-    const int wm = mean > 48 ? 4 : mean > 24 ? 2 : 1, rows = 32 * wm;
+    const MtShape shape = mt_shape(n, top, n_real, hidden, F, FS, mv_compute_units());
+    const int rows = 32 * shape.wm;
     PairTables t;
     t.max_tiles = (int)(pairs / rows + (n_real < n_pairs ? n_real : n_pairs) + 1);
     t.sorted = ints;
@@ -306,17 +383,14 @@ extern "C" int mv_moe_pairs(const void* x, long ldx, int n, int hidden, const vo
     t.n_tiles = t.tile_rows + t.max_tiles;
     hipLaunchKernelGGL(moe_pairs_kernel, dim3(1), dim3(1024), 0, stream, ids, (int)n_pairs, n_real, FS ? n : 0, rows, t);
     if (mv_check_launch("moe_pairs")) return 1;
-    // columns of a tile: half as many where a step's few tiles leave compute units idle
-    const int units = mv_compute_units();
     MoeTileArgs a{(const bf16*)x, ldx, (const bf16*)w_gate_up, (long)hidden, t, weights, top, (int)n_pairs, n_real, F, FS, hidden,
                   (bf16*)act, out, (long)(F > FS ? F : FS), hidden, 0, GatedPair{limit, slope}};
-    const long busy = n_pairs < n_real ? n_pairs : n_real;                     // tiles, at most, of a step of few rows
-    if (launch_moe_tiles<true>(a, wm, wm == 1 && busy * ((F + 63) / 64) < units ? 2 : 4, stream)) return 1;
+    if (launch_moe_tiles<true>(a, shape.wm, shape.in, stream)) return 1;
     a.A = (const bf16*)act;
     a.lda = a.ld_act;
     a.W = (const bf16*)w_down;
     a.ldw = (long)n_real * F + FS;
-    if (launch_moe_tiles<false>(a, wm, wm == 1 && busy * ((hidden + 127) / 128) < units ? 2 : 4, stream)) return 1;
+    if (launch_moe_tiles<false>(a, shape.wm, shape.down, stream)) return 1;
     hipLaunchKernelGGL(moe_pairs_combine_kernel, dim3(n), dim3(256), 0, stream, out, ids, top, (int)n_pairs, n_real, FS ? 1 : 0, (const bf16*)x,
                        ldx, dense, ld_dense, identity, (bf16*)y, ldy, hidden);
     return mv_check_launch("moe_pairs_combine");
