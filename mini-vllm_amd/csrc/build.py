@@ -32,7 +32,7 @@ COMMON_SOURCES = ["runtime.hip", "elementwise.hip", "gemm_ref.hip", "attention_r
                   "recurrent_delta_chunks.hip", "pair_norm.hip", "qkv_conv.hip", "recurrent_gated.hip", "recurrent_unit.hip"]
 VARIANT_SOURCES: Dict[str, List[str]] = {
     "f32": COMMON_SOURCES + ["attention_exact.hip"],
-    "bf16": COMMON_SOURCES + ["gemm_skinny.hip", "gemm_mid.hip", "gemm_tile.hip", "gemm_deep.hip", "moe_tile.hip", "gemm_lt.hip", "attention_fast.hip",
+    "bf16": COMMON_SOURCES + ["gemm_skinny.hip", "gemm_mid.hip", "gemm_tile.hip", "gemm_deep.hip", "gemm_pair.hip", "moe_tile.hip", "gemm_lt.hip", "attention_fast.hip",
                               "attention_prefill.hip", "attention_latent_prompt.hip", "attention_latent_heads.hip"],
 }
 # libraries a variant links against

@@ -1,0 +1,226 @@
+// The gated pair for prompts, rows by the hundred and thousand (bfloat16 in and out, float sums, MFMA):
+//     C[M, I] = pair(A Wg^T (+ bias), A Wu^T (+ bias)),  A [M, K],  W = [Wg | Wu] of [2 I, K]
+// with the activation on the float sums, so that the two products never go to memory.
+//
+// A workgroup of eight waves makes a tile of 64 to 256 rows by 64 to 192 weight rows (half gate, half up) and has a compute unit to itself;
+// operands come through an LDS ring as in gemm_tile.hip, their reads run under the products. What bounds it: a chunk of 64 columns takes
+// 0.15 us (the barrier, and waves that wait for the last of them) and 0.385 us for every 128 x 128 of the tile, 1.39 PFLOP/s, half of it
+// the matrix unit, the rest LDS and issue; and a workgroup takes 3.5 us to its first products and from its last. So tiles are large, and
+// which of the twelve shapes depends on how many whole rounds of compute units they make (mv_gemm_pair_shape): 2,048 x 6144 x 1024
+// is one of 256 x 192. There 36.7 us with the library's product and the activation behind it, 27.7 here; 1,536 rows 34.8 (gemm_tile.hip)
+// and 22.5; 1,024 23.4 and 17.6; 512 17.4 and 13.3; 1,024 x 12288 x 2048 71 and 47; 4,096 x 6144 x 1024 69 and 55. Large products of a long K
+// stay with the library (4,096 x 24576 x 4096: 593 us with the activation, 700 here).
+#include "gemm_ring.h"
+
+#include <cmath>
+
+struct PairArgs {
+    const bf16* A;
+    long lda;
+    const bf16* W;
+    const bf16* bias;
+    bf16* C;
+    long ldc;
+    int M, I, K;
+    int tiles_m, tiles, wide_stores;
+    GatedPair pair;
+};
+
+// Eight waves, four down the rows and two along the columns, each with WM x WN products of 16 x 16.
+template <int WM, int WN, int STAGES>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gemm_pair_kernel(PairArgs a) {
+    constexpr int BM = 64 * WM, BN = 32 * WN, WAVES = 8;
+    constexpr int ROWS = BM + BN, INSTR = ROWS / 8, REPS = (INSTR + WAVES - 1) / WAVES, LEAST = INSTR / WAVES, STAGE = ROWS * 8;
+    static_assert(WN % 2 == 0, "a wave's weight tiles are half gate, half up");
+    static_assert(STAGES >= 2 && STAGES <= 4 && STAGES * STAGE * 16 <= 163840 && (STAGES - 1) * REPS <= 63, "the ring does not fit");
+    __shared__ uint4 ring[STAGES * STAGE];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / MV_WAVE), lane = tid % MV_WAVE, i = lane % 16, g = lane / 16;
+    const int wm = wave / 2, wn = wave % 2;
+    // an XCD has a run of tiles, the rows changing fastest: a band of the weight goes into one L2
+    const int run = (a.tiles + GT_XCDS - 1) / GT_XCDS, id = blockIdx.x % GT_XCDS * run + blockIdx.x / GT_XCDS;
+    if ((int)blockIdx.x / GT_XCDS >= run || id >= a.tiles) return;
+    const int tm = id % a.tiles_m, tn = id / a.tiles_m;
+    const int m0 = tm * BM, n0 = tn * (BN / 2), n = a.K / GT_KC;
+
+    // this lane's share of the loads, and the operands: as in gemm_tile.hip
+    const int lrow = lane / 8, piece = (lane % 8) ^ lrow;
+    const char* src[REPS];
+#pragma unroll
+    for (int rep = 0; rep < REPS; ++rep) {
+        const int row = 8 * (wave + WAVES * rep) + lrow;
+        if (row < BM) {
+            src[rep] = reinterpret_cast<const char*>(a.A + (size_t)min(m0 + row, a.M - 1) * a.lda + 8 * piece);
+        } else {
+            const int r = row - BM;
+            const int w = r < BN / 2 ? min(n0 + r, a.I - 1) : min(a.I + n0 + r - BN / 2, 2 * a.I - 1);
+            src[rep] = reinterpret_cast<const char*>(a.W + (size_t)w * a.K + 8 * piece);
+        }
+    }
+    auto fetch = [&](int c, uint4* stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int rep = 0; rep < REPS; ++rep)
+            if (INSTR % WAVES == 0 || rep < LEAST || wave < INSTR % WAVES)
+                gt_load_to_lds(src[rep] + (size_t)c * (GT_KC * sizeof(bf16)), (__attribute__((address_space(3))) void*)(stage + (wave + WAVES * rep) * 64));
+    };
+    int a_off[WM], w_off[WN];
+#pragma unroll
+    for (int t = 0; t < WM; ++t) a_off[t] = (16 * (WM * wm + t) + i) * 8;
+#pragma unroll
+    for (int t = 0; t < WN; ++t) {
+        const int group = t < WN / 2 ? (WN / 2) * wn + t : (WN / 2) * (2 + wn) + (t - WN / 2);
+        w_off[t] = (BM + 16 * group + i) * 8;
+    }
+    const int sw0 = g ^ (i & 7), sw1 = (4 + g) ^ (i & 7);
+    floatx4_t acc[WN][WM];
+#pragma unroll
+    for (int t = 0; t < WN; ++t)
+#pragma unroll
+        for (int u = 0; u < WM; ++u) acc[t][u] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    struct Operands {
+        TFrag a[WM], w[WN];
+    };
+    auto read = [&](const uint4* stage, int sw, Operands& o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < WN; ++t) o.w[t].u = stage[w_off[t] + sw];
+#pragma unroll
+        for (int u = 0; u < WM; ++u) o.a[u].u = stage[a_off[u] + sw];
+    };
+    auto multiply = [&](const Operands& o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < WM; ++u)
+#pragma unroll
+            for (int t = 0; t < WN; ++t) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[t].v, o.a[u].v, acc[t][u], 0, 0, 0);
+    };
+    auto landed = [&](int later) __attribute__((always_inline)) {      // this wave's loads, but for those of `later` chunks
+        switch (later) {
+            case 0: GT_WAIT_VMCNT(0); break;
+            case 1: GT_WAIT_VMCNT(LEAST); break;
+            case 2: GT_WAIT_VMCNT(2 * LEAST); break;
+            default: GT_WAIT_VMCNT(3 * LEAST); break;
+        }
+    };
+    // Chunk k lives in stage k % STAGES; its operands are read in two halves of 32 columns, each while the products of the half before run.
+    // The barrier stands between the halves: then everybody's reads of chunk k are back, so chunk k + STAGES may come into its stage,
+    // and everybody's loads of chunk k + 1 have landed.
+#pragma unroll
+    for (int k = 0; k < STAGES; ++k)
+        if (k < n) fetch(k, ring + k * STAGE);
+    Operands even, odd;
+    landed(n - 1 < STAGES - 1 ? n - 1 : STAGES - 1);
+    __builtin_amdgcn_s_barrier();
+    read(ring, sw0, even);
+    int st = 0;
+    for (int k = 0; k < n; ++k) {
+        uint4* stage = ring + st * STAGE;
+        st = st + 1 == STAGES ? 0 : st + 1;
+        read(stage, sw1, odd);
+        multiply(even);
+        // (a read, then some products, in turn: as the compiler has them, all reads first, 3 % slower)
+#pragma unroll
+        for (int x = 0; x < WM + WN; ++x) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, WM * WN / (WM + WN) > 0 ? WM * WN / (WM + WN) : 1, 0);
+        }
+        if (k + 1 < n) landed(n - k - 2 < STAGES - 2 ? n - k - 2 : STAGES - 2);
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_s_barrier();
+        if (k + STAGES < n) fetch(k + STAGES, stage);
+        if (k + 1 < n) read(ring + st * STAGE, sw0, even);
+        multiply(odd);
+    }
+
+    // lane l holds C[row 16 u + l % 16][columns 4 (l / 16) .. + 3 of tile t]
+    constexpr int TOUT = WN / 2;
+#pragma unroll
+    for (int t = 0; t < TOUT; ++t) {
+        const int col = n0 + 16 * (TOUT * wn + t) + 4 * g;
+        float bv[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
+        if (a.bias != nullptr) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (col + e < a.I) {
+                    bv[e] = to_f(a.bias[col + e]);
+                    bu[e] = to_f(a.bias[a.I + col + e]);
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < WM; ++u) {
+            const int row = m0 + 16 * (WM * wm + u) + i;
+            if (row >= a.M || col >= a.I) continue;
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = a.pair.of_short(acc[t][u][e] + bv[e], acc[t + TOUT][u][e] + bu[e]);
+            bf16* to = a.C + (size_t)row * a.ldc + col;
+            if (a.wide_stores && col + 3 < a.I) {
+                *reinterpret_cast<uint2*>(to) = uint2{f32x2_to_bf16x2_bits(v[0], v[1]), f32x2_to_bf16x2_bits(v[2], v[3])};
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (col + e < a.I) to[e] = from_f<bf16>(v[e]);
+            }
+        }
+    }
+}
+
+// rows << 16 | weight rows of the tile that M rows against a pair [N = 2 I, K] have on a device of so many compute units; 0: the pair is left to
+// the other kernels. Times in us, ours as said above (tiles wider than tall a little behind, rounds beyond the first 6 % longer each:
+// the rows no longer come from L2); the library's with the activation behind it 8.5, the products at 1.1 to 1.5 PFLOP/s by K or the weight at
+// 4.2 TB/s, and 6 bytes a result at 5 TB/s. Below the size where the library would serve (1,536 rows, weights of 64 MB) the tiled product
+// would, level at 128 rows and behind from there. Over 68 shapes, 129 to 8,192 rows, K of 512 to 4,096, the choice is 1 % behind the best
+// on average, and 2 % behind what ran there before at worst (2,560 x 6144 x 1024); above 6,144 rows the library is ahead again.
+extern "C" int mv_gemm_pair_shape(int M, int N, int K, int units) {
+    if (M <= 128 || M > 6144 || N % 2 || K % GT_KC || N <= 0 || K <= 0 || (double)N * K >= 240e6) return 0;
+    const double chunks = K / GT_KC, memory = 2.0 * N * K / 5e6;
+    int best = 0;
+    double least = 0;
+    for (int bm = 64; bm <= 256; bm += 64)
+        for (int bn = 64; bn <= 192; bn += 64) {
+            const double tiles = (double)((M + bm - 1) / bm) * ((N / 2 + bn / 2 - 1) / (bn / 2)), rounds = ceil(tiles / units);
+            const double one = 3.5 + chunks * (0.15 + 0.385 * bm * bn / 16384.0 + (bn > bm ? 0.01 * (bn - bm) / 64 : 0.0));
+            const double time = 2.0 + fmax(rounds * one * (1.0 + 0.06 * (rounds - 1)), memory);
+            if (best == 0 || time < least) {
+                best = bm << 16 | bn;
+                least = time;
+            }
+        }
+    const double rate = 1.1e9 + 0.4e9 * fmin(1.0, K / 4096.0);
+    const double other = 8.5 + fmax(2.0 * M * N * K / rate, 2.0 * N * K / 4.2e6) + 3.0 * M * N / 5e6;
+    return least < (M > 1536 || 2.0 * N * K >= 64.0 * 1024 * 1024 ? 1.05 : 1.0) * other ? best : 0;
+}
+
+// C [M, I] bf16 (pitch ldc) = pair(A Wg^T (+ bias), A Wu^T (+ bias)) for the packed weight [N = 2 I, K]: K a multiple of 64, A and W at
+// 16-byte addresses, pitch lda a multiple of eight. `tile`: as mv_gemm_pair_shape says, or another of 64, 128, 192, 256 rows by 64, 128, 192.
+extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* bias, void* C, long ldc, int M, int N, int K, float limit, float slope,
+                            int tile, hipStream_t stream) {
+    MV_REQUIRE(M > 0 && N > 0 && K > 0 && K % GT_KC == 0 && N % 2 == 0, "gemm_pair: bad sizes M=%d N=%d K=%d", M, N, K);
+    MV_REQUIRE(A && W && C && lda >= K && lda % 8 == 0 && ((uintptr_t)A | (uintptr_t)W) % 16 == 0 && ldc >= N / 2,
+               "gemm_pair: operands not aligned or pitches too small");
+    const int bm = tile >> 16, bn = tile & 0xffff;
+    MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 128 || bn == 192), "gemm_pair: no tile of %d x %d", bm, bn);
+    const int tiles_m = (M + bm - 1) / bm;
+    const long tiles = (long)tiles_m * ((N / 2 + bn / 2 - 1) / (bn / 2));
+    MV_REQUIRE(tiles < (1L << 30), "gemm_pair: too many tiles");
+    const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N / 2, K, tiles_m, (int)tiles,
+                     ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{limit, slope}};
+    const dim3 grid((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
+#define GP_LAUNCH(WM, WN, S) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, S>), grid, dim3(512), 0, stream, a)
+    if (bn == 192) {
+        if (bm == 256) GP_LAUNCH(4, 6, 2);
+        else if (bm == 192) GP_LAUNCH(3, 6, 3);
+        else if (bm == 128) GP_LAUNCH(2, 6, 4);
+        else GP_LAUNCH(1, 6, 4);
+    } else if (bn == 128) {
+        if (bm == 256) GP_LAUNCH(4, 4, 3);
+        else if (bm == 192) GP_LAUNCH(3, 4, 4);
+        else if (bm == 128) GP_LAUNCH(2, 4, 4);
+        else GP_LAUNCH(1, 4, 4);
+    } else {
+        if (bm == 256) GP_LAUNCH(4, 2, 4);
+        else if (bm == 192) GP_LAUNCH(3, 2, 4);
+        else if (bm == 128) GP_LAUNCH(2, 2, 4);
+        else GP_LAUNCH(1, 2, 4);
+    }
+#undef GP_LAUNCH
+    return mv_check_launch("gemm_pair");
+}

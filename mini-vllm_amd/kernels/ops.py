@@ -54,7 +54,7 @@ LIBRARY_TALL_WEIGHT_GATED = 240 * 1000 * 1000
 # library, where it is ahead of both (measured on MI355X, weights rotating so that they come from memory):
 # a gated pair with the activation in its epilogue from 32 rows on (0.6B sizes at 64 rows: 7.7 us
 # against the weight-streaming kernel's 11.4 and the library's 13.8 with the activation as a kernel of
-# its own; at 1,024 rows 21.6 against 24.6; level from 1,536 on), for weights of 64 MB and more up to 128
+# its own; from 129 rows on gemm_pair.hip is ahead of both where it takes the size), for weights of 64 MB and more up to 128
 # rows (8B sizes at 64 rows 44 against 51 us; at 256 the library is ahead); a plain product against a
 # small weight with at least 4,096 rows (enough tiles without splitting K) from 40 to 512 rows (0.6B qkv
 # at 64 rows 6.8 against 7.8 us, at 256 rows 7.2 against the library's 9.0; weights with fewer rows go to
@@ -2692,6 +2692,23 @@ class Ops:
                       0 if work is None else work.numel(), force, float(limit), float(slope), int(square_relu), self._stream())
         return True
 
+    def _gemm_pair(self, a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor], limit: float, slope: float) -> bool:
+        """The gated pair of a prompt's rows in one pass (gemm_pair.hip, whose ``mv_gemm_pair_shape`` says for which sizes); False, with
+        nothing done, where it is left to the other kernels."""
+        if not self.use_tiled_gemm or not self.lib.has("mv_gemm_pair"):
+            return False
+        (M, K), N = a.shape, w.shape[0]
+        tile = self.lib.dll.mv_gemm_pair_shape(M, N, K, self.compute_units)
+        if (not tile or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or not w.is_contiguous()
+                or w.shape[1] != K or a.stride(1) != 1 or a.stride(0) % 8 or a.data_ptr() % 16 or w.data_ptr() % 16
+                or out.shape != (M, N // 2) or out.stride(1) != 1):
+            return False
+        self._act(a, "gemm input"); self._act(out, "swiglu output"); _dev(w, "gate_up weight")
+        self._note("mv_gemm_pair", self._size(a, w, out), 2 * M * N * K)
+        self.lib.call("mv_gemm_pair", a.data_ptr(), a.stride(0), w.data_ptr(), _ptr(bias), out.data_ptr(), out.stride(0), M, N, K, float(limit),
+                      float(slope), tile, self._stream())
+        return True
+
     @staticmethod
     def wants_mid(M: int, N: int, K: int) -> bool:
         """Whether a product of M rows with an [N, K] weight goes to the kernel that splits K (it takes
@@ -2839,6 +2856,8 @@ class Ops:
             return False
         M, K = a.shape
         two_i = w_gate_up.shape[0]
+        if self._gemm_pair(a, w_gate_up, out, bias, limit, slope):
+            return True
         if self.wants_tile(M, two_i, K, gated=True) and self.gemm_tile(
                 a, w_gate_up, out, bias, gated=True, limit=limit, slope=slope):
             return True

@@ -1,0 +1,55 @@
+"""The gated pair of a prompt's rows: every shape of tile and its edges, against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def pair(x, w, bias, limit, slope):
+    p = x.double() @ w.double().T + (0 if bias is None else bias.double())
+    g, u = p[:, :p.shape[1] // 2], p[:, p.shape[1] // 2:]
+    if limit > 0:
+        g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+        return g * torch.sigmoid(slope * g) * (u + 1)
+    return g * torch.sigmoid(slope * g) * u
+
+
+@pytest.mark.parametrize("bm", [64, 128, 192, 256])
+@pytest.mark.parametrize("bn", [64, 128, 192])
+@pytest.mark.parametrize("M, I, K, bias, limit", [(1, 8, 64, False, 0.0), (255, 100, 128, True, 0.0), (257, 97, 192, True, 1.5), (300, 192, 640, False, 0.0),
+                                                  (577, 333, 320, True, 1.5)])
+def test_tiles(bm, bn, M, I, K, bias, limit):
+    """Rows, columns and chunks of K that end inside, at and behind a tile and the ring's stages; columns at odd places, pitches of the
+    rows. Sums are float: what remains is the rounding of the result to bfloat16, 2^-9 of it (2^-8 with the sums' own error where
+    gate and up nearly cancel)."""
+    from minivllm_amd.kernels.ops import get_ops
+    ops = get_ops(torch.bfloat16)
+    g = torch.Generator(device=DEV).manual_seed(M + I)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x = rand(M, K + 8).bfloat16()[:, :K]
+    w = (rand(2 * I, K) / K ** 0.5 * 2).bfloat16()
+    b = rand(2 * I).bfloat16() if bias else None
+    out = torch.full((M + 1, I + 3), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.lib.call("mv_gemm_pair", x.data_ptr(), x.stride(0), w.data_ptr(), 0 if b is None else b.data_ptr(), out.data_ptr(), out.stride(0), M, 2 * I, K,
+                 limit, 1.702 if limit else 1.0, bm << 16 | bn, torch.cuda.current_stream().cuda_stream)
+    want = pair(x, w, b, limit, 1.702 if limit else 1.0)
+    error = (out[:M, :I].double() - want).abs()
+    assert bool((error <= 2.0 ** -8 * want.abs() + 1e-4).all())
+    assert bool((out[M] == 7.0).all()) and bool((out[:, I:] == 7.0).all())
+
+
+@pytest.mark.parametrize("M, I, K", [(129, 3072, 1024), (512, 3072, 1024), (2048, 768, 512)])
+def test_prompts_take_it(M, I, K):
+    """Through the engine's entry point, which leaves these sizes to it, with and without the pitch that stores of four need."""
+    from minivllm_amd.kernels.ops import get_ops
+    ops = get_ops(torch.bfloat16)
+    x, w = torch.randn(M, K, device=DEV).bfloat16(), (torch.randn(2 * I, K, device=DEV) / K ** 0.5).bfloat16()
+    for pitch in (I, I + 1):
+        out = torch.zeros(M, pitch, dtype=torch.bfloat16, device=DEV)[:, :I]
+        ops.ledger = []
+        assert ops.gemm_swiglu(x, w, out)
+        ran, ops.ledger = [e[0] for e in ops.ledger], None
+        assert ran == ["mv_gemm_pair"]
+        want = pair(x, w, None, 0.0, 1.0)
+        assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
