@@ -17,9 +17,13 @@ __device__ __forceinline__ void decay_dots(const W* __restrict__ w2t_c, size_t i
                                            int j1, float (&acc)[NT]) {
     int j = j0;
     for (; j + 8 <= j1; j += 8) {
+        W raw[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) raw[e] = w2t_c[(size_t)(j + e) * inner];
+        __builtin_amdgcn_sched_barrier(0);                     // (16-bit loads would be waited for one by one)
         float w[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) w[e] = to_f(w2t_c[(size_t)(j + e) * inner]);
+        for (int e = 0; e < 8; ++e) w[e] = to_f(raw[e]);
 #pragma unroll
         for (int e = 0; e < 8; ++e)
 #pragma unroll
