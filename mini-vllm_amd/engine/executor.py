@@ -26,7 +26,7 @@ import torch
 
 from ..cache.manager import CacheManager, GroupSpec, groups_from_needs
 from ..config.engine_config import EngineConfig, compute_dtype_name
-from ..kernels.ops import Ops, dtype_from_name
+from ..kernels.ops import Ops, StateRows, dtype_from_name
 from ..models.causal_lm import CausalLM, expected_tensors
 from ..models.registry import Architecture, load_config
 from ..parts.base import Runtime, Workspace
@@ -220,6 +220,8 @@ class Executor:
                 self.state_tensors[call] = {name: torch.zeros((self.num_state_slots,) + tuple(dims), dtype=dt,
                                                               device=self.device)
                                             for name, (dims, dt) in shapes.items()}
+        if self.state_tensors:
+            self._state_rows = StateRows([t for tensors in self.state_tensors.values() for t in tensors.values()])
         if cfg.kv_cache_num_blocks is not None:
             given = cfg.kv_cache_num_blocks
             sizes = [int(given)] * len(self.groups) if isinstance(given, int) else [int(n) for n in given]
@@ -510,16 +512,12 @@ class Executor:
         return self.model.forward(ctx)
 
     def _zero_new_states(self, seqs: Sequence[SeqStep]) -> None:
-        """A request that starts at position 0 starts from a cleared state: one indexed fill per
-        state tensor, whatever the number of such requests."""
+        """A request that starts at position 0 starts from a cleared state: its row of every state tensor."""
         if not self.has_state:
             return
         fresh = [s.state_slot for s in seqs if s.start == 0]
         if fresh:
-            index = torch.tensor(fresh, dtype=torch.int64, device=self.device)
-            for tensors in self.state_tensors.values():
-                for t in tensors.values():
-                    t.index_fill_(0, index, 0)
+            self.ops.zero_rows(self._state_rows, fresh)
 
     def _context_cap(self, seqs: Sequence[SeqStep]) -> int:
         """The context length a decode graph is planned for: the next power of two (at least

@@ -29,6 +29,7 @@ _LIBRARY = r"^((Custom_)?Cijk_|void hipblaslt|hipblaslt|.*rocblaslt)|\b" + _OWN
 KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_embedding": (r"\bembedding(_gather)?_kernel", None, 1),
     "mv_gather_rows": (r"\bembedding_kernel", None, 1),
+    "mv_zero_rows": (r"\bzero_rows_kernel", None, 1),
     "mv_add_rmsnorm": (r"\badd_rmsnorm(_vec)?_kernel", None, 1),
     "mv_add_rmsnorm_split": (r"\badd_rmsnorm(_vec)?_kernel", None, 1),
     "mv_rmsnorm": (r"\brmsnorm_kernel", None, 1),

@@ -377,6 +377,8 @@ _OPTIONAL_SIGNATURES = {
     # y, ldy, x, ldx, rows, cols, dtype, stream
     "mv_add_rows": (c_int, [c_void_p, c_long, c_void_p, c_long, c_int, c_int, c_int, c_void_p]),
     "mv_launch_empty": (c_int, [c_int, c_int, c_void_p, c_void_p]),
+    # table, tensors, longest, rows, count, bound, stream
+    "mv_zero_rows": (c_int, [c_void_p, c_int, c_long, c_void_p, c_int, c_int, c_void_p]),
 }
 
 

@@ -7,6 +7,7 @@ from __future__ import annotations
 
 from typing import Optional, Sequence
 
+import ctypes
 import math
 import operator
 import os
@@ -144,6 +145,22 @@ def _weight_code(w: torch.Tensor, what: str) -> int:
 
 
 _SQUARED = object()      # what ``Ops.gemm`` returns when the product's kernel applied the squared ReLU too
+
+
+class StateRows:
+    """Tensors of one row per request whose rows ``Ops.zero_rows`` clears together, listed on the device."""
+
+    def __init__(self, tensors: Sequence[torch.Tensor]):
+        self.tensors = [t for t in tensors if t.numel()]
+        for t in self.tensors:
+            _dev(t, "state")
+            if not t.is_contiguous() or t.shape[0] != self.tensors[0].shape[0]:
+                raise KernelLibraryError("zero_rows: contiguous tensors with the same number of rows are served")
+        sizes = [t[0].numel() * t.element_size() for t in self.tensors]
+        self.rows = self.tensors[0].shape[0] if self.tensors else 0
+        self.longest, self.bytes = max(sizes, default=0), sum(sizes)
+        self.table = torch.tensor([[t.data_ptr(), n] for t, n in zip(self.tensors, sizes)], dtype=torch.int64,
+                                  device=self.tensors[0].device if self.tensors else None)
 
 
 class SplitSum:
@@ -333,6 +350,15 @@ class Ops:
         self._note("mv_gather_rows", n * (8 * out.shape[1] + 4))      # (a name of its own: "mv_embedding" starts a model step)
         self.lib.call("mv_embedding", index.data_ptr(), table.data_ptr(), DTYPE_F32, out.data_ptr(), n, table.shape[1],
                       table.shape[0], 1.0, self._stream())
+
+    def zero_rows(self, states: "StateRows", rows: Sequence[int]) -> None:
+        """Sets the given rows of all the tensors in ``states`` to zero, in one launch (per 64 rows)."""
+        if not states.tensors:
+            return
+        picked = (ctypes.c_int * len(rows))(*rows)
+        self._note("mv_zero_rows", len(rows) * states.bytes)
+        self.lib.call("mv_zero_rows", states.table.data_ptr(), len(states.tensors), states.longest, ctypes.addressof(picked),
+                      len(rows), states.rows, self._stream())
 
     def add_rmsnorm(self, resid: torch.Tensor, delta: Optional[torch.Tensor], weight: Optional[torch.Tensor],
                     eps: float, out: Optional[torch.Tensor], rows: Optional[torch.Tensor] = None,
