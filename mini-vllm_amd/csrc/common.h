@@ -216,6 +216,15 @@ int mv_fail(const char* fmt, ...);
 int mv_check_launch(const char* what);
 int mv_compute_units();     // of the current device (runtime.hip)
 
+// Rows that a recorded step of M rows is padded to, or a step of its class not recorded could be: at most an eighth more. What adds in
+// another order than the kernel beside it is chosen by these, so that a step gives the same bits recorded and not.
+inline int mv_class_rows(int M) {
+    if (M <= 8) return M;
+    int step = 16;
+    while (M > 8 * step) step *= 2;
+    return (M + step - 1) / step * step;
+}
+
 #define MV_REQUIRE(cond, ...)                      \
     do {                                           \
         if (!(cond)) return mv_fail(__VA_ARGS__);  \

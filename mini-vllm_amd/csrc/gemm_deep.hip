@@ -269,13 +269,6 @@ static long deep_tiles(int shape, int M, int columns, bool gated) {
 // pairs of a longer K have no such end: 500 x 1024 x 8192 56.7 / 27.1.
 // The other kernels add in other orders, so which one serves is decided by the rows that a recorded step is padded to (all shapes
 // here add a weight up in one order): a step gives the same bits recorded and not.
-static int class_rows(int M) {
-    if (M <= 8) return M;
-    int step = 16;                                   // at most an eighth more
-    while (M > 8 * step) step *= 2;
-    return (M + step - 1) / step * step;
-}
-
 static int served_shape(int M, int N, int K, bool gated) {
     if (M <= 0 || N <= 0 || K < 2 * GD_KC || K % GD_KC || (gated && N % 2)) return 0;
     const int columns = gated ? N / 2 : N;
@@ -296,7 +289,7 @@ static int served_shape(int M, int N, int K, bool gated) {
 }
 
 static int deep_shape(int M, int N, int K, bool gated) {
-    return M < (1 << 24) && served_shape(class_rows(M), N, K, gated) ? served_shape(M, N, K, gated) : 0;
+    return M < (1 << 24) && served_shape(mv_class_rows(M), N, K, gated) ? served_shape(M, N, K, gated) : 0;
 }
 
 extern "C" int mv_gemm_deep_shape(int M, int N, int K, int gated) { return deep_shape(M, N, K, gated != 0); }

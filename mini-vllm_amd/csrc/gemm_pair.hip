@@ -163,30 +163,44 @@ gemm_pair_kernel(PairArgs a) {
     }
 }
 
-// rows << 16 | weight rows of the tile that M rows against a pair [N = 2 I, K] have on a device of so many compute units; 0: the pair is left to
-// the other kernels. Times in us, ours as said above (tiles wider than tall a little behind, rounds beyond the first 6 % longer each:
-// the rows no longer come from L2); the library's with the activation behind it 8.5, the products at 1.1 to 1.5 PFLOP/s by K or the weight at
-// 4.2 TB/s, and 6 bytes a result at 5 TB/s. Below the size where the library would serve (1,536 rows, weights of 64 MB) the tiled product
-// would, level at 128 rows and behind from there. Over 68 shapes, 129 to 8,192 rows, K of 512 to 4,096, the choice is 1 % behind the best
-// on average, and 2 % behind what ran there before at worst (2,560 x 6144 x 1024); above 6,144 rows the library is ahead again.
-extern "C" int mv_gemm_pair_shape(int M, int N, int K, int units) {
-    if (M <= 128 || M > 6144 || N % 2 || K % GT_KC || N <= 0 || K <= 0 || (double)N * K >= 240e6) return 0;
+struct PairTile {
+    int tile;            // rows << 16 | weight rows
+    double time, other;  // us, estimated: with that tile, and with what serves where this product does not
+};
+
+// Times in us, ours as said above (tiles wider than tall a little behind, rounds beyond the first 6 % longer each: the rows no longer come
+// from L2); the library's with the activation behind it 8.5, the products at 1.1 to 1.5 PFLOP/s by K or the weight at 4.2 TB/s, and 6 bytes
+// a result at 5 TB/s. Below the size where the library would serve (1,536 rows, weights of 64 MB) the tiled product would, level at 128
+// rows and behind from there.
+static PairTile pair_tile(int M, int N, int K, int units) {
     const double chunks = K / GT_KC, memory = 2.0 * N * K / 5e6;
-    int best = 0;
-    double least = 0;
+    PairTile best{0, 0, 0};
     for (int bm = 64; bm <= 256; bm += 64)
         for (int bn = 64; bn <= 192; bn += 64) {
             const double tiles = (double)((M + bm - 1) / bm) * ((N / 2 + bn / 2 - 1) / (bn / 2)), rounds = ceil(tiles / units);
             const double one = 3.5 + chunks * (0.15 + 0.385 * bm * bn / 16384.0 + (bn > bm ? 0.01 * (bn - bm) / 64 : 0.0));
             const double time = 2.0 + fmax(rounds * one * (1.0 + 0.06 * (rounds - 1)), memory);
-            if (best == 0 || time < least) {
-                best = bm << 16 | bn;
-                least = time;
+            if (best.tile == 0 || time < best.time) {
+                best.tile = bm << 16 | bn;
+                best.time = time;
             }
         }
     const double rate = 1.1e9 + 0.4e9 * fmin(1.0, K / 4096.0);
-    const double other = 8.5 + fmax(2.0 * M * N * K / rate, 2.0 * N * K / 4.2e6) + 3.0 * M * N / 5e6;
-    return least < (M > 1536 || 2.0 * N * K >= 64.0 * 1024 * 1024 ? 1.05 : 1.0) * other ? best : 0;
+    best.other = 8.5 + fmax(2.0 * M * N * K / rate, 2.0 * N * K / 4.2e6) + 3.0 * M * N / 5e6;
+    return best;
+}
+
+// rows << 16 | weight rows of the tile that M rows against a pair [N = 2 I, K] have on a device of so many compute units; 0: the pair is left to
+// the other kernels. Over 68 shapes, 129 to 8,192 rows, K of 512 to 4,096, the choice is 1 % behind the best on average, and 2 % behind what
+// ran there before at worst (2,560 x 6144 x 1024); above 6,144 rows the library is ahead again. Whether the pair comes here is decided by
+// the rows that a recorded step is padded to (the library rounds gate and up in front of the activation), the tile by the rows there
+// are: every tile adds in one order.
+extern "C" int mv_gemm_pair_shape(int M, int N, int K, int units) {
+    if (M <= 128 || M > 6144 || N % 2 || K % GT_KC || N <= 0 || K <= 0 || (double)N * K >= 240e6) return 0;
+    const int padded = mv_class_rows(M);
+    const PairTile p = pair_tile(padded, N, K, units);
+    if (p.time >= (padded > 1536 || 2.0 * N * K >= 64.0 * 1024 * 1024 ? 1.05 : 1.0) * p.other) return 0;
+    return M == padded ? p.tile : pair_tile(M, N, K, units).tile;
 }
 
 // C [M, I] bf16 (pitch ldc) = pair(A Wg^T (+ bias), A Wu^T (+ bias)) for the packed weight [N = 2 I, K]: K a multiple of 64, A and W at

@@ -3,6 +3,8 @@ import ctypes
 
 import pytest
 
+from minivllm_amd.engine.executor import GRAPH_BUCKETS, TOKEN_BUCKETS
+
 
 @pytest.fixture(scope="module")
 def shape():
@@ -21,3 +23,13 @@ def test_served(shape, rows, n, k, bm, bn):
                                         (4096, 12288, 2048), (300, 51200, 5120), (300, 6145, 1024), (300, 6144, 1000)])
 def test_left_where_it_was(shape, rows, n, k):
     assert shape(rows, n, k, 256) == 0
+
+
+@pytest.mark.parametrize("n, k", [(6144, 1024), (1536, 1024), (5632, 1024), (8192, 1024), (3072, 1024), (5632, 2048), (12288, 2048), (19456, 2560),
+                                  (24576, 4096)])
+@pytest.mark.parametrize("classes", [GRAPH_BUCKETS, TOKEN_BUCKETS], ids=["decode", "prompt"])
+def test_a_class_has_one_product(shape, n, k, classes):
+    """What serves instead rounds elsewhere, so a step of a size class must take the same one recorded (padded to the class) and not."""
+    for rows in range(129, classes[-1] + 1):
+        padded = next(b for b in classes if b >= rows)
+        assert bool(shape(rows, n, k, 256)) == bool(shape(padded, n, k, 256)), (rows, padded)
