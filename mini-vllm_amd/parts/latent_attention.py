@@ -157,7 +157,7 @@ class LatentAttention(Mixer):
         self.w_o = tensors["o"]
         # ... and in the order in which the heads' own keys and values are made from the latents
         self.heads_operands = None
-        if spec.window is None and rt.dtype == torch.bfloat16 == self.w_uk.dtype == self.w_uv.dtype \
+        if spec.window is None and spec.scale > 0 and rt.dtype == torch.bfloat16 == self.w_uk.dtype == self.w_uv.dtype \
                 and rt.ops.latent_heads_serve(spec.plain_dim, spec.value_dim, spec.kv_rank, spec.rot_dim):
             self.heads_operands = latent_operands(self.w_uk), latent_operands(self.w_uv_rows)
 
