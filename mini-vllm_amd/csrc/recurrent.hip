@@ -543,6 +543,45 @@ extern "C" int mv_delta_step(const void* packed, long ld, int n, int H, int D, i
 }
 
 // ---------------------------------------------------------------------------------------
+// Finishing a head of 64 channels: sixteen lanes have four neighbouring channels each, a wave four heads, and everything a head reads is
+// asked for at once; sums run in wave_sum's order, so the bits are those of a channel a lane. What bounds it are the bytes (16 MB at 2,048
+// rows of 16 heads). With a wave a head, a channel a lane and gate and weight read behind the sum, the way to memory was waited for two or
+// three times: 2,048 rows 12.3 us (delta rule), 12.9 (gated), 14.4 (mLSTM, whose normaliser is a third), here 5.6, 6.1 and 6.5; 640 rows 5.0
+// to 5.7, here 3.3 to 3.5; 8 rows alike.
+// ---------------------------------------------------------------------------------------
+#define FINISH_DIM 64
+#define FINISH_HEADS 16            // of a workgroup
+
+// four neighbouring numbers at an address that is a multiple of their size
+__device__ __forceinline__ void load_four(const float* p, float (&v)[4]) {
+    const float4 x = *reinterpret_cast<const float4*>(p);
+    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+}
+__device__ __forceinline__ void store_four(float* p, const float (&v)[4]) { *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ void load_four(const bf16* p, float (&v)[4]) {
+    const uint2 x = *reinterpret_cast<const uint2*>(p);
+    v[0] = __uint_as_float(x.x << 16); v[1] = __uint_as_float(x.x & 0xffff0000u);
+    v[2] = __uint_as_float(x.y << 16); v[3] = __uint_as_float(x.y & 0xffff0000u);
+}
+__device__ __forceinline__ void store_four(bf16* p, const float (&v)[4]) {
+    *reinterpret_cast<uint2*>(p) = uint2{f32x2_to_bf16x2_bits(v[0], v[1]), f32x2_to_bf16x2_bits(v[2], v[3])};
+}
+
+// The sum of squares over a head, added in the order that wave_sum adds a channel a lane.
+__device__ __forceinline__ float finish_square_sum(const float (&x)[4]) {
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = fmaf(x[e], x[e], 0.f);
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += __shfl_xor(v[e], o, MV_WAVE);
+    return (v[0] + v[2]) + (v[1] + v[3]);
+}
+
+static bool finish_aligned(const void* p, long pitch, size_t item) { return (uintptr_t)p % (4 * item) == 0 && pitch % 4 == 0; }
+
+// ---------------------------------------------------------------------------------------
 // Delta rule, finish. One wave per (row, head):
 //   y[t][c] = o[t][c] / sqrt(mean over the head of o^2 + eps) * weight[c] * sigmoid(g[t][c])
 // ---------------------------------------------------------------------------------------
@@ -566,6 +605,24 @@ delta_finish_kernel(const float* __restrict__ raw, const T* __restrict__ packed,
         y[d] = from_f<T>(o[d] * rinv * weight.at((size_t)head * D + d) * sigmoid_f(to_f(g[d])));
 }
 
+// The same for heads of 64.
+template <typename T>
+__global__ void __launch_bounds__(256)
+delta_finish_head_kernel(const float* __restrict__ raw, const T* __restrict__ packed, long ld, WeightPtr weight, int H, float eps,
+                         T* __restrict__ out, long ldo, int n) {
+    const long unit = (long)blockIdx.x * FINISH_HEADS + threadIdx.x / 16;
+    if (unit >= (long)n * H) return;
+    const int t = (int)(unit / H), c = (int)(unit % H) * FINISH_DIM + threadIdx.x % 16 * 4, inner = H * FINISH_DIM;
+    float o[4], g[4], w[4], y[4];
+    load_four(raw + (size_t)t * inner + c, o);
+    load_four(packed + (size_t)t * ld + 3 * (size_t)inner + c, g);
+    weight.at_few<4>((size_t)c, w);
+    const float rinv = 1.f / sqrtf(finish_square_sum(o) / (float)FINISH_DIM + eps);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = o[e] * rinv * w[e] * sigmoid_f(g[e]);
+    store_four(out + (size_t)t * ldo + c, y);
+}
+
 extern "C" int mv_delta_finish(const float* raw, const void* packed, long ld, const void* weight, int weight_dtype, int n,
                                int H, int D, float eps, void* out, long ldo, int dtype, hipStream_t stream) {
     MV_REQUIRE(n >= 0 && H > 0 && D > 0 && eps > 0.f, "delta_finish: bad sizes n=%d H=%d D=%d", n, H, D);
@@ -574,6 +631,14 @@ extern "C" int mv_delta_finish(const float* raw, const void* packed, long ld, co
     if (n == 0) return 0;
     const long units = (long)n * H;
     WeightPtr w{weight, weight_dtype};
+    const size_t item = mv_dtype_size(dtype);
+    if (D == FINISH_DIM && finish_aligned(raw, 0, 4) && finish_aligned(packed, ld, item) && finish_aligned(weight, 0, mv_dtype_size(weight_dtype))
+        && finish_aligned(out, ldo, item)) {
+        MV_DISPATCH_T(dtype, "delta_finish",
+                      hipLaunchKernelGGL(delta_finish_head_kernel<T>, dim3((unsigned)((units + FINISH_HEADS - 1) / FINISH_HEADS)), dim3(256), 0, stream,
+                                         raw, (const T*)packed, ld, w, H, eps, (T*)out, ldo, n));
+        return mv_check_launch("delta_finish");
+    }
     MV_DISPATCH_T(dtype, "delta_finish",
                   hipLaunchKernelGGL(delta_finish_kernel<T>, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, stream, raw,
                                      (const T*)packed, ld, w, H, D, eps, (T*)out, ldo, n));
@@ -1127,6 +1192,35 @@ state_finish_kernel(const float* __restrict__ raw, const float* __restrict__ gat
     }
 }
 
+// The same for heads of 64; G: the gates' element type.
+template <typename T, typename G>
+__global__ void __launch_bounds__(256)
+state_finish_head_kernel(const float* __restrict__ raw, const float* __restrict__ gates, const G* __restrict__ packed, long ld, long g_off,
+                         WeightPtr weight, int shared_weight, int silu_gate, int normaliser, float denom_eps, int H, float eps,
+                         const int* __restrict__ token_seq, T* __restrict__ out, long ldo, int n) {
+    const long unit = (long)blockIdx.x * FINISH_HEADS + threadIdx.x / 16;
+    if (unit >= (long)n * H) return;
+    const int t = (int)(unit / H), head = (int)(unit % H), d = threadIdx.x % 16 * 4, c = head * FINISH_DIM + d;
+    const int seq = token_seq[t];
+    float o[4], z[4], w[4], x[4], y[4], scale = 1.f;
+    if (normaliser) {                                      // rows of 65 numbers
+        const float* p = raw + unit * (FINISH_DIM + 1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = p[d + e];
+        scale = 1.f / (fmaxf(fabsf(p[FINISH_DIM]), gates[unit * 4 + 2]) + denom_eps);
+    } else {
+        load_four(raw + unit * FINISH_DIM + d, o);
+    }
+    load_four(packed + (size_t)t * ld + g_off + c, z);
+    weight.at_few<4>((size_t)(shared_weight ? d : c), w);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = o[e] * scale;
+    const float rinv = scale / sqrtf(finish_square_sum(x) / (float)FINISH_DIM + eps);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = seq < 0 ? 0.f : o[e] * rinv * w[e] * (silu_gate ? silu_f(z[e]) : sigmoid_f(z[e]));
+    store_four(out + (size_t)t * ldo + c, y);
+}
+
 extern "C" int mv_state_finish(const float* raw, const float* gates, const void* packed, long ld, long g_off,
                                const void* weight, int weight_dtype, int shared_weight, int silu_gate, int normaliser,
                                float denom_eps, int n, int H, int DV, float eps, const int* token_seq, void* out, long ldo,
@@ -1138,6 +1232,17 @@ extern "C" int mv_state_finish(const float* raw, const float* gates, const void*
     if (n == 0) return 0;
     const long units = (long)n * H;
     WeightPtr w{weight, weight_dtype};
+    if (DV == FINISH_DIM && (gate_dtype == MV_F32 || gate_dtype == dtype) && (normaliser || finish_aligned(raw, 0, 4))
+        && finish_aligned(packed, ld, mv_dtype_size(gate_dtype)) && g_off % 4 == 0 && finish_aligned(weight, 0, mv_dtype_size(weight_dtype))
+        && finish_aligned(out, ldo, mv_dtype_size(dtype))) {
+        const dim3 grid((unsigned)((units + FINISH_HEADS - 1) / FINISH_HEADS));
+#define FINISH_LAUNCH(G)                                                                                                                        \
+    hipLaunchKernelGGL((state_finish_head_kernel<T, G>), grid, dim3(256), 0, stream, raw, gates, (const G*)packed, ld, g_off, w, shared_weight, \
+                       silu_gate, normaliser, denom_eps, H, eps, token_seq, (T*)out, ldo, n)
+        MV_DISPATCH_T(dtype, "state_finish", if (gate_dtype == MV_F32) FINISH_LAUNCH(float); else FINISH_LAUNCH(T));
+#undef FINISH_LAUNCH
+        return mv_check_launch("state_finish");
+    }
     MV_DISPATCH_T(dtype, "state_finish",
                   hipLaunchKernelGGL(state_finish_kernel<T>, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, stream, raw, gates,
                                      WeightPtr{packed, gate_dtype}, ld, g_off, w, shared_weight, silu_gate, normaliser, denom_eps, H, DV,

@@ -54,7 +54,7 @@ KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_token_shift": (r"\btoken_shift_kernel", None, 1),
     "mv_delta_prepare": (r"\bdelta_prepare_kernel", None, 1),
     "mv_delta_scan": (r"\bdelta_scan_kernel", None, 1),
-    "mv_delta_finish": (r"\bdelta_finish_kernel", None, 1),
+    "mv_delta_finish": (r"\bdelta_finish(_head)?_kernel", None, 1),
     "mv_delta_step": (r"\bdelta_step_kernel", None, 1),
     "mv_norm_add_norm": (r"\bnorm_add_norm(_vec)?_kernel", None, 1),
     "mv_soft_cap": (r"\bsoft_cap_kernel", None, 1),
@@ -64,7 +64,7 @@ KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_mlstm_prepare": (r"\bmlstm_gates_kernel", r"\bmlstm_prepare_kernel", 2),
     "mv_state_scan": (r"\bstate_scan_kernel", None, 1),
     "mv_delta_chunks": (r"\bdelta_chunk_kernel", r"\bdelta_chunk_walk_kernel", 2),
-    "mv_state_finish": (r"\bstate_finish_kernel", None, 1),
+    "mv_state_finish": (r"\bstate_finish(_head)?_kernel", None, 1),
     "mv_state_step": (r"\bstate_step_kernel", r"\bconv_state_kernel", 2),
     "mv_latent_prepare": (r"\blatent_prepare_kernel", None, 1),
     "mv_head_linear": (r"\bhead_linear_kernel", None, 1),
