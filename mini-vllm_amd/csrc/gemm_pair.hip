@@ -10,6 +10,14 @@
 // is one of 256 x 192. There 36.7 us with the library's product and the activation behind it, 27.7 here; 1,536 rows 34.8 (gemm_tile.hip)
 // and 22.5; 1,024 23.4 and 17.6; 512 17.4 and 13.3; 1,024 x 12288 x 2048 71 and 47; 4,096 x 6144 x 1024 69 and 55. Large products of a long K
 // stay with the library (4,096 x 24576 x 4096: 593 us with the activation, 700 here).
+//
+// The same kernel without the activation is mv_gemm_round: plain products whose tiles are one round of the compute units, which the
+// library is behind at where its own tiles leave units idle, above all for N that are no multiple of 256 (projections packed beside
+// one another). us, the library / here: 224 x 3104 x 1024 12.0 / 7.9, 1,024 17.3 / 14.1, 2,048 23.6 / 21.3; 2,048 x 5184 x 1024 34.0 / 29.4, 552
+// 16.0 / 13.3; 1,000 x 592 x 1024 8.9 / 7.1; 1,424 x 1024 x 1024 10.9 / 9.2; 2,048 x 2080 x 512 15.7 / 10.5. A tile takes what its operands take
+// through the compute unit, 192 KB of a 128 x 64 tile with K of 1,024 in 8 us; long K (2,048 x 1024 x 3072 23.4 / 23.9), N that fill the chip
+// with the library's 256 x 128 (2,048 x 4096 x 1024 22.6 / 22.9) and more than one round (4,096 x 3104 x 1024 37.9 / 42.2) stay where they were.
+#include "gemm_deep.h"
 #include "gemm_ring.h"
 
 #include <cmath>
@@ -21,18 +29,19 @@ struct PairArgs {
     const bf16* bias;
     bf16* C;
     long ldc;
-    int M, I, K;
+    int M, I, K;                       // plain: I = N
     int tiles_m, tiles, wide_stores;
     GatedPair pair;
 };
 
 // Eight waves, four down the rows and two along the columns, each with WM x WN products of 16 x 16.
-template <int WM, int WN, int STAGES>
+// GATED: half of the weight rows are gates and half are ups, else C is the product itself.
+template <int WM, int WN, int STAGES, bool GATED>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_pair_kernel(PairArgs a) {
     constexpr int BM = 64 * WM, BN = 32 * WN, WAVES = 8;
     constexpr int ROWS = BM + BN, INSTR = ROWS / 8, REPS = (INSTR + WAVES - 1) / WAVES, LEAST = INSTR / WAVES, STAGE = ROWS * 8;
-    static_assert(WN % 2 == 0, "a wave's weight tiles are half gate, half up");
+    static_assert(!GATED || WN % 2 == 0, "a wave's weight tiles are half gate, half up");
     static_assert(STAGES >= 2 && STAGES <= 4 && STAGES * STAGE * 16 <= 163840 && (STAGES - 1) * REPS <= 63, "the ring does not fit");
     __shared__ uint4 ring[STAGES * STAGE];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / MV_WAVE), lane = tid % MV_WAVE, i = lane % 16, g = lane / 16;
@@ -41,7 +50,7 @@ gemm_pair_kernel(PairArgs a) {
     const int run = (a.tiles + GT_XCDS - 1) / GT_XCDS, id = blockIdx.x % GT_XCDS * run + blockIdx.x / GT_XCDS;
     if ((int)blockIdx.x / GT_XCDS >= run || id >= a.tiles) return;
     const int tm = id % a.tiles_m, tn = id / a.tiles_m;
-    const int m0 = tm * BM, n0 = tn * (BN / 2), n = a.K / GT_KC;
+    const int m0 = tm * BM, n0 = tn * (GATED ? BN / 2 : BN), n = a.K / GT_KC;
 
     // this lane's share of the loads, and the operands: as in gemm_tile.hip
     const int lrow = lane / 8, piece = (lane % 8) ^ lrow;
@@ -53,7 +62,7 @@ gemm_pair_kernel(PairArgs a) {
             src[rep] = reinterpret_cast<const char*>(a.A + (size_t)min(m0 + row, a.M - 1) * a.lda + 8 * piece);
         } else {
             const int r = row - BM;
-            const int w = r < BN / 2 ? min(n0 + r, a.I - 1) : min(a.I + n0 + r - BN / 2, 2 * a.I - 1);
+            const int w = !GATED || r < BN / 2 ? min(n0 + r, a.I - 1) : min(a.I + n0 + r - BN / 2, 2 * a.I - 1);
             src[rep] = reinterpret_cast<const char*>(a.W + (size_t)w * a.K + 8 * piece);
         }
     }
@@ -68,7 +77,7 @@ gemm_pair_kernel(PairArgs a) {
     for (int t = 0; t < WM; ++t) a_off[t] = (16 * (WM * wm + t) + i) * 8;
 #pragma unroll
     for (int t = 0; t < WN; ++t) {
-        const int group = t < WN / 2 ? (WN / 2) * wn + t : (WN / 2) * (2 + wn) + (t - WN / 2);
+        const int group = !GATED ? WN * wn + t : t < WN / 2 ? (WN / 2) * wn + t : (WN / 2) * (2 + wn) + (t - WN / 2);
         w_off[t] = (BM + 16 * group + i) * 8;
     }
     const int sw0 = g ^ (i & 7), sw1 = (4 + g) ^ (i & 7);
@@ -131,7 +140,7 @@ gemm_pair_kernel(PairArgs a) {
     }
 
     // lane l holds C[row 16 u + l % 16][columns 4 (l / 16) .. + 3 of tile t]
-    constexpr int TOUT = WN / 2;
+    constexpr int TOUT = GATED ? WN / 2 : WN;
 #pragma unroll
     for (int t = 0; t < TOUT; ++t) {
         const int col = n0 + 16 * (TOUT * wn + t) + 4 * g;
@@ -141,7 +150,7 @@ gemm_pair_kernel(PairArgs a) {
             for (int e = 0; e < 4; ++e)
                 if (col + e < a.I) {
                     bv[e] = to_f(a.bias[col + e]);
-                    bu[e] = to_f(a.bias[a.I + col + e]);
+                    if constexpr (GATED) bu[e] = to_f(a.bias[a.I + col + e]);
                 }
         }
 #pragma unroll
@@ -150,7 +159,10 @@ gemm_pair_kernel(PairArgs a) {
             if (row >= a.M || col >= a.I) continue;
             float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = a.pair.of_short(acc[t][u][e] + bv[e], acc[t + TOUT][u][e] + bu[e]);
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (GATED) v[e] = a.pair.of_short(acc[t][u][e] + bv[e], acc[t + TOUT][u][e] + bu[e]);
+                else v[e] = acc[t][u][e] + bv[e];
+            }
             bf16* to = a.C + (size_t)row * a.ldc + col;
             if (a.wide_stores && col + 3 < a.I) {
                 *reinterpret_cast<uint2*>(to) = uint2{f32x2_to_bf16x2_bits(v[0], v[1]), f32x2_to_bf16x2_bits(v[2], v[3])};
@@ -218,7 +230,7 @@ extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* 
     const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N / 2, K, tiles_m, (int)tiles,
                      ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{limit, slope}};
     const dim3 grid((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
-#define GP_LAUNCH(WM, WN, S) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, S>), grid, dim3(512), 0, stream, a)
+#define GP_LAUNCH(WM, WN, S) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, S, true>), grid, dim3(512), 0, stream, a)
     if (bn == 192) {
         if (bm == 256) GP_LAUNCH(4, 6, 2);
         else if (bm == 192) GP_LAUNCH(3, 6, 3);
@@ -237,4 +249,77 @@ extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* 
     }
 #undef GP_LAUNCH
     return mv_check_launch("gemm_pair");
+}
+
+// Columns of the plain product's tiles, and its time in us with tiles of bm x bn in one round, 0.05 apart from the measured ones (standard
+// deviation; 671 of 130 to 4,096 rows, K of 256 to 4,096): operands into LDS (bm + bn), out of it and through the matrix unit (bm bn), both slower
+// the more units are at it.
+static const int kRoundColumns[] = {64, 96, 128, 192};
+static double round_time(int bm, int bn, int K, double tiles, int units) {
+    const double chunks = K / GT_KC, sides = (bm + bn) / 256.0;
+    return 0.46 + 4.41 * sides + chunks * (0.204 - 0.080 * sides + 0.311 * bm * bn / 16384.0 + 0.165 * sides * tiles / units);
+}
+static PairTile round_tile(int M, int N, int K, int units) {
+    PairTile best{0, 0, 0};
+    for (int bm = 64; bm <= 256; bm += 64)
+        for (int bn : kRoundColumns) {
+            const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn), time = round_time(bm, bn, K, tiles, units);
+            if (tiles <= units && (best.tile == 0 || time < best.time)) {
+                best.tile = bm << 16 | bn;
+                best.time = time;
+            }
+        }
+    best.other = N % 256 ? 10.2 + 2.0 * M * N * K / 1.15e9 : 7.5 + 2.0 * M * N * K / 1.3e9;
+    return best;
+}
+
+// rows << 16 | columns of the tile that M rows against a plain weight [N, K] have, 0: the library's (or gemm_deep.hip's). The library's
+// times are taken as its better ones, 1.15 PFLOP/s behind 10.2 us, 1.3 behind 7.5 where N is a multiple of its tiles: over 133 shapes, 160 to
+// 4,096 rows, of the 95 that come here one is 4 % behind it and the others up to 43 % ahead. Decided by the rows of the step's class, as above.
+extern "C" int mv_gemm_round_shape(int M, int N, int K, int units) {
+    if (M <= 128 || M > 8192 || N <= 0 || K <= 0 || K % GT_KC || (double)N * K >= 240e6 || mv_gemm_deep_shape(M, N, K, 0)) return 0;
+    const int padded = mv_class_rows(M);
+    const PairTile p = round_tile(padded, N, K, units);
+    if (p.tile == 0 || p.time >= p.other) return 0;
+    return M == padded ? p.tile : round_tile(M, N, K, units).tile;
+}
+
+// C [M, N] bf16 (pitch ldc) = A W^T (+ bias), operands as above. `tile`: 64 to 256 rows by 64, 96, 128, 192 columns.
+extern "C" int mv_gemm_round(const void* A, long lda, const void* W, const void* bias, void* C, long ldc, int M, int N, int K, int tile,
+                             hipStream_t stream) {
+    MV_REQUIRE(M > 0 && N > 0 && K > 0 && K % GT_KC == 0, "gemm_round: bad sizes M=%d N=%d K=%d", M, N, K);
+    MV_REQUIRE(A && W && C && lda >= K && lda % 8 == 0 && ((uintptr_t)A | (uintptr_t)W) % 16 == 0 && ldc >= N,
+               "gemm_round: operands not aligned or pitches too small");
+    const int bm = tile >> 16, bn = tile & 0xffff;
+    MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 96 || bn == 128 || bn == 192), "gemm_round: no tile of %d x %d", bm, bn);
+    const int tiles_m = (M + bm - 1) / bm;
+    const long tiles = (long)tiles_m * ((N + bn - 1) / bn);
+    MV_REQUIRE(tiles < (1L << 30), "gemm_round: too many tiles");
+    const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N, K, tiles_m, (int)tiles,
+                     ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{0.f, 1.f}};
+    const dim3 grid((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
+#define GR_LAUNCH(WM, WN, S) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, S, false>), grid, dim3(512), 0, stream, a)
+    if (bn == 192) {
+        if (bm == 256) GR_LAUNCH(4, 6, 2);
+        else if (bm == 192) GR_LAUNCH(3, 6, 3);
+        else if (bm == 128) GR_LAUNCH(2, 6, 4);
+        else GR_LAUNCH(1, 6, 4);
+    } else if (bn == 128) {
+        if (bm == 256) GR_LAUNCH(4, 4, 3);
+        else if (bm == 192) GR_LAUNCH(3, 4, 4);
+        else if (bm == 128) GR_LAUNCH(2, 4, 4);
+        else GR_LAUNCH(1, 4, 4);
+    } else if (bn == 96) {
+        if (bm == 256) GR_LAUNCH(4, 3, 3);
+        else if (bm == 192) GR_LAUNCH(3, 3, 4);
+        else if (bm == 128) GR_LAUNCH(2, 3, 4);
+        else GR_LAUNCH(1, 3, 4);
+    } else {
+        if (bm == 256) GR_LAUNCH(4, 2, 4);
+        else if (bm == 192) GR_LAUNCH(3, 2, 4);
+        else if (bm == 128) GR_LAUNCH(2, 2, 4);
+        else GR_LAUNCH(1, 2, 4);
+    }
+#undef GR_LAUNCH
+    return mv_check_launch("gemm_round");
 }

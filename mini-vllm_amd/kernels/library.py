@@ -240,6 +240,9 @@ _OPTIONAL_SIGNATURES = {
     "mv_gemm_pair_shape": (c_int, [c_int, c_int, c_int, c_int]),
     # A, lda, W, bias, C, ldc, M, N, K, limit, slope, tile, stream
     "mv_gemm_pair": (c_int, [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_float, c_float, c_int, c_void_p]),
+    "mv_gemm_round_shape": (c_int, [c_int, c_int, c_int, c_int]),
+    # A, lda, W, bias, C, ldc, M, N, K, tile, stream
+    "mv_gemm_round": (c_int, [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_int, c_void_p]),
     "mv_moe_pairs_shape": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "mv_moe_pairs_ints": (c_long, [c_int, c_int, c_int, c_int]),
     # x, ldx, n, hidden, w_gate_up, w_down, n_real, identity, F, FS, ids, weights, top, dense, ld_dense, ints, act, out, y, ldy,

@@ -2556,13 +2556,15 @@ class Ops:
 
     def _library_product(self, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor) -> bool:
         """out = a @ w^T (+ bias) by the library (hipBLASLt), bf16 in, bf16 or float32 out; bf16 outputs of shapes that
-        ``gemm_deep.hip`` is faster at are made there, inside the same entry point. The library is
+        ``gemm_pair.hip`` or ``gemm_deep.hip`` is faster at are made there, the latter inside the same entry point. The library is
         called directly where the kernel library was built with it (a call costs a third of the host
         time of the tensor library's dispatcher, which matters for prompt steps of small models);
         else, for bf16 output, through ``torch.mm``. False, with nothing done, when the library has
         no algorithm for the shape."""
         M, K = a.shape
         N = w.shape[0]
+        if self._gemm_round(a, w, bias, out):
+            return True
         rest = self._rows_behind_whole_rounds(M, N)
         if rest:
             return self._library_product(a[:M - rest], w, bias, out[:M - rest]) and \
@@ -2586,6 +2588,21 @@ class Ops:
             torch.mm(a, wt, out=out)
         else:
             torch.addmm(bias, a, wt, out=out)
+        return True
+
+    def _gemm_round(self, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor) -> bool:
+        """A plain product whose tiles are one round of the compute units (gemm_pair.hip, whose ``mv_gemm_round_shape`` says for which
+        sizes); False, with nothing done, where it is left to the library."""
+        if not self.use_tiled_gemm or not self.lib.has("mv_gemm_round"):
+            return False
+        (M, K), N = a.shape, w.shape[0]
+        tile = self.lib.dll.mv_gemm_round_shape(M, N, K, self.compute_units)
+        if (not tile or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or not w.is_contiguous()
+                or a.stride(1) != 1 or out.stride(1) != 1 or a.stride(0) % 8 or a.data_ptr() % 16 or w.data_ptr() % 16):
+            return False
+        self._note("mv_gemm_round", self._size(a, w, out), 2 * M * N * K)
+        self.lib.call("mv_gemm_round", a.data_ptr(), a.stride(0), w.data_ptr(), _ptr(bias), out.data_ptr(), out.stride(0), M, N, K, tile,
+                      self._stream())
         return True
 
     def _library_allowed(self, M: int, N: int, K: int, with_bias: bool, out_dtype: torch.dtype = torch.bfloat16) -> bool:

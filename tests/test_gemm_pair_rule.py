@@ -7,9 +7,14 @@ from minivllm_amd.engine.executor import GRAPH_BUCKETS, TOKEN_BUCKETS
 
 
 @pytest.fixture(scope="module")
-def shape():
+def lib():
     from minivllm_amd.csrc import build
-    return ctypes.CDLL(build.find_library("bf16") or build.build("bf16")).mv_gemm_pair_shape
+    return ctypes.CDLL(build.find_library("bf16") or build.build("bf16"))
+
+
+@pytest.fixture(scope="module")
+def shape(lib):
+    return lib.mv_gemm_pair_shape
 
 
 @pytest.mark.parametrize("rows, n, k, bm, bn", [(320, 6144, 1024, 64, 128), (640, 6144, 1024, 128, 128), (1024, 6144, 1024, 128, 192),
@@ -30,6 +35,28 @@ def test_left_where_it_was(shape, rows, n, k):
 @pytest.mark.parametrize("classes", [GRAPH_BUCKETS, TOKEN_BUCKETS], ids=["decode", "prompt"])
 def test_a_class_has_one_product(shape, n, k, classes):
     """What serves instead rounds elsewhere, so a step of a size class must take the same one recorded (padded to the class) and not."""
+    for rows in range(129, classes[-1] + 1):
+        padded = next(b for b in classes if b >= rows)
+        assert bool(shape(rows, n, k, 256)) == bool(shape(padded, n, k, 256)), (rows, padded)
+
+
+@pytest.mark.parametrize("rows, n, k, bm, bn", [(224, 3104, 1024, 64, 64), (576, 1024, 1024, 64, 64), (1024, 3104, 1024, 128, 128),
+                                                (2048, 5184, 1024, 256, 192), (2048, 4112, 1024, 192, 192), (1024, 3072, 256, 128, 96)])
+def test_plain_products_served(lib, rows, n, k, bm, bn):
+    assert divmod(lib.mv_gemm_round_shape(rows, n, k, 256), 1 << 16) == (bm, bn)
+
+
+# one request's and few rows, long K, full tiles of the library's, more than a round; what gemm_deep.hip takes
+@pytest.mark.parametrize("rows, n, k", [(128, 5184, 1024), (2048, 1024, 3072), (2048, 1024, 2048), (2048, 4096, 1024), (4096, 3104, 1024), (4415, 24576, 4096),
+                                        (512, 1024, 2048), (160, 1040, 1024), (300, 5184, 1000), (1024, 151936, 1024)])
+def test_plain_products_left_where_they_were(lib, rows, n, k):
+    assert lib.mv_gemm_round_shape(rows, n, k, 256) == 0
+
+
+@pytest.mark.parametrize("n, k", [(5184, 1024), (3104, 1024), (1024, 1024), (592, 1024), (2080, 512), (6176, 2048), (3072, 256), (1024, 2048)])
+@pytest.mark.parametrize("classes", [GRAPH_BUCKETS, TOKEN_BUCKETS], ids=["decode", "prompt"])
+def test_a_class_has_one_plain_product(lib, n, k, classes):
+    shape = lib.mv_gemm_round_shape
     for rows in range(129, classes[-1] + 1):
         padded = next(b for b in classes if b >= rows)
         assert bool(shape(rows, n, k, 256)) == bool(shape(padded, n, k, 256)), (rows, padded)

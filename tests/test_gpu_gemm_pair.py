@@ -53,3 +53,40 @@ def test_prompts_take_it(M, I, K):
         assert ran == ["mv_gemm_pair"]
         want = pair(x, w, None, 0.0, 1.0)
         assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("bm", [64, 128, 192, 256])
+@pytest.mark.parametrize("bn", [64, 96, 128, 192])
+@pytest.mark.parametrize("M, N, K, bias", [(1, 8, 64, False), (255, 101, 128, True), (257, 193, 192, True), (300, 384, 640, False), (577, 333, 320, True)])
+def test_plain_tiles(bm, bn, M, N, K, bias):
+    """As above without the activation: the result is rounded by half a step of its eight bits, 2^-8 of it at most; sums of up to 640
+    terms of a tenth in float32 are off by 1e-5 at most."""
+    from minivllm_amd.kernels.ops import get_ops
+    ops = get_ops(torch.bfloat16)
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x, w = rand(M, K + 8).bfloat16()[:, :K], (rand(N, K) / K ** 0.5).bfloat16()
+    b = rand(N).bfloat16() if bias else None
+    out = torch.full((M + 1, N + 3), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.lib.call("mv_gemm_round", x.data_ptr(), x.stride(0), w.data_ptr(), 0 if b is None else b.data_ptr(), out.data_ptr(), out.stride(0), M, N, K,
+                 bm << 16 | bn, torch.cuda.current_stream().cuda_stream)
+    want = x.double() @ w.double().T + (0 if b is None else b.double())
+    assert bool(((out[:M, :N].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all())
+    assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("M, N, K", [(600, 5184, 1024), (1000, 592, 1024), (2048, 3104, 1024), (700, 1024, 1024)])
+def test_plain_products_of_prompts_take_it(M, N, K):
+    """Through the engine's entry point, rows with and without a pitch that loads of eight need."""
+    from minivllm_amd.kernels.ops import get_ops
+    ops = get_ops(torch.bfloat16)
+    w, b = (torch.randn(N, K, device=DEV) / K ** 0.5).bfloat16(), torch.randn(N, device=DEV).bfloat16()
+    for pitch in (K, K + 8, K + 4):
+        x = torch.randn(M, pitch, device=DEV).bfloat16()[:, :K]
+        out = torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
+        ops.ledger = []
+        ops.gemm(x, w, out, bias=b)
+        ran, ops.ledger = [e[0] for e in ops.ledger], None
+        assert (ran == ["mv_gemm_round"]) == (pitch % 8 == 0)
+        want = x.double() @ w.double().T + b.double()
+        assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
