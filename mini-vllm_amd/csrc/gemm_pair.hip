@@ -182,7 +182,7 @@ struct PairTile {
 
 // Times in us, ours as said above (tiles wider than tall a little behind, rounds beyond the first 6 % longer each: the rows no longer come
 // from L2); the library's with the activation behind it 8.5, the products at 1.1 to 1.5 PFLOP/s by K or the weight at 4.2 TB/s, and 6 bytes
-// a result at 5 TB/s. Below the size where the library would serve (1,536 rows, weights of 64 MB) the tiled product would, level at 128
+// a result at 5 TB/s. Below the size where the library would serve (1,536 rows) the tiled product would, level at 128
 // rows and behind from there.
 static PairTile pair_tile(int M, int N, int K, int units) {
     const double chunks = K / GT_KC, memory = 2.0 * N * K / 5e6;
@@ -204,14 +204,15 @@ static PairTile pair_tile(int M, int N, int K, int units) {
 
 // rows << 16 | weight rows of the tile that M rows against a pair [N = 2 I, K] have on a device of so many compute units; 0: the pair is left to
 // the other kernels. Over 68 shapes, 129 to 8,192 rows, K of 512 to 4,096, the choice is 1 % behind the best on average, and 2 % behind what
-// ran there before at worst (2,560 x 6144 x 1024); above 6,144 rows the library is ahead again. Whether the pair comes here is decided by
+// ran there before at worst (2,560 x 6144 x 1024); above 6,144 rows the library is ahead again. Weights of 64 MB and
+// more are left to it at every number of rows: there a pair is two calls, the product and its activation. Whether the pair comes here is decided by
 // the rows that a recorded step is padded to (the library rounds gate and up in front of the activation), the tile by the rows there
 // are: every tile adds in one order.
 extern "C" int mv_gemm_pair_shape(int M, int N, int K, int units) {
-    if (M <= 128 || M > 6144 || N % 2 || K % GT_KC || N <= 0 || K <= 0 || (double)N * K >= 240e6) return 0;
+    if (M <= 128 || M > 6144 || N % 2 || K % GT_KC || N <= 0 || K <= 0 || 2.0 * N * K >= 64.0 * 1024 * 1024) return 0;
     const int padded = mv_class_rows(M);
     const PairTile p = pair_tile(padded, N, K, units);
-    if (p.time >= (padded > 1536 || 2.0 * N * K >= 64.0 * 1024 * 1024 ? 1.05 : 1.0) * p.other) return 0;
+    if (p.time >= (padded > 1536 ? 1.05 : 1.0) * p.other) return 0;
     return M == padded ? p.tile : pair_tile(M, N, K, units).tile;
 }
 

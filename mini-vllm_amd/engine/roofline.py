@@ -43,7 +43,7 @@ KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_scale_rows": (r"\bscale_rows_kernel", None, 1),
     "mv_gemm_ref": (r"\bgemm_nt(_wave|_ring)?_kernel", None, 1),
     "mv_gemm_mid": (r"\bgemm_mid_kernel", r"\bgemm_mid_reduce_kernel", 2),
-    "mv_gemm_tile": (r"\bgemm_(tile|deep)_kernel", r"\bgemm_mid_reduce_kernel", 2),
+    "mv_gemm_tile": (r"\bgemm_(tile|deep|pair)_kernel", r"\bgemm_mid_reduce_kernel", 2),
     "mv_gemm_lt": (_LIBRARY, _LIBRARY, 3),
     "mv_attention_ref": (r"\battention_ref_kernel", None, 1),
     "mv_attention_exact": (r"\battention_exact_kernel", None, 1),

@@ -2554,7 +2554,7 @@ class Ops:
         rest = M % step
         return rest if step in (2048, 4096) and M > step and rest <= 1024 else 0
 
-    def _library_product(self, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor) -> bool:
+    def _library_product(self, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, part: bool = False) -> bool:
         """out = a @ w^T (+ bias) by the library (hipBLASLt), bf16 in, bf16 or float32 out; bf16 outputs of shapes that
         ``gemm_pair.hip`` or ``gemm_deep.hip`` is faster at are made there, the latter inside the same entry point. The library is
         called directly where the kernel library was built with it (a call costs a third of the host
@@ -2563,12 +2563,12 @@ class Ops:
         no algorithm for the shape."""
         M, K = a.shape
         N = w.shape[0]
-        if self._gemm_round(a, w, bias, out):
+        if not part and self._gemm_round(a, w, bias, out):      # (``part`` of a product's rows stays with the rest of them)
             return True
         rest = self._rows_behind_whole_rounds(M, N)
         if rest:
-            return self._library_product(a[:M - rest], w, bias, out[:M - rest]) and \
-                self._library_product(a[M - rest:], w, bias, out[M - rest:])
+            return self._library_product(a[:M - rest], w, bias, out[:M - rest], True) and \
+                self._library_product(a[M - rest:], w, bias, out[M - rest:], True)
         if self.lib.has("mv_gemm_lt") and a.stride(1) == 1 and out.stride(1) == 1 and a.data_ptr() % 16 == 0 \
                 and out.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
             if self._lt_work is None:
@@ -2741,8 +2741,8 @@ class Ops:
         return True
 
     def _gemm_pair(self, a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor], limit: float, slope: float) -> bool:
-        """The gated pair of a prompt's rows in one pass (gemm_pair.hip, whose ``mv_gemm_pair_shape`` says for which sizes); False, with
-        nothing done, where it is left to the other kernels."""
+        """The gated pair of a prompt's rows in one pass (gemm_pair.hip, whose ``mv_gemm_pair_shape`` says for which sizes; those that the
+        tiled product would have reach it inside that entry point); False, with nothing done, where it is left to the other kernels."""
         if not self.use_tiled_gemm or not self.lib.has("mv_gemm_pair"):
             return False
         (M, K), N = a.shape, w.shape[0]
@@ -2904,10 +2904,10 @@ class Ops:
             return False
         M, K = a.shape
         two_i = w_gate_up.shape[0]
-        if self._gemm_pair(a, w_gate_up, out, bias, limit, slope):
-            return True
         if self.wants_tile(M, two_i, K, gated=True) and self.gemm_tile(
                 a, w_gate_up, out, bias, gated=True, limit=limit, slope=slope):
+            return True
+        if self._gemm_pair(a, w_gate_up, out, bias, limit, slope):
             return True
         if self.prefers_library(M, two_i, K, gated=True) and self._library_allowed(M, two_i, K, False):
             return False

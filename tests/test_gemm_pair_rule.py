@@ -19,12 +19,12 @@ def shape(lib):
 
 @pytest.mark.parametrize("rows, n, k, bm, bn", [(320, 6144, 1024, 64, 128), (640, 6144, 1024, 128, 128), (1024, 6144, 1024, 128, 192),
                                                 (1280, 6144, 1024, 256, 128), (1536, 6144, 1024, 192, 192), (2048, 6144, 1024, 256, 192),
-                                                (1024, 12288, 2048, 256, 192), (200, 24576, 4096, 128, 192), (512, 1536, 512, 64, 64)])
+                                                (1024, 12288, 2048, 256, 192), (512, 1536, 512, 64, 64)])
 def test_served(shape, rows, n, k, bm, bn):
     assert divmod(shape(rows, n, k, 256), 1 << 16) == (bm, bn)
 
 
-@pytest.mark.parametrize("rows, n, k", [(96, 6144, 1024), (128, 6144, 1024), (800, 24576, 4096), (4415, 24576, 4096), (8192, 6144, 1024),
+@pytest.mark.parametrize("rows, n, k", [(96, 6144, 1024), (128, 6144, 1024), (200, 24576, 4096), (800, 24576, 4096), (4415, 24576, 4096), (8192, 6144, 1024),
                                         (4096, 12288, 2048), (300, 51200, 5120), (300, 6145, 1024), (300, 6144, 1000)])
 def test_left_where_it_was(shape, rows, n, k):
     assert shape(rows, n, k, 256) == 0
