@@ -13,7 +13,9 @@ DEV = "cuda:0"
     (20, 64, 448, 0, 96, 2, (32, 256, 64)), (1500, 64, 64, 64, 24, 2, (64, 128, 128)), (1100, 320, 64, 64, 96, 2, (64, 128, 256)),
     (1100, 64, 192, 64, 96, 2, (64, 256, 128)), (300, 64, 64, 64, 150, 2, (96, 128, 128)), (300, 576, 64, 64, 150, 2, (96, 128, 256)),
     (300, 64, 192, 64, 150, 2, (96, 256, 128)), (1100, 320, 448, 64, 24, 2, (128, 128, 128)), (1500, 832, 192, 64, 48, 2, (128, 128, 256)),
-    (1500, 320, 448, 64, 48, 2, (128, 256, 128)), (1500, 576, 448, 64, 24, 2, (160, 128, 128)), (1000, 1024, 768, 768, 32, 4, (160, 256, 256))])
+    (1500, 320, 448, 64, 48, 2, (128, 256, 128)), (1500, 576, 448, 64, 24, 2, (160, 128, 128)), (1000, 1024, 768, 768, 32, 4, (160, 256, 256)),
+    # as many pairs as the threads that sort them keep, and more
+    (2048, 64, 64, 64, 24, 4, (96, 128, 128)), (2100, 64, 64, 64, 24, 4, (96, 128, 128))])
 def test_tiles(n, hid, F, FS, E, top, tiles, limit):
     """Full and partial tiles, an expert that most tokens chose, empty ones, tokens without an expert. bfloat16 operands summed in float,
     activations rounded once to bfloat16 (2^-9 of each of F terms of random sign): 1e-2 of the largest output, and each row's share of it."""
