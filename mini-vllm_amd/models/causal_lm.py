@@ -180,7 +180,7 @@ class CausalLM:
         """What the mixers choose for a step whose sequences bring ``lens`` tokens from positions ``starts`` on
         (``Mixer.step_path``)."""
         if self._choosers is None:
-            alike = {(type(m), getattr(m, "spec", m)): m for m in self.mixers if m is not None and m.step_path([1], [0]) is not None}
+            alike = {m.chooses_by(): m for m in self.mixers if m is not None and m.step_path([1], [0]) is not None}
             self._choosers = list(alike.values())
         return tuple(m.step_path(lens, starts) for m in self._choosers)
 

@@ -522,6 +522,11 @@ class Mixer(Part):
         (``starts``), or None. Steps with another choice get recordings of their own."""
         return None
 
+    def chooses_by(self) -> Tuple:
+        """All that ``step_path`` depends on besides its arguments and the engine: mixers for which this is equal choose alike, and
+        one of them is asked for all. A mixer whose choice hangs on more than its spec adds that here."""
+        return type(self), getattr(self, "spec", self)
+
     def reserve(self, tokens: int, seqs: int) -> None:
         """Sizes the scratch (``rt.workspace``) whose need depends on how a step is cut, for any cut of up to ``tokens``
         tokens into up to ``seqs`` sequences. (What depends on the number of tokens alone, a run of that many sizes.)"""

@@ -169,6 +169,9 @@ class LatentAttention(Mixer):
             return None
         return self.rt.ops.latent_shares(self.spec.num_heads, -1 if self.spec.window is None else self.spec.window, lens, starts)
 
+    def chooses_by(self):
+        return super().chooses_by() + (self.heads_operands is not None,)       # (how this layer's maps are stored)
+
     def reserve(self, tokens: int, seqs: int) -> None:
         most = self.rt.ops.latent_heads_most(self.spec.num_heads, tokens, seqs, self.rt.max_positions) if self.heads_operands is not None else 0
         if most:

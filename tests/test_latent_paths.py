@@ -59,3 +59,26 @@ def test_room_for_own_keys_is_bounded():
     for lens, starts in (([512], [0]), ([128] * 4, [896] * 4), ([2] * 4, [1022] * 4), ([2], [0]), ([100, 100, 100], [924, 100, 0])):
         assert Ops.latent_heads(ops, 16, lens, starts) <= most
     assert Ops.latent_heads(ops, 64, [64], [40000]) == 0 and Ops.latent_heads_most(ops, 64, 8192, 256, 40960) == 512
+
+
+def test_layers_of_one_spec_that_store_their_maps_differently_choose_for_themselves():
+    """A layer whose maps are stored in 32 bits stays in the latent's space, its neighbour of the same spec does not: a recording's key
+    holds both choices, whichever layer comes last."""
+    import torch
+    from minivllm_amd.models.causal_lm import CausalLM
+    from minivllm_amd.parts.latent_attention import LatentAttention, LatentAttentionSpec
+    spec = LatentAttentionSpec(hidden_size=256, num_heads=2, plain_dim=128, value_dim=128, kv_rank=128)
+    ops = SimpleNamespace(compute_units=256, latent_heads_serve=lambda *sizes: True, latent_shares_serve=lambda *sizes: True)
+    ops.latent_heads, ops.latent_shares = lambda *a: Ops.latent_heads(ops, *a), lambda *a: Ops.latent_shares(ops, *a)
+    rt = SimpleNamespace(dtype=torch.bfloat16, ops=ops)
+
+    def layer(*wide):
+        return LatentAttention(spec, {name: torch.zeros(decl.shape, dtype=torch.float32 if name in wide else torch.bfloat16)
+                                      for name, decl in LatentAttention.tensors(spec).items()}, rt)
+    both = [layer(), layer("uk")]
+    lens, starts = [100], [0]
+    own, latent = (m.step_path(lens, starts) for m in both)
+    assert own != latent
+    for mixers in (both, both[::-1], both + [layer(), layer("uv"), None]):
+        assert set(CausalLM.step_paths(SimpleNamespace(_choosers=None, mixers=mixers), lens, starts)) == {own, latent}
+    assert len(CausalLM.step_paths(SimpleNamespace(_choosers=None, mixers=[layer(), layer(), layer()]), lens, starts)) == 1
