@@ -733,6 +733,7 @@ class Executor:
             largest = next(b for b in GRAPH_BUCKETS if b >= min(self.config.max_num_batched_seqs, GRAPH_BUCKETS[-1]))
             pad_ctx = self._padding_step(largest)
             pad_ctx.attention_plan.max_context_len = self.config.max_model_len
+            self.model.reserve(largest, largest, portions=False)
             self.model.forward(pad_ctx)
             most = min(self.config.prompt_graph_max_tokens, self.config.max_num_batched_tokens, TOKEN_BUCKETS[-1])
             if most > largest:

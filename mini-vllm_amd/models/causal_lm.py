@@ -184,10 +184,11 @@ class CausalLM:
             self._choosers = list(alike.values())
         return tuple(m.step_path(lens, starts) for m in self._choosers)
 
-    def reserve(self, tokens: int, seqs: int) -> None:
-        """Sizes the scratch of mixers and feed-forwards for any cut of up to ``tokens`` tokens into up to ``seqs`` sequences."""
+    def reserve(self, tokens: int, seqs: int, portions: bool = True) -> None:
+        """Sizes the scratch of mixers and feed-forwards for any cut of up to ``tokens`` tokens into up to ``seqs`` sequences
+        (without ``portions``: of one token each)."""
         for mixer in self.mixers:
-            if mixer is not None:
+            if mixer is not None and portions:
                 mixer.reserve(tokens, seqs)
         for ffn in self.ffns:
             if ffn is not None:

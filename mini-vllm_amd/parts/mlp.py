@@ -44,12 +44,18 @@ class SwiGLU(FeedForward):
     def first_product(self):
         return self.w_gate_up.shape[0], self.w_gate_up.shape[1], True
 
+    def reserve(self, tokens: int) -> None:
+        self._gate_up(tokens)            # (which numbers of rows go in one pass does not grow with them)
+
+    def _gate_up(self, n: int) -> torch.Tensor:
+        return self.rt.workspace.get("ffn.gate_up", (n, 2 * self.spec.intermediate_size), self.rt.dtype)
+
     def forward(self, x: torch.Tensor, ctx, fold=None) -> torch.Tensor:
         spec, rt, ops = self.spec, self.rt, self.rt.ops
         n = x.shape[0]
         act = rt.workspace.get("ffn.act", (n, spec.intermediate_size), rt.dtype)
-        if not ops.gemm_swiglu(x, self.w_gate_up, act):      # one pass over the weight for few rows
-            gu = rt.workspace.get("ffn.gate_up", (n, 2 * spec.intermediate_size), rt.dtype)
+        if not ops.gemm_swiglu(x, self.w_gate_up, act):      # one pass over the weight where a kernel takes the rows
+            gu = self._gate_up(n)
             if not isinstance(x, torch.Tensor):
                 x = x.materialize()
             ops.gemm(x, self.w_gate_up, gu)
@@ -184,12 +190,18 @@ class ClampedGLU(FeedForward):
     def first_product(self):
         return self.w_gate_up.shape[0], self.w_gate_up.shape[1], True
 
+    def reserve(self, tokens: int) -> None:
+        self._gate_up(tokens)            # (which numbers of rows go in one pass does not grow with them)
+
+    def _gate_up(self, n: int) -> torch.Tensor:
+        return self.rt.workspace.get("ffn.gate_up", (n, 2 * self.spec.intermediate_size), self.rt.dtype)
+
     def forward(self, x: torch.Tensor, ctx, fold=None) -> torch.Tensor:
         spec, rt, ops = self.spec, self.rt, self.rt.ops
         n = x.shape[0]
         act = rt.workspace.get("ffn.act", (n, spec.intermediate_size), rt.dtype)
         if not ops.gemm_swiglu(x, self.w_gate_up, act, self.b_gate_up, limit=spec.limit, slope=spec.slope):
-            gu = rt.workspace.get("ffn.gate_up", (n, 2 * spec.intermediate_size), rt.dtype)
+            gu = self._gate_up(n)
             if not isinstance(x, torch.Tensor):
                 x = x.materialize()
             ops.gemm(x, self.w_gate_up, gu, self.b_gate_up)

@@ -192,7 +192,12 @@ class RoutedExperts(FeedForward):
         for n in (tokens, min(tokens, (self.LARGE_STEP - 1) // max(1, self.spec.num_experts))):
             if n > 0 and self.spec.num_experts and not self.wants_pairs(n):
                 self._all_experts_scratch(n)
-                return
+                break
+        if self.spec.shared_size and not self.shared_packed:
+            self._shared_gate_up(tokens)            # (which numbers of rows go in one pass does not grow with them)
+
+    def _shared_gate_up(self, n: int) -> torch.Tensor:
+        return self.rt.workspace.get("moe.shared_gate_up", (n, 2 * self.spec.shared_size), self.rt.dtype)
 
     def _all_experts_scratch(self, n: int):
         spec, rt = self.spec, self.rt
@@ -230,7 +235,7 @@ class RoutedExperts(FeedForward):
             raise NotImplementedError("a shared expert with matrices of its own is a gated SiLU pair")
         act = ws.get("moe.shared_act", (n, FS), rt.dtype)
         if not ops.gemm_swiglu(x, self.w_shared_gate_up, act):
-            gu = ws.get("moe.shared_gate_up", (n, 2 * FS), rt.dtype)
+            gu = self._shared_gate_up(n)
             ops.gemm(x, self.w_shared_gate_up, gu)
             ops.swiglu(gu, act)
         ys = ws.get("moe.shared_out", (n, spec.hidden_size), rt.dtype)

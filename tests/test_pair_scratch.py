@@ -1,0 +1,47 @@
+"""Between a gated pair's two products lies a buffer that steps of one pass do not need: it is there before the cache is sized, also
+where the largest step goes in one pass and a smaller one does not."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from minivllm_amd.parts.base import Workspace
+from minivllm_amd.parts.mlp import ClampedGLU, ClampedGLUSpec, SwiGLU, SwiGLUSpec
+from minivllm_amd.parts.moe import RoutedExperts, RoutedExpertsSpec
+
+
+def part_of(cls, spec, one_pass):
+    ops = SimpleNamespace(use_fast_kernels=True, gemm_swiglu=lambda x, w, out, *a, **k: one_pass(x.shape[0]), gemm=lambda *a, **k: None,
+                          swiglu=lambda *a, **k: None, add_rows=lambda *a: None)
+    rt = SimpleNamespace(dtype=torch.bfloat16, ops=ops, workspace=Workspace(torch.device("cpu")))
+    return cls(spec, {name: torch.zeros(decl.shape, dtype=torch.bfloat16) for name, decl in cls.tensors(spec).items()}, rt)
+
+
+@pytest.mark.parametrize("cls, spec", [
+    (SwiGLU, SwiGLUSpec(hidden_size=64, intermediate_size=128)),
+    (ClampedGLU, ClampedGLUSpec(hidden_size=64, intermediate_size=128, limit=7.0)),
+    # (experts whose chosen pairs may go through the plain kernels: the shared one keeps matrices of its own)
+    (RoutedExperts, RoutedExpertsSpec(hidden_size=64, expert_size=96, num_experts=4, top=2, shared_size=32, grouped_min_weight=1))])
+@pytest.mark.parametrize("one_pass", [lambda n: n > 128, lambda n: n < 100 or n > 128, lambda n: n != 77, lambda n: n > 1])
+def test_no_smaller_step_needs_more(cls, spec, one_pass):
+    part, most = part_of(cls, spec, one_pass), 300
+    ws = part.rt.workspace
+    if cls is RoutedExperts:
+        assert not part.shared_packed
+        run = lambda n: part._add_shared(torch.zeros(n, 64), torch.zeros(n, 64))
+    else:
+        run = lambda n: part.forward(torch.zeros(n, 64), None)
+    part.reserve(most)
+    run(most)
+    ws.frozen = True                     # (a buffer that would have to grow raises)
+    for n in range(1, most + 1):
+        run(n)
+
+
+def test_the_rule_for_one_pass_is_not_monotone():
+    """What makes the buffer necessary: more rows go in one pass where fewer do not."""
+    import ctypes
+    from minivllm_amd.csrc import build
+    shape = ctypes.CDLL(build.find_library("bf16") or build.build("bf16")).mv_gemm_pair_shape
+    assert shape(1024, 256, 128, 256) and not shape(128, 256, 128, 256)
+    assert shape(2048, 12288, 2048, 256) and not shape(1792, 12288, 2048, 256)
