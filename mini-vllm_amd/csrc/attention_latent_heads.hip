@@ -15,10 +15,9 @@
 //   kr  [b][t][step s of DR / 32][lane]             the rotated channels, the same for all heads
 //   v   [b][h][tile dt of 8][lane]                  channel 16 dt + rho of keys 8 g .. 8 g + 7
 // What bounds it: a wave's block of 32 keys is a chain (scores, maximum, exponentials, sums) of 0.6 us, and a compute unit's two
-// workgroups take 0.75 us for one each, LDS 70 % busy with the operands (wide units read them for twice the columns). 256 + 64, 16
+// workgroups take 0.75 us for one each, LDS 70 % busy with the operands. 256 + 64, 16
 // heads, one request of 200 / 1,000 / 2,048 / 8,000 tokens: 50 / 111 / 193 / 1,248 us in the latent's space with its maps in and out,
-// 16 / 31 / 55 / 342 here (2,048: 11.5 for the keys and values, 42 for attention, 510 TFLOP/s of what causality leaves; 8,000: 35 and
-// 304, 1,079 TFLOP/s).
+// 16 / 31 / 55 / 438 here (2,048: 11.5 for the keys and values, 42 for attention, 510 TFLOP/s of what causality leaves).
 //
 // These are the operands of v_mfma_f32_16x16x32_bf16 as attention_prefill.hip holds them in LDS (the order of a tile's keys lets a
 // lane's probabilities be the second product's operand as they are), so a load instruction is a kilobyte of whole lines.
@@ -27,6 +26,7 @@
 #define ALH_DIM 128                                            // plain channels of a head, and channels of its values
 #define ALH_WAVES 4
 #define ALH_THREADS (64 * ALH_WAVES)
+#define ALH_TOKENS (16 * ALH_WAVES)                            // of a unit
 #define ALH_KEYS 32
 #define ALH_TILE 512                                           // pieces of a block's k, and of its v, a head
 #define ALH_LOG2E 1.4426950408889634f
@@ -189,13 +189,14 @@ struct AlhArgs {
     int n, fold;
 };
 
-// A workgroup of four waves serves one head of a unit, a run of 64 NT tokens of a request; each wave has 16 NT of them. Blocks of 32 keys
+// A workgroup of four waves serves one head of a unit, a run of 64 tokens of a request; each wave has 16 of them. Blocks of 32 keys
 // walk through four LDS stages in two pairs as in attention_prefill.hip: two blocks to a barrier, which stands between the two;
-// a block's operands come from LDS while the block before is computed.
-template <int DRS, int NT>
+// a block's operands come from LDS while the block before is computed. (32 tokens a wave read the operands half as often, but 100
+// registers of them do not fit: 4,100 tokens of one request 439 us with its keys and values, 8,000 1,125, so 151 and 438.)
+template <int DRS>
 __global__ void __launch_bounds__(ALH_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 attention_latent_heads_kernel(AlhArgs a) {
-    constexpr int DS = 4 + DRS, DT = 8, TOKENS = 16 * ALH_WAVES * NT;
+    constexpr int DS = 4 + DRS, DT = 8;
     constexpr int KR0 = ALH_TILE, V0 = ALH_TILE + 2 * DRS * 64, STAGE = V0 + ALH_TILE;     // pieces
     __shared__ uint4 ring[4 * STAGE];                          // (80 KB with 64 rotary channels: two workgroups a compute unit)
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / MV_WAVE), lane = tid % MV_WAVE;
@@ -214,61 +215,52 @@ attention_latent_heads_kernel(AlhArgs a) {
     const int n_all = gridDim.y, half = (n_all + 1) / 2, y = blockIdx.y;
     const int u = (!a.fold || y < half) ? n_all - 1 - y : y - half;
     const auto len_of = [&](int s) { return a.cu_seqlens[s + 1] - a.cu_seqlens[s]; };
-    const AlhPlace at = alh_find(u, a.n_seqs, [&](int s) { return (len_of(s) + TOKENS - 1) / TOKENS; },
+    const AlhPlace at = alh_find(u, a.n_seqs, [&](int s) { return (len_of(s) + ALH_TOKENS - 1) / ALH_TOKENS; },
                                  [&](int s) { return alh_blocks(len_of(s), a.context_lens[s]); });
     if (at.seq < 0) return;
     const int first_row = __builtin_amdgcn_readfirstlane(a.cu_seqlens[at.seq]);
-    const int t0 = first_row + at.in * TOKENS;
-    const int left = __builtin_amdgcn_readfirstlane(len_of(at.seq)) - at.in * TOKENS, nt = left < TOKENS ? left : TOKENS;
+    const int t0 = first_row + at.in * ALH_TOKENS;
+    const int left = __builtin_amdgcn_readfirstlane(len_of(at.seq)) - at.in * ALH_TOKENS, nt = left < ALH_TOKENS ? left : ALH_TOKENS;
     const int pos0 = __builtin_amdgcn_readfirstlane(a.positions[t0]);     // (a request's rows follow each other)
     const int last = (pos0 + nt - 1) / ALH_KEYS;                          // the walk's last block
 
-    int col_pos[NT], col_tok[NT];
-    AlhFrag qop[NT][DS];
+    const int col = wave * 16 + i;
+    const bool ok = col < nt;
+    const int col_tok = t0 + (ok ? col : nt - 1);              // (columns that do not exist: another's, never stored)
+    const int col_pos = ok ? pos0 + col : -1;
+    AlhFrag qop[DS];
+    const bf16* row = a.q + (size_t)col_tok * a.ldq + (size_t)head * (ALH_DIM + 32 * DRS) + 8 * g;
 #pragma unroll
-    for (int ct = 0; ct < NT; ++ct) {
-        const int col = (wave * NT + ct) * 16 + i;
-        const bool ok = col < nt;
-        col_tok[ct] = t0 + (ok ? col : nt - 1);                // (columns that do not exist: another's, never stored)
-        col_pos[ct] = ok ? pos0 + col : -1;
-        const bf16* row = a.q + (size_t)col_tok[ct] * a.ldq + (size_t)head * (ALH_DIM + 32 * DRS) + 8 * g;
+    for (int s = 0; s < DS; ++s) qop[s].u = *reinterpret_cast<const uint4*>(row + 32 * s);
+    if constexpr (DRS == 2) {                                  // channel c of the rotary part turns with c + 32: the same lane holds both
+        const float* cs = a.table + (size_t)(pos0 + (ok ? col : nt - 1)) * 64 + 8 * g;
+        float c[8], s[8];
+        Vec8<float>::load(cs, c);
+        Vec8<float>::load(cs + 32, s);
+        AlhFrag lo = qop[4], hi = qop[5];
+        float x[8], z[8];
 #pragma unroll
-        for (int s = 0; s < DS; ++s) qop[ct][s].u = *reinterpret_cast<const uint4*>(row + 32 * s);
-        if constexpr (DRS == 2) {                              // channel c of the rotary part turns with c + 32: the same lane holds both
-            const float* cs = a.table + (size_t)(pos0 + (ok ? col : nt - 1)) * 64 + 8 * g;
-            float c[8], s[8];
-            Vec8<float>::load(cs, c);
-            Vec8<float>::load(cs + 32, s);
-            AlhFrag lo = qop[ct][4], hi = qop[ct][5];
-            float x[8], z[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float p = __uint_as_float((uint32_t)lo.h[e] << 16), n = __uint_as_float((uint32_t)hi.h[e] << 16);
-                x[e] = p * c[e] - n * s[e];
-                z[e] = n * c[e] + p * s[e];
-            }
-            qop[ct][4].u = uint4{f32x2_to_bf16x2_bits(x[0], x[1]), f32x2_to_bf16x2_bits(x[2], x[3]), f32x2_to_bf16x2_bits(x[4], x[5]), f32x2_to_bf16x2_bits(x[6], x[7])};
-            qop[ct][5].u = uint4{f32x2_to_bf16x2_bits(z[0], z[1]), f32x2_to_bf16x2_bits(z[2], z[3]), f32x2_to_bf16x2_bits(z[4], z[5]), f32x2_to_bf16x2_bits(z[6], z[7])};
+        for (int e = 0; e < 8; ++e) {
+            const float p = __uint_as_float((uint32_t)lo.h[e] << 16), n = __uint_as_float((uint32_t)hi.h[e] << 16);
+            x[e] = p * c[e] - n * s[e];
+            z[e] = n * c[e] + p * s[e];
         }
+        qop[4].u = uint4{f32x2_to_bf16x2_bits(x[0], x[1]), f32x2_to_bf16x2_bits(x[2], x[3]), f32x2_to_bf16x2_bits(x[4], x[5]), f32x2_to_bf16x2_bits(x[6], x[7])};
+        qop[5].u = uint4{f32x2_to_bf16x2_bits(z[0], z[1]), f32x2_to_bf16x2_bits(z[2], z[3]), f32x2_to_bf16x2_bits(z[4], z[5]), f32x2_to_bf16x2_bits(z[6], z[7])};
     }
     // blocks up to bm need no mask: all the wave's columns exist and see all their keys
-    const int wave0 = pos0 + wave * NT * 16;
-    const int bm = (wave + 1) * NT * 16 <= nt && wave0 >= ALH_KEYS - 1 ? (wave0 - (ALH_KEYS - 1)) / ALH_KEYS : -1;
+    const int wave0 = pos0 + wave * 16;
+    const int bm = (wave + 1) * 16 <= nt && wave0 >= ALH_KEYS - 1 ? (wave0 - (ALH_KEYS - 1)) / ALH_KEYS : -1;
 
-    float m_run[NT];
-    floatx4_t acc[NT][DT], l_run[NT];                          // (a row of ones times the weights: a lane's four are one number)
+    float m_run = -INFINITY;
+    floatx4_t acc[DT], l_run = floatx4_t{0.f, 0.f, 0.f, 0.f};  // (a row of ones times the weights: a lane's four are one number)
 #pragma unroll
-    for (int ct = 0; ct < NT; ++ct) {
-        m_run[ct] = -INFINITY;
-        l_run[ct] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) acc[ct][dt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int dt = 0; dt < DT; ++dt) acc[dt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
     const float sc = a.scale * ALH_LOG2E;
     AlhFrag ones;
     ones.u = uint4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
 
-    // a block's way into LDS: five (three without a rotary part: four) loads of a kilobyte a wave
+    // a block's way into LDS: five loads of a kilobyte a wave (four without a rotary part)
     auto fetch = [&](int j, uint4* stage) __attribute__((always_inline)) {
         const int b = at.before + (j < last ? j : last);       // (past the end: the last block again, it does no harm)
         const size_t own = ((size_t)b * a.H + head) * ALH_TILE;
@@ -301,65 +293,54 @@ attention_latent_heads_kernel(AlhArgs a) {
     // the two products with the softmax between them; behind the score products, asks for the next block's keys and (now) this block's values
     auto compute = [&](int j, const KOps& ko, VOps& vo, const uint4* v_now, const uint4* k_next, KOps& kn, const bool ask_v) __attribute__((always_inline)) {
         const int base = ALH_KEYS * j;
-        float p[NT][2][4];
+        float p[2][4];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t) {
+            floatx4_t s4 = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int ct = 0; ct < NT; ++ct) {
-                floatx4_t s4 = floatx4_t{0.f, 0.f, 0.f, 0.f};
+            for (int s = 0; s < DS; ++s) s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ko.f[t][s].v, qop[s].v, s4, 0, 0, 0);
 #pragma unroll
-                for (int s = 0; s < DS; ++s) s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ko.f[t][s].v, qop[ct][s].v, s4, 0, 0, 0);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) p[ct][t][e] = s4[e];
-            }
+            for (int e = 0; e < 4; ++e) p[t][e] = s4[e];
+        }
         __builtin_amdgcn_sched_barrier(0);
         if (ask_v) read_v(v_now, vo);
         read_k(k_next, kn);
         __builtin_amdgcn_sched_barrier(0);
         if (j > bm) {                                          // (the same for the wave; kept a branch, see attention_prefill.hip)
             asm volatile("");
-#pragma unroll
-            for (int ct = 0; ct < NT; ++ct) {
-                const int hi = col_pos[ct] - base - 8 * g;
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) p[ct][t][e] = 4 * t + e <= hi ? p[ct][t][e] : -INFINITY;
-            }
-        }
-        AlhFrag pop[NT];
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-            float mx = -INFINITY;
+            const int hi = col_pos - base - 8 * g;
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) mx = fmaxf(mx, p[ct][t][e]);
-            // (the exponentials' reference only follows a maximum that has overtaken it by 2^8: until then nothing is rescaled)
-            if (__any(mx * sc > m_run[ct] + 8.f)) {
-                mx = fmaxf(mx, __shfl_xor(mx, 16, MV_WAVE));
-                mx = fmaxf(mx, __shfl_xor(mx, 32, MV_WAVE));
-                const float m_new = fmaxf(m_run[ct], mx * sc), ref = m_new == -INFINITY ? 0.f : m_new;
-                const float corr = __builtin_amdgcn_exp2f(m_run[ct] - ref);
-                l_run[ct] *= corr;
-                m_run[ct] = m_new;
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) acc[ct][dt] *= corr;
-            }
-            const float ref = m_run[ct] == -INFINITY ? 0.f : m_run[ct];
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) pop[ct].v[4 * t + e] = (__bf16)__builtin_amdgcn_exp2f(fmaf(p[ct][t][e], sc, -ref));
+                for (int e = 0; e < 4; ++e) p[t][e] = 4 * t + e <= hi ? p[t][e] : -INFINITY;
         }
+        AlhFrag pop;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mx = fmaxf(mx, p[t][e]);
+        // (the exponentials' reference only follows a maximum that has overtaken it by 2^8: until then nothing is rescaled)
+        if (__any(mx * sc > m_run + 8.f)) {
+            mx = fmaxf(mx, __shfl_xor(mx, 16, MV_WAVE));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, MV_WAVE));
+            const float m_new = fmaxf(m_run, mx * sc), ref = m_new == -INFINITY ? 0.f : m_new;
+            const float corr = __builtin_amdgcn_exp2f(m_run - ref);
+            l_run *= corr;
+            m_run = m_new;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) acc[dt] *= corr;
+        }
+        const float ref = m_run == -INFINITY ? 0.f : m_run;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) pop.v[4 * t + e] = (__bf16)__builtin_amdgcn_exp2f(fmaf(p[t][e], sc, -ref));
         // the denominator is the sum of the weights as the values see them, rounded, so that what rounding does to all of them alike cancels
         // (one layer against 64 bits, 100 to 4,000 tokens: 0.1 to 1 % nearer; a product more instead of eight additions, the same time)
+        l_run = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pop.v, l_run, 0, 0, 0);
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct) l_run[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pop[ct].v, l_run[ct], 0, 0, 0);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int ct = 0; ct < NT; ++ct) acc[ct][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vo.f[dt].v, pop[ct].v, acc[ct][dt], 0, 0, 0);
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vo.f[dt].v, pop.v, acc[dt], 0, 0, 0);
     };
 
     uint4 *s0 = ring, *s1 = ring + STAGE, *s2 = ring + 2 * STAGE, *s3 = ring + 3 * STAGE;
@@ -392,32 +373,29 @@ attention_latent_heads_kernel(AlhArgs a) {
     }
     GT_WAIT_VMCNT(0);                                          // (a workgroup ends with nothing on its way into its LDS)
 
+    const float l = l_run[0];
+    if (!ok) return;
+    float inv = 1.f / l;
+    if (a.sink != nullptr) {                                   // one more term of the denominator, without a value
+        const float sk = a.sink[head] * ALH_LOG2E, m = fmaxf(m_run, sk), f = exp2f(m_run - m);
+        inv = f / fmaf(f, l, exp2f(sk - m));
+    }
+    const bf16* gates = a.gate == nullptr ? nullptr : a.gate + (size_t)col_tok * a.ldg + (a.gate_per_head ? head : head * ALH_DIM);
+    if (gates != nullptr && a.gate_per_head) inv *= 1.f / (1.f + expf(-to_f(*gates)));
+    bf16* to = a.out + (size_t)col_tok * a.ldo + (size_t)head * ALH_DIM + 4 * g;
 #pragma unroll
-    for (int ct = 0; ct < NT; ++ct) {
-        const float l = l_run[ct][0];
-        if (col_pos[ct] < 0) continue;
-        float inv = 1.f / l;
-        if (a.sink != nullptr) {                               // one more term of the denominator, without a value
-            const float sk = a.sink[head] * ALH_LOG2E, m = fmaxf(m_run[ct], sk), f = exp2f(m_run[ct] - m);
-            inv = f / fmaf(f, l, exp2f(sk - m));
-        }
-        const bf16* gates = a.gate == nullptr ? nullptr : a.gate + (size_t)col_tok[ct] * a.ldg + (a.gate_per_head ? head : head * ALH_DIM);
-        if (gates != nullptr && a.gate_per_head) inv *= 1.f / (1.f + expf(-to_f(*gates)));
-        bf16* to = a.out + (size_t)col_tok[ct] * a.ldo + (size_t)head * ALH_DIM + 4 * g;
+    for (int dt = 0; dt < DT; ++dt) {
+        float o[4];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            float o[4];
+        for (int e = 0; e < 4; ++e) o[e] = acc[dt][e] * inv;
+        if (gates != nullptr && !a.gate_per_head)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = acc[ct][dt][e] * inv;
-            if (gates != nullptr && !a.gate_per_head)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] *= 1.f / (1.f + expf(-to_f(gates[16 * dt + 4 * g + e])));
-            *reinterpret_cast<uint2*>(to + 16 * dt) = uint2{f32x2_to_bf16x2_bits(o[0], o[1]), f32x2_to_bf16x2_bits(o[2], o[3])};
-        }
+            for (int e = 0; e < 4; ++e) o[e] *= 1.f / (1.f + expf(-to_f(gates[16 * dt + 4 * g + e])));
+        *reinterpret_cast<uint2*>(to + 16 * dt) = uint2{f32x2_to_bf16x2_bits(o[0], o[1]), f32x2_to_bf16x2_bits(o[2], o[3])};
     }
 }
 
-extern "C" int mv_attention_latent_heads_tokens(int wide) { return 16 * ALH_WAVES * (wide ? 2 : 1); }
+extern "C" int mv_attention_latent_heads_tokens() { return ALH_TOKENS; }
 extern "C" int mv_attention_latent_heads_keys() { return ALH_KEYS; }
 // 1: heads of `plain` + DR channels and values of `vdim` over a latent of R are served
 extern "C" int mv_attention_latent_heads_serves(int plain, int vdim, int R, int DR) {
@@ -447,12 +425,12 @@ extern "C" int mv_latent_expand(const void* pages, const int* block_table, int b
     return mv_check_launch("latent_expand");
 }
 
-// `units`: runs of mv_attention_latent_heads_tokens(wide) tokens of the step's requests, or an upper bound (the rest of the grid
+// `units`: runs of mv_attention_latent_heads_tokens() tokens of the step's requests, or an upper bound (the rest of the grid
 // ends at once); `busy`: how many hold tokens, as far as the caller knows. A request's rows stand at neighbouring positions.
 // `padding`: there may be rows of no request; they become zeros.
 extern "C" int mv_attention_latent_heads(const void* q, long ldq, void* out, long ldo, const void* k, const void* kr, const void* v,
                                          const int* positions, const int* token_seq, const int* cu_seqlens, const int* context_lens, int n_seqs,
-                                         int units, int busy, int wide, int n, int padding, int H, int DR, float scale, const float* table,
+                                         int units, int busy, int n, int padding, int H, int DR, float scale, const float* table,
                                          const float* sink, const void* gate, long ldg, int gate_per_head, hipStream_t stream) {
     MV_REQUIRE(n >= 0 && n_seqs >= 0 && units >= 0 && units <= 65535 && H > 0 && (DR == 0 || DR == 64), "attention_latent_heads: bad sizes n=%d H=%d DR=%d units=%d", n, H, DR, units);
     MV_REQUIRE(ldq >= (long)H * (ALH_DIM + DR) && ldq % 8 == 0 && ldo >= (long)H * ALH_DIM && ldo % 4 == 0 && (!gate || ldg >= (gate_per_head ? H : (long)H * ALH_DIM)),
@@ -467,14 +445,9 @@ extern "C" int mv_attention_latent_heads(const void* q, long ldq, void* out, lon
     const AlhArgs a{(const bf16*)q, ldq, (bf16*)out, ldo, (const uint4*)k, (const uint4*)kr, (const uint4*)v, positions, cu_seqlens, context_lens, n_seqs, H,
                     scale, table, sink, (const bf16*)gate, ldg, gate_per_head, padding ? token_seq : nullptr, n, fold};
     const dim3 grid(H, units > 0 ? units : 1);
-#define ALH_LAUNCH(DRS, NT) hipLaunchKernelGGL((attention_latent_heads_kernel<DRS, NT>), grid, dim3(ALH_THREADS), 0, stream, a)
-    if (DR == 64) {
-        if (wide) ALH_LAUNCH(2, 2);
-        else ALH_LAUNCH(2, 1);
-    } else {
-        if (wide) ALH_LAUNCH(0, 2);
-        else ALH_LAUNCH(0, 1);
-    }
+#define ALH_LAUNCH(DRS) hipLaunchKernelGGL(attention_latent_heads_kernel<DRS>, grid, dim3(ALH_THREADS), 0, stream, a)
+    if (DR == 64) ALH_LAUNCH(2);
+    else ALH_LAUNCH(0);
 #undef ALH_LAUNCH
     return mv_check_launch("attention_latent_heads");
 }

@@ -218,16 +218,16 @@ _OPTIONAL_SIGNATURES = {
                                            c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p,
                                            c_void_p]),
     # the same up to sink, then max_context, work, work_floats, stream
-    "mv_attention_latent_heads_tokens": (c_int, [c_int]),
+    "mv_attention_latent_heads_tokens": (c_int, []),
     "mv_attention_latent_heads_keys": (c_int, []),
     "mv_attention_latent_heads_serves": (c_int, [c_int, c_int, c_int, c_int]),
     # pages, block_table, bt_width, page_size, cu_seqlens, context_lens, n_seqs, w_k, w_v, H, R, DR, k, kr, v, blocks, stream
     "mv_latent_expand": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int,
                                  c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
-    # q, ldq, out, ldo, k, kr, v, positions, token_seq, cu_seqlens, context_lens, n_seqs, units, busy, wide, n, padding, H, DR, scale, table,
+    # q, ldq, out, ldo, k, kr, v, positions, token_seq, cu_seqlens, context_lens, n_seqs, units, busy, n, padding, H, DR, scale, table,
     # sink, gate, ldg, gate_per_head, stream
     "mv_attention_latent_heads": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
-                                          c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_void_p,
+                                          c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_void_p,
                                           c_void_p, c_long, c_int, c_void_p]),
     "mv_attention_latent_split_mfma": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
                                                c_void_p, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p, c_int, c_void_p, c_long,

@@ -1626,15 +1626,14 @@ class Ops:
             self._act(gate, "output gate")
             if gate.dim() != 2 or gate.shape[0] != n or gate.stride(1) != 1 or (gate.shape[1] < heads if gate_per_head else gate.shape[1] != heads * 128):
                 raise KernelLibraryError("attention_latent_heads: the gate must be [n, heads * 128], or [n, >= heads] with one number a head")
-        tokens = self.lib.dll.mv_attention_latent_heads_tokens
-        wide = plan.busy_units(tokens(1)) * heads >= 2 * self.compute_units
-        units, busy = plan.units(tokens(int(wide))), plan.busy_units(tokens(int(wide)))
+        tokens = self.lib.dll.mv_attention_latent_heads_tokens()
+        units, busy = plan.units(tokens), plan.busy_units(tokens)
         pitch = lambda t: t.stride(0) if n > 1 else t.shape[1]
         self._note("mv_attention_latent_heads", self._size(q, out) + plan.kv_tokens * heads * (256 + rot_dim) * 2,
                    2 * plan.attention_pairs * heads * (256 + rot_dim))
         self.lib.call("mv_attention_latent_heads", q.data_ptr(), pitch(q), out.data_ptr(), pitch(out), k.data_ptr(), kr.data_ptr(), v.data_ptr(),
                       positions.data_ptr(), token_seq.data_ptr(), plan.cu_seqlens.data_ptr(), context_lens.data_ptr(), plan.n_seqs, units, busy,
-                      int(wide), n, int(plan.bound is not None or sum(plan.q_lens) != n), heads, rot_dim, float(scale), _ptr(table), _ptr(sink),
+                      n, int(plan.bound is not None or sum(plan.q_lens) != n), heads, rot_dim, float(scale), _ptr(table), _ptr(sink),
                       _ptr(gate), pitch(gate) if gate is not None else 0, int(gate_per_head), self._stream())
 
     def latent_shares(self, heads: int, window: int, lens: Sequence[int], starts: Sequence[int]) -> bool:
