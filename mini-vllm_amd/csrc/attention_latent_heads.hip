@@ -14,10 +14,18 @@
 //   k   [b][h][tile t of 2][step s of 4][lane]      lane (g, rho) = 16 g + rho: channels 32 s + 8 g.. of key 8 (rho / 4) + 4 t + rho % 4
 //   kr  [b][t][step s of DR / 32][lane]             the rotated channels, the same for all heads
 //   v   [b][h][tile dt of 8][lane]                  channel 16 dt + rho of keys 8 g .. 8 g + 7
-// What bounds it: a wave's block of 32 keys is a chain (scores, maximum, exponentials, sums) of 0.6 us, and a compute unit's two
-// workgroups take 0.75 us for one each, LDS 70 % busy with the operands. 256 + 64, 16
-// heads, one request of 200 / 1,000 / 2,048 / 8,000 tokens: 50 / 111 / 193 / 1,248 us in the latent's space with its maps in and out,
-// 16 / 31 / 55 / 438 here (2,048: 11.5 for the keys and values, 42 for attention, 510 TFLOP/s of what causality leaves).
+// What bounds it: a wave's block of 32 keys is a chain (scores, maximum, exponentials, sums) of 0.7 us, and a compute unit's two
+// workgroups take 0.85 us for one each, LDS 60 % busy with the operands. 256 + 64, 16 heads, one request of 200 / 1,000 / 2,048 /
+// 8,000 tokens, us by events around 30 calls: in the latent's space with its maps in and out 56 / 117 / 202 / 1,265, here 32 / 40 / 68 / 553
+// (2,048: 11.5 for the keys and values).
+//
+// Precision: the keys and values are rounded to 16 bits here where the carried queries and the sums of latents are there, so two
+// roundings that both have are taken out: the weights and the turned channels of the queries are two operands each, the rounded
+// number and what that leaves (13 products more beside 21; 2,048 tokens 59.5 -> 68 us). Error against 64 bits over that of the
+// latent's space, scores of a deviation of 0.3 / 1 / 3, 65 to 8,000 tokens and 100 to 300 behind 500 to 2,000: 0.76 to 0.92, 0.69 to
+// 0.92, 0.90 to 0.91; with neither 0.90 to 1.03, 0.79 to 1.01, 1.00 to 1.04, with the weights' alone up to 1.01, with the queries' alone
+// up to 1.02. Without a rotary part there is no turned channel, and sharp weights (a deviation of 3) are up to 4 % further off than in
+// the latent's space: models of that kind stay there (LatentAttention.heads_operands).
 //
 // These are the operands of v_mfma_f32_16x16x32_bf16 as attention_prefill.hip holds them in LDS (the order of a tile's keys lets a
 // lane's probabilities be the second product's operand as they are), so a load instruction is a kilobyte of whole lines.
@@ -228,7 +236,7 @@ attention_latent_heads_kernel(AlhArgs a) {
     const bool ok = col < nt;
     const int col_tok = t0 + (ok ? col : nt - 1);              // (columns that do not exist: another's, never stored)
     const int col_pos = ok ? pos0 + col : -1;
-    AlhFrag qop[DS];
+    AlhFrag qop[DS], qrest[DRS > 0 ? DRS : 1];                 // (rest: what the turned channels' rounding leaves)
     const bf16* row = a.q + (size_t)col_tok * a.ldq + (size_t)head * (ALH_DIM + 32 * DRS) + 8 * g;
 #pragma unroll
     for (int s = 0; s < DS; ++s) qop[s].u = *reinterpret_cast<const uint4*>(row + 32 * s);
@@ -245,8 +253,13 @@ attention_latent_heads_kernel(AlhArgs a) {
             x[e] = p * c[e] - n * s[e];
             z[e] = n * c[e] + p * s[e];
         }
-        qop[4].u = uint4{f32x2_to_bf16x2_bits(x[0], x[1]), f32x2_to_bf16x2_bits(x[2], x[3]), f32x2_to_bf16x2_bits(x[4], x[5]), f32x2_to_bf16x2_bits(x[6], x[7])};
-        qop[5].u = uint4{f32x2_to_bf16x2_bits(z[0], z[1]), f32x2_to_bf16x2_bits(z[2], z[3]), f32x2_to_bf16x2_bits(z[4], z[5]), f32x2_to_bf16x2_bits(z[6], z[7])};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            qop[4].v[e] = (__bf16)x[e];
+            qop[5].v[e] = (__bf16)z[e];
+            qrest[0].v[e] = (__bf16)(x[e] - (float)qop[4].v[e]);
+            qrest[1].v[e] = (__bf16)(z[e] - (float)qop[5].v[e]);
+        }
     }
     // blocks up to bm need no mask: all the wave's columns exist and see all their keys
     const int wave0 = pos0 + wave * 16;
@@ -300,6 +313,8 @@ attention_latent_heads_kernel(AlhArgs a) {
 #pragma unroll
             for (int s = 0; s < DS; ++s) s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ko.f[t][s].v, qop[s].v, s4, 0, 0, 0);
 #pragma unroll
+            for (int s = 0; s < DRS; ++s) s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ko.f[t][4 + s].v, qrest[s].v, s4, 0, 0, 0);
+#pragma unroll
             for (int e = 0; e < 4; ++e) p[t][e] = s4[e];
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -314,7 +329,7 @@ attention_latent_heads_kernel(AlhArgs a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) p[t][e] = 4 * t + e <= hi ? p[t][e] : -INFINITY;
         }
-        AlhFrag pop;
+        AlhFrag pop, rest;
         float mx = -INFINITY;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -335,12 +350,18 @@ attention_latent_heads_kernel(AlhArgs a) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) pop.v[4 * t + e] = (__bf16)__builtin_amdgcn_exp2f(fmaf(p[t][e], sc, -ref));
-        // the denominator is the sum of the weights as the values see them, rounded, so that what rounding does to all of them alike cancels
-        // (one layer against 64 bits, 100 to 4,000 tokens: 0.1 to 1 % nearer; a product more instead of eight additions, the same time)
+            for (int e = 0; e < 4; ++e) {
+                const float w = __builtin_amdgcn_exp2f(fmaf(p[t][e], sc, -ref));
+                pop.v[4 * t + e] = (__bf16)w;
+                rest.v[4 * t + e] = (__bf16)(w - (float)pop.v[4 * t + e]);
+            }
+        // (the denominator too is a product, with a row of ones)
         l_run = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pop.v, l_run, 0, 0, 0);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vo.f[dt].v, pop.v, acc[dt], 0, 0, 0);
+        l_run = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, rest.v, l_run, 0, 0, 0);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vo.f[dt].v, rest.v, acc[dt], 0, 0, 0);
     };
 
     uint4 *s0 = ring, *s1 = ring + STAGE, *s2 = ring + 2 * STAGE, *s3 = ring + 3 * STAGE;

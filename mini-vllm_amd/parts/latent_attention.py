@@ -155,9 +155,10 @@ class LatentAttention(Mixer):
         self.w_uk_rows = self.w_uk.transpose(1, 2).contiguous()
         self.w_uv_rows = tensors["uv"].view(spec.num_heads, spec.value_dim, spec.kv_rank).contiguous()
         self.w_o = tensors["o"]
-        # ... and in the order in which the heads' own keys and values are made from the latents
+        # ... and in the order in which the heads' own keys and values are made from the latents (without a rotary part that is less
+        # precise than the latent's space, see attention_latent_heads.hip)
         self.heads_operands = None
-        if spec.window is None and spec.scale > 0 and rt.dtype == torch.bfloat16 == self.w_uk.dtype == self.w_uv.dtype \
+        if spec.window is None and spec.scale > 0 and spec.rot_dim and rt.dtype == torch.bfloat16 == self.w_uk.dtype == self.w_uv.dtype \
                 and rt.ops.latent_heads_serve(spec.plain_dim, spec.value_dim, spec.kv_rank, spec.rot_dim):
             self.heads_operands = latent_operands(self.w_uk), latent_operands(self.w_uv_rows)
 

@@ -125,3 +125,47 @@ def test_a_recorded_model_follows_the_eager_one():
             assert float((got - plain).abs().max() / plain.abs().max()) <= 2e-2, cut
     entries = [{e[0] for e in ledger} for ledger in recorded.graph_ledger.values()]
     assert entries and all("mv_attention_latent_heads" in e and "mv_attention_latent_prompt" not in e for e in entries)
+
+
+@pytest.mark.parametrize("spread", [0.3, 1.0, 3.0])
+@pytest.mark.parametrize("n, start", [(65, 0), (200, 0), (700, 0), (90, 500)])
+def test_no_further_from_64_bits_than_the_latents_space(n, start, spread):
+    """Both ways of the same attention, scores of three deviations. Whichever roundings one way has in place of the other's, its error
+    is no larger (0.75 to 0.93 of it, measured over 65 to 8,000 tokens)."""
+    from minivllm_amd.engine.step import AttentionPlan
+    from minivllm_amd.kernels.ops import Ops, latent_operands
+    from minivllm_amd.parts import Workspace
+    R, dr, H, ps = 256, 64, 4, 16
+    ops, gen, ctx, scale = Ops(torch.bfloat16), torch.Generator().manual_seed(n), n + start, 192 ** -0.5
+    rand = lambda *shape: torch.randn(*shape, generator=gen)
+    lat, q = rand(ctx, R + dr).bfloat16(), (rand(n, H * (128 + dr)) * spread).bfloat16()
+    w_k, w_v = (rand(H, 128, R) / math.sqrt(R)).bfloat16(), (rand(H, 128, R) / math.sqrt(R)).bfloat16()
+    angle = torch.arange(ctx)[:, None] * (1e4 ** (-torch.arange(0, dr, 2) / dr))[None]
+    table = torch.cat([angle.cos(), angle.sin()], 1).float()
+    want = torch.empty(n, H, 128, dtype=torch.float64)
+    cos, sin = table[start:, :32].double(), table[start:, 32:].double()
+    hidden = torch.arange(ctx)[None] > torch.arange(start, ctx)[:, None]
+    for h in range(H):
+        x, c = q.double().view(n, H, -1)[:, h], lat[:, :R].double()
+        a, b = x[:, 128:160], x[:, 160:]
+        s = x[:, :128] @ (c @ w_k[h].double().T).T + torch.cat([a * cos - b * sin, b * cos + a * sin], -1) @ lat[:, R:].double().T
+        want[:, h] = torch.softmax((s * scale).masked_fill(hidden, -math.inf), -1) @ (c @ w_v[h].double().T)
+    i32 = lambda x: torch.tensor(list(x), dtype=torch.int32, device=DEV)
+    npages = -(-ctx // ps)
+    pages = torch.zeros(npages, ps, R + dr, dtype=torch.bfloat16, device=DEV)
+    pages.view(-1, R + dr)[:ctx] = lat.to(DEV)
+    bt, positions, seq, cl, cu = i32(range(npages)).view(1, -1), i32(range(start, ctx)), i32([0] * n), i32([ctx]), i32([0, n])
+    plan = AttentionPlan(decode_only=False, max_q_len=n, max_context_len=ctx, n_seqs=1, q_lens=[n], cu_seqlens=cu,
+                         workspace=Workspace(torch.device(DEV)), starts=[start])
+    blocks = -(-ctx // 32)
+    scratch = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device=DEV)
+    k, v, kr, own, latent = scratch(blocks, H, 4096), scratch(blocks, H, 4096), scratch(blocks, 32 * dr), scratch(n, H * 128), scratch(n, H * 128)
+    q, w_k, w_v, table = q.to(DEV), w_k.to(DEV), w_v.to(DEV), table.to(DEV)
+    ops.latent_expand(pages, bt, ps, plan, cl, latent_operands(w_k), latent_operands(w_v), H, R, dr, blocks, k, kr, v)
+    ops.attention_latent_heads(q, own, k, kr, v, plan, positions, seq, cl, H, dr, scale, table)
+    qa, mixed = torch.empty(n, H, R + dr, device=DEV), torch.empty(n, H, R, device=DEV)
+    ops.head_linear(q.unflatten(1, (H, 128 + dr)), w_k, qa, seq, tail=dr, table=table, positions=positions, w_rows=w_k.transpose(1, 2).contiguous())
+    ops.attention_latent(qa, mixed, pages, bt, ps, positions, seq, H, R, dr, scale, plan=plan, pages_t=pages[:, :, :R].transpose(1, 2).contiguous())
+    ops.head_linear(mixed, w_v.transpose(1, 2).contiguous(), latent, seq, w_rows=w_v)
+    off = [float((o.double().cpu() - want.flatten(1)).norm() / want.norm()) for o in (own, latent)]
+    assert off[0] <= off[1], off

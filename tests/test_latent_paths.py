@@ -67,14 +67,15 @@ def test_layers_of_one_spec_that_store_their_maps_differently_choose_for_themsel
     import torch
     from minivllm_amd.models.causal_lm import CausalLM
     from minivllm_amd.parts.latent_attention import LatentAttention, LatentAttentionSpec
-    spec = LatentAttentionSpec(hidden_size=256, num_heads=2, plain_dim=128, value_dim=128, kv_rank=128)
+    spec = LatentAttentionSpec(hidden_size=256, num_heads=2, plain_dim=128, rot_dim=64, value_dim=128, kv_rank=128)
     ops = SimpleNamespace(compute_units=256, latent_heads_serve=lambda *sizes: True, latent_shares_serve=lambda *sizes: True)
     ops.latent_heads, ops.latent_shares = lambda *a: Ops.latent_heads(ops, *a), lambda *a: Ops.latent_shares(ops, *a)
     rt = SimpleNamespace(dtype=torch.bfloat16, ops=ops)
 
     def layer(*wide):
         return LatentAttention(spec, {name: torch.zeros(decl.shape, dtype=torch.float32 if name in wide else torch.bfloat16)
-                                      for name, decl in LatentAttention.tensors(spec).items()}, rt)
+                                      for name, decl in LatentAttention.tensors(spec).items()}, rt,
+                               SimpleNamespace(rotary=lambda: (torch.zeros(1, 64), False)))
     both = [layer(), layer("uk")]
     lens, starts = [100], [0]
     own, latent = (m.step_path(lens, starts) for m in both)
@@ -82,3 +83,14 @@ def test_layers_of_one_spec_that_store_their_maps_differently_choose_for_themsel
     for mixers in (both, both[::-1], both + [layer(), layer("uv"), None]):
         assert set(CausalLM.step_paths(SimpleNamespace(_choosers=None, mixers=mixers), lens, starts)) == {own, latent}
     assert len(CausalLM.step_paths(SimpleNamespace(_choosers=None, mixers=[layer(), layer(), layer()]), lens, starts)) == 1
+
+
+def test_maps_without_a_rotary_part_stay_in_the_latents_space():
+    import torch
+    from minivllm_amd.parts.latent_attention import LatentAttention, LatentAttentionSpec
+    ops = SimpleNamespace(latent_heads_serve=lambda *sizes: True)
+    for rot_dim in (0, 64):
+        spec = LatentAttentionSpec(hidden_size=256, num_heads=2, plain_dim=128, rot_dim=rot_dim, value_dim=128, kv_rank=128)
+        part = LatentAttention(spec, {name: torch.zeros(decl.shape, dtype=torch.bfloat16) for name, decl in LatentAttention.tensors(spec).items()},
+                               SimpleNamespace(dtype=torch.bfloat16, ops=ops), SimpleNamespace(rotary=lambda: (torch.zeros(1, 64), False)))
+        assert (part.heads_operands is not None) is (rot_dim > 0)
