@@ -196,14 +196,24 @@ struct GatedPair {
         }
         return g / (1.f + expf(-g)) * u;
     }
-    // The same from the hardware's reciprocal and power of two (1 ulp each) for results that are rounded to 16 bits next: some 10
-    // instructions a number instead of 40, which the last waves of a product's workgroup do not hide.
+    // The same in few instructions (12 a number instead of 35), which the last waves of a product's workgroup do not hide, for results
+    // that are rounded to 16 bits next.
     __device__ __forceinline__ float of_short(float g, float u) const {
         if (limit > 0.f) {
             const float gc = fminf(g, limit), uc = fminf(fmaxf(u, -limit), limit);
-            return gc * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504f * slope * gc)) * (uc + 1.f);
+            return gc * sigmoid_short(slope * gc) * (uc + 1.f);
         }
-        return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504f * g)) * u;
+        return g * sigmoid_short(g) * u;
+    }
+    // 1 / (1 + 2^t) by the hardware, t the rounded -s log2(e), and what t's rounding is worth: with m = -s - t ln(2) the power is m of itself
+    // larger, the quotient m (1 - quotient) of itself smaller (the power may be infinite, the quotient is at most 1). Error of g sigmoid(g) u
+    // against 64 bits in 2^-24, root mean square, for |g| up to 8 / 40 / 60: 0.93 / 0.98 / 0.97 (`of` 0.79 / 0.76 / 0.75; without m 1.8 / 12 / 26),
+    // at most 4.6 (`of` 3.7): of the results in 16 bits the same but for one in 10^4 at most.
+    static __device__ __forceinline__ float sigmoid_short(float s) {
+        const float x = __builtin_amdgcn_fmed3f(s, -200.f, 200.f), t = -1.44269504f * x;
+        const float r = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(t));
+        const float m = fmaf(t, 1.90465497e-9f, fmaf(t, -0.693147182f, -x));
+        return fmaf(r, fmaf(m, r, -m), r);
     }
 };
 

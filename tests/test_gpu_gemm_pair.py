@@ -90,3 +90,21 @@ def test_plain_products_of_prompts_take_it(M, N, K):
         assert (ran == ["mv_gemm_round"]) == (pitch % 8 == 0)
         want = x.double() @ w.double().T + b.double()
         assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("lo, hi, limit", [(-60, -40, 0.0), (-40, -8, 0.0), (-8, 8, 0.0), (-8, 8, 7.0)])
+def test_the_activation_is_float32_up_to_the_rounding(lo, hi, limit):
+    """Gates and ups that are exact: what the activation is off shows where a result is not the 16-bit number nearest to the exact one.
+    At 2^-24 x 5 off (a limit's slope * g is rounded in front of the exponential, 2^-24 x 12) 1.5e-4 (3.7e-4) of the results lie
+    close enough to the middle of two, which are at least 2^-8 apart, if all are off that far the wrong way."""
+    from minivllm_amd.kernels.ops import get_ops
+    ops = get_ops(torch.bfloat16)
+    gen, M, I, K = torch.Generator(device=DEV).manual_seed(7), 512, 2048, 64
+    rand = lambda n, a, b: (torch.rand(n, generator=gen, device=DEV) * (b - a) + a).bfloat16()
+    x, w = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV), torch.zeros(2 * I, K, dtype=torch.bfloat16, device=DEV)
+    x[:, 0], x[:, 1], w[:I, 0], w[I:, 1] = rand(M, 0.95, 1.0), rand(M, 1.0, 2.0), rand(I, lo, hi), rand(I, 0.5, 3.0)
+    out = torch.empty(M, I, dtype=torch.bfloat16, device=DEV)
+    ops.lib.call("mv_gemm_pair", x.data_ptr(), K, w.data_ptr(), 0, out.data_ptr(), I, M, 2 * I, K, limit, 1.702 if limit else 1.0, 128 << 16 | 128,
+                 torch.cuda.current_stream().cuda_stream)
+    want = pair(x, w, None, limit, 1.702 if limit else 1.0)
+    assert float((out != want.float().bfloat16()).double().mean()) <= (3.7e-4 if limit else 1.5e-4)
