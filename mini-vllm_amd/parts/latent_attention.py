@@ -174,9 +174,16 @@ class LatentAttention(Mixer):
         return super().chooses_by() + (self.heads_operands is not None,)       # (how this layer's maps are stored)
 
     def reserve(self, tokens: int, seqs: int) -> None:
-        most = self.rt.ops.latent_heads_most(self.spec.num_heads, tokens, seqs, self.rt.max_positions) if self.heads_operands is not None else 0
+        if self.heads_operands is None:
+            return
+        most = self.rt.ops.latent_heads_most(self.spec.num_heads, tokens, seqs, self.rt.max_positions)
         if most:
             self._heads_scratch(most)
+        self._latent_scratch(tokens)             # (a step may stay in the latent's space where a larger one does not)
+
+    def _latent_scratch(self, n: int):
+        ws, H, R = self.rt.workspace, self.spec.num_heads, self.spec.kv_rank
+        return ws.get("latent.qa", (n, H, R + self.spec.rot_dim), torch.float32), ws.get("latent.mixed", (n, H, R), torch.float32)
 
     def _heads_scratch(self, blocks: int):
         ws, H = self.rt.workspace, self.spec.num_heads
@@ -211,10 +218,9 @@ class LatentAttention(Mixer):
                                        self.sink, gate, spec.head_gate)
             y = ws.get("mixer.out", (n, spec.hidden_size), rt.dtype)
             return ops.gemm(heads, self.w_o, y, defer_sum=True) or y
-        qa = ws.get("latent.qa", (n, H, R + dr), torch.float32)
+        qa, mixed = self._latent_scratch(n)
         ops.head_linear(q.unflatten(1, (H, spec.plain_dim + dr)), self.w_uk, qa, ctx.token_seq, tail=dr, table=self.table,
                         positions=ctx.positions, w_rows=self.w_uk_rows)
-        mixed = ws.get("latent.mixed", (n, H, R), torch.float32)
         ops.attention_latent(qa, mixed, pages, kv.block_table, kv.page_size, ctx.positions, ctx.token_seq, H, R, dr,
                              spec.scale, plan=ctx.attention_plan, pages_t=pages_t, window=spec.window, sink=self.sink)
         ops.head_linear(mixed, self.w_uv, heads, ctx.token_seq, gate=gate, w_rows=self.w_uv_rows, gate_per_head=spec.head_gate)
