@@ -34,10 +34,10 @@ def step(part, lens, starts):
     return part.rt.ops.latent_expand.called
 
 
-@pytest.mark.parametrize("largest, own", [(([300], [0]), True), (([30] * 10, [0] * 10), True), (([66] + [1] * 60, [0] + [500] * 60), False)])
+@pytest.mark.parametrize("largest, own", [(([300], [0]), True), (([30] * 10, [0] * 10), True), (([66] + [1] * 234, [0] + [500] * 234), False)])
 def test_scratch_stands_at_the_start(largest, own):
     part = layer()
-    part.reserve(300, 64)
+    part.reserve(300, 256)
     assert step(part, *largest) is own
     part.rt.workspace.frozen = True                  # (a buffer that would have to grow raises)
     ways = {step(part, *cut) for cut in [([64], [0]), ([1] * 60, [500] * 60), ([200], [300]), ([66] + [1] * 60, [0] + [500] * 60), ([4] * 60, [508] * 60)]}
