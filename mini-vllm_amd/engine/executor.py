@@ -278,6 +278,7 @@ class Executor:
             table = list(range(s * pages_per_seq, (s + 1) * pages_per_seq))
             seqs.append(SeqStep(tokens=[0] * per_seq, start=0, block_tables=[table] * len(self.groups),
                                 state_slot=s % self.num_state_slots, want=[per_seq - 1]))
+        self.ops.reserve_library(self.device)
         self.model.reserve(num_tokens, self.config.max_num_batched_seqs)
         self.step(seqs)
         if self.config.use_cuda_graph and self.model.graph_safe:

@@ -2570,10 +2570,7 @@ class Ops:
                 self._library_product(a[M - rest:], w, bias, out[M - rest:], True)
         if self.lib.has("mv_gemm_lt") and a.stride(1) == 1 and out.stride(1) == 1 and a.data_ptr() % 16 == 0 \
                 and out.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
-            if self._lt_work is None:
-                if torch.cuda.is_current_stream_capturing():
-                    raise KernelLibraryError("the library's workspace must be made before a capture")
-                self._lt_work = torch.empty(int(self.lib.dll.mv_gemm_lt_workspace()), dtype=torch.uint8, device=a.device)
+            self.reserve_library(a.device)
             self._note("mv_gemm_lt", self._size(a, w, out), 2 * M * N * K)
             return self.lib.offer("mv_gemm_lt", a.data_ptr(), a.stride(0) if M > 1 else K, w.data_ptr(), _ptr(bias),
                                   out.data_ptr(), out.stride(0) if M > 1 else N, _CODES[out.dtype], M, N, K,
@@ -2588,6 +2585,14 @@ class Ops:
         else:
             torch.addmm(bias, a, wt, out=out)
         return True
+
+    def reserve_library(self, device: torch.device) -> None:
+        """The workspace that library products share, made once. An engine asks for it before it sizes its cache: the step that it
+        sizes its scratch by may hold no such product."""
+        if self._lt_work is None and self.use_library_gemm and self.lib.has("mv_gemm_lt"):
+            if torch.cuda.is_current_stream_capturing():
+                raise KernelLibraryError("the library's workspace must be made before a capture")
+            self._lt_work = torch.empty(int(self.lib.dll.mv_gemm_lt_workspace()), dtype=torch.uint8, device=device)
 
     def _gemm_round(self, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor) -> bool:
         """A plain product whose tiles are one round of the compute units (gemm_pair.hip, whose ``mv_gemm_round_shape`` says for which

@@ -45,3 +45,25 @@ def test_the_rule_for_one_pass_is_not_monotone():
     shape = ctypes.CDLL(build.find_library("bf16") or build.build("bf16")).mv_gemm_pair_shape
     assert shape(1024, 256, 128, 256) and not shape(128, 256, 128, 256)
     assert shape(2048, 12288, 2048, 256) and not shape(1792, 12288, 2048, 256)
+
+
+def test_the_librarys_workspace_is_there_before_the_dry_run():
+    """The dry run's own products may all be the engine's; a smaller step's need not be."""
+    from unittest.mock import MagicMock, patch
+    from minivllm_amd.engine.executor import Executor
+    from minivllm_amd.kernels.ops import Ops
+    engine = MagicMock(page_size=16, num_state_slots=4, groups=[None],
+                       config=SimpleNamespace(max_num_batched_seqs=4, max_model_len=64, use_cuda_graph=False))
+    ops = SimpleNamespace(_lt_work=None, use_library_gemm=True,
+                          lib=SimpleNamespace(has=lambda name: True, dll=SimpleNamespace(mv_gemm_lt_workspace=lambda: 1 << 20)))
+    engine.ops.reserve_library = lambda device: Ops.reserve_library(ops, torch.device("cpu"))
+    engine.step = lambda seqs: seen.append(ops._lt_work)
+    seen = []
+    with patch("torch.cuda.synchronize"), patch("torch.cuda.empty_cache"), patch("torch.cuda.is_current_stream_capturing", return_value=False):
+        Executor._warmup(engine, 64)
+        assert len(seen) == 1 and seen[0].numel() == 1 << 20
+        Ops.reserve_library(ops, torch.device("cpu"))
+        assert ops._lt_work is seen[0]
+        ops.use_library_gemm, ops._lt_work = False, None             # (the float32 engine has no such product)
+        Ops.reserve_library(ops, torch.device("cpu"))
+        assert ops._lt_work is None
