@@ -109,7 +109,8 @@ DECODE_ATTENTION_WAVES = 4
 # (sequence, kv head) pairs of one decode step whose keys may be split over workgroups
 # steps of up to so many rows carry queries into a latent's space, and sums out of it, in float32
 HEAD_LINEAR_FLOAT_ROWS = 64
-# (block of 32 keys, head) pairs whose keys and values a latent attention may make at a time: 16 KiB each, 512 MiB of scratch
+# (block of 32 keys, head) pairs whose keys and values a latent attention may make at a time: 16 KiB each, 512 MiB of scratch at most, in
+# the engine's workspace and once more in that of its recordings
 LATENT_HEADS_MOST = 1 << 15
 SPLIT_COUNTERS = 1 << 16
 # from this many tokens on, value rows are written to their pages 16 tokens of a kv head at a time
@@ -1576,9 +1577,17 @@ class Ops:
         return room if own < latent else 0
 
     def latent_heads_most(self, heads: int, tokens: int, seqs: int, positions: int) -> int:
-        """The most that ``latent_heads`` says for any step of up to ``tokens`` tokens of ``seqs`` requests of up to ``positions`` positions."""
-        blocks = seqs * -(-positions // 32)
-        return min(LATENT_HEADS_MOST // heads, blocks + max(4, blocks // 4)) if tokens > 1 else 0
+        """The most that ``latent_heads`` says for any step of up to ``tokens`` tokens of ``seqs`` requests of up to ``positions`` positions:
+        scratch is made for so many. Where the latent's space takes less anyhow follows from the two sides of that rule,
+        with each side of its maxima and the most that the sums can be."""
+        if tokens <= HEAD_LINEAR_FLOAT_ROWS:
+            return 0
+        longest, rows, units = -(-positions // 32), -(-heads // 16), self.compute_units
+        maps, carried = 0.26e-3 * heads * 32, 1.6e-3 * heads * tokens
+        walks = (9.0 * rows * (tokens + 7 * seqs) / 8 + (0.2 * rows - heads / 160) * tokens * longest) / units
+        worth = max((12.0 + carried + 0.8 * longest) / maps, (3.0 + carried + walks) / max(maps - 1.4 * rows / units, 1e-9))
+        blocks = int(min(seqs * longest, worth))
+        return min(LATENT_HEADS_MOST // heads, blocks + max(4, blocks // 4))
 
     def latent_expand(self, pages: torch.Tensor, block_table: torch.Tensor, page_size: int, plan, context_lens: torch.Tensor, w_k: torch.Tensor,
                       w_v: torch.Tensor, heads: int, kv_rank: int, rot_dim: int, blocks: int, k: torch.Tensor, kr: torch.Tensor,

@@ -94,3 +94,36 @@ def test_maps_without_a_rotary_part_stay_in_the_latents_space():
         part = LatentAttention(spec, {name: torch.zeros(decl.shape, dtype=torch.bfloat16) for name, decl in LatentAttention.tensors(spec).items()},
                                SimpleNamespace(dtype=torch.bfloat16, ops=ops), SimpleNamespace(rotary=lambda: (torch.zeros(1, 64), False)))
         assert (part.heads_operands is not None) is (rot_dim > 0)
+
+
+def mixed_load(rng, steps, positions):
+    """Steps of one to three prompt portions beside up to fifteen requests that decode."""
+    for _ in range(steps):
+        lens, starts = [1] * rng.randint(0, 15), []
+        starts += [rng.randint(20, positions - 1) for _ in lens]
+        for _ in range(rng.randint(1, 3)):
+            lens.append(rng.randint(20, 500))
+            starts.append(rng.choice([0, rng.randint(0, positions - 500)]))
+        yield lens, starts
+
+
+@pytest.mark.parametrize("heads, units", [(1, 256), (3, 64), (16, 256), (16, 304), (20, 128), (64, 256), (128, 256)])
+def test_the_room_reserved_holds_every_step(heads, units):
+    import random
+    rng, ops, own = random.Random(heads), SimpleNamespace(compute_units=units), 0
+    cuts = list(mixed_load(rng, 400, 1900)) + list(mixed_load(rng, 200, 4000))
+    for _ in range(600):                                 # portions of any length at any place, none of them decoded tokens
+        n = int(2 ** rng.uniform(0, 5))
+        cuts.append(([int(2 ** rng.uniform(1, 9)) for _ in range(n)], [rng.choice([0, rng.randint(0, 3000)]) for _ in range(n)]))
+    for lens, starts in cuts:
+        room = Ops.latent_heads(ops, heads, lens, starts)
+        own += room > 0
+        assert room <= Ops.latent_heads_most(ops, heads, sum(lens), len(lens), max(map(sum, zip(lens, starts))))
+    assert own > 100
+
+
+def test_no_room_is_reserved_that_no_step_can_take():
+    ops = SimpleNamespace(compute_units=256)
+    assert Ops.latent_heads_most(ops, 16, 64, 256, 4096) == 0
+    # 256 requests of 4,096 positions have 32,768 blocks; beside 512 tokens the latent's space is ahead from 1,000 on
+    assert 800 <= Ops.latent_heads_most(ops, 16, 512, 256, 4096) <= 1250
