@@ -82,7 +82,10 @@ __device__ __forceinline__ AlhPlace alh_find(int at, int n_seqs, Of of_request, 
 
 // A workgroup makes one head's keys and values of two neighbouring blocks (64 keys). The latents come from the pages a quarter a
 // wave, into LDS in operand order; each wave takes 32 of the 128 channels of K and of V, its weights straight from memory (in
-// operand order too: [head][tile of 16 channels][32 inputs][lane]).
+// operand order too: [head][tile of 16 channels][32 inputs][lane]). `blocks` of a recording is what its size class may hold, up to
+// some ten times what a step does: workgroups walk over the pairs of blocks, twice as many of them as stand on the chip at once, and end
+// at the first pair that holds nothing (16 heads, 2,048 tokens, room for 1,000 blocks more: 14.7 us, 12.1 without them; with a workgroup for
+// every pair 34.8 and 11.2).
 template <int RS, int DRS>                                     // k-steps of the latent and of the rotary part
 __global__ void __launch_bounds__(ALH_THREADS)
 latent_expand_kernel(const bf16* __restrict__ pages, const int* __restrict__ block_table, int bt_width, int page_size,
@@ -93,89 +96,94 @@ latent_expand_kernel(const bf16* __restrict__ pages, const int* __restrict__ blo
     __shared__ uint4 lat[4 * RS * 64];                         // [16 keys][k-step][lane]
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / MV_WAVE), lane = tid % MV_WAVE;
     const int r = lane % 16, g = lane / 16, head = blockIdx.x;
-    // this wave's sixteen keys: half `wave % 2` of block `wave / 2`
-    int limit[2];                                              // keys of the two blocks that there are
-    bool any = false;
+    for (int pair = blockIdx.y; 2 * pair < blocks; pair += gridDim.y) {
+        // this wave's sixteen keys: half `wave % 2` of block `wave / 2`
+        int limit[2];                                          // keys of the two blocks that there are
+        bool any = false;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const int block = 2 * blockIdx.y + b;
-        limit[b] = -1;
-        if (block < blocks) {
-            const auto of = [&](int s) { return alh_blocks(cu_seqlens[s + 1] - cu_seqlens[s], context_lens[s]); };
-            const AlhPlace at = alh_find(block, n_seqs, of, [](int) { return 0; });
-            if (at.seq >= 0) {
-                const int left = context_lens[at.seq] - ALH_KEYS * at.in;
-                limit[b] = left < ALH_KEYS ? left : ALH_KEYS;
-                any = true;
-                if (wave / 2 == b) {
-                    const int key = 16 * (wave % 2) + r, have = key < limit[b] ? key : limit[b] - 1;
-                    const int pos = ALH_KEYS * at.in + have, entry = pos / page_size;
-                    const bf16* row = pages + ((size_t)block_table[(size_t)at.seq * bt_width + entry] * page_size + (pos - entry * page_size)) * DK + 8 * g;
-                    const bool on = key < limit[b];
-                    AlhFrag c[RS];
+        for (int b = 0; b < 2; ++b) {
+            const int block = 2 * pair + b;
+            limit[b] = -1;
+            if (block < blocks) {
+                const auto of = [&](int s) { return alh_blocks(cu_seqlens[s + 1] - cu_seqlens[s], context_lens[s]); };
+                const AlhPlace at = alh_find(block, n_seqs, of, [](int) { return 0; });
+                if (at.seq >= 0) {
+                    const int left = context_lens[at.seq] - ALH_KEYS * at.in;
+                    limit[b] = left < ALH_KEYS ? left : ALH_KEYS;
+                    any = true;
+                    if (wave / 2 == b) {
+                        const int key = 16 * (wave % 2) + r, have = key < limit[b] ? key : limit[b] - 1;
+                        const int pos = ALH_KEYS * at.in + have, entry = pos / page_size;
+                        const bf16* row = pages + ((size_t)block_table[(size_t)at.seq * bt_width + entry] * page_size + (pos - entry * page_size)) * DK + 8 * g;
+                        const bool on = key < limit[b];
+                        AlhFrag c[RS];
 #pragma unroll
-                    for (int s = 0; s < RS; ++s) c[s].u = *reinterpret_cast<const uint4*>(row + 32 * s);
-                    if (head == 0) {
-                        const int t = (key / 4) % 2, rho = 4 * (key / 8) + key % 4;
+                        for (int s = 0; s < RS; ++s) c[s].u = *reinterpret_cast<const uint4*>(row + 32 * s);
+                        if (head == 0) {
+                            const int t = (key / 4) % 2, rho = 4 * (key / 8) + key % 4;
 #pragma unroll
-                        for (int s = 0; s < DRS; ++s) {
-                            const uint4 x = *reinterpret_cast<const uint4*>(row + R + 32 * s);
-                            kr_out[(((size_t)block * 2 + t) * DRS + s) * 64 + 16 * g + rho] = on ? x : uint4{0u, 0u, 0u, 0u};
+                            for (int s = 0; s < DRS; ++s) {
+                                const uint4 x = *reinterpret_cast<const uint4*>(row + R + 32 * s);
+                                kr_out[(((size_t)block * 2 + t) * DRS + s) * 64 + 16 * g + rho] = on ? x : uint4{0u, 0u, 0u, 0u};
+                            }
                         }
+#pragma unroll
+                        for (int s = 0; s < RS; ++s) lat[(wave * RS + s) * 64 + lane] = on ? c[s].u : uint4{0u, 0u, 0u, 0u};
                     }
+                }
+            }
+            if (limit[b] < 0 && wave / 2 == b)
 #pragma unroll
-                    for (int s = 0; s < RS; ++s) lat[(wave * RS + s) * 64 + lane] = on ? c[s].u : uint4{0u, 0u, 0u, 0u};
+                for (int s = 0; s < RS; ++s) lat[(wave * RS + s) * 64 + lane] = uint4{0u, 0u, 0u, 0u};
+        }
+        if (!any) return;                                      // (the same for every wave; nor are there blocks behind)
+        __syncthreads();
+        int maps = 0;
+        asm volatile("" : "+s"(maps));                         // (the maps are read again for every pair: kept, a wave has the unit to itself)
+#pragma unroll
+        for (int which = 0; which < 2; ++which) {
+            const uint4* w = (which == 0 ? w_k : w_v) + maps + ((size_t)head * 8 + 2 * wave) * RS * 64 + lane;
+            AlhFrag fw[2][RS];
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int s = 0; s < RS; ++s) fw[dt][s].u = w[(dt * RS + s) * 64];
+            floatx4_t acc[4][2];
+#pragma unroll
+            for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) acc[ct][dt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+                for (int s = 0; s < RS; ++s) {
+                    AlhFrag fc;
+                    fc.u = lat[(ct * RS + s) * 64 + lane];
+#pragma unroll
+                    for (int dt = 0; dt < 2; ++dt)
+                        acc[ct][dt] = which == 0 ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[dt][s].v, fc.v, acc[ct][dt], 0, 0, 0)
+                                                 : __builtin_amdgcn_mfma_f32_16x16x32_bf16(fc.v, fw[dt][s].v, acc[ct][dt], 0, 0, 0);
+                }
+#pragma unroll
+            for (int ct = 0; ct < 4; ++ct) {
+                if (limit[ct / 2] < 0) continue;
+                const size_t tile = ((size_t)(2 * pair + ct / 2) * H + head) * ALH_TILE;
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) {
+                    const int d16 = 2 * wave + dt;                 // which sixteen channels
+                    uint2 bits{f32x2_to_bf16x2_bits(acc[ct][dt][0], acc[ct][dt][1]), f32x2_to_bf16x2_bits(acc[ct][dt][2], acc[ct][dt][3])};
+                    uint2* to;
+                    if (which == 0) {                              // four channels 16 d16 + 4 g.. of key r
+                        const int key = 16 * (ct % 2) + r, t = (key / 4) % 2, rho = 4 * (key / 8) + key % 4;
+                        to = reinterpret_cast<uint2*>(k_out + tile + (t * 4 + d16 / 2) * 64 + 16 * (2 * (d16 % 2) + g / 2) + rho) + g % 2;
+                    } else {                                       // four keys 4 g.. of channel r
+                        to = reinterpret_cast<uint2*>(v_out + tile + d16 * 64 + 16 * (2 * (ct % 2) + g / 2) + r) + g % 2;
+                    }
+                    *to = bits;
                 }
             }
         }
-        if (limit[b] < 0 && wave / 2 == b)
-#pragma unroll
-            for (int s = 0; s < RS; ++s) lat[(wave * RS + s) * 64 + lane] = uint4{0u, 0u, 0u, 0u};
-    }
-    if (!any) return;                                          // (the same for every wave)
-    __syncthreads();
-#pragma unroll
-    for (int which = 0; which < 2; ++which) {
-        const uint4* w = (which == 0 ? w_k : w_v) + ((size_t)head * 8 + 2 * wave) * RS * 64 + lane;
-        AlhFrag fw[2][RS];
-#pragma unroll
-        for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-            for (int s = 0; s < RS; ++s) fw[dt][s].u = w[(dt * RS + s) * 64];
-        floatx4_t acc[4][2];
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-            for (int dt = 0; dt < 2; ++dt) acc[ct][dt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-            for (int s = 0; s < RS; ++s) {
-                AlhFrag fc;
-                fc.u = lat[(ct * RS + s) * 64 + lane];
-#pragma unroll
-                for (int dt = 0; dt < 2; ++dt)
-                    acc[ct][dt] = which == 0 ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[dt][s].v, fc.v, acc[ct][dt], 0, 0, 0)
-                                             : __builtin_amdgcn_mfma_f32_16x16x32_bf16(fc.v, fw[dt][s].v, acc[ct][dt], 0, 0, 0);
-            }
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct) {
-            if (limit[ct / 2] < 0) continue;
-            const size_t tile = ((size_t)(2 * blockIdx.y + ct / 2) * H + head) * ALH_TILE;
-#pragma unroll
-            for (int dt = 0; dt < 2; ++dt) {
-                const int d16 = 2 * wave + dt;                 // which sixteen channels
-                uint2 bits{f32x2_to_bf16x2_bits(acc[ct][dt][0], acc[ct][dt][1]), f32x2_to_bf16x2_bits(acc[ct][dt][2], acc[ct][dt][3])};
-                uint2* to;
-                if (which == 0) {                              // four channels 16 d16 + 4 g.. of key r
-                    const int key = 16 * (ct % 2) + r, t = (key / 4) % 2, rho = 4 * (key / 8) + key % 4;
-                    to = reinterpret_cast<uint2*>(k_out + tile + (t * 4 + d16 / 2) * 64 + 16 * (2 * (d16 % 2) + g / 2) + rho) + g % 2;
-                } else {                                       // four keys 4 g.. of channel r
-                    to = reinterpret_cast<uint2*>(v_out + tile + d16 * 64 + 16 * (2 * (ct % 2) + g / 2) + r) + g % 2;
-                }
-                *to = bits;
-            }
-        }
+        __syncthreads();                                       // (the latents have been read)
     }
 }
 
@@ -434,7 +442,8 @@ extern "C" int mv_latent_expand(const void* pages, const int* block_table, int b
                    && ((uintptr_t)pages | (uintptr_t)w_k | (uintptr_t)w_v | (uintptr_t)k | (uintptr_t)kr | (uintptr_t)v) % 16 == 0,
                "latent_expand: missing or unaligned operand");
     if (blocks == 0 || n_seqs == 0) return 0;
-    const dim3 grid(H, (blocks + 1) / 2);
+    const int pairs = (blocks + 1) / 2, at_once = 4 * mv_compute_units() / H + 1;
+    const dim3 grid(H, pairs < at_once ? pairs : at_once);
 #define ALH_EXPAND(RS, DRS)                                                                                                            \
     hipLaunchKernelGGL((latent_expand_kernel<RS, DRS>), grid, dim3(ALH_THREADS), 0, stream, (const bf16*)pages, block_table, bt_width, page_size, \
                        cu_seqlens, context_lens, n_seqs, (const uint4*)w_k, (const uint4*)w_v, H, (uint4*)k, (uint4*)kr, (uint4*)v, blocks)

@@ -1560,7 +1560,7 @@ class Ops:
         Steps of up to HEAD_LINEAR_FLOAT_ROWS tokens stay in the latent's space whatever they take: the weighted sum of latents goes through
         its map in float32 there, where the heads' own values are rounded (one layer of 20 tokens against 64 bits 1.95e-3, with its own
         values 2.54e-3; from 100 to 4,000 tokens, where both round, 2.57e-3 to 3.29e-3 and 2.61e-3 to 3.30e-3).
-        The count is a multiple of 4, of an eighth of it or more, so that steps of similar sizes share a recording."""
+        The count is a multiple of 4, of an eighth of it or more, so that steps of similar sizes share the scratch's views."""
         if not lens or max(lens) < 2 or sum(lens) <= HEAD_LINEAR_FLOAT_ROWS:
             return 0
         q, s = np.asarray(lens), np.asarray(starts)
@@ -1578,7 +1578,7 @@ class Ops:
 
     def latent_heads_most(self, heads: int, tokens: int, seqs: int, positions: int) -> int:
         """The most that ``latent_heads`` says for any step of up to ``tokens`` tokens of ``seqs`` requests of up to ``positions`` positions:
-        scratch is made for so many. Where the latent's space takes less anyhow follows from the two sides of that rule,
+        scratch and recordings are made for so many. Where the latent's space takes less anyhow follows from the two sides of that rule,
         with each side of its maxima and the most that the sums can be."""
         if tokens <= HEAD_LINEAR_FLOAT_ROWS:
             return 0

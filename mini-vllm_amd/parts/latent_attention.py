@@ -163,9 +163,8 @@ class LatentAttention(Mixer):
             self.heads_operands = latent_operands(self.w_uk), latent_operands(self.w_uv_rows)
 
     def step_path(self, lens: Sequence[int], starts: Sequence[int]):
-        blocks = self.rt.ops.latent_heads(self.spec.num_heads, lens, starts) if self.heads_operands is not None else 0
-        if blocks:
-            return "heads", blocks
+        if self.heads_operands is not None and self.rt.ops.latent_heads(self.spec.num_heads, lens, starts):
+            return "heads"
         if not self.rt.ops.latent_shares_serve(self.spec.kv_rank, self.spec.rot_dim):
             return None
         return self.rt.ops.latent_shares(self.spec.num_heads, -1 if self.spec.window is None else self.spec.window, lens, starts)
@@ -211,6 +210,8 @@ class LatentAttention(Mixer):
             gate = packed[:, self.gate_offset:self.gate_offset + (H if spec.head_gate else H * spec.value_dim)]
         plan = ctx.attention_plan
         blocks = ops.latent_heads(H, *plan.cut()) if self.heads_operands is not None and not plan.decode_only else 0
+        if blocks and plan.bound is not None:            # (a recording serves every step of its class that chooses so)
+            blocks = ops.latent_heads_most(H, *plan.bound, plan.max_context_len)
         if blocks and q.data_ptr() % 16 == 0 and q.stride(0) % 8 == 0:
             k, kr, v = self._heads_scratch(blocks)
             ops.latent_expand(pages, kv.block_table, kv.page_size, plan, ctx.context_lens, *self.heads_operands, H, R, dr, blocks, k, kr, v)

@@ -169,3 +169,89 @@ def test_no_further_from_64_bits_than_the_latents_space(n, start, spread):
     ops.head_linear(mixed, w_v.transpose(1, 2).contiguous(), latent, seq, w_rows=w_v)
     off = [float((o.double().cpu() - want.flatten(1)).norm() / want.norm()) for o in (own, latent)]
     assert off[0] <= off[1], off
+
+
+@pytest.mark.parametrize("R, dr, H, lens, starts, surplus", [
+    (256, 64, 2, [70, 1], [0, 40], 1),                     # an odd number of blocks
+    (256, 64, 2, [70, 1], [0, 40], 3000),                  # grid shorter than the room
+    (128, 64, 64, [66, 3, 1], [2400, 31, 700], 0),         # three and more turns of a workgroup
+    (256, 0, 64, [66, 3, 1], [2400, 31, 700], 500)])
+def test_keys_and_values_are_made_whatever_the_room(R, dr, H, lens, starts, surplus):
+    """Every block that there is, its sums as float32 has them, and nothing behind the last: workgroups walk over the blocks."""
+    from minivllm_amd.engine.step import AttentionPlan
+    from minivllm_amd.kernels.ops import Ops, latent_operands
+    ops, gen, ps = Ops(torch.bfloat16), torch.Generator().manual_seed(1), 16
+    rand = lambda *shape: torch.randn(*shape, generator=gen)
+    context = [q + s for q, s in zip(lens, starts)]
+    pages_of = [-(-c // ps) for c in context]
+    pages = rand(sum(pages_of), ps, R + dr).bfloat16().to(DEV)
+    table, at = torch.zeros(len(lens), max(pages_of), dtype=torch.int32), 0
+    for i, p in enumerate(pages_of):
+        table[i, :p] = torch.arange(at, at + p)
+        at += p
+    w_k, w_v = ((rand(H, 128, R) / math.sqrt(R)).bfloat16().to(DEV) for _ in range(2))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    plan = AttentionPlan(decode_only=False, max_q_len=max(lens), max_context_len=max(context), n_seqs=len(lens), q_lens=lens, starts=starts,
+                         cu_seqlens=i32([0] + torch.tensor(lens).cumsum(0).tolist()))
+    per = [-(-c // 32) for c in context]
+    real, blocks = sum(per), sum(per) + surplus
+    mark = lambda *shape: torch.full(shape, 7.0, dtype=torch.bfloat16, device=DEV)
+    k, v, kr = mark(blocks, H, 4096), mark(blocks, H, 4096), mark(blocks, 32 * max(dr, 1))
+    ops.latent_expand(pages, table.to(DEV), ps, plan, i32(context), latent_operands(w_k), latent_operands(w_v), H, R, dr, blocks, k, kr, v)
+    slot = torch.arange(32)                                # (of a key in its block: tile, and place in the tile)
+    tile, rho = slot // 4 % 2, 4 * (slot // 8) + slot % 4
+    for i, c in enumerate(context):
+        lat = torch.zeros(32 * per[i], R + dr, dtype=torch.bfloat16, device=DEV)
+        lat[:c] = pages[table[i, :pages_of[i]].to(DEV).long()].reshape(-1, R + dr)[:c]
+        first = sum(per[:i])
+        # k [block, head, tile, 4 steps, 4 groups, 16 keys, 8]; v [block, head, 8 tiles, 4 groups of 8 keys, 16 channels, 8 keys]
+        got_k = k[first:first + per[i]].view(-1, H, 2, 4, 4, 16, 8)[:, :, tile, :, :, rho]          # [32, block, head, step, group, 8]
+        got_k = got_k.permute(1, 0, 2, 3, 4, 5).reshape(-1, H, 128)
+        got_v = v[first:first + per[i]].view(-1, H, 8, 4, 16, 8).permute(0, 3, 5, 1, 2, 4).reshape(-1, H, 128)
+        for got, w in ((got_k, w_k), (got_v, w_v)):
+            want = (lat[:, :R].double().cpu() @ w.double().cpu().reshape(H * 128, R).T).view(-1, H, 128).to(DEV)
+            assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all())
+        if dr:
+            got = kr[first:first + per[i]].view(-1, 2, dr // 32, 4, 16, 8)[:, tile, :, :, rho].permute(1, 0, 2, 3, 4).reshape(-1, dr)
+            assert torch.equal(got, lat[:, R:])
+    assert bool((k[real:] == 7).all()) and bool((v[real:] == 7).all()) and bool((kr[real:] == 7).all())
+
+
+def test_one_recording_serves_the_contexts_of_its_class():
+    """Recorded with few keys and replayed with many, and the other way: the bits of the eager step, whose rooms follow its own keys."""
+    from minivllm_amd.config import EngineConfig
+    from minivllm_amd.engine.executor import Executor
+    from minivllm_amd.engine.step import SeqStep
+    from minivllm_amd.models import config_from_dict, expected_tensors
+    from minivllm_amd.weights.device_random import DeviceRandomSource
+    latent = {"heads": 2, "dim": 128, "rot_dim": 64, "vdim": 128, "q_rank": 64, "kv_rank": 128, "scale": 0.07, "rot": {"dims": 64, "base": 1e4}}
+
+    def executor(graphs):
+        arch, cfg = config_from_dict({"architecture": "Dutilix", "vocab": 256, "width": 128, "norm": {"eps": 1e-5}, "torch_dtype": "bfloat16",
+                                      "logit_scale": 1.0, "layers": [{"type": "latent_attention", "mixer": latent,
+                                                                      "mlp": {"kind": "dense", "ff": 128}}] * 2})
+        source = DeviceRandomSource(expected_tensors(arch, cfg), 1, torch.bfloat16, torch.device(DEV), std=0.08)
+        return Executor(EngineConfig(model="", dtype="bfloat16", max_model_len=1024, max_num_batched_tokens=1024, max_num_batched_seqs=16,
+                                     kv_cache_block_size=16, kv_cache_num_blocks=256, use_cuda_graph=graphs), model=(arch, cfg, source))
+    recorded, eager = executor(True), executor(False)
+    gen = torch.Generator().manual_seed(3)
+    text = [torch.randint(0, 256, (1024,), generator=gen).tolist() for _ in range(2)]
+    tables = [list(range(64 * s, 64 * s + 64)) for s in range(2)]
+
+    def both(cut):
+        made = [SeqStep(tokens=text[s][start:start + q], start=start, block_tables=[tables[s]], state_slot=s, want=[q - 1]) for s, q, start in cut]
+        return recorded.step(made).clone(), eager.step(made).clone()
+    for s in range(2):                                     # contexts that later steps follow, and rewrite with the same numbers
+        for start in range(0, 1024, 512):
+            both([(s, 512, start)])
+    before = len(recorded._mixed_graphs)
+    for order in (1, -1):
+        for cut in [[(0, 100, 0)], [(0, 98, 31)], [(0, 112, 300)], [(0, 97, 927)], [(0, 112, 912)]][::order]:
+            got, plain = both(cut)
+            assert torch.equal(got, plain), cut
+    assert len(recorded._mixed_graphs) == before + 1
+    for cut in [[(0, 60, 0), (1, 45, 3)], [(0, 60, 900), (1, 45, 970)], [(0, 111, 913), (1, 1, 1023)]]:
+        got, plain = both(cut)
+        assert torch.equal(got, plain), cut
+    assert len(recorded._mixed_graphs) == before + 2
+    assert all("mv_attention_latent_heads" in {e[0] for e in ledger} for key, ledger in recorded.graph_ledger.items() if key[1] == 112)

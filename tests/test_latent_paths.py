@@ -107,6 +107,28 @@ def mixed_load(rng, steps, positions):
         yield lens, starts
 
 
+def size_class(lens, starts):
+    """Tokens, sequences and context that a recording of such a step is made for."""
+    from minivllm_amd.engine.executor import GRAPH_BUCKETS, TOKEN_BUCKETS
+    cap = max(1024, 1 << (max(map(sum, zip(lens, starts))) - 1).bit_length())
+    return next(b for b in TOKEN_BUCKETS if b >= sum(lens)), next(b for b in GRAPH_BUCKETS if b >= len(lens)), cap
+
+
+def test_a_growing_context_needs_no_recording_of_its_own():
+    """Of a size class there is one recording for each of the three ways, whatever the keys that its steps' contexts hold."""
+    import random
+    import torch
+    from minivllm_amd.parts.latent_attention import LatentAttention
+    ops = SimpleNamespace(compute_units=256, latent_shares_serve=lambda *sizes: True)
+    ops.latent_heads, ops.latent_shares = lambda *a: Ops.latent_heads(ops, *a), lambda *a: Ops.latent_shares(ops, *a)
+    part = SimpleNamespace(rt=SimpleNamespace(ops=ops), heads_operands=(), spec=SimpleNamespace(num_heads=16, window=None, kv_rank=256, rot_dim=64))
+    keys = {}
+    for lens, starts in mixed_load(random.Random(1), 1500, 1900):
+        keys.setdefault(size_class(lens, starts), set()).add(LatentAttention.step_path(part, lens, starts))
+    assert len(keys) > 50 and max(map(len, keys.values())) <= 3
+    assert sum(map(len, keys.values())) <= 1.5 * len(keys)
+
+
 @pytest.mark.parametrize("heads, units", [(1, 256), (3, 64), (16, 256), (16, 304), (20, 128), (64, 256), (128, 256)])
 def test_the_room_reserved_holds_every_step(heads, units):
     import random
@@ -119,6 +141,8 @@ def test_the_room_reserved_holds_every_step(heads, units):
         room = Ops.latent_heads(ops, heads, lens, starts)
         own += room > 0
         assert room <= Ops.latent_heads_most(ops, heads, sum(lens), len(lens), max(map(sum, zip(lens, starts))))
+        if sum(lens) <= 2048:
+            assert room <= Ops.latent_heads_most(ops, heads, *size_class(lens, starts))
     assert own > 100
 
 
