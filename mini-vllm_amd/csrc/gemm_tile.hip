@@ -403,6 +403,7 @@ static int tile_launch(const void* A, long lda, const void* W, const void* bias,
     MV_REQUIRE(((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0, "gemm_tile: operands must be 16-byte aligned");
     MV_REQUIRE(c_dtype == MV_F32 || c_dtype == MV_BF16, "gemm_tile: bad output dtype %d", c_dtype);
     MV_REQUIRE(!gated || N % 2 == 0, "gemm_tile: the gated form takes an even N");
+    MV_REQUIRE(!square_relu || !gated, "gemm_tile: the squared ReLU needs no gated pair");
     MV_REQUIRE(ldc >= (gated ? N / 2 : N), "gemm_tile: ldc=%ld too small for N=%d", ldc, N);
     MV_REQUIRE((long)M * N < (1L << 31), "gemm_tile: %d x %d outputs exceed the index range", M, N);
     const TilePlan p = tile_plan(M, gated ? N / 2 : N, K, gated != 0, force);
@@ -419,7 +420,7 @@ static int tile_launch(const void* A, long lda, const void* W, const void* bias,
                "gemm_tile: the work area holds %ld floats, %ld are needed", work_floats, (long)p.F * M * N);
     MV_REQUIRE(partial == nullptr || (p.F == 1 && P > 0 && eps > 0.f),
                "gemm_tile: rows without their norm's division need an unsplit K (F=%d), their sums (P=%d) and eps", p.F, P);
-    MV_REQUIRE(!square_relu || (p.F == 1 && !gated), "gemm_tile: the squared ReLU needs an unsplit K (F=%d) and no gated pair", p.F);
+    MV_REQUIRE(!square_relu || p.F == 1, "gemm_tile: the squared ReLU needs an unsplit K (F=%d)", p.F);
     TileArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, C, ldc, c_dtype == MV_F32, p.F > 1 ? work : nullptr,
                M, N, K, p.F, p.chunks_per_split, p.tiles_m, p.tiles_n, gated ? N / 2 : 0, partial, P, eps, pair,
                square_relu};

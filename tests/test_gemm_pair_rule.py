@@ -60,3 +60,14 @@ def test_a_class_has_one_plain_product(lib, n, k, classes):
     for rows in range(129, classes[-1] + 1):
         padded = next(b for b in classes if b >= rows)
         assert bool(shape(rows, n, k, 256)) == bool(shape(padded, n, k, 256)), (rows, padded)
+
+
+@pytest.mark.parametrize("M, N, K", [(1024, 6144, 1024), (64, 6144, 1024)])
+def test_a_pair_with_a_squared_relu_stays_refused(lib, M, N, K):
+    """Whichever kernel would take the pair: none of them squares it. (Refused in front of any launch: the addresses are made up.)"""
+    lib.mv_last_error.restype = ctypes.c_char_p
+    p, i, n, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_long, ctypes.c_float
+    lib.mv_gemm_tile.argtypes = [p, n, p, p, p, n, i, i, i, i, i, p, n, i, f, f, i, p]
+    address, bf16 = 1 << 20, 1
+    assert lib.mv_gemm_tile(address, K, address, None, address, N // 2, bf16, M, N, K, 1, None, 0, 0, 0.0, 1.0, 1, None)
+    assert b"squared ReLU" in lib.mv_last_error()
