@@ -30,7 +30,7 @@ struct PairArgs {
     bf16* C;
     long ldc;
     int M, I, K;                       // plain: I = N
-    int tiles_m, tiles, wide_stores;
+    int tiles, fast, by_columns, wide_stores;    // fast: tiles of the side that changes fastest
     GatedPair pair;
 };
 
@@ -46,10 +46,11 @@ gemm_pair_kernel(PairArgs a) {
     __shared__ uint4 ring[STAGES * STAGE];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / MV_WAVE), lane = tid % MV_WAVE, i = lane % 16, g = lane / 16;
     const int wm = wave / 2, wn = wave % 2;
-    // an XCD has a run of tiles, the rows changing fastest: a band of the weight goes into one L2
+    // An XCD has a run of tiles. Rows change fastest, so that a band of the weight goes into one L2; with more rows than weight rows
+    // columns do, and it is a band of the rows: else every L2 reads all of the larger operand (5,564 x 736 x 1024 19.6 us, so 15.8).
     const int run = (a.tiles + GT_XCDS - 1) / GT_XCDS, id = blockIdx.x % GT_XCDS * run + blockIdx.x / GT_XCDS;
     if ((int)blockIdx.x / GT_XCDS >= run || id >= a.tiles) return;
-    const int tm = id % a.tiles_m, tn = id / a.tiles_m;
+    const int quick = id % a.fast, slow = id / a.fast, tm = a.by_columns ? slow : quick, tn = a.by_columns ? quick : slow;
     const int m0 = tm * BM, n0 = tn * (GATED ? BN / 2 : BN), n = a.K / GT_KC;
 
     // this lane's share of the loads, and the operands: as in gemm_tile.hip
@@ -225,11 +226,11 @@ extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* 
                "gemm_pair: operands not aligned or pitches too small");
     const int bm = tile >> 16, bn = tile & 0xffff;
     MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 128 || bn == 192), "gemm_pair: no tile of %d x %d", bm, bn);
-    const int tiles_m = (M + bm - 1) / bm;
-    const long tiles = (long)tiles_m * ((N / 2 + bn / 2 - 1) / (bn / 2));
+    const int tiles_m = (M + bm - 1) / bm, tiles_n = (N / 2 + bn / 2 - 1) / (bn / 2), by_columns = M > N;
+    const long tiles = (long)tiles_m * tiles_n;
     MV_REQUIRE(tiles < (1L << 30), "gemm_pair: too many tiles");
-    const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N / 2, K, tiles_m, (int)tiles,
-                     ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{limit, slope}};
+    const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N / 2, K, (int)tiles,
+                     by_columns ? tiles_n : tiles_m, by_columns, ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{limit, slope}};
     const dim3 grid((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
 #define GP_LAUNCH(WM, WN, S) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, S, true>), grid, dim3(512), 0, stream, a)
     if (bn == 192) {
@@ -293,11 +294,11 @@ extern "C" int mv_gemm_round(const void* A, long lda, const void* W, const void*
                "gemm_round: operands not aligned or pitches too small");
     const int bm = tile >> 16, bn = tile & 0xffff;
     MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 96 || bn == 128 || bn == 192), "gemm_round: no tile of %d x %d", bm, bn);
-    const int tiles_m = (M + bm - 1) / bm;
-    const long tiles = (long)tiles_m * ((N + bn - 1) / bn);
+    const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn, by_columns = M > N;
+    const long tiles = (long)tiles_m * tiles_n;
     MV_REQUIRE(tiles < (1L << 30), "gemm_round: too many tiles");
-    const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N, K, tiles_m, (int)tiles,
-                     ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{0.f, 1.f}};
+    const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N, K, (int)tiles,
+                     by_columns ? tiles_n : tiles_m, by_columns, ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{0.f, 1.f}};
     const dim3 grid((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
 #define GR_LAUNCH(WM, WN, S) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, S, false>), grid, dim3(512), 0, stream, a)
     if (bn == 192) {
