@@ -204,8 +204,10 @@ static PairTile pair_tile(int M, int N, int K, int units) {
 }
 
 // rows << 16 | weight rows of the tile that M rows against a pair [N = 2 I, K] have on a device of so many compute units; 0: the pair is left to
-// the other kernels. Over 68 shapes, 129 to 8,192 rows, K of 512 to 4,096, the choice is 1 % behind the best on average, and 2 % behind what
-// ran there before at worst (2,560 x 6144 x 1024); above 6,144 rows the library is ahead again. Weights of 64 MB and
+// the other kernels. Over 68 shapes, 129 to 8,192 rows, K of 512 to 4,096, the choice is 1 % behind the best on average; above 6,144 rows the
+// library is ahead again. Above 1,536 rows a pair may be estimated up to 5 % behind the library with its activation (98 pairs of 1,552 to 6,144
+// rows: 1.0 to 2.1 times as fast) but for N of its tiles, where the estimate is too high for it and has to be 3 % ahead: 4,096 x 4096 x 2048
+// 66.8 us there and 75.6 here, 5,120 x 6144 x 1024 78 and 81, 4,096 x 8192 x 1024 81 and 84; 2,560 x 6144 x 1024 43.4 both. Weights of 64 MB and
 // more are left to it at every number of rows: there a pair is two calls, the product and its activation. Whether the pair comes here is decided by
 // the rows that a recorded step is padded to (the library rounds gate and up in front of the activation), the tile by the rows there
 // are: every tile adds in one order.
@@ -213,7 +215,7 @@ extern "C" int mv_gemm_pair_shape(int M, int N, int K, int units) {
     if (M <= 128 || M > 6144 || N % 2 || K % GT_KC || N <= 0 || K <= 0 || 2.0 * N * K >= 64.0 * 1024 * 1024) return 0;
     const int padded = mv_class_rows(M);
     const PairTile p = pair_tile(padded, N, K, units);
-    if (p.time >= (padded > 1536 ? 1.05 : 1.0) * p.other) return 0;
+    if (p.time >= (padded <= 1536 ? 1.0 : N % 256 ? 1.05 : 0.97) * p.other) return 0;
     return M == padded ? p.tile : pair_tile(M, N, K, units).tile;
 }
 

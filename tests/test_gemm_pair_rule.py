@@ -62,6 +62,12 @@ def test_a_class_has_one_plain_product(lib, n, k, classes):
         assert bool(shape(rows, n, k, 256)) == bool(shape(padded, n, k, 256)), (rows, padded)
 
 
+@pytest.mark.parametrize("rows, n, k, here", [(4096, 4096, 2048, False), (5120, 6144, 1024, False), (4096, 8192, 1024, False), (4096, 6144, 1024, True),
+                                              (2560, 6144, 1024, True), (2048, 8192, 1024, True), (5784, 4896, 768, True), (1655, 10528, 1024, True)])
+def test_a_weight_of_the_librarys_tiles_has_to_be_ahead(shape, rows, n, k, here):
+    assert (shape(rows, n, k, 256) != 0) is here
+
+
 @pytest.mark.parametrize("M, N, K", [(1024, 6144, 1024), (64, 6144, 1024)])
 def test_a_pair_with_a_squared_relu_stays_refused(lib, M, N, K):
     """Whichever kernel would take the pair: none of them squares it. (Refused in front of any launch: the addresses are made up.)"""
