@@ -92,6 +92,20 @@ def test_plain_products_of_prompts_take_it(M, N, K):
         assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
 
 
+@pytest.mark.parametrize("M", [129, 150, 160, 256])
+def test_short_prompts_stay_with_the_deep_product(M):
+    """Pairs of few weight rows that both kernels serve: the bits of the one that the tiled product had them in."""
+    from minivllm_amd.kernels.ops import get_ops
+    ops, N, K = get_ops(torch.bfloat16), 2048, 1024
+    assert ops.lib.dll.mv_gemm_deep_shape(M, N, K, 1) and ops.lib.dll.mv_gemm_pair_shape(M, N, K, 256) and ops.wants_tile(M, N, K, gated=True)
+    x, w = torch.randn(M, K, device=DEV).bfloat16(), (torch.randn(N, K, device=DEV) / K ** 0.5).bfloat16()
+    got, deep = (torch.zeros(M, N // 2, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    assert ops.gemm_swiglu(x, w, got)
+    ops.lib.call("mv_gemm_deep", x.data_ptr(), K, w.data_ptr(), 0, deep.data_ptr(), N // 2, 1, M, N, K, 1, 0, 0, 0.0, 0.0, 1.0, 0, 0,
+                 torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(got, deep)
+
+
 @pytest.mark.parametrize("lo, hi, limit", [(-60, -40, 0.0), (-40, -8, 0.0), (-8, 8, 0.0), (-8, 8, 7.0)])
 def test_the_activation_is_float32_up_to_the_rounding(lo, hi, limit):
     """Gates and ups that are exact: what the activation is off shows where a result is not the 16-bit number nearest to the exact one.
