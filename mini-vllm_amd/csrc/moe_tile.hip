@@ -366,6 +366,15 @@ static int mt_rows(int n, long n_pairs, int n_real, int hidden, int F, int FS, i
     return best;
 }
 
+// The same where the rows of a tile are known. Tiles of up to 64 rows wait for the weights: there a workgroup to itself has less on its way
+// at the ends of a long K, and a second round that few units have costs as much as the first; the smaller tiles share units and end more
+// evenly. us, with 256 columns / 128: 64 experts of 768 x 2048, 8 a token, 8 rows 135 / 118, 64 rows 157 / 143; 128 of 384 x 1024, 33 rows 73 / 66; 16 of
+// 1536 x 4096, 2 a token, 256 rows 150 / 141. One round of short tiles stays wide: 32 of 768 x 1024 beside a shared one, 100 rows 45 / 48.
+static int mt_columns_of(int wm, double row_tiles, int n_out, int halves, int K, int units) {
+    const double wide = row_tiles * ((n_out * halves + 255) / 256);
+    return wm <= 2 && (wide > units || K > 1024) ? 128 : mt_columns(row_tiles, n_out, halves, units);
+}
+
 struct MtShape {
     int wm, in, down;          // rows of a tile in 32s, columns of a tile of the first product and of the second
 };
@@ -374,8 +383,8 @@ static MtShape mt_shape(int n, int top, int n_real, int hidden, int F, int FS, i
     const int wm = mt_rows(n, n_pairs, n_real, hidden, F, FS, units), rows = 32 * wm;
     const double tiles = mt_tiles(n_real, (double)n_pairs / n_real, rows) + (FS ? (n + rows - 1) / rows : 0);
     // (a step of few rows whose tiles leave compute units idle has narrow ones)
-    return MtShape{wm, wm == 1 && busy * ((F + 63) / 64) < units ? 64 : mt_columns(tiles, F > FS ? F : FS, 2, units),
-                   wm == 1 && busy * ((hidden + 127) / 128) < units ? 64 : mt_columns(tiles, hidden, 1, units)};
+    return MtShape{wm, wm == 1 && busy * ((F + 63) / 64) < units ? 64 : mt_columns_of(wm, tiles, F > FS ? F : FS, 2, hidden, units),
+                   wm == 1 && busy * ((hidden + 127) / 128) < units ? 64 : mt_columns_of(wm, tiles, hidden, 1, F, units)};
 }
 // rows | columns << 10 | columns of the second product << 20 of the tiles that mv_moe_pairs has on a device of so many compute units
 extern "C" int mv_moe_pairs_shape(int n, int top, int n_real, int hidden, int F, int FS, int units) {

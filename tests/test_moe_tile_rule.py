@@ -15,3 +15,11 @@ def test_tiles_of_measured_mixtures(n, E, top, hid, F, FS, rows, columns, down):
     lib = kernel_build.find_library("bf16") or kernel_build.build("bf16")
     shape = ctypes.CDLL(lib).mv_moe_pairs_shape(n, top, E, hid, F, FS, 256)
     assert (shape & 1023, shape >> 10 & 1023, shape >> 20) == (rows, columns, down)
+
+
+@pytest.mark.parametrize("n, E, top, hid, F, FS, rows, columns, down", [
+    (8, 64, 8, 2048, 768, 0, 32, 128, 128), (128, 64, 8, 2048, 768, 0, 32, 128, 128), (256, 64, 8, 2048, 768, 0, 64, 128, 128),
+    (33, 128, 8, 1024, 384, 0, 32, 128, 128), (8, 128, 8, 1024, 384, 0, 32, 256, 256), (33, 16, 2, 4096, 1536, 0, 32, 128, 128),
+    (400, 16, 2, 4096, 1536, 0, 64, 128, 128), (600, 16, 2, 4096, 1536, 0, 96, 256, 256)])
+def test_low_tiles_are_wide_in_one_short_round_only(n, E, top, hid, F, FS, rows, columns, down):
+    test_tiles_of_measured_mixtures(n, E, top, hid, F, FS, rows, columns, down)
