@@ -122,7 +122,7 @@ def test_a_recorded_model_follows_the_eager_one():
             made = [SeqStep(tokens=text[s][start:start + q], start=start, block_tables=[tables[s]], state_slot=s, want=[q - 1])
                     for s, (q, start) in enumerate(cut)]
             got, plain = recorded.step(made).clone(), eager.step(made).clone()
-            assert float((got - plain).abs().max() / plain.abs().max()) <= 2e-2, cut
+            assert torch.equal(got, plain), cut                # (both choose by the step and its class, and add in the same orders)
     entries = [{e[0] for e in ledger} for ledger in recorded.graph_ledger.values()]
     assert entries and all("mv_attention_latent_heads" in e and "mv_attention_latent_prompt" not in e for e in entries)
 

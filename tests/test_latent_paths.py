@@ -142,7 +142,8 @@ def test_the_room_reserved_holds_every_step(heads, units):
         own += room > 0
         assert room <= Ops.latent_heads_most(ops, heads, sum(lens), len(lens), max(map(sum, zip(lens, starts))))
         if sum(lens) <= 2048:
-            assert room <= Ops.latent_heads_most(ops, heads, *size_class(lens, starts))
+            of_class = Ops.latent_heads_most(ops, heads, *size_class(lens, starts))
+            assert room <= of_class <= Ops.latent_heads_most(ops, heads, 2048, 64, 4096)           # (what an engine of such steps reserves)
     assert own > 100
 
 
