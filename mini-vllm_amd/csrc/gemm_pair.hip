@@ -7,8 +7,8 @@
 // 0.15 us (the barrier, and waves that wait for the last of them) and 0.385 us for every 128 x 128 of the tile, 1.39 PFLOP/s, half of it
 // the matrix unit, the rest LDS and issue; and a workgroup takes 3.5 us to its first products and from its last. So tiles are large, and
 // which of the twelve shapes depends on how many whole rounds of compute units they make (mv_gemm_pair_shape): 2,048 x 6144 x 1024
-// is one of 256 x 192. There 36.7 us with the library's product and the activation behind it, 27.7 here; 1,536 rows 34.8 (gemm_tile.hip)
-// and 22.5; 1,024 23.4 and 17.6; 512 17.4 and 13.3; 1,024 x 12288 x 2048 71 and 47; 4,096 x 6144 x 1024 69 and 55. Large products of a long K
+// is one of 256 x 192. There 36.4 us with the library's product and the activation behind it, 27.5 here; 1,536 rows 34.7 (gemm_tile.hip)
+// and 22.4; 1,024 23.5 and 17.8; 512 17.2 and 13.4; 1,024 x 12288 x 2048 72 and 47; 4,096 x 6144 x 1024 66 and 57. Large products of a long K
 // stay with the library (4,096 x 24576 x 4096: 593 us with the activation, 700 here).
 //
 // The same kernel without the activation is mv_gemm_round: plain products whose tiles are one round of the compute units, which the

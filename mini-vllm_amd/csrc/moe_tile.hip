@@ -1,6 +1,6 @@
 // A mixture's products over the chosen (token, expert) pairs only (bfloat16, MFMA; see moe.hip for what the mixture is),
 // through the LDS ring of gemm_tile.hip: the rows of a tile are pairs of one expert, gathered by the addresses their loads
-// take, so that a weight is read once for up to 128 pairs.
+// take, so that a weight is read once for up to 160 pairs.
 //
 //   moe_pairs     lays the pairs out expert by expert (`sorted`: pair numbers, a pair is token * top + place; a shared expert
 //                 that every token uses is one more expert, its pairs n * top + token) and cuts every expert's run into tiles
@@ -337,8 +337,9 @@ static int mt_columns(double row_tiles, int n_out, int halves, int units) {
 
 // Rows of a tile, in 32s. A tile takes as long as its operands take through its compute unit, 77 KB a us: (rows + columns) * 128 bytes a
 // chunk of 64 columns of K; tiles come in rounds; and the weights come from memory whatever the tiles. Of 1 to 5 the one with the least
-// sum over both products: within 2 % of the best of all ten shapes over 22 mixtures (mean pairs an expert 5 to 750, 8 to 64 experts,
-// 768 x 1024, 768 x 2048 and 3072 x 4096), the worst one 12 %. 32 experts of 768 x 1024, 4 a token, and a shared one: 256 tokens tiles of 64
+// sum over both products: 1.5 % behind the best of all shapes on average over 98 mixtures (0.25 to 512 pairs an expert, 8 to 128 experts, 256 x 512
+// to 1536 x 4096), the worst one 13 %, where rounds are estimated nearly even (8 experts of 1024 x 2048, 2 a token, and a shared one, 2,048 tokens:
+// 160 rows 149 us, 128 rows 132). 32 experts of 768 x 1024, 4 a token, and a shared one: 256 tokens tiles of 64
 // rows 50 us, of 128 55; 1,000 tokens (125 pairs an expert) 160 rows 66.5, 128 rows 78, the last tiles of the experts with more than 128
 // being a round of their own; 1,500 tokens 128 rows 96, 160 rows 103; 2,048 tokens 160 rows 112, 128 rows 118.
 static int mt_rows(int n, long n_pairs, int n_real, int hidden, int F, int FS, int units) {

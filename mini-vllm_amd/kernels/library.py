@@ -217,7 +217,6 @@ _OPTIONAL_SIGNATURES = {
     "mv_attention_latent_prompt": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
                                            c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p,
                                            c_void_p]),
-    # the same up to sink, then max_context, work, work_floats, stream
     "mv_attention_latent_heads_tokens": (c_int, []),
     "mv_attention_latent_heads_keys": (c_int, []),
     "mv_attention_latent_heads_serves": (c_int, [c_int, c_int, c_int, c_int]),
@@ -229,6 +228,7 @@ _OPTIONAL_SIGNATURES = {
     "mv_attention_latent_heads": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                           c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_void_p,
                                           c_void_p, c_long, c_int, c_void_p]),
+    # as mv_attention_latent_mfma up to sink, then max_context, work, work_floats, stream
     "mv_attention_latent_split_mfma": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
                                                c_void_p, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p, c_int, c_void_p, c_long,
                                                c_void_p]),

@@ -107,12 +107,12 @@ DECODE_ATTENTION_WAVES = 4
 # the workgroup kernel splits a sequence's keys until about one workgroup for every compute unit is
 # in flight (``Ops.compute_units``)
 # (sequence, kv head) pairs of one decode step whose keys may be split over workgroups
+SPLIT_COUNTERS = 1 << 16
 # steps of up to so many rows carry queries into a latent's space, and sums out of it, in float32
 HEAD_LINEAR_FLOAT_ROWS = 64
 # (block of 32 keys, head) pairs whose keys and values a latent attention may make at a time: 16 KiB each, 512 MiB of scratch at most, in
 # the engine's workspace and once more in that of its recordings
 LATENT_HEADS_MOST = 1 << 15
-SPLIT_COUNTERS = 1 << 16
 # from this many tokens on, value rows are written to their pages 16 tokens of a kv head at a time
 STORE_V_SPLIT_TOKENS = 64
 
@@ -1555,11 +1555,12 @@ class Ops:
         prompt stays where it is unless the contexts are short. Both times in us as measured on an MI355X (256 + 64, 16 and 64 heads): the
         maps 0.26 a thousand (key, head) pairs; a walk 0.8 a block of 32 keys, 512 workgroups of 64 tokens at a time; against
         1.6 a thousand (token, head) pairs for carrying queries in and sums out, and ``latent_shares``' 1.6 a block, 256 workgroups at a
-        time. Own keys / latents: one prompt of 20 tokens 11 / 20, 200 16 / 50, 2,048 55 / 193, 16 tokens behind 2,000 50 / 147; beside 16
-        tokens 8 requests decoding at 1,000 62 / 69, at 300 27 / 36, 64 at 1,000 420 / 85; beside 300 tokens 16 at 1,900 192 / 128.
+        time. Own keys / latents: one prompt of 200 tokens 25 / 51, 2,048 65 / 192, 90 tokens behind 2,000 64 / 168; beside 80 tokens 8 requests
+        decoding at 1,000 67 / 82, at 300 28 / 50; beside 16 tokens 64 at 1,000 458 / 85; beside 300 tokens 16 at 1,900 208 / 127. Over 70 drawn steps
+        for which this says own keys, 8 to 64 heads, they took at most 0.91 of the other's time.
         Steps of up to HEAD_LINEAR_FLOAT_ROWS tokens stay in the latent's space whatever they take: the weighted sum of latents goes through
-        its map in float32 there, where the heads' own values are rounded (one layer of 20 tokens against 64 bits 1.95e-3, with its own
-        values 2.54e-3; from 100 to 4,000 tokens, where both round, 2.57e-3 to 3.29e-3 and 2.61e-3 to 3.30e-3).
+        its map in float32 there, where the heads' own values are rounded (one layer of 20 tokens against 64 bits 2.15e-3, with its own
+        values 2.39e-3, of 64 tokens 2.27e-3 and 2.44e-3; of 65 to 1,000, where both round, 2.76e-3 to 2.95e-3 and 2.46e-3 to 2.50e-3).
         The count is a multiple of 4, of an eighth of it or more, so that steps of similar sizes share the scratch's views."""
         if not lens or max(lens) < 2 or sum(lens) <= HEAD_LINEAR_FLOAT_ROWS:
             return 0
@@ -1838,7 +1839,7 @@ class Ops:
     def moe_pairs(self, x: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, experts: int, identity: int, ff: int, shared: int,
                   ids: torch.Tensor, weights: torch.Tensor, dense: Optional[torch.Tensor], ints: torch.Tensor, act: torch.Tensor,
                   out: torch.Tensor, y: torch.Tensor, limit: float = 0.0, slope: float = 1.0) -> bool:
-        """What ``moe_grouped`` computes, for widths that are multiples of 64, every expert's pairs in tiles of up to 128 rows;
+        """What ``moe_grouped`` computes, for widths that are multiples of 64, every expert's pairs in tiles of up to 160 rows;
         ``shared`` > 0: a shared expert of that width is added, its gate and up rows behind the others' in ``w_gate_up``
         [2 * experts * ff + 2 * shared, hidden], its columns behind the others' in ``w_down`` [hidden, experts * ff + shared]. With
         pairs = n * top (n more with a shared expert), ``act`` [pairs, max(ff, shared)] and ``out`` float32 [pairs, hidden] are scratch,
