@@ -198,8 +198,10 @@ struct GatedPair {
     }
     // The same in few instructions (12 a number instead of 35), which the last waves of a product's workgroup do not hide, for results
     // that are rounded to 16 bits next.
+    __device__ __forceinline__ float of_short(float g, float u) const { return limit > 0.f ? of_short<true>(g, u) : of_short<false>(g, u); }
+    template <bool CLAMPED>
     __device__ __forceinline__ float of_short(float g, float u) const {
-        if (limit > 0.f) {
+        if constexpr (CLAMPED) {
             const float gc = fminf(g, limit), uc = fminf(fmaxf(u, -limit), limit);
             return gc * sigmoid_short(slope * gc) * (uc + 1.f);
         }

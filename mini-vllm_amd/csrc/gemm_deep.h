@@ -14,5 +14,6 @@ extern "C" int mv_gemm_deep_fold(const void* A, long lda, const void* W, const v
 
 // ... and the gated pairs that gemm_pair.hip takes over from the tiled product: the tile, 0: not served
 extern "C" int mv_gemm_pair_shape(int M, int N, int K, int units);
+extern "C" int mv_gemm_pair_reaches(long lda, int N, int K);
 extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* bias, void* C, long ldc, int M, int N, int K, float limit, float slope,
                             int tile, hipStream_t stream);

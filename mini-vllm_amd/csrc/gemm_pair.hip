@@ -7,8 +7,8 @@
 // 0.15 us (the barrier, and waves that wait for the last of them) and 0.385 us for every 128 x 128 of the tile, 1.39 PFLOP/s, half of it
 // the matrix unit, the rest LDS and issue; and a workgroup takes 3.5 us to its first products and from its last. So tiles are large, and
 // which of the twelve shapes depends on how many whole rounds of compute units they make (mv_gemm_pair_shape): 2,048 x 6144 x 1024
-// is one of 256 x 192. There 36.4 us with the library's product and the activation behind it, 27.5 here; 1,536 rows 34.7 (gemm_tile.hip)
-// and 22.4; 1,024 23.5 and 17.8; 512 17.2 and 13.4; 1,024 x 12288 x 2048 72 and 47; 4,096 x 6144 x 1024 66 and 57. Large products of a long K
+// is one of 256 x 192. There 36.4 us with the library's product and the activation behind it, 27.2 here; 1,536 rows 34.7 (gemm_tile.hip)
+// and 21.8; 1,024 23.5 and 17.6; 512 17.2 and 12.9; 1,024 x 12288 x 2048 72 and 47; 4,096 x 6144 x 1024 66 and 52.8. Large products of a long K
 // stay with the library (4,096 x 24576 x 4096: 593 us with the activation, 700 here).
 //
 // The same kernel without the activation is mv_gemm_round: plain products whose tiles are one round of the compute units, which the
@@ -21,6 +21,7 @@
 #include "gemm_ring.h"
 
 #include <cmath>
+#include <type_traits>
 
 struct PairArgs {
     const bf16* A;
@@ -36,14 +37,22 @@ struct PairArgs {
 
 // Eight waves, four down the rows and two along the columns, each with WM x WN products of 16 x 16.
 // GATED: half of the weight rows are gates and half are ups, else C is the product itself.
-template <int WM, int WN, int STAGES, bool GATED>
+// Rows and weight rows have rings of their own, of SA and SB chunks (SB >= SA). A tile of 256 x 192 has room for no third chunk of both, but
+// for two of the rows and four of the weight, which comes from memory. A load's address is one scalar base an operand, advanced by a
+// chunk, and 32 bits a lane that do not change (64 bits a lane: two vector additions a load). With both, and the epilogue's forms apart,
+// us, weights that take turns, in turn with the kernel before: gated 6144 x 1024, 512 / 1,024 / 1,536 / 2,048 / 4,096 rows 13.2 -> 12.9, 18.2 -> 17.6,
+// 22.9 -> 21.8, 27.8 -> 27.2, 55.0 -> 52.8; plain 2,048 x 5184 x 1024 28.9 -> 28.2, 2,048 x 1024 x 2048 15.6 -> 13.6, x 3072 21.1 -> 18.9.
+template <int WM, int WN, int SA, int SB, bool GATED>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_pair_kernel(PairArgs a) {
     constexpr int BM = 64 * WM, BN = 32 * WN, WAVES = 8;
-    constexpr int ROWS = BM + BN, INSTR = ROWS / 8, REPS = (INSTR + WAVES - 1) / WAVES, LEAST = INSTR / WAVES, STAGE = ROWS * 8;
+    constexpr int LA = WM, GROUPS = BN / 8, LB = (GROUPS + WAVES - 1) / WAVES, LEAST = GROUPS / WAVES;      // a wave's loads of a chunk (of the weight: or LEAST)
+    constexpr int STAGE_A = BM * 8, STAGE_B = BN * 8;
     static_assert(!GATED || WN % 2 == 0, "a wave's weight tiles are half gate, half up");
-    static_assert(STAGES >= 2 && STAGES <= 4 && STAGES * STAGE * 16 <= 163840 && (STAGES - 1) * REPS <= 63, "the ring does not fit");
-    __shared__ uint4 ring[STAGES * STAGE];
+    static_assert(SA >= 2 && SB >= SA && (SA * STAGE_A + SB * STAGE_B) * 16 <= 163840, "the rings do not fit");
+    static_assert((SA - 1) * LA + (SB - 1) * LB <= 63, "more loads on their way than the counter holds");
+    __shared__ uint4 ring[SA * STAGE_A + SB * STAGE_B];
+    uint4* const ring_b = ring + SA * STAGE_A;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / MV_WAVE), lane = tid % MV_WAVE, i = lane % 16, g = lane / 16;
     const int wm = wave / 2, wn = wave % 2;
     // An XCD has a run of tiles. Rows change fastest, so that a band of the weight goes into one L2; with more rows than weight rows
@@ -53,25 +62,32 @@ gemm_pair_kernel(PairArgs a) {
     const int quick = id % a.fast, slow = id / a.fast, tm = a.by_columns ? slow : quick, tn = a.by_columns ? quick : slow;
     const int m0 = tm * BM, n0 = tn * (GATED ? BN / 2 : BN), n = a.K / GT_KC;
 
-    // this lane's share of the loads, and the operands: as in gemm_tile.hip
+    // this lane's share of the loads (eight rows of a chunk an instruction, pieces swizzled as in gemm_tile.hip); the entry points have made
+    // sure that the offsets fit into 32 bits
     const int lrow = lane / 8, piece = (lane % 8) ^ lrow;
-    const char* src[REPS];
+    uint32_t off_a[LA], off_b[LB];
 #pragma unroll
-    for (int rep = 0; rep < REPS; ++rep) {
-        const int row = 8 * (wave + WAVES * rep) + lrow;
-        if (row < BM) {
-            src[rep] = reinterpret_cast<const char*>(a.A + (size_t)min(m0 + row, a.M - 1) * a.lda + 8 * piece);
-        } else {
-            const int r = row - BM;
-            const int w = !GATED || r < BN / 2 ? min(n0 + r, a.I - 1) : min(a.I + n0 + r - BN / 2, 2 * a.I - 1);
-            src[rep] = reinterpret_cast<const char*>(a.W + (size_t)w * a.K + 8 * piece);
-        }
+    for (int r = 0; r < LA; ++r) off_a[r] = ((uint32_t)min(8 * (wave + WAVES * r) + lrow, a.M - 1 - m0) * (uint32_t)a.lda + 8 * piece) * 2;
+#pragma unroll
+    for (int r = 0; r < LB; ++r) {
+        const int row = 8 * (wave + WAVES * r) + lrow;
+        const int w = !GATED || row < BN / 2 ? min(n0 + row, a.I - 1) : min(a.I + n0 + row - BN / 2, 2 * a.I - 1);
+        off_b[r] = ((uint32_t)w * (uint32_t)a.K + 8 * piece) * 2;
     }
-    auto fetch = [&](int c, uint4* stage) __attribute__((always_inline)) {
+    const char* const from_a = reinterpret_cast<const char*>(a.A + (size_t)m0 * a.lda);
+    const char* const from_b = reinterpret_cast<const char*>(a.W);
+    auto fetch_a = [&](int c, int stage) __attribute__((always_inline)) {
 #pragma unroll
-        for (int rep = 0; rep < REPS; ++rep)
-            if (INSTR % WAVES == 0 || rep < LEAST || wave < INSTR % WAVES)
-                gt_load_to_lds(src[rep] + (size_t)c * (GT_KC * sizeof(bf16)), (__attribute__((address_space(3))) void*)(stage + (wave + WAVES * rep) * 64));
+        for (int r = 0; r < LA; ++r)
+            gt_load_to_lds_from(from_a + (size_t)c * (GT_KC * sizeof(bf16)), off_a[r],
+                                (__attribute__((address_space(3))) void*)(ring + stage * STAGE_A + (wave + WAVES * r) * 64));
+    };
+    auto fetch_b = [&](int c, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < LB; ++r)
+            if (GROUPS % WAVES == 0 || r < LEAST || wave < GROUPS % WAVES)
+                gt_load_to_lds_from(from_b + (size_t)c * (GT_KC * sizeof(bf16)), off_b[r],
+                                    (__attribute__((address_space(3))) void*)(ring_b + stage * STAGE_B + (wave + WAVES * r) * 64));
     };
     int a_off[WM], w_off[WN];
 #pragma unroll
@@ -79,7 +95,7 @@ gemm_pair_kernel(PairArgs a) {
 #pragma unroll
     for (int t = 0; t < WN; ++t) {
         const int group = !GATED ? WN * wn + t : t < WN / 2 ? (WN / 2) * wn + t : (WN / 2) * (2 + wn) + (t - WN / 2);
-        w_off[t] = (BM + 16 * group + i) * 8;
+        w_off[t] = (16 * group + i) * 8;
     }
     const int sw0 = g ^ (i & 7), sw1 = (4 + g) ^ (i & 7);
     floatx4_t acc[WN][WM];
@@ -90,11 +106,11 @@ gemm_pair_kernel(PairArgs a) {
     struct Operands {
         TFrag a[WM], w[WN];
     };
-    auto read = [&](const uint4* stage, int sw, Operands& o) __attribute__((always_inline)) {
+    auto read = [&](int sa, int sb, int sw, Operands& o) __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < WN; ++t) o.w[t].u = stage[w_off[t] + sw];
+        for (int t = 0; t < WN; ++t) o.w[t].u = ring_b[sb * STAGE_B + w_off[t] + sw];
 #pragma unroll
-        for (int u = 0; u < WM; ++u) o.a[u].u = stage[a_off[u] + sw];
+        for (int u = 0; u < WM; ++u) o.a[u].u = ring[sa * STAGE_A + a_off[u] + sw];
     };
     auto multiply = [&](const Operands& o) __attribute__((always_inline)) {
 #pragma unroll
@@ -102,29 +118,27 @@ gemm_pair_kernel(PairArgs a) {
 #pragma unroll
             for (int t = 0; t < WN; ++t) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[t].v, o.a[u].v, acc[t][u], 0, 0, 0);
     };
-    auto landed = [&](int later) __attribute__((always_inline)) {      // this wave's loads, but for those of `later` chunks
-        switch (later) {
-            case 0: GT_WAIT_VMCNT(0); break;
-            case 1: GT_WAIT_VMCNT(LEAST); break;
-            case 2: GT_WAIT_VMCNT(2 * LEAST); break;
-            default: GT_WAIT_VMCNT(3 * LEAST); break;
-        }
-    };
-    // Chunk k lives in stage k % STAGES; its operands are read in two halves of 32 columns, each while the products of the half before run.
-    // The barrier stands between the halves: then everybody's reads of chunk k are back, so chunk k + STAGES may come into its stage,
-    // and everybody's loads of chunk k + 1 have landed.
-#pragma unroll
-    for (int k = 0; k < STAGES; ++k)
-        if (k < n) fetch(k, ring + k * STAGE);
+    // Chunk k lives in stages k % SA and k % SB; its operands are read in two halves of 32 columns, each while the products of the half
+    // before run. The barrier stands between the halves: then everybody's reads of chunk k are back, so chunks k + SA of the rows and
+    // k + SB of the weight may come into its stages, and everybody's loads of chunk k + 1 have landed. A wave's loads behind those of
+    // chunk k + 1 are then, with all there are to ask for, SA - 2 whole chunks, and the weight's of the turn that asked for the
+    // chunk's rows where its own were asked for before; at the end, where some are missing, all are waited for.
+    constexpr int STEADY = (SA - 2) * (LA + LEAST) + (SB > SA ? LEAST : 0);
+    for (int j = -SB; j < 0; ++j) {                    // (as the turns in front of the first would)
+        if (j + SA >= 0 && j + SA < n) fetch_a(j + SA, j + SA);
+        if (j + SB < n) fetch_b(j + SB, j + SB);
+    }
     Operands even, odd;
-    landed(n - 1 < STAGES - 1 ? n - 1 : STAGES - 1);
+    if (n > SB) GT_WAIT_VMCNT((SA - 1) * (LA + LEAST));
+    else GT_WAIT_VMCNT(0);
     __builtin_amdgcn_s_barrier();
-    read(ring, sw0, even);
-    int st = 0;
+    read(0, 0, sw0, even);
+    int sa = 0, sb = 0;
     for (int k = 0; k < n; ++k) {
-        uint4* stage = ring + st * STAGE;
-        st = st + 1 == STAGES ? 0 : st + 1;
-        read(stage, sw1, odd);
+        const int old_a = sa, old_b = sb;
+        sa = sa + 1 == SA ? 0 : sa + 1;
+        sb = sb + 1 == SB ? 0 : sb + 1;
+        read(old_a, old_b, sw1, odd);
         multiply(even);
         // (a read, then some products, in turn: as the compiler has them, all reads first, 3 % slower)
 #pragma unroll
@@ -132,49 +146,71 @@ gemm_pair_kernel(PairArgs a) {
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, WM * WN / (WM + WN) > 0 ? WM * WN / (WM + WN) : 1, 0);
         }
-        if (k + 1 < n) landed(n - k - 2 < STAGES - 2 ? n - k - 2 : STAGES - 2);
+        if (k + SB <= n) GT_WAIT_VMCNT(STEADY);
+        else GT_WAIT_VMCNT(0);
         __builtin_amdgcn_s_waitcnt(0xc07f);
         __builtin_amdgcn_s_barrier();
-        if (k + STAGES < n) fetch(k + STAGES, stage);
-        if (k + 1 < n) read(ring + st * STAGE, sw0, even);
+        if (k + SA < n) fetch_a(k + SA, old_a);
+        if (k + SB < n) fetch_b(k + SB, old_b);
+        if (k + 1 < n) read(sa, sb, sw0, even);
         multiply(odd);
     }
 
     // lane l holds C[row 16 u + l % 16][columns 4 (l / 16) .. + 3 of tile t]
     constexpr int TOUT = GATED ? WN / 2 : WN;
+    // The forms that are in use have code of their own, with nothing in it to be jumped over: what a wave fetches of it for the first time
+    // is on its way (2,048 x 6144 x 1024: all in one 29.4 us, apart 27.2).
+    auto store = [&](auto bias, auto clamped, auto whole) __attribute__((always_inline)) {
+        constexpr bool BIAS = decltype(bias)::value, WHOLE = decltype(whole)::value;
 #pragma unroll
-    for (int t = 0; t < TOUT; ++t) {
-        const int col = n0 + 16 * (TOUT * wn + t) + 4 * g;
-        float bv[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
-        if (a.bias != nullptr) {
+        for (int t = 0; t < TOUT; ++t) {
+            const int col = n0 + 16 * (TOUT * wn + t) + 4 * g;
+            float bv[4], bu[4];
+            if constexpr (BIAS) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (col + e < a.I) {
-                    bv[e] = to_f(a.bias[col + e]);
-                    if constexpr (GATED) bu[e] = to_f(a.bias[a.I + col + e]);
+                for (int e = 0; e < 4; ++e) {
+                    const int c = min(col + e, a.I - 1);
+                    bv[e] = a.bias != nullptr ? to_f(a.bias[c]) : 0.f;
+                    bu[e] = GATED && a.bias != nullptr ? to_f(a.bias[a.I + c]) : 0.f;
                 }
-        }
-#pragma unroll
-        for (int u = 0; u < WM; ++u) {
-            const int row = m0 + 16 * (WM * wm + u) + i;
-            if (row >= a.M || col >= a.I) continue;
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if constexpr (GATED) v[e] = a.pair.of_short(acc[t][u][e] + bv[e], acc[t + TOUT][u][e] + bu[e]);
-                else v[e] = acc[t][u][e] + bv[e];
             }
-            bf16* to = a.C + (size_t)row * a.ldc + col;
-            if (a.wide_stores && col + 3 < a.I) {
-                *reinterpret_cast<uint2*>(to) = uint2{f32x2_to_bf16x2_bits(v[0], v[1]), f32x2_to_bf16x2_bits(v[2], v[3])};
-            } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (col + e < a.I) to[e] = from_f<bf16>(v[e]);
+            for (int u = 0; u < WM; ++u) {
+                const int row = m0 + 16 * (WM * wm + u) + i;
+                if (row >= a.M || col >= a.I) continue;
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = BIAS ? acc[t][u][e] + bv[e] : acc[t][u][e];
+                    if constexpr (GATED) v[e] = a.pair.of_short<decltype(clamped)::value>(v[e], BIAS ? acc[t + TOUT][u][e] + bu[e] : acc[t + TOUT][u][e]);
+                }
+                bf16* to = a.C + (size_t)row * a.ldc + col;
+                if (WHOLE || (a.wide_stores && col + 3 < a.I)) {
+                    *reinterpret_cast<uint2*>(to) = uint2{f32x2_to_bf16x2_bits(v[0], v[1]), f32x2_to_bf16x2_bits(v[2], v[3])};
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (col + e < a.I) to[e] = from_f<bf16>(v[e]);
+                }
             }
         }
+    };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    const bool whole = a.wide_stores && a.I % 4 == 0;
+    if (GATED && a.pair.limit > 0.f) {
+        if (!whole) store(yes, yes, no);
+        else if (a.bias != nullptr) store(yes, yes, yes);
+        else store(no, yes, yes);
+    } else {
+        if (!whole) store(yes, no, no);
+        else if (a.bias != nullptr) store(yes, no, yes);
+        else store(no, no, yes);
     }
 }
+
+// 1: a tile's rows, lda apart, and the weight lie within the 32 bits of a lane's offset (what does not is left to the other kernels)
+extern "C" int mv_gemm_pair_reaches(long lda, int N, int K) { return lda < 1L << 23 && (long)N * K < 1L << 31; }
 
 struct PairTile {
     int tile;            // rows << 16 | weight rows
@@ -226,6 +262,7 @@ extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* 
     MV_REQUIRE(M > 0 && N > 0 && K > 0 && K % GT_KC == 0 && N % 2 == 0, "gemm_pair: bad sizes M=%d N=%d K=%d", M, N, K);
     MV_REQUIRE(A && W && C && lda >= K && lda % 8 == 0 && ((uintptr_t)A | (uintptr_t)W) % 16 == 0 && ldc >= N / 2,
                "gemm_pair: operands not aligned or pitches too small");
+    MV_REQUIRE(mv_gemm_pair_reaches(lda, N, K), "gemm_pair: rows %ld apart or a weight of %d x %d are too long", lda, N, K);
     const int bm = tile >> 16, bn = tile & 0xffff;
     MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 128 || bn == 192), "gemm_pair: no tile of %d x %d", bm, bn);
     const int tiles_m = (M + bm - 1) / bm, tiles_n = (N / 2 + bn / 2 - 1) / (bn / 2), by_columns = M > N;
@@ -234,22 +271,22 @@ extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* 
     const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N / 2, K, (int)tiles,
                      by_columns ? tiles_n : tiles_m, by_columns, ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{limit, slope}};
     const dim3 grid((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
-#define GP_LAUNCH(WM, WN, S) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, S, true>), grid, dim3(512), 0, stream, a)
+#define GP_LAUNCH(WM, WN, SA, SB) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, SA, SB, true>), grid, dim3(512), 0, stream, a)
     if (bn == 192) {
-        if (bm == 256) GP_LAUNCH(4, 6, 2);
-        else if (bm == 192) GP_LAUNCH(3, 6, 3);
-        else if (bm == 128) GP_LAUNCH(2, 6, 4);
-        else GP_LAUNCH(1, 6, 4);
+        if (bm == 256) GP_LAUNCH(4, 6, 2, 4);
+        else if (bm == 192) GP_LAUNCH(3, 6, 3, 3);
+        else if (bm == 128) GP_LAUNCH(2, 6, 4, 4);
+        else GP_LAUNCH(1, 6, 4, 4);
     } else if (bn == 128) {
-        if (bm == 256) GP_LAUNCH(4, 4, 3);
-        else if (bm == 192) GP_LAUNCH(3, 4, 4);
-        else if (bm == 128) GP_LAUNCH(2, 4, 4);
-        else GP_LAUNCH(1, 4, 4);
+        if (bm == 256) GP_LAUNCH(4, 4, 3, 3);
+        else if (bm == 192) GP_LAUNCH(3, 4, 4, 4);
+        else if (bm == 128) GP_LAUNCH(2, 4, 4, 4);
+        else GP_LAUNCH(1, 4, 4, 4);
     } else {
-        if (bm == 256) GP_LAUNCH(4, 2, 4);
-        else if (bm == 192) GP_LAUNCH(3, 2, 4);
-        else if (bm == 128) GP_LAUNCH(2, 2, 4);
-        else GP_LAUNCH(1, 2, 4);
+        if (bm == 256) GP_LAUNCH(4, 2, 4, 4);
+        else if (bm == 192) GP_LAUNCH(3, 2, 4, 4);
+        else if (bm == 128) GP_LAUNCH(2, 2, 4, 4);
+        else GP_LAUNCH(1, 2, 4, 4);
     }
 #undef GP_LAUNCH
     return mv_check_launch("gemm_pair");
@@ -294,6 +331,7 @@ extern "C" int mv_gemm_round(const void* A, long lda, const void* W, const void*
     MV_REQUIRE(M > 0 && N > 0 && K > 0 && K % GT_KC == 0, "gemm_round: bad sizes M=%d N=%d K=%d", M, N, K);
     MV_REQUIRE(A && W && C && lda >= K && lda % 8 == 0 && ((uintptr_t)A | (uintptr_t)W) % 16 == 0 && ldc >= N,
                "gemm_round: operands not aligned or pitches too small");
+    MV_REQUIRE(mv_gemm_pair_reaches(lda, N, K), "gemm_round: rows %ld apart or a weight of %d x %d are too long", lda, N, K);
     const int bm = tile >> 16, bn = tile & 0xffff;
     MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 96 || bn == 128 || bn == 192), "gemm_round: no tile of %d x %d", bm, bn);
     const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn, by_columns = M > N;
@@ -302,27 +340,27 @@ extern "C" int mv_gemm_round(const void* A, long lda, const void* W, const void*
     const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N, K, (int)tiles,
                      by_columns ? tiles_n : tiles_m, by_columns, ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{0.f, 1.f}};
     const dim3 grid((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
-#define GR_LAUNCH(WM, WN, S) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, S, false>), grid, dim3(512), 0, stream, a)
+#define GR_LAUNCH(WM, WN, SA, SB) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, SA, SB, false>), grid, dim3(512), 0, stream, a)
     if (bn == 192) {
-        if (bm == 256) GR_LAUNCH(4, 6, 2);
-        else if (bm == 192) GR_LAUNCH(3, 6, 3);
-        else if (bm == 128) GR_LAUNCH(2, 6, 4);
-        else GR_LAUNCH(1, 6, 4);
+        if (bm == 256) GR_LAUNCH(4, 6, 2, 4);
+        else if (bm == 192) GR_LAUNCH(3, 6, 3, 3);
+        else if (bm == 128) GR_LAUNCH(2, 6, 4, 4);
+        else GR_LAUNCH(1, 6, 4, 4);
     } else if (bn == 128) {
-        if (bm == 256) GR_LAUNCH(4, 4, 3);
-        else if (bm == 192) GR_LAUNCH(3, 4, 4);
-        else if (bm == 128) GR_LAUNCH(2, 4, 4);
-        else GR_LAUNCH(1, 4, 4);
+        if (bm == 256) GR_LAUNCH(4, 4, 3, 3);
+        else if (bm == 192) GR_LAUNCH(3, 4, 4, 4);
+        else if (bm == 128) GR_LAUNCH(2, 4, 4, 4);
+        else GR_LAUNCH(1, 4, 4, 4);
     } else if (bn == 96) {
-        if (bm == 256) GR_LAUNCH(4, 3, 3);
-        else if (bm == 192) GR_LAUNCH(3, 3, 4);
-        else if (bm == 128) GR_LAUNCH(2, 3, 4);
-        else GR_LAUNCH(1, 3, 4);
+        if (bm == 256) GR_LAUNCH(4, 3, 3, 3);
+        else if (bm == 192) GR_LAUNCH(3, 3, 4, 4);
+        else if (bm == 128) GR_LAUNCH(2, 3, 4, 4);
+        else GR_LAUNCH(1, 3, 4, 4);
     } else {
-        if (bm == 256) GR_LAUNCH(4, 2, 4);
-        else if (bm == 192) GR_LAUNCH(3, 2, 4);
-        else if (bm == 128) GR_LAUNCH(2, 2, 4);
-        else GR_LAUNCH(1, 2, 4);
+        if (bm == 256) GR_LAUNCH(4, 2, 4, 4);
+        else if (bm == 192) GR_LAUNCH(3, 2, 4, 4);
+        else if (bm == 128) GR_LAUNCH(2, 2, 4, 4);
+        else GR_LAUNCH(1, 2, 4, 4);
     }
 #undef GR_LAUNCH
     return mv_check_launch("gemm_round");

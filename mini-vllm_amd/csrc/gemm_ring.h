@@ -24,3 +24,11 @@ __device__ __forceinline__ void gt_load_to_lds(const void* src, __attribute__((a
                  : "v"(src), "s"(lds_base)
                  : "memory", "m0");
 }
+
+// The same from a scalar base and 32 bits a lane.
+__device__ __forceinline__ void gt_load_to_lds_from(const void* base, uint32_t offset, __attribute__((address_space(3))) void* lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(offset), "s"(base), "s"(lds_base)
+                 : "memory", "m0");
+}

@@ -413,7 +413,7 @@ static int tile_launch(const void* A, long lda, const void* W, const void* bias,
         return mv_gemm_deep(A, lda, W, bias, C, ldc, c_dtype, M, N, K, gated, partial, P, eps, pair.limit, pair.slope, square_relu, 0, stream);
     // (pairs that gemm_deep.hip serves stay there: K of 1,024, 2048 to 3072 weight rows, 130 to 256 rows 7.3 to 7.7 us, in gemm_pair.hip 7.4 to
     // 7.9, weights from memory, 6.7 and 7.8 from the last cache; K of 768 level)
-    if (force == 0 && p.F == 1 && c_dtype == MV_BF16 && gated && partial == nullptr)
+    if (force == 0 && p.F == 1 && c_dtype == MV_BF16 && gated && partial == nullptr && mv_gemm_pair_reaches(lda, N, K))
         if (const int tile = mv_gemm_pair_shape(M, N, K, mv_compute_units()))
             return mv_gemm_pair(A, lda, W, bias, C, ldc, M, N, K, pair.limit, pair.slope, tile, stream);
     MV_REQUIRE(tile_shape_served(p, gated != 0), "gemm_tile: no kernel for wave tiles %d x %d%s", p.wm, p.wn,

@@ -238,6 +238,7 @@ _OPTIONAL_SIGNATURES = {
     "mv_moe_grouped": (c_int, [c_void_p, c_long, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int,
                                c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_float, c_float, c_void_p]),
     "mv_gemm_pair_shape": (c_int, [c_int, c_int, c_int, c_int]),
+    "mv_gemm_pair_reaches": (c_int, [c_long, c_int, c_int]),
     # A, lda, W, bias, C, ldc, M, N, K, limit, slope, tile, stream
     "mv_gemm_pair": (c_int, [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_float, c_float, c_int, c_void_p]),
     "mv_gemm_round_shape": (c_int, [c_int, c_int, c_int, c_int]),

@@ -2611,7 +2611,8 @@ class Ops:
             return False
         (M, K), N = a.shape, w.shape[0]
         tile = self.lib.dll.mv_gemm_round_shape(M, N, K, self.compute_units)
-        if (not tile or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or not w.is_contiguous()
+        if (not tile or not self.lib.dll.mv_gemm_pair_reaches(a.stride(0), N, K)
+                or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or not w.is_contiguous()
                 or a.stride(1) != 1 or out.stride(1) != 1 or a.stride(0) % 8 or a.data_ptr() % 16 or w.data_ptr() % 16):
             return False
         self._note("mv_gemm_round", self._size(a, w, out), 2 * M * N * K)
@@ -2761,7 +2762,8 @@ class Ops:
             return False
         (M, K), N = a.shape, w.shape[0]
         tile = self.lib.dll.mv_gemm_pair_shape(M, N, K, self.compute_units)
-        if (not tile or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or not w.is_contiguous()
+        if (not tile or not self.lib.dll.mv_gemm_pair_reaches(a.stride(0), N, K)
+                or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or not w.is_contiguous()
                 or w.shape[1] != K or a.stride(1) != 1 or a.stride(0) % 8 or a.data_ptr() % 16 or w.data_ptr() % 16
                 or out.shape != (M, N // 2) or out.stride(1) != 1):
             return False

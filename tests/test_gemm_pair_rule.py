@@ -77,3 +77,12 @@ def test_a_pair_with_a_squared_relu_stays_refused(lib, M, N, K):
     address, bf16 = 1 << 20, 1
     assert lib.mv_gemm_tile(address, K, address, None, address, N // 2, bf16, M, N, K, 1, None, 0, 0, 0.0, 1.0, 1, None)
     assert b"squared ReLU" in lib.mv_last_error()
+
+
+@pytest.mark.parametrize("lda, n, k, reaches", [(1024, 6144, 1024, 1), ((1 << 23) - 8, 6144, 1024, 1), (1 << 23, 6144, 1024, 0), (1 << 40, 64, 64, 0),
+                                                (4096, (1 << 19) - 1, 4096, 1), (4096, 1 << 19, 4096, 0)])
+def test_offsets_of_a_tile_fit_into_32_bits(lib, lda, n, k, reaches):
+    """A lane's byte offset is at most that of row 255 of a tile, or of the weight's last row, and a chunk's 128 bytes."""
+    lib.mv_gemm_pair_reaches.argtypes = [ctypes.c_long, ctypes.c_int, ctypes.c_int]
+    assert lib.mv_gemm_pair_reaches(lda, n, k) == reaches
+    assert not reaches or max(255 * lda, (n - 1) * k) * 2 + 128 < 1 << 32
