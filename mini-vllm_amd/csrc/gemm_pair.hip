@@ -33,18 +33,34 @@ struct PairArgs {
     int M, I, K;                       // plain: I = N
     int tiles, fast, by_columns, wide_stores;    // fast: tiles of the side that changes fastest
     GatedPair pair;
+    // rows behind a folded norm: P partial sums of squares each; PAIR_FOLD writes them
+    float* partial;
+    int P;
+    float eps;
+    // PAIR_FOLD
+    float* resid;
+    long ldr;
+    WeightPtr norm_weight;
+    int unit_offset;
+    bf16* weighted;
+    long ldw;
 };
 
+// PAIR_FOLD: the product in front of a residual add and a norm; _SCALED: behind one (see gemm_deep.hip for both)
+enum PairForm { PAIR_PLAIN = 0, PAIR_GATED = 1, PAIR_FOLD = 2, PAIR_PLAIN_SCALED = 3, PAIR_GATED_SCALED = 4 };
+
 // Eight waves, four down the rows and two along the columns, each with WM x WN products of 16 x 16.
-// GATED: half of the weight rows are gates and half are ups, else C is the product itself.
+// Gated: half of the weight rows are gates and half are ups, else C is the product itself.
 // Rows and weight rows have rings of their own, of SA and SB chunks (SB >= SA). A tile of 256 x 192 has room for no third chunk of both, but
 // for two of the rows and four of the weight, which comes from memory. A load's address is one scalar base an operand, advanced by a
 // chunk, and 32 bits a lane that do not change (64 bits a lane: two vector additions a load). With both, and the epilogue's forms apart,
 // us, weights that take turns, in turn with the kernel before: gated 6144 x 1024, 512 / 1,024 / 1,536 / 2,048 / 4,096 rows 13.2 -> 12.9, 18.2 -> 17.6,
 // 22.9 -> 21.8, 27.8 -> 27.2, 55.0 -> 52.8; plain 2,048 x 5184 x 1024 28.9 -> 28.2, 2,048 x 1024 x 2048 15.6 -> 13.6, x 3072 21.1 -> 18.9.
-template <int WM, int WN, int SA, int SB, bool GATED>
+template <int WM, int WN, int SA, int SB, int FORM>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_pair_kernel(PairArgs a) {
+    constexpr bool GATED = FORM == PAIR_GATED || FORM == PAIR_GATED_SCALED, SCALED = FORM == PAIR_PLAIN_SCALED || FORM == PAIR_GATED_SCALED;
+    constexpr bool FOLD = FORM == PAIR_FOLD;
     constexpr int BM = 64 * WM, BN = 32 * WN, WAVES = 8;
     constexpr int LA = WM, GROUPS = BN / 8, LB = (GROUPS + WAVES - 1) / WAVES, LEAST = GROUPS / WAVES;      // a wave's loads of a chunk (of the weight: or LEAST)
     constexpr int STAGE_A = BM * 8, STAGE_B = BN * 8;
@@ -61,6 +77,35 @@ gemm_pair_kernel(PairArgs a) {
     if ((int)blockIdx.x / GT_XCDS >= run || id >= a.tiles) return;
     const int quick = id % a.fast, slow = id / a.fast, tm = a.by_columns ? slow : quick, tn = a.by_columns ? quick : slow;
     const int m0 = tm * BM, n0 = tn * (GATED ? BN / 2 : BN), n = a.K / GT_KC;
+
+    // what the end needs from memory is asked for here, in front of everything
+    // The sums of squares of the tile's rows: SHARE threads a row, of whose quads thread j of eight (a thread is 8 / SHARE of them) adds up
+    // number j, j + 8, .. and the eight are added in pairs, in one order for every tile.
+    constexpr int SHARE = BM == 64 ? 8 : BM == 128 ? 4 : 2, MINE = 8 / SHARE;
+    float4 sq[SCALED ? MINE : 1];
+    const float4* sq_row = nullptr;
+    int quads = 0;
+    if constexpr (SCALED) {
+        quads = a.P / 4;
+        sq_row = reinterpret_cast<const float4*>(a.partial + (size_t)min(m0 + tid / SHARE, a.M - 1) * a.P);
+#pragma unroll
+        for (int e = 0; e < MINE; ++e) {
+            const int q = tid % SHARE * MINE + e;
+            sq[e] = q < quads ? sq_row[q] : float4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    float4 old[FOLD ? WN : 1][FOLD ? WM : 1];
+    float nw[FOLD ? WN : 1][4];
+    if constexpr (FOLD) {
+#pragma unroll
+        for (int t = 0; t < WN; ++t) {
+            const int col = min(n0 + 16 * (WN * wn + t) + 4 * g, a.I - 4);
+            a.norm_weight.at_few<4>(col, nw[t]);
+#pragma unroll
+            for (int u = 0; u < WM; ++u)
+                old[t][u] = *reinterpret_cast<const float4*>(a.resid + (size_t)min(m0 + 16 * (WM * wm + u) + i, a.M - 1) * a.ldr + col);
+        }
+    }
 
     // this lane's share of the loads (eight rows of a chunk an instruction, pieces swizzled as in gemm_tile.hip); the entry points have made
     // sure that the offsets fit into 32 bits
@@ -158,6 +203,70 @@ gemm_pair_kernel(PairArgs a) {
 
     // lane l holds C[row 16 u + l % 16][columns 4 (l / 16) .. + 3 of tile t]
     constexpr int TOUT = GATED ? WN / 2 : WN;
+    if constexpr (FOLD) {
+        // resid += bf16(product (+ bias)), as the add behind a rounded product makes it; a wave's columns leave each row's sum of squares
+        const float off = a.unit_offset ? 1.f : 0.f;
+        float ssq[WM];
+#pragma unroll
+        for (int u = 0; u < WM; ++u) ssq[u] = 0.f;
+#pragma unroll
+        for (int t = 0; t < WN; ++t) {
+            const int col = n0 + 16 * (WN * wn + t) + 4 * g;
+            float b[4] = {0.f, 0.f, 0.f, 0.f};
+            if (a.bias != nullptr) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) b[e] = to_f(a.bias[min(col + e, a.I - 1)]);
+            }
+#pragma unroll
+            for (int u = 0; u < WM; ++u) {
+                const int row = m0 + 16 * (WM * wm + u) + i;
+                if (row >= a.M || col >= a.I) continue;                 // (columns beyond the last come in fours)
+                const float was[4] = {old[t][u].x, old[t][u].y, old[t][u].z, old[t][u].w};
+                float x[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    x[e] = was[e] + __uint_as_float((uint32_t)f32_to_bf16_bits(acc[t][u][e] + b[e]) << 16);
+                    ssq[u] = fmaf(x[e], x[e], ssq[u]);
+                }
+                *reinterpret_cast<float4*>(a.resid + (size_t)row * a.ldr + col) = float4{x[0], x[1], x[2], x[3]};
+                *reinterpret_cast<uint2*>(a.weighted + (size_t)row * a.ldw + col) =
+                    uint2{f32x2_to_bf16x2_bits(x[0] * (nw[t][0] + off), x[1] * (nw[t][1] + off)),
+                          f32x2_to_bf16x2_bits(x[2] * (nw[t][2] + off), x[3] * (nw[t][3] + off))};
+            }
+        }
+        const int part = n0 / (16 * WN) + wn;
+#pragma unroll
+        for (int u = 0; u < WM; ++u) {
+            ssq[u] += __shfl_xor(ssq[u], 16, MV_WAVE);
+            ssq[u] += __shfl_xor(ssq[u], 32, MV_WAVE);
+            const int row = m0 + 16 * (WM * wm + u) + i;
+            if (g == 0 && row < a.M && part < a.P) a.partial[(size_t)row * a.P + part] = ssq[u];
+        }
+        return;
+    }
+    float rinv[WM];
+    if constexpr (SCALED) {
+        float s[MINE];
+#pragma unroll
+        for (int e = 0; e < MINE; ++e) {
+            for (int q = tid % SHARE * MINE + e + 8; q < quads; q += 8) {
+                const float4 v = sq_row[q];
+                sq[e].x += v.x; sq[e].y += v.y; sq[e].z += v.z; sq[e].w += v.w;
+            }
+            s[e] = (sq[e].x + sq[e].y) + (sq[e].z + sq[e].w);
+        }
+#pragma unroll
+        for (int o = 1; o < MINE; o <<= 1)
+#pragma unroll
+            for (int e = 0; e < MINE; e += 2 * o) s[e] += s[e + o];
+#pragma unroll
+        for (int o = 1; o < SHARE; o <<= 1) s[0] += __shfl_xor(s[0], o, MV_WAVE);
+        float* const sh = reinterpret_cast<float*>(ring);               // (behind the last barrier nobody reads the rings)
+        if (tid % SHARE == 0 && tid / SHARE < BM) sh[tid / SHARE] = rsqrtf(s[0] / (float)a.K + a.eps);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < WM; ++u) rinv[u] = sh[16 * (WM * wm + u) + i];
+    }
     // The forms that are in use have code of their own, with nothing in it to be jumped over: what a wave fetches of it for the first time
     // is on its way (2,048 x 6144 x 1024: all in one 29.4 us, apart 27.2).
     auto store = [&](auto bias, auto clamped, auto whole) __attribute__((always_inline)) {
@@ -165,7 +274,7 @@ gemm_pair_kernel(PairArgs a) {
 #pragma unroll
         for (int t = 0; t < TOUT; ++t) {
             const int col = n0 + 16 * (TOUT * wn + t) + 4 * g;
-            float bv[4], bu[4];
+            float bv[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
             if constexpr (BIAS) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -181,8 +290,12 @@ gemm_pair_kernel(PairArgs a) {
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    v[e] = BIAS ? acc[t][u][e] + bv[e] : acc[t][u][e];
-                    if constexpr (GATED) v[e] = a.pair.of_short<decltype(clamped)::value>(v[e], BIAS ? acc[t + TOUT][u][e] + bu[e] : acc[t + TOUT][u][e]);
+                    auto sum = [&](float x, float b) __attribute__((always_inline)) {
+                        if constexpr (SCALED) return fmaf(x, rinv[u], BIAS ? b : 0.f);
+                        else return BIAS ? x + b : x;
+                    };
+                    v[e] = sum(acc[t][u][e], bv[e]);
+                    if constexpr (GATED) v[e] = a.pair.of_short<decltype(clamped)::value>(v[e], sum(acc[t + TOUT][u][e], bu[e]));
                 }
                 bf16* to = a.C + (size_t)row * a.ldc + col;
                 if (WHOLE || (a.wide_stores && col + 3 < a.I)) {
@@ -255,23 +368,33 @@ extern "C" int mv_gemm_pair_shape(int M, int N, int K, int units) {
     return M == padded ? p.tile : pair_tile(M, N, K, units).tile;
 }
 
-// C [M, I] bf16 (pitch ldc) = pair(A Wg^T (+ bias), A Wu^T (+ bias)) for the packed weight [N = 2 I, K]: K a multiple of 64, A and W at
-// 16-byte addresses, pitch lda a multiple of eight. `tile`: as mv_gemm_pair_shape says, or another of 64, 128, 192, 256 rows by 64, 128, 192.
-extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* bias, void* C, long ldc, int M, int N, int K, float limit, float slope,
-                            int tile, hipStream_t stream) {
-    MV_REQUIRE(M > 0 && N > 0 && K > 0 && K % GT_KC == 0 && N % 2 == 0, "gemm_pair: bad sizes M=%d N=%d K=%d", M, N, K);
-    MV_REQUIRE(A && W && C && lda >= K && lda % 8 == 0 && ((uintptr_t)A | (uintptr_t)W) % 16 == 0 && ldc >= N / 2,
-               "gemm_pair: operands not aligned or pitches too small");
-    MV_REQUIRE(mv_gemm_pair_reaches(lda, N, K), "gemm_pair: rows %ld apart or a weight of %d x %d are too long", lda, N, K);
-    const int bm = tile >> 16, bn = tile & 0xffff;
-    MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 128 || bn == 192), "gemm_pair: no tile of %d x %d", bm, bn);
-    const int tiles_m = (M + bm - 1) / bm, tiles_n = (N / 2 + bn / 2 - 1) / (bn / 2), by_columns = M > N;
+static int check_pair(const char* what, const void* A, long lda, const void* W, int M, int N, int K) {
+    MV_REQUIRE(M > 0 && N > 0 && K > 0 && K % GT_KC == 0, "%s: bad sizes M=%d N=%d K=%d", what, M, N, K);
+    MV_REQUIRE(A && W && lda >= K && lda % 8 == 0 && ((uintptr_t)A | (uintptr_t)W) % 16 == 0, "%s: operands not aligned or pitches too small", what);
+    MV_REQUIRE(mv_gemm_pair_reaches(lda, N, K), "%s: rows %ld apart or a weight of %d x %d are too long", what, lda, N, K);
+    return 0;
+}
+
+// the tile's sides, and how an XCD's run goes through the tiles
+static int place_tiles(const char* what, PairArgs& a, int N, bool gated, int bm, int bn, dim3& grid) {
+    const int wide = gated ? bn / 2 : bn, tiles_m = (a.M + bm - 1) / bm, tiles_n = (a.I + wide - 1) / wide;
     const long tiles = (long)tiles_m * tiles_n;
-    MV_REQUIRE(tiles < (1L << 30), "gemm_pair: too many tiles");
-    const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N / 2, K, (int)tiles,
-                     by_columns ? tiles_n : tiles_m, by_columns, ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{limit, slope}};
-    const dim3 grid((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
-#define GP_LAUNCH(WM, WN, SA, SB) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, SA, SB, true>), grid, dim3(512), 0, stream, a)
+    MV_REQUIRE(tiles < (1L << 30), "%s: too many tiles", what);
+    a.tiles = (int)tiles;
+    a.by_columns = a.M > N;
+    a.fast = a.by_columns ? tiles_n : tiles_m;
+    a.wide_stores = a.ldc % 4 == 0 && (uintptr_t)a.C % 8 == 0;
+    grid = dim3((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
+    return 0;
+}
+
+template <int FORM>
+static int launch_pair(const char* what, PairArgs& a, int N, int tile, hipStream_t stream) {
+    const int bm = tile >> 16, bn = tile & 0xffff;
+    MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 128 || bn == 192), "%s: no tile of %d x %d", what, bm, bn);
+    dim3 grid;
+    if (place_tiles(what, a, N, true, bm, bn, grid)) return 1;
+#define GP_LAUNCH(WM, WN, SA, SB) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, SA, SB, FORM>), grid, dim3(512), 0, stream, a)
     if (bn == 192) {
         if (bm == 256) GP_LAUNCH(4, 6, 2, 4);
         else if (bm == 192) GP_LAUNCH(3, 6, 3, 3);
@@ -289,7 +412,17 @@ extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* 
         else GP_LAUNCH(1, 2, 4, 4);
     }
 #undef GP_LAUNCH
-    return mv_check_launch("gemm_pair");
+    return mv_check_launch(what);
+}
+
+// C [M, I] bf16 (pitch ldc) = pair(A Wg^T (+ bias), A Wu^T (+ bias)) for the packed weight [N = 2 I, K]: K a multiple of 64, A and W at
+// 16-byte addresses, pitch lda a multiple of eight. `tile`: as mv_gemm_pair_shape says, or another of 64, 128, 192, 256 rows by 64, 128, 192.
+extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* bias, void* C, long ldc, int M, int N, int K, float limit, float slope,
+                            int tile, hipStream_t stream) {
+    if (check_pair("gemm_pair", A, lda, W, M, N, K)) return 1;
+    MV_REQUIRE(C && N % 2 == 0 && ldc >= N / 2, "gemm_pair: N=%d is odd or ldc=%ld too small", N, ldc);
+    PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N / 2, K, 0, 0, 0, 0, GatedPair{limit, slope}};
+    return launch_pair<PAIR_GATED>("gemm_pair", a, N, tile, stream);
 }
 
 // Columns of the plain product's tiles, and its time in us with tiles of bm x bn in one round, 0.05 apart from the measured ones (standard
@@ -325,22 +458,13 @@ extern "C" int mv_gemm_round_shape(int M, int N, int K, int units) {
     return M == padded ? p.tile : round_tile(M, N, K, units).tile;
 }
 
-// C [M, N] bf16 (pitch ldc) = A W^T (+ bias), operands as above. `tile`: 64 to 256 rows by 64, 96, 128, 192 columns.
-extern "C" int mv_gemm_round(const void* A, long lda, const void* W, const void* bias, void* C, long ldc, int M, int N, int K, int tile,
-                             hipStream_t stream) {
-    MV_REQUIRE(M > 0 && N > 0 && K > 0 && K % GT_KC == 0, "gemm_round: bad sizes M=%d N=%d K=%d", M, N, K);
-    MV_REQUIRE(A && W && C && lda >= K && lda % 8 == 0 && ((uintptr_t)A | (uintptr_t)W) % 16 == 0 && ldc >= N,
-               "gemm_round: operands not aligned or pitches too small");
-    MV_REQUIRE(mv_gemm_pair_reaches(lda, N, K), "gemm_round: rows %ld apart or a weight of %d x %d are too long", lda, N, K);
+template <int FORM>
+static int launch_round(const char* what, PairArgs& a, int tile, hipStream_t stream) {
     const int bm = tile >> 16, bn = tile & 0xffff;
-    MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 96 || bn == 128 || bn == 192), "gemm_round: no tile of %d x %d", bm, bn);
-    const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn, by_columns = M > N;
-    const long tiles = (long)tiles_m * tiles_n;
-    MV_REQUIRE(tiles < (1L << 30), "gemm_round: too many tiles");
-    const PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N, K, (int)tiles,
-                     by_columns ? tiles_n : tiles_m, by_columns, ldc % 4 == 0 && (uintptr_t)C % 8 == 0, GatedPair{0.f, 1.f}};
-    const dim3 grid((unsigned)((tiles + GT_XCDS - 1) / GT_XCDS * GT_XCDS));
-#define GR_LAUNCH(WM, WN, SA, SB) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, SA, SB, false>), grid, dim3(512), 0, stream, a)
+    MV_REQUIRE(bm >= 64 && bm <= 256 && bm % 64 == 0 && (bn == 64 || bn == 96 || bn == 128 || bn == 192), "%s: no tile of %d x %d", what, bm, bn);
+    dim3 grid;
+    if (place_tiles(what, a, a.I, false, bm, bn, grid)) return 1;
+#define GR_LAUNCH(WM, WN, SA, SB) hipLaunchKernelGGL((gemm_pair_kernel<WM, WN, SA, SB, FORM>), grid, dim3(512), 0, stream, a)
     if (bn == 192) {
         if (bm == 256) GR_LAUNCH(4, 6, 2, 4);
         else if (bm == 192) GR_LAUNCH(3, 6, 3, 3);
@@ -363,5 +487,85 @@ extern "C" int mv_gemm_round(const void* A, long lda, const void* W, const void*
         else GR_LAUNCH(1, 2, 4, 4);
     }
 #undef GR_LAUNCH
-    return mv_check_launch("gemm_round");
+    return mv_check_launch(what);
+}
+
+// C [M, N] bf16 (pitch ldc) = A W^T (+ bias), operands as above. `tile`: 64 to 256 rows by 64, 96, 128, 192 columns.
+extern "C" int mv_gemm_round(const void* A, long lda, const void* W, const void* bias, void* C, long ldc, int M, int N, int K, int tile,
+                             hipStream_t stream) {
+    if (check_pair("gemm_round", A, lda, W, M, N, K)) return 1;
+    MV_REQUIRE(C && ldc >= N, "gemm_round: ldc=%ld too small for N=%d", ldc, N);
+    PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, N, K, 0, 0, 0, 0, GatedPair{0.f, 1.f}};
+    return launch_round<PAIR_PLAIN>("gemm_round", a, tile, stream);
+}
+
+// ---- the norms between two products taken apart (see gemm_deep.hip), for prompts and steps with prompts in them, 129 to 1,024 rows:
+// there an add and a norm of their own are 3.5 to 4.5 us, most of it what any kernel costs. What serves is decided by the rows of a step's
+// class, and the sums of squares are added in an order that the rows there are have no part in.
+// us, weights of the 0.6B sizes that take turns, before / with it: output projection and add + norm, 256 rows 10.2 / 7.2, 512 12.9 / 9.1, 552 15.2 / 12.7,
+// 1,000 16.1 / 13.9; down and add + norm 12.1 / 8.8, 15.8 / 11.2, 18.8 / 17.1, 20.1 / 17.8; the gated pair 9.5 / 10.0, 12.5 / 12.9, 12.9 / 13.6,
+// 17.5 / 18.3; queries, keys and values, 512 rows 10.8 / 10.1, 552 14.0 / 12.1, 1,000 14.3 both. With more rows the sums' way through memory
+// at the products' ends costs what the norm's kernel does: 2,048 rows, all four, 98.5 / 98.4.
+#define PN_MIN_ROWS 128
+#define PN_MAX_ROWS 1024
+
+// Behind the norm: the tile of gemm_pair.hip, or 1 for a tile of gemm_deep.hip, or 0: not served.
+static int behind_norm_tile(int M, int N, int K, bool gated, int units) {
+    if (M <= PN_MIN_ROWS || M > PN_MAX_ROWS || N <= 0 || K <= 0 || K % GT_KC || (gated && N % 2)) return 0;
+    const int padded = mv_class_rows(M);
+    if (padded > PN_MAX_ROWS) return 0;
+    if (mv_gemm_deep_shape(padded, N, K, gated)) return 1;
+    if (gated) return mv_gemm_pair_shape(M, N, K, units);
+    return round_tile(padded, N, K, units).tile ? round_tile(M, N, K, units).tile : 0;
+}
+extern "C" int mv_gemm_behind_norm_serves(int M, int N, int K, int gated, int units) { return behind_norm_tile(M, N, K, gated != 0, units) != 0; }
+
+// C [M, N] bf16 = A W^T / rms (+ bias), or the gated pair of it [M, N / 2], rms[m] = sqrt(sum_p partial[m][p] / K + eps); operands as above,
+// partial at a 16-byte address, P a multiple of four.
+extern "C" int mv_gemm_behind_norm(const void* A, long lda, const void* W, const void* bias, void* C, long ldc, int M, int N, int K, int gated, float limit,
+                                   float slope, const float* partial, int P, float eps, hipStream_t stream) {
+    if (check_pair("gemm_behind_norm", A, lda, W, M, N, K)) return 1;
+    MV_REQUIRE(C && (!gated || N % 2 == 0) && ldc >= (gated ? N / 2 : N), "gemm_behind_norm: N=%d is odd or ldc=%ld too small", N, ldc);
+    MV_REQUIRE(partial != nullptr && (uintptr_t)partial % 16 == 0 && P > 0 && P % 4 == 0 && eps > 0.f,
+               "gemm_behind_norm: the partial sums (P=%d, in fours) or eps are missing or not aligned", P);
+    const int tile = behind_norm_tile(M, N, K, gated != 0, mv_compute_units());
+    MV_REQUIRE(tile != 0, "gemm_behind_norm: M=%d N=%d K=%d is not served", M, N, K);
+    if (tile == 1)
+        return mv_gemm_deep(A, lda, W, bias, C, ldc, MV_BF16, M, N, K, gated, partial, P, eps, limit, slope, 0, mv_gemm_deep_shape(mv_class_rows(M), N, K, gated),
+                            stream);
+    PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, (bf16*)C, ldc, M, gated ? N / 2 : N, K, 0, 0, 0, 0, GatedPair{limit, slope},
+               const_cast<float*>(partial), P, eps};
+    return gated ? launch_pair<PAIR_GATED_SCALED>("gemm_behind_norm", a, N, tile, stream) : launch_round<PAIR_PLAIN_SCALED>("gemm_behind_norm", a, tile, stream);
+}
+
+extern "C" int mv_gemm_into_norm_rows() { return PN_MAX_ROWS; }
+// In front of it: partial sums a row, 0: not served. One round of tiles of 64 x 64 where gemm_deep.hip takes no more rows.
+extern "C" int mv_gemm_into_norm_parts(int M, int N, int K, int units) {
+    if (M <= PN_MIN_ROWS || M > PN_MAX_ROWS || N <= 0 || K <= 0 || N % 128 || K % GT_KC || (long)N * K >= 8L << 20) return 0;
+    const int padded = mv_class_rows(M);
+    if (padded > PN_MAX_ROWS) return 0;
+    if (mv_gemm_deep_shape(padded, N, K, 0)) return mv_gemm_deep_fold_parts(N);
+    return (long)((padded + 63) / 64) * (N / 64) <= units ? N / 32 : 0;
+}
+
+// resid [M, N] += bf16(A W^T (+ bias)), weighted = bf16(resid * norm_weight (+ 1 with unit_offset)), partial [M, P] = sums of resid^2 over N / P columns each.
+extern "C" int mv_gemm_into_norm(const void* A, long lda, const void* W, const void* bias, float* resid, long ldr, const void* norm_weight,
+                                 int norm_weight_dtype, int unit_offset, void* weighted, long ldw, float* partial, int P, int M, int N, int K,
+                                 hipStream_t stream) {
+    if (check_pair("gemm_into_norm", A, lda, W, M, N, K)) return 1;
+    MV_REQUIRE(P > 0 && P == mv_gemm_into_norm_parts(M, N, K, mv_compute_units()), "gemm_into_norm: M=%d N=%d K=%d is not served with %d partial sums", M, N, K, P);
+    if (mv_gemm_deep_shape(mv_class_rows(M), N, K, 0))
+        return mv_gemm_deep_fold(A, lda, W, bias, resid, ldr, norm_weight, norm_weight_dtype, unit_offset, weighted, ldw, partial, P, M, N, K,
+                                 mv_gemm_deep_shape(mv_class_rows(M), N, K, 0), stream);
+    MV_REQUIRE(resid != nullptr && weighted != nullptr && partial != nullptr && ldr >= N && ldw >= N && ldr % 4 == 0 && ldw % 4 == 0
+               && (uintptr_t)resid % 16 == 0 && (uintptr_t)weighted % 8 == 0,
+               "gemm_into_norm: the residual, the weighted rows or the partial sums are missing or not aligned (ldr=%ld, ldw=%ld)", ldr, ldw);
+    MV_REQUIRE(mv_valid_dtype(norm_weight_dtype) && norm_weight != nullptr && (uintptr_t)norm_weight % 16 == 0,
+               "gemm_into_norm: the norm weight is missing, of an unknown type or not 16-byte aligned");
+    PairArgs a{(const bf16*)A, lda, (const bf16*)W, (const bf16*)bias, nullptr, 0, M, N, K, 0, 0, 0, 0, GatedPair{0.f, 1.f}, partial, P, 0.f,
+               resid, ldr, WeightPtr{norm_weight, norm_weight_dtype}, unit_offset, (bf16*)weighted, ldw};
+    dim3 grid;
+    if (place_tiles("gemm_into_norm", a, N, false, 64, 64, grid)) return 1;
+    hipLaunchKernelGGL((gemm_pair_kernel<1, 2, 4, 4, PAIR_FOLD>), grid, dim3(512), 0, stream, a);
+    return mv_check_launch("gemm_into_norm");
 }

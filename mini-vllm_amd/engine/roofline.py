@@ -73,6 +73,8 @@ KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_attention_latent_prompt": (r"\battention_latent_prompt_kernel", None, 1),
     "mv_gemm_pair": (r"\bgemm_pair_kernel", None, 1),
     "mv_gemm_round": (r"\bgemm_pair_kernel", None, 1),
+    "mv_gemm_behind_norm": (r"\bgemm_(deep|pair)_kernel", None, 1),
+    "mv_gemm_into_norm": (r"\bgemm_(deep|pair)_kernel", None, 1),
     "mv_latent_expand": (r"\blatent_expand_kernel", None, 1),
     "mv_attention_latent_heads": (r"\battention_latent_heads_kernel", None, 1),
     "mv_attention_latent_mfma": (r"\battention_latent_mfma_kernel", None, 1),

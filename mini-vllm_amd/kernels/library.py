@@ -244,6 +244,15 @@ _OPTIONAL_SIGNATURES = {
     "mv_gemm_round_shape": (c_int, [c_int, c_int, c_int, c_int]),
     # A, lda, W, bias, C, ldc, M, N, K, tile, stream
     "mv_gemm_round": (c_int, [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_int, c_void_p]),
+    "mv_gemm_behind_norm_serves": (c_int, [c_int, c_int, c_int, c_int, c_int]),
+    # A, lda, W, bias, C, ldc, M, N, K, gated, limit, slope, partial, P, eps, stream
+    "mv_gemm_behind_norm": (c_int, [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p,
+                                    c_int, c_float, c_void_p]),
+    "mv_gemm_into_norm_rows": (c_int, []),
+    "mv_gemm_into_norm_parts": (c_int, [c_int, c_int, c_int, c_int]),
+    # A, lda, W, bias, resid, ldr, norm weight, its dtype, unit_offset, weighted, ldw, partial, P, M, N, K, stream
+    "mv_gemm_into_norm": (c_int, [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_int, c_int, c_void_p, c_long, c_void_p, c_int,
+                                  c_int, c_int, c_int, c_void_p]),
     "mv_moe_pairs_shape": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "mv_moe_pairs_ints": (c_long, [c_int, c_int, c_int, c_int]),
     # x, ldx, n, hidden, w_gate_up, w_down, n_real, identity, F, FS, ids, weights, top, dense, ld_dense, ints, act, out, y, ldy,

@@ -2483,6 +2483,10 @@ class Ops:
         lda = a.stride(0) if M > 1 else K
         ldc = out.stride(0) if M > 1 else N
         fast = self.use_fast_kernels and not exact and wcode == DTYPE_BF16
+        if fast and fold is not None and not square_relu:
+            rows = self._gemm_into_norm(a, w, bias, fold, out)
+            if rows is not None:
+                return rows
         if (fast and self.prefers_library(M, N, K) and self._library_serves(out)
                 and self._library_allowed(M, N, K, bias is not None, out.dtype)
                 and self._library_product(a, w, bias, out)):
@@ -2790,6 +2794,10 @@ class Ops:
         slower). Where both this and the fused add + norm + product kernel could serve (up to 16
         rows), this is taken: the product behind reads finished bf16 rows instead of normalising
         them in every workgroup (0.6B sizes: a step of 1, 8, 16 sequences 5, 3, 4 % faster)."""
+        if rows > SKINNY_WIDE_MAX_M and consumer is not None:      # prompts, as far as gemm_pair.hip says
+            n, k, gated = consumer
+            return (self.use_fast_kernels and self.use_tiled_gemm and self.dtype == torch.bfloat16 and self.lib.has("mv_gemm_behind_norm")
+                    and k == width and bool(self.lib.dll.mv_gemm_behind_norm_serves(rows, n, k, int(gated), self.compute_units)))
         if not (self.use_fast_kernels and self.dtype == torch.bfloat16 and self.lib.has("mv_gemm_skinny_fold")
                 and self.lib.has("mv_gemm_skinny_scaled") and 0 < rows <= SKINNY_WIDE_MAX_M and width % 4 == 0):
             return False
@@ -2800,10 +2808,37 @@ class Ops:
                 and not (self.wants_mid(rows, n, k) and self.lib.has("mv_gemm_mid"))
                 and not self.prefers_library(rows, n, k, gated=gated))
 
-    def _fold_serves(self, fold, out: torch.Tensor, M: int, N: int) -> bool:
+    def most_fold_rows(self, width: int) -> int:
+        """The rows of the largest step whose norms of this width may be folded (``can_fold_norm``)."""
+        if not (self.use_fast_kernels and self.dtype == torch.bfloat16):
+            return 0
+        if self.use_tiled_gemm and self.lib.has("mv_gemm_into_norm_rows") and width % 128 == 0:
+            return int(self.lib.dll.mv_gemm_into_norm_rows())
+        return SKINNY_WIDE_MAX_M
+
+    def _gemm_into_norm(self, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], fold, out: torch.Tensor) -> Optional["WeightedRows"]:
+        """The product in front of a prompt's residual add and norm, both in its epilogue (gemm_pair.hip, whose ``mv_gemm_into_norm_parts``
+        says for which sizes); None, with nothing done, where they stay apart."""
+        (M, K), N = a.shape, w.shape[0]
+        if M <= SKINNY_WIDE_MAX_M or not self.use_tiled_gemm or not self.lib.has("mv_gemm_into_norm"):
+            return None
+        P = int(self.lib.dll.mv_gemm_into_norm_parts(M, N, K, self.compute_units))
+        if (not P or a.stride(0) % 8 or a.data_ptr() % 16 or w.data_ptr() % 16 or not self.lib.dll.mv_gemm_pair_reaches(a.stride(0), N, K)
+                or not self._fold_fits(fold, out, M, N)):
+            return None
         resid = fold.stream.resid
-        return (M <= SKINNY_WIDE_MAX_M and out.dtype == self.dtype and self.lib.has("mv_gemm_skinny_fold")
-                and resid.dtype == torch.float32 and resid.shape == (M, N) and resid.stride(1) == 1
+        self._note("mv_gemm_into_norm", M * K * 2 + N * K * 2 + M * N * (8 + 2) + M * P * 4, 2 * M * N * K + 4 * M * N)
+        self.lib.call("mv_gemm_into_norm", a.data_ptr(), a.stride(0), w.data_ptr(), _ptr(bias), resid.data_ptr(), resid.stride(0), fold.weight.data_ptr(),
+                      _weight_code(fold.weight, "norm weight"), int(fold.unit_offset), fold.weighted.data_ptr(), fold.weighted.stride(0),
+                      fold.partial.data_ptr(), P, M, N, K, self._stream())
+        return WeightedRows(self, fold, P)
+
+    def _fold_serves(self, fold, out: torch.Tensor, M: int, N: int) -> bool:
+        return M <= SKINNY_WIDE_MAX_M and self.lib.has("mv_gemm_skinny_fold") and self._fold_fits(fold, out, M, N)
+
+    def _fold_fits(self, fold, out: torch.Tensor, M: int, N: int) -> bool:
+        resid = fold.stream.resid
+        return (out.dtype == self.dtype and resid.dtype == torch.float32 and resid.shape == (M, N) and resid.stride(1) == 1
                 and fold.weight.numel() == N and fold.weight.is_contiguous()
                 and fold.weighted.shape == (M, N) and fold.weighted.stride(1) == 1 and fold.weighted.dtype == self.dtype
                 and N % 4 == 0 and (M == 1 or (resid.stride(0) % 4 == 0 and fold.weighted.stride(0) % 4 == 0))
@@ -2817,6 +2852,8 @@ class Ops:
         mean square; False if the shape is not taken (nothing has been done then)."""
         a = rows.weighted
         M, K = a.shape
+        if M > SKINNY_WIDE_MAX_M:
+            return self._gemm_behind_norm(rows, w, out, bias, swiglu, limit, slope)
         if (not self.use_fast_kernels or not self.lib.has("mv_gemm_skinny_scaled") or M == 0
                 or not self.streams_rows(M, w.shape[0], K)
                 or w.dtype != torch.bfloat16 or not w.is_contiguous() or w.shape[1] != K or K % 32
@@ -2847,6 +2884,24 @@ class Ops:
         self.lib.call("mv_gemm_skinny_scaled", a.data_ptr(), a.stride(0) if M > 1 else K, w.data_ptr(), _ptr(bias),
                       out.data_ptr(), out.stride(0) if M > 1 else N, rows.partial.data_ptr(), rows.P, rows.eps, M, N, K,
                       int(swiglu), float(limit), float(slope), self._stream())
+        return True
+
+    def _gemm_behind_norm(self, rows: "WeightedRows", w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor], gated: bool,
+                          limit: float, slope: float) -> bool:
+        """The same for a prompt's rows (gemm_pair.hip)."""
+        a = rows.weighted
+        (M, K), N = a.shape, w.shape[0]
+        if (not self.use_fast_kernels or not self.use_tiled_gemm or not self.lib.has("mv_gemm_behind_norm") or w.dtype != torch.bfloat16
+                or not self.lib.dll.mv_gemm_behind_norm_serves(M, N, K, int(gated), self.compute_units) or not w.is_contiguous() or w.shape[1] != K
+                or a.stride(1) != 1 or a.stride(0) % 8 or a.data_ptr() % 16 or w.data_ptr() % 16
+                or not self.lib.dll.mv_gemm_pair_reaches(a.stride(0), N, K) or rows.P % 4 or rows.partial.data_ptr() % 16
+                or out.shape != (M, N // 2 if gated else N) or out.stride(1) != 1 or out.dtype != torch.bfloat16
+                or (bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != N))):
+            return False
+        rows.take()
+        self._note("mv_gemm_behind_norm", self._size(a, w, out) + M * rows.P * 4, 2 * M * N * K)
+        self.lib.call("mv_gemm_behind_norm", a.data_ptr(), a.stride(0), w.data_ptr(), _ptr(bias), out.data_ptr(), out.stride(0), M, N, K, int(gated),
+                      float(limit), float(slope), rows.partial.data_ptr(), rows.P, rows.eps, self._stream())
         return True
 
     def scale_rows(self, weighted: torch.Tensor, partial: torch.Tensor, P: int, eps: float, out: torch.Tensor) -> None:

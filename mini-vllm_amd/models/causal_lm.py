@@ -185,7 +185,7 @@ class CausalLM:
         return tuple(m.step_path(lens, starts) for m in self._choosers)
 
     def reserve(self, tokens: int, seqs: int, portions: bool = True) -> None:
-        """Sizes the scratch of mixers and feed-forwards for any cut of up to ``tokens`` tokens into up to ``seqs`` sequences
+        """Sizes the scratch of mixers, feed-forwards and blocks for any cut of up to ``tokens`` tokens into up to ``seqs`` sequences
         (without ``portions``: of one token each)."""
         for mixer in self.mixers:
             if mixer is not None and portions:
@@ -193,6 +193,9 @@ class CausalLM:
         for ffn in self.ffns:
             if ffn is not None:
                 ffn.reserve(tokens)
+        for block in self.blocks:
+            if hasattr(block, "reserve"):
+                block.reserve(tokens)
 
     # ------------------------------------------------------------------------------------
     def forward(self, ctx) -> torch.Tensor:

@@ -38,6 +38,11 @@ class PreNormBlock(Block):
 
     accepts_next_norm = True
 
+    def reserve(self, tokens: int) -> None:
+        for norm in (self.norm_mixer, self.norm_ffn):
+            if hasattr(norm, "reserve"):
+                norm.reserve(tokens)
+
     def entry_norm(self) -> Norm:
         return self.norm_mixer
 

@@ -73,11 +73,17 @@ class RMSNorm(Norm):
         n, size = stream.resid.shape[0], self.spec.size
         if consumer is None or consumer[1] != size or not self.rt.ops.can_fold_norm(n, size, consumer):
             return None
-        ws = self.rt.workspace
-        return NormFold(self, stream, self.weight, self.spec.eps, self.spec.unit_offset,
-                        ws.get("fold.weighted", (n, size), self.rt.dtype),
-                        ws.get("fold.partial", (n * ((size + 3) // 4),), torch.float32),
-                        ws.get("normed", (n, size), self.rt.dtype))
+        return NormFold(self, stream, self.weight, self.spec.eps, self.spec.unit_offset, *self._fold_scratch(n))
+
+    def _fold_scratch(self, n: int):
+        ws, size = self.rt.workspace, self.spec.size
+        return (ws.get("fold.weighted", (n, size), self.rt.dtype), ws.get("fold.partial", (n * ((size + 3) // 4),), torch.float32),
+                ws.get("normed", (n, size), self.rt.dtype))
+
+    def reserve(self, tokens: int) -> None:
+        n = min(tokens, self.rt.ops.most_fold_rows(self.spec.size))
+        if n > 0:
+            self._fold_scratch(n)
 
     def pending(self, stream: HiddenStream, ctx):
         """Deferred when the step is small enough for the fused add + norm + product kernel; rows that

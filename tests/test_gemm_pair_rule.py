@@ -86,3 +86,17 @@ def test_offsets_of_a_tile_fit_into_32_bits(lib, lda, n, k, reaches):
     lib.mv_gemm_pair_reaches.argtypes = [ctypes.c_long, ctypes.c_int, ctypes.c_int]
     assert lib.mv_gemm_pair_reaches(lda, n, k) == reaches
     assert not reaches or max(255 * lda, (n - 1) * k) * 2 + 128 < 1 << 32
+
+
+@pytest.mark.parametrize("n, k, gated", [(1024, 2048, None), (1024, 3072, None), (384, 64, None), (2048, 1024, None), (6144, 1024, 1), (2048, 1024, 1), (4096, 1024, 0),
+                                         (5184, 1024, 0), (592, 1024, 0)])
+@pytest.mark.parametrize("classes", [GRAPH_BUCKETS, TOKEN_BUCKETS], ids=["decode", "prompt"])
+def test_a_class_has_one_way_through_a_norm(lib, n, k, gated, classes):
+    serves = (lambda m: lib.mv_gemm_into_norm_parts(m, n, k, 256)) if gated is None else lambda m: lib.mv_gemm_behind_norm_serves(m, n, k, gated, 256)
+    for rows in range(97, min(classes[-1], 1200) + 1):
+        assert serves(rows) == serves(next(b for b in classes if b >= rows)), rows
+
+
+def test_sizes_whose_norm_stays_apart(lib):
+    assert all(lib.mv_gemm_into_norm_parts(m, n, k, 256) == 0 for m, n, k in [(128, 1024, 2048), (1025, 1024, 2048), (300, 4096, 4096), (300, 1088, 2048), (300, 1024, 2000)])
+    assert all(lib.mv_gemm_behind_norm_serves(*a, 256) == 0 for a in [(128, 4096, 1024, 0), (1025, 4096, 1024, 0), (600, 24576, 4096, 1), (1024, 20480, 1024, 0), (300, 6145, 1024, 1)])

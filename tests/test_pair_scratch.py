@@ -67,3 +67,19 @@ def test_the_librarys_workspace_is_there_before_the_dry_run():
         ops.use_library_gemm, ops._lt_work = False, None             # (the float32 engine has no such product)
         Ops.reserve_library(ops, torch.device("cpu"))
         assert ops._lt_work is None
+
+
+def test_scratch_of_folded_norms_is_there_before_the_dry_run():
+    """The largest step folds no norm, smaller ones do."""
+    from minivllm_amd.parts import NORMS, RMSNormSpec
+    from minivllm_amd.parts.block import PreNormBlock
+    most = 1024
+    ops = SimpleNamespace(most_fold_rows=lambda width: most, can_fold_norm=lambda n, size, consumer: n <= most)
+    rt = SimpleNamespace(dtype=torch.bfloat16, ops=ops, workspace=Workspace(torch.device("cpu")))
+    norm = NORMS.get("rmsnorm")(RMSNormSpec(size=128), {"weight": torch.ones(128)}, rt)
+    block = PreNormBlock(None, {"mixer": norm, "ffn": norm}, None, SimpleNamespace())
+    block.reserve(4096)
+    rt.workspace.frozen = True
+    for n in (1, 97, 512, most):
+        assert norm.fold(SimpleNamespace(resid=torch.zeros(n, 128)), None, (64, 128, False)) is not None
+    assert norm.fold(SimpleNamespace(resid=torch.zeros(most + 1, 128)), None, (64, 128, False)) is None
