@@ -20,10 +20,11 @@
 // What bounded these before was one chain of about 0.2 us a token for every (request, head, 16 columns), 64 workgroups
 // for a head count of 16; the chunks' work is spread over every compute unit and the chain is one product of DK x DK with
 // DK x 16 a chunk. Measured on one prompt of
-// 2,048 tokens, 16 heads of 64 x 64 (us, scan against the two kernels here): GENERAL 438 -> 48 + 42, GATED 477 -> 40 + 42,
-// SUM with 65 columns 411 -> 30 + 26; CHANNEL on prompts of 941 and 483 tokens 215 -> 36 + 23. The chunk kernel waits for
-// its own phases (eight waves a workgroup hide that best: four took 90, 49, 36 and 45), the walk for a round of matrix unit,
-// LDS and barrier a chunk, 0.6 us (0.4 with nothing read or written behind the first steps).
+// 2,048 tokens, 16 heads of 64 x 64 (us, scan against the two kernels here): GENERAL 438 -> 48 + 37, GATED 477 -> 40 + 37,
+// SUM with 65 columns 411 -> 30 + 26; CHANNEL on prompts of 941 and 483 tokens 215 -> 36 + 21. The chunk kernel waits for
+// its own phases (eight waves a workgroup hide that best: four took 90, 49, 36 and 45; of GENERAL's 48 us the loads are 12, the products inside
+// the runs 10, what makes T, W and U 9 and the maps, which are 50 MB to write, 16), the walk for a round of matrix unit, LDS and barrier a chunk,
+// 0.53 us.
 //
 // Layouts are those of the scans: states [..][H][DV][DK] (a head's matrix column by column), out [n][H][DV]. M [chunks][H][DK][DK],
 // N [chunks][H][DV][DK] and Q [n][H][DK] pass from one kernel to the other in the order of quad_of.
@@ -468,8 +469,11 @@ delta_chunk_walk_kernel(DeltaChunkArgs A, float* __restrict__ state, const int* 
     const int v = v0 + i;
     const bool live = v < DV;
     const int vc = live ? v : 0;
-    auto unit_of = [&](int c) { return (size_t)(c0 + (c < chunks ? c : chunks - 1)) * H + head; };   // (chunk, head)
+    const int steps = (chunks + DEPTH - 1) / DEPTH * DEPTH;
 
+    // A step: what the step before left in LDS is asked for, then, while it comes, what a later step reads of memory, into the registers that
+    // the step before has used; then the products, and the workgroup meets. (Asked for at a step's end, with addresses made anew from the chunk's number, it
+    // stood between the state and the barrier: 2,048 tokens, 16 heads of 64 42 -> 37 us, 8 heads of 128 73 -> 66, two requests of 4,096 86 -> 76.)
     if (wave < KT) {
         float* st = state + (((size_t)state_slots[seq] * H + head) * DV + vc) * DK + 16 * wave + 4 * g;
         float4 s = *reinterpret_cast<const float4*>(st);
@@ -479,30 +483,39 @@ delta_chunk_walk_kernel(DeltaChunkArgs A, float* __restrict__ state, const int* 
         float decay[DEPTH];
         const uint32_t m_at = 4u * quad_of(wave, 16, 0, DK, i, g);
         const uint32_t n_at = live ? 4u * quad_of(v0 / 16, min(16, DV - v0), wave, DK, i, g) : NOWHERE;
-        auto fetch = [&](int d, int c) __attribute__((always_inline)) {
-            const size_t unit = unit_of(c);
+        const size_t unit0 = (size_t)c0 * H + head, step_m = (size_t)H * (READ ? DK * DK : 1), step_n = (size_t)H * DV * DK;
+        const float *next_m = A.M + unit0 * (READ ? DK * DK : 1), *next_n = A.N + unit0 * DV * DK;
+        int left = chunks - 1;                                              // chunks behind the next one to ask for
+        auto fetch = [&](int d) __attribute__((always_inline)) {
             if constexpr (READ) {
-                const BufferWindow w(A.M + unit * DK * DK, 4u * DK * DK);
+                const BufferWindow w(next_m, 4u * DK * DK);
 #pragma unroll
                 for (int k = 0; k < KT; ++k) m[d][k] = w.load4(m_at, 1024 * k);
             } else {
-                decay[d] = A.M[unit];
+                decay[d] = *next_m;
             }
-            nn[d] = BufferWindow(A.N + unit * DV * DK, 4u * DV * DK).load4(n_at, 0);
+            nn[d] = BufferWindow(next_n, 4u * DV * DK).load4(n_at, 0);
+            next_m += left > 0 ? step_m : 0;                                // (behind the last chunk the last again)
+            next_n += left > 0 ? step_n : 0;
+            --left;
         };
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) fetch(d, d);
+        for (int d = 0; d < DEPTH - 1; ++d) fetch(d);
         __builtin_amdgcn_s_setprio(2);                                      // (the chain of the states is what the walk waits for)
         __syncthreads();
-        for (int b = 0; b < chunks; b += DEPTH) {
+        for (int b = 0; b < steps; b += DEPTH) {
 #pragma unroll
             for (int d = 0; d < DEPTH; ++d) {
                 const int c = b + d;
-                floatx4_t acc{nn[d].x, nn[d].y, nn[d].z, nn[d].w}, acc2{0.f, 0.f, 0.f, 0.f};
+                float4 sv[READ ? KT : 1];
                 if constexpr (READ) {
-                    float4 sv[KT];
 #pragma unroll
                     for (int k = 0; k < KT; ++k) sv[k] = *reinterpret_cast<const float4*>(&sS[d % 2][i][16 * k + 4 * g]);
+                }
+                fetch((d + DEPTH - 1) % DEPTH);
+                __builtin_amdgcn_sched_barrier(0);
+                floatx4_t acc{nn[d].x, nn[d].y, nn[d].z, nn[d].w}, acc2{0.f, 0.f, 0.f, 0.f};
+                if constexpr (READ) {
 #pragma unroll
                     for (int k = 0; k < KT; k += 2) {
                         mfma4(acc, m[d][k], sv[k]);
@@ -518,7 +531,6 @@ delta_chunk_walk_kernel(DeltaChunkArgs A, float* __restrict__ state, const int* 
                 const bool moves = live && c < chunks;
                 s = float4{moves ? acc[0] : s.x, moves ? acc[1] : s.y, moves ? acc[2] : s.z, moves ? acc[3] : s.w};
                 *reinterpret_cast<float4*>(&sS[(d + 1) % 2][i][16 * wave + 4 * g]) = s;
-                fetch(d, c + DEPTH);
                 __syncthreads();
             }
         }
@@ -526,41 +538,51 @@ delta_chunk_walk_kernel(DeltaChunkArgs A, float* __restrict__ state, const int* 
         __syncthreads();
     } else {
         const int ow = wave - KT, tile = ow % 2, half = ow / 2;             // 16 tokens, half of the key channels
+        const int last = len - (chunks - 1) * DC_TOKENS;                    // tokens of the last chunk
         float4 qv[DEPTH][KT / 2];
         float ov[DEPTH][4];
         // rows of a chunk behind the request's last fall outside the windows: they read zero and store nothing
-        auto rows_of = [&](int c) { return len - c * DC_TOKENS < DC_TOKENS ? len - c * DC_TOKENS : DC_TOKENS; };
         const uint32_t o_row = 4u * H * DV;
         uint32_t o_at[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) o_at[q] = half == 0 && live ? (16 * tile + 4 * g + q) * o_row + 4u * v : NOWHERE;
-        auto out_rows = [&](int c, bool some) __attribute__((always_inline)) {
-            const int cc = c < 0 ? 0 : c < chunks ? c : chunks - 1;
-            return BufferWindow(A.out + ((size_t)(begin + cc * DC_TOKENS) * H + head) * DV, some ? (rows_of(cc) - 1) * o_row + 4u * DV : 0u);
-        };
-        auto fetch = [&](int d, int c) __attribute__((always_inline)) {
-            const int cc = c < chunks ? c : chunks - 1;
-            const int count = rows_of(cc), rows = max(0, min(16, count - 16 * tile));
-            const BufferWindow w(A.Q + ((size_t)(begin + cc * DC_TOKENS) * H + (size_t)head * count) * DK, 4u * count * DK);
-            const uint32_t q_at = 4u * quad_of(tile, rows, half * (KT / 2), DK, i, g);
+        const uint32_t o_bytes = (DC_TOKENS - 1) * o_row + 4u * DV, o_last = (last - 1) * o_row + 4u * DV;
+        const int rows_last = max(0, min(16, last - 16 * tile));
+        const uint32_t q_at = 4u * quad_of(tile, 16, half * (KT / 2), DK, i, g);
+        const uint32_t q_last = 4u * quad_of(tile, rows_last, half * (KT / 2), DK, i, g);
+        const size_t step_q = (size_t)DC_TOKENS * H * DK, step_o = (size_t)DC_TOKENS * H * DV;
+        const float* next_q = A.Q + ((size_t)begin * H + (size_t)head * (chunks > 1 ? DC_TOKENS : last)) * DK;
+        const float* next_o = A.out + ((size_t)begin * H + head) * DV;
+        float* store_o = A.out + ((size_t)begin * H + head) * DV;
+        int left = chunks - 1;
+        auto fetch = [&](int d) __attribute__((always_inline)) {
+            const bool end = left <= 0;
+            const BufferWindow w(next_q, 4u * (end ? last : DC_TOKENS) * DK);
+            const uint32_t at = end ? q_last : q_at, more = end ? 64u * rows_last : 1024u;
 #pragma unroll
-            for (int k = 0; k < KT / 2; ++k) qv[d][k] = w.load4(q_at + 64 * rows * k, 0);
-            const BufferWindow o = out_rows(c, true);
+            for (int k = 0; k < KT / 2; ++k) qv[d][k] = w.load4(at + more * k, 0);
+            const BufferWindow o(next_o, end ? o_last : o_bytes);
 #pragma unroll
             for (int q = 0; q < 4; ++q) ov[d][q] = o.load(o_at[q], 0);
+            // (the last chunk's heads lie closer together)
+            next_q += end ? 0 : left == 1 ? step_q - (size_t)head * (DC_TOKENS - last) * DK : step_q;
+            next_o += end ? 0 : step_o;
+            --left;
         };
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) fetch(d, d);
+        for (int d = 0; d < DEPTH - 1; ++d) fetch(d);
         floatx4_t held{0.f, 0.f, 0.f, 0.f};                                 // this wave's half of the step before
-        auto store = [&](int c) __attribute__((always_inline)) {            // the tile of chunk c, its other half from LDS
-            const floatx4_t o = held + sO[c & 1][ow ^ 2][lane];
-            const BufferWindow w = out_rows(c, c >= 0 && c < chunks);
+        auto store = [&](int c, const floatx4_t& other) __attribute__((always_inline)) {    // the tile of chunk c
+            const floatx4_t o = held + other;
+            const bool there = c >= 0 && c < chunks;
+            const BufferWindow w(store_o, there ? (c == chunks - 1 ? o_last : o_bytes) : 0u);
 #pragma unroll
             for (int q = 0; q < 4; ++q) w.store(o[q], o_at[q]);
+            store_o += there ? step_o : 0;
         };
         sO[1][ow][lane] = held;                                             // (what the first step reads; it stores nothing)
         __syncthreads();
-        for (int b = 0; b < chunks; b += DEPTH) {
+        for (int b = 0; b < steps; b += DEPTH) {
 #pragma unroll
             for (int d = 0; d < DEPTH; ++d) {
                 const int c = b + d;
@@ -568,18 +590,20 @@ delta_chunk_walk_kernel(DeltaChunkArgs A, float* __restrict__ state, const int* 
 #pragma unroll
                 for (int k = 0; k < KT / 2; ++k)
                     sv[k] = *reinterpret_cast<const float4*>(&sS[d % 2][i][half * (DK / 2) + 16 * k + 4 * g]);
-                store(c - 1);
+                const floatx4_t other = sO[(d + 1) % 2][ow ^ 2][lane];
+                fetch((d + DEPTH - 1) % DEPTH);
+                __builtin_amdgcn_sched_barrier(0);
                 floatx4_t acc{ov[d][0], ov[d][1], ov[d][2], ov[d][3]};      // (zero for the second half)
 #pragma unroll
                 for (int k = 0; k < KT / 2; ++k) mfma4(acc, qv[d][k], sv[k]);
+                store(c - 1, other);
                 held = acc;
                 sO[d % 2][ow][lane] = acc;
-                fetch(d, c + DEPTH);
                 __syncthreads();
             }
         }
         __syncthreads();
-        store((chunks + DEPTH - 1) / DEPTH * DEPTH - 1);
+        store(steps - 1, sO[1][ow ^ 2][lane]);
     }
 }
 
