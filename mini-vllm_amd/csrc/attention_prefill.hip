@@ -56,6 +56,7 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 #define AP_WAVES 4
 #define AP_THREADS (64 * AP_WAVES)
 #define LOG2E 1.4426950408889634f
+#define AP_PART_BLOCKS 8      // blocks of 32 keys the second part of a walk has at least
 
 // Two workgroups share a compute unit (LDS and latency hiding are sized for that), so a wave may
 // use half of a SIMD's registers: the accumulators stay in the vector registers and the operand
@@ -80,16 +81,27 @@ struct SigmoidArgs {
     int first;                 // kept first positions (softmax weights with a window; 0: none)
 };
 
+// SPLIT: walks of more than `limit` blocks are cut in two, a workgroup each. Whoever is done first leaves its sums in memory and counts itself
+// in, the other adds them to its own (both rounded alike: the bits do not depend on who that is). The grid has all
+// first parts, then all second ones: a compute unit whose walks were short gets a second part. Without it a prompt is done when its last
+// tokens' walk is, at 0.55 us a block for 16 columns a wave alone on its compute unit (two share one at 0.76, and 0.7 / 1.09 for 32 columns), while the
+// work would take half as long evenly dealt out.
+struct SplitWalk {
+    int limit;                 // blocks of the first part, even; 0: whole walks
+    float* partials;           // [units * kv heads][2][columns * (D + 2)], at a 16-byte address
+    int* counters;             // [units * kv heads], zero between launches
+};
+
 // SCORED (softmax weights): capped scores, a distance bias, a sink in the denominator (see attention_score.h).
 // NARROW: units whose columns fit one tile take a walk of their own (below). Only for steps that may have such units: the
 // code beside it costs the others' walk 3 us of 43 at 2,048 tokens, though not one of its instructions is executed there.
-template <int D, int NT, int KW, bool SIG, bool SCORED, bool NARROW>
+template <int D, int NT, int KW, bool SIG, bool SCORED, bool NARROW, bool SPLIT>
 __global__ void __launch_bounds__(AP_THREADS * KW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __restrict__ out, long out_stride,
                          const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
                          const int* __restrict__ block_table, int bt_width, int page_size, int page_shift,
                          const int* __restrict__ positions, const int* __restrict__ cu_seqlens, int n_seqs, int H,
-                         int Hkv, float scale, int window, int fold, SigmoidArgs sig, ScoreForm form) {
+                         int Hkv, float scale, int window, int fold, SigmoidArgs sig, ScoreForm form, SplitWalk split) {
     constexpr int DS = D / 32;                 // k-steps of the score product
     constexpr int DT = D / 16;                 // d tiles of the output product
     constexpr int COLS = 16 * AP_WAVES * NT;   // columns of a workgroup
@@ -132,10 +144,13 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
     // bring about the same number of key blocks together.
     // Every wave finds the unit by itself, 64 requests at a time: a walk over the requests by one thread waits for
     // memory at each of them (2 us of a step of 20 requests).
-    int seq = -1, t0 = 0, nt = 0;
+    int seq = -1, t0 = 0, nt = 0, unit = 0, part = 0;
     {
-        const int n_all = gridDim.y, half = (n_all + 1) / 2;
-        int u = (!fold || (int)blockIdx.y < half) ? n_all - 1 - (int)blockIdx.y : (int)blockIdx.y - half;
+        const int n_all = SPLIT ? (int)gridDim.y / 2 : (int)gridDim.y, half = (n_all + 1) / 2;
+        part = SPLIT && (int)blockIdx.y >= n_all ? 1 : 0;
+        const int y = (int)blockIdx.y - part * n_all;
+        int u = (SPLIT || !fold || y < half) ? n_all - 1 - y : y - half;
+        unit = u;
         // (a step of one prompt needs no more than its first request's two numbers, which come with the other lanes' own)
         int s = lane, first = s < n_seqs ? cu_seqlens[s] : 0, len = s < n_seqs ? cu_seqlens[s + 1] - first : 0;
         const int first0 = __builtin_amdgcn_readfirstlane(first), len0 = __builtin_amdgcn_readfirstlane(len);
@@ -180,6 +195,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
     // a unit whose columns fit one tile (a decoding request in a step with prompts, a prompt's last tokens)
     static_assert(!NARROW || KW > 1 || NT == 1, "this form has no registers to spare");
     const bool narrow = NARROW && ncols <= 16;
+    if (SPLIT && narrow && part > 0) return;         // its waves take turns with the blocks already
     const int* bt = block_table + (size_t)seq * bt_width;
 
     // ---- this lane's columns
@@ -244,6 +260,20 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
     const int kept_first = SIG ? 0 : sig.first;
     const int nf = (kept_first > 0 && b0 > 0) ? ((kept_first + 31) / 32 < b0 ? (kept_first + 31) / 32 : b0) : 0;
 
+    // the blocks of the walk that are this workgroup's: w0 and on, w1 not any more. The first part has whole pairs of blocks: no
+    // block past its end is computed, which its columns may see.
+    int w0 = 0, w1 = nf + b1 - b0 + 1;
+    bool in_parts = false;
+    if (SPLIT && !narrow) {
+        in_parts = w1 >= split.limit + AP_PART_BLOCKS;
+        if (part == 1) {
+            if (!in_parts) return;
+            w0 = w1 > 2 * split.limit ? ((w1 + 1) / 2 + 1) & ~1 : split.limit;      // (no more than half of a long walk behind)
+        } else if (in_parts) {
+            w1 = w1 > 2 * split.limit ? ((w1 + 1) / 2 + 1) & ~1 : split.limit;
+        }
+    }
+
     float m_run[NT], l_run[NT];
     floatx4_t acc_o[NT][DT];
 #pragma unroll
@@ -307,10 +337,10 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
         k_lane = k_head + (size_t)hk * D * sizeof(bf16) + k_off[0];
         v_lane = v_head + (size_t)hv * sizeof(bf16) + v_off[0];
     }
-    // round j of the walk: key group kg has the (j * KW + kg)-th block of the walk, the nf blocks of kept
+    // round j of the walk: key group kg has the (w0 + j * KW + kg)-th block of the walk, the nf blocks of kept
     // first positions, then b0, b0 + 1, ...
     auto block_of = [&](int j) {
-        const int idx = j * KW + kg;
+        const int idx = (SPLIT ? w0 : 0) + j * KW + kg;
         return idx < nf ? idx : b0 + idx - nf;
     };
     auto page_ids = [&](int j) {
@@ -564,6 +594,18 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
         return inv;
     };
 
+    auto write_out = [&](int ct, float inv, const floatx4_t (&sums)[DT]) __attribute__((always_inline)) {
+        if (!col_ok[ct]) return;
+        bf16* orow = out + (size_t)col_tok[ct] * out_stride + (size_t)col_head[ct] * D;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            uint2 packed;
+            packed.x = f32x2_to_bf16x2_bits(sums[dt][0] * inv, sums[dt][1] * inv);
+            packed.y = f32x2_to_bf16x2_bits(sums[dt][2] * inv, sums[dt][3] * inv);
+            *reinterpret_cast<uint2*>(orow + 16 * dt + 4 * g) = packed;
+        }
+    };
+
     // ---- a narrow unit: every wave walks blocks of its own, operands from the pages straight into registers a block ahead
     // (each is used by this wave alone: LDS would only add a barrier to every two blocks), and the waves' sums are joined at the
     // end. In the wide form one wave of four has columns, and a walk takes four times the rounds: 17 decoding requests of
@@ -668,7 +710,7 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
         return;
     }
 
-    const int rounds = (nf + b1 - b0 + KW) / KW;    // the same for every wave: they meet at the barriers
+    const int rounds = (w1 - w0 + KW - 1) / KW;     // the same for every wave: they meet at the barriers
     PageIds ids_a, ids_b;
     KOps k_even, k_odd;
     VOps vals;
@@ -837,19 +879,74 @@ attention_prefill_kernel(const bf16* __restrict__ q, long q_stride, bf16* __rest
         if (kg != 0) return;
     }
 
+    if constexpr (SPLIT) if (in_parts) {
+        // ---- the two parts' sums: stored through to memory and read back the same way (the parts may run on compute units that share no
+        // cache), counted in when the workgroup's stores have arrived; nobody waits for another.
+        static_assert(KW == 1, "a key group has no counter of its own");
+        __shared__ int sh_last;
+        int* const counter = split.counters + (size_t)unit * Hkv + kvh;
+        float* const room = split.partials + ((size_t)unit * Hkv + kvh) * (2 * COLS * (D + 2));
+        int t_own = tid;                             // (made anew here: these addresses are not to live through the walk)
+        asm volatile("" : "+v"(t_own));
+        // a part's room: pairs of sums by thread, then maximum and sum of weights by column
+        const auto room_of = [&](int p) { return reinterpret_cast<unsigned long long*>(room + p * (COLS * (D + 2))); };
+        const auto sums_at = [&](int ct, int dt, int h) { return ((ct * DT + dt) * 2 + h) * AP_THREADS + t_own; };
+        const auto tops_at = [&](int ct) { return COLS * D / 2 + (cw * NT + ct) * 16 + i; };
+        const auto pair_of = [](float a, float b) { return (unsigned long long)__float_as_uint(b) << 32 | __float_as_uint(a); };
+        const auto half_of = [](unsigned long long two, int h) { return __uint_as_float((unsigned)(two >> (32 * h))); };
+        // the other one is counted already: nobody will read this one's
+        if (tid == 0) sh_last = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (!sh_last) {
+            unsigned long long* const mine = room_of(part);
 #pragma unroll
-    for (int ct = 0; ct < NT; ++ct) {
-        if (!col_ok[ct]) continue;
-        const float inv = finish(ct, m_run[ct], l_run[ct]);
-        bf16* orow = out + (size_t)col_tok[ct] * out_stride + (size_t)col_head[ct] * D;
+            for (int ct = 0; ct < NT; ++ct) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            uint2 packed;
-            packed.x = f32x2_to_bf16x2_bits(acc_o[ct][dt][0] * inv, acc_o[ct][dt][1] * inv);
-            packed.y = f32x2_to_bf16x2_bits(acc_o[ct][dt][2] * inv, acc_o[ct][dt][3] * inv);
-            *reinterpret_cast<uint2*>(orow + 16 * dt + 4 * g) = packed;
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        __hip_atomic_store(mine + sums_at(ct, dt, h), pair_of(acc_o[ct][dt][2 * h], acc_o[ct][dt][2 * h + 1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (g == 0) __hip_atomic_store(mine + tops_at(ct), pair_of(m_run[ct], l_run[ct]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            __builtin_amdgcn_s_waitcnt(0);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __syncthreads();
+            if (tid == 0) sh_last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            if (!sh_last) return;
         }
+        if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long* const its = room_of(1 - part);
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) {
+            const unsigned long long top = __hip_atomic_load(its + tops_at(ct), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            unsigned long long two[DT][2];
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) two[dt][h] = __hip_atomic_load(its + sums_at(ct, dt, h), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const float m1 = half_of(top, 0), l1 = half_of(top, 1), m_fin = fmaxf(m_run[ct], m1);
+            // (sigmoid weights are plain sums)
+            const float f0 = SIG ? 1.f : m_run[ct] == -INFINITY ? 0.f : exp2f(m_run[ct] - m_fin);
+            const float f1 = SIG ? 1.f : m1 == -INFINITY ? 0.f : exp2f(m1 - m_fin);
+            // each product rounded, then added: the same whichever of the two is here
+            const auto join = [&](float own, float other) {
+#pragma clang fp contract(off)
+                return f0 * own + f1 * other;
+            };
+            const float inv = finish(ct, m_fin, join(l_run[ct], l1));
+            floatx4_t o[DT];
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[dt][r] = join(acc_o[ct][dt][r], half_of(two[dt][r / 2], r % 2));
+            write_out(ct, inv, o);
+        }
+        return;
     }
+
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct) write_out(ct, finish(ct, m_run[ct], l_run[ct]), acc_o[ct]);
 }
 
 extern "C" int mv_attention_prefill_unit_tokens(int group, int nt) {
@@ -859,7 +956,7 @@ extern "C" int mv_attention_prefill_unit_tokens(int group, int nt) {
 }
 
 template <int D, int NT, int KW, bool SIG = false, bool SCORED = false>
-static int launch_prefill(int narrow, dim3 grid, hipStream_t stream, const void* q, long q_stride, void* out, long out_stride,
+static int launch_prefill(const SplitWalk& split, int narrow, dim3 grid, hipStream_t stream, const void* q, long q_stride, void* out, long out_stride,
                           const void* k_pages, const void* v_pages, const int* block_table, int bt_width,
                           int page_size, int page_shift, const int* positions, const int* cu_seqlens, int n_seqs,
                           int H, int Hkv, float scale, int window, int fold, SigmoidArgs sig = SigmoidArgs{0, nullptr, nullptr, 0, 0},
@@ -869,15 +966,38 @@ static int launch_prefill(int narrow, dim3 grid, hipStream_t stream, const void*
     const auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, threads, 0, stream, (const bf16*)q, q_stride, (bf16*)out, out_stride, (const bf16*)k_pages,
                            (const bf16*)v_pages, block_table, bt_width, page_size, page_shift, positions, cu_seqlens, n_seqs, H, Hkv, scale,
-                           window, fold, sig, form);
+                           window, fold, sig, form, split);
     };
-    if constexpr (KW > 1 || NT == 1) {
-        if (narrow) {
-            launch(attention_prefill_kernel<D, NT, KW, SIG, SCORED, true>);
+    if constexpr (KW == 1 && !(SIG && NT == 2)) {
+        if (split.limit > 0) {
+            grid.y *= 2;
+            if constexpr (NT == 1) {
+                if (narrow) {
+                    launch(attention_prefill_kernel<D, NT, KW, SIG, SCORED, true, true>);
+                    return 0;
+                }
+            }
+            launch(attention_prefill_kernel<D, NT, KW, SIG, SCORED, false, true>);
             return 0;
         }
     }
-    launch(attention_prefill_kernel<D, NT, KW, SIG, SCORED, false>);
+    if constexpr (KW > 1 || NT == 1) {
+        if (narrow) {
+            launch(attention_prefill_kernel<D, NT, KW, SIG, SCORED, true, false>);
+            return 0;
+        }
+    }
+    launch(attention_prefill_kernel<D, NT, KW, SIG, SCORED, false, false>);
+    return 0;
+}
+
+// Floats of the room that the two parts of a unit of one kv head have.
+extern "C" int mv_attention_prefill_part_floats(int nt, int D) { return 2 * 16 * AP_WAVES * nt * (D + 2); }
+
+static int check_split(const char* what, int kw, int limit, const float* partials, const int* counters, int n_units) {
+    MV_REQUIRE(limit >= 0 && limit % 2 == 0 && limit < (1 << 24) && (limit == 0 || (kw == 1 && partials != nullptr && counters != nullptr && (uintptr_t)partials % 16 == 0)),
+               "%s: walks in parts of %d blocks (an even number, workgroups of four waves, room for their sums and counters)", what, limit);
+    MV_REQUIRE(limit == 0 || 2L * n_units <= 65535, "%s: %d units in two parts exceed one launch", what, n_units);
     return 0;
 }
 
@@ -885,6 +1005,8 @@ static int launch_prefill(int narrow, dim3 grid, hipStream_t stream, const void*
 // the workgroups, for steps too small to fill the chip otherwise).
 // kw: key groups per workgroup (2: eight waves, the walk over a unit's keys takes half as many rounds).
 // narrow: some request may bring so few tokens that its columns fit one tile of 16 (the kernel that serves these apart).
+// limit: walks of more blocks are cut in two (SPLIT above), 0: not; partials: n_units * Hkv * mv_attention_prefill_part_floats(nt, D) floats at a 16-byte
+// address, counters: int [n_units * Hkv], zero before the first launch (every launch leaves them zero); launches that share them must not overlap.
 // n_units = sum over sequences of ceil(q_len / unit tokens(group, nt)), or an upper bound of it (units
 // beyond the step's own end at once); n_busy = the units that hold tokens, as far as the caller knows
 // (n_units if it knows no better): it decides how the units are dealt out. grid = (kv heads, units).
@@ -893,7 +1015,9 @@ extern "C" int mv_attention_prefill(const void* q, long q_stride, void* out, lon
                                     const int* positions, const int* cu_seqlens, int n_seqs, int n_units, int n_busy,
                                     int nt, int kw, int narrow, int H, int Hkv, int D, float scale, int window, int first,
                                     const void* gate, long gate_stride, float cap, const float* slopes, int sink,
-                                    hipStream_t stream) {
+                                    float* partials, int* counters, int limit, hipStream_t stream) {
+    if (check_split("attention_prefill", kw, limit, partials, counters, n_units)) return 1;
+    const SplitWalk split{limit, partials, counters};
     MV_REQUIRE(kw == 1 || kw == 2, "attention_prefill: %d key groups per workgroup (1 or 2)", kw);
     MV_REQUIRE(first >= 0 && (gate == nullptr || gate_stride >= H), "attention_prefill: bad count of kept first positions or "
                "gate rows too short");
@@ -924,10 +1048,10 @@ extern "C" int mv_attention_prefill(const void* q, long q_stride, void* out, lon
     const ScoreForm form{cap, slopes, sink};
     const bool scored = cap > 0.f || slopes != nullptr || sink;
 #define AP_LAUNCH(DD, NN, KK)                                                                                      \
-    rc = scored ? launch_prefill<DD, NN, KK, false, true>(narrow, grid, stream, q, q_stride, out, out_stride, k_pages, v_pages,   \
+    rc = scored ? launch_prefill<DD, NN, KK, false, true>(split, narrow, grid, stream, q, q_stride, out, out_stride, k_pages, v_pages,   \
                                                           block_table, bt_width, page_size, page_shift, positions,      \
                                                           cu_seqlens, n_seqs, H, Hkv, scale, window, fold, extra, form) \
-                : launch_prefill<DD, NN, KK>(narrow, grid, stream, q, q_stride, out, out_stride, k_pages, v_pages, block_table, \
+                : launch_prefill<DD, NN, KK>(split, narrow, grid, stream, q, q_stride, out, out_stride, k_pages, v_pages, block_table, \
                                              bt_width, page_size, page_shift, positions, cu_seqlens, n_seqs, H, Hkv,    \
                                              scale, window, fold, extra)
     if (kw == 2) {
@@ -954,7 +1078,10 @@ extern "C" int mv_attention_prefill_sigmoid(const void* q, long q_stride, void* 
                                             const int* positions, const int* cu_seqlens, int n_seqs, int n_units,
                                             int n_busy, int nt, int kw, int narrow, int H, int Hkv, int D, float scale, int window,
                                             int chunk, const float* bias, const void* gate, long gate_stride,
-                                            hipStream_t stream) {
+                                            float* partials, int* counters, int limit, hipStream_t stream) {
+    if (check_split("attention_prefill_sigmoid", kw, limit, partials, counters, n_units)) return 1;
+    MV_REQUIRE(limit == 0 || nt == 1, "attention_prefill_sigmoid: walks of %d column tiles a wave are not cut", nt);
+    const SplitWalk split{limit, partials, counters};
     MV_REQUIRE(kw == 1 || kw == 2, "attention_prefill_sigmoid: %d key groups per workgroup (1 or 2)", kw);
     MV_REQUIRE(H > 0 && Hkv > 0 && H % Hkv == 0, "attention_prefill_sigmoid: %d heads are not a multiple of %d kv heads",
                H, Hkv);
@@ -980,7 +1107,7 @@ extern "C" int mv_attention_prefill_sigmoid(const void* q, long q_stride, void* 
     const SigmoidArgs sig{chunk, bias, (const bf16*)gate, gate_stride, 0};
     int rc = 0;
 #define AP_LAUNCH(DD, NN, KK)                                                                                          \
-    rc = launch_prefill<DD, NN, KK, true>(narrow, grid, stream, q, q_stride, out, out_stride, k_pages, v_pages, block_table,     \
+    rc = launch_prefill<DD, NN, KK, true>(split, narrow, grid, stream, q, q_stride, out, out_stride, k_pages, v_pages, block_table,     \
                                           bt_width, page_size, page_shift, positions, cu_seqlens, n_seqs, H, Hkv, scale, \
                                           window, fold, sig)
     if (kw == 2) {

@@ -324,12 +324,13 @@ _OPTIONAL_SIGNATURES = {
     # sink, stream
     "mv_attention_prefill": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int,
                                      c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
-                                     c_float, c_int, c_int, c_void_p, c_long, c_float, c_void_p, c_int, c_void_p]),
+                                     c_float, c_int, c_int, c_void_p, c_long, c_float, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p]),
+    "mv_attention_prefill_part_floats": (c_int, [c_int, c_int]),
     "mv_attention_prefill_unit_tokens": (c_int, [c_int, c_int]),
-    # as mv_attention_prefill up to window, then chunk, bias, gate, gate_stride, stream
+    # as mv_attention_prefill up to window, then chunk, bias, gate, gate_stride, partials, counters, limit, stream
     "mv_attention_prefill_sigmoid": (c_int, [c_void_p, c_long, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int,
                                              c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
-                                             c_float, c_int, c_int, c_void_p, c_void_p, c_long, c_void_p]),
+                                             c_float, c_int, c_int, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_void_p]),
     # packed, ld, n, n_seqs, H, G, DK, DV, taps, conv_w, a_log, dt_bias, weight_dtype, conv_state, unit_eps, token_seq,
     # cu_seqlens, state_slots, qk, vals, gates, dtype, stream
     "mv_gdelta_prepare": (c_int, [c_void_p, c_long, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,

@@ -108,6 +108,8 @@ DECODE_ATTENTION_WAVES = 4
 # in flight (``Ops.compute_units``)
 # (sequence, kv head) pairs of one decode step whose keys may be split over workgroups
 SPLIT_COUNTERS = 1 << 16
+# units times kv heads of a prompt step whose walks may be cut in two (room for their sums: 133 KB each with 32 columns a wave and heads of 128)
+PROMPT_SPLIT_UNITS = 1280
 # steps of up to so many rows carry queries into a latent's space, and sums out of it, in float32
 HEAD_LINEAR_FLOAT_ROWS = 64
 # (block of 32 keys, head) pairs whose keys and values a latent attention may make at a time: 16 KiB each, 512 MiB of scratch at most, in
@@ -2397,15 +2399,18 @@ class Ops:
         if (self.use_fast_kernels and plan is not None and self.lib.has("mv_attention_prefill_sigmoid")
                 and head_dim == value_dim and head_dim in (64, 128) and page_size >= 16 and not page_size & (page_size - 1)
                 and qs % 8 == 0 and os_ % 4 == 0 and q.data_ptr() % 16 == 0 and out.data_ptr() % 8 == 0):
-            nt, kw, n_units, n_busy = self._prefill_variant(plan, group, num_kv_heads)
+            # (sums of sigmoid weights: the walk of 32 columns a wave has no registers left for being cut)
+            keys = min((x for x in (w + 1, c) if x > 0), default=None)
+            nt, kw, n_units, n_busy, limit = self._prefill_variant(plan, group, num_kv_heads, keys, narrow_sums=True)
             if nt:
+                split = self._prefill_room(plan.workspace, limit, nt, n_units, num_kv_heads, head_dim)
                 self._note_attention("mv_attention_prefill_sigmoid", self._chunk_priced(plan, c), n, num_heads, num_kv_heads,
                                      head_dim, 2)
-                self.lib.call("mv_attention_prefill_sigmoid", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
+                self._decode_launch("mv_attention_prefill_sigmoid", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
                               v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size,
                               positions.data_ptr(), plan.cu_seqlens.data_ptr(), plan.n_seqs, n_units, n_busy, nt, kw, int(plan.has_short(16 // group + 1)),
                               num_heads, num_kv_heads, head_dim, float(scale), w, c, _ptr(bias), _ptr(gate), gate_stride,
-                              self._stream())
+                              *split, self._stream())
                 return
         self._note_attention("mv_attention_sigmoid_ref", self._chunk_priced(plan, c), n, num_heads, num_kv_heads, head_dim,
                              q.element_size())
@@ -3217,9 +3222,20 @@ class Ops:
                       DECODE_ATTENTION_WAVES, token_seq.data_ptr(), self._stream())
         return True
 
-    def _prefill_variant(self, plan, group: int, Hkv: int):
-        """(column tiles per wave, key groups per workgroup, units, busy units) of the MFMA prompt
-        attention for this step; column tiles 0: the kernel does not serve ``group`` heads per kv head."""
+    def _prefill_variant(self, plan, group: int, Hkv: int, keys: Optional[int] = None, narrow_sums: bool = False):
+        """(column tiles per wave, key groups per workgroup, units, busy units, blocks of a walk's first part) of the MFMA prompt
+        attention for this step; column tiles 0: the kernel does not serve ``group`` heads per kv head, blocks 0: walks are not cut.
+        ``keys``: the most a column sees where a window or a chunk says so; ``narrow_sums``: only walks of 16 columns a wave may be cut."""
+        if plan.prefill_variant is None:
+            for nt in (1,) if narrow_sums else (2, 1):
+                limit = self._prefill_limit(plan, nt, group, Hkv, keys)
+                if limit:
+                    u = self.lib.dll.mv_attention_prefill_unit_tokens(group, nt)
+                    return nt, 1, plan.units(u), plan.busy_units(u), limit
+        elif len(plan.prefill_variant) > 2:
+            nt, kw, limit = plan.prefill_variant
+            u = self.lib.dll.mv_attention_prefill_unit_tokens(group, nt)
+            return nt, kw, plan.units(u), plan.busy_units(u), limit
         # 128 columns per workgroup (each operand read from LDS feeds two MFMAs) when that still leaves
         # two workgroups for every compute unit, else 64 (measured on MI355X: 2048 tokens of one
         # sequence with 8 kv heads are faster with 64, 4096 tokens or 8 x 512 with 128)
@@ -3240,7 +3256,7 @@ class Ops:
                 raise KernelLibraryError(f"attention: {nt} column tiles a wave do not serve {group} heads per kv head")
             n_units, n_busy = plan.units(u), plan.busy_units(u)
         if nt == 0:
-            return 0, 0, 0, 0
+            return 0, 0, 0, 0, 0
         # two key groups per workgroup (eight waves) halve the walk over long contexts; they pay while
         # the grid leaves compute units waiting for the longest walk (measured on MI355X, 8 kv heads:
         # faster below two four-wave workgroups per compute unit, 33.9 against 35.3 us at 1,792 tokens,
@@ -3250,7 +3266,51 @@ class Ops:
         kw = 2 if plan.max_context_len >= PREFILL_TWO_GROUPS_FROM and n_busy * Hkv < 2 * self.compute_units else 1
         if plan.prefill_variant is not None:
             kw = int(plan.prefill_variant[1])
-        return nt, kw, n_units, n_busy
+        return nt, kw, n_units, n_busy, 0
+
+    def _prefill_limit(self, plan, nt: int, group: int, Hkv: int, keys: Optional[int]) -> int:
+        """Blocks of the first part of a walk cut in two with ``nt`` column tiles a wave, 0: not cut. The limit is some more than what
+        a slot (two workgroups a compute unit) gets if a single prompt of the step's rows is dealt out evenly; several prompts, whose walks
+        are shorter, are cut more rarely. us whole / cut: 16 heads on 8, 1,800 rows 40.3 / 34.1, 2,048 42.3 / 38.9, 2,500 60.3 / 50.2, 3,000 71 / 62,
+        4,096 111 / 86, 6,000 192 / 171; 32 heads 1,500 rows 41.8 / 38.7, 2,048 57.8 / 51.3, 2,600 81.6 / 75.3. From four 32-column units a compute unit on
+        the dispatch evens walks out by itself (8,192 rows 276.9 / 278.0), below the lower ends the joining takes what it gives (1,408 rows
+        28.4 / 28.3, 32 heads 1,000 rows 25.4 / 25.9)."""
+        u = self.lib.dll.mv_attention_prefill_unit_tokens(group, nt)
+        if u <= 0 or not self.lib.has("mv_attention_prefill_part_floats"):
+            return 0
+        units, busy, cus = plan.units(u), plan.busy_units(u), self.compute_units
+        if units * Hkv > PROMPT_SPLIT_UNITS:
+            return 0
+        rows = plan.bound[0] if plan.bound is not None else sum(plan.q_lens)
+        blocks = rows / 32
+        mean = (blocks + 1) / 2 * busy * Hkv / (2 * cus)
+        if nt == 2:
+            limit = int(1.15 * mean / 2 + 0.999) * 2
+            serves = 1.25 * cus <= busy * Hkv < 4 * cus and limit >= 20
+        else:
+            limit = int(1.3 * mean / 2 + 0.999) * 2
+            serves = 1.5 * cus <= busy * Hkv and limit >= 24
+        longest = blocks if keys is None else min(blocks, (keys + u) / 32 + 2)
+        return limit if serves and longest >= limit + 8 else 0
+
+    def _prefill_room(self, workspace, limit: int, nt: int, n_units: int, Hkv: int, D: int):
+        """(partial sums, counters, blocks of a first part) for the kernel."""
+        if limit == 0:
+            return None, None, 0
+        partials = workspace.get("attn.prompt_partials", (n_units * Hkv * int(self.lib.dll.mv_attention_prefill_part_floats(nt, D)),), torch.float32)
+        return partials.data_ptr(), self._split_counters(n_units * Hkv, partials), limit
+
+    def reserve_prompt_attention(self, workspace, tokens: int, seqs: int, H: int, Hkv: int, D: int) -> None:
+        """Room for the parts of walks of any step of up to ``tokens`` tokens of up to ``seqs`` sequences (``_prefill_limit``)."""
+        if not (self.use_fast_kernels and self.dtype == torch.bfloat16 and D in (64, 128) and self.lib.has("mv_attention_prefill_part_floats")):
+            return
+        dll, floats = self.lib.dll, 0
+        for nt, least in ((1, 1.5), (2, 1.25)):
+            u = dll.mv_attention_prefill_unit_tokens(H // Hkv, nt)
+            if u > 0 and (tokens // u + seqs) * Hkv >= least * self.compute_units:
+                floats = max(floats, min(PROMPT_SPLIT_UNITS, (tokens // u + seqs) * Hkv) * int(dll.mv_attention_prefill_part_floats(nt, D)))
+        if floats:
+            workspace.get("attn.prompt_partials", (floats,), torch.float32)
 
     def _attention_fast(self, q, qs, out, os_, k_pages, v_pages, block_table, page_size, positions, token_seq,
                         H, Hkv, D, scale, window, plan, first: int = 0, gate=None, gs: int = 0, form=(0.0, 0, 0)) -> bool:
@@ -3276,15 +3336,16 @@ class Ops:
             return True
         if page_size & (page_size - 1):
             return False
-        nt, kw, n_units, n_busy = self._prefill_variant(plan, group, Hkv)
+        nt, kw, n_units, n_busy, limit = self._prefill_variant(plan, group, Hkv, None if window < 0 else window + 1 + first + 32)
         if nt == 0:
             return False
         self._note_attention("mv_attention_prefill", priced, q.shape[0], H, Hkv, D, 2)
-        self.lib.call("mv_attention_prefill", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
+        self._decode_launch("mv_attention_prefill", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
                       v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size,
                       positions.data_ptr(), plan.cu_seqlens.data_ptr(), n_seqs, n_units, n_busy, nt, kw,
                       int(plan.has_short(16 // group + 1)), H, Hkv, D,
-                      float(scale), window, first, _ptr(gate), gs, *form, self._stream())
+                      float(scale), window, first, _ptr(gate), gs, *form,
+                      *self._prefill_room(plan.workspace, limit, nt, n_units, Hkv, D), self._stream())
         return True
 
     # ------------------------------------------------------------------------------------

@@ -293,6 +293,11 @@ class Attention(Mixer):
                                                             device=self.w_qkv.device)], dim=0).contiguous()
             self.width += pad
 
+    def reserve(self, tokens: int, seqs: int) -> None:
+        spec = self.spec
+        if spec.v_head_dim == spec.head_dim:
+            self.rt.ops.reserve_prompt_attention(self.rt.workspace, tokens, seqs, spec.num_heads, spec.num_kv_heads, spec.head_dim)
+
     def first_product(self):
         return self.w_qkv.shape[0], self.w_qkv.shape[1], False
 

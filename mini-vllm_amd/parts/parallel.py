@@ -74,6 +74,9 @@ class ParallelMixer(Mixer):
         self.width = self.w_packed.shape[0]
         self.w_left, self.w_right = tensors["left_out"].contiguous(), tensors["right_out"].to(tensors["left_out"].dtype).contiguous()
 
+    def reserve(self, tokens: int, seqs: int) -> None:
+        self.left.reserve(tokens, seqs)
+
     def first_product(self):
         return self.w_packed.shape[0], self.w_packed.shape[1], False
 
@@ -151,6 +154,9 @@ class ParallelSum(Mixer):
         self.w_o[:, self.right_column:self.right_column + out_r] = self.right.w_o
         self.left.w_qkv = self.left.w_o = self.right.w_packed = self.right.w_o = None
         self.gaps = [(a, b) for a, b in ((out_l, self.right_column), (self.right_column + out_r, self.inner)) if b > a]
+
+    def reserve(self, tokens: int, seqs: int) -> None:
+        self.left.reserve(tokens, seqs)
 
     def first_product(self):
         return self.w_packed.shape[0], self.w_packed.shape[1], False
