@@ -50,7 +50,20 @@ struct DeltaChunkArgs {
     int H, G, DV;
     const int* cu_seqlens; int n_seqs;
     float* M; float* N; float* Q; float* out;
+    // ROWS: what the general rule's vectors are made of beside the rows (see delta_prepare_kernel)
+    int rank; const void* w2t; const void* w0; const void* a_bias; int weights_f32; float decay_rate, key_eps;
 };
+
+#define DC_MAX_RANK 64             // of the decays' products: a lane holds its operands of all of it
+template <typename T>
+__device__ __forceinline__ float4 four_of(const T* p) {
+    if constexpr (sizeof(T) == 4) {
+        return *reinterpret_cast<const float4*>(p);
+    } else {
+        const uint2 u = *reinterpret_cast<const uint2*>(p);
+        return float4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u)};
+    }
+}
 
 #define DC_THREADS 512
 
@@ -121,7 +134,10 @@ __device__ __forceinline__ size_t quad_of(int tile_row, int rows, int k_tile, in
 }
 
 // ---- what concerns one chunk alone: workgroup (chunk, head)
-template <typename T, int DK, int RULE>
+// ROWS (general rule, heads of 64): the vectors are made here from the packed rows [r | k | v | g | a | w1], the decays' products over the rank on the
+// MFMA units, and not by a kernel that leaves them in memory as floats: 42 MB written and read again for 2,048 rows of 16 heads.
+// us, prepare + chunks / this: 2,048 rows 21.0 + 47.4 / 52.5, 552 rows 15.4 + 24.5 / 27.5. Where a step has requests for the scan too, those want the vectors.
+template <typename T, int DK, int RULE, bool ROWS>
 __global__ void __launch_bounds__(DC_THREADS)
 delta_chunk_kernel(DeltaChunkArgs A) {
     constexpr int C = DC_TOKENS, R16 = DC_RUN;
@@ -150,50 +166,100 @@ delta_chunk_kernel(DeltaChunkArgs A) {
 
     // the chunk's vectors; rows beyond its tokens change nothing (decay one, everything else zero)
     const int group = RULE == RULE_GENERAL ? head : head / (H / A.G);
-    for (int x = tid; x < C * (DK / 4); x += DC_THREADS) {
-        const int t = x / (DK / 4), c = (x % (DK / 4)) * 4;
+    if constexpr (ROWS) {
+        static_assert(RULE == RULE_GENERAL && C * (DK / 4) == DC_THREADS && DK / 4 == 16 && 2 * (DK / 16) == DC_THREADS / 64, "four channels a thread, a tile of decays a wave");
+        constexpr int PT = DC_MAX_RANK + 4;
+        static_assert(C * PT <= (2 * MROWS + M2ROWS) * PC, "no room for the rows of the decays' products");
+        float (*th)[PT] = reinterpret_cast<float (*)[PT]>(once);               // (used up before A and A' come)
+        const int t = tid / 16, c = (tid % 16) * 4, inner = H * DK, col = head * DK + c;
         const bool ok = t < count;
-        const size_t row = row0 + (ok ? t : 0);
-        const float4 zero{0.f, 0.f, 0.f, 0.f};
-        auto at = [&](const float* p) __attribute__((always_inline)) { return *reinterpret_cast<const float4*>(p + c); };
-        float4 w, a = zero, xx, r, b = zero;
-        if constexpr (RULE == RULE_GENERAL) {
-            const float* v = A.vec + (row * H + head) * 5 * DK;
-            w = at(v); b = at(v + DK); a = at(v + 2 * DK); xx = at(v + 3 * DK); r = at(v + 4 * DK);
-            b = float4{-b.x, -b.y, -b.z, -b.w};
-        } else {
-            const float* v = A.vec + (row * A.G + group) * 2 * DK;
-            r = at(v);
-            xx = at(v + DK);
-            if constexpr (RULE == RULE_CHANNEL) {
-                const float* d = A.decay + row * A.ldz + (size_t)head * DK;
-                w = A.decay4 ? at(d) : float4{d[c], d[c + 1], d[c + 2], d[c + 3]};
-            } else {
-                const float d = A.gates[(row * H + head) * 4];
-                w = float4{d, d, d, d};
+        const T* row = (const T*)A.vals + (size_t)(row0 + (ok ? t : 0)) * A.ldv;
+        const float4 r = four_of(row + col), k = four_of(row + inner + col), v = four_of(row + 2 * (size_t)inner + col), az = four_of(row + 4 * (size_t)inner + col);
+        const float4 z = four_of(row + 5 * (size_t)inner + (c < A.rank ? c : 0));
+        // the wave's tile of decays: tokens 16 rt .., channels 16 ct ..; its weights are on their way meanwhile
+        const int rt = wave % 2, ct = wave / 2, ch = head * DK + 16 * ct + i;
+        float4 w2[DC_MAX_RANK / 16];
+        float4 ab;
+        float b0;
+        auto weights = [&](const auto* w2t, const auto* w0, const auto* a_bias) __attribute__((always_inline)) {
+#pragma unroll
+            for (int b = 0; b < DC_MAX_RANK / 16; ++b) {
+                const auto* at = w2t + (size_t)min(16 * b + 4 * g, A.rank - 4) * inner + ch;       // (the rank is a multiple of 16)
+                w2[b] = float4{to_f(at[0]), to_f(at[inner]), to_f(at[2 * inner]), to_f(at[3 * inner])};
             }
-            if constexpr (READ) {
-                const float beta = RULE == RULE_CHANNEL ? A.gates[row * H + head] : A.gates[(row * H + head) * 4 + 1];
-                a = float4{w.x * xx.x, w.y * xx.y, w.z * xx.z, w.w * xx.w};
-                xx = float4{beta * xx.x, beta * xx.y, beta * xx.z, beta * xx.w};
-            }
+            b0 = to_f(w0[ch]);
+            ab = four_of(a_bias + col);
+        };
+        if (A.weights_f32) weights((const float*)A.w2t, (const float*)A.w0, (const float*)A.a_bias);
+        else weights((const bf16*)A.w2t, (const bf16*)A.w0, (const bf16*)A.a_bias);
+        const float inv = 1.f / sqrtf(lanes_sum<16>(fmaf(k.x, k.x, fmaf(k.y, k.y, fmaf(k.z, k.z, k.w * k.w)))) + A.key_eps);
+        const float4 u{k.x * inv, k.y * inv, k.z * inv, k.w * inv};
+        const float4 b{-sigmoid_f(az.x + ab.x) * u.x, -sigmoid_f(az.y + ab.y) * u.y, -sigmoid_f(az.z + ab.z) * u.z, -sigmoid_f(az.w + ab.w) * u.w};
+        // (two names for the choice would be a choice between addresses, and both in scratch)
+        auto there = [&](const float4& x) __attribute__((always_inline)) { return ok ? x : float4{0.f, 0.f, 0.f, 0.f}; };
+        *reinterpret_cast<float4*>(&sX[t][c]) = there(k);
+        *reinterpret_cast<float4*>(&sR[t][c]) = there(r);
+        *reinterpret_cast<float4*>(&sA[t][c]) = there(u);
+        *reinterpret_cast<float4*>(&sB[t][c]) = there(b);
+        *reinterpret_cast<float4*>(&sV[t][c]) = there(v);
+        if (c < A.rank) *reinterpret_cast<float4*>(&th[t][c]) = float4{tanhf(z.x), tanhf(z.y), tanhf(z.z), tanhf(z.w)};
+        __syncthreads();
+        floatx4_t acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int b = 0; b < DC_MAX_RANK / 16; ++b)
+            if (16 * b < A.rank)
+                mfma4(acc, *reinterpret_cast<const float4*>(&th[16 * rt + i][16 * b + 4 * g]), w2[b]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int at = 16 * rt + 4 * g + q;
+            sW[at][16 * ct + i] = at < count ? expf(-A.decay_rate * sigmoid_f(acc[q] + b0)) : 1.f;
         }
-        *reinterpret_cast<float4*>(&sW[t][c]) = ok ? w : float4{1.f, 1.f, 1.f, 1.f};
-        *reinterpret_cast<float4*>(&sX[t][c]) = ok ? xx : float4{0.f, 0.f, 0.f, 0.f};
-        *reinterpret_cast<float4*>(&sR[t][c]) = ok ? r : float4{0.f, 0.f, 0.f, 0.f};
-        if constexpr (READ) *reinterpret_cast<float4*>(&sA[t][c]) = ok ? a : float4{0.f, 0.f, 0.f, 0.f};
-        if constexpr (PAIR) *reinterpret_cast<float4*>(&sB[t][c]) = ok ? b : float4{0.f, 0.f, 0.f, 0.f};
-    }
-    for (int x = tid; x < C * DVMAX; x += DC_THREADS) {
-        const int t = x / DVMAX, j = x % DVMAX;
-        const bool ok = t < count && j < DV;
-        const size_t row = row0 + (ok ? t : 0);
-        const int jj = ok ? j : 0;
-        float v;
-        if constexpr (RULE == RULE_GENERAL) v = to_f(((const T*)A.vals)[row * A.ldv + 2 * (size_t)H * DK + (size_t)head * DK + jj]);
-        else v = ((const float*)A.vals)[(row * H + head) * DV + jj];
-        if constexpr (RULE == RULE_SUM) v *= A.gates[(row * H + head) * 4 + 1];
-        sV[t][j] = ok ? v : 0.f;
+    } else {
+        for (int x = tid; x < C * (DK / 4); x += DC_THREADS) {
+            const int t = x / (DK / 4), c = (x % (DK / 4)) * 4;
+            const bool ok = t < count;
+            const size_t row = row0 + (ok ? t : 0);
+            const float4 zero{0.f, 0.f, 0.f, 0.f};
+            auto at = [&](const float* p) __attribute__((always_inline)) { return *reinterpret_cast<const float4*>(p + c); };
+            float4 w, a = zero, xx, r, b = zero;
+            if constexpr (RULE == RULE_GENERAL) {
+                const float* v = A.vec + (row * H + head) * 5 * DK;
+                w = at(v); b = at(v + DK); a = at(v + 2 * DK); xx = at(v + 3 * DK); r = at(v + 4 * DK);
+                b = float4{-b.x, -b.y, -b.z, -b.w};
+            } else {
+                const float* v = A.vec + (row * A.G + group) * 2 * DK;
+                r = at(v);
+                xx = at(v + DK);
+                if constexpr (RULE == RULE_CHANNEL) {
+                    const float* d = A.decay + row * A.ldz + (size_t)head * DK;
+                    w = A.decay4 ? at(d) : float4{d[c], d[c + 1], d[c + 2], d[c + 3]};
+                } else {
+                    const float d = A.gates[(row * H + head) * 4];
+                    w = float4{d, d, d, d};
+                }
+                if constexpr (READ) {
+                    const float beta = RULE == RULE_CHANNEL ? A.gates[row * H + head] : A.gates[(row * H + head) * 4 + 1];
+                    a = float4{w.x * xx.x, w.y * xx.y, w.z * xx.z, w.w * xx.w};
+                    xx = float4{beta * xx.x, beta * xx.y, beta * xx.z, beta * xx.w};
+                }
+            }
+            *reinterpret_cast<float4*>(&sW[t][c]) = ok ? w : float4{1.f, 1.f, 1.f, 1.f};
+            *reinterpret_cast<float4*>(&sX[t][c]) = ok ? xx : float4{0.f, 0.f, 0.f, 0.f};
+            *reinterpret_cast<float4*>(&sR[t][c]) = ok ? r : float4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (READ) *reinterpret_cast<float4*>(&sA[t][c]) = ok ? a : float4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (PAIR) *reinterpret_cast<float4*>(&sB[t][c]) = ok ? b : float4{0.f, 0.f, 0.f, 0.f};
+        }
+        for (int x = tid; x < C * DVMAX; x += DC_THREADS) {
+            const int t = x / DVMAX, j = x % DVMAX;
+            const bool ok = t < count && j < DV;
+            const size_t row = row0 + (ok ? t : 0);
+            const int jj = ok ? j : 0;
+            float v;
+            if constexpr (RULE == RULE_GENERAL) v = to_f(((const T*)A.vals)[row * A.ldv + 2 * (size_t)H * DK + (size_t)head * DK + jj]);
+            else v = ((const float*)A.vals)[(row * H + head) * DV + jj];
+            if constexpr (RULE == RULE_SUM) v *= A.gates[(row * H + head) * 4 + 1];
+            sV[t][j] = ok ? v : 0.f;
+        }
     }
     __syncthreads();
 
@@ -614,9 +680,9 @@ extern "C" int mv_delta_chunks_serve(int rule, int DK, int DV) {
     return rule >= RULE_GENERAL && rule <= RULE_SUM && (DK == 64 || DK == 128) && DV >= 1 && DV <= DK + 16;
 }
 
-template <typename T, int DK, int RULE>
+template <typename T, int DK, int RULE, bool ROWS = false>
 static int launch_delta_chunks(const DeltaChunkArgs& A, float* state, const int* state_slots, int chunks, hipStream_t stream) {
-    hipLaunchKernelGGL((delta_chunk_kernel<T, DK, RULE>), dim3(chunks, A.H), dim3(DC_THREADS), 0, stream, A);
+    hipLaunchKernelGGL((delta_chunk_kernel<T, DK, RULE, ROWS>), dim3(chunks, A.H), dim3(DC_THREADS), 0, stream, A);
     if (mv_check_launch("delta_chunk")) return 1;
     hipLaunchKernelGGL((delta_chunk_walk_kernel<DK, RULE != RULE_SUM>), dim3(A.n_seqs, A.H, (A.DV + 15) / 16), dim3((DK / 16 + 4) * 64), 0,
                        stream, A, state, state_slots);
@@ -639,7 +705,7 @@ extern "C" int mv_delta_chunks(int rule, const float* vec, const float* gates, c
     MV_REQUIRE(H <= 65535, "delta_chunks: too many heads");
     if (n == 0 || n_seqs == 0 || chunks == 0) return 0;
     const int decay4 = ldz % 4 == 0 && (uintptr_t)decay % 16 == 0;
-    const DeltaChunkArgs A{vec, gates, decay, ldz, decay4, vals, ldv, H, G, DV, cu_seqlens, n_seqs, M, N, Q, out};
+    const DeltaChunkArgs A{vec, gates, decay, ldz, decay4, vals, ldv, H, G, DV, cu_seqlens, n_seqs, M, N, Q, out, 0, nullptr, nullptr, nullptr, 0, 0.f, 0.f};
 #define DC_LAUNCH(T, RULE)                                                                                   \
     return DK == 64 ? launch_delta_chunks<T, 64, RULE>(A, state, state_slots, chunks, stream)               \
                     : launch_delta_chunks<T, 128, RULE>(A, state, state_slots, chunks, stream)
@@ -650,5 +716,25 @@ extern "C" int mv_delta_chunks(int rule, const float* vec, const float* gates, c
         default: DC_LAUNCH(float, RULE_SUM);
     }
 #undef DC_LAUNCH
+    return 0;
+}
+
+// 1: mv_delta_chunks_rows serves heads of this size and decays of this rank, rows this far apart
+extern "C" int mv_delta_chunks_rows_serve(int D, int rank, long ld) { return D == 64 && rank > 0 && rank <= DC_MAX_RANK && rank % 16 == 0 && ld % 8 == 0; }
+
+// mv_delta_chunks under the general rule straight from the packed rows, without the vectors of mv_delta_prepare (ROWS above).
+extern "C" int mv_delta_chunks_rows(const void* packed, long ld, int rank, const void* w2t, const void* w0, const void* a_bias, int weight_dtype,
+                                    float decay_rate, float key_eps, float* state, const int* cu_seqlens, const int* state_slots, int n_seqs, int n, int H,
+                                    int D, int chunks, float* M, float* N, float* Q, float* out, int dtype, hipStream_t stream) {
+    MV_REQUIRE(n >= 0 && n_seqs >= 0 && H > 0 && H <= 65535 && chunks >= 0, "delta_chunks_rows: bad sizes n=%d seqs=%d H=%d", n, n_seqs, H);
+    MV_REQUIRE(mv_delta_chunks_rows_serve(D, rank, ld) && ld >= 5L * H * D + rank, "delta_chunks_rows: heads of %d, rank %d, rows of %ld columns are not served", D, rank, ld);
+    MV_REQUIRE(packed && w2t && w0 && a_bias && state && cu_seqlens && state_slots && M && N && Q && out, "delta_chunks_rows: missing operand");
+    MV_REQUIRE(mv_valid_dtype(weight_dtype) && key_eps > 0.f, "delta_chunks_rows: an unknown weight type, or key_eps is not positive");
+    MV_REQUIRE((uintptr_t)packed % 16 == 0 && (uintptr_t)a_bias % 16 == 0 && (uintptr_t)state % 16 == 0 && (uintptr_t)M % 16 == 0 && (uintptr_t)N % 16 == 0
+               && (uintptr_t)Q % 16 == 0, "delta_chunks_rows: operands must be 16-byte aligned");
+    if (n == 0 || n_seqs == 0 || chunks == 0) return 0;
+    const DeltaChunkArgs A{nullptr, nullptr, nullptr, 0, 0, packed, ld, H, H, D, cu_seqlens, n_seqs, M, N, Q, out, rank, w2t, w0, a_bias,
+                           weight_dtype == MV_F32, decay_rate, key_eps};
+    MV_DISPATCH_T(dtype, "delta_chunks_rows", { return (launch_delta_chunks<T, 64, RULE_GENERAL, true>(A, state, state_slots, chunks, stream)); });
     return 0;
 }

@@ -799,6 +799,39 @@ class Ops:
         self._matrix_chunks("delta_chunks", "delta", coef, None, None, packed, packed.stride(0) if n > 1 else packed.shape[1], state,
                             cu_seqlens, state_slots, n_seqs, n, heads, heads, dim, dim, maps, sums, queries, out)
 
+    def delta_chunks_rows_serve(self, packed: torch.Tensor, dim: int, rank: int, a_bias: torch.Tensor) -> bool:
+        """Whether ``delta_chunks_rows`` takes these rows."""
+        ld = packed.stride(0) if packed.shape[0] > 1 else packed.shape[1]
+        return (self.lib.has("mv_delta_chunks_rows") and packed.data_ptr() % 16 == 0 and a_bias.data_ptr() % 16 == 0
+                and bool(self.lib.dll.mv_delta_chunks_rows_serve(dim, rank, ld)))
+
+    def delta_chunks_rows(self, packed: torch.Tensor, heads: int, dim: int, rank: int, w2t: torch.Tensor, w0: torch.Tensor, a_bias: torch.Tensor,
+                          decay_rate: float, key_eps: float, state: torch.Tensor, cu_seqlens: torch.Tensor, state_slots: torch.Tensor, n_seqs: int,
+                          maps: torch.Tensor, sums: torch.Tensor, queries: torch.Tensor, out: torch.Tensor) -> None:
+        """``delta_prepare`` and ``delta_chunks`` in one, for steps whose requests all bring ``delta_chunk_line`` tokens and more: the vectors
+        never lie in memory."""
+        self._act(packed, "delta rows")
+        n, inner, chunks = packed.shape[0], heads * dim, sums.shape[0]
+        if packed.dim() != 2 or packed.stride(1) != 1 or packed.shape[1] < 5 * inner + rank:
+            raise KernelLibraryError(f"delta_chunks_rows: rows {tuple(packed.shape)} do not hold 5 x {inner} + {rank} columns")
+        if out.dtype != torch.float32 or tuple(out.shape) != (n, inner) or not out.is_contiguous():
+            raise KernelLibraryError(f"delta_chunks_rows: the output must be float32 [{n}, {inner}]")
+        self._delta_state(state, heads, dim, "delta_chunks_rows")
+        self._ints(n, cu_seqlens=(cu_seqlens, n_seqs + 1), state_slots=(state_slots, n_seqs))
+        wcode = self._delta_weights(heads, dim, rank, w2t, w0, a_bias, "delta_chunks_rows")
+        for t, shape, name in ((maps, (chunks, heads, dim, dim), "chunk maps"), (sums, (chunks, heads, dim, dim), "chunk sums"),
+                               (queries, (n, heads, dim), "chunk queries")):
+            _dev(t, name)
+            if t.dtype != torch.float32 or tuple(t.shape) != shape or not t.is_contiguous():
+                raise KernelLibraryError(f"delta_chunks_rows: the {name} must be contiguous float32 {shape}")
+        C = self.delta_chunk_tokens()
+        size = (n * (4 * inner + rank) * packed.element_size() + self._size(w2t, out) + 2 * self._size(maps, sums, queries)
+                + 2 * min(n_seqs, max(n, 1)) * inner * dim * 4)
+        self._note("mv_delta_chunks_rows", size, n * inner * (2 * rank + 6 * C + 8 * dim))
+        self.lib.call("mv_delta_chunks_rows", packed.data_ptr(), packed.stride(0) if n > 1 else packed.shape[1], rank, w2t.data_ptr(), w0.data_ptr(),
+                      a_bias.data_ptr(), wcode, float(decay_rate), float(key_eps), state.data_ptr(), cu_seqlens.data_ptr(), state_slots.data_ptr(),
+                      n_seqs, n, heads, dim, chunks, maps.data_ptr(), sums.data_ptr(), queries.data_ptr(), out.data_ptr(), self.code, self._stream())
+
     def delta_step(self, packed: torch.Tensor, heads: int, dim: int, rank: int, w2t: torch.Tensor, w0: torch.Tensor,
                    a_bias: torch.Tensor, norm_weight: torch.Tensor, decay_rate: float, key_eps: float, eps: float,
                    state: torch.Tensor, token_seq: torch.Tensor, state_slots: torch.Tensor, out: torch.Tensor) -> None:

@@ -27,7 +27,7 @@ from typing import Dict, Optional
 import torch
 
 from .base import PartSpec, Runtime, TensorDecl, register_mixer
-from .matrix_state import ChunkedRecurrence, recurrence
+from .matrix_state import ChunkedRecurrence, recurrence, step_chunk_scratch, step_paths
 
 
 @dataclass(frozen=True)
@@ -101,14 +101,20 @@ class DeltaRule(ChunkedRecurrence):
                            self.norm, spec.decay_rate, spec.key_eps, spec.out_norm_eps, ctx.state(call), ctx.token_seq,
                            ctx.state_slots, gated)
         else:
-            # float32 [n, heads, 5, head_dim]: decay, rate * unit key, unit key, key, receptance
-            coef = ws.get("delta.coef", (n, spec.num_heads, 5, spec.head_dim), torch.float32)
-            ops.delta_prepare(packed, spec.num_heads, spec.head_dim, spec.decay_rank, self.w2_t, self.w0, self.a_bias,
-                              spec.decay_rate, spec.key_eps, coef)
             raw = ws.get("delta.raw", (n, inner), torch.float32)
-            recurrence(rt, ctx, "delta", n, spec.num_heads, spec.head_dim, spec.head_dim, raw, ops.delta_scan,
-                       self.chunks(ops.delta_chunks), packed, coef, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs,
-                       spec.num_heads, spec.head_dim)
+            sizes = spec.num_heads, spec.head_dim, spec.head_dim
+            if (self.chunks(ops.delta_chunks) is not None and step_paths(rt, ctx, "delta", *sizes) == (True, False)
+                    and ops.delta_chunks_rows_serve(packed, spec.head_dim, spec.decay_rank, self.a_bias)):
+                ops.delta_chunks_rows(packed, spec.num_heads, spec.head_dim, spec.decay_rank, self.w2_t, self.w0, self.a_bias, spec.decay_rate,
+                                      spec.key_eps, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs,
+                                      *step_chunk_scratch(rt, ctx, "delta", n, *sizes), raw)
+            else:
+                # float32 [n, heads, 5, head_dim]: decay, rate * unit key, unit key, key, receptance
+                coef = ws.get("delta.coef", (n, spec.num_heads, 5, spec.head_dim), torch.float32)
+                ops.delta_prepare(packed, spec.num_heads, spec.head_dim, spec.decay_rank, self.w2_t, self.w0, self.a_bias,
+                                  spec.decay_rate, spec.key_eps, coef)
+                recurrence(rt, ctx, "delta", n, *sizes, raw, ops.delta_scan, self.chunks(ops.delta_chunks), packed, coef, ctx.state(call),
+                           ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, spec.num_heads, spec.head_dim)
             ops.delta_finish(raw, packed, self.norm, spec.num_heads, spec.head_dim, spec.out_norm_eps, gated)
         y = ws.get("mixer.out", (n, spec.hidden_size), rt.dtype)
         return ops.gemm(gated, self.w_o, y, defer_sum=True) or y

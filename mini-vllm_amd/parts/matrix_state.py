@@ -99,23 +99,31 @@ def _paths(ops, rule: str, heads: int, dk: int, dv: int, lens: Sequence[int]) ->
 def recurrence(rt: Runtime, ctx, rule: str, n: int, heads: int, dk: int, dv: int, raw: torch.Tensor, scan, chunks, *operands) -> None:
     """A mixer's recurrence over the step's rows into ``raw``: requests of many tokens as products over chunks of tokens
     (``chunks``, None: not in this engine), the others, and heads of sizes these do not take, token by token (``scan``)."""
-    ops, ws, plan = rt.ops, rt.workspace, ctx.attention_plan
-    if plan is None or chunks is None:
+    in_chunks, scanned = step_paths(rt, ctx, rule, heads, dk, dv) if chunks is not None else (False, True)
+    if not in_chunks:
         scan(*operands, raw)
         return
-    line = ops.delta_chunk_line()
+    chunks(*operands, *step_chunk_scratch(rt, ctx, rule, n, heads, dk, dv), raw)
+    if scanned:
+        scan(*operands, raw, below=rt.ops.delta_chunk_line())
+
+
+def step_paths(rt: Runtime, ctx, rule: str, heads: int, dk: int, dv: int) -> Tuple[bool, bool]:
+    """Whether the step's requests of many tokens go in chunks, and whether any requests are scanned."""
+    ops, plan = rt.ops, ctx.attention_plan
+    if plan is None:
+        return False, True
     if plan.bound is None or plan.path_lens:
-        in_chunks, scanned = _paths(ops, rule, heads, dk, dv, plan.q_lens if plan.bound is None else plan.path_lens)
-    else:
-        short = plan.has_short(line)
-        in_chunks = plan.has_long(CHUNKS_BESIDE_SHORT_CLASS if short else line) and ops.delta_chunks_serve(rule, dk, dv)
-        scanned = short or not in_chunks
-    if in_chunks:
-        chunks(*operands, *_chunk_scratch(ws, rule, n, heads, dk, dv, plan.units(ops.delta_chunk_tokens(), line)), raw)
-        if scanned:
-            scan(*operands, raw, below=line)
-    else:
-        scan(*operands, raw)
+        return _paths(ops, rule, heads, dk, dv, plan.q_lens if plan.bound is None else plan.path_lens)
+    line = ops.delta_chunk_line()
+    short = plan.has_short(line)
+    in_chunks = plan.has_long(CHUNKS_BESIDE_SHORT_CLASS if short else line) and ops.delta_chunks_serve(rule, dk, dv)
+    return in_chunks, short or not in_chunks
+
+
+def step_chunk_scratch(rt: Runtime, ctx, rule: str, n: int, heads: int, dk: int, dv: int):
+    units = ctx.attention_plan.units(rt.ops.delta_chunk_tokens(), rt.ops.delta_chunk_line())
+    return _chunk_scratch(rt.workspace, rule, n, heads, dk, dv, units)
 
 
 def _chunk_scratch(ws, rule: str, n: int, heads: int, dk: int, dv: int, units: int):

@@ -163,3 +163,47 @@ def test_many_requests_and_the_scan_alone_agree(rule):
         states.append(state)
     close(rows[0], rows[1].double().cpu(), 2e-5, "rows")
     close(states[0], states[1].double().cpu(), 2e-5, "states")
+
+
+# the general rule's vectors made in the chunks' kernel: a rank of one to four blocks, requests that end inside a run and inside a chunk, of the least
+# number of tokens, with a request that brings none between them
+@pytest.mark.parametrize("H, rank, weights", [(2, 16, torch.bfloat16), (3, 64, torch.float32), (1, 48, torch.bfloat16)])
+@pytest.mark.parametrize("lens", [[128], [193, 0, 160], [145, 271]])
+def test_chunks_straight_from_the_rows(H, rank, weights, lens):
+    """Against the recurrence in float64 from the same rows: errors of float32 sums, 2^-24 a term, over what a chunk adds up."""
+    dtype, D, rate, eps, pad = torch.bfloat16, 64, 0.6, 1e-6, 8
+    ops, n = ops_for(dtype), sum(lens)
+    inner = H * D
+    g = torch.Generator().manual_seed(rank + n)
+    rows = torch.randn(n, 5 * inner + rank + pad, generator=g).to(dtype)
+    rows[:, 5 * inner + rank:] = float("nan")
+    w2t, w0, ab = ((torch.randn(*s, generator=g) * f).to(weights) for s, f in (((rank, inner), rank ** -0.5), ((inner,), 1.0), ((inner,), 1.0)))
+    f = rows.double()
+    r, k, v, _, a = (f[:, j * inner:(j + 1) * inner].view(n, H, D) for j in range(5))
+    w = torch.exp(-rate * torch.sigmoid(torch.tanh(f[:, 5 * inner:5 * inner + rank]) @ w2t.double() + w0.double())).view(n, H, D)
+    u = k / (k.pow(2).sum(-1, keepdim=True) + eps).sqrt()
+    plain = w, u, -torch.sigmoid(a + ab.double().view(H, D)) * u, k, r, v
+    slots = list(range(len(lens)))[::-1]
+    state = torch.randn(len(lens), H, D, D, generator=g)
+    packed, cu = rows.to(DEV), i32([0] + torch.tensor(lens).cumsum(0).tolist())
+    units = sum(-(-x // ops.delta_chunk_tokens()) for x in lens) + 2
+    scratch = [torch.empty(units, H, D, D, device=DEV), torch.empty(units, H, D, D, device=DEV), torch.empty(n, H, D, device=DEV)]
+    raw, dstate = torch.empty(n, inner, device=DEV), state.to(DEV)
+    weights_dev = [t.to(DEV) for t in (w2t, w0, ab)]
+    assert ops.delta_chunks_rows_serve(packed, D, rank, weights_dev[2])
+    ops.delta_chunks_rows(packed, H, D, rank, *weights_dev, rate, eps, dstate, cu, i32(slots), len(lens), *scratch, raw)
+    # ... and as close as the vectors laid out in memory are
+    coef, raw2, dstate2 = torch.empty(n, H, 5, D, device=DEV), torch.empty(n, inner, device=DEV), state.to(DEV)
+    ops.delta_prepare(packed, H, D, rank, *weights_dev, rate, eps, coef)
+    ops.delta_chunks(packed, coef, dstate2, cu, i32(slots), len(lens), H, D, *scratch, raw2)
+    first = 0
+    for s, count in enumerate(lens):
+        if count:
+            want, S = walk([t[first:first + count] for t in plain], state[slots[s]].double().transpose(1, 2))
+            for got, got2, ref in ((raw[first:first + count].view(count, H, D), raw2[first:first + count].view(count, H, D), want),
+                                   (dstate[slots[s]].transpose(1, 2), dstate2[slots[s]].transpose(1, 2), S)):
+                err, err2 = (float((x.double().cpu() - ref).norm() / ref.norm()) for x in (got, got2))
+                assert err <= 5e-6 and err <= 1.5 * err2 + 2.0 ** -24, (err, err2)
+        else:
+            assert torch.equal(dstate[slots[s]].cpu(), state[slots[s]])
+        first += count
