@@ -52,6 +52,8 @@ struct DeltaChunkArgs {
     float* M; float* N; float* Q; float* out;
     // ROWS: what the general rule's vectors are made of beside the rows (see delta_prepare_kernel)
     int rank; const void* w2t; const void* w0; const void* a_bias; int weights_f32; float decay_rate, key_eps;
+    // ... and those of the channel and gated rules (see channel_prepare_kernel, gdelta_prepare_kernel); `decay` are the rows in front of the exponentials then
+    const void* conv_w; const void* a_log; const void* dt_bias; const void* conv_state; const int* state_slots; int gate_off; float unit_eps;
 };
 
 #define DC_MAX_RANK 64             // of the decays' products: a lane holds its operands of all of it
@@ -137,7 +139,10 @@ __device__ __forceinline__ size_t quad_of(int tile_row, int rows, int k_tile, in
 // ROWS (general rule, heads of 64): the vectors are made here from the packed rows [r | k | v | g | a | w1], the decays' products over the rank on the
 // MFMA units, and not by a kernel that leaves them in memory as floats: 42 MB written and read again for 2,048 rows of 16 heads.
 // us, prepare + chunks / this: 2,048 rows 21.0 + 47.4 / 52.5, 552 rows 15.4 + 24.5 / 27.5. Where a step has requests for the scan too, those want the vectors.
-template <typename T, int DK, int RULE, bool ROWS>
+// ROWS of 2 to 4 (channel and gated rules, heads of 64 x 64): so many taps of the convolution that queries, keys and values pass first;
+// a token's four rows are read by four threads each, from L1. us, prepare + chunks / this: gated, 2,048 rows, 16 heads in 8 groups 21.5 + 41.1 / 47.1;
+// channel, 941 and 483 rows, 16 heads in 8 groups 29.2 + 36.5 / 41.4.
+template <typename T, int DK, int RULE, int ROWS>
 __global__ void __launch_bounds__(DC_THREADS)
 delta_chunk_kernel(DeltaChunkArgs A) {
     constexpr int C = DC_TOKENS, R16 = DC_RUN;
@@ -166,7 +171,7 @@ delta_chunk_kernel(DeltaChunkArgs A) {
 
     // the chunk's vectors; rows beyond its tokens change nothing (decay one, everything else zero)
     const int group = RULE == RULE_GENERAL ? head : head / (H / A.G);
-    if constexpr (ROWS) {
+    if constexpr (ROWS == 1) {
         static_assert(RULE == RULE_GENERAL && C * (DK / 4) == DC_THREADS && DK / 4 == 16 && 2 * (DK / 16) == DC_THREADS / 64, "four channels a thread, a tile of decays a wave");
         constexpr int PT = DC_MAX_RANK + 4;
         static_assert(C * PT <= (2 * MROWS + M2ROWS) * PC, "no room for the rows of the decays' products");
@@ -214,6 +219,68 @@ delta_chunk_kernel(DeltaChunkArgs A) {
             const int at = 16 * rt + 4 * g + q;
             sW[at][16 * ct + i] = at < count ? expf(-A.decay_rate * sigmoid_f(acc[q] + b0)) : 1.f;
         }
+    } else if constexpr (ROWS > 1) {
+        static_assert((RULE == RULE_CHANNEL || RULE == RULE_GATED) && C * (DK / 4) == DC_THREADS && DK / 4 == 16, "four channels a thread");
+        constexpr int TAPS = ROWS;
+        const int t = tid / 16, c = (tid % 16) * 4, G = A.G, width = 2 * G * DK + H * DK;
+        const bool ok = t < count;
+        const int row = row0 + (ok ? t : 0), first = A.cu_seqlens[seq];
+        const T* const rows = (const T*)A.vals;
+        const T* const kept = (const T*)A.conv_state + (size_t)A.state_slots[seq] * (TAPS - 1) * width;
+        const T* in[TAPS];                             // the inputs' rows: of the step, or what was kept from before it
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+            const int r = row - (TAPS - 1) + j;
+            in[j] = r >= first ? rows + (size_t)r * A.ldv : kept + (size_t)(TAPS - 1 + r - first) * width;
+        }
+        const T* const gates = rows + (size_t)row * A.ldv + A.gate_off + head;
+        const float beta = sigmoid_f(to_f(gates[0]));
+        auto make = [&](const auto* conv_w, const auto* a_log, const auto* dt_bias) __attribute__((always_inline)) {
+            auto conv = [&](int col) __attribute__((always_inline)) {
+                float w[4 * TAPS], acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int x = 0; x < TAPS; ++x) {
+                    const float4 f = four_of(conv_w + (size_t)col * TAPS + 4 * x);
+                    w[4 * x] = f.x; w[4 * x + 1] = f.y; w[4 * x + 2] = f.z; w[4 * x + 3] = f.w;
+                }
+#pragma unroll
+                for (int j = 0; j < TAPS; ++j) {
+                    const float4 f = four_of(in[j] + col);
+                    acc[0] = fmaf(w[j], f.x, acc[0]);
+                    acc[1] = fmaf(w[TAPS + j], f.y, acc[1]);
+                    acc[2] = fmaf(w[2 * TAPS + j], f.z, acc[2]);
+                    acc[3] = fmaf(w[3 * TAPS + j], f.w, acc[3]);
+                }
+                return float4{silu_f(acc[0]), silu_f(acc[1]), silu_f(acc[2]), silu_f(acc[3])};
+            };
+            auto inverse_length = [&](const float4& x) __attribute__((always_inline)) {
+                return 1.f / sqrtf(lanes_sum<16>(fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, x.w * x.w)))) + A.unit_eps);
+            };
+            const float4 q = conv(group * DK + c), k = conv(G * DK + group * DK + c), v = conv(2 * G * DK + head * DK + c);
+            float w[4];
+            const float rate = -expf(to_f(a_log[head]));
+            if constexpr (RULE == RULE_CHANNEL) {
+                const float4 z = *reinterpret_cast<const float4*>(A.decay + (size_t)row * A.ldz + (size_t)head * DK + c), bias = four_of(dt_bias + head * DK + c);
+                w[0] = expf(rate * softplus_f(z.x + bias.x));
+                w[1] = expf(rate * softplus_f(z.y + bias.y));
+                w[2] = expf(rate * softplus_f(z.z + bias.z));
+                w[3] = expf(rate * softplus_f(z.w + bias.w));
+            } else {
+                w[0] = w[1] = w[2] = w[3] = expf(rate * softplus_f(to_f(gates[H]) + to_f(dt_bias[head])));
+            }
+            const float iq = 1.f / sqrtf((float)DK) * inverse_length(q), ik = inverse_length(k);
+            const float4 u{k.x * ik, k.y * ik, k.z * ik, k.w * ik};
+            auto put = [&](float (*to)[P], float x, float y, float z, float e, float none) __attribute__((always_inline)) {
+                *reinterpret_cast<float4*>(&to[t][c]) = ok ? float4{x, y, z, e} : float4{none, none, none, none};
+            };
+            put(sW, w[0], w[1], w[2], w[3], 1.f);
+            put(sR, q.x * iq, q.y * iq, q.z * iq, q.w * iq, 0.f);
+            put(sA, w[0] * u.x, w[1] * u.y, w[2] * u.z, w[3] * u.w, 0.f);
+            put(sX, beta * u.x, beta * u.y, beta * u.z, beta * u.w, 0.f);
+            *reinterpret_cast<float4*>(&sV[t][c]) = ok ? float4{v.x, v.y, v.z, v.w} : float4{0.f, 0.f, 0.f, 0.f};
+        };
+        if (A.weights_f32) make((const float*)A.conv_w, (const float*)A.a_log, (const float*)A.dt_bias);
+        else make((const bf16*)A.conv_w, (const bf16*)A.a_log, (const bf16*)A.dt_bias);
     } else {
         for (int x = tid; x < C * (DK / 4); x += DC_THREADS) {
             const int t = x / (DK / 4), c = (x % (DK / 4)) * 4;
@@ -680,7 +747,7 @@ extern "C" int mv_delta_chunks_serve(int rule, int DK, int DV) {
     return rule >= RULE_GENERAL && rule <= RULE_SUM && (DK == 64 || DK == 128) && DV >= 1 && DV <= DK + 16;
 }
 
-template <typename T, int DK, int RULE, bool ROWS = false>
+template <typename T, int DK, int RULE, int ROWS = 0>
 static int launch_delta_chunks(const DeltaChunkArgs& A, float* state, const int* state_slots, int chunks, hipStream_t stream) {
     hipLaunchKernelGGL((delta_chunk_kernel<T, DK, RULE, ROWS>), dim3(chunks, A.H), dim3(DC_THREADS), 0, stream, A);
     if (mv_check_launch("delta_chunk")) return 1;
@@ -705,7 +772,8 @@ extern "C" int mv_delta_chunks(int rule, const float* vec, const float* gates, c
     MV_REQUIRE(H <= 65535, "delta_chunks: too many heads");
     if (n == 0 || n_seqs == 0 || chunks == 0) return 0;
     const int decay4 = ldz % 4 == 0 && (uintptr_t)decay % 16 == 0;
-    const DeltaChunkArgs A{vec, gates, decay, ldz, decay4, vals, ldv, H, G, DV, cu_seqlens, n_seqs, M, N, Q, out, 0, nullptr, nullptr, nullptr, 0, 0.f, 0.f};
+    const DeltaChunkArgs A{vec, gates, decay, ldz, decay4, vals, ldv, H, G, DV, cu_seqlens, n_seqs, M, N, Q, out, 0, nullptr, nullptr, nullptr, 0, 0.f, 0.f,
+                           nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0.f};
 #define DC_LAUNCH(T, RULE)                                                                                   \
     return DK == 64 ? launch_delta_chunks<T, 64, RULE>(A, state, state_slots, chunks, stream)               \
                     : launch_delta_chunks<T, 128, RULE>(A, state, state_slots, chunks, stream)
@@ -734,7 +802,53 @@ extern "C" int mv_delta_chunks_rows(const void* packed, long ld, int rank, const
                && (uintptr_t)Q % 16 == 0, "delta_chunks_rows: operands must be 16-byte aligned");
     if (n == 0 || n_seqs == 0 || chunks == 0) return 0;
     const DeltaChunkArgs A{nullptr, nullptr, nullptr, 0, 0, packed, ld, H, H, D, cu_seqlens, n_seqs, M, N, Q, out, rank, w2t, w0, a_bias,
-                           weight_dtype == MV_F32, decay_rate, key_eps};
-    MV_DISPATCH_T(dtype, "delta_chunks_rows", { return (launch_delta_chunks<T, 64, RULE_GENERAL, true>(A, state, state_slots, chunks, stream)); });
+                           weight_dtype == MV_F32, decay_rate, key_eps, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0.f};
+    MV_DISPATCH_T(dtype, "delta_chunks_rows", { return (launch_delta_chunks<T, 64, RULE_GENERAL, 1>(A, state, state_slots, chunks, stream)); });
     return 0;
+}
+
+// 1: mv_delta_chunks_conv serves heads of these sizes, so many taps, rows this far apart (ldz: the decays', 0: none)
+extern "C" int mv_delta_chunks_conv_serve(int DK, int DV, int taps, long ld, long ldz) {
+    return DK == 64 && DV == 64 && taps >= 2 && taps <= 4 && ld % 8 == 0 && ldz % 4 == 0;
+}
+
+// mv_delta_chunks under the channel or the gated rule straight from the packed rows, without the vectors of mv_channel_prepare and mv_gdelta_prepare
+// (ROWS above), and the convolution's kept inputs moved on behind it. gate_off: the column of the strengths, the gated rule's decays H behind them;
+// z: the channel rule's decays in front of bias and exponential, rows ldz apart, left as they are.
+extern "C" int mv_delta_chunks_conv(int rule, const void* packed, long ld, int gate_off, int taps, const void* conv_w, const void* a_log, const void* dt_bias,
+                                    int weight_dtype, void* conv_state, float unit_eps, const float* z, long ldz, float* state, const int* cu_seqlens,
+                                    const int* state_slots, int n_seqs, int n, int H, int G, int DK, int DV, int chunks, float* M, float* N, float* Q, float* out,
+                                    int dtype, hipStream_t stream) {
+    const bool channel = rule == RULE_CHANNEL;
+    MV_REQUIRE(n >= 0 && n_seqs >= 0 && H > 0 && H <= 65535 && G > 0 && H % G == 0 && chunks >= 0, "delta_chunks_conv: bad sizes n=%d seqs=%d H=%d G=%d", n, n_seqs, H, G);
+    MV_REQUIRE((channel || rule == RULE_GATED) && mv_delta_chunks_conv_serve(DK, DV, taps, ld, channel ? ldz : 0),
+               "delta_chunks_conv: rule %d with heads of %d x %d, %d taps, rows of %ld is not served", rule, DK, DV, taps, ld);
+    const long width = 2L * G * DK + (long)H * DV;
+    MV_REQUIRE(gate_off >= width && ld >= (long)gate_off + (channel ? 1 : 2) * H, "delta_chunks_conv: rows of %ld columns are too short", ld);
+    MV_REQUIRE(packed && conv_w && a_log && dt_bias && conv_state && state && cu_seqlens && state_slots && M && N && Q && out
+               && (!channel || (z && ldz >= (long)H * DK)), "delta_chunks_conv: missing operand");
+    MV_REQUIRE(mv_valid_dtype(weight_dtype) && unit_eps > 0.f && (width + 255) / 256 <= 65535, "delta_chunks_conv: bad constants");
+    MV_REQUIRE(((uintptr_t)packed | (uintptr_t)conv_w | (uintptr_t)dt_bias | (uintptr_t)conv_state | (uintptr_t)z | (uintptr_t)state | (uintptr_t)M | (uintptr_t)N
+                | (uintptr_t)Q) % 16 == 0, "delta_chunks_conv: operands must be 16-byte aligned");
+    if (n == 0 || n_seqs == 0 || chunks == 0) return 0;
+    const DeltaChunkArgs A{nullptr, nullptr, z, ldz, 1, packed, ld, H, G, DV, cu_seqlens, n_seqs, M, N, Q, out, 0, nullptr, nullptr, nullptr,
+                           weight_dtype == MV_F32, 0.f, 0.f, conv_w, a_log, dt_bias, conv_state, state_slots, gate_off, unit_eps};
+    int rc = 1;
+#define DC_CONV(RULE)                                                                                                            \
+    MV_DISPATCH_T(dtype, "delta_chunks_conv", {                                                                                  \
+        rc = taps == 4   ? launch_delta_chunks<T, 64, RULE, 4>(A, state, state_slots, chunks, stream)                            \
+             : taps == 3 ? launch_delta_chunks<T, 64, RULE, 3>(A, state, state_slots, chunks, stream)                            \
+                         : launch_delta_chunks<T, 64, RULE, 2>(A, state, state_slots, chunks, stream);                           \
+    })
+    if (channel) {
+        DC_CONV(RULE_CHANNEL);
+    } else {
+        DC_CONV(RULE_GATED);
+    }
+#undef DC_CONV
+    if (rc) return rc;
+    MV_DISPATCH_T(dtype, "conv_state",
+                  hipLaunchKernelGGL(conv_state_kernel<T>, dim3(n_seqs, (unsigned)((width + 255) / 256)), dim3(256), 0, stream, (const T*)packed, ld, (int)width,
+                                     taps, (T*)conv_state, cu_seqlens, state_slots));
+    return mv_check_launch("conv_state");
 }

@@ -832,6 +832,54 @@ class Ops:
                       a_bias.data_ptr(), wcode, float(decay_rate), float(key_eps), state.data_ptr(), cu_seqlens.data_ptr(), state_slots.data_ptr(),
                       n_seqs, n, heads, dim, chunks, maps.data_ptr(), sums.data_ptr(), queries.data_ptr(), out.data_ptr(), self.code, self._stream())
 
+    def delta_chunks_conv_serve(self, packed: torch.Tensor, dk: int, dv: int, taps: int, conv_w: torch.Tensor, dt_bias: torch.Tensor,
+                                conv_state: Optional[torch.Tensor], z: Optional[torch.Tensor] = None) -> bool:
+        """Whether ``delta_chunks_conv`` takes these rows."""
+        if conv_state is None or not self.lib.has("mv_delta_chunks_conv"):
+            return False
+        pitch = lambda t: t.stride(0) if t.shape[0] > 1 else t.shape[1]
+        return (all(t.data_ptr() % 16 == 0 for t in (packed, conv_w, dt_bias, conv_state) + (() if z is None else (z,)))
+                and bool(self.lib.dll.mv_delta_chunks_conv_serve(dk, dv, taps, pitch(packed), 0 if z is None else pitch(z))))
+
+    def delta_chunks_conv(self, rule: str, packed: torch.Tensor, gate_off: int, heads: int, groups: int, dk: int, dv: int, taps: int,
+                          conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor, conv_state: torch.Tensor, unit_eps: float,
+                          z: Optional[torch.Tensor], state: torch.Tensor, cu_seqlens: torch.Tensor, state_slots: torch.Tensor, n_seqs: int,
+                          maps: torch.Tensor, sums: torch.Tensor, queries: torch.Tensor, out: torch.Tensor) -> None:
+        """``gated_delta_prepare`` and ``state_chunks`` ("gated"), or ``channel_prepare`` and ``channel_chunks`` ("channel", ``z`` left as it
+        is), in one, for steps whose requests all bring ``delta_chunk_line`` tokens and more: the vectors never lie in memory. ``gate_off``: the
+        column of the strengths, the gated rule's decays behind them."""
+        what, channel = "delta_chunks_conv", rule == "channel"
+        self._act(packed, "delta rows"); self._act(conv_state, "convolution state")
+        n, C, chunks = packed.shape[0], 2 * groups * dk + heads * dv, sums.shape[0]
+        if packed.dim() != 2 or packed.stride(1) != 1 or packed.shape[1] < gate_off + (1 if channel else 2) * heads or gate_off < C:
+            raise KernelLibraryError(f"{what}: rows {tuple(packed.shape)} are too short")
+        if conv_state.dim() != 3 or tuple(conv_state.shape[1:]) != (taps - 1, C) or not conv_state.is_contiguous():
+            raise KernelLibraryError(f"{what}: the convolution's state must be [slots, {taps - 1}, {C}]")
+        bias = heads * dk if channel else heads
+        for t, numel, name in ((conv_w, C * taps, "convolution taps"), (a_log, heads, "A_log"), (dt_bias, bias, "dt_bias")):
+            _dev(t, name)
+            if t.numel() != numel or not t.is_contiguous() or t.dtype != conv_w.dtype:
+                raise KernelLibraryError(f"{what}: {name} must be {numel} contiguous elements of the taps' dtype")
+        if channel:
+            _dev(z, "decay rows")
+            if z.dtype != torch.float32 or z.dim() != 2 or z.shape[0] != n or z.shape[1] < heads * dk or z.stride(1) != 1:
+                raise KernelLibraryError(f"{what}: decay rows must be float32 [{n}, >= {heads * dk}]")
+        for t, shape, name in ((maps, (chunks, heads, dk, dk), "chunk maps"), (sums, (chunks, heads, dv, dk), "chunk sums"),
+                               (queries, (n, heads, dk), "chunk queries"), (out, (n, heads, dv), "output"), (state, (state.shape[0], heads, dv, dk), "state")):
+            _dev(t, name)
+            if t.dtype != torch.float32 or tuple(t.shape) != shape or not t.is_contiguous():
+                raise KernelLibraryError(f"{what}: the {name} must be contiguous float32 {shape}")
+        self._ints(n, cu_seqlens=(cu_seqlens, n_seqs + 1), state_slots=(state_slots, n_seqs))
+        size = (n * (C + 2 * heads) * packed.element_size() + self._size(conv_w, out) + 2 * self._size(maps, sums, queries)
+                + (4 * n * heads * dk if channel else 0) + 2 * min(n_seqs, max(n, 1)) * heads * dv * dk * 4)
+        c = self.delta_chunk_tokens()
+        self._note("mv_delta_chunks_conv", size, 2 * n * C * taps + n * heads * (2 * c * (2 * dk + dv) + 4 * dk * (dk + dv)))
+        self.lib.call("mv_delta_chunks_conv", self.CHUNK_RULES[rule], packed.data_ptr(), packed.stride(0) if n > 1 else packed.shape[1], int(gate_off), taps,
+                      conv_w.data_ptr(), a_log.data_ptr(), dt_bias.data_ptr(), _weight_code(conv_w, "convolution taps"), conv_state.data_ptr(),
+                      float(unit_eps), _ptr(z), 0 if z is None else (z.stride(0) if n > 1 else z.shape[1]), state.data_ptr(), cu_seqlens.data_ptr(),
+                      state_slots.data_ptr(), n_seqs, n, heads, groups, dk, dv, chunks, maps.data_ptr(), sums.data_ptr(), queries.data_ptr(), out.data_ptr(),
+                      self.code, self._stream())
+
     def delta_step(self, packed: torch.Tensor, heads: int, dim: int, rank: int, w2t: torch.Tensor, w0: torch.Tensor,
                    a_bias: torch.Tensor, norm_weight: torch.Tensor, decay_rate: float, key_eps: float, eps: float,
                    state: torch.Tensor, token_seq: torch.Tensor, state_slots: torch.Tensor, out: torch.Tensor) -> None:

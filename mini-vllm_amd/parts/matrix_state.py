@@ -236,15 +236,21 @@ class GatedDelta(ChunkedRecurrence):
                 dt_bias=self.dt_bias, conv_state=ctx.state(call, "conv") if spec.conv_taps > 1 else None,
                 unit_eps=spec.unit_eps):
             return ops.gemm(gated, self.w_o, y, defer_sum=True) or y
-        qk = ws.get("mstate.qk", (n, G, 2, dk), torch.float32)
-        vals = ws.get("mstate.vals", (n, H, dv), torch.float32)
+        conv_state = ctx.state(call, "conv") if spec.conv_taps > 1 else None
         gates = ws.get("mstate.gates", (n, H, 4), torch.float32)
-        ops.gated_delta_prepare(packed, H, G, dk, dv, spec.conv_taps, self.conv_w, self.a_log, self.dt_bias,
-                                ctx.state(call, "conv") if spec.conv_taps > 1 else None, spec.unit_eps, ctx.token_seq,
-                                ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, gates)
         raw = ws.get("mstate.raw", (n, H, dv), torch.float32)
-        recurrence(rt, ctx, "gated", n, H, dk, dv, raw, ops.state_scan, self.chunks(ops.state_chunks), qk, vals, gates,
-                   ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv, True)
+        if (self.chunks(ops.state_chunks) is not None and step_paths(rt, ctx, "gated", H, dk, dv) == (True, False)
+                and ops.delta_chunks_conv_serve(packed, dk, dv, spec.conv_taps, self.conv_w, self.dt_bias, conv_state)):
+            ops.delta_chunks_conv("gated", packed, 2 * G * dk + 2 * H * dv, H, G, dk, dv, spec.conv_taps, self.conv_w, self.a_log, self.dt_bias,
+                                  conv_state, spec.unit_eps, None, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs,
+                                  *step_chunk_scratch(rt, ctx, "gated", n, H, dk, dv), raw)
+        else:
+            qk = ws.get("mstate.qk", (n, G, 2, dk), torch.float32)
+            vals = ws.get("mstate.vals", (n, H, dv), torch.float32)
+            ops.gated_delta_prepare(packed, H, G, dk, dv, spec.conv_taps, self.conv_w, self.a_log, self.dt_bias, conv_state, spec.unit_eps,
+                                    ctx.token_seq, ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, gates)
+            recurrence(rt, ctx, "gated", n, H, dk, dv, raw, ops.state_scan, self.chunks(ops.state_chunks), qk, vals, gates,
+                       ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv, True)
         ops.state_finish(raw, gates, packed, self.gate_offset, self.norm, H, dv, spec.out_norm_eps, ctx.token_seq, gated,
                          shared_weight=True, silu_gate=True)
         return ops.gemm(gated, self.w_o, y, defer_sum=True) or y
@@ -412,14 +418,20 @@ class ChannelDelta(ChunkedRecurrence):
             return ops.gemm(gated, self.w_o, y, defer_sum=True, fold=fold) or y
         z = ws.get("mstate.z", (n, H * (dk + dv)), torch.float32)
         ops.gemm(packed[:, self.low_offset:self.low_offset + self.low_width], self.w_second, z)
-        qk = ws.get("mstate.qk", (n, G, 2, dk), torch.float32)
-        vals = ws.get("mstate.vals", (n, H, dv), torch.float32)
-        beta = ws.get("mstate.beta", (n, H), torch.float32)
-        ops.channel_prepare(packed, H, G, dk, dv, spec.conv_taps, self.b_offset, self.conv_w, self.a_log, self.dt_bias, conv_state,
-                            spec.unit_eps, ctx.token_seq, ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, beta, z)
         raw = ws.get("mstate.raw", (n, H, dv), torch.float32)
-        recurrence(rt, ctx, "channel", n, H, dk, dv, raw, ops.channel_scan, self.chunks(ops.channel_chunks), qk, vals, beta, z,
-                   ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv)
+        if (self.chunks(ops.channel_chunks) is not None and step_paths(rt, ctx, "channel", H, dk, dv) == (True, False)
+                and ops.delta_chunks_conv_serve(packed, dk, dv, spec.conv_taps, self.conv_w, self.dt_bias, conv_state, z)):
+            ops.delta_chunks_conv("channel", packed, self.b_offset, H, G, dk, dv, spec.conv_taps, self.conv_w, self.a_log, self.dt_bias, conv_state,
+                                  spec.unit_eps, z, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs,
+                                  *step_chunk_scratch(rt, ctx, "channel", n, H, dk, dv), raw)
+        else:
+            qk = ws.get("mstate.qk", (n, G, 2, dk), torch.float32)
+            vals = ws.get("mstate.vals", (n, H, dv), torch.float32)
+            beta = ws.get("mstate.beta", (n, H), torch.float32)
+            ops.channel_prepare(packed, H, G, dk, dv, spec.conv_taps, self.b_offset, self.conv_w, self.a_log, self.dt_bias, conv_state,
+                                spec.unit_eps, ctx.token_seq, ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, beta, z)
+            recurrence(rt, ctx, "channel", n, H, dk, dv, raw, ops.channel_scan, self.chunks(ops.channel_chunks), qk, vals, beta, z,
+                       ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, G, dk, dv)
         ops.state_finish(raw, None, z, H * dk, self.norm, H, dv, spec.out_norm_eps, ctx.token_seq, gated, shared_weight=True,
                          silu_gate=False)
         return ops.gemm(gated, self.w_o, y, defer_sum=True, fold=fold) or y

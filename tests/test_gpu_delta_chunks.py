@@ -207,3 +207,51 @@ def test_chunks_straight_from_the_rows(H, rank, weights, lens):
         else:
             assert torch.equal(dstate[slots[s]].cpu(), state[slots[s]])
         first += count
+
+
+# the convolution's rules' vectors made in the chunks' kernel: every number of taps, groups of one and two heads, requests that start behind kept inputs,
+# end inside a run and inside a chunk, bring the least number of tokens or none
+@pytest.mark.parametrize("rule", ["gated", "channel"])
+@pytest.mark.parametrize("H, G, taps, weights", [(2, 1, 4, torch.bfloat16), (3, 3, 3, torch.float32), (4, 2, 2, torch.bfloat16)])
+@pytest.mark.parametrize("lens", [[128], [193, 0, 160], [145, 271]])
+def test_chunks_straight_from_convolved_rows(rule, H, G, taps, weights, lens):
+    """Against the vectors laid out in memory and the chunks behind them: the same terms, whose lengths are added up in another order, 2^-24 a term over
+    the 64 channels of a length and the tokens of a request. The kept inputs are the same bits."""
+    dtype, D, eps = torch.bfloat16, 64, 1e-6
+    ops, n, channel = ops_for(dtype), sum(lens), rule == "channel"
+    C = 2 * G * D + H * D
+    gate_off = C + H * D
+    g = torch.Generator().manual_seed(17 * taps + n)
+    rand = lambda *s: torch.randn(*s, generator=g)
+    packed = rand(n, (gate_off + 2 * H + 7) // 8 * 8 + 8).to(dtype).to(DEV)
+    conv_w, a_log = (rand(C, taps) / taps ** 0.5).to(weights).to(DEV), (rand(H) - 1).to(weights).to(DEV)
+    dt_bias = rand(H * D if channel else H).to(weights).to(DEV)
+    kept, state = rand(len(lens) + 1, taps - 1, C).to(dtype).to(DEV), rand(len(lens) + 1, H, D, D).to(DEV)
+    z = rand(n, 2 * H * D).to(DEV) if channel else None
+    ends = torch.tensor([0] + lens).cumsum(0).tolist()
+    cu, slots, count = i32(ends), i32(list(range(len(lens), 0, -1))), len(lens)
+    token_seq = i32([s for s, q in enumerate(lens) for _ in range(q)])
+    units = sum(-(-x // ops.delta_chunk_tokens()) for x in lens) + 2
+    scratch = [torch.empty(units, H, D, D, device=DEV), torch.empty(units, H, D, D, device=DEV), torch.empty(n, H, D, device=DEV)]
+    results = []
+    for straight in (True, False):
+        k2, s2, raw, z2 = kept.clone(), state.clone(), torch.empty(n, H, D, device=DEV), z.clone() if channel else None
+        if straight:
+            assert ops.delta_chunks_conv_serve(packed, D, D, taps, conv_w, dt_bias, k2, z2)
+            ops.delta_chunks_conv(rule, packed, gate_off, H, G, D, D, taps, conv_w, a_log, dt_bias, k2, eps, z2, s2, cu, slots, count, *scratch, raw)
+            assert z2 is None or torch.equal(z2, z)
+        else:
+            qk, vals = torch.empty(n, G, 2, D, device=DEV), torch.empty(n, H, D, device=DEV)
+            if channel:
+                beta = torch.empty(n, H, device=DEV)
+                ops.channel_prepare(packed, H, G, D, D, taps, gate_off, conv_w, a_log, dt_bias, k2, eps, token_seq, cu, slots, count, qk, vals, beta, z2)
+                ops.channel_chunks(qk, vals, beta, z2, s2, cu, slots, count, H, G, D, D, *scratch, raw)
+            else:
+                gates = torch.empty(n, H, 4, device=DEV)
+                ops.gated_delta_prepare(packed, H, G, D, D, taps, conv_w, a_log, dt_bias, k2, eps, token_seq, cu, slots, count, qk, vals, gates)
+                ops.state_chunks(qk, vals, gates, s2, cu, slots, count, H, G, D, D, True, *scratch, raw)
+        results.append((raw, s2, k2))
+    for got, want in zip(results[0][:2], results[1][:2]):
+        assert bool(torch.isfinite(want).all())
+        assert float((got.double() - want.double()).norm() / want.double().norm()) <= 16 * 2.0 ** -24 * 64 ** 0.5
+    assert torch.equal(results[0][2], results[1][2])
