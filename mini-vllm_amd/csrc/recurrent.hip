@@ -993,7 +993,7 @@ extern "C" int mv_mlstm_prepare(const void* packed, long ld, int n, int n_seqs, 
     const long gate_off = 2L * H * DK + 2L * H * DV;
     MV_REQUIRE(ld >= gate_off + 2L * H, "mlstm_prepare: rows of %ld columns are too short", ld);
     MV_REQUIRE(mv_valid_dtype(weight_dtype) && packed && i_bias && f_bias && max_state && token_seq && cu_seqlens && state_slots
-               && qk && vals && gates, "mlstm_prepare: missing operand");
+               && gates && (qk == nullptr) == (vals == nullptr), "mlstm_prepare: missing operand");
     MV_REQUIRE(cap > 0.f && H <= 65535, "mlstm_prepare: bad constants");
     if (n == 0 || n_seqs == 0) return 0;
     WeightPtr ib{i_bias, weight_dtype}, fb{f_bias, weight_dtype};
@@ -1003,6 +1003,7 @@ extern "C" int mv_mlstm_prepare(const void* packed, long ld, int n, int n_seqs, 
                   hipLaunchKernelGGL(mlstm_gates_kernel<T>, dim3(n_seqs, H), dim3(threads), 0, stream, (const T*)packed, ld, H,
                                      gate_off, ib, fb, cap, max_state, cu_seqlens, state_slots, gates));
     if (mv_check_launch("mlstm_gates")) return 1;
+    if (qk == nullptr) return 0;               // the gates alone
     MV_DISPATCH_T(dtype, "mlstm_prepare",
                   hipLaunchKernelGGL(mlstm_prepare_kernel<T>, dim3(n, H), dim3(128), 0, stream, (const T*)packed, ld, H, DK, DV,
                                      token_seq, qk, vals));

@@ -139,6 +139,7 @@ __device__ __forceinline__ size_t quad_of(int tile_row, int rows, int k_tile, in
 // ROWS (general rule, heads of 64): the vectors are made here from the packed rows [r | k | v | g | a | w1], the decays' products over the rank on the
 // MFMA units, and not by a kernel that leaves them in memory as floats: 42 MB written and read again for 2,048 rows of 16 heads.
 // us, prepare + chunks / this: 2,048 rows 21.0 + 47.4 / 52.5, 552 rows 15.4 + 24.5 / 27.5. Where a step has requests for the scan too, those want the vectors.
+// The mLSTM's (heads of 64 x 64) too: prepare + chunks / this at 2,048 rows of 16 heads 14.7 + 29.6 / 25.6.
 // ROWS of 2 to 4 (channel and gated rules, heads of 64 x 64): so many taps of the convolution that queries, keys and values pass first;
 // a token's four rows are read by four threads each, from L1. us, prepare + chunks / this: gated, 2,048 rows, 16 heads in 8 groups 21.5 + 41.1 / 47.1;
 // channel, 941 and 483 rows, 16 heads in 8 groups 29.2 + 36.5 / 41.4.
@@ -171,7 +172,25 @@ delta_chunk_kernel(DeltaChunkArgs A) {
 
     // the chunk's vectors; rows beyond its tokens change nothing (decay one, everything else zero)
     const int group = RULE == RULE_GENERAL ? head : head / (H / A.G);
-    if constexpr (ROWS == 1) {
+    if constexpr (ROWS == 1 && RULE == RULE_SUM) {
+        // (the scan's floats, bit for bit: the gates are there, the values have a column of ones behind them)
+        static_assert(C * (DK / 4) == DC_THREADS && DVMAX == DK + 16, "four channels a thread");
+        const int t = tid / 16, c = (tid % 16) * 4;
+        const bool ok = t < count;
+        const size_t row = row0 + (ok ? t : 0);
+        const T* p = (const T*)A.vals + row * A.ldv + (size_t)head * DK + c;
+        const size_t inner = (size_t)H * DK;
+        const float4 q = four_of(p), k = four_of(p + inner), v = four_of(p + 2 * inner);
+        const float w = A.gates[(row * H + head) * 4], b = A.gates[(row * H + head) * 4 + 1], qs = 1.f / sqrtf((float)DK);
+        auto put = [&](float* to, float x, float y, float z, float e, float none) __attribute__((always_inline)) {
+            *reinterpret_cast<float4*>(to) = ok ? float4{x, y, z, e} : float4{none, none, none, none};
+        };
+        put(&sW[t][c], w, w, w, w, 1.f);
+        put(&sX[t][c], k.x, k.y, k.z, k.w, 0.f);
+        put(&sR[t][c], q.x * qs, q.y * qs, q.z * qs, q.w * qs, 0.f);
+        put(&sV[t][c], v.x * b, v.y * b, v.z * b, v.w * b, 0.f);
+        if (c < 16) put(&sV[t][DK + c], c == 0 ? b : 0.f, 0.f, 0.f, 0.f, 0.f);
+    } else if constexpr (ROWS == 1) {
         static_assert(RULE == RULE_GENERAL && C * (DK / 4) == DC_THREADS && DK / 4 == 16 && 2 * (DK / 16) == DC_THREADS / 64, "four channels a thread, a tile of decays a wave");
         constexpr int PT = DC_MAX_RANK + 4;
         static_assert(C * PT <= (2 * MROWS + M2ROWS) * PC, "no room for the rows of the decays' products");
@@ -851,4 +870,19 @@ extern "C" int mv_delta_chunks_conv(int rule, const void* packed, long ld, int g
                   hipLaunchKernelGGL(conv_state_kernel<T>, dim3(n_seqs, (unsigned)((width + 255) / 256)), dim3(256), 0, stream, (const T*)packed, ld, (int)width,
                                      taps, (T*)conv_state, cu_seqlens, state_slots));
     return mv_check_launch("conv_state");
+}
+
+// mv_delta_chunks under the mLSTM's rule straight from the packed rows [q | k | v | ..] of heads of 64 x 64 and the gates that mv_mlstm_prepare
+// leaves; DV = 65 columns, the last one the normaliser. Rows ld apart, a multiple of eight.
+extern "C" int mv_delta_chunks_sum_rows(const void* packed, long ld, const float* gates, float* state, const int* cu_seqlens, const int* state_slots, int n_seqs,
+                                        int n, int H, int chunks, float* M, float* N, float* Q, float* out, int dtype, hipStream_t stream) {
+    MV_REQUIRE(n >= 0 && n_seqs >= 0 && H > 0 && H <= 65535 && chunks >= 0, "delta_chunks_sum_rows: bad sizes n=%d seqs=%d H=%d", n, n_seqs, H);
+    MV_REQUIRE(ld >= 3L * H * 64 && ld % 8 == 0, "delta_chunks_sum_rows: rows of %ld columns are not served", ld);
+    MV_REQUIRE(packed && gates && state && cu_seqlens && state_slots && M && N && Q && out, "delta_chunks_sum_rows: missing operand");
+    MV_REQUIRE(((uintptr_t)packed | (uintptr_t)state | (uintptr_t)N | (uintptr_t)Q) % 16 == 0, "delta_chunks_sum_rows: operands must be 16-byte aligned");
+    if (n == 0 || n_seqs == 0 || chunks == 0) return 0;
+    const DeltaChunkArgs A{nullptr, gates, nullptr, 0, 0, packed, ld, H, H, 65, cu_seqlens, n_seqs, M, N, Q, out, 0, nullptr, nullptr, nullptr, 0, 0.f, 0.f,
+                           nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0.f};
+    MV_DISPATCH_T(dtype, "delta_chunks_sum_rows", { return (launch_delta_chunks<T, 64, RULE_SUM, 1>(A, state, state_slots, chunks, stream)); });
+    return 0;
 }

@@ -65,6 +65,7 @@ KERNELS_OF: Dict[str, Tuple[str, Optional[str], int]] = {
     "mv_state_scan": (r"\bstate_scan_kernel", None, 1),
     "mv_delta_chunks": (r"\bdelta_chunk_kernel", r"\bdelta_chunk_walk_kernel", 2),
     "mv_delta_chunks_conv": (r"\bdelta_chunk_kernel", r"\b(delta_chunk_walk|conv_state)_kernel", 3),
+    "mv_delta_chunks_sum_rows": (r"\bdelta_chunk_kernel", r"\bdelta_chunk_walk_kernel", 2),
     "mv_delta_chunks_rows": (r"\bdelta_chunk_kernel", r"\bdelta_chunk_walk_kernel", 2),
     "mv_state_finish": (r"\bstate_finish(_head)?_kernel", None, 1),
     "mv_state_step": (r"\bstate_step_kernel", r"\bconv_state_kernel", 2),

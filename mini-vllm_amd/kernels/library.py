@@ -355,6 +355,9 @@ _OPTIONAL_SIGNATURES = {
     # out, dtype, stream
     "mv_delta_chunks_rows": (c_int, [c_void_p, c_long, c_int, c_void_p, c_void_p, c_void_p, c_int, c_float, c_float, c_void_p, c_void_p, c_void_p,
                                      c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
+    # packed, ld, gates, state, cu_seqlens, state_slots, n_seqs, n, H, chunks, M, N, Q, out, dtype, stream
+    "mv_delta_chunks_sum_rows": (c_int, [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
+                                         c_void_p, c_void_p, c_int, c_void_p]),
     "mv_delta_chunks_conv_serve": (c_int, [c_int, c_int, c_int, c_long, c_long]),
     # rule, packed, ld, gate_off, taps, conv_w, a_log, dt_bias, weight_dtype, conv_state, unit_eps, z, ldz, state, cu_seqlens, state_slots, n_seqs,
     # n, H, G, DK, DV, chunks, M, N, Q, out, dtype, stream

@@ -960,16 +960,20 @@ class Ops:
 
     def mlstm_prepare(self, packed: torch.Tensor, heads: int, dk: int, dv: int, i_bias: torch.Tensor, f_bias: torch.Tensor,
                       cap: float, max_state: torch.Tensor, token_seq: torch.Tensor, cu_seqlens: torch.Tensor,
-                      state_slots: torch.Tensor, n_seqs: int, qk: torch.Tensor, vals: torch.Tensor, gates: torch.Tensor) -> None:
+                      state_slots: torch.Tensor, n_seqs: int, qk: Optional[torch.Tensor], vals: Optional[torch.Tensor], gates: torch.Tensor) -> None:
         """From rows [q | k (heads*dk each) | v | g (heads*dv each) | i | f (heads each)]: q * dk^-1/2 and k as floats,
         the values with a one behind them (vals [n, heads, dv + 1]), and the stabilised gates: with
         i' = cap tanh((i + i_bias)/cap), f' = logsigmoid(cap tanh((f + f_bias)/cap)) and the running maximum
-        m' = max(f' + m, i') (max_state [slots, heads], read and advanced), gates = (exp(f' + m - m'), exp(i' - m'), exp(-m'), 0)."""
+        m' = max(f' + m, i') (max_state [slots, heads], read and advanced), gates = (exp(f' + m - m'), exp(i' - m'), exp(-m'), 0).
+        ``qk`` and ``vals`` None: the gates alone (``mlstm_chunks``)."""
         self._act(packed, "mlstm rows")
         n = packed.shape[0]
         if packed.dim() != 2 or packed.stride(1) != 1 or packed.shape[1] < 2 * heads * (dk + dv) + 2 * heads:
             raise KernelLibraryError(f"mlstm_prepare: rows {tuple(packed.shape)} are too short")
-        self._state_vectors(n, heads, heads, dk, dv + 1, qk, vals, gates, "mlstm_prepare")
+        if qk is not None:
+            self._state_vectors(n, heads, heads, dk, dv + 1, qk, vals, gates, "mlstm_prepare")
+        elif vals is not None or gates.dtype != torch.float32 or tuple(gates.shape) != (n, heads, 4) or not gates.is_contiguous() or not gates.is_cuda:
+            raise KernelLibraryError(f"mlstm_prepare: gates alone must be contiguous float32 {(n, heads, 4)}")
         for t, name in ((i_bias, "input gate bias"), (f_bias, "forget gate bias")):
             _dev(t, name)
             if t.numel() != heads or not t.is_contiguous() or t.dtype != i_bias.dtype:
@@ -978,12 +982,41 @@ class Ops:
         if max_state.dtype != torch.float32 or max_state.dim() != 2 or max_state.shape[1] != heads or not max_state.is_contiguous():
             raise KernelLibraryError(f"mlstm_prepare: the running maximum must be float32 [slots, {heads}]")
         self._ints(n, token_seq=(token_seq, n), cu_seqlens=(cu_seqlens, n_seqs + 1), state_slots=(state_slots, n_seqs))
-        self._note("mv_mlstm_prepare", n * (2 * heads * dk + heads * dv + 2 * heads) * packed.element_size() + self._size(qk, vals, gates),
+        self._note("mv_mlstm_prepare", n * (2 * heads * dk + heads * dv + 2 * heads) * packed.element_size() + self._size(*(t for t in (qk, vals, gates) if t is not None)),
                    40 * n * heads)
         self.lib.call("mv_mlstm_prepare", packed.data_ptr(), packed.stride(0) if n > 1 else packed.shape[1], n, n_seqs, heads, dk,
                       dv, i_bias.data_ptr(), f_bias.data_ptr(), _weight_code(i_bias, "gate bias"), float(cap),
-                      max_state.data_ptr(), token_seq.data_ptr(), cu_seqlens.data_ptr(), state_slots.data_ptr(), qk.data_ptr(),
-                      vals.data_ptr(), gates.data_ptr(), self.code, self._stream())
+                      max_state.data_ptr(), token_seq.data_ptr(), cu_seqlens.data_ptr(), state_slots.data_ptr(), _ptr(qk),
+                      _ptr(vals), gates.data_ptr(), self.code, self._stream())
+
+    def mlstm_chunks_serve(self, packed: torch.Tensor, dk: int, dv: int) -> bool:
+        """Whether ``mlstm_chunks`` takes these rows."""
+        ld = packed.stride(0) if packed.shape[0] > 1 else packed.shape[1]
+        return self.lib.has("mv_delta_chunks_sum_rows") and dk == 64 and dv == 64 and ld % 8 == 0 and packed.data_ptr() % 16 == 0
+
+    def mlstm_chunks(self, packed: torch.Tensor, gates: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor, state_slots: torch.Tensor,
+                     n_seqs: int, heads: int, dk: int, dv: int, maps: torch.Tensor, sums: torch.Tensor, queries: torch.Tensor,
+                     out: torch.Tensor) -> None:
+        """``state_chunks`` for the mLSTM's packed rows and the gates of ``mlstm_prepare`` without its vectors, for steps whose requests all bring
+        ``delta_chunk_line`` tokens and more: the same bits."""
+        self._act(packed, "mlstm rows")
+        n, chunks = packed.shape[0], sums.shape[0]
+        if packed.dim() != 2 or packed.stride(1) != 1 or packed.shape[1] < 2 * heads * dk + heads * dv or not self.mlstm_chunks_serve(packed, dk, dv):
+            raise KernelLibraryError(f"mlstm_chunks: rows {tuple(packed.shape)} with heads of {dk} x {dv} are not served")
+        for t, shape, name in ((gates, (n, heads, 4), "gates"), (maps, (chunks, heads), "chunk maps"), (sums, (chunks, heads, dv + 1, dk), "chunk sums"),
+                               (queries, (n, heads, dk), "chunk queries"), (out, (n, heads, dv + 1), "output"),
+                               (state, (state.shape[0], heads, dv + 1, dk), "state")):
+            _dev(t, name)
+            if t.dtype != torch.float32 or tuple(t.shape) != shape or not t.is_contiguous():
+                raise KernelLibraryError(f"mlstm_chunks: the {name} must be contiguous float32 {shape}")
+        self._ints(n, cu_seqlens=(cu_seqlens, n_seqs + 1), state_slots=(state_slots, n_seqs))
+        c, dvs = self.delta_chunk_tokens(), dv + 1
+        self._note("mv_delta_chunks_sum_rows", n * (2 * heads * dk + heads * dv) * packed.element_size() + self._size(gates, out)
+                   + 2 * self._size(maps, sums, queries) + 2 * min(n_seqs, max(n, 1)) * heads * dvs * dk * 4,
+                   n * heads * (2 * c * (2 * dk + dvs) + 2 * dk * (dk + dvs)))
+        self.lib.call("mv_delta_chunks_sum_rows", packed.data_ptr(), packed.stride(0) if n > 1 else packed.shape[1], gates.data_ptr(), state.data_ptr(),
+                      cu_seqlens.data_ptr(), state_slots.data_ptr(), n_seqs, n, heads, chunks, maps.data_ptr(), sums.data_ptr(), queries.data_ptr(),
+                      out.data_ptr(), self.code, self._stream())
 
     def state_scan(self, qk: torch.Tensor, vals: torch.Tensor, gates: torch.Tensor, state: torch.Tensor,
                    cu_seqlens: torch.Tensor, state_slots: torch.Tensor, n_seqs: int, heads: int, groups: int, dk: int,

@@ -313,14 +313,21 @@ class MLSTM(ChunkedRecurrence):
                 ctx.state_slots, ctx.n_seqs, gated, i_bias=self.i_bias, f_bias=self.f_bias, cap=spec.gate_cap,
                 max_state=ctx.state(call, "max"), denom_eps=spec.denom_eps):
             return ops.gemm(gated, self.w_o, y, defer_sum=True) or y
-        qk = ws.get("mstate.qk", (n, H, 2, dk), torch.float32)
-        vals = ws.get("mstate.vals", (n, H, dv + 1), torch.float32)
         gates = ws.get("mstate.gates", (n, H, 4), torch.float32)
-        ops.mlstm_prepare(packed, H, dk, dv, self.i_bias, self.f_bias, spec.gate_cap, ctx.state(call, "max"), ctx.token_seq,
-                          ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, gates)
         raw = ws.get("mstate.raw", (n, H, dv + 1), torch.float32)
-        recurrence(rt, ctx, "sum", n, H, dk, dv + 1, raw, ops.state_scan, self.chunks(ops.state_chunks), qk, vals, gates, ctx.state(call),
-                   ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, H, dk, dv + 1, False)
+        prepare = (packed, H, dk, dv, self.i_bias, self.f_bias, spec.gate_cap, ctx.state(call, "max"), ctx.token_seq, ctx.cu_seqlens,
+                   ctx.state_slots, ctx.n_seqs)
+        if (self.chunks(ops.state_chunks) is not None and step_paths(rt, ctx, "sum", H, dk, dv + 1) == (True, False)
+                and ops.mlstm_chunks_serve(packed, dk, dv)):
+            ops.mlstm_prepare(*prepare, None, None, gates)
+            ops.mlstm_chunks(packed, gates, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, dk, dv,
+                             *step_chunk_scratch(rt, ctx, "sum", n, H, dk, dv + 1), raw)
+        else:
+            qk = ws.get("mstate.qk", (n, H, 2, dk), torch.float32)
+            vals = ws.get("mstate.vals", (n, H, dv + 1), torch.float32)
+            ops.mlstm_prepare(*prepare, qk, vals, gates)
+            recurrence(rt, ctx, "sum", n, H, dk, dv + 1, raw, ops.state_scan, self.chunks(ops.state_chunks), qk, vals, gates, ctx.state(call),
+                       ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, H, dk, dv + 1, False)
         ops.state_finish(raw, gates, packed, self.gate_offset, self.norm, H, dv, spec.out_norm_eps, ctx.token_seq, gated,
                          shared_weight=False, silu_gate=False, normaliser=True, denom_eps=spec.denom_eps)
         return ops.gemm(gated, self.w_o, y, defer_sum=True) or y

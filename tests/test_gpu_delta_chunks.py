@@ -255,3 +255,32 @@ def test_chunks_straight_from_convolved_rows(rule, H, G, taps, weights, lens):
         assert bool(torch.isfinite(want).all())
         assert float((got.double() - want.double()).norm() / want.double().norm()) <= 16 * 2.0 ** -24 * 64 ** 0.5
     assert torch.equal(results[0][2], results[1][2])
+
+
+@pytest.mark.parametrize("H", [1, 3])
+@pytest.mark.parametrize("lens", [[128], [193, 0, 160], [145, 271]])
+def test_mlstm_chunks_straight_from_the_rows(H, lens):
+    """The bits of the vectors laid out in memory and the chunks behind them: heads of 64 x 64, requests that end inside a run and inside a chunk."""
+    ops, n, D = ops_for(torch.bfloat16), sum(lens), 64
+    g = torch.Generator().manual_seed(H + n)
+    packed = torch.randn(n, (4 * H * D + 2 * H + 7) // 8 * 8 + 8, generator=g).bfloat16().to(DEV)
+    bias = [torch.randn(H, generator=g).bfloat16().to(DEV) for _ in range(2)]
+    cu, slots, count = i32(torch.tensor([0] + lens).cumsum(0).tolist()), i32(list(range(len(lens), 0, -1))), len(lens)
+    token_seq = i32([s for s, q in enumerate(lens) for _ in range(q)])
+    state = torch.randn(len(lens) + 1, H, D + 1, D, generator=g).to(DEV)
+    units = sum(-(-x // ops.delta_chunk_tokens()) for x in lens) + 2
+    scratch = [torch.empty(units, H, device=DEV), torch.empty(units, H, D + 1, D, device=DEV), torch.empty(n, H, D, device=DEV)]
+    results = []
+    for straight in (True, False):
+        s2, raw, gates, most = state.clone(), torch.empty(n, H, D + 1, device=DEV), torch.empty(n, H, 4, device=DEV), torch.zeros(len(lens) + 1, H, device=DEV)
+        qk, vals = (None, None) if straight else (torch.empty(n, H, 2, D, device=DEV), torch.empty(n, H, D + 1, device=DEV))
+        ops.mlstm_prepare(packed, H, D, D, *bias, 15.0, most, token_seq, cu, slots, count, qk, vals, gates)
+        if straight:
+            assert ops.mlstm_chunks_serve(packed, D, D)
+            ops.mlstm_chunks(packed, gates, s2, cu, slots, count, H, D, D, *scratch, raw)
+        else:
+            ops.state_chunks(qk, vals, gates, s2, cu, slots, count, H, H, D, D + 1, False, *scratch, raw)
+        results.append((raw, s2, gates, most))
+    assert bool(torch.isfinite(results[1][0]).all())
+    for got, want in zip(*results):
+        assert torch.equal(got, want)
