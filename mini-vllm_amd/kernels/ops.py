@@ -3424,7 +3424,7 @@ class Ops:
             if u > 0 and (tokens // u + seqs) * Hkv >= least * self.compute_units:
                 floats = max(floats, min(PROMPT_SPLIT_UNITS, (tokens // u + seqs) * Hkv) * int(dll.mv_attention_prefill_part_floats(nt, D)))
         if floats:
-            workspace.get("attn.prompt_partials", (floats,), torch.float32)
+            self._split_counters(1, workspace.get("attn.prompt_partials", (floats,), torch.float32))      # (nor are these made while recording)
 
     def _attention_fast(self, q, qs, out, os_, k_pages, v_pages, block_table, page_size, positions, token_seq,
                         H, Hkv, D, scale, window, plan, first: int = 0, gate=None, gs: int = 0, form=(0.0, 0, 0)) -> bool:
