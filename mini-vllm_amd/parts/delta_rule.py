@@ -88,6 +88,10 @@ class DeltaRule(ChunkedRecurrence):
         self.w0, self.a_bias = tensors["w0"], tensors["a_bias"]
         self.norm, self.w_o = tensors["norm"], tensors["o"]
 
+    def vectors(self, n: int):
+        # float32 [n, heads, 5, head_dim]: decay, rate * unit key, unit key, key, receptance
+        return self.rt.workspace.get("delta.coef", (n, self.spec.num_heads, 5, self.spec.head_dim), torch.float32),
+
     def forward(self, x: torch.Tensor, ctx, call: int) -> torch.Tensor:
         spec, rt, ops, ws = self.spec, self.rt, self.rt.ops, self.rt.workspace
         n, inner = x.shape[0], spec.inner
@@ -109,8 +113,7 @@ class DeltaRule(ChunkedRecurrence):
                                       spec.key_eps, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs,
                                       *step_chunk_scratch(rt, ctx, "delta", n, *sizes), raw)
             else:
-                # float32 [n, heads, 5, head_dim]: decay, rate * unit key, unit key, key, receptance
-                coef = ws.get("delta.coef", (n, spec.num_heads, 5, spec.head_dim), torch.float32)
+                coef, = self.vectors(n)
                 ops.delta_prepare(packed, spec.num_heads, spec.head_dim, spec.decay_rank, self.w2_t, self.w0, self.a_bias,
                                   spec.decay_rate, spec.key_eps, coef)
                 recurrence(rt, ctx, "delta", n, *sizes, raw, ops.delta_scan, self.chunks(ops.delta_chunks), packed, coef, ctx.state(call),

@@ -144,8 +144,14 @@ class ChunkedRecurrence(Mixer):
     def step_path(self, lens: Sequence[int], starts: Sequence[int]):
         return None if self.chunks(self) is None else _paths(self.rt.ops, *self.recurrence_sizes, lens)
 
+    def vectors(self, n: int) -> Tuple[torch.Tensor, ...]:
+        """Scratch for the float vectors of ``n`` rows that a scan, and the chunks beside one, read. A step whose requests all go in chunks may
+        do without."""
+        raise NotImplementedError
+
     def reserve(self, tokens: int, seqs: int) -> None:
         (rule, heads, dk, dv), ops = self.recurrence_sizes, self.rt.ops
+        self.vectors(tokens)
         line = ops.delta_chunk_line()
         if self.chunks(rule) is not None and tokens >= line and ops.delta_chunks_serve(rule, dk, dv):
             most = min(tokens, int(_chunk_tokens_worth(rule, heads, dk, dv, min(tokens, self.rt.max_positions))))
@@ -221,6 +227,11 @@ class GatedDelta(ChunkedRecurrence):
         self.dt_bias = tensors["dt_bias"].to(self.conv_w.dtype).contiguous()
         self.norm, self.w_o = tensors["norm"].to(self.conv_w.dtype).contiguous(), tensors["o"]
 
+    def vectors(self, n: int):
+        spec, ws = self.spec, self.rt.workspace
+        return (ws.get("mstate.qk", (n, spec.num_kv_heads, 2, spec.key_dim), torch.float32),
+                ws.get("mstate.vals", (n, spec.num_heads, spec.value_dim), torch.float32))
+
     def forward(self, x: torch.Tensor, ctx, call: int) -> torch.Tensor:
         spec, rt, ops, ws = self.spec, self.rt, self.rt.ops, self.rt.workspace
         n, H, G, dk, dv = x.shape[0], spec.num_heads, spec.num_kv_heads, spec.key_dim, spec.value_dim
@@ -245,8 +256,7 @@ class GatedDelta(ChunkedRecurrence):
                                   conv_state, spec.unit_eps, None, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs,
                                   *step_chunk_scratch(rt, ctx, "gated", n, H, dk, dv), raw)
         else:
-            qk = ws.get("mstate.qk", (n, G, 2, dk), torch.float32)
-            vals = ws.get("mstate.vals", (n, H, dv), torch.float32)
+            qk, vals = self.vectors(n)
             ops.gated_delta_prepare(packed, H, G, dk, dv, spec.conv_taps, self.conv_w, self.a_log, self.dt_bias, conv_state, spec.unit_eps,
                                     ctx.token_seq, ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, gates)
             recurrence(rt, ctx, "gated", n, H, dk, dv, raw, ops.state_scan, self.chunks(ops.state_chunks), qk, vals, gates,
@@ -300,6 +310,11 @@ class MLSTM(ChunkedRecurrence):
         self.f_bias = tensors["f_bias"].to(self.i_bias.dtype).contiguous()
         self.norm, self.w_o = tensors["norm"].to(self.i_bias.dtype).contiguous(), tensors["o"]
 
+    def vectors(self, n: int):
+        spec, ws = self.spec, self.rt.workspace
+        return (ws.get("mstate.qk", (n, spec.num_heads, 2, spec.key_dim), torch.float32),
+                ws.get("mstate.vals", (n, spec.num_heads, spec.value_dim + 1), torch.float32))
+
     def forward(self, x: torch.Tensor, ctx, call: int) -> torch.Tensor:
         spec, rt, ops, ws = self.spec, self.rt, self.rt.ops, self.rt.workspace
         n, H, dk, dv = x.shape[0], spec.num_heads, spec.key_dim, spec.value_dim
@@ -323,8 +338,7 @@ class MLSTM(ChunkedRecurrence):
             ops.mlstm_chunks(packed, gates, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, dk, dv,
                              *step_chunk_scratch(rt, ctx, "sum", n, H, dk, dv + 1), raw)
         else:
-            qk = ws.get("mstate.qk", (n, H, 2, dk), torch.float32)
-            vals = ws.get("mstate.vals", (n, H, dv + 1), torch.float32)
+            qk, vals = self.vectors(n)
             ops.mlstm_prepare(*prepare, qk, vals, gates)
             recurrence(rt, ctx, "sum", n, H, dk, dv + 1, raw, ops.state_scan, self.chunks(ops.state_chunks), qk, vals, gates, ctx.state(call),
                        ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, H, H, dk, dv + 1, False)
@@ -409,6 +423,12 @@ class ChannelDelta(ChunkedRecurrence):
     def first_product(self):
         return self.w_packed.shape[0], self.w_packed.shape[1], False
 
+    def vectors(self, n: int):
+        spec, ws = self.spec, self.rt.workspace
+        return (ws.get("mstate.qk", (n, spec.num_kv_heads, 2, spec.key_dim), torch.float32),
+                ws.get("mstate.vals", (n, spec.num_heads, spec.value_dim), torch.float32),
+                ws.get("mstate.beta", (n, spec.num_heads), torch.float32))
+
     def forward(self, x: torch.Tensor, ctx, call: int, fold=None) -> torch.Tensor:
         spec, rt, ops, ws = self.spec, self.rt, self.rt.ops, self.rt.workspace
         n, H, G, dk, dv = x.shape[0], spec.num_heads, spec.num_kv_heads, spec.key_dim, spec.value_dim
@@ -432,9 +452,7 @@ class ChannelDelta(ChunkedRecurrence):
                                   spec.unit_eps, z, ctx.state(call), ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs,
                                   *step_chunk_scratch(rt, ctx, "channel", n, H, dk, dv), raw)
         else:
-            qk = ws.get("mstate.qk", (n, G, 2, dk), torch.float32)
-            vals = ws.get("mstate.vals", (n, H, dv), torch.float32)
-            beta = ws.get("mstate.beta", (n, H), torch.float32)
+            qk, vals, beta = self.vectors(n)
             ops.channel_prepare(packed, H, G, dk, dv, spec.conv_taps, self.b_offset, self.conv_w, self.a_log, self.dt_bias, conv_state,
                                 spec.unit_eps, ctx.token_seq, ctx.cu_seqlens, ctx.state_slots, ctx.n_seqs, qk, vals, beta, z)
             recurrence(rt, ctx, "channel", n, H, dk, dv, raw, ops.channel_scan, self.chunks(ops.channel_chunks), qk, vals, beta, z,

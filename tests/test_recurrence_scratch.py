@@ -1,10 +1,43 @@
 """What the recurrences over chunks take as scratch is there before the cache is sized, however later steps are cut."""
 import random
+from types import SimpleNamespace
+from unittest.mock import MagicMock
 
 import pytest
 import torch
 
 from minivllm_amd.engine.step import AttentionPlan
+from minivllm_amd.parts import MIXERS, Workspace
+from minivllm_amd.parts.delta_rule import DeltaRuleSpec
+from minivllm_amd.parts.matrix_state import ChannelDeltaSpec, GatedDeltaSpec, MLSTMSpec
+
+SIZES = dict(hidden_size=64, num_heads=2, key_dim=64, value_dim=64)
+SPECS = [DeltaRuleSpec(hidden_size=64, num_heads=2, head_dim=64, decay_rank=64), GatedDeltaSpec(num_kv_heads=1, conv_taps=4, **SIZES), MLSTMSpec(**SIZES),
+         ChannelDeltaSpec(num_kv_heads=1, conv_taps=4, decay_rank=16, gate_rank=16, **SIZES)]
+
+
+@pytest.mark.parametrize("spec", SPECS, ids=lambda spec: spec.kind)
+def test_vectors_of_short_requests_have_room_before_any_come(spec):
+    """An engine of so few requests that its dry step's all go in chunks, straight from the packed rows: a short request beside long ones, or alone, and
+    requests so many that all are scanned, want their rows' vectors in memory."""
+    ops = MagicMock(compute_units=256)
+    ops.delta_chunk_line.return_value, ops.delta_chunk_tokens.return_value, ops.gemm.return_value = 128, 32, None
+    for straight in ("delta_chunks_rows", "delta_chunks_conv", "mlstm_chunks"):
+        getattr(ops, straight + "_serve").return_value = True
+    rt = SimpleNamespace(dtype=torch.bfloat16, ops=ops, workspace=Workspace(torch.device("meta")), max_positions=1024)
+    cls = MIXERS.get(spec.kind)
+    part = cls(spec, {name: torch.zeros(decl.shape, dtype=torch.bfloat16, device="meta") for name, decl in cls.tensors(spec).items()}, rt)
+
+    def step(lens):
+        plan = AttentionPlan(decode_only=False, max_q_len=max(lens), max_context_len=max(lens), n_seqs=len(lens), q_lens=lens)
+        ops.reset_mock()
+        part.forward(torch.zeros(sum(lens), 64, dtype=torch.bfloat16, device="meta"), MagicMock(attention_plan=plan), 0)
+        return any(getattr(ops, straight).called for straight in ("delta_chunks_rows", "delta_chunks_conv", "mlstm_chunks"))
+
+    part.reserve(1024, 4)
+    assert step([512, 512]), "the dry step wants no vectors"
+    rt.workspace.frozen = True                  # (a buffer that would have to grow raises)
+    assert not any(step(lens) for lens in ([1000, 24], [700, 100, 100, 124], [100], [127] * 8))
 
 
 def test_no_cut_has_more_units():
