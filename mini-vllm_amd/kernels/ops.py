@@ -3341,7 +3341,7 @@ class Ops:
         attention for this step; column tiles 0: the kernel does not serve ``group`` heads per kv head, blocks 0: walks are not cut.
         ``keys``: the most a column sees where a window or a chunk says so; ``narrow_sums``: only walks of 16 columns a wave may be cut."""
         if plan.prefill_variant is None:
-            for nt in (1,) if narrow_sums else (2, 1):
+            for nt in () if plan.workspace is None else (1,) if narrow_sums else (2, 1):     # (no room for the parts' sums: whole walks)
                 limit = self._prefill_limit(plan, nt, group, Hkv, keys)
                 if limit:
                     u = self.lib.dll.mv_attention_prefill_unit_tokens(group, nt)
@@ -3411,6 +3411,8 @@ class Ops:
         """(partial sums, counters, blocks of a first part) for the kernel."""
         if limit == 0:
             return None, None, 0
+        if workspace is None:
+            raise KernelLibraryError("attention: a plan without a workspace has no room for walks in two parts")
         partials = workspace.get("attn.prompt_partials", (n_units * Hkv * int(self.lib.dll.mv_attention_prefill_part_floats(nt, D)),), torch.float32)
         return partials.data_ptr(), self._split_counters(n_units * Hkv, partials), limit
 

@@ -8,6 +8,7 @@ import torch
 
 from minivllm_amd.csrc import build
 from minivllm_amd.engine.step import AttentionPlan
+from minivllm_amd.kernels.library import KernelLibraryError
 from minivllm_amd.kernels.ops import PROMPT_SPLIT_UNITS, Ops
 from minivllm_amd.parts.base import Workspace
 
@@ -23,7 +24,8 @@ def rule():
 
 
 def plan_of(lens, bound=None):
-    return AttentionPlan(decode_only=False, max_q_len=max(lens), max_context_len=max(lens), n_seqs=len(lens), q_lens=() if bound else list(lens), bound=bound)
+    return AttentionPlan(decode_only=False, max_q_len=max(lens), max_context_len=max(lens), n_seqs=len(lens), q_lens=() if bound else list(lens), bound=bound,
+                         workspace=Workspace(torch.device("meta")))
 
 
 @pytest.mark.parametrize("H, Hkv", HEADS)
@@ -59,3 +61,16 @@ def test_the_lines():
     assert variant([2048], keys=1024)[4] == 0 and variant([2048], keys=2048)[4] == 44          # a window that no walk leaves
     assert variant([4096], sums=True)[:2] != (2, 1) or variant([4096], sums=True)[4] == 0      # sums of sigmoid weights: 16 columns a wave only
     assert ops._prefill_variant(plan_of([2048], bound=(2048, 1)), 2, 8)[4] == 44
+
+
+@pytest.mark.parametrize("rows", [1408, 2048, 4096])
+def test_a_plan_without_a_workspace_has_whole_walks(rows):
+    """As every plan had before walks were cut; a forced cut has no room and is refused."""
+    ops, plan, whole = rule(), plan_of([rows]), plan_of([rows])
+    plan.workspace, ops_whole = None, rule()
+    ops_whole._prefill_limit = lambda *args: 0
+    nt, kw, units, busy, limit = ops._prefill_variant(plan, 2, 8)
+    assert (nt, kw, units, busy, limit) == ops_whole._prefill_variant(whole, 2, 8)
+    assert ops._prefill_room(plan.workspace, limit, nt, units, 8, 128) == (None, None, 0)
+    with pytest.raises(KernelLibraryError):
+        ops._prefill_room(None, 16, nt, units, 8, 128)
