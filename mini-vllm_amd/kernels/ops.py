@@ -2518,9 +2518,10 @@ class Ops:
             nt, kw, n_units, n_busy, limit = self._prefill_variant(plan, group, num_kv_heads, keys, narrow_sums=True)
             if nt:
                 split = self._prefill_room(plan.workspace, limit, nt, n_units, num_kv_heads, head_dim)
+                counters = lambda: self._prompt_counters(plan.workspace, n_units * num_kv_heads) if limit else None
                 self._note_attention("mv_attention_prefill_sigmoid", self._chunk_priced(plan, c), n, num_heads, num_kv_heads,
                                      head_dim, 2)
-                self._decode_launch("mv_attention_prefill_sigmoid", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
+                self._counted_launch(counters, "mv_attention_prefill_sigmoid", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
                               v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size,
                               positions.data_ptr(), plan.cu_seqlens.data_ptr(), plan.n_seqs, n_units, n_busy, nt, kw, int(plan.has_short(16 // group + 1)),
                               num_heads, num_kv_heads, head_dim, float(scale), w, c, _ptr(bias), _ptr(gate), gate_stride,
@@ -3242,16 +3243,21 @@ class Ops:
         return self._attn_counters.data_ptr()
 
     def _decode_launch(self, entry: str, *args) -> None:
-        """Launches a decode attention; should the launch fail, the split counters are put back to
-        zero (outside a capture) before the error goes on: a launch that stopped half-way may have
+        """Launches a decode attention (``_counted_launch`` on this ``Ops``' counters)."""
+        self._counted_launch(lambda: self._attn_counters, entry, *args)
+
+    def _counted_launch(self, counters, entry: str, *args) -> None:
+        """Launches a kernel whose workgroups count themselves in; should the launch fail, what ``counters()`` gives (None:
+        nothing) is put back to zero (outside a capture) before the error goes on: a launch that stopped half-way may have
         left some counted."""
         try:
             self.lib.call(entry, *args)
         except Exception:
-            if self._attn_counters is not None and not torch.cuda.is_current_stream_capturing():
+            counted = counters()
+            if counted is not None and not torch.cuda.is_current_stream_capturing():
                 try:
                     torch.cuda.synchronize()
-                    self._attn_counters.zero_()
+                    counted.zero_()
                 except Exception:
                     pass
             raise
@@ -3408,13 +3414,19 @@ class Ops:
         return limit if serves and longest >= limit + 8 else 0
 
     def _prefill_room(self, workspace, limit: int, nt: int, n_units: int, Hkv: int, D: int):
-        """(partial sums, counters, blocks of a first part) for the kernel."""
+        """(partial sums, counters, blocks of a first part) for the kernel. Both lie in the plan's workspace: launches that share one follow each
+        other on one stream, those of two workspaces may overlap."""
         if limit == 0:
             return None, None, 0
         if workspace is None:
             raise KernelLibraryError("attention: a plan without a workspace has no room for walks in two parts")
         partials = workspace.get("attn.prompt_partials", (n_units * Hkv * int(self.lib.dll.mv_attention_prefill_part_floats(nt, D)),), torch.float32)
-        return partials.data_ptr(), self._split_counters(n_units * Hkv, partials), limit
+        return partials.data_ptr(), self._prompt_counters(workspace, n_units * Hkv).data_ptr(), limit
+
+    @staticmethod
+    def _prompt_counters(workspace, n: int = 0) -> torch.Tensor:
+        """One counter for every (unit, kv head) of a prompt step with walks in two parts: zero at first, and again behind every launch."""
+        return workspace.get("attn.prompt_counters", (max(n, PROMPT_SPLIT_UNITS),), torch.int32, zeroed=True)
 
     def reserve_prompt_attention(self, workspace, tokens: int, seqs: int, H: int, Hkv: int, D: int) -> None:
         """Room for the parts of walks of any step of up to ``tokens`` tokens of up to ``seqs`` sequences (``_prefill_limit``)."""
@@ -3426,7 +3438,8 @@ class Ops:
             if u > 0 and (tokens // u + seqs) * Hkv >= least * self.compute_units:
                 floats = max(floats, min(PROMPT_SPLIT_UNITS, (tokens // u + seqs) * Hkv) * int(dll.mv_attention_prefill_part_floats(nt, D)))
         if floats:
-            self._split_counters(1, workspace.get("attn.prompt_partials", (floats,), torch.float32))      # (nor are these made while recording)
+            workspace.get("attn.prompt_partials", (floats,), torch.float32)
+            self._prompt_counters(workspace)
 
     def _attention_fast(self, q, qs, out, os_, k_pages, v_pages, block_table, page_size, positions, token_seq,
                         H, Hkv, D, scale, window, plan, first: int = 0, gate=None, gs: int = 0, form=(0.0, 0, 0)) -> bool:
@@ -3455,13 +3468,15 @@ class Ops:
         nt, kw, n_units, n_busy, limit = self._prefill_variant(plan, group, Hkv, None if window < 0 else window + 1 + first + 32)
         if nt == 0:
             return False
+        split = self._prefill_room(plan.workspace, limit, nt, n_units, Hkv, D)
+        counters = lambda: self._prompt_counters(plan.workspace, n_units * Hkv) if limit else None
         self._note_attention("mv_attention_prefill", priced, q.shape[0], H, Hkv, D, 2)
-        self._decode_launch("mv_attention_prefill", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
+        self._counted_launch(counters, "mv_attention_prefill", q.data_ptr(), qs, out.data_ptr(), os_, k_pages.data_ptr(),
                       v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], page_size,
                       positions.data_ptr(), plan.cu_seqlens.data_ptr(), n_seqs, n_units, n_busy, nt, kw,
                       int(plan.has_short(16 // group + 1)), H, Hkv, D,
                       float(scale), window, first, _ptr(gate), gs, *form,
-                      *self._prefill_room(plan.workspace, limit, nt, n_units, Hkv, D), self._stream())
+                      *split, self._stream())
         return True
 
     # ------------------------------------------------------------------------------------

@@ -300,7 +300,8 @@ class Workspace:
         self.retain = retain
         self.frozen = False
 
-    def get(self, name: str, shape: Sequence[int], dtype: torch.dtype) -> torch.Tensor:
+    def get(self, name: str, shape: Sequence[int], dtype: torch.dtype, zeroed: bool = False) -> torch.Tensor:
+        """``zeroed``: a buffer made now holds zeros; one that is there is left as it is."""
         vkey = (name, dtype, tuple(shape))
         view = self._views.get(vkey)          # making a view costs as much as a launch: keep them
         if view is not None:
@@ -315,7 +316,7 @@ class Workspace:
                 raise RuntimeError(f"workspace buffer {name!r} would have to grow to {n} elements while frozen")
             if buf is not None and self.retain:
                 self._retired.append(buf)
-            buf = torch.empty(max(n, 1), dtype=dtype, device=self.device)
+            buf = (torch.zeros if zeroed else torch.empty)(max(n, 1), dtype=dtype, device=self.device)
             self._buffers[key] = buf
             for k in [k for k in self._views if k[0] == name and k[1] == dtype]:
                 del self._views[k]             # views of the replaced buffer

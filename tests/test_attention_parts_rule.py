@@ -18,7 +18,8 @@ HEADS = [(16, 8), (32, 8), (64, 8), (4, 2), (24, 24), (6, 2)]
 def rule():
     ops = SimpleNamespace(lib=SimpleNamespace(has=lambda name: True, dll=ctypes.CDLL(build.find_library("bf16") or build.build("bf16"))),
                           compute_units=256, use_fast_kernels=True, dtype=torch.bfloat16, _attn_counters=None)
-    for name in ("_prefill_limit", "_prefill_room", "_split_counters", "reserve_prompt_attention", "_prefill_variant"):
+    ops._prompt_counters = Ops._prompt_counters
+    for name in ("_prefill_limit", "_prefill_room", "_counted_launch", "reserve_prompt_attention", "_prefill_variant"):
         setattr(ops, name, getattr(Ops, name).__get__(ops))
     return ops
 
@@ -74,3 +75,26 @@ def test_a_plan_without_a_workspace_has_whole_walks(rows):
     assert ops._prefill_room(plan.workspace, limit, nt, units, 8, 128) == (None, None, 0)
     with pytest.raises(KernelLibraryError):
         ops._prefill_room(None, 16, nt, units, 8, 128)
+
+
+def test_two_workspaces_share_no_counters(monkeypatch):
+    """Steps on two streams have a workspace each and may overlap, also on one ``Ops``: what a launch counts in is its workspace's, zero at first; a launch
+    that fails leaves zeros behind, in its own."""
+    ops, room = rule(), [Workspace(torch.device("cpu")) for _ in range(2)]
+    taken = [ops._prefill_room(ws, 16, 1, 40, 8, 128) for ws in room]
+    assert len({pointer for r in taken for pointer in r[:2]}) == 4 and ops._attn_counters is None
+    counters = [ops._prompt_counters(ws, 320) for ws in room]
+    assert [c.data_ptr() for c in counters] == [r[1] for r in taken] and not any(bool(c.any()) for c in counters)
+    for c in counters:
+        c[5] = 1
+    room[0].frozen = True
+    assert ops._prefill_room(room[0], 30, 1, 20, 8, 128)[1] == taken[0][1] and int(counters[0][5]) == 1      # (those of a launch on its way)
+
+    def fails(entry, *args):
+        raise KernelLibraryError(entry)
+    ops.lib.call = fails
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
+    with pytest.raises(KernelLibraryError):
+        ops._counted_launch(lambda: counters[0], "mv_attention_prefill")
+    assert not bool(counters[0].any()) and int(counters[1][5]) == 1

@@ -54,7 +54,7 @@ def test_walks_in_two_parts(nt, limit, H, Hkv, D, ps, window, first):
                       **({"keep_first": first} if first else {}))
         outs.append(out)
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
-    assert not bool(ops._attn_counters.any())
+    assert not bool(ops._prompt_counters(plan.workspace).any())
     want = torch.zeros(n, H, D, dtype=torch.float64)
     for i in range(n):
         s, p = int(token_seq[i]), int(positions[i])
