@@ -32,17 +32,11 @@ from ..models.registry import Architecture, load_config
 from ..parts.base import Runtime, Workspace
 from ..weights.loader import check_tensors, open_model_folder
 from ..weights.source import DeviceTensors, TensorSource
-from .step import AttentionPlan, KVView, SeqStep, StepContext
+from .step import TOKEN_BUCKETS, AttentionPlan, KVView, SeqStep, StepContext
 
 logger = logging.getLogger(__name__)
 
 GRAPH_BUCKETS = [1, 2, 4, 8] + list(range(16, 257, 16))     # as the reference's (graph.py:11-12)
-# token counts that steps with prompt portions are padded to when they are replayed from a graph:
-# at most an eighth more than the step holds (from 9 tokens on 16, up to 8 tokens 8: there the products change hands, and a step
-# is to add in the same order recorded and not; gemm_deep.hip knows these classes)
-TOKEN_BUCKETS = ([8] + list(range(16, 129, 16)) + list(range(160, 257, 32)) + list(range(320, 513, 64))
-                 + list(range(640, 1025, 128)) + list(range(1280, 2049, 256)) + list(range(2560, 4097, 512))
-                 + list(range(5120, 8193, 1024)))
 # graphs of such steps kept at a time (the one used longest ago goes first)
 MIXED_GRAPHS_KEPT = 64
 

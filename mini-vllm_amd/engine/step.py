@@ -16,6 +16,18 @@ from typing import Dict, List, Optional, Sequence
 
 import torch
 
+# token counts that steps with prompt portions are padded to when they are replayed from a graph:
+# at most an eighth more than the step holds (from 9 tokens on 16, up to 8 tokens 8: there the products change hands, and a step
+# is to add in the same order recorded and not; gemm_deep.hip knows these classes)
+TOKEN_BUCKETS = ([8] + list(range(16, 129, 16)) + list(range(160, 257, 32)) + list(range(320, 513, 64))
+                 + list(range(640, 1025, 128)) + list(range(1280, 2049, 256)) + list(range(2560, 4097, 512))
+                 + list(range(5120, 8193, 1024)))
+
+
+def class_rows(tokens: int) -> int:
+    """The rows of a step of so many tokens when it is recorded (more than the largest class: the tokens)."""
+    return next((b for b in TOKEN_BUCKETS if b >= tokens), tokens)
+
 
 @dataclass
 class SeqStep:

@@ -5,7 +5,7 @@ the HIP library on the current stream. Tensors must live on the GPU: there is no
 """
 from __future__ import annotations
 
-from typing import Optional, Sequence
+from typing import Optional, Sequence, Tuple
 
 import ctypes
 import math
@@ -2514,8 +2514,7 @@ class Ops:
                 and head_dim == value_dim and head_dim in (64, 128) and page_size >= 16 and not page_size & (page_size - 1)
                 and qs % 8 == 0 and os_ % 4 == 0 and q.data_ptr() % 16 == 0 and out.data_ptr() % 8 == 0):
             # (sums of sigmoid weights: the walk of 32 columns a wave has no registers left for being cut)
-            keys = min((x for x in (w + 1, c) if x > 0), default=None)
-            nt, kw, n_units, n_busy, limit = self._prefill_variant(plan, group, num_kv_heads, keys, narrow_sums=True)
+            nt, kw, n_units, n_busy, limit = self._prefill_variant(plan, group, num_kv_heads, self._keys_seen(w, chunk=c), narrow_sums=True)
             if nt:
                 split = self._prefill_room(plan.workspace, limit, nt, n_units, num_kv_heads, head_dim)
                 counters = lambda: self._prompt_counters(plan.workspace, n_units * num_kv_heads) if limit else None
@@ -3347,11 +3346,10 @@ class Ops:
         attention for this step; column tiles 0: the kernel does not serve ``group`` heads per kv head, blocks 0: walks are not cut.
         ``keys``: the most a column sees where a window or a chunk says so; ``narrow_sums``: only walks of 16 columns a wave may be cut."""
         if plan.prefill_variant is None:
-            for nt in () if plan.workspace is None else (1,) if narrow_sums else (2, 1):     # (no room for the parts' sums: whole walks)
-                limit = self._prefill_limit(plan, nt, group, Hkv, keys)
-                if limit:
-                    u = self.lib.dll.mv_attention_prefill_unit_tokens(group, nt)
-                    return nt, 1, plan.units(u), plan.busy_units(u), limit
+            nt, limit = self._prompt_parts(plan, group, Hkv, keys, narrow_sums)
+            if limit:
+                u = self.lib.dll.mv_attention_prefill_unit_tokens(group, nt)
+                return nt, 1, plan.units(u), plan.busy_units(u), limit
         elif len(plan.prefill_variant) > 2:
             nt, kw, limit = plan.prefill_variant
             u = self.lib.dll.mv_attention_prefill_unit_tokens(group, nt)
@@ -3388,30 +3386,85 @@ class Ops:
             kw = int(plan.prefill_variant[1])
         return nt, kw, n_units, n_busy, 0
 
-    def _prefill_limit(self, plan, nt: int, group: int, Hkv: int, keys: Optional[int]) -> int:
-        """Blocks of the first part of a walk cut in two with ``nt`` column tiles a wave, 0: not cut. The limit is some more than what
-        a slot (two workgroups a compute unit) gets if a single prompt of the step's rows is dealt out evenly; several prompts, whose walks
-        are shorter, are cut more rarely. us whole / cut: 16 heads on 8, 1,800 rows 40.3 / 34.1, 2,048 42.3 / 38.9, 2,500 60.3 / 50.2, 3,000 71 / 62,
-        4,096 111 / 86, 6,000 192 / 171; 32 heads 1,500 rows 41.8 / 38.7, 2,048 57.8 / 51.3, 2,600 81.6 / 75.3. From four 32-column units a compute unit on
-        the dispatch evens walks out by itself (8,192 rows 276.9 / 278.0), below the lower ends the joining takes what it gives (1,408 rows
-        28.4 / 28.3, 32 heads 1,000 rows 25.4 / 25.9)."""
-        u = self.lib.dll.mv_attention_prefill_unit_tokens(group, nt)
-        if u <= 0 or not self.lib.has("mv_attention_prefill_part_floats"):
-            return 0
-        units, busy, cus = plan.units(u), plan.busy_units(u), self.compute_units
-        if units * Hkv > PROMPT_SPLIT_UNITS:
-            return 0
-        rows = plan.bound[0] if plan.bound is not None else sum(plan.q_lens)
-        blocks = rows / 32
-        mean = (blocks + 1) / 2 * busy * Hkv / (2 * cus)
-        if nt == 2:
-            limit = int(1.15 * mean / 2 + 0.999) * 2
-            serves = 1.25 * cus <= busy * Hkv < 4 * cus and limit >= 20
-        else:
-            limit = int(1.3 * mean / 2 + 0.999) * 2
-            serves = 1.5 * cus <= busy * Hkv and limit >= 24
-        longest = blocks if keys is None else min(blocks, (keys + u) / 32 + 2)
-        return limit if serves and longest >= limit + 8 else 0
+    def _prompt_parts(self, plan, group: int, Hkv: int, keys: Optional[int], narrow_sums: bool) -> Tuple[int, int]:
+        """``_cut_walks`` for a plan; (0, 0), whole walks, also where it does not say where its requests start or has no room for the parts' sums."""
+        lens, starts = plan.cut()
+        if not starts and plan.bound is None and len(plan.q_lens) == 1:
+            lens, starts = plan.q_lens, (max(0, plan.max_context_len - plan.q_lens[0]),)
+        if not starts or plan.workspace is None:
+            return 0, 0
+        rows = plan.bound[0] if plan.bound is not None else sum(lens)
+        nt, limit = self._cut_walks(lens, starts, rows, group, Hkv, keys, narrow_sums, plan.bound is not None)
+        if limit and plan.units(self.lib.dll.mv_attention_prefill_unit_tokens(group, nt)) * Hkv > PROMPT_SPLIT_UNITS:
+            return 0, 0
+        return nt, limit
+
+    def _cut_walks(self, lens: Sequence[int], starts: Sequence[int], rows: int, group: int, Hkv: int, keys: Optional[int], narrow_sums: bool,
+                   recorded: bool) -> Tuple[int, int]:
+        """(column tiles a wave, blocks of the first part) with which the prompt attention cuts the walks of a step in two whose requests bring ``lens``
+        tokens from positions ``starts`` on, in ``rows`` rows; (0, 0): whole walks. ``keys``, ``narrow_sums``: as in ``_prefill_variant``.
+
+        Cut are steps of which one request has four fifths of the walks: several prompts of a size end together anyhow. The limit is some more
+        than what a slot (two workgroups a compute unit) gets if that request's walks are dealt out evenly. us whole / cut, heads of 128 on 8 kv heads;
+        16 heads: 1,700 rows 34.0 / 30.3, 2,048 39.7 / 37.6, 3,000 65.5 / 59.3, 4,096 101 / 81, 5,000 146 / 125, 1,900 and 148 42.4 / 36.7; 32 heads: 1,536
+        39.3 / 37.2, 2,048 55.9 / 50.2, 3,000 95.9 / 89.2. Not cut: two of 1,024 24.9 / 30.5, four of 512 17.4 / 20.3, eight of 256 13.5 / 15.3, two of 2,000 60.7 /
+        70.8. Behind a context walks are longer and more alike: 3,000 rows behind 1,024 keys 102 / 79, 4,096 behind 2,048 160 / 142, 1,536 behind 1,024 55 / 45
+        and behind 4,096 137 / 111, but 2,048 behind 1,024 61 whole and 74 cut at what no context would ask for, behind 2,048 82 and 90. There the step waits for the
+        slots, not for the last walk: with a whole number of rounds nothing is won, with little more than one and walks about alike, halves are half a round less
+        (32 heads, 3,000 behind 4,096 310 / 277).
+
+        Lower ends: the joining takes what it gives (16 heads, 1,408 rows 28.4 / 28.3); from four 32-column units a compute unit on the dispatch evens walks
+        out by itself (8,192 rows 276.9 / 278.0). A recording's limit is one of two an octave behind a context or beside other requests, and that of the class's
+        rows otherwise: a class has few recordings."""
+        if not self.lib.has("mv_attention_prefill_part_floats"):
+            return 0, 0
+        cus, units_of = self.compute_units, self.lib.dll.mv_attention_prefill_unit_tokens
+        for nt in (1,) if narrow_sums else (2, 1):
+            u = units_of(group, nt)
+            full = -(-rows // u) * Hkv if u > 0 else 0
+            if full < (1.25 if nt == 2 else 1.5) * cus or (nt == 2 and full >= 4 * cus):
+                continue
+            walks = [-(-q // u) * (2 * s + q) / 64 for q, s in zip(lens, starts)]
+            most = max(walks)
+            if most < 0.8 * sum(walks):
+                continue
+            start, brings = next((s, q) for w, q, s in zip(walks, lens, starts) if w == most)
+            tokens = rows if start == 0 else sum(lens)
+            units = -(-tokens // u)
+            busy, mean, longest = units * Hkv, (start + tokens / 2) / 32, (start + brings) / 32
+            share = max(units * (mean + 0.5), sum(walks)) * Hkv / (2 * cus)
+            limit = int((1.15 if nt == 2 else 1.3) * share / 2 + 0.999) * 2
+            seen = longest if keys is None else min(longest, (keys + u) / 32 + 2)
+            if nt == 2:
+                serves = limit >= 20 and seen >= (max(limit + 8, 1.1 * limit, 44) if busy >= 2 * cus else limit + 8)
+                alike = 2 * cus < full <= 3 * cus and longest >= 100
+            else:
+                serves = limit >= 24 and seen >= max(limit + 8, 1.3 * limit if full >= 2 * cus and start > 0 else 0)
+                alike = longest >= 48 if full < 2 * cus else 2 * cus < full <= 3 * cus and longest >= 100
+            if not serves:
+                if not alike or keys is not None or mean < 0.7 * longest:
+                    continue
+                limit = int(longest / 5) * 2
+            if recorded and (start > 0 or len(lens) > 1):
+                step = max(2, 1 << (limit - 1).bit_length() - 2)
+                down = limit // step * step
+                limit = down if (limit - down) * 2 <= step or down + step + 8 > seen else down + step
+            return nt, limit
+        return 0, 0
+
+    def prompt_attention_path(self, lens: Sequence[int], starts: Sequence[int], rows: int, H: int, Hkv: int, D: int, window: Optional[int] = None,
+                              first: int = 0, chunk: Optional[int] = None, sigmoid: bool = False):
+        """What the prompt attention of a step recorded for ``rows`` rows chooses by its requests' lengths and places (``Mixer.step_path``),
+        None: nothing."""
+        if not (self.use_fast_kernels and self.dtype == torch.bfloat16 and D in (64, 128) and self.lib.has("mv_attention_prefill_part_floats")):
+            return None
+        return self._cut_walks(lens, starts, rows, H // Hkv, Hkv, self._keys_seen(window, first, chunk), sigmoid, True)
+
+    @staticmethod
+    def _keys_seen(window: Optional[int], first: int = 0, chunk: Optional[int] = None) -> Optional[int]:
+        """The most keys that a column of the prompt attention sees, None: as many as there are."""
+        bounds = [] if window is None or window < 0 else [window + 1 + first + 32]
+        return min(bounds + ([chunk] if chunk else []), default=None)
 
     def _prefill_room(self, workspace, limit: int, nt: int, n_units: int, Hkv: int, D: int):
         """(partial sums, counters, blocks of a first part) for the kernel. Both lie in the plan's workspace: launches that share one follow each
@@ -3465,7 +3518,7 @@ class Ops:
             return True
         if page_size & (page_size - 1):
             return False
-        nt, kw, n_units, n_busy, limit = self._prefill_variant(plan, group, Hkv, None if window < 0 else window + 1 + first + 32)
+        nt, kw, n_units, n_busy, limit = self._prefill_variant(plan, group, Hkv, self._keys_seen(window, first))
         if nt == 0:
             return False
         split = self._prefill_room(plan.workspace, limit, nt, n_units, Hkv, D)

@@ -43,10 +43,11 @@ runs ``conv_store`` and ``attend_scored``, which another part may call like thos
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import Dict, Optional, Tuple
+from typing import Dict, Optional, Sequence, Tuple
 
 import torch
 
+from ..engine.step import class_rows
 from .base import (CacheNeed, KeepAll, KeepChunks, KeepWindow, KeepWindowAndFirst, KeyValueNeed, Mixer, PartSpec, Runtime,
                    TensorDecl, register_mixer)
 
@@ -297,6 +298,17 @@ class Attention(Mixer):
         spec = self.spec
         if spec.v_head_dim == spec.head_dim:
             self.rt.ops.reserve_prompt_attention(self.rt.workspace, tokens, seqs, spec.num_heads, spec.num_kv_heads, spec.head_dim)
+
+    def step_path(self, lens: Sequence[int], starts: Sequence[int]):
+        spec = self.spec
+        if spec.v_head_dim != spec.head_dim:
+            return None
+        return self.rt.ops.prompt_attention_path(lens, starts, class_rows(sum(lens)), spec.num_heads, spec.num_kv_heads, spec.head_dim, spec.window,
+                                                 spec.keep_first, spec.chunk, spec.weighting == "sigmoid")
+
+    def chooses_by(self):
+        spec = self.spec
+        return Attention, spec.num_heads, spec.num_kv_heads, spec.head_dim, spec.v_head_dim, spec.window, spec.keep_first, spec.chunk, spec.weighting
 
     def first_product(self):
         return self.w_qkv.shape[0], self.w_qkv.shape[1], False

@@ -13,7 +13,7 @@ In a step of single tokens the left side's cache write runs in the right side's 
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import Dict, Optional
+from typing import Dict, Optional, Sequence
 
 import torch
 
@@ -76,6 +76,12 @@ class ParallelMixer(Mixer):
 
     def reserve(self, tokens: int, seqs: int) -> None:
         self.left.reserve(tokens, seqs)
+
+    def step_path(self, lens: Sequence[int], starts: Sequence[int]):
+        return self.left.step_path(lens, starts)
+
+    def chooses_by(self):
+        return self.left.chooses_by()
 
     def first_product(self):
         return self.w_packed.shape[0], self.w_packed.shape[1], False
@@ -157,6 +163,12 @@ class ParallelSum(Mixer):
 
     def reserve(self, tokens: int, seqs: int) -> None:
         self.left.reserve(tokens, seqs)
+
+    def step_path(self, lens: Sequence[int], starts: Sequence[int]):
+        return self.left.step_path(lens, starts)
+
+    def chooses_by(self):
+        return self.left.chooses_by()
 
     def first_product(self):
         return self.w_packed.shape[0], self.w_packed.shape[1], False

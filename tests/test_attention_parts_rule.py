@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from minivllm_amd.csrc import build
-from minivllm_amd.engine.step import AttentionPlan
+from minivllm_amd.engine.step import AttentionPlan, class_rows
 from minivllm_amd.kernels.library import KernelLibraryError
 from minivllm_amd.kernels.ops import PROMPT_SPLIT_UNITS, Ops
 from minivllm_amd.parts.base import Workspace
@@ -19,14 +19,19 @@ def rule():
     ops = SimpleNamespace(lib=SimpleNamespace(has=lambda name: True, dll=ctypes.CDLL(build.find_library("bf16") or build.build("bf16"))),
                           compute_units=256, use_fast_kernels=True, dtype=torch.bfloat16, _attn_counters=None)
     ops._prompt_counters = Ops._prompt_counters
-    for name in ("_prefill_limit", "_prefill_room", "_counted_launch", "reserve_prompt_attention", "_prefill_variant"):
+    ops._keys_seen = Ops._keys_seen
+    for name in ("_prompt_parts", "_cut_walks", "prompt_attention_path", "_prefill_room", "_counted_launch", "reserve_prompt_attention", "_prefill_variant"):
         setattr(ops, name, getattr(Ops, name).__get__(ops))
     return ops
 
 
-def plan_of(lens, bound=None):
-    return AttentionPlan(decode_only=False, max_q_len=max(lens), max_context_len=max(lens), n_seqs=len(lens), q_lens=() if bound else list(lens), bound=bound,
-                         workspace=Workspace(torch.device("meta")))
+def plan_of(lens, bound=None, starts=None):
+    starts = [0] * len(lens) if starts is None else starts
+    plan = AttentionPlan(decode_only=False, max_q_len=max(lens), max_context_len=max(map(sum, zip(lens, starts))), n_seqs=len(lens),
+                         q_lens=() if bound else list(lens), starts=list(starts), bound=bound, workspace=Workspace(torch.device("meta")))
+    if bound:
+        plan.path_lens, plan.path_starts = tuple(lens), tuple(starts)
+    return plan
 
 
 @pytest.mark.parametrize("H, Hkv", HEADS)
@@ -42,7 +47,8 @@ def test_any_steps_parts_fit_what_is_reserved(H, Hkv, D):
             total = rng.randint(n, tokens)
             ends = sorted(rng.sample(range(1, total), n - 1)) if n > 1 else []
             lens = [b - a for a, b in zip([0] + ends, ends + [total])]
-            for plan in (plan_of(lens), plan_of(lens, bound=(total, rng.randint(n, seqs)))):
+            starts = [rng.choice([0, 0, rng.randint(0, 9000)]) for _ in lens]
+            for plan in (plan_of(lens, starts=starts), plan_of(lens, (total, rng.randint(n, seqs)), starts)):
                 nt, kw, units, busy, limit = ops._prefill_variant(plan, H // Hkv, Hkv)
                 if limit:
                     cut += 1
@@ -54,7 +60,7 @@ def test_any_steps_parts_fit_what_is_reserved(H, Hkv, D):
 
 def test_the_lines():
     ops = rule()
-    variant = lambda lens, H=16, keys=None, sums=False: ops._prefill_variant(plan_of(lens), H // 8, 8, keys, sums)
+    variant = lambda lens, H=16, keys=None, sums=False, **more: ops._prefill_variant(plan_of(lens, **more), H // 8, 8, keys, sums)
     assert variant([1408])[:2] == (1, 2) and variant([1408])[4] == 0
     assert variant([2048])[:2] == (1, 1) and variant([2048])[4] == 44
     assert variant([4096])[:2] == (2, 1) and variant([4096])[4] in (74, 76)
@@ -64,12 +70,65 @@ def test_the_lines():
     assert ops._prefill_variant(plan_of([2048], bound=(2048, 1)), 2, 8)[4] == 44
 
 
+WHOLE = {16: [[1024, 1024], [900, 1200], [1100, 700], [512] * 4, [256] * 8, [700] * 4, [1333] * 3, [1569, 805, 1625], [2000, 2000]],
+         32: [[1024, 1024], [1177, 604], [1100, 700], [512] * 4, [256] * 8, [2000, 2000]], 64: [[1024, 1024], [1200], [512] * 4]}
+
+
+@pytest.mark.parametrize("H", WHOLE)
+def test_prompts_without_a_long_walk_of_their_own_stay_whole(H):
+    """... in the launch that such a step has without the rule: no second half of a grid that ends at once, heavy units beside light ones, two key groups."""
+    ops, uncut = rule(), rule()
+    uncut._cut_walks = lambda *args: (0, 0)
+    for lens in WHOLE[H]:
+        for bound in (None, (class_rows(sum(lens)), 8)):
+            plan = plan_of(lens, bound)
+            assert ops._prefill_variant(plan, H // 8, 8) == uncut._prefill_variant(plan, H // 8, 8), lens
+
+
+def test_the_walks_are_those_behind_the_contexts():
+    """A portion's walks begin at position zero: the limit grows with the context, and walks that are about equally long stay whole where they make
+    whole rounds. One long prompt beside others that are short is cut as it is alone."""
+    ops = rule()
+    variant = lambda lens, starts, H=16: ops._prefill_variant(plan_of(lens, starts=starts), H // 8, 8)
+    for start in (1024, 2048, 4096, 8192):
+        assert variant([2048], [start])[4] == 0 and variant([4096], [8192])[4] == 0
+    limits = [variant([3000], [start])[4] for start in (0, 256, 1024, 2048, 4096)]
+    assert limits == sorted(limits) and limits[0] < 50 and limits[-1] > 140
+    assert all(variant([rows], [start])[4] > 0 for rows, start in ((1536, 1024), (1536, 8192), (1700, 2048), (4096, 2048), (5000, 8192)))
+    assert variant([1900, 148], [0, 0])[4] > 0 and variant([3500, 100, 100], [0, 0, 0])[4] > 0
+    assert variant([2000] + [1] * 40, [0] + list(range(1100, 1500, 10)))[4] == 0               # decoding requests have more walks than the prompt
+    plan = plan_of([900, 1148])
+    plan.starts = ()                                                      # (a plan that does not say where they start)
+    assert ops._prefill_variant(plan, 2, 8)[4] == 0
+
+
+@pytest.mark.parametrize("H, Hkv", HEADS)
+def test_a_recordings_key_says_how_it_was_cut(H, Hkv):
+    """Every step of a class that is cut alike runs the same launch: what the key holds is what the launch rule makes of any of its steps, and a class has
+    few keys though its contexts differ."""
+    ops, rng, keys = rule(), random.Random(H), {}
+    for _ in range(3000):
+        lens, starts = [rng.randint(600, 2048)], [rng.choice([0, rng.randint(1, 4000)])]
+        if rng.random() < 0.3:
+            lens, starts = lens + [rng.randint(1, 200)], starts + [rng.randint(0, 1000)]
+        if sum(lens) > 2048:
+            continue
+        rows, seqs = class_rows(sum(lens)), len(lens)
+        nt, limit = key = ops.prompt_attention_path(lens, starts, rows, H, Hkv, 128)
+        got = ops._prefill_variant(plan_of(lens, (rows, seqs), starts), H // Hkv, Hkv)
+        assert (got[0], got[4]) == key if limit else got[4] == 0
+        cap = max(1024, 1 << (max(map(sum, zip(lens, starts))) - 1).bit_length())
+        keys.setdefault((rows, seqs, cap), set()).add(key)
+    assert max(map(len, keys.values())) <= 7 and sum(map(len, keys.values())) <= 3 * len(keys)
+    assert ops.prompt_attention_path([2048], [0], 2048, H, Hkv, 96) is None
+
+
 @pytest.mark.parametrize("rows", [1408, 2048, 4096])
 def test_a_plan_without_a_workspace_has_whole_walks(rows):
     """As every plan had before walks were cut; a forced cut has no room and is refused."""
     ops, plan, whole = rule(), plan_of([rows]), plan_of([rows])
     plan.workspace, ops_whole = None, rule()
-    ops_whole._prefill_limit = lambda *args: 0
+    ops_whole._cut_walks = lambda *args: (0, 0)
     nt, kw, units, busy, limit = ops._prefill_variant(plan, 2, 8)
     assert (nt, kw, units, busy, limit) == ops_whole._prefill_variant(whole, 2, 8)
     assert ops._prefill_room(plan.workspace, limit, nt, units, 8, 128) == (None, None, 0)

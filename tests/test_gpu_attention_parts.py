@@ -88,25 +88,99 @@ def test_sums_of_sigmoid_weights_in_two_parts(chunk, gated):
         assert float((out - outs[0]).norm() / outs[0].norm()) <= 2 * 2.0 ** -9
 
 
-@pytest.mark.parametrize("rows", [[2048], [1700], [4000], [900, 1200]])
-def test_the_rule_cuts_long_walks(rows):
-    """What the launch rule chooses for whole prompts gives what whole walks give, to the roundings of bfloat16 weights and results: 2^-9 each."""
+@pytest.mark.parametrize("rows, starts", [([2048], [0]), ([1700], [0]), ([4000], [0]), ([1500, 300], [0, 0]), ([1536], [1000]), ([1700], [4096]), ([3000], [700])])
+def test_the_rule_cuts_long_walks(rows, starts):
+    """What the launch rule chooses gives what whole walks give, to the roundings of bfloat16 weights and results: 2^-9 each."""
     ops, dtype, H, Hkv, D, ps = ops_for(torch.bfloat16), torch.bfloat16, 16, 8, 128, 16
-    n, pages = sum(rows), [-(-r // ps) for r in rows]
+    ctx = [r + s for r, s in zip(rows, starts)]
+    n, pages = sum(rows), [-(-c // ps) for c in ctx]
     g = torch.Generator(device="cuda").manual_seed(7)
     rand = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)
     q, kp, vp = rand(n, H * D), rand(sum(pages), Hkv, ps, D), rand(sum(pages), Hkv, D, ps)
     bt = torch.zeros(len(rows), max(pages), dtype=torch.int32)
     for s, p in enumerate(pages):
         bt[s, :p] = torch.arange(p) + sum(pages[:s])
-    pos = torch.cat([torch.arange(r) for r in rows]).int().cuda()
+    pos = torch.cat([torch.arange(s, s + r) for r, s in zip(rows, starts)]).int().cuda()
     seq = torch.cat([torch.full((r,), s) for s, r in enumerate(rows)]).int().cuda()
     outs = []
     for variant in ((1, 1), None):
-        plan = make_plan(rows, rows)
-        plan.prefill_variant = variant
+        plan = make_plan(rows, ctx)
+        plan.starts, plan.prefill_variant = starts, variant
         out = torch.full((n, H * D), float("nan"), dtype=dtype, device="cuda")
         ops.attention(q, out, kp, vp, bt.cuda(), ps, pos, seq, H, Hkv, D, D ** -0.5, None, plan=plan)
         outs.append(out.double())
-    assert ops._prefill_variant(plan, 2, Hkv)[4] > 0
+    limit = ops._prefill_variant(plan, 2, Hkv)[4]
+    assert limit > 0 and max(-(-c // 32) for c in ctx) >= limit + 8
     assert float((outs[1] - outs[0]).norm() / outs[0].norm()) <= 2 * 2.0 ** -9
+
+
+@pytest.mark.parametrize("nt", [1, 2])
+@pytest.mark.parametrize("form", [{"softcap": 20.0}, {"slopes": True}, {"sink": True}, {"softcap": 10.0, "slopes": True, "sink": True}])
+def test_scored_walks_in_two_parts(nt, form):
+    """Capped scores, a distance bias and a sink, which the two parts' maxima and sums count in once: as the whole walks, to the roundings of bfloat16."""
+    ops, dtype, H, Hkv, D, ps, n = ops_for(torch.bfloat16), torch.bfloat16, 4, 2, 64, 16, 900
+    g = torch.Generator(device="cuda").manual_seed(11)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)
+    q, kp, vp = rand(n, H * D), rand(-(-n // ps), Hkv, ps, D), rand(-(-n // ps), Hkv, D, ps)
+    pos, seq = torch.arange(n, dtype=torch.int32, device="cuda"), torch.zeros(n, dtype=torch.int32, device="cuda")
+    bt = torch.arange(-(-n // ps), dtype=torch.int32, device="cuda").view(1, -1)
+    if "slopes" in form:
+        form = dict(form, slopes=torch.tensor([2.0 ** -(h + 3) for h in range(H)], device="cuda"))
+    outs = []
+    for variant in ((nt, 1), (nt, 1, 2), (nt, 1, 12)):
+        plan = make_plan([n], [n])
+        plan.prefill_variant = variant
+        out = torch.full((n, H * D), float("nan"), dtype=dtype, device="cuda")
+        ops.attention(q, out, kp, vp, bt, ps, pos, seq, H, Hkv, D, D ** -0.5, None, plan=plan, **form)
+        outs.append(out.double())
+    for out in outs[1:]:
+        assert float((out - outs[0]).norm() / outs[0].norm()) <= 2 * 2.0 ** -9
+
+
+def test_a_recording_cuts_the_walks_of_any_step_of_its_class():
+    """Recorded for a class with more units than its steps have, replayed with eager work between for other cuts of it, one long prompt or several short ones,
+    behind contexts and not: the eager whole walks' results to the roundings of bfloat16, the same bits again, and counters at zero after every replay."""
+    from minivllm_amd.engine.step import class_rows
+    ops, dtype, H, Hkv, D, ps, rows, seqs = ops_for(torch.bfloat16), torch.bfloat16, 16, 8, 128, 16, 2048, 4
+    steps = [([2048], [0]), ([1900], [0]), ([1793], [100]), ([1800, 100, 1], [0, 0, 900]), ([500, 600, 700], [0, 300, 0]), ([2000], [0])]
+    g = torch.Generator(device="cuda").manual_seed(13)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)
+    pages = 4 * 128
+    q, kp, vp = rand(rows, H * D), rand(pages, Hkv, ps, D), rand(pages, Hkv, D, ps)
+    bt = torch.arange(pages, dtype=torch.int32, device="cuda").view(seqs, -1)
+
+    def tensors(lens, starts):
+        pad = [0] * (rows - sum(lens))
+        pos = torch.tensor([p for r, s in zip(lens, starts) for p in range(s, s + r)] + pad, dtype=torch.int32)
+        seq = torch.tensor([i for i, r in enumerate(lens) for _ in range(r)] + [-1] * len(pad), dtype=torch.int32)
+        ends = np.cumsum([0] + lens).tolist()
+        return pos, seq, torch.tensor(ends + [ends[-1]] * (seqs - len(lens)), dtype=torch.int32)
+    pos, seq, cu = (t.cuda() for t in tensors(*steps[0]))
+    plan = make_plan([2048], [2048])
+    plan.bound, plan.bound_least, plan.q_lens, plan.path_lens, plan.path_starts = (rows, seqs), 1793, (), tuple(steps[0][0]), tuple(steps[0][1])
+    plan.n_seqs, plan.cu_seqlens = seqs, cu
+    assert class_rows(1793) == rows and ops._prefill_variant(plan, H // Hkv, Hkv)[4] == 44
+    out = torch.zeros(rows, H * D, dtype=dtype, device="cuda")
+    run = lambda: ops.attention(q, out, kp, vp, bt, ps, pos, seq, H, Hkv, D, D ** -0.5, None, plan=plan)
+    run()
+    torch.cuda.synchronize()
+    plan.workspace.frozen = True
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    counters = ops._prompt_counters(plan.workspace)
+    seen = {}
+    for lens, starts in steps + steps[::-1]:
+        for t, new in zip((pos, seq, cu), tensors(lens, starts)):
+            t.copy_(new)
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert not bool(counters.any())
+        n = sum(lens)
+        whole = make_plan(lens, [r + s for r, s in zip(lens, starts)])
+        whole.prefill_variant = (1, 1)
+        ref = torch.empty(n, H * D, dtype=dtype, device="cuda")
+        ops.attention(q[:n], ref, kp, vp, bt[:len(lens)].contiguous(), ps, pos[:n], seq[:n], H, Hkv, D, D ** -0.5, None, plan=whole)
+        assert float((out[:n].double() - ref.double()).norm() / ref.double().norm()) <= 2 * 2.0 ** -9
+        assert torch.equal(seen.setdefault(str((lens, starts)), out[:n].clone()), out[:n])
