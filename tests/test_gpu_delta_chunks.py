@@ -215,8 +215,9 @@ def test_chunks_straight_from_the_rows(H, rank, weights, lens):
 @pytest.mark.parametrize("H, G, taps, weights", [(2, 1, 4, torch.bfloat16), (3, 3, 3, torch.float32), (4, 2, 2, torch.bfloat16)])
 @pytest.mark.parametrize("lens", [[128], [193, 0, 160], [145, 271]])
 def test_chunks_straight_from_convolved_rows(rule, H, G, taps, weights, lens):
-    """Against the vectors laid out in memory and the chunks behind them: the same terms, whose lengths are added up in another order, 2^-24 a term over
-    the 64 channels of a length and the tokens of a request. The kept inputs are the same bits."""
+    """Against the recurrence in float64 from the same rows: errors of float32 sums, 2^-24 a term over the 64 channels of a length and the tokens of a
+    request, and no larger than those of the vectors laid out in memory and the chunks behind them, which add up the same terms in another
+    order. The kept inputs are the same bits."""
     dtype, D, eps = torch.bfloat16, 64, 1e-6
     ops, n, channel = ops_for(dtype), sum(lens), rule == "channel"
     C = 2 * G * D + H * D
@@ -255,6 +256,28 @@ def test_chunks_straight_from_convolved_rows(rule, H, G, taps, weights, lens):
         assert bool(torch.isfinite(want).all())
         assert float((got.double() - want.double()).norm() / want.double().norm()) <= 16 * 2.0 ** -24 * 64 ** 0.5
     assert torch.equal(results[0][2], results[1][2])
+    f, taps_w, rate, bias = packed.double().cpu(), conv_w.double().cpu(), -torch.exp(a_log.double().cpu()), dt_bias.double().cpu()
+    for s, count in enumerate(lens):
+        first, slot = ends[s], len(lens) - s
+        if not count:
+            assert torch.equal(results[0][1][slot], state[slot])
+            continue
+        rows = f[first:first + count]
+        inputs = torch.cat([kept[slot].double().cpu(), rows[:, :C]])
+        x = torch.nn.functional.silu(sum(inputs[j:j + count] * taps_w[:, j] for j in range(taps)))
+        lengths = lambda t: t / (t.pow(2).sum(-1, keepdim=True) + eps).sqrt()
+        q, k = (lengths(x[:, j * G * D:(j + 1) * G * D].view(count, G, D)).repeat_interleave(H // G, 1) for j in range(2))
+        v, beta = x[:, 2 * G * D:].view(count, H, D), torch.sigmoid(rows[:, gate_off:gate_off + H])[..., None]
+        if channel:
+            before = z[first:first + count, :H * D].double().cpu() + bias
+            w = torch.exp(rate[:, None] * torch.nn.functional.softplus(before).view(count, H, D))
+        else:
+            w = torch.exp(rate * torch.nn.functional.softplus(rows[:, gate_off + H:gate_off + 2 * H] + bias))[..., None]
+        want, S = walk((w, w * k, -beta * k, beta * k, q * D ** -0.5, v), state[slot].double().cpu().transpose(1, 2))
+        for straight, laid_out, ref in ((results[0][0][first:first + count], results[1][0][first:first + count], want),
+                                        (results[0][1][slot].transpose(1, 2), results[1][1][slot].transpose(1, 2), S)):
+            err, err2 = (float((t.double().cpu() - ref).norm() / ref.norm()) for t in (straight, laid_out))
+            assert err <= 5e-6 and err <= 1.5 * err2 + 2.0 ** -24, (err, err2)
 
 
 @pytest.mark.parametrize("H", [1, 3])
