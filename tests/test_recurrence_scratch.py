@@ -57,8 +57,10 @@ def test_no_cut_has_more_units():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("graphs", [True, False])
-def test_scratch_stands_at_the_start(graphs):
-    """An engine that sizes its cache from the memory that is left: first long prompts of every kind of cut allocate no scratch."""
+@pytest.mark.parametrize("requests, rank", [(64, 8), (4, 64)])
+def test_scratch_stands_at_the_start(graphs, requests, rank):
+    """An engine that sizes its cache from the memory that is left: first long prompts of every kind of cut allocate no scratch. With four requests its
+    dry step's all go in chunks, and with a rank of 64 straight from the packed rows."""
     from minivllm_amd.config import EngineConfig
     from minivllm_amd.engine.executor import Executor
     from minivllm_amd.engine.step import SeqStep
@@ -67,14 +69,16 @@ def test_scratch_stands_at_the_start(graphs):
     mlp = {"kind": "dense", "ff": 128}
     arch, cfg = config_from_dict({"architecture": "Bolapel", "vocab": 256, "width": 128, "norm": {"eps": 1e-5}, "torch_dtype": "bfloat16",
                                   "logit_softcap": 20.0,
-                                  "layers": [{"type": "general_delta", "mixer": {"heads": 2, "dim": 64, "rank": 8}, "mlp": mlp}]})
+                                  "layers": [{"type": "general_delta", "mixer": {"heads": 2, "dim": 64, "rank": rank}, "mlp": mlp}]})
     source = DeviceRandomSource(expected_tensors(arch, cfg), 1, torch.bfloat16, torch.device("cuda:0"), std=0.05)
-    ex = Executor(EngineConfig(model="", dtype="bfloat16", max_model_len=1024, max_num_batched_tokens=1024, max_num_batched_seqs=64,
+    ex = Executor(EngineConfig(model="", dtype="bfloat16", max_model_len=1024, max_num_batched_tokens=1024, max_num_batched_seqs=requests,
                                kv_cache_block_size=16, gpu_memory_utilization=0.05, use_cuda_graph=graphs), model=(arch, cfg, source))
     areas = lambda: [ws.bytes() for ws in (ex.rt.workspace, ex._graph_workspace) if ws is not None]
     at_start = areas()
     assert len(at_start) == 1 + graphs
-    for lens in ([1024], [129] * 7, [700] + [1] * 60, [128], [383, 385, 200, 50]):
+    for lens in ([1024], [129] * 7, [700] + [1] * 60, [128], [383, 385, 200, 50], [900, 24], [1]):
+        if len(lens) > requests:
+            continue
         ex.step([SeqStep(tokens=[i % 256 for i in range(q)], start=0, block_tables=[[]] * len(ex.groups), state_slot=s, want=[q - 1])
                  for s, q in enumerate(lens)])
         torch.cuda.synchronize()
