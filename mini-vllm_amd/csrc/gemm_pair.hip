@@ -13,10 +13,11 @@
 //
 // The same kernel without the activation is mv_gemm_round: plain products whose tiles are one round of the compute units, which the
 // library is behind at where its own tiles leave units idle, above all for N that are no multiple of 256 (projections packed beside
-// one another). us, the library / here: 224 x 3104 x 1024 12.0 / 7.9, 1,024 17.3 / 14.1, 2,048 23.6 / 21.3; 2,048 x 5184 x 1024 34.0 / 29.4, 552
-// 16.0 / 13.3; 1,000 x 592 x 1024 8.9 / 7.1; 1,424 x 1024 x 1024 10.9 / 9.2; 2,048 x 2080 x 512 15.7 / 10.5. A tile takes what its operands take
-// through the compute unit, 192 KB of a 128 x 64 tile with K of 1,024 in 8 us; long K (2,048 x 1024 x 3072 23.4 / 23.9), N that fill the chip
-// with the library's 256 x 128 (2,048 x 4096 x 1024 22.6 / 22.9) and more than one round (4,096 x 3104 x 1024 37.9 / 42.2) stay where they were.
+// one another). us, the library / here: 224 x 3104 x 1024 12.0 / 8.0, 1,024 16.7 / 14.3, 2,048 23.0 / 21.0; 2,048 x 5184 x 1024 33.5 / 29.3, 552
+// 15.4 / 13.9; 1,000 x 592 x 1024 9.1 / 6.4; 2,048 x 2080 x 512 15.5 / 10.3. A tile takes what its operands take
+// through the compute unit, 192 KB of a 128 x 64 tile with K of 1,024 in 8 us; long K (2,048 x 1024 x 3072 22.8 / 23.5), N that fill the chip
+// with the library's 256 x 128 (2,048 x 4096 x 1024 21.5 / 23.0) and more than one round (4,096 x 3104 x 1024 37.6 / 38.5) stay where they were, and
+// so do some that the rule takes for slower than they are (1,424 x 1024 x 1024 10.7 / 8.3, 1,100 x 2048 x 2048 23.1 / 18.3).
 #include "gemm_deep.h"
 #include "gemm_ring.h"
 
@@ -55,7 +56,7 @@ enum PairForm { PAIR_PLAIN = 0, PAIR_GATED = 1, PAIR_FOLD = 2, PAIR_PLAIN_SCALED
 // for two of the rows and four of the weight, which comes from memory. A load's address is one scalar base an operand, advanced by a
 // chunk, and 32 bits a lane that do not change (64 bits a lane: two vector additions a load). With both, and the epilogue's forms apart,
 // us, weights that take turns, in turn with the kernel before: gated 6144 x 1024, 512 / 1,024 / 1,536 / 2,048 / 4,096 rows 13.2 -> 12.9, 18.2 -> 17.6,
-// 22.9 -> 21.8, 27.8 -> 27.2, 55.0 -> 52.8; plain 2,048 x 5184 x 1024 28.9 -> 28.2, 2,048 x 1024 x 2048 15.6 -> 13.6, x 3072 21.1 -> 18.9.
+// 22.9 -> 21.8, 27.8 -> 27.2, 55.0 -> 52.8; plain 1,024 x 3104 x 1024 14.8 -> 14.3, 2,048 x 1024 x 2048 16.7 -> 16.2, x 3072 and 2,048 x 5184 x 1024 level.
 template <int WM, int WN, int SA, int SB, int FORM>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_pair_kernel(PairArgs a) {
@@ -425,8 +426,8 @@ extern "C" int mv_gemm_pair(const void* A, long lda, const void* W, const void* 
     return launch_pair<PAIR_GATED>("gemm_pair", a, N, tile, stream);
 }
 
-// Columns of the plain product's tiles, and its time in us with tiles of bm x bn in one round, 0.05 apart from the measured ones (standard
-// deviation; 671 of 130 to 4,096 rows, K of 256 to 4,096): operands into LDS (bm + bn), out of it and through the matrix unit (bm bn), both slower
+// Columns of the plain product's tiles, and its time in us with tiles of bm x bn in one round, fitted to 671 of 130 to 4,096 rows, K of 256 to
+// 4,096, before the kernel's loads had a scalar base: of the kernel now 37 such took 3 % less, with a standard deviation of 6 %: operands into LDS (bm + bn), out of it and through the matrix unit (bm bn), both slower
 // the more units are at it.
 static const int kRoundColumns[] = {64, 96, 128, 192};
 static double round_time(int bm, int bn, int K, double tiles, int units) {

@@ -143,6 +143,8 @@ __device__ __forceinline__ size_t quad_of(int tile_row, int rows, int k_tile, in
 // ROWS of 2 to 4 (channel and gated rules, heads of 64 x 64): so many taps of the convolution that queries, keys and values pass first;
 // a token's four rows are read by four threads each, from L1. us, prepare + chunks / this: gated, 2,048 rows, 16 heads in 8 groups 21.5 + 41.1 / 47.1;
 // channel, 941 and 483 rows, 16 heads in 8 groups 29.2 + 36.5 / 41.4.
+// Heads of 128 have their vectors laid out still: a thread makes four channels of one token here, the workgroup 32 x 64, which is what
+// the designs' heads are at 0.6B and above.
 template <typename T, int DK, int RULE, int ROWS>
 __global__ void __launch_bounds__(DC_THREADS)
 delta_chunk_kernel(DeltaChunkArgs A) {

@@ -198,7 +198,7 @@ class SplitSum:
 
 class WeightedRows:
     """What ``Ops.gemm(..., fold=...)`` returns when it took the residual add and the norm into its
-    product: the rows of the new residual times the norm's weight (``weighted``, the activation
+    product (``Ops.can_fold_norm`` says in which steps): the rows of the new residual times the norm's weight (``weighted``, the activation
     type) and, per row, ``P`` partial sums of squares. ``Ops.gemm`` / ``Ops.gemm_swiglu`` take it as
     their input and divide their output rows by the root mean square; ``materialize()`` gives the
     normalised rows to anything else. Used once."""
@@ -2569,11 +2569,12 @@ class Ops:
         ``a`` may be a pending norm (parts.base.PendingNorm): then the residual add, the norm and
         the product run as one kernel when the step has at most 16 rows, else the norm runs first.
         ``a`` may also be ``WeightedRows``: the output rows are then divided by the rows' root mean
-        square where the weight-streaming kernel takes the shape, else the rows are normalised first.
+        square where a kernel that does so takes the shape (``can_fold_norm``), else the rows are normalised first.
 
         ``fold`` (parts.base.NormFold) offers the residual add and the norm behind this product: when
-        the weight-streaming kernel takes the shape it adds the product to the residual, leaves the
-        rows weighted for the norm, and ``WeightedRows`` is returned; ``out`` is not written then."""
+        the weight-streaming kernel takes the shape, or gemm_pair.hip or gemm_deep.hip does for a prompt's rows, it adds
+        the product to the residual, leaves the rows weighted for the norm, and ``WeightedRows`` is returned; ``out`` is
+        not written then."""
         if not isinstance(a, torch.Tensor):
             if isinstance(a, WeightedRows):
                 if not exact and self._gemm_scaled(a, w, out, bias, swiglu=False):
@@ -2906,9 +2907,10 @@ class Ops:
 
     def can_fold_norm(self, rows: int, width: int, consumer=None) -> bool:
         """Whether a residual add and a norm over ``rows`` x ``width`` may be offered to the product in
-        front of them (``gemm(..., fold=...)``): steps of up to SKINNY_MAX_M rows, when the product
-        behind the norm (``consumer`` = (weight rows, weight columns, gated)) is one the
-        weight-streaming kernel takes — behind any other the rows would have to be normalised by a
+        front of them (``gemm(..., fold=...)``): steps of up to SKINNY_WIDE_MAX_M rows, when the product
+        behind the norm (``consumer`` = (weight rows, weight columns, gated); unknown: up to SKINNY_MAX_M rows) is one the
+        weight-streaming kernel takes, and prompts of 129 to ``most_fold_rows`` rows, when it is one that gemm_pair.hip or
+        gemm_deep.hip takes from such rows (``mv_gemm_behind_norm``) — behind any other the rows would have to be normalised by a
         kernel of their own, and nothing is gained (32B sizes, where gate/up goes to the library: 2 %
         slower). Where both this and the fused add + norm + product kernel could serve (up to 16
         rows), this is taken: the product behind reads finished bf16 rows instead of normalising

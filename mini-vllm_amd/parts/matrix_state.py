@@ -70,7 +70,7 @@ CHUNKS_BESIDE_SHORT_CLASS = 1024
 # 140 / 168, channel decays 151 / 285; four of 512, 64 heads 235 / 361, 171 / 236, 167 / 151, 167 / 247; one of 2,048,
 # 64 heads 450 / 342, 476 / 216, 411 / 155, 474 / 230; 16 of 256, 16 heads of 128 442 / 548, 237 / 512, 227 / 225, 274 / 525.
 # (Since then the walk along the chunks takes 37 us instead of 57 at 2,048 tokens, the general rule's chunks 52 instead of 67 and the vectors'
-# kernels in front of them, 15 to 29 us, are gone: the line lies on the scan's side of where the two meet now.)
+# kernels in front of them, 15 to 29 us, are gone where no request is scanned: the line lies on the scan's side of where the two meet now.)
 _SCAN_TOKEN = {64: 0.22, 128: 0.32}
 _CHUNKS_ONCE = {64: (18.0, 0.013), 128: (29.0, 0.018)}
 _CHUNKS_TOKEN_HEAD = {"delta": {64: 2.4, 128: 7.6}, "gated": {64: 1.55, 128: 7.0}, "channel": {64: 1.6, 128: 7.1},
